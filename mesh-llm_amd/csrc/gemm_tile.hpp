@@ -1,0 +1,192 @@
+// Main loop of the large-tile products: 16-bit operands (f16 or bf16) straight from memory into LDS, f32 sums on the matrix cores.
+//
+// A workgroup of WM x WT waves owns a tile of 64 WM weight rows x 64 WT tokens, a wave 64 x 64 of it (2 x 2 blocks of
+// v_mfma_f32_32x32x16).  K goes by in steps of 32: a step's operands are (WM + WT) * 4 chunks of 1 KB, one per 16 rows, and
+// a chunk is one global_load_lds_dwordx4 of a wave.  Three stages of LDS: while step k is multiplied step k + 1 has
+// been requested and step k + 2 is being requested, so a wave waits with the loads of one step still in flight (vmcnt(PER),
+// exact because every wave issues the same number of loads per step) and one barrier per step serves both ways: behind it the step has
+// landed for everybody, and everybody is done with the stage that the next loads overwrite.
+//
+// What bounds it: the clock.  256 x 128 tiles reach 1110-1250 TFLOP/s (M 28672, K 4096 and M 4096, K 14336, 2048 tokens), at
+// which the chip lowers its clock; 128 of those tiles alone run at 82% of the matrix cores' nominal rate, 256 at 50%.
+// 64 x 64 per wave measured against 128 x 64 per wave (half the waves): 436 against 502 us for M 28672, K 4096; steps of 64 with
+// two stages 604, with three 466; four stages of 32 462; s_setprio around the products 432 against 436-496.
+//
+// The loads are issued by inline asm because the compiler counts LDS writes of the builtin as conflicting with the
+// fragment reads of the other stages across the loop's back edge and waits for all of them.  The asm has no outputs; its
+// operands are read when it issues.
+#pragma once
+
+#include <type_traits>
+
+#include "mesh_common.hpp"
+
+namespace mesh {
+
+typedef float gt_f16v __attribute__((ext_vector_type(16)));
+typedef uint32_t gt_u4 __attribute__((ext_vector_type(4)));
+typedef _Float16 gt_h8 __attribute__((ext_vector_type(8)));
+typedef __bf16 gt_b8 __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ gt_f16v gt_mma(gt_h8 a, gt_h8 b, gt_f16v c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ gt_f16v gt_mma(gt_b8 a, gt_b8 b, gt_f16v c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
+
+// How the operands lie in memory.
+//   GT_BLOCKS: blocks of 16 rows, element (r, k) at ((k / 8) * 16 + r % 16) * 8 + k % 8 of the block's 16 * K: a chunk is
+//              contiguous, and in LDS (the same order) a fragment read covers 256 contiguous bytes per 16 lanes.
+//   GT_ROWS:   plain rows of K elements.  A chunk is 64 bytes of each of 16 rows, kept in LDS as 16-byte piece p of row r at
+//              position p ^ ((r / 4) % 4), so that 16 rows' same piece falls on all 64 banks; the swizzle is
+//              applied to the source address, because the destination of such a load is linear in the lane.
+// Half lines of 16 rows cost the address path four times a contiguous chunk's lines: M 28672, K 4096, 2048 tokens take 410 us with
+// both operands in blocks, 465 with only the weights, 530 with plain rows (M 4096, K 14336: 187, 192, 233).
+enum GtLayout { GT_BLOCKS = 0, GT_ROWS = 1 };
+
+constexpr int GT_K = 32;                       // elements of K per step
+constexpr int GT_STAGES = 3;
+constexpr int gt_lds_bytes(int WM, int WT) { return GT_STAGES * (WM + WT) * 4096; }
+// waves per SIMD of the workgroups that a CU's 160 KB of LDS hold
+constexpr int gt_waves_per_simd(int WM, int WT) { return 160 * 1024 / gt_lds_bytes(WM, WT) * WM * WT / 4; }
+
+// Tile and split of a product.  Three tiles are built: 128 x 128 (weight rows x tokens), 256 x 128, 256 x 192.  A launch's time goes
+// as the rounds its workgroups make over the CUs times the tile's size times its share of K; the small tile reads more LDS
+// per product (1.2).  A slice costs writing and reading its result, and split_ns once where the reader is a launch of its own.
+// Measured, us (M, K, tokens):
+//   28672, 4096, 2048: 256x128 432, 128x128 500      28672, 4096, 333: 256x192 88, 256x128 106, 128x128 105
+//   6144, 4096, 2048:  128x128 94, 256x128 98        4096, 14336, 333: 256x128 in 4 slices 46, 128x128 in 2 57, whole 99
+//   2048, 8192, 900:   128x128 in 2 slices 37, in 4 38, whole 55; 256x128 in 4 41        4096, 4096, 333: in 2 slices 19, whole 29
+struct GtPlan {
+    int wm = 2, wt = 2, slices = 1, k_slice = 0;       // waves (of 64 rows) by waves (of 64 tokens); steps of a slice
+};
+inline int gt_n_cu() {
+    static const int n = [] {
+        int dev = 0, cu = 0;
+        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cu <= 0) cu = 256;
+        return cu;
+    }();
+    return n;
+}
+// slices_max, slices_room: the most slices the caller takes, and has room for
+inline GtPlan gt_plan(int M, int T, int K, int slices_max, size_t slices_room, double split_ns, int n_cu = gt_n_cu()) {
+    static constexpr struct { int wm, wt; double ns; } tiles[3] = {{4, 2, 11.4}, {2, 2, 6.8}, {4, 3, 17.0}};      // ns: one round's time per element of K
+    GtPlan best;
+    double least = 0;
+    const int steps = K / GT_K;
+    for (const auto &t : tiles)
+        for (int s = 1; s <= slices_max && (size_t)s <= slices_room && (s == 1 || K / s >= 256); s *= 2) {
+            const long n = (long)((M + 64 * t.wm - 1) / (64 * t.wm)) * ((T + 64 * t.wt - 1) / (64 * t.wt)) * s;
+            const int k_slice = (steps + s - 1) / s;
+            const double cost = (double)((n + n_cu - 1) / n_cu) * t.ns * k_slice * GT_K + (s > 1 ? s * (double)T * M * 0.00145 + split_ns : 0.0);
+            if (least != 0 && cost >= least) continue;
+            least = cost;
+            best.wm = t.wm; best.wt = t.wt; best.k_slice = k_slice;
+            best.slices = (steps + k_slice - 1) / k_slice;      // no empty slice
+        }
+    return best;
+}
+
+// acc += W x over steps [k0, k0 + n_steps), n_steps >= 1.  w, x: 16-bit elements, rows of ldw and ldx (GT_BLOCKS: both K); w_block, x_block: first 16-row block of the
+// tile; w_blocks: blocks the matrix holds; x_rows: rows x holds (GT_BLOCKS: up to a whole block).  Blocks and rows past the end
+// repeat the last one; what they multiply is never stored.  SWAP: result rows = tokens, columns (lanes) = weight rows.
+template <class V, GtLayout LW, GtLayout LX, int WM, int WT, bool SWAP>
+__device__ __forceinline__ void gt_multiply(char *smem, gt_f16v (&acc)[2][2], const void *w, int ldw, const void *x, int ldx, int k0, int n_steps, int w_block, int w_blocks,
+                                            int x_block, int x_rows) {
+    constexpr int WAVES = WM * WT, CHUNKS = (WM + WT) * 4, PER = (CHUNKS + WAVES - 1) / WAVES, STAGE = CHUNKS * 1024;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
+    // this wave's chunks: uniform base, byte offset of the lane, place in the stage.  (A wave with fewer chunks than PER brings the last
+    // one again: the same bytes to the same place, and every wave has PER loads per step in flight.)
+    const char *src[PER];
+    uint32_t off[PER], place[PER], step_bytes[PER];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const int c = wave * PER + j < CHUNKS ? wave * PER + j : CHUNKS - 1;
+        const bool is_w = c < WM * 4;
+        int b = is_w ? w_block + c : x_block + c - WM * 4;
+        const int last = is_w ? w_blocks - 1 : (x_rows - 1) / 16;
+        b = b < last ? b : last;
+        const int ld = is_w ? ldw : ldx;
+        src[j] = static_cast<const char *>(is_w ? w : x) + (size_t)b * 32 * (size_t)ld;
+        place[j] = lds0 + c * 1024;
+        const bool blocks = (is_w ? LW : LX) == GT_BLOCKS;
+        step_bytes[j] = blocks ? 1024 : 64;             // from one step's chunk to the next one's
+        if (blocks) {
+            off[j] = (uint32_t)k0 * 1024u + lane * 16;
+        } else {
+            int r = lane >> 2;
+            const int piece = (lane & 3) ^ ((r >> 2) & 3);
+            if (!is_w && r > x_rows - 1 - 16 * b) r = x_rows - 1 - 16 * b;
+            off[j] = (uint32_t)r * (uint32_t)ld * 2u + piece * 16 + (uint32_t)k0 * 64u;
+        }
+    }
+    auto load = [&](int stage, int k) {
+        const uint32_t at = (uint32_t)(k < n_steps ? k : n_steps - 1);        // (past the end: the last step again, read by nobody)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"         // (m0 is reserved: named so that the compiler keeps its own uses away)
+#pragma unroll
+        for (int j = 0; j < PER; ++j)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(place[j] + stage * STAGE)), "v"(off[j] + at * step_bytes[j]), "s"(src[j])
+                         : "memory", "m0");
+#pragma clang diagnostic pop
+    };
+    // fragments of this wave's 64 rows: lane -> row lane % 32 of a 32-row half, 8 elements from 8 * (lane / 32) of a k16 step
+    const int r16 = lane & 15, half = lane >> 5;
+    const int in_blocks = ((lane & 31) >> 4) * 1024 + half * 256 + r16 * 16, in_rows = ((lane & 31) >> 4) * 1024 + r16 * 64 + (half ^ (r16 >> 2)) * 16;
+    const int wf_at = (wave % WM) * 4096 + (LW == GT_BLOCKS ? in_blocks : in_rows), xf_at = (WM + wave / WM) * 4096 + (LX == GT_BLOCKS ? in_blocks : in_rows);
+    V wf[2][2], xf[2][2];
+    auto read = [&](const char *st, int ks) {
+        auto place_of = [&](GtLayout l, int at) { return l == GT_BLOCKS ? at + 512 * ks : at ^ (32 * ks); };
+#pragma unroll
+        for (int j = 0; j < 2; ++j) xf[ks][j] = *reinterpret_cast<const V *>(st + place_of(LX, xf_at) + 2048 * j);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) wf[ks][i] = *reinterpret_cast<const V *>(st + place_of(LW, wf_at) + 2048 * i);
+    };
+    auto step = [&](int stage, auto more, int next_stage, int next_k) {
+        const char *st = smem + stage * STAGE;
+        read(st, 0);
+        if constexpr (decltype(more)::value) load(next_stage, next_k);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            if (ks == 0) read(st, 1);
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] = SWAP ? gt_mma(xf[ks][i], wf[ks][j], acc[i][j]) : gt_mma(wf[ks][i], xf[ks][j], acc[i][j]);
+            if (ks == 0) {
+                // the second half's fragments are requested between the first half's products
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __builtin_amdgcn_s_setprio(0);
+    };
+    load(0, 0);
+    load(1, 1);
+    int k = 0;
+    for (; k + GT_STAGES <= n_steps; k += GT_STAGES) {
+#pragma unroll
+        for (int i = 0; i < GT_STAGES; ++i) {
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(PER) : "memory");
+            step(i, std::true_type{}, (i + 2) % GT_STAGES, k + i + 2);
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (k < n_steps) step(0, std::false_type{}, 0, 0);
+    if (k + 1 < n_steps) step(1, std::false_type{}, 0, 0);
+}
+
+// 1-D grid of row tiles x token tiles: the workgroups a die is dealt (every eighth) take a contiguous run of tiles, the token tile
+// running fastest, so that a die's cache keeps the weight rows of its run
+__device__ __forceinline__ void gt_place(int tile, int n_tiles, int n_ttiles, int &mt, int &tt) {
+    const int per = n_tiles >> 3, whole = per << 3;
+    if (tile < whole) tile = (tile & 7) * per + (tile >> 3);
+    mt = tile / n_ttiles;
+    tt = tile % n_ttiles;
+}
+
+}  // namespace mesh

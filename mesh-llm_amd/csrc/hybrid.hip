@@ -29,7 +29,9 @@ int hybrid_session_alloc(mesh_session *s) {
     h.xa = buf(B * (size_t)hm.width_pad * ab);
     h.acta = buf(B * (size_t)hm.act_max * std::max(ab, sizeof(float)));        // (the single-token step keeps f32 vectors in it)
     h.big = fbuf(B * (size_t)hm.in_max);
-    h.y = fbuf(B * E);
+    // room for the slices of a product that few tiles cover: as many tiles as there are CUs, and one result at least
+    h.y_floats = std::max(B * E, std::min(B * E * LINEAR_SLICES_MAX, (size_t)8 << 20));
+    h.y = fbuf(h.y_floats);
     h.q = fbuf(B * (size_t)hm.q_max);
     h.part = fbuf(2 * 3 * STEP_PARTS_MAX);
     h.ws = fbuf(hm.state_max ? min_gru_workspace((int)B, hm.state_max) : 0);
@@ -393,11 +395,20 @@ int hybrid_run_layers(mesh_session *s, int T, int max_keys) {
         return linear(W, x, act, T, y, ldy, s->tune.linear_tile_min_tokens, stream);
     };
     // the residual stream after a sublayer, and the next one's input
-    auto add = [&](const float *y, const RowNorm &post, const RowNorm &pre) {
+    auto add = [&](const float *y, int slices, const RowNorm &post, const RowNorm &pre) {
         ProfScope ps(s, MESH_PROF_PREP);
-        return residual_norm_rows(s->x, y, post, pre, eps, T, E, h.xa, act, hm.width_pad, stream);
+        return residual_norm_rows(s->x, y, slices, (size_t)T * E, post, pre, eps, T, E, h.xa, act, hm.width_pad, stream);
     };
-    if ((rc = add(nullptr, RowNorm{}, hm.layers[0].pre1)) != MESH_OK) return rc;
+    // a sublayer's last product, added to it
+    auto close = [&](const LinearWeight &W, const RowNorm &post, const RowNorm &pre) {
+        int slices;
+        {
+            ProfScope ps(s, MESH_PROF_GEMV);
+            slices = linear_sliced(W, h.acta, act, T, h.y, (size_t)T * E, h.y_floats, s->tune.linear_tile_min_tokens, stream);
+        }
+        return slices < 0 ? slices : add(h.y, slices, post, pre);
+    };
+    if ((rc = add(nullptr, 1, RowNorm{}, hm.layers[0].pre1)) != MESH_OK) return rc;
     for (size_t il = 0; il < hm.layers.size(); ++il) {
         const HybridLayer &L = hm.layers[il];
         const MixerSpec &m = L.spec.mixer;
@@ -418,7 +429,7 @@ int hybrid_run_layers(mesh_session *s, int T, int max_keys) {
             ProfScope ps(s, MESH_PROF_PREP);
             if ((rc = min_gru(a, T, stream)) != MESH_OK) return rc;
         }
-        if ((rc = product(L.out, h.acta, h.y, E)) != MESH_OK || (rc = add(h.y, L.post1, L.spec.ff ? L.pre2 : after)) != MESH_OK) return rc;
+        if ((rc = close(L.out, L.post1, L.spec.ff ? L.pre2 : after)) != MESH_OK) return rc;
         if (L.spec.ff) {
             if (hm.spec.ff == FF_POLY_NORM) {
                 if ((rc = product(L.up, h.xa, h.big, L.spec.ff)) != MESH_OK) return rc;
@@ -428,14 +439,14 @@ int hybrid_run_layers(mesh_session *s, int T, int max_keys) {
                 ProfScope ps(s, MESH_PROF_GEMV);
                 if ((rc = linear_relu2(L.up, h.xa, act, T, h.acta, L.down.Kp, s->tune.linear_tile_min_tokens, stream)) != MESH_OK) return rc;
             }
-            if ((rc = product(L.down, h.acta, h.y, E)) != MESH_OK || (rc = add(h.y, L.post2, after)) != MESH_OK) return rc;
+            if ((rc = close(L.down, L.post2, after)) != MESH_OK) return rc;
         }
         if (!hm.side()) continue;
         int slices;
         const size_t slice = (size_t)T * hm.spec.side_dim;
         {
             ProfScope ps(s, MESH_PROF_GEMV);
-            if ((slices = linear_sliced(L.side_gate, h.xa, act, T, h.big, slice, s->tune.linear_tile_min_tokens, stream)) < 0) return slices;
+            if ((slices = linear_sliced(L.side_gate, h.xa, act, T, h.big, slice, (size_t)st->n_batch_max * hm.in_max, s->tune.linear_tile_min_tokens, stream)) < 0) return slices;
         }
         {
             ProfScope ps(s, MESH_PROF_PREP);
@@ -443,7 +454,7 @@ int hybrid_run_layers(mesh_session *s, int T, int max_keys) {
                                      hm.spec.side_dim, h.acta, act, L.side_proj.Kp, stream)) != MESH_OK)
                 return rc;
         }
-        if ((rc = product(L.side_proj, h.acta, h.y, E)) != MESH_OK || (rc = add(h.y, L.post_side, RowNorm{})) != MESH_OK) return rc;
+        if ((rc = close(L.side_proj, L.post_side, RowNorm{})) != MESH_OK) return rc;
     }
     return MESH_OK;
 }
@@ -455,7 +466,7 @@ int hybrid_finish(mesh_session *s, int T, float **x) {
     if (!hybrid_single_step(s, T)) return MESH_OK;
     *x = h.tail_step.x;
     ProfScope ps(s, MESH_PROF_PREP);
-    return residual_norm_rows(h.tail_step.x, h.tail_step.y, h.tail_step.post, RowNorm{}, hm.spec.eps, 1, hm.spec.width, h.xa, hm.act, hm.width_pad, s->stream);
+    return residual_norm_rows(h.tail_step.x, h.tail_step.y, 1, 0, h.tail_step.post, RowNorm{}, hm.spec.eps, 1, hm.spec.width, h.xa, hm.act, hm.width_pad, s->stream);
 }
 
 int hybrid_logits(mesh_session *s, int T, const int32_t *d_rows, int n_rows, float *d_out) {

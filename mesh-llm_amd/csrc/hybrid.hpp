@@ -64,6 +64,7 @@ struct HybridPending {
 
 struct HybridSession {
     void *xa = nullptr, *acta = nullptr;                // activations of the products: the residual stream, and a sublayer's inside
+    size_t y_floats = 0;                                // room in y (linear_sliced)
     float *big = nullptr, *y = nullptr, *q = nullptr, *ws = nullptr, *x2 = nullptr;
     float *part = nullptr;                              // two sets of STEP_PARTS_MAX x 3 partial sums
     std::vector<uint8_t *> k, v;                        // per local layer (attention; latent attention: k, its rows)

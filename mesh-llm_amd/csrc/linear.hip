@@ -6,19 +6,16 @@
 // v_mfma_f32_16x16x32_bf16: step j multiplies element j of every lane's 8, and the sum over lanes groups and steps covers
 // the same 32 products.
 //
-// linear_tile_kernel is the large-tile product (128 weight rows x 128 tokens x 64 k): both operands go from memory to
-// LDS without passing through registers, two stages, one barrier per stage.  Rows of 64 elements are 128 bytes, eight
-// 16-byte pieces; piece p of row r is kept at position p ^ ((r >> 1) & 7), so that the 16 rows a fragment read touches at
-// a time fall on all 64 banks.  The destination of such a load is linear in the lane, so the swizzle is applied to the
-// source address.
+// linear_tile_kernel is the large-tile product of gemm_tile.hpp: plain bf16 activation rows, weights in blocks of 16 rows where the
+// stage keeps such a copy, else plain rows.
 #include "linear.hpp"
+
+#include "gemm_tile.hpp"
 
 namespace mesh {
 
 typedef __bf16 ln_b8 __attribute__((ext_vector_type(8)));
 typedef float ln_f4 __attribute__((ext_vector_type(4)));
-typedef float ln_f16 __attribute__((ext_vector_type(16)));
-typedef uint32_t ln_u4 __attribute__((ext_vector_type(4)));
 
 constexpr int ROWS_WAVES = 4;
 
@@ -113,100 +110,35 @@ __global__ __launch_bounds__(64 * ROWS_WAVES) void linear_rows_kernel(const uint
 }
 
 // ---- large tile -----------------------------------------------------------------------------------------------
-constexpr int TILE_M = 128, TILE_T = 128, TILE_K = 64, TILE_THREADS = 256;
-
-typedef const __attribute__((address_space(1))) uint32_t *ln_gptr;
-typedef __attribute__((address_space(3))) uint32_t *ln_lptr;
-
-__device__ __forceinline__ void tile_copy16(const uint16_t *src, uint16_t *lds_base) {
-    __builtin_amdgcn_global_load_lds((ln_gptr)(src), (ln_lptr)(lds_base), 16, 0, 0);
-}
-
-// 1-D grid of (row blocks x token blocks); the workgroups a die is dealt (every eighth) take a contiguous run of tiles with
-// the token block running fastest, so that the weight rows of a run stay in that die's cache
-template <LinearOut OUT>
-__global__ __launch_bounds__(TILE_THREADS) void linear_tile_kernel(const uint16_t *w, const uint16_t *x, void *y, int K, int M, int T, int ldy,
-                                                                   int n_tblocks, int n_tiles, int k_slice, size_t y_slice) {
-    // blockIdx.y: slice of K and the partial result it writes
-    const int k_begin = blockIdx.y * k_slice, k_end = k_begin + k_slice < K ? k_begin + k_slice : K;
-    y = static_cast<float *>(y) + blockIdx.y * y_slice;          // (slices are f32 results)
-    __shared__ __align__(16) uint16_t sW0[TILE_M * TILE_K], sW1[TILE_M * TILE_K], sX0[TILE_T * TILE_K], sX1[TILE_T * TILE_K];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    int tile = blockIdx.x;
-    {
-        const int per = n_tiles >> 3, whole = per << 3;
-        if (tile < whole) tile = (tile & 7) * per + (tile >> 3);
-    }
-    const int mb = tile / n_tblocks, tb = tile % n_tblocks;
-    const int wm = (wave & 1) * 64, wt = (wave >> 1) * 64;      // this wave's 64 x 64 corner of the tile
-    // staging: instruction j of a wave brings rows 32 * wave + 8 * j .. + 8, lane -> (row lane / 8, position lane % 8)
-    const uint16_t *gw[4], *gx[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int r = wave * 32 + j * 8 + (lane >> 3);
-        const int piece = (lane & 7) ^ ((r >> 1) & 7);
-        gw[j] = w + (size_t)(mb * TILE_M + r) * K + piece * 8;
-        const int t = tb * TILE_T + r;
-        gx[j] = x + (size_t)(t < T ? t : T - 1) * K + piece * 8;
-    }
-    auto stage = [&](uint16_t *dw, uint16_t *dx, int k) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            tile_copy16(gw[j] + k, dw + (wave * 32 + j * 8) * TILE_K);
-            tile_copy16(gx[j] + k, dx + (wave * 32 + j * 8) * TILE_K);
-        }
-    };
-    ln_f16 acc[2][2];
+// blockIdx.y: slice of K (k_slice steps) and the partial result it writes, y_slice floats apart
+template <LinearOut OUT, GtLayout LW, int WM, int WT>
+__global__ __launch_bounds__(64 * WM * WT, gt_waves_per_simd(WM, WT)) void linear_tile_kernel(const uint16_t *w, const uint16_t *x, void *y, int K, int M, int T, int ldy, int row_blocks,
+                                                                                           int n_ttiles, int n_tiles, int k_slice, size_t y_slice) {
+    __shared__ __align__(1024) char smem[gt_lds_bytes(WM, WT)];
+    int mt, tt;
+    gt_place(blockIdx.x, n_tiles, n_ttiles, mt, tt);
+    const int n_all = K / GT_K, k0 = blockIdx.y * k_slice, n_steps = n_all - k0 < k_slice ? n_all - k0 : k_slice;
+    gt_f16v acc[2][2];
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
             for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.f;
-    const int r32 = lane & 31, half = lane >> 5;
-    const int sw = (r32 >> 1) & 7;                // (row >> 1) & 7 is the same for the rows 32 and 64 further down
-    auto multiply = [&](const uint16_t *dw, const uint16_t *dx) {
-#pragma unroll
-        for (int ks = 0; ks < TILE_K / 16; ++ks) {
-            const int at = ((2 * ks + half) ^ sw) * 8;
-            ln_b8 xf[2], wf[2];
-#pragma unroll
-            for (int a = 0; a < 2; ++a) {
-                xf[a] = *reinterpret_cast<const ln_b8 *>(dx + (wt + 32 * a + r32) * TILE_K + at);
-                wf[a] = *reinterpret_cast<const ln_b8 *>(dw + (wm + 32 * a + r32) * TILE_K + at);
-            }
-            // result: rows = tokens, columns (lanes) = weight rows, so that a store covers whole lines of y
-#pragma unroll
-            for (int a = 0; a < 2; ++a)
-#pragma unroll
-                for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[a], wf[b], acc[a][b], 0, 0, 0);
-        }
-    };
-    // One barrier per stage: behind it every wave's loads of this stage have landed, and every wave is done reading the
-    // other stage, which the next loads overwrite.
-    auto arrive = [&]() {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-    };
-    stage(sW0, sX0, k_begin);
-    for (int k = k_begin; k < k_end; k += 2 * TILE_K) {
-        arrive();
-        if (k + TILE_K < k_end) stage(sW1, sX1, k + TILE_K);
-        multiply(sW0, sX0);
-        if (k + TILE_K >= k_end) break;
-        arrive();
-        if (k + 2 * TILE_K < k_end) stage(sW0, sX0, k + 2 * TILE_K);
-        multiply(sW1, sX1);
-    }
+    gt_multiply<gt_b8, LW, GT_ROWS, WM, WT, true>(smem, acc, w, K, x, K, k0, n_steps, mt * WM * 4, row_blocks * 8, tt * WT * 4, T);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int m0 = (mt * WM + wave % WM) * 64, t0 = (tt * WT + wave / WM) * 64;
+    y = static_cast<float *>(y) + blockIdx.y * y_slice;          // (slices are f32 results)
+    // register i of a lane: token 8 * (i / 4) + 4 * (lane / 32) + i % 4, weight row lane % 32: a store covers whole lines of y
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
-        const int m = mb * TILE_M + wm + 32 * b + r32;
+        const int m = m0 + 32 * b + (lane & 31);
         if (m >= M) continue;
 #pragma unroll
         for (int a = 0; a < 2; ++a)
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-                const int t = tb * TILE_T + wt + 32 * a + 8 * (i >> 2) + 4 * half + (i & 3);
+                const int t = t0 + 32 * a + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
                 if (t < T) linear_store<ACT_BF16, OUT>(y, (size_t)t * ldy + m, acc[a][b][i]);
             }
     }
@@ -224,49 +156,68 @@ static int launch_rows(const LinearWeight &W, const void *x, int T, void *y, int
     return MESH_OK;
 }
 
-template <LinearOut OUT>
-static int launch_tile(const LinearWeight &W, const void *x, int T, void *y, int ldy, int M, int slices, size_t stride, hipStream_t stream) {
-    const int mblocks = (M + TILE_M - 1) / TILE_M, tblocks = (T + TILE_T - 1) / TILE_T;
-    const int steps = W.Kp / TILE_K, k_slice = (steps + slices - 1) / slices * TILE_K;
-    MESH_LAUNCH((linear_tile_kernel<OUT>), dim3((unsigned)(mblocks * tblocks), (unsigned)slices), dim3(TILE_THREADS), 0, stream, W.w, static_cast<const uint16_t *>(x), y, W.Kp, M,
-                T, ldy, tblocks, mblocks * tblocks, k_slice, stride);
+__global__ __launch_bounds__(256) void linear_blocks_kernel(const uint16_t *w, uint16_t *dst, int K, size_t pieces) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;        // 16-byte piece of dst: row i % 16 of its block, k from 8 * (i / 16 % (K / 8))
+    if (i >= pieces) return;
+    const size_t k8 = i / 16 % (K / 8), row = i / (2 * (size_t)K) * 16 + i % 16;
+    reinterpret_cast<uint4 *>(dst)[i] = *reinterpret_cast<const uint4 *>(w + row * K + k8 * 8);
+}
+
+int linear_make_blocks(const LinearWeight &W, uint16_t *dst, hipStream_t stream) {
+    if (!W.w || !dst || W.Mp % 16 || W.Kp % 8) return fail(MESH_ERR_INVALID, "linear_make_blocks: bad operands (%d x %d)", W.M, W.K);
+    const size_t pieces = (size_t)W.Mp * W.Kp / 8;
+    MESH_LAUNCH(linear_blocks_kernel, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, stream, W.w, dst, W.Kp, pieces);
     MESH_LAUNCH_CHECK();
     return MESH_OK;
+}
+
+template <LinearOut OUT, GtLayout LW>
+static int launch_tile_layout(const uint16_t *w, const LinearWeight &W, const void *x, int T, void *y, int ldy, int M, const GtPlan &p, size_t stride, hipStream_t stream) {
+    const int row_blocks = W.Mp / 128, mtiles = (M + 64 * p.wm - 1) / (64 * p.wm), ttiles = (T + 64 * p.wt - 1) / (64 * p.wt);
+    const dim3 grid((unsigned)(mtiles * ttiles), (unsigned)p.slices), block((unsigned)(64 * p.wm * p.wt));
+    const uint16_t *xb = static_cast<const uint16_t *>(x);
+    if (p.wt == 3) MESH_LAUNCH((linear_tile_kernel<OUT, LW, 4, 3>), grid, block, 0, stream, w, xb, y, W.Kp, M, T, ldy, row_blocks, ttiles, mtiles * ttiles, p.k_slice, stride);
+    else if (p.wm == 4) MESH_LAUNCH((linear_tile_kernel<OUT, LW, 4, 2>), grid, block, 0, stream, w, xb, y, W.Kp, M, T, ldy, row_blocks, ttiles, mtiles * ttiles, p.k_slice, stride);
+    else MESH_LAUNCH((linear_tile_kernel<OUT, LW, 2, 2>), grid, block, 0, stream, w, xb, y, W.Kp, M, T, ldy, row_blocks, ttiles, mtiles * ttiles, p.k_slice, stride);
+    MESH_LAUNCH_CHECK();
+    return MESH_OK;
+}
+template <LinearOut OUT>
+static int launch_tile(const LinearWeight &W, const void *x, int T, void *y, int ldy, int M, const GtPlan &p, size_t stride, hipStream_t stream) {
+    return W.blocks ? launch_tile_layout<OUT, GT_BLOCKS>(W.blocks, W, x, T, y, ldy, M, p, stride, stream) : launch_tile_layout<OUT, GT_ROWS>(W.w, W, x, T, y, ldy, M, p, stride, stream);
 }
 
 static bool linear_ok(const LinearWeight &W, const void *x, int T, const void *y, int ldy) {
     return W.w && x && y && W.M >= 1 && W.Kp % LINEAR_K_PAD == 0 && W.Mp % LINEAR_ROW_PAD == 0 && W.Mp >= W.M && W.Kp >= W.K && ldy >= W.M && (T + 63) / 64 <= 65535;
 }
 
-int linear_sliced(const LinearWeight &W, const void *x, ActType act, int T, float *y, size_t stride, int big_from, hipStream_t stream) {
-    const int tiles = (W.M + TILE_M - 1) / TILE_M * ((T + TILE_T - 1) / TILE_T), steps = W.Kp / TILE_K;
-    int slices = 128 / (tiles > 0 ? tiles : 1);
-    if (slices > LINEAR_SLICES_MAX) slices = LINEAR_SLICES_MAX;
-    if (slices > steps / 4) slices = steps / 4;                  // (a slice of at least four steps)
-    if (slices > 1) slices = (steps + (steps + slices - 1) / slices - 1) / ((steps + slices - 1) / slices);        // every slice has some
-    if (act == ACT_F32 || T < big_from || slices <= 1 || stride < (size_t)T * W.M) {
+int linear_sliced(const LinearWeight &W, const void *x, ActType act, int T, float *y, size_t stride, size_t y_floats, int big_from, hipStream_t stream) {
+    if (T <= 0) return 1;
+    if (!linear_ok(W, x, T, y, W.M) || stride < (size_t)T * W.M || y_floats < stride) return fail(MESH_ERR_INVALID, "linear_sliced: bad operands (%d x %d, %d tokens)", W.M, W.K, T);
+    GtPlan p;
+    if (act == ACT_BF16 && T >= big_from) p = gt_plan(W.M, T, W.Kp, LINEAR_SLICES_MAX, y_floats / stride, 0.0);
+    if (p.slices <= 1) {
         const int rc = linear(W, x, act, T, y, W.M, big_from, stream);
         return rc == MESH_OK ? 1 : rc;
     }
-    if (!linear_ok(W, x, T, y, W.M)) return fail(MESH_ERR_INVALID, "linear_sliced: bad operands (%d x %d, %d tokens)", W.M, W.K, T);
-    const int rc = launch_tile<LINEAR_OUT_F32>(W, x, T, y, W.M, W.M, slices, stride, stream);
-    return rc == MESH_OK ? slices : rc;
+    const int rc = launch_tile<LINEAR_OUT_F32>(W, x, T, y, W.M, W.M, p, stride, stream);
+    return rc == MESH_OK ? p.slices : rc;
 }
 
 int linear(const LinearWeight &W, const void *x, ActType act, int T, float *y, int ldy, int big_from, hipStream_t stream) {
     if (T <= 0) return MESH_OK;
     if (!linear_ok(W, x, T, y, ldy)) return fail(MESH_ERR_INVALID, "linear: bad operands (%d x %d, %d tokens)", W.M, W.K, T);
     if (act == ACT_F32) return launch_rows<ACT_F32, LINEAR_OUT_F32>(W, x, T, y, ldy, W.M, stream);
-    if (T < big_from || W.M < TILE_M) return launch_rows<ACT_BF16, LINEAR_OUT_F32>(W, x, T, y, ldy, W.M, stream);
-    return launch_tile<LINEAR_OUT_F32>(W, x, T, y, ldy, W.M, 1, 0, stream);
+    if (T < big_from || W.M < 128) return launch_rows<ACT_BF16, LINEAR_OUT_F32>(W, x, T, y, ldy, W.M, stream);
+    return launch_tile<LINEAR_OUT_F32>(W, x, T, y, ldy, W.M, gt_plan(W.M, T, W.Kp, 1, 1, 0.0), 0, stream);
 }
 
 int linear_relu2(const LinearWeight &W, const void *x, ActType act, int T, void *out, int ld, int big_from, hipStream_t stream) {
     if (T <= 0) return MESH_OK;
     if (!linear_ok(W, x, T, out, ld) || ld > W.Mp) return fail(MESH_ERR_INVALID, "linear_relu2: bad operands (%d x %d, %d tokens)", W.M, W.K, T);
     if (act == ACT_F32) return launch_rows<ACT_F32, LINEAR_OUT_RELU2>(W, x, T, out, ld, ld, stream);
-    if (T < big_from || W.M < TILE_M) return launch_rows<ACT_BF16, LINEAR_OUT_RELU2>(W, x, T, out, ld, ld, stream);
-    return launch_tile<LINEAR_OUT_RELU2>(W, x, T, out, ld, ld, 1, 0, stream);
+    if (T < big_from || W.M < 128) return launch_rows<ACT_BF16, LINEAR_OUT_RELU2>(W, x, T, out, ld, ld, stream);
+    return launch_tile<LINEAR_OUT_RELU2>(W, x, T, out, ld, ld, gt_plan(ld, T, W.Kp, 1, 1, 0.0), 0, stream);
 }
 
 }  // namespace mesh

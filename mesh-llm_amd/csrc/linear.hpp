@@ -15,11 +15,16 @@ inline size_t act_bytes(ActType a) { return a == ACT_BF16 ? 2 : 4; }
 constexpr int LINEAR_ROW_PAD = 128, LINEAR_K_PAD = 64;
 struct LinearWeight {
     const uint16_t *w = nullptr;
+    const uint16_t *blocks = nullptr;      // optional second copy in the large tile's layout (gemm_tile.hpp: GT_BLOCKS)
     int M = 0, K = 0, Mp = 0, Kp = 0;
     bool present() const { return w != nullptr; }
 };
 inline int linear_rows_padded(int M) { return (M + LINEAR_ROW_PAD - 1) / LINEAR_ROW_PAD * LINEAR_ROW_PAD; }
 inline int linear_k_padded(int K) { return (K + LINEAR_K_PAD - 1) / LINEAR_K_PAD * LINEAR_K_PAD; }
+
+// Writes W in the large tile's layout: linear_blocks_bytes(W) bytes at dst.
+inline size_t linear_blocks_bytes(const LinearWeight &W) { return (size_t)W.Mp * W.Kp * 2; }
+int linear_make_blocks(const LinearWeight &W, uint16_t *dst, hipStream_t stream);
 
 // y[t][m] = sum_k W[m][k] x[t][k] for t < T.  x: rows of W.Kp elements of `act` (columns from K on hold zeros), 16-byte
 // aligned; y: f32 rows of ldy.  big_from: bf16 calls of at least this many tokens take the large-tile kernel.
@@ -28,11 +33,11 @@ int linear(const LinearWeight &W, const void *x, ActType act, int T, float *y, i
 // product that follows.
 int linear_relu2(const LinearWeight &W, const void *x, ActType act, int T, void *out, int ld, int big_from, hipStream_t stream);
 
-// The same for a matrix of few rows (hundreds), which leaves the large tile with few workgroups: K is cut into slices, each of
-// which writes its own partial y, `stride` floats apart; the reader adds them in order.  Returns the slice count (1: y is
-// the product) or a negative status.  y holds at least LINEAR_SLICES_MAX * T * W.M floats.
+// The same for a result that few large tiles cover: where that is faster K is cut into slices, each of which writes its own
+// partial y, `stride` floats apart; the reader adds them in order.  Returns the slice count (1: y is the product) or a
+// negative status.  y has room for y_floats; slices that do not fit are not made.
 constexpr int LINEAR_SLICES_MAX = 8;
-int linear_sliced(const LinearWeight &W, const void *x, ActType act, int T, float *y, size_t stride, int big_from, hipStream_t stream);
+int linear_sliced(const LinearWeight &W, const void *x, ActType act, int T, float *y, size_t stride, size_t y_floats, int big_from, hipStream_t stream);
 
 // ---- one token ------------------------------------------------------------------------------------------------
 // A mat-vec whose workgroups derive the input vector themselves from what the launch before them left, and whose epilogue

@@ -59,41 +59,80 @@ __global__ __launch_bounds__(ROW_THREADS) void embed_rows_kernel(const uint16_t 
     }
 }
 
-template <ActType ACT, int V>
-__global__ __launch_bounds__(ROW_THREADS) void residual_norm_kernel(float *x, const float *y, const float *gain, float eps, int n, void *out, int ld) {
+// y as its producer left it: partial products `stride` floats apart, added in order
+struct SlicedRows {
+    const float *y;
+    int slices;
+    size_t stride;
+};
+template <int V> __device__ __forceinline__ RowVec<V> sliced_load(const SlicedRows &s, size_t at) {
+    RowVec<V> r = row_load<V>(s.y + at);
+    for (int k = 1; k < s.slices; ++k) {
+        const RowVec<V> p = row_load<V>(s.y + k * s.stride + at);
+#pragma unroll
+        for (int j = 0; j < V; ++j) r.v[j] += p.v[j];
+    }
+    return r;
+}
+
+// NV groups of V elements of y stay in a thread's registers (NV 0: rows of any length, read again)
+template <ActType ACT, int V, int NV>
+__global__ __launch_bounds__(ROW_THREADS) void residual_norm_kernel(float *x, const SlicedRows y, const float *gain, float eps, int n, void *out, int ld) {
     __shared__ float scratch[ROW_WAVES];
     const size_t at = (size_t)blockIdx.x * n, to = (size_t)blockIdx.x * ld;
-    float rinv = 0.f;
-    if (y) {
-        float ss = 0.f;
-#pragma unroll 4
-        for (int i = threadIdx.x * V; i < n; i += ROW_THREADS * V) {
-            const RowVec<V> r = row_load<V>(y + at + i);
+    RowVec<V> keep[NV ? NV : 1];
+    auto squares = [](const RowVec<V> &r, float ss) {
 #pragma unroll
-            for (int j = 0; j < V; ++j) ss = fmaf(r.v[j], r.v[j], ss);
+        for (int j = 0; j < V; ++j) ss = fmaf(r.v[j], r.v[j], ss);
+        return ss;
+    };
+    float rinv = 0.f;
+    if (y.y) {
+        float ss = 0.f;
+        if constexpr (NV > 0) {
+#pragma unroll
+            for (int k = 0; k < NV; ++k) {
+                const int i = (k * ROW_THREADS + (int)threadIdx.x) * V;
+                if (i < n) keep[k] = sliced_load<V>(y, at + i);
+            }
+#pragma unroll
+            for (int k = 0; k < NV; ++k)
+                if ((k * ROW_THREADS + (int)threadIdx.x) * V < n) ss = squares(keep[k], ss);
+        } else {
+#pragma unroll 4
+            for (int i = threadIdx.x * V; i < n; i += ROW_THREADS * V) ss = squares(sliced_load<V>(y, at + i), ss);
         }
         rinv = 1.0f / sqrtf(row_sum(ss, scratch) / (float)n + eps);
     }
-#pragma unroll 4
-    for (int i = threadIdx.x * V; i < ld; i += ROW_THREADS * V) {
+    auto put = [&](int i, const RowVec<V> &r) {
         RowVec<V> v = {};
         if (i < n) {
             v = row_load<V>(x + at + i);
-            if (y) {
-                const RowVec<V> r = row_load<V>(y + at + i), g = row_load<V>(gain + i);
+            if (y.y) {
+                const RowVec<V> g = row_load<V>(gain + i);
 #pragma unroll
                 for (int j = 0; j < V; ++j) v.v[j] = v.v[j] + r.v[j] * rinv * g.v[j];
                 row_store<V>(x + at + i, v);
             }
         }
         act_store_row<ACT, V>(out, to + i, v);
+    };
+    int done = 0;
+    if constexpr (NV > 0) {
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+            const int i = (k * ROW_THREADS + (int)threadIdx.x) * V;
+            if (i < ld) put(i, keep[k]);
+        }
+        done = NV * ROW_THREADS * V;
     }
+    for (int i = done + threadIdx.x * V; i < ld; i += ROW_THREADS * V) put(i, NV == 0 && y.y && i < n ? sliced_load<V>(y, at + i) : RowVec<V>{});
 }
 
 // The same with layer norms on both sides: x += post(y), act = pre(x).  A thread keeps its NV groups of V elements of the row
 // in registers (NV 0: rows of any length, read again for every pass).  Means first, then squared deviations.
 template <ActType ACT, int V, int NV>
-__global__ __launch_bounds__(ROW_THREADS) void layer_norm_kernel(const float *src, const int32_t *row, float *x, const float *y, const RowNorm post, const RowNorm pre,
+__global__ __launch_bounds__(ROW_THREADS) void layer_norm_kernel(const float *src, const int32_t *row, float *x, const SlicedRows y, const RowNorm post, const RowNorm pre,
                                                                  float eps, int n, void *out, int ld) {
     __shared__ float scratch[ROW_WAVES];
     constexpr int NR = NV ? NV : 1;
@@ -111,28 +150,28 @@ __global__ __launch_bounds__(ROW_THREADS) void layer_norm_kernel(const float *sr
             for (int i = threadIdx.x * V; i < n; i += ROW_THREADS * V) fn(i, r[0]);
         }
     };
-    auto moments = [&](const float *p, float &mean, float &rstd) {
+    auto moments = [&](const SlicedRows &p, float &mean, float &rstd) {
         float s = 0.f;
         each([&](int i, RowVec<V> &v) {
-            if (NV == 0) v = row_load<V>(p + i);
+            if (NV == 0) v = sliced_load<V>(p, at + i);
 #pragma unroll
             for (int j = 0; j < V; ++j) s += v.v[j];
         });
         mean = row_sum(s, scratch) * inv_n;
         float d2 = 0.f;
         each([&](int i, RowVec<V> &v) {
-            if (NV == 0) v = row_load<V>(p + i);
+            if (NV == 0) v = sliced_load<V>(p, at + i);
 #pragma unroll
             for (int j = 0; j < V; ++j) { const float d = v.v[j] - mean; d2 = fmaf(d, d, d2); }
         });
         rstd = 1.0f / sqrtf(row_sum(d2, scratch) * inv_n + eps);
     };
     float mean, rstd;
-    if (y) {
-        if (NV > 0) each([&](int i, RowVec<V> &v) { v = row_load<V>(y + at + i); });
-        moments(y + at, mean, rstd);
+    if (y.y) {
+        if (NV > 0) each([&](int i, RowVec<V> &v) { v = sliced_load<V>(y, at + i); });
+        moments(y, mean, rstd);
         each([&](int i, RowVec<V> &v) {
-            if (NV == 0) v = row_load<V>(y + at + i);
+            if (NV == 0) v = sliced_load<V>(y, at + i);
             const RowVec<V> g = row_load<V>(post.gain + i), b = row_load<V>(post.bias + i), xv = row_load<V>(src + at + i);
 #pragma unroll
             for (int j = 0; j < V; ++j) v.v[j] = xv.v[j] + ((v.v[j] - mean) * rstd * g.v[j] + b.v[j]);
@@ -144,7 +183,7 @@ __global__ __launch_bounds__(ROW_THREADS) void layer_norm_kernel(const float *sr
     }
     if (!out) return;
     mean = 0.f; rstd = 1.f;
-    if (pre.kind == NORM_LAYER) moments(src + at, mean, rstd);
+    if (pre.kind == NORM_LAYER) moments(SlicedRows{src, 1, 0}, mean, rstd);
     each([&](int i, RowVec<V> &v) {
         if (NV == 0) v = row_load<V>(src + at + i);
         RowVec<V> o = v;
@@ -159,7 +198,7 @@ __global__ __launch_bounds__(ROW_THREADS) void layer_norm_kernel(const float *sr
 }
 
 template <ActType ACT>
-static int launch_layer_norm(const float *src, const int32_t *row, float *x, const float *y, const RowNorm &post, const RowNorm &pre, float eps, int rows, int n, void *out, int ld,
+static int launch_layer_norm(const float *src, const int32_t *row, float *x, const SlicedRows &y, const RowNorm &post, const RowNorm &pre, float eps, int rows, int n, void *out, int ld,
                              hipStream_t stream) {
     const dim3 grid((unsigned)rows), block(ROW_THREADS);
     const int groups = n % 4 == 0 ? (n + 4 * ROW_THREADS - 1) / (4 * ROW_THREADS) : 0;
@@ -289,23 +328,36 @@ int embed_rows(const uint16_t *table, int ldt, const int32_t *tok, const int32_t
 
 static bool norm_ok(const RowNorm &nm) { return nm.kind == NORM_NONE || (nm.gain && (nm.kind == NORM_RMS || nm.bias)); }
 
-int residual_norm_rows(float *x, const float *y, const RowNorm &post, const RowNorm &pre, float eps, int T, int n, void *out, ActType act, int ld, hipStream_t stream) {
+template <ActType ACT>
+static int launch_residual_norm(float *x, const SlicedRows &y, const float *gain, float eps, int T, int n, void *out, int ld, hipStream_t stream) {
+    const dim3 grid((unsigned)T), block(ROW_THREADS);
+    const int groups = n % 4 == 0 ? (n + 4 * ROW_THREADS - 1) / (4 * ROW_THREADS) : 0;
+    if (groups == 1) MESH_LAUNCH((residual_norm_kernel<ACT, 4, 1>), grid, block, 0, stream, x, y, gain, eps, n, out, ld);
+    else if (groups == 2) MESH_LAUNCH((residual_norm_kernel<ACT, 4, 2>), grid, block, 0, stream, x, y, gain, eps, n, out, ld);
+    else if (groups >= 3 && groups <= 4) MESH_LAUNCH((residual_norm_kernel<ACT, 4, 4>), grid, block, 0, stream, x, y, gain, eps, n, out, ld);
+    else if (groups) MESH_LAUNCH((residual_norm_kernel<ACT, 4, 0>), grid, block, 0, stream, x, y, gain, eps, n, out, ld);
+    else MESH_LAUNCH((residual_norm_kernel<ACT, 1, 0>), grid, block, 0, stream, x, y, gain, eps, n, out, ld);
+    MESH_LAUNCH_CHECK();
+    return MESH_OK;
+}
+
+int residual_norm_rows(float *x, const float *y, int slices, size_t slice_stride, const RowNorm &post, const RowNorm &pre, float eps, int T, int n, void *out, ActType act, int ld, hipStream_t stream) {
     if (T <= 0) return MESH_OK;
-    if (ld < n || !norm_ok(post) || !norm_ok(pre) || (y && post.kind == NORM_NONE) || pre.kind == NORM_RMS) return fail(MESH_ERR_INVALID, "residual_norm_rows: bad operands");
+    if (ld < n || !norm_ok(post) || !norm_ok(pre) || (y && post.kind == NORM_NONE) || pre.kind == NORM_RMS || slices < 1) return fail(MESH_ERR_INVALID, "residual_norm_rows: bad operands");
+    const SlicedRows ys{y, slices, slice_stride};
     if (post.kind == NORM_LAYER || pre.kind == NORM_LAYER) {
         if (y && post.kind != NORM_LAYER) return fail(MESH_ERR_UNSUPPORTED, "residual_norm_rows: no kernel for norm %d before norm %d", (int)post.kind, (int)pre.kind);
-        return act == ACT_BF16 ? launch_layer_norm<ACT_BF16>(x, nullptr, x, y, post, pre, eps, T, n, out, ld, stream)
-                               : launch_layer_norm<ACT_F32>(x, nullptr, x, y, post, pre, eps, T, n, out, ld, stream);
+        return act == ACT_BF16 ? launch_layer_norm<ACT_BF16>(x, nullptr, x, ys, post, pre, eps, T, n, out, ld, stream)
+                               : launch_layer_norm<ACT_F32>(x, nullptr, x, ys, post, pre, eps, T, n, out, ld, stream);
     }
-    MESH_ROW_LAUNCH(residual_norm_kernel, act, n % 4 == 0, dim3((unsigned)T), dim3(ROW_THREADS), x, y, post.gain, eps, n, out, ld);
-    return MESH_OK;
+    return act == ACT_BF16 ? launch_residual_norm<ACT_BF16>(x, ys, post.gain, eps, T, n, out, ld, stream) : launch_residual_norm<ACT_F32>(x, ys, post.gain, eps, T, n, out, ld, stream);
 }
 
 int layer_norm_rows(const float *x, const int32_t *row, const RowNorm &norm, float eps, int n_rows, int n, void *out, ActType act, int ld, hipStream_t stream) {
     if (n_rows <= 0) return MESH_OK;
     if (ld < n || norm.kind != NORM_LAYER || !norm_ok(norm)) return fail(MESH_ERR_INVALID, "layer_norm_rows: bad operands");
-    return act == ACT_BF16 ? launch_layer_norm<ACT_BF16>(x, row, nullptr, nullptr, RowNorm{}, norm, eps, n_rows, n, out, ld, stream)
-                           : launch_layer_norm<ACT_F32>(x, row, nullptr, nullptr, RowNorm{}, norm, eps, n_rows, n, out, ld, stream);
+    return act == ACT_BF16 ? launch_layer_norm<ACT_BF16>(x, row, nullptr, SlicedRows{nullptr, 1, 0}, RowNorm{}, norm, eps, n_rows, n, out, ld, stream)
+                           : launch_layer_norm<ACT_F32>(x, row, nullptr, SlicedRows{nullptr, 1, 0}, RowNorm{}, norm, eps, n_rows, n, out, ld, stream);
 }
 
 int scalar_norm_rows(const float *x, const int32_t *row, const float *gain, float eps, int n_rows, int n, void *out, ActType act, int ld, hipStream_t stream) {

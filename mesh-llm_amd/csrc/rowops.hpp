@@ -18,8 +18,9 @@ struct RowNorm {
 // sin and cos of pos * freq[i]
 int embed_rows(const uint16_t *table, int ldt, const int32_t *tok, const int32_t *pos, const float *freq, float scale, int T, int n, float *x, hipStream_t stream);
 
-// x[t] += post(y[t]) (y null: x as it is), and act[t] = pre(x[t]): post RMS with pre NONE, or both LAYER
-int residual_norm_rows(float *x, const float *y, const RowNorm &post, const RowNorm &pre, float eps, int T, int n, void *out, ActType act, int ld, hipStream_t stream);
+// x[t] += post(y[t]) (y null: x as it is), and act[t] = pre(x[t]): post RMS with pre NONE, or both LAYER; y as the sum of
+// `slices` partial products (linear_sliced)
+int residual_norm_rows(float *x, const float *y, int slices, size_t slice_stride, const RowNorm &post, const RowNorm &pre, float eps, int T, int n, void *out, ActType act, int ld, hipStream_t stream);
 
 // act[i] = layer norm of x[row[i]] for i < n_rows (row null: i)
 int layer_norm_rows(const float *x, const int32_t *row, const RowNorm &norm, float eps, int n_rows, int n, void *out, ActType act, int ld, hipStream_t stream);

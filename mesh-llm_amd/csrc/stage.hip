@@ -242,6 +242,14 @@ int stage_select_device(const mesh_stage_opts *opts, mesh_stage *st) {
     return MESH_OK;
 }
 
+// Second copies of the weights that the large tile reads faster are kept where they take at most an eighth of the memory that is
+// free once the stage is loaded: the rest belongs to the caller's sessions.
+bool stage_copies_fit(size_t bytes) {
+    size_t free_bytes = 0, total = 0;
+    if (hipMemGetInfo(&free_bytes, &total) != hipSuccess) { (void)hipGetLastError(); return false; }
+    return bytes <= free_bytes / 8;
+}
+
 // what every kind of model takes from the options
 static int stage_common_opts(const mesh_stage_opts *opts, mesh_stage *st) {
     int rc;

@@ -68,6 +68,7 @@ int session_attention(mesh_session *s, int layer, const float *d_q, const mesh_b
 int stage_decode_dev(mesh_session *s, const mesh_batch *b, const void *d_in, int in_fmt, void *d_out, int out_fmt, size_t out_cap, size_t *out_len);
 // shared by the runners
 int stage_select_device(const mesh_stage_opts *opts, mesh_stage *st);
+bool stage_copies_fit(size_t bytes);
 int sess_alloc(mesh_session *s, void **p, size_t bytes);
 int attn_splits_for(const Tuning &tune, int T, int n_kv, int max_keys, bool quantised);
 // names the kernel class of the launches made while it lives (mesh_session_profile)

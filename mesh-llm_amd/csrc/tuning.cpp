@@ -15,6 +15,7 @@ const TuningField *tuning_fields() {
         {"gemm_layout", &Tuning::gemm_layout, 0, 1, TUNE_STAGE},
         {"gemm_min_tokens", &Tuning::gemm_min_tokens, 1, 1 << 20, TUNE_STAGE},
         {"skinny_min_tokens", &Tuning::skinny_min_tokens, 0, 1 << 20, TUNE_STAGE},
+        {"tile_copies", &Tuning::tile_copies, 0, 1, TUNE_STAGE},
         {"gemm_splitk", &Tuning::gemm_splitk, 0, 1, TUNE_SESSION},
         {"chunk_kv16", &Tuning::chunk_kv16, 0, 1, TUNE_SESSION},
         {"gemv_rope", &Tuning::gemv_rope, 0, 1, TUNE_SESSION},

@@ -18,6 +18,7 @@ struct Tuning {
     int gemm_layout = 1;           // stages that can be handed prefill-sized calls keep a GEMM-layout copy of their projections
     int gemm_min_tokens = 17;      // calls with at least this many tokens take the large-tile MFMA GEMM
     int skinny_min_tokens = 0;     // ... and at least this many the skinny MFMA GEMM; 0 = 4 with skinny_f16, 5 without
+    int tile_copies = 1;           // stages that can be handed prefill-sized calls keep second copies of their projections for the large tile (gemm_tile.hpp)
     // --- SESSION: mesh_session_set_option
     int gemm_splitk = 1;           // GEMM launches too narrow to fill the chip split K over workgroups
     int chunk_kv16 = 1;            // long prefill chunks over a quantised cache decode a layer's rows once into an f16 copy

@@ -1,0 +1,49 @@
+"""The large-tile products at the edges of their tiles: rows, tokens and steps along K that leave remainders, every tile shape and
+split that the plan picks, against the plain oracle."""
+import os
+import sys
+
+import numpy as np
+import pytest
+
+sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
+import nadosun_util as N
+from folder_util import error, open_stage, run
+from oracle.nadosun import NadosunOracle
+from util import mesh
+
+pytestmark = pytest.mark.gpu
+
+# rms of a row's difference over the rms of all rows: the bound of the other bf16 comparisons with this oracle
+BF16_LIMIT = 2e-2
+
+
+@pytest.mark.parametrize("width,ff,tokens", [
+    (136, 130, 128),        # one tile of rows and a few rows more, one of tokens
+    (136, 1090, 129),       # a row of tokens past the tile; down projection of 34 steps, whole or in slices of 17
+    (320, 1160, 191),       # 38 steps: two left behind whole rounds of the stages
+    (256, 4100, 383),       # down projection in several slices, the last one shorter
+    (128, 28800, 250),      # enough tiles of 256 x 128 to fill the chip
+    (128, 28800, 300),      # 256 x 192: the second tile of tokens mostly empty
+    (128, 28804, 385),      # one token in the last tile, four rows in the last block
+])
+def test_products_of_many_tokens(tmp_path, width, ff, tokens):
+    """A feed-forward of `ff` behind attention over `tokens` tokens: products of (rows, K) = (ff, width) and (width, ff)."""
+    cfg = N.config(64, width, 8, [N.attention(2, 1, 64, 50, ff=ff)])
+    w = N.random_weights(cfg, 3)
+    folder = N.write_folder(str(tmp_path / "model"), cfg, w)
+    t = N.prompt(cfg, tokens, 9)
+    want = NadosunOracle(cfg, w).forward(t)[-100:]
+    plain = open_stage(folder, "bf16", n_ctx=512, batch=512, tuning={"tile_copies": 0})
+    st = open_stage(folder, "bf16", n_ctx=512, batch=512)
+    got = run(st, t, [tokens], last=100)
+    # the same tiles over weights in plain rows: the same products in the same order
+    assert np.array_equal(run(plain, t, [tokens], last=100), got)
+    plain.close()
+    rows = run(st, t, [tokens], last=100, linear_tile_min_tokens=1 << 20)      # the weight-streaming kernel on the same inputs
+    st.close()
+    assert np.isfinite(got).all()
+    assert error(got, want) < BF16_LIMIT, (width, ff, tokens, error(got, want))
+    # the two add the same products of the same bf16 values in another order (1e-6); a result next to a rounding point of the next
+    # product's bf16 input moves by 2^-8 of itself there: a small share of what the oracle's bound allows for all inputs
+    assert error(got, rows) < BF16_LIMIT / 2, (width, ff, tokens, error(got, rows))
