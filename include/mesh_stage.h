@@ -277,8 +277,8 @@ int mesh_session_f16_saturations(mesh_session *session, uint64_t *count);
  *     gemm_min_tokens=17   calls of at least this many tokens run the large-tile MFMA GEMM
  *     skinny_min_tokens=0  calls of at least this many (and fewer than the above) run the skinny MFMA GEMM;
  *                          0 = 4 with skinny_f16, 5 without
- *     tile_copies=1        second copies of the projections for prefill-sized calls (bf16 models: as many bytes again),
- *                          where they take at most an eighth of the GPU's free memory
+ *     tile_copies=1        second copies of the projections for prefill-sized calls (bf16 models: as many bytes again; K-quant models:
+ *                          2 bytes per weight, f16), where they take at most an eighth of the GPU's free memory
  *   session level:
  *     gemm_splitk=1        GEMM launches too narrow to fill the chip split K over workgroups
  *     chunk_kv16=1         long prefill chunks over a quantised cache decode a layer's rows once into an f16 copy
@@ -299,6 +299,7 @@ int mesh_session_f16_saturations(mesh_session *session, uint64_t *count);
  *     moe_router_tail=1    small decode batches: the router launch's last workgroup routes and groups the pairs
  *     moe_fuse_quant=1     the expert combine step quantises for the next layer
  *     moe_gemm=1, moe_gemm_min_pairs=4   prefill-sized expert products on the large-tile GEMM
+ *     tile_min_tokens=129  K-quant products of at least this many tokens on the large tile, over the copies of tile_copies
  *     grouped_oversub=8    grouped expert mat-vec: workgroups per compute unit and item
  *     linear_tile_min_tokens=128  bf16 products of at least this many tokens on the large matrix-core tile
  *     latent_chunk_min_tokens=128  latent attention: chunks of at least this many tokens project their sequence's keys and values

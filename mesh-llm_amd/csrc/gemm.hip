@@ -785,6 +785,15 @@ __global__ __launch_bounds__(256) void gemm_splitk_epilogue_kernel(GemmArgs a, i
     }
 }
 
+int gemm_add_slices(const GemmArgs &k, int row_blocks, hipStream_t stream) {
+    const int t_pad = k.y16_k8 ? (k.T + 15) & ~15 : k.T;
+    const size_t n = (size_t)t_pad * row_blocks * (k.y16_k8 ? GM / 8 : GM / 4);
+    const unsigned blocks = (unsigned)std::min<size_t>((n + 255) / 256, 4096);
+    MESH_LAUNCH(gemm_splitk_epilogue_kernel, dim3(blocks), dim3(256), 0, stream, k, row_blocks);
+    MESH_LAUNCH_CHECK();
+    return MESH_OK;
+}
+
 template <int TYPE, bool PACKED, bool XDIRECT, bool SPLIT, bool NARROW, bool GROUPED = false>
 static int launch_gemm_kernel(const GemmArgs &k, dim3 grid, hipStream_t stream) {
     // two stages of the weight slab, and of the activation slab unless the activations bypass LDS: 73 728 / 36 864 B
@@ -796,14 +805,7 @@ static int launch_gemm_kernel(const GemmArgs &k, dim3 grid, hipStream_t stream) 
     }
     MESH_LAUNCH((gemm_kq_kernel<TYPE, PACKED, XDIRECT, SPLIT, NARROW, GROUPED>), grid, dim3(GEMM_THREADS), smem, stream, k);
     MESH_LAUNCH_CHECK();
-    if (SPLIT) {
-        const int t_pad = k.y16_k8 ? (k.T + 15) & ~15 : k.T;
-        const size_t n = (size_t)t_pad * grid.x * (k.y16_k8 ? GM / 8 : GM / 4);
-        const unsigned blocks = (unsigned)std::min<size_t>((n + 255) / 256, 4096);
-        MESH_LAUNCH(gemm_splitk_epilogue_kernel, dim3(blocks), dim3(256), 0, stream, k, (int)grid.x);
-        MESH_LAUNCH_CHECK();
-    }
-    return MESH_OK;
+    return SPLIT ? gemm_add_slices(k, (int)grid.x, stream) : MESH_OK;
 }
 
 static int gemm_n_cu() {
@@ -843,6 +845,7 @@ static int split_plan(const GemmArgs &a, int row_blocks, int t_blocks, int *k_pe
 
 int gemm_split_count(const GemmArgs &a) {
     if (a.M <= 0 || a.K <= 0 || a.T <= 0) return 1;
+    if (gemm_tile_takes(a)) return gemm_tile_slices(a);
     const int row_blocks = a.y16_k8 ? (a.M + GM / 2 - 1) / (GM / 2) : (a.M + GM - 1) / GM;
     int kps;
     return split_plan(a, row_blocks, (a.T + GN - 1) / GN, &kps);
@@ -851,15 +854,16 @@ int gemm_split_count(const GemmArgs &a) {
 int gemm_kquant(const GemmArgs &a, hipStream_t stream) {
     if (!a.X || a.M <= 0 || a.K <= 0 || a.T <= 0) return fail(MESH_ERR_INVALID, "gemm: null pointer or empty shape");
     if (a.y16_k8 || a.n_seg > 1) {
-        if (!a.Wp || (a.y16_k8 && (a.n_seg > 1 || a.bias || a.residual)) || a.n_seg > 3)
+        if ((!a.Wp && !gemm_tile_takes(a)) || (a.y16_k8 && (a.n_seg > 1 || a.bias || a.residual)) || a.n_seg > 3)
             return fail(MESH_ERR_INVALID, "gemm: multi-matrix and SwiGLU launches need the GEMM layout (and no bias / residual for SwiGLU)");
         for (int i = 0; i < a.n_seg && !a.y16_k8; ++i)
             if (!a.seg_Y[i] || a.seg_M[i] <= 0 || a.seg_M[i] % 4 || a.seg_ldy[i] % 4 || (i + 1 < a.n_seg && a.seg_M[i] % GM) || (a.residual))
                 return fail(MESH_ERR_INVALID, "gemm: bad matrix %d of a multi-matrix launch", i);
-    } else if (!a.W || !a.Y) return fail(MESH_ERR_INVALID, "gemm: null pointer");
+    } else if ((!a.W && !gemm_tile_takes(a)) || !a.Y) return fail(MESH_ERR_INVALID, "gemm: null pointer");
     if (a.K % QK_K || a.M % 4 || a.ldx % 8 || a.ldy % 4 || (a.residual && a.ldres % 4))
         return fail(MESH_ERR_INVALID, "gemm: shape M=%d K=%d not supported (K %% 256, M %% 4)", a.M, a.K);
     if ((reinterpret_cast<uintptr_t>(a.X) | reinterpret_cast<uintptr_t>(a.Y)) & 15) return fail(MESH_ERR_INVALID, "gemm: X and Y must be 16-byte aligned");
+    if (gemm_tile_takes(a)) return gemm_tile(a, stream);
     GemmArgs k = a;
     k.M_pad = (a.M + TILE_ROWS - 1) / TILE_ROWS * TILE_ROWS;
     const int row_blocks = a.y16_k8 ? (a.M + GM / 2 - 1) / (GM / 2) : (a.M + GM - 1) / GM;
@@ -939,6 +943,34 @@ int gemm_pack(int type, const void *tiled, void *packed, int64_t M, int64_t K, h
     if (grid.y > 65535u) return fail(MESH_ERR_UNSUPPORTED, "gemm_pack: %lld rows are too many", (long long)M);
     if (type == MESH_Q4_K) MESH_LAUNCH(gemm_pack_kernel<MESH_Q4_K>, grid, dim3(256), 0, stream, static_cast<const uint8_t *>(tiled), nullptr, static_cast<uint8_t *>(packed), M_pad, nsb);
     else MESH_LAUNCH(gemm_pack_kernel<MESH_Q6_K>, grid, dim3(256), 0, stream, static_cast<const uint8_t *>(tiled), nullptr, static_cast<uint8_t *>(packed), M_pad, nsb);
+    MESH_LAUNCH_CHECK();
+    return MESH_OK;
+}
+
+// one workgroup per chunk: thread s forms its (row, sub-block) as the staging thread of the GEMM does
+template <int TYPE>
+__global__ __launch_bounds__(256) void gemm_tile_copy_kernel(const uint8_t *__restrict__ packed, _Float16 *__restrict__ tile, int pair) {
+    const int kc = blockIdx.x, mb = blockIdx.y, n_steps = gridDim.x, s = threadIdx.x, h = s & 1;
+    int r = s >> 1;
+    PackedSub<TYPE> sub;
+    sub.load(packed + ((size_t)mb * n_steps + kc) * PackedSub<TYPE>::CHUNK, s);
+    __align__(16) _Float16 v[32];
+    sub.store(v);
+    if (pair) r = (r & 32) * 2 + (r >> 6) * 32 + (r & 31);
+    _Float16 *dst = tile + (size_t)(mb * 8 + (r >> 4)) * 16 * n_steps * GK + ((size_t)(kc * 8 + h * 4) * 16 + (r & 15)) * 8;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) *reinterpret_cast<uint4 *>(dst + j * 128) = reinterpret_cast<const uint4 *>(v)[j];
+}
+
+size_t gemm_tile_bytes(int64_t M, int64_t K) { return (size_t)((M + GM - 1) / GM) * GM * (size_t)K * 2; }
+size_t gemm_tile_pair_bytes(int64_t M, int64_t K) { return (size_t)((M + GM / 2 - 1) / (GM / 2)) * GM * (size_t)K * 2; }
+
+int gemm_tile_copy(int type, const void *packed, void *tile, int64_t M, int64_t K, bool pair, hipStream_t stream) {
+    if (!packed || !tile || gemm_packed_bytes(type, M, K) == 0) return fail(MESH_ERR_INVALID, "gemm_tile_copy: bad arguments (type %d, M %lld, K %lld)", type, (long long)M, (long long)K);
+    const int rows = pair ? GM / 2 : GM;
+    const dim3 grid((unsigned)(K / GK), (unsigned)((M + rows - 1) / rows));
+    if (type == MESH_Q4_K) MESH_LAUNCH(gemm_tile_copy_kernel<MESH_Q4_K>, grid, dim3(256), 0, stream, static_cast<const uint8_t *>(packed), static_cast<_Float16 *>(tile), pair ? 1 : 0);
+    else MESH_LAUNCH(gemm_tile_copy_kernel<MESH_Q6_K>, grid, dim3(256), 0, stream, static_cast<const uint8_t *>(packed), static_cast<_Float16 *>(tile), pair ? 1 : 0);
     MESH_LAUNCH_CHECK();
     return MESH_OK;
 }

@@ -10,6 +10,8 @@ constexpr int SKINNY_ITEM_PAIRS = 16;      // pairs per work item of an expert l
 struct GemmArgs {
     const void *W = nullptr;         // tiled q4_K / q6_K matrix [M][K]
     const void *Wp = nullptr;        // optional: the same matrix in the GEMM layout (gemm_pack); used instead of W when set
+    const void *Wt = nullptr;        // optional: the same weights as f16 in the large tile's layout (gemm_tile_copy); used for calls of tile_min_tokens
+    int tile_min_tokens = 1 << 30;   // tokens with k8-major activations.  n_seg matrices: one copy of them back to back, of any types.
     int type = -1;
     int M = 0, K = 0, T = 0;
     int M_pad = 0;                   // filled in by gemm_kquant
@@ -76,6 +78,18 @@ int gemm_pack(int type, const void *tiled, void *packed, int64_t M, int64_t K, h
 // gate / up pair for the SwiGLU launch: row block b = gate rows [64b, 64b + 64) followed by up rows [64b, 64b + 64)
 size_t gemm_packed_pair_bytes(int type, int64_t M, int64_t K);
 int gemm_pack_pair(int type, const void *gate_tiled, const void *up_tiled, void *packed, int64_t M, int64_t K, hipStream_t stream);
+
+// f16 copy of a GEMM-layout matrix for the large tile (gemm_tile.hpp: GT_BLOCKS), rows padded to 128: the very weights the GEMM
+// forms from its layout, 2 bytes each.  A pair: per 128-row block 32 gate rows, their 32 up rows, the next 32 and 32, so that a wave
+// holds a gate row and its up row in the same lane.
+size_t gemm_tile_bytes(int64_t M, int64_t K);
+size_t gemm_tile_pair_bytes(int64_t M, int64_t K);
+int gemm_tile_copy(int type, const void *packed, void *tile, int64_t M, int64_t K, bool pair, hipStream_t stream);
+// The launch itself (gemm_kquant calls it): whether `a` takes it, its slices along K, and the product.
+bool gemm_tile_takes(const GemmArgs &a);
+int gemm_tile_slices(const GemmArgs &a);
+int gemm_tile(const GemmArgs &a, hipStream_t stream);
+int gemm_add_slices(const GemmArgs &a, int row_blocks, hipStream_t stream);
 
 // Skinny GEMM for a batch of decode steps (gemm_skinny.hip): up to three tiled K-quant matrices sharing the
 // activations, any T (processed 16 columns at a time), epilogues as in the mat-vec kernel, integer dot products on

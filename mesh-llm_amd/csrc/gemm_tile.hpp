@@ -2,15 +2,17 @@
 //
 // A workgroup of WM x WT waves owns a tile of 64 WM weight rows x 64 WT tokens, a wave 64 x 64 of it (2 x 2 blocks of
 // v_mfma_f32_32x32x16).  K goes by in steps of 32: a step's operands are (WM + WT) * 4 chunks of 1 KB, one per 16 rows, and
-// a chunk is one global_load_lds_dwordx4 of a wave.  Three stages of LDS: while step k is multiplied step k + 1 has
-// been requested and step k + 2 is being requested, so a wave waits with the loads of one step still in flight (vmcnt(PER),
-// exact because every wave issues the same number of loads per step) and one barrier per step serves both ways: behind it the step has
-// landed for everybody, and everybody is done with the stage that the next loads overwrite.
+// a chunk is one global_load_lds_dwordx4 of a wave.  LDS holds STAGES steps: while step k is multiplied the ones behind it have
+// been requested, so a wave waits with the loads of STAGES - 2 steps still in flight (vmcnt, exact because every wave
+// issues the same number of loads per step) and one barrier per step serves both ways: behind it the step has landed for
+// everybody, and everybody is done with the stage that the next loads overwrite.
 //
-// What bounds it: the clock.  256 x 128 tiles reach 1110-1250 TFLOP/s (M 28672, K 4096 and M 4096, K 14336, 2048 tokens), at
-// which the chip lowers its clock; 128 of those tiles alone run at 82% of the matrix cores' nominal rate, 256 at 50%.
-// 64 x 64 per wave measured against 128 x 64 per wave (half the waves): 436 against 502 us for M 28672, K 4096; steps of 64 with
-// two stages 604, with three 466; four stages of 32 462; s_setprio around the products 432 against 436-496.
+// What bounds it: with every CU at work the clock (M 4096, K 14336, 2048 tokens: 1100-1250 TFLOP/s; half the CUs alone reach
+// 82% of the matrix cores' nominal rate, all of them 50%), with few workgroups the latency of weights that come from
+// memory.  Measured, weights cold, us (M, K, tokens): 64 x 64 per wave 436 against 502 with 128 x 64 (28672, 4096, 2048, weights
+// warm); steps of 64 in two stages 604; s_setprio around the products 432 against 436-496.  Stages of the 128 x 128 tile, 3 / 5 / 8:
+// 48 / 39 / 40 (6144, 4096, 512), 154 / 121 / 121 (4096, 14336, 512); of 256 x 128, 3 / 4 / 6: 224 / 206 / 203 (4096, 14336, 2048),
+// 35 / 37 / 41 (8192, 2048, 900).
 //
 // The loads are issued by inline asm because the compiler counts LDS writes of the builtin as conflicting with the
 // fragment reads of the other stages across the loop's back edge and waits for all of them.  The asm has no outputs; its
@@ -42,20 +44,20 @@ __device__ __forceinline__ gt_f16v gt_mma(gt_b8 a, gt_b8 b, gt_f16v c) { return 
 enum GtLayout { GT_BLOCKS = 0, GT_ROWS = 1 };
 
 constexpr int GT_K = 32;                       // elements of K per step
-constexpr int GT_STAGES = 3;
-constexpr int gt_lds_bytes(int WM, int WT) { return GT_STAGES * (WM + WT) * 4096; }
+constexpr int gt_stages(int WM, int WT) { return WM == 2 ? 5 : WT == 2 ? 4 : 3; }
+constexpr int gt_lds_bytes(int WM, int WT, int STAGES) { return STAGES * (WM + WT) * 4096; }
+constexpr int gt_lds_bytes(int WM, int WT) { return gt_lds_bytes(WM, WT, gt_stages(WM, WT)); }
 // waves per SIMD of the workgroups that a CU's 160 KB of LDS hold
 constexpr int gt_waves_per_simd(int WM, int WT) { return 160 * 1024 / gt_lds_bytes(WM, WT) * WM * WT / 4; }
 
-// Tile and split of a product.  Three tiles are built: 128 x 128 (weight rows x tokens), 256 x 128, 256 x 192.  A launch's time goes
-// as the rounds its workgroups make over the CUs times the tile's size times its share of K; the small tile reads more LDS
-// per product (1.2).  A slice costs writing and reading its result, and split_ns once where the reader is a launch of its own.
-// Measured, us (M, K, tokens):
-//   28672, 4096, 2048: 256x128 432, 128x128 500      28672, 4096, 333: 256x192 88, 256x128 106, 128x128 105
-//   6144, 4096, 2048:  128x128 94, 256x128 98        4096, 14336, 333: 256x128 in 4 slices 46, 128x128 in 2 57, whole 99
-//   2048, 8192, 900:   128x128 in 2 slices 37, in 4 38, whole 55; 256x128 in 4 41        4096, 4096, 333: in 2 slices 19, whole 29
+// Tile and split of a product.  Four tiles are built; a launch's time goes as the rounds its workgroups make over the CUs times a
+// round's time per element of K, which grows with the share of the chip at work (the clock).  A slice costs writing and
+// reading its result, and split_ns once where the reader is a launch of its own.  Measured with cold weights, us (M, K, tokens):
+//   28672, 4096, 2048: 256x256 419, 256x192 431, 256x128 451, 128x128 479     28672, 4096, 512: 111, 154, 121, 139
+//   28672, 4096, 256:  88, 85, 74, 79        6144, 4096, 2048: 100, 140, 110, 108        6144, 4096, 512: 72, 62, 55, 39
+//   4096, 4096, 2048:  84, 71, 68, 76        4096, 4096, 512: 71, 61, 54, 38             2048, 8192, 900: 129, 119, 88, 53
 struct GtPlan {
-    int wm = 2, wt = 2, slices = 1, k_slice = 0;       // waves (of 64 rows) by waves (of 64 tokens); steps of a slice
+    int wm = 2, wt = 2, slices = 1, k_slice = 0;       // waves (of 64 rows) by waves (of 64 tokens), one of the tiles below; steps of a slice
 };
 inline int gt_n_cu() {
     static const int n = [] {
@@ -67,15 +69,17 @@ inline int gt_n_cu() {
 }
 // slices_max, slices_room: the most slices the caller takes, and has room for
 inline GtPlan gt_plan(int M, int T, int K, int slices_max, size_t slices_room, double split_ns, int n_cu = gt_n_cu()) {
-    static constexpr struct { int wm, wt; double ns; } tiles[3] = {{4, 2, 11.4}, {2, 2, 6.8}, {4, 3, 17.0}};      // ns: one round's time per element of K
+    // one round's time per element of K: a few workgroups, and what a full chip adds
+    static constexpr struct { int wm, wt; double few, full; } tiles[4] = {{2, 2, 9.2, 0.3}, {4, 2, 13.0, 3.5}, {4, 3, 14.0, 7.0}, {4, 4, 15.5, 10.5}};
     GtPlan best;
     double least = 0;
     const int steps = K / GT_K;
     for (const auto &t : tiles)
-        for (int s = 1; s <= slices_max && (size_t)s <= slices_room && (s == 1 || K / s >= 256); s *= 2) {
+        for (int s = 1; s <= slices_max && (s == 1 || ((size_t)s <= slices_room && K / s >= 256)); s *= 2) {
             const long n = (long)((M + 64 * t.wm - 1) / (64 * t.wm)) * ((T + 64 * t.wt - 1) / (64 * t.wt)) * s;
             const int k_slice = (steps + s - 1) / s;
-            const double cost = (double)((n + n_cu - 1) / n_cu) * t.ns * k_slice * GT_K + (s > 1 ? s * (double)T * M * 0.00145 + split_ns : 0.0);
+            const double ns = t.few + t.full * (n < n_cu ? (double)n / n_cu : 1.0);
+            const double cost = (double)((n + n_cu - 1) / n_cu) * ns * k_slice * GT_K + (s > 1 ? s * (double)T * M * 0.00145 + split_ns : 0.0);
             if (least != 0 && cost >= least) continue;
             least = cost;
             best.wm = t.wm; best.wt = t.wt; best.k_slice = k_slice;
@@ -87,7 +91,7 @@ inline GtPlan gt_plan(int M, int T, int K, int slices_max, size_t slices_room, d
 // acc += W x over steps [k0, k0 + n_steps), n_steps >= 1.  w, x: 16-bit elements, rows of ldw and ldx (GT_BLOCKS: both K); w_block, x_block: first 16-row block of the
 // tile; w_blocks: blocks the matrix holds; x_rows: rows x holds (GT_BLOCKS: up to a whole block).  Blocks and rows past the end
 // repeat the last one; what they multiply is never stored.  SWAP: result rows = tokens, columns (lanes) = weight rows.
-template <class V, GtLayout LW, GtLayout LX, int WM, int WT, bool SWAP>
+template <class V, GtLayout LW, GtLayout LX, int WM, int WT, bool SWAP, int STAGES = gt_stages(WM, WT)>
 __device__ __forceinline__ void gt_multiply(char *smem, gt_f16v (&acc)[2][2], const void *w, int ldw, const void *x, int ldx, int k0, int n_steps, int w_block, int w_blocks,
                                             int x_block, int x_rows) {
     constexpr int WAVES = WM * WT, CHUNKS = (WM + WT) * 4, PER = (CHUNKS + WAVES - 1) / WAVES, STAGE = CHUNKS * 1024;
@@ -165,19 +169,29 @@ __device__ __forceinline__ void gt_multiply(char *smem, gt_f16v (&acc)[2][2], co
         }
         __builtin_amdgcn_s_setprio(0);
     };
-    load(0, 0);
-    load(1, 1);
-    int k = 0;
-    for (; k + GT_STAGES <= n_steps; k += GT_STAGES) {
 #pragma unroll
-        for (int i = 0; i < GT_STAGES; ++i) {
-            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(PER) : "memory");
-            step(i, std::true_type{}, (i + 2) % GT_STAGES, k + i + 2);
+    for (int i = 0; i < STAGES - 1; ++i) load(i, i);
+    int k = 0;
+    for (; k + STAGES <= n_steps; k += STAGES) {
+#pragma unroll
+        for (int i = 0; i < STAGES; ++i) {
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(PER * (STAGES - 2)) : "memory");
+            step(i, std::true_type{}, (i + STAGES - 1) % STAGES, k + i + STAGES - 1);
         }
     }
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (k < n_steps) step(0, std::false_type{}, 0, 0);
-    if (k + 1 < n_steps) step(1, std::false_type{}, 0, 0);
+#pragma unroll
+    for (int i = 0; i < STAGES - 1; ++i)
+        if (k + i < n_steps) step(i, std::false_type{}, 0, 0);
+}
+
+__device__ __forceinline__ void gt_clear(gt_f16v (&acc)[2][2]) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.f;
 }
 
 // 1-D grid of row tiles x token tiles: the workgroups a die is dealt (every eighth) take a contiguous run of tiles, the token tile

@@ -29,8 +29,8 @@ int hybrid_session_alloc(mesh_session *s) {
     h.xa = buf(B * (size_t)hm.width_pad * ab);
     h.acta = buf(B * (size_t)hm.act_max * std::max(ab, sizeof(float)));        // (the single-token step keeps f32 vectors in it)
     h.big = fbuf(B * (size_t)hm.in_max);
-    // room for the slices of a product that few tiles cover: as many tiles as there are CUs, and one result at least
-    h.y_floats = std::max(B * E, std::min(B * E * LINEAR_SLICES_MAX, (size_t)8 << 20));
+    // room for the slices of a product that few tiles cover (as many 128 x 128 tiles as there are CUs), and one result at least
+    h.y_floats = std::max(B * E, std::min(B * E * LINEAR_SLICES_MAX, (size_t)4 << 20));
     h.y = fbuf(h.y_floats);
     h.q = fbuf(B * (size_t)hm.q_max);
     h.part = fbuf(2 * 3 * STEP_PARTS_MAX);

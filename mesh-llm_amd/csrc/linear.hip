@@ -119,12 +119,7 @@ __global__ __launch_bounds__(64 * WM * WT, gt_waves_per_simd(WM, WT)) void linea
     gt_place(blockIdx.x, n_tiles, n_ttiles, mt, tt);
     const int n_all = K / GT_K, k0 = blockIdx.y * k_slice, n_steps = n_all - k0 < k_slice ? n_all - k0 : k_slice;
     gt_f16v acc[2][2];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.f;
+    gt_clear(acc);
     gt_multiply<gt_b8, LW, GT_ROWS, WM, WT, true>(smem, acc, w, K, x, K, k0, n_steps, mt * WM * 4, row_blocks * 8, tt * WT * 4, T);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int m0 = (mt * WM + wave % WM) * 64, t0 = (tt * WT + wave / WM) * 64;
@@ -176,7 +171,8 @@ static int launch_tile_layout(const uint16_t *w, const LinearWeight &W, const vo
     const int row_blocks = W.Mp / 128, mtiles = (M + 64 * p.wm - 1) / (64 * p.wm), ttiles = (T + 64 * p.wt - 1) / (64 * p.wt);
     const dim3 grid((unsigned)(mtiles * ttiles), (unsigned)p.slices), block((unsigned)(64 * p.wm * p.wt));
     const uint16_t *xb = static_cast<const uint16_t *>(x);
-    if (p.wt == 3) MESH_LAUNCH((linear_tile_kernel<OUT, LW, 4, 3>), grid, block, 0, stream, w, xb, y, W.Kp, M, T, ldy, row_blocks, ttiles, mtiles * ttiles, p.k_slice, stride);
+    if (p.wt == 4) MESH_LAUNCH((linear_tile_kernel<OUT, LW, 4, 4>), grid, block, 0, stream, w, xb, y, W.Kp, M, T, ldy, row_blocks, ttiles, mtiles * ttiles, p.k_slice, stride);
+    else if (p.wt == 3) MESH_LAUNCH((linear_tile_kernel<OUT, LW, 4, 3>), grid, block, 0, stream, w, xb, y, W.Kp, M, T, ldy, row_blocks, ttiles, mtiles * ttiles, p.k_slice, stride);
     else if (p.wm == 4) MESH_LAUNCH((linear_tile_kernel<OUT, LW, 4, 2>), grid, block, 0, stream, w, xb, y, W.Kp, M, T, ldy, row_blocks, ttiles, mtiles * ttiles, p.k_slice, stride);
     else MESH_LAUNCH((linear_tile_kernel<OUT, LW, 2, 2>), grid, block, 0, stream, w, xb, y, W.Kp, M, T, ldy, row_blocks, ttiles, mtiles * ttiles, p.k_slice, stride);
     MESH_LAUNCH_CHECK();

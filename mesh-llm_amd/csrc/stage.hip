@@ -207,6 +207,39 @@ struct Loader {
         }
         return MESH_OK;
     }
+    // f16 copies for the large tile of what the dense layers hold in the GEMM layout: their bytes, or (bytes null) the copies.  The
+    // attention projections of mixture-of-experts layers keep the GEMM layout alone: the copies took 2-3% off their chunks.
+    int tile_copies(size_t *bytes) {
+        int rc;
+        auto one = [&](void **dst, size_t n, auto fill) -> int {
+            if (bytes) { *bytes += n; return MESH_OK; }
+            void *p = nullptr;
+            if ((rc = dev_alloc(&p, n)) != MESH_OK || (rc = fill(static_cast<uint8_t *>(p))) != MESH_OK) return rc;
+            *dst = p;
+            return MESH_OK;
+        };
+        auto copy = [&](const DevTensor &t, uint8_t *p) { return gemm_tile_copy(t.type, t.gemm, p, t.M, t.K, false, nullptr); };
+        for (LayerWeights &L : st.layers) {
+            if (!L.gate_up_gemm) continue;
+            const DevTensor &q = L.wq, &k = L.wk, &v = L.wv;
+            if (q.gemm && k.gemm && v.gemm && q.K == k.K && q.K == v.K && q.M % 128 == 0 && k.M % 128 == 0) {
+                const size_t qb = gemm_tile_bytes(q.M, q.K), kb = gemm_tile_bytes(k.M, k.K);
+                if ((rc = one(&L.qkv_tile, qb + kb + gemm_tile_bytes(v.M, v.K), [&](uint8_t *p) -> int {
+                         int r;
+                         if ((r = copy(q, p)) != MESH_OK || (r = copy(k, p + qb)) != MESH_OK) return r;
+                         return copy(v, p + qb + kb);
+                     })) != MESH_OK)
+                    return rc;
+            }
+            for (DevTensor *t : {&L.wo, &L.w_down})
+                if (t->gemm && (rc = one(&t->tile, gemm_tile_bytes(t->M, t->K), [&](uint8_t *p) -> int { return copy(*t, p); })) != MESH_OK) return rc;
+            if ((rc = one(&L.gate_up_tile, gemm_tile_pair_bytes(L.w_gate.M, L.w_gate.K), [&](uint8_t *p) -> int {
+                    return gemm_tile_copy(L.w_gate.type, L.gate_up_gemm, p, L.w_gate.M, L.w_gate.K, true, nullptr);
+                })) != MESH_OK)
+                return rc;
+        }
+        return MESH_OK;
+    }
     // the expert matrices of a mixture-of-experts layer, for prefill chunks (expert launches of the large-tile GEMM): every
     // expert's gate / up pair and down projection in the GEMM layout, experts back to back
     int pack_experts(LayerWeights &L) {
@@ -355,6 +388,10 @@ int stage_open(const char *path, int layer_begin, int layer_end, const mesh_stag
             // tied embeddings: the output projection is token_embd
             if ((rc = ld.load("token_embd.weight", st->output, E, -1, 1, true, true, false)) != MESH_OK) return rc;
         }
+    }
+    if (ld.gemm_layout && st->tune.tile_copies && st->n_batch_max >= st->tune.tile_min_tokens) {
+        size_t bytes = 0;
+        if ((rc = ld.tile_copies(&bytes)) != MESH_OK || (stage_copies_fit(bytes) && (rc = ld.tile_copies(nullptr)) != MESH_OK)) return rc;
     }
     // inverse frequencies by ggml's f32 recurrence: theta_i = theta_{i-1} * base^(-2/n_rot)
     {
@@ -636,7 +673,7 @@ static bool layer_is_kquant_dense(const LayerWeights &L) {
 
 static GemmArgs gemm_of(const DevTensor &w, const uint16_t *x16, int ldx, int T, float *y, int ldy, const DevTensor *bias) {
     GemmArgs g;
-    g.W = w.data; g.Wp = w.gemm; g.type = w.type; g.M = (int)w.M; g.K = (int)w.K; g.T = T;
+    g.W = w.data; g.Wp = w.gemm; g.Wt = w.tile; g.type = w.type; g.M = (int)w.M; g.K = (int)w.K; g.T = T;
     g.X = reinterpret_cast<const _Float16 *>(x16); g.ldx = ldx; g.Y = y; g.ldy = ldy;
     g.bias = bias && bias->present() ? static_cast<const float *>(bias->data) : nullptr;
     return g;
@@ -659,7 +696,7 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
     // a mixture-of-experts stage keeps the integer kernel, whose activation layout its expert launches share
     const bool sk16 = skinny && s->tune.skinny_f16 && L.w_gate.present() && f16ffn;
     const bool sk8 = skinny && !sk16;
-    auto gemm_k8 = [&](GemmArgs g) { g.x_k8 = k8; g.part = s->tune.gemm_splitk ? s->gemm_part : nullptr; g.part_bytes = s->gemm_part_bytes; g.sat = s->f16_sat; g.big_tile = s->tune.gemm_big; g.narrow_tile = s->tune.gemm_narrow; return g; };
+    auto gemm_k8 = [&](GemmArgs g) { g.x_k8 = k8; g.part = s->tune.gemm_splitk ? s->gemm_part : nullptr; g.part_bytes = s->gemm_part_bytes; g.sat = s->f16_sat; g.big_tile = s->tune.gemm_big; g.tile_min_tokens = s->tune.tile_min_tokens; g.narrow_tile = s->tune.gemm_narrow; return g; };
     auto rope_of = [&]() {
         GemvRope r;
         r.pos = s->d_pos; r.seq = s->d_seq; r.inv_freq = st->rope_inv_freq;
@@ -725,12 +762,14 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
         if ((rc = gemm_skinny(qa, stream)) != MESH_OK) return rc;
     } else {
         ProfScope ps(s, MESH_PROF_GEMV);
-        if (L.qkv_fused >= 2 && s->tune.gemm_fused) {
-            // q, k (and v when it is of the same K-quant type) as one launch over their back-to-back GEMM-layout copies
+        const bool tile = L.qkv_tile && k8 && T >= s->tune.tile_min_tokens;
+        if ((tile || L.qkv_fused >= 2) && s->tune.gemm_fused) {
+            // q, k (and v when it is of the same K-quant type, or with the f16 copies) as one launch over their back-to-back copies
             const DevTensor *w[3] = {&L.wq, &L.wk, &L.wv}, *b[3] = {&L.bq, &L.bk, &L.bv};
             float *y[3] = {s->q, s->k, s->v};
             GemmArgs g = gemm_k8(gemm_of(L.wq, s->xn16, E, T, s->q, QD, nullptr));
-            g.n_seg = L.qkv_fused;
+            g.n_seg = tile ? 3 : L.qkv_fused;
+            g.Wt = L.qkv_tile;
             g.M = 0;
             for (int i = 0; i < g.n_seg; ++i) {
                 g.seg_begin[i] = g.M / 128;
@@ -742,7 +781,7 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
             // RoPE and the KV append ride in the second kernel of split launches (both launches must be split)
             if (s->tune.gemv_rope && hp.rope_mode == ROPE_MODE_NORM && st->k_type == MESH_F16 && st->v_type == MESH_F16 && !L.q_norm.present() &&
                 !L.k_norm.present() && hp.head_dim % 4 == 0 && hp.n_rot % 2 == 0 && gemm_split_count(g) > 1 &&
-                (L.qkv_fused == 3 || gemm_split_count(gv) > 1)) {
+                (g.n_seg == 3 || gemm_split_count(gv) > 1)) {
                 GemvRope r;
                 r.pos = s->d_pos; r.seq = s->d_seq; r.inv_freq = st->rope_inv_freq;
                 r.kcache = reinterpret_cast<uint16_t *>(s->kcache + il * s->k_layer_bytes);
@@ -754,7 +793,7 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
                 rope_fused = true;
             }
             if ((rc = gemm_kquant(g, stream)) != MESH_OK) return rc;
-            if (L.qkv_fused == 2 && (rc = gemm_kquant(gv, stream)) != MESH_OK) return rc;
+            if (g.n_seg == 2 && (rc = gemm_kquant(gv, stream)) != MESH_OK) return rc;
         } else {
         if ((rc = gemm_kquant(gemm_k8(gemm_of(L.wq, s->xn16, E, T, s->q, QD, &L.bq)), stream)) != MESH_OK) return rc;
         if ((rc = gemm_kquant(gemm_k8(gemm_of(L.wk, s->xn16, E, T, s->k, KD, &L.bk)), stream)) != MESH_OK) return rc;
@@ -900,6 +939,7 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
         ProfScope ps(s, MESH_PROF_GEMV);
         GemmArgs g = gemm_k8(gemm_of(L.w_gate, s->xn16, E, T, nullptr, FF, nullptr));
         g.Wp = L.gate_up_gemm;
+        g.Wt = L.gate_up_tile;
         g.y16_k8 = f16ffn;
         if ((rc = gemm_kquant(g, stream)) != MESH_OK) return rc;
     } else {

@@ -34,6 +34,7 @@ void hparams_from_spec(const ModelSpec &s, HParams &hp);
 struct DevTensor {
     void *data = nullptr;
     void *gemm = nullptr;   // K-quant projections of stages that can take prefill-sized calls: second copy in the GEMM layout (gemm.hpp)
+    void *tile = nullptr;   // ... and f16 copy for the large tile (gemm_tile.hpp)
     int type = -1;
     int64_t K = 0;       // row length (ggml ne[0])
     int64_t M = 0;       // rows (ggml ne[1]); for 1-D tensors M = 1
@@ -52,6 +53,8 @@ struct LayerWeights {
     // packed as a SwiGLU pair.
     int qkv_fused = 0;
     void *gate_up_gemm = nullptr;
+    // f16 copies for the large tile: q, k and v back to back whatever their types, gate / up as a pair (gemm.hpp: gemm_tile_copy)
+    void *qkv_tile = nullptr, *gate_up_tile = nullptr;
     // mixture of experts: every expert's gate / up pair and down projection in the GEMM layout, experts back to back
     void *exps_gate_up_gemm = nullptr, *exps_down_gemm = nullptr;
     size_t exps_gate_up_stride = 0, exps_down_stride = 0;

@@ -7,9 +7,11 @@ import numpy as np
 import pytest
 
 sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
+import models
 import nadosun_util as N
 from folder_util import error, open_stage, run
 from oracle.nadosun import NadosunOracle
+from oracle.stage import StageOracle
 from util import mesh
 
 pytestmark = pytest.mark.gpu
@@ -47,3 +49,38 @@ def test_products_of_many_tokens(tmp_path, width, ff, tokens):
     # the two add the same products of the same bf16 values in another order (1e-6); a result next to a rounding point of the next
     # product's bf16 input moves by 2^-8 of itself there: a small share of what the oracle's bound allows for all inputs
     assert error(got, rows) < BF16_LIMIT / 2, (width, ff, tokens, error(got, rows))
+
+
+def kquant(n_embd, n_head, n_kv, n_ff):
+    return dict(arch="llama", n_layer=1, n_embd=n_embd, n_head=n_head, n_head_kv=n_kv, head_dim=128, n_ff=n_ff, n_vocab=256, eps=1e-5, rope=1e4)
+
+
+@pytest.mark.parametrize("shape,tokens", [
+    ((512, 4, 1, 768), 129),        # matrices of one launch that end inside a tile of 256 rows; slices along K; a token past the tile
+    ((512, 4, 1, 768), 143),        # the last block of 16 tokens one short
+    ((256, 2, 1, 28672), 140),      # 256 x 192, most of it empty
+    ((256, 2, 1, 14336), 256),      # 256 x 128
+    ((256, 2, 1, 28672), 256),      # 256 x 256
+    ((1024, 8, 2, 2816), 385),      # down projection of 88 steps in slices; three query heads' worth of rows in the last tile
+])
+def test_kquant_products_of_many_tokens(tmp_path, shape, tokens):
+    """A chunk through one layer over f16 copies, against the oracle and against the GEMM that forms the same weights as it goes."""
+    m = mesh()
+    cfg = kquant(*shape)
+    path = str(tmp_path / "model.gguf")
+    tensors = models.write_model(path, cfg, [0], seed=7)
+    x = np.random.Generator(np.random.PCG64(tokens)).standard_normal((tokens, cfg["n_embd"])).astype(np.float32)
+    want = StageOracle(cfg, tensors, 0, 1, 512, blas=True).forward(x, np.arange(tokens))
+    got = {}
+    for copies in (0, 1):
+        st = m.Stage(path, 0, 1, n_ctx=512, n_batch_max=512, tuning={"tile_copies": copies})
+        ses = st.session()
+        got[copies] = ses.decode(x, np.arange(tokens)).view(np.float32).reshape(want.shape)
+        assert ses.f16_saturations() == 0
+        ses.close()
+        st.close()
+    norm = np.linalg.norm(want)
+    # f16 activations over one layer: 11 bits in the inputs of four products (the bound of the other f16 paths)
+    assert np.linalg.norm(got[1] - want) / norm < 3e-3, (shape, tokens)
+    # the same f16 weights and inputs summed in another order: what a rounding point of the next input next to a sum can move
+    assert np.linalg.norm(got[1] - got[0]) / norm < 1e-3, (shape, tokens)
