@@ -60,6 +60,14 @@ __device__ __forceinline__ half2v h2_splat(float v) {
     return half2v{h, h};
 }
 
+// eight nibbles (elements 0..3 in the bytes of lo, 4..7 in those of hi) in the GEMM layout's order: element e at nibble e / 2 + 4 (e % 2)
+__device__ __forceinline__ uint32_t pair_nibbles(uint32_t lo, uint32_t hi) {
+    uint32_t r = 0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) r |= (((e < 4 ? lo : hi) >> (8 * (e & 3))) & 0xFu) << (4 * (e >> 1) + 16 * (e & 1));
+    return r;
+}
+
 // Raw bytes of one (row, 32-element sub-block) of a tile: what a staging thread prefetches one k-step ahead.
 template <int TYPE> struct RawSub;
 
@@ -97,11 +105,11 @@ template <> struct RawSub<MESH_Q4_K> {
         const int sh = (c & 1) * 16 + h * 8;
         const half2v sc_c = q4k_sc_c(d, dmin, (scw >> sh) & 0xFFu, (mnw >> sh) & 0xFFu);
         const uint32_t w[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
-        uint32_t n[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) n[j] = ((w[2 * j] >> (4 * h)) & 0x0F0F0F0Fu) | (((w[2 * j + 1] >> (4 * h)) & 0x0F0F0F0Fu) << 4);
-        *reinterpret_cast<uint4 *>(chunk + s * 16) = make_uint4(n[0], n[1], n[2], n[3]);
-        *reinterpret_cast<uint2 *>(chunk + 4096 + s * 8) = make_uint2(__builtin_bit_cast(uint32_t, sc_c), hdr.x & 0xFFFFu);
+        for (int j = 0; j < 4; ++j)
+            *reinterpret_cast<uint32_t *>(chunk + (s - h + (j & 1)) * 16 + (2 * h + (j >> 1)) * 4) = pair_nibbles((w[2 * j] >> (4 * h)) & 0x0F0F0F0Fu, (w[2 * j + 1] >> (4 * h)) & 0x0F0F0F0Fu);
+        *reinterpret_cast<uint2 *>(chunk + 4096 + s * 8) =
+            make_uint2(__builtin_bit_cast(uint32_t, sc_c), (hdr.x & 0xFFFFu) | (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(-72.f * (float)sc_c[0])) << 16);
     }
 };
 
@@ -153,72 +161,97 @@ template <> struct RawSub<MESH_Q6_K> {
             const uint32_t nib = (t4 & 2) ? (lw[j] >> 4) & 0x0F0F0F0Fu : lw[j] & 0x0F0F0F0Fu;
             q[j] = nib | (((hw[j] >> (2 * t4)) & 0x03030303u) << 4);
         }
-        uint32_t n[4], hb2[2] = {0u, 0u};
+        uint32_t hb2[2] = {0u, 0u};
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            n[j] = (q[2 * j] & 0x0F0F0F0Fu) | ((q[2 * j + 1] & 0x0F0F0F0Fu) << 4);
-            hb2[j >> 1] |= (((q[2 * j] >> 4) & 0x03030303u) | (((q[2 * j + 1] >> 4) & 0x03030303u) << 2)) << (4 * (j & 1));
+            *reinterpret_cast<uint32_t *>(chunk + (s - h + (j & 1)) * 16 + (2 * h + (j >> 1)) * 4) = pair_nibbles(q[2 * j] & 0x0F0F0F0Fu, q[2 * j + 1] & 0x0F0F0F0Fu);
+            // element e of the eight: bits 2 P and up of the word's lower half (e even) or upper half, P = 4 (j / 2) + e / 2
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                hb2[j & 1] |= ((q[2 * j + (e >> 2)] >> (8 * (e & 3) + 4)) & 3u) << (2 * (4 * (j >> 1) + (e >> 1)) + 16 * (e & 1));
         }
-        *reinterpret_cast<uint4 *>(chunk + s * 16) = make_uint4(n[0], n[1], n[2], n[3]);
-        *reinterpret_cast<uint2 *>(chunk + 4096 + s * 8) = make_uint2(hb2[0], hb2[1]);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) *reinterpret_cast<uint32_t *>(chunk + 4096 + (s - h + j) * 8 + h * 4) = hb2[j];
         *reinterpret_cast<uint2 *>(chunk + 6144 + s * 8) = make_uint2(__builtin_bit_cast(uint32_t, s01), d & 0xFFFFu);
     }
 };
 
-// The same (row, sub-block) out of the GEMM layout: two or three loads at the thread's own slot of the chunk.
+// Half a row of a chunk out of the GEMM layout (gemm.hpp): slot s = 2 row + h holds elements 16 j + 8 h .. + 7, j = 0..3, of the
+// row's 64: what one lane of a v_mfma_f32_32x32x16_f16 fragment holds in each of four steps.
+// Eight weights of it are a dword of nibbles, element e at nibble e / 2 + 4 (e % 2): one shift puts a pair into bits 4..7 and
+// 20..23, where or-ing 0x5400 makes two f16 of exactly 64 + q (64 to 127: sixteenths in the lowest bits), and one packed fma with
+// the scale then takes the offset off: (64 + q) sc - (64 + off) sc is (q - off) sc, exactly or rounded once, as (q - off)
+// times sc is; 72 sc (off 8, sc <= 63) and 96 sc (off 32, |sc| <= 128) are f16.  15 instructions for 8 weights of q4_K, 23 of q6_K.
 template <int TYPE> struct PackedSub;
+__device__ __forceinline__ half2v fma2(uint32_t x, half2v b, half2v c) { return __builtin_elementwise_fma(__builtin_bit_cast(half2v, x), b, c); }
+// (x & mask) | y in one instruction: it takes one constant from scalar registers, so the other has to be held in a vector register
+__device__ __forceinline__ uint32_t and_or(uint32_t x, uint32_t mask, uint32_t y) {
+    uint32_t r;
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "s"(mask), "v"(y));
+    return r;
+}
+__device__ __forceinline__ uint32_t nibble_pair(uint32_t w, int p) { return and_or(p == 0 ? w << 4 : w >> (4 * (p - 1)), 0x00F000F0u, 0x54005400u); }
 template <> struct PackedSub<MESH_Q4_K> {
     static constexpr int CHUNK = 6144;
     uint4 q;
-    uint2 sm;          // {f16 sc, f16 c}, {f16 d, -}
-    __device__ __forceinline__ void load(const uint8_t *__restrict__ chunk, int s) {
+    uint4 sm;          // per 32 elements: {f16 sc, f16 c}, {f16 d, f16 -72 sc}
+    __device__ __forceinline__ void load(const uint8_t *__restrict__ chunk, unsigned s) {
         q = *reinterpret_cast<const uint4 *>(chunk + s * 16);
-        sm = *reinterpret_cast<const uint2 *>(chunk + 4096 + s * 8);
+        sm = *reinterpret_cast<const uint4 *>(chunk + 4096 + (s >> 1) * 16);
     }
-    __device__ __forceinline__ void store(_Float16 *dst) const {
-        const half2v sc = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(sm.x, sm.x, 0x01000100u));
-        const half2v cc = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(sm.x, sm.x, 0x03020302u));
-        const half2v dd = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(sm.y, sm.y, 0x01000100u));
-        const half2v off = {(_Float16)1032.f, (_Float16)1032.f};
-        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-        uint4 *d4 = reinterpret_cast<uint4 *>(dst);
+    // the eight weights of step j (known at compile time)
+    __device__ __forceinline__ uint4 form(int j) const {
+        const uint32_t a = j < 2 ? sm.x : sm.z, b = j < 2 ? sm.y : sm.w;
+        const half2v sc = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(a, a, 0x01000100u)), cc = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(a, a, 0x03020302u));
+        const half2v dd = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(b, b, 0x01000100u)), off = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(b, b, 0x03020302u));
+        const uint32_t w = j == 0 ? q.x : j == 1 ? q.y : j == 2 ? q.z : q.w;
+        uint32_t o[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            uint4 o;
-            dequant4(w[j] & 0x0F0F0F0Fu, off, sc, dd, cc, o.x, o.y);
-            dequant4((w[j] >> 4) & 0x0F0F0F0Fu, off, sc, dd, cc, o.z, o.w);
-            d4[j] = o;
-        }
+        for (int p = 0; p < 4; ++p) o[p] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(fma2(nibble_pair(w, p), sc, off), dd, cc));
+        return make_uint4(o[0], o[1], o[2], o[3]);
     }
 };
 template <> struct PackedSub<MESH_Q6_K> {
     static constexpr int CHUNK = 8192;
     uint4 q;
     uint2 hb;
-    uint2 sc;          // {f16 sc of elements 0..15, f16 sc of elements 16..31}, {f16 d, -}
-    __device__ __forceinline__ void load(const uint8_t *__restrict__ chunk, int s) {
+    uint4 sc;          // f16 sc of elements 0..15, of 16..31, f16 d, -, f16 sc of elements 32..47, of 48..63, f16 d, -
+    __device__ __forceinline__ void load(const uint8_t *__restrict__ chunk, unsigned s) {
         q = *reinterpret_cast<const uint4 *>(chunk + s * 16);
         hb = *reinterpret_cast<const uint2 *>(chunk + 4096 + s * 8);
-        sc = *reinterpret_cast<const uint2 *>(chunk + 6144 + s * 8);
+        sc = *reinterpret_cast<const uint4 *>(chunk + 6144 + (s >> 1) * 16);
     }
-    __device__ __forceinline__ void store(_Float16 *dst) const {
-        const half2v s0 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(sc.x, sc.x, 0x01000100u));
-        const half2v s1 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(sc.x, sc.x, 0x03020302u));
-        const half2v dd = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(sc.y, sc.y, 0x01000100u));
-        const half2v off = {(_Float16)1056.f, (_Float16)1056.f}, zero = {(_Float16)0.f, (_Float16)0.f};
-        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-        uint4 *d4 = reinterpret_cast<uint4 *>(dst);
+    __device__ __forceinline__ uint4 form(int j) const {
+        const half2v s = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(j < 2 ? sc.x : sc.z, j < 2 ? sc.x : sc.z, j & 1 ? 0x03020302u : 0x01000100u));
+        const half2v off = s * half2v{(_Float16)-96.f, (_Float16)-96.f};
+        const half2v dd = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(sc.y, sc.y, 0x01000100u)), zero = {(_Float16)0.f, (_Float16)0.f};
+        const uint32_t w = j == 0 ? q.x : j == 1 ? q.y : j == 2 ? q.z : q.w, hw = j < 2 ? hb.x : hb.y;
+        uint32_t o[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t hs = (j < 2 ? hb.x : hb.y) >> (4 * (j & 1));
-            const half2v s = j < 2 ? s0 : s1;
-            uint4 o;
-            dequant4((w[j] & 0x0F0F0F0Fu) | ((hs & 0x03030303u) << 4), off, s, dd, zero, o.x, o.y);
-            dequant4(((w[j] >> 4) & 0x0F0F0F0Fu) | (((hs >> 2) & 0x03030303u) << 4), off, s, dd, zero, o.z, o.w);
-            d4[j] = o;
+        for (int p = 0; p < 4; ++p) {
+            const int at = 2 * (4 * (j & 1) + p);
+            const uint32_t x = and_or(at < 8 ? hw << (8 - at) : hw >> (at - 8), 0x03000300u, nibble_pair(w, p));
+            o[p] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(fma2(x, s, off), dd, zero));
         }
+        return make_uint4(o[0], o[1], o[2], o[3]);
     }
 };
+// ... to its places in a row of the weight slab, dst being the row's element 8 h
+template <int TYPE>
+__device__ __forceinline__ void store_sub(const PackedSub<TYPE> &w, _Float16 *dst) {
+    uint4 *d4 = reinterpret_cast<uint4 *>(dst);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) d4[2 * j] = w.form(j);
+}
+
+// Workgroup barrier that orders LDS only.  __syncthreads() also waits for every outstanding global load, i.e. at the end
+// of each k-step for the activation fragments requested a moment ago for the NEXT step -- with one matrix-core wave per
+// SIMD nothing else would run during that wait.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 
 // Role split: waves 0-3 only multiply (each a 64 x 64 corner of the tile out of LDS stage kc & 1), waves 4-7 only
 // stage (fetch the raw weight bytes and activations of step kc + 2, dequantise step kc + 1 into the other LDS
@@ -230,26 +263,16 @@ template <> struct PackedSub<MESH_Q6_K> {
 // 16 k is four contiguous 256-byte pieces of that layout, so each lane fetches its 16 bytes straight from memory (L2),
 // four k16 steps ahead, into a ring of registers.  That halves the LDS reads per MFMA and leaves the staging waves only
 // the weights.
-// GROUPED: an expert launch (gemm.hpp): the workgroup's token tile and matrix come from a.tiles[blockIdx.y].
-template <int TYPE, bool PACKED, bool XDIRECT, bool SPLIT, bool NARROW, bool GROUPED = false>
+template <int TYPE, bool PACKED, bool XDIRECT, bool SPLIT, bool NARROW>
 __global__ __launch_bounds__(GEMM_THREADS) void gemm_kq_kernel(GemmArgs a) {
-    static_assert(!GROUPED || (PACKED && XDIRECT && !SPLIT && !NARROW), "expert launches: GEMM layout, k8-major activations, one k range");
     extern __shared__ __align__(16) _Float16 gemm_smem[];
     _Float16 *Ws = gemm_smem;                                  // [2][GM][LDS_LD]
     _Float16 *Xs = gemm_smem + 2 * GM * LDS_LD;                // [2][GN][LDS_LD]
     constexpr int TB = TYPE == MESH_Q4_K ? Q4K_TILE_BYTES : Q6K_TILE_BYTES;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // token tile [t0, t_end) of this workgroup and its matrix
-    int t0 = blockIdx.y * GN, t_end = a.T;
+    const int t0 = blockIdx.y * GN, t_end = a.T;
     const uint8_t *Wp = static_cast<const uint8_t *>(a.Wp);
-    if constexpr (GROUPED) {
-        if ((int)blockIdx.y >= *a.n_tiles) return;
-        const int4 tl = reinterpret_cast<const int4 *>(a.tiles)[blockIdx.y];
-        Wp += (size_t)tl.x * a.expert_stride;
-        t0 = tl.y;
-        t_end = tl.y + tl.z;
-    }
     const int m0 = blockIdx.x * GM;
     const int nsb = a.K / QK_K, n_all = a.K / GK;
     // k-steps [k0, k0 + n_steps) of this workgroup: all of them, or slice blockIdx.z of a split launch
@@ -281,9 +304,9 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_kq_kernel(GemmArgs a) {
             }
         };
         auto stage = [&](int kc, int buf, const Sub &w, const uint4 (&x)[4]) {
-            _Float16 *wdst = Ws + (buf * GM + srow) * LDS_LD + 32 * sh;
+            _Float16 *wdst = Ws + (buf * GM + srow) * LDS_LD + (PACKED ? 8 : 32) * sh;
             if constexpr (PACKED) {
-                w.store(wdst);
+                store_sub(w, wdst);
             } else if (wlive) {
                 w.store((k0 + kc) & 3, sh, wdst);
             } else {
@@ -489,6 +512,129 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_kq_kernel(GemmArgs a) {
         }
 }
 
+// ---- expert launches ------------------------------------------------------------------------------------------------------
+// 128 weight rows x the pairs of one tile of the list (1 to 128 of one expert) per workgroup of four waves.  A wave owns 32 rows
+// and all pairs: a lane of the multiplied fragment holds one row, and the GEMM layout's slot (row, half of a chunk) is
+// that lane's, so it forms the fragments of four MFMA steps from its own 32 or 40 bytes, in registers.  The activations go through LDS, k8-major as they lie in memory: 16-byte pieces at consecutive
+// addresses both ways.  NT groups of 32 pairs: an expert's remainder costs the groups it fills.
+// Bound by forming the weights (72 vector instructions per 2048 of them and wave) next to multiplying them, and by how evenly the
+// tiles fill the chip.  Gate / up of 64 experts of 2 x 768 rows x 2048 (q4_K), 4800 pairs of a Zipf router (86 tiles, 44 of at most
+// 32 pairs): 98 us with the staging waves of gemm_kq_kernel on tiles of 128 columns, 80 with fragments formed in registers, 70 with
+// the larger tiles first (moe_sort) and and_or; down projection of 2048 x 768: 53 -> 40 (q4_K), 56 -> 46 (q6_K).  113 MB of weights
+// at the rate of a large copy: 22 us.
+// Rows of a SwiGLU pair are dealt out so that a wave holds 16 gate rows and the 16 up rows of the same outputs, in one lane's
+// registers e and e + 8.
+constexpr int EXPERT_THREADS = 256;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+template <int TYPE, int NT>
+__device__ __forceinline__ void expert_tile(const GemmArgs &a, const uint8_t *wp, int bx, int t0, int t_end, u32x4 *xs) {
+    constexpr int AHEAD = 4, STEP = NT * 256;                  // chunks of weights on their way; 16-byte pieces of a chunk's activations
+    const int tid = threadIdx.x, lane = tid & 63, hh = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n_steps = a.K / GK;
+    const bool pair = a.y16_k8 != nullptr;
+    const int r = lane & 31;
+    const unsigned slot = 2 * (pair ? 16 * wave + (r & 15) + (r >> 4) * 64 : 32 * wave + r) + hh;
+    wp += (size_t)bx * n_steps * PackedSub<TYPE>::CHUNK;
+    const int n_blk = (a.T + 15) >> 4;
+    const u32x4 *const xbase = reinterpret_cast<const u32x4 *>(a.X + (size_t)(t0 >> 4) * 16 * a.K);
+    unsigned xo[NT];                                           // 16-byte pieces from the tile's first block
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+        const int b = 2 * i + (tid >> 7), last = n_blk - 1 - (t0 >> 4);        // (blocks past the list re-read the last one, never stored)
+        xo[i] = (unsigned)(b < last ? b : last) * (unsigned)(2 * a.K) + (unsigned)(tid & 127);
+    }
+    float16v acc[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[j][e] = 0.f;
+    PackedSub<TYPE> rw[AHEAD];
+    u32x4 rx[NT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i) rx[i] = xbase[xo[i]];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) rw[u].load(wp + (size_t)u * PackedSub<TYPE>::CHUNK, slot);       // (K is a multiple of 256)
+#pragma unroll
+    for (int i = 0; i < NT; ++i) xs[(0) * STEP + i * 256 + tid] = rx[i];
+#pragma unroll
+    for (int i = 0; i < NT; ++i) rx[i] = (xbase + 128)[xo[i]];
+    lds_barrier();
+    const int at = (lane & 15) + ((lane >> 4) & 1) * 128 + hh * 16;
+    for (int kc0 = 0; kc0 < n_steps; kc0 += AHEAD) {
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+            const int kc = kc0 + u;
+            // (the other buffer was read a step ago; the step's barrier hands it over)
+#pragma unroll
+            for (int i = 0; i < NT; ++i) xs[((u + 1) & 1) * STEP + i * 256 + tid] = rx[i];
+#pragma unroll
+            for (int i = 0; i < NT; ++i) rx[i] = (xbase + (size_t)(kc + 2 < n_steps ? kc + 2 : n_steps - 1) * 128)[xo[i]];
+            const u32x4 *x = xs + (u & 1) * STEP + at;
+            u32x4 f[2][NT];
+#pragma unroll
+            for (int j = 0; j < NT; ++j) f[0][j] = x[j * 256];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int st = 0; st < 4; ++st) {
+                if (st < 3)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j) f[(st + 1) & 1][j] = x[j * 256 + (st + 1) * 32];
+                const half8 w = __builtin_bit_cast(half8, rw[u].form(st));
+#pragma unroll
+                for (int j = 0; j < NT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w, __builtin_bit_cast(half8, f[st & 1][j]), acc[j], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            rw[u].load(wp + (size_t)(kc + AHEAD < n_steps ? kc + AHEAD : n_steps - 1) * PackedSub<TYPE>::CHUNK, slot);
+            lds_barrier();
+        }
+    }
+    const int t_pad = (t_end + 15) & ~15;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const int t = t0 + 32 * j + r;
+        if (t >= (pair ? t_pad : t_end)) continue;
+        if (pair) {
+#pragma unroll
+            for (int e4 = 0; e4 < 2; ++e4) {
+                const int m = bx * (GM / 2) + 16 * wave + 8 * e4 + 4 * hh;
+                if (m >= a.M) continue;
+                float o[4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const float g = acc[j][4 * e4 + c], up = acc[j][8 + 4 * e4 + c];
+                    o[c] = t < t_end ? g / (1.0f + expf(-g)) * up : 0.f;       // padding columns of the last token block hold zeros
+                }
+                note_f16_clamp(a.sat, o[0], o[1], o[2], o[3]);
+                *reinterpret_cast<uint2 *>(a.y16_k8 + (size_t)(t >> 4) * 16 * a.M + ((size_t)(m >> 3) * 16 + (t & 15)) * 8 + (m & 7)) =
+                    make_uint2(pack_h2(o[0], o[1]), pack_h2(o[2], o[3]));
+            }
+        } else {
+#pragma unroll
+            for (int e4 = 0; e4 < 4; ++e4) {
+                const int m = bx * GM + 32 * wave + 8 * e4 + 4 * hh;
+                if (m >= a.M) continue;
+                *reinterpret_cast<float4 *>(a.Y + (size_t)t * a.ldy + m) = make_float4(acc[j][4 * e4], acc[j][4 * e4 + 1], acc[j][4 * e4 + 2], acc[j][4 * e4 + 3]);
+            }
+        }
+    }
+}
+template <int TYPE>
+__global__ __launch_bounds__(EXPERT_THREADS, 2) void gemm_expert_kernel(GemmArgs a) {
+    __shared__ u32x4 xs[2 * 4 * 256];
+    // workgroups go to the eight XCDs in turn: every row block of a tile on one of them, whose L2 fetches the tile's activations once
+    const int g = (int)(blockIdx.y * gridDim.x + blockIdx.x), by = (g >> 3) / (int)gridDim.x * 8 + (g & 7), bx = (g >> 3) % (int)gridDim.x;
+    if (by >= *a.n_tiles) return;
+    const int4 tl = reinterpret_cast<const int4 *>(a.tiles)[by];
+    const uint8_t *wp = static_cast<const uint8_t *>(a.Wp) + (size_t)tl.x * a.expert_stride;
+    switch ((tl.z + 31) >> 5) {
+        case 1: return expert_tile<TYPE, 1>(a, wp, bx, tl.y, tl.y + tl.z, xs);
+        case 2: return expert_tile<TYPE, 2>(a, wp, bx, tl.y, tl.y + tl.z, xs);
+        case 3: return expert_tile<TYPE, 3>(a, wp, bx, tl.y, tl.y + tl.z, xs);
+        default: return expert_tile<TYPE, 4>(a, wp, bx, tl.y, tl.y + tl.z, xs);
+    }
+}
+
 // ---- the same product on a 256 x 128 workgroup tile ----------------------------------------------------------
 // What bounds the 128 x 128 kernel above is operand traffic, not the matrix cores: a wave that owns 64 x 64 of the tile
 // needs 1 KB of fragments per v_mfma_f32_32x32x16_f16 (2 x 2 register blocking: two weight fragments from LDS and two
@@ -502,14 +648,6 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_kq_kernel(GemmArgs a) {
 // a workgroup takes row blocks 2 * blockIdx.x and + 1, one per pair of matrix-core waves, so everything that depends on
 // the row block (matrix of a multi-matrix launch, SwiGLU pairing) is per wave.
 constexpr int BGM = 256;
-// Workgroup barrier that orders LDS only.  __syncthreads() also waits for every outstanding global load, i.e. at the end
-// of each k-step for the activation fragments requested a moment ago for the NEXT step -- with one matrix-core wave per
-// SIMD nothing else would run during that wait.
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
 template <int TYPE>
 __global__ __launch_bounds__(GEMM_THREADS) void gemm_big_kernel(GemmArgs a) {
     extern __shared__ __align__(16) _Float16 gemm_smem[];
@@ -525,15 +663,15 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_big_kernel(GemmArgs a) {
         const int st = tid - 256;
         const uint8_t *chunk0 = static_cast<const uint8_t *>(a.Wp) + (size_t)(2 * blockIdx.x) * n_steps * Sub::CHUNK;
         const uint8_t *chunk1 = chunk0 + (size_t)n_steps * Sub::CHUNK;
-        _Float16 *dst = Ws + (st >> 1) * LDS_LD + 32 * (st & 1);
+        _Float16 *dst = Ws + (st >> 1) * LDS_LD + 8 * (st & 1);
         Sub rw[2][2];
         auto fetch = [&](int kc, Sub (&w)[2]) {
             w[0].load(chunk0 + (size_t)kc * Sub::CHUNK, st);
             w[1].load(chunk1 + (size_t)kc * Sub::CHUNK, st);
         };
         auto stage = [&](int buf, const Sub (&w)[2]) {
-            w[0].store(dst + buf * BGM * LDS_LD);
-            w[1].store(dst + (buf * BGM + GM) * LDS_LD);
+            store_sub(w[0], dst + buf * BGM * LDS_LD);
+            store_sub(w[1], dst + (buf * BGM + GM) * LDS_LD);
         };
         fetch(0, rw[0]);
         fetch(n_steps > 1 ? 1 : 0, rw[1]);
@@ -794,16 +932,16 @@ int gemm_add_slices(const GemmArgs &k, int row_blocks, hipStream_t stream) {
     return MESH_OK;
 }
 
-template <int TYPE, bool PACKED, bool XDIRECT, bool SPLIT, bool NARROW, bool GROUPED = false>
+template <int TYPE, bool PACKED, bool XDIRECT, bool SPLIT, bool NARROW>
 static int launch_gemm_kernel(const GemmArgs &k, dim3 grid, hipStream_t stream) {
     // two stages of the weight slab, and of the activation slab unless the activations bypass LDS: 73 728 / 36 864 B
     constexpr size_t smem = sizeof(_Float16) * 2 * (GM + (XDIRECT ? 0 : GN)) * LDS_LD;
     static bool attr_set = false;
     if (!attr_set) {
-        MESH_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_kq_kernel<TYPE, PACKED, XDIRECT, SPLIT, NARROW, GROUPED>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+        MESH_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_kq_kernel<TYPE, PACKED, XDIRECT, SPLIT, NARROW>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
         attr_set = true;
     }
-    MESH_LAUNCH((gemm_kq_kernel<TYPE, PACKED, XDIRECT, SPLIT, NARROW, GROUPED>), grid, dim3(GEMM_THREADS), smem, stream, k);
+    MESH_LAUNCH((gemm_kq_kernel<TYPE, PACKED, XDIRECT, SPLIT, NARROW>), grid, dim3(GEMM_THREADS), smem, stream, k);
     MESH_LAUNCH_CHECK();
     return SPLIT ? gemm_add_slices(k, (int)grid.x, stream) : MESH_OK;
 }
@@ -872,11 +1010,11 @@ int gemm_kquant(const GemmArgs &a, hipStream_t stream) {
         if (!a.Wp || !a.x_k8 || !a.n_tiles || a.max_tiles <= 0 || a.n_seg > 1 || a.bias || a.residual || a.rope.pos || a.expert_stride % 16)
             return fail(MESH_ERR_INVALID, "gemm: an expert launch needs the GEMM layout, k8-major activations and a plain or SwiGLU epilogue");
         if (a.type != MESH_Q4_K && a.type != MESH_Q6_K) return fail(MESH_ERR_UNSUPPORTED, "gemm: no MFMA kernel for ggml type %d", a.type);
-        const dim3 g((unsigned)row_blocks, (unsigned)a.max_tiles);
-        k.ksplit = 1;
-        k.k_per_split = a.K / GK;
-        return a.type == MESH_Q4_K ? launch_gemm_kernel<MESH_Q4_K, true, true, false, false, true>(k, g, stream)
-                                   : launch_gemm_kernel<MESH_Q6_K, true, true, false, false, true>(k, g, stream);
+        const dim3 g((unsigned)row_blocks, (unsigned)((a.max_tiles + 7) / 8 * 8));       // (the kernel deals them to the XCDs in eights)
+        if (a.type == MESH_Q4_K) MESH_LAUNCH(gemm_expert_kernel<MESH_Q4_K>, g, dim3(EXPERT_THREADS), 0, stream, k);
+        else MESH_LAUNCH(gemm_expert_kernel<MESH_Q6_K>, g, dim3(EXPERT_THREADS), 0, stream, k);
+        MESH_LAUNCH_CHECK();
+        return MESH_OK;
     }
     dim3 grid((unsigned)row_blocks, (unsigned)((a.T + GN - 1) / GN));
     // A launch of fewer workgroups than CUs walks all of K in each of them while the rest of the chip idles: split K
@@ -954,12 +1092,10 @@ __global__ __launch_bounds__(256) void gemm_tile_copy_kernel(const uint8_t *__re
     int r = s >> 1;
     PackedSub<TYPE> sub;
     sub.load(packed + ((size_t)mb * n_steps + kc) * PackedSub<TYPE>::CHUNK, s);
-    __align__(16) _Float16 v[32];
-    sub.store(v);
     if (pair) r = (r & 32) * 2 + (r >> 6) * 32 + (r & 31);
-    _Float16 *dst = tile + (size_t)(mb * 8 + (r >> 4)) * 16 * n_steps * GK + ((size_t)(kc * 8 + h * 4) * 16 + (r & 15)) * 8;
+    _Float16 *dst = tile + (size_t)(mb * 8 + (r >> 4)) * 16 * n_steps * GK + ((size_t)(kc * 8 + h) * 16 + (r & 15)) * 8;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) *reinterpret_cast<uint4 *>(dst + j * 128) = reinterpret_cast<const uint4 *>(v)[j];
+    for (int j = 0; j < 4; ++j) *reinterpret_cast<uint4 *>(dst + j * 256) = sub.form(j);
 }
 
 size_t gemm_tile_bytes(int64_t M, int64_t K) { return (size_t)((M + GM - 1) / GM) * GM * (size_t)K * 2; }

@@ -63,13 +63,13 @@ int gemm_split_count(const GemmArgs &a);
 
 // GEMM layout of a K-quant matrix: a second copy for the prefill GEMM, arranged by the workgroup tile that consumes it.
 // One chunk per (128-row block, 64-element k-step), chunks of a row block consecutive in k.  A chunk holds, for each of
-// the 256 (row, 32-element sub-block) pairs s = 2 * row + half, what the staging thread s needs, at s * stride of
-// each section, so that every load of a staging wave covers one contiguous kilobyte:
-//   q4_K (6144 B): [256 x 16 B quants: dword j = elements 8j..8j+3 in the low nibbles, 8j+4..8j+7 in the high ones]
-//                  [256 x 8 B: f16 sc (the integer block scale), f16 c = 8 d sc - dmin m, f16 d, unused]
-//   q6_K (8192 B): [256 x 16 B low nibbles, same order][256 x 8 B upper two bits: byte b of dword j/2 holds, from
-//                  bit 4*(j%2), the bits of element 8j+b and, two bits up, of element 8j+4+b]
-//                  [256 x 8 B: f16 sc of elements 0..15, f16 sc of elements 16..31, f16 d, unused]
+// the 256 slots s = 2 * row + h (elements 16 j + 8 h .. + 7, j = 0..3, of the row's 64), what a thread that forms them
+// needs, at s * stride of each section, and per row the scales; a load of a wave covers whole lines:
+//   q4_K (6144 B): [256 x 16 B quants: dword j, element e of its eight at nibble e / 2 + 4 (e % 2)]
+//                  [128 x 16 B, per 32 elements: f16 sc (the integer block scale), f16 c = 8 d sc - dmin m, f16 d, f16 -72 sc]
+//   q6_K (8192 B): [256 x 16 B low nibbles, same order][256 x 8 B upper two bits: those of element e of dword j in dword j / 2
+//                  at bit 2 P + 16 (e % 2), P = 4 (j % 2) + e / 2]
+//                  [128 x 16 B, per 32 elements: f16 sc of the first 16, f16 sc of the others, f16 d, unused]
 // The kernel forms a weight as ((q - offset) * sc) * d + c: an exact small integer times the super-block's own f16
 // scale, rounded once.  The fields are the ones the kernel would otherwise derive from the block headers, so both
 // layouts give the same bits.  Rows beyond M are zero.

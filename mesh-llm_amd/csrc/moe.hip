@@ -550,7 +550,7 @@ int moe_combine_slots(float *x, const float *y, const float *w, const int32_t *s
 
 // ---- pairs sorted by expert for the large-tile GEMM ------------------------------------------------------------
 // One workgroup: counts per expert (LDS atomics), a scan over the experts for the first slot (a multiple of 16) and the
-// first tile of each, then every pair takes the next free slot of its expert.  Which slot of its expert a pair gets
+// tiles of each, then every pair takes the next free slot of its expert.  Which slot of its expert a pair gets
 // depends on the order the atomics land in; nothing computed from the slots does (a column of a matrix product depends
 // on that column alone, and the combine step finds its rows through slot_of_pair).
 constexpr int SORT_THREADS = 1024;
@@ -558,42 +558,63 @@ __global__ __launch_bounds__(SORT_THREADS) void moe_sort_kernel(const int32_t *_
                                                                 int32_t *__restrict__ slot_of_pair, int32_t *__restrict__ pair_of_slot,
                                                                 int32_t *__restrict__ tiles, int32_t *__restrict__ counts) {
     extern __shared__ int32_t s_lds[];
-    int32_t *s_cnt = s_lds, *s_off = s_cnt + n_expert, *s_tile = s_off + n_expert, *s_cur = s_tile + n_expert;
+    int32_t *s_cnt = s_lds, *s_off = s_cnt + n_expert, *s_full = s_off + n_expert, *s_rest = s_full + n_expert;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int e = tid; e < n_expert; e += SORT_THREADS) { s_cnt[e] = 0; s_cur[e] = 0; }
+    for (int e = tid; e < n_expert; e += SORT_THREADS) s_cnt[e] = 0;
     for (int sl = tid; sl < cap_slots; sl += SORT_THREADS) pair_of_slot[sl] = -1;
     __syncthreads();
     for (int p = tid; p < n_pairs; p += SORT_THREADS) atomicAdd(&s_cnt[ids[p]], 1);
     __syncthreads();
     if (wave == 0) {
-        // exclusive prefixes of padded slots and of tiles per expert: each lane sums a run of experts, the runs are scanned across the wave
+        // exclusive prefixes over the experts: each lane sums a run of them, the runs are scanned across the wave.  [0]: padded
+        // slots; [1..4]: tiles of more than 96, 64, 32 and 0 pairs.  The list begins with the largest tiles and ends with the
+        // smallest: workgroups start in its order, and a long one that starts last is waited for with the chip idle.
         const int per = (n_expert + 63) / 64, e0 = lane * per;
-        int my_s = 0, my_t = 0;
-        for (int e = e0; e < e0 + per && e < n_expert; ++e) { my_s += (s_cnt[e] + 15) & ~15; my_t += (s_cnt[e] + 127) >> 7; }
-        int in_s = my_s, in_t = my_t;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int vs = __shfl_up(in_s, o), vt = __shfl_up(in_t, o);
-            if (lane >= o) { in_s += vs; in_t += vt; }
-        }
-        int run_s = in_s - my_s, run_t = in_t - my_t;
+        int mine[5] = {0, 0, 0, 0, 0}, run[5], base[5];
         for (int e = e0; e < e0 + per && e < n_expert; ++e) {
-            s_off[e] = run_s; s_tile[e] = run_t;
-            run_s += (s_cnt[e] + 15) & ~15; run_t += (s_cnt[e] + 127) >> 7;
+            const int c = s_cnt[e], rest = c & 127;
+            mine[0] += (c + 15) & ~15;
+            mine[1] += c >> 7;
+#pragma unroll
+            for (int k = 1; k < 5; ++k) mine[k] += rest && 4 - ((rest - 1) >> 5) == k ? 1 : 0;
         }
-        if (lane == 63) { counts[0] = in_t; counts[1] = in_s; }
+        int total = 0;
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+            int in = mine[k];
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int v = __shfl_up(in, o);
+                if (lane >= o) in += v;
+            }
+            const int sum = __shfl(in, 63);
+            base[k] = k < 1 ? 0 : total;
+            run[k] = base[k] + in - mine[k];
+            if (k == 0) { if (lane == 0) counts[1] = sum; } else total += sum;
+        }
+        if (lane == 0) counts[0] = total;
+        for (int e = e0; e < e0 + per && e < n_expert; ++e) {
+            const int c = s_cnt[e], rest = c & 127;
+            s_off[e] = run[0]; run[0] += (c + 15) & ~15;
+            s_full[e] = run[1]; run[1] += c >> 7;
+#pragma unroll
+            for (int k = 1; k < 5; ++k)
+                if (rest && 4 - ((rest - 1) >> 5) == k) s_rest[e] = run[k]++;
+        }
     }
     __syncthreads();
     for (int e = tid; e < n_expert; e += SORT_THREADS) {
         const int cnt = s_cnt[e];
         for (int j = 0; j * 128 < cnt; ++j) {
-            int32_t *tl = tiles + (size_t)(s_tile[e] + j) * 4;
-            tl[0] = e; tl[1] = s_off[e] + 128 * j; tl[2] = cnt - 128 * j < 128 ? cnt - 128 * j : 128; tl[3] = 0;
+            const int n = cnt - 128 * j < 128 ? cnt - 128 * j : 128;
+            int32_t *tl = tiles + (size_t)(n == 128 ? s_full[e] + j : s_rest[e]) * 4;
+            tl[0] = e; tl[1] = s_off[e] + 128 * j; tl[2] = n; tl[3] = 0;
         }
     }
+    __syncthreads();
     for (int p = tid; p < n_pairs; p += SORT_THREADS) {
         const int e = ids[p];
-        const int sl = s_off[e] + atomicAdd(&s_cur[e], 1);
+        const int sl = atomicAdd(&s_off[e], 1);
         slot_of_pair[p] = sl;
         pair_of_slot[sl] = p;
     }

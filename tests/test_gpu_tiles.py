@@ -84,3 +84,38 @@ def test_kquant_products_of_many_tokens(tmp_path, shape, tokens):
     assert np.linalg.norm(got[1] - want) / norm < 3e-3, (shape, tokens)
     # the same f16 weights and inputs summed in another order: what a rounding point of the next input next to a sum can move
     assert np.linalg.norm(got[1] - got[0]) / norm < 1e-3, (shape, tokens)
+
+
+@pytest.mark.parametrize("n_embd,ff,tokens", [
+    (256, 256, 17),         # one round of four steps along K; every expert in a tile of at most 32 pairs
+    (512, 256, 65),
+    (256, 512, 150),        # an expert past one tile of 128
+    (512, 768, 301),        # remainders of one to four groups of 32 pairs
+])
+def test_expert_products_over_ragged_loads(tmp_path, n_embd, ff, tokens):
+    """A chunk through two expert layers (q4_K and q6_K down projections) whose experts get from a few pairs to most tokens: the
+    expert tiles against the oracle and against the 16-pair integer kernel."""
+    m = mesh()
+    cfg = dict(arch="qwen3moe", n_layer=2, n_embd=n_embd, n_head=4, n_head_kv=2, head_dim=128, n_ff=0, n_vocab=256, eps=1e-6, rope=1e6,
+               n_expert=24, n_expert_used=3, n_ff_exp=ff, qk_norm=True)
+    path = str(tmp_path / "model.gguf")
+    tensors = models.write_model(path, cfg, [0, 1], seed=5, router="zipf")
+    x = models.zipf_hidden_state(np.random.Generator(np.random.PCG64(tokens)), tokens, n_embd)
+    orc = StageOracle(cfg, tensors, 0, 2, 512, blas=True)
+    want = orc.forward(x, np.arange(tokens)) - x
+    got, ids = {}, {}
+    for tiles in (0, 1):
+        st = m.Stage(path, 0, 2, n_ctx=512, n_batch_max=512)
+        ses = st.session(moe_gemm=tiles, moe_gemm_min_pairs=1)
+        got[tiles] = ses.decode(x, np.arange(tokens)).view(np.float32).reshape(want.shape) - x
+        ids[tiles] = np.sort(ses.moe_last_ids(tokens), axis=1)
+        assert ses.f16_saturations() == 0
+        ses.close()
+        st.close()
+    # a token whose routing a rounding point moved is another computation: at most a few near ties, not compared
+    same = (ids[0] == np.sort(np.stack(orc.last_expert_ids), axis=1)).all(axis=1) & (ids[0] == ids[1]).all(axis=1)
+    assert same.mean() > 0.97
+    norm = np.linalg.norm(want[same])
+    # f16 activations: 11 bits in the inputs of the four products of each layer, and once more through the second layer
+    assert np.linalg.norm((got[1] - want)[same]) / norm < 6e-3
+    assert np.linalg.norm((got[1] - got[0])[same]) / norm < 6e-3
