@@ -263,7 +263,7 @@ __device__ __forceinline__ void lds_barrier() {
 // 16 k is four contiguous 256-byte pieces of that layout, so each lane fetches its 16 bytes straight from memory (L2),
 // four k16 steps ahead, into a ring of registers.  That halves the LDS reads per MFMA and leaves the staging waves only
 // the weights.
-template <int TYPE, bool PACKED, bool XDIRECT, bool SPLIT, bool NARROW>
+template <int TYPE, bool PACKED, bool XDIRECT, bool SPLIT>
 __global__ __launch_bounds__(GEMM_THREADS) void gemm_kq_kernel(GemmArgs a) {
     extern __shared__ __align__(16) _Float16 gemm_smem[];
     _Float16 *Ws = gemm_smem;                                  // [2][GM][LDS_LD]
@@ -340,11 +340,9 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_kq_kernel(GemmArgs a) {
     }
 
     // ---- multiplying waves
-    // wave's corner of the tile: 64 rows x 64 tokens; NARROW (calls of at most 64 tokens, whose upper token half would
-    // be padding): 32 rows x the lower 64 tokens, so all four waves multiply real columns
-    static_assert(!NARROW || XDIRECT, "the narrow tile reads its activations from the k8-major layout");
-    constexpr int MI = NARROW ? 1 : 2;
-    const int wm = NARROW ? wave * 32 : (wave & 1) * 64, wn = NARROW ? 0 : (wave >> 1) * 64;
+    // wave's corner of the tile: 64 rows x 64 tokens
+    constexpr int MI = 2;
+    const int wm = (wave & 1) * 64, wn = (wave >> 1) * 64;
     float16v acc[MI][2];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
@@ -391,7 +389,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_kq_kernel(GemmArgs a) {
             }
             __syncthreads();
         }
-    } else if constexpr (!NARROW) {
+    } else {
     __syncthreads();
     for (int kc = 0; kc < n_steps; ++kc) {
         const int buf = kc & 1;
@@ -435,11 +433,9 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_kq_kernel(GemmArgs a) {
         // SwiGLU pair: the waves of the upper half of the tile hold the up rows of the gate rows in the lower half, at
         // the same (register, lane).  They hand them over through LDS (free by now: the staging waves have left, and
         // the barrier makes sure every matrix-core wave has read its last fragments).
-        // (NARROW: waves 2 and 3 hold the up rows of the gate rows of waves 0 and 1)
         float *xch = reinterpret_cast<float *>(gemm_smem);         // [pair of waves][64 registers][64 lanes]
-        const bool is_up = NARROW ? wave >= 2 : wm != 0;
-        const int pair = NARROW ? (wave & 1) * 2 : (wn >> 6) * 4;  // first 16-register group of this pair of waves
-        const int gm = NARROW ? (wave & 1) * 32 : 0;               // gate rows of this wave inside the block's 64
+        const bool is_up = wm != 0;
+        const int pair = (wn >> 6) * 4;  // first 16-register group of this pair of waves
         __syncthreads();
         if (is_up) {
 #pragma unroll
@@ -460,7 +456,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_kq_kernel(GemmArgs a) {
                 if (t >= t_pad) continue;
 #pragma unroll
                 for (int e4 = 0; e4 < 4; ++e4) {
-                    const int m = (int)blockIdx.x * (GM / 2) + gm + 32 * i + 8 * e4 + 4 * (lane >> 5);
+                    const int m = (int)blockIdx.x * (GM / 2) + 32 * i + 8 * e4 + 4 * (lane >> 5);
                     if (m >= a.M) continue;
                     float o[4];
 #pragma unroll
@@ -524,44 +520,55 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_kq_kernel(GemmArgs a) {
 // at the rate of a large copy: 22 us.
 // Rows of a SwiGLU pair are dealt out so that a wave holds 16 gate rows and the 16 up rows of the same outputs, in one lane's
 // registers e and e + 8.
-constexpr int EXPERT_THREADS = 256;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-template <int TYPE, int NT>
-__device__ __forceinline__ void expert_tile(const GemmArgs &a, const uint8_t *wp, int bx, int t0, int t_end, u32x4 *xs) {
+// KG groups of four waves, each over its own part of the k-steps; the partial products meet in LDS.
+// The k order of the sums is the 128-column tile's, within a group.
+// MODE: REG_DENSE, REG_SPLIT (raw sums of slice blockIdx.z to a.part), REG_EXPERT (one group).
+enum { REG_DENSE, REG_SPLIT, REG_EXPERT };
+constexpr int reg_lds_bytes(int NT, int KG) { return KG * NT * 8192; }        // two buffers of activations per group; half the groups' sums
+template <int TYPE, int NT, int MODE, int KG>
+__device__ __forceinline__ void reg_tile(const GemmArgs &a, const uint8_t *wp, int bx, int t0, int t_end, int k0, int n_steps, u32x4 *lds) {
     constexpr int AHEAD = 4, STEP = NT * 256;                  // chunks of weights on their way; 16-byte pieces of a chunk's activations
-    const int tid = threadIdx.x, lane = tid & 63, hh = lane >> 5;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int n_steps = a.K / GK;
-    const bool pair = a.y16_k8 != nullptr;
-    const int r = lane & 31;
+    const int tid = threadIdx.x & 255, lane = tid & 63, hh = lane >> 5, r = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), group = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+    const int n_all = a.K / GK;
+    // this group's k-steps [k0, k0 + n) and the rounds that every group walks (the barriers are the workgroup's)
+    const int per = (n_steps + KG - 1) / KG;
+    k0 += group * per;
+    const int n = KG == 1 ? n_steps : n_steps - group * per < per ? n_steps - group * per : per;
+    const bool pair = MODE != REG_SPLIT && a.y16_k8 != nullptr;
     const unsigned slot = 2 * (pair ? 16 * wave + (r & 15) + (r >> 4) * 64 : 32 * wave + r) + hh;
-    wp += (size_t)bx * n_steps * PackedSub<TYPE>::CHUNK;
+    wp += ((size_t)bx * n_all + k0) * PackedSub<TYPE>::CHUNK;
     const int n_blk = (a.T + 15) >> 4;
-    const u32x4 *const xbase = reinterpret_cast<const u32x4 *>(a.X + (size_t)(t0 >> 4) * 16 * a.K);
+    const u32x4 *const xbase = reinterpret_cast<const u32x4 *>(a.X + (size_t)(t0 >> 4) * 16 * a.K) + (size_t)k0 * 128;
     unsigned xo[NT];                                           // 16-byte pieces from the tile's first block
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
         const int b = 2 * i + (tid >> 7), last = n_blk - 1 - (t0 >> 4);        // (blocks past the list re-read the last one, never stored)
         xo[i] = (unsigned)(b < last ? b : last) * (unsigned)(2 * a.K) + (unsigned)(tid & 127);
     }
+    u32x4 *xs = lds + group * 2 * STEP;
     float16v acc[NT];
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[j][e] = 0.f;
+    const int last = n > 0 ? n - 1 : 0;                        // (a group without steps of its own reads the first and multiplies none)
+    if (n <= 0) { wp -= (size_t)k0 * PackedSub<TYPE>::CHUNK; }
+    const u32x4 *const xb = n > 0 ? xbase : xbase - (size_t)k0 * 128;
     PackedSub<TYPE> rw[AHEAD];
     u32x4 rx[NT];
 #pragma unroll
-    for (int i = 0; i < NT; ++i) rx[i] = xbase[xo[i]];
+    for (int i = 0; i < NT; ++i) rx[i] = xb[xo[i]];
 #pragma unroll
-    for (int u = 0; u < AHEAD; ++u) rw[u].load(wp + (size_t)u * PackedSub<TYPE>::CHUNK, slot);       // (K is a multiple of 256)
+    for (int u = 0; u < AHEAD; ++u) rw[u].load(wp + (size_t)(MODE == REG_EXPERT || u < last ? u : last) * PackedSub<TYPE>::CHUNK, slot);
 #pragma unroll
-    for (int i = 0; i < NT; ++i) xs[(0) * STEP + i * 256 + tid] = rx[i];
+    for (int i = 0; i < NT; ++i) xs[i * 256 + tid] = rx[i];
 #pragma unroll
-    for (int i = 0; i < NT; ++i) rx[i] = (xbase + 128)[xo[i]];
+    for (int i = 0; i < NT; ++i) rx[i] = (xb + (size_t)(1 < last ? 1 : last) * 128)[xo[i]];
     lds_barrier();
     const int at = (lane & 15) + ((lane >> 4) & 1) * 128 + hh * 16;
-    for (int kc0 = 0; kc0 < n_steps; kc0 += AHEAD) {
+    for (int kc0 = 0; kc0 < per; kc0 += AHEAD) {
 #pragma unroll
         for (int u = 0; u < AHEAD; ++u) {
             const int kc = kc0 + u;
@@ -569,32 +576,68 @@ __device__ __forceinline__ void expert_tile(const GemmArgs &a, const uint8_t *wp
 #pragma unroll
             for (int i = 0; i < NT; ++i) xs[((u + 1) & 1) * STEP + i * 256 + tid] = rx[i];
 #pragma unroll
-            for (int i = 0; i < NT; ++i) rx[i] = (xbase + (size_t)(kc + 2 < n_steps ? kc + 2 : n_steps - 1) * 128)[xo[i]];
+            for (int i = 0; i < NT; ++i) rx[i] = (xb + (size_t)(kc + 2 < last ? kc + 2 : last) * 128)[xo[i]];
             const u32x4 *x = xs + (u & 1) * STEP + at;
-            u32x4 f[2][NT];
+            if (MODE == REG_EXPERT || kc < n) {                // (an expert's K is a multiple of 256)
+                u32x4 f[2][NT];
 #pragma unroll
-            for (int j = 0; j < NT; ++j) f[0][j] = x[j * 256];
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int st = 0; st < 4; ++st) {
-                if (st < 3)
-#pragma unroll
-                    for (int j = 0; j < NT; ++j) f[(st + 1) & 1][j] = x[j * 256 + (st + 1) * 32];
-                const half8 w = __builtin_bit_cast(half8, rw[u].form(st));
-#pragma unroll
-                for (int j = 0; j < NT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w, __builtin_bit_cast(half8, f[st & 1][j]), acc[j], 0, 0, 0);
+                for (int j = 0; j < NT; ++j) f[0][j] = x[j * 256];
                 __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int st = 0; st < 4; ++st) {
+                    if (st < 3)
+#pragma unroll
+                        for (int j = 0; j < NT; ++j) f[(st + 1) & 1][j] = x[j * 256 + (st + 1) * 32];
+                    const half8 w = __builtin_bit_cast(half8, rw[u].form(st));
+#pragma unroll
+                    for (int j = 0; j < NT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w, __builtin_bit_cast(half8, f[st & 1][j]), acc[j], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
-            rw[u].load(wp + (size_t)(kc + AHEAD < n_steps ? kc + AHEAD : n_steps - 1) * PackedSub<TYPE>::CHUNK, slot);
+            rw[u].load(wp + (size_t)(kc + AHEAD < last ? kc + AHEAD : last) * PackedSub<TYPE>::CHUNK, slot);
             lds_barrier();
         }
     }
-    const int t_pad = (t_end + 15) & ~15;
+    // the groups' sums, the upper half of them added to the lower until one is left
 #pragma unroll
-    for (int j = 0; j < NT; ++j) {
-        const int t = t0 + 32 * j + r;
-        if (t >= (pair ? t_pad : t_end)) continue;
-        if (pair) {
+    for (int half = KG / 2; half > 0; half /= 2) {
+        float *part = reinterpret_cast<float *>(lds) + ((group % half) * 4 + wave) * NT * 1024 + lane;
+        if (group >= half && group < 2 * half) {
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) part[(j * 16 + e) * 64] = acc[j][e];
+        }
+        __syncthreads();
+        if (group < half) {
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[j][e] += part[(j * 16 + e) * 64];
+        }
+        if (half > 1) __syncthreads();
+    }
+    if (group > 0) return;
+    if constexpr (MODE == REG_SPLIT) {
+        // slice of a split launch: the raw sums go to part[slice][token][row of the launch]
+        const size_t ld = (size_t)gridDim.x * GM;
+        float *P = a.part + (size_t)blockIdx.z * a.T * ld + (size_t)bx * GM + 32 * wave + 4 * hh;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            const int t = t0 + 32 * j + r;
+            if (t >= t_end) continue;
+#pragma unroll
+            for (int e4 = 0; e4 < 4; ++e4)
+                *reinterpret_cast<float4 *>(P + (size_t)t * ld + 8 * e4) = make_float4(acc[j][4 * e4], acc[j][4 * e4 + 1], acc[j][4 * e4 + 2], acc[j][4 * e4 + 3]);
+        }
+        return;
+    }
+    if (pair) {
+        const int t_pad = (t_end + 15) & ~15;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            const int t = t0 + 32 * j + r;
+            if (t >= t_pad) continue;
 #pragma unroll
             for (int e4 = 0; e4 < 2; ++e4) {
                 const int m = bx * (GM / 2) + 16 * wave + 8 * e4 + 4 * hh;
@@ -609,30 +652,69 @@ __device__ __forceinline__ void expert_tile(const GemmArgs &a, const uint8_t *wp
                 *reinterpret_cast<uint2 *>(a.y16_k8 + (size_t)(t >> 4) * 16 * a.M + ((size_t)(m >> 3) * 16 + (t & 15)) * 8 + (m & 7)) =
                     make_uint2(pack_h2(o[0], o[1]), pack_h2(o[2], o[3]));
             }
-        } else {
+        }
+        return;
+    }
+    float *Y = a.Y;
+    const float *bias = MODE == REG_DENSE ? a.bias : nullptr, *res = MODE == REG_DENSE ? a.residual : nullptr;
+    int M = a.M, ldy = a.ldy, mb0 = bx * GM;
+    if (MODE == REG_DENSE && a.n_seg > 1) {
+        // (selected, not indexed: a dynamically indexed kernel-argument array would be spilled to scratch)
+        const int sg = (bx >= a.seg_begin[1] ? 1 : 0) + (a.n_seg > 2 && bx >= a.seg_begin[2] ? 1 : 0);
+        Y = sg == 0 ? a.seg_Y[0] : sg == 1 ? a.seg_Y[1] : a.seg_Y[2];
+        bias = sg == 0 ? a.seg_bias[0] : sg == 1 ? a.seg_bias[1] : a.seg_bias[2];
+        M = sg == 0 ? a.seg_M[0] : sg == 1 ? a.seg_M[1] : a.seg_M[2];
+        ldy = sg == 0 ? a.seg_ldy[0] : sg == 1 ? a.seg_ldy[1] : a.seg_ldy[2];
+        mb0 = (bx - (sg == 0 ? 0 : sg == 1 ? a.seg_begin[1] : a.seg_begin[2])) * GM;
+    }
 #pragma unroll
-            for (int e4 = 0; e4 < 4; ++e4) {
-                const int m = bx * GM + 32 * wave + 8 * e4 + 4 * hh;
-                if (m >= a.M) continue;
-                *reinterpret_cast<float4 *>(a.Y + (size_t)t * a.ldy + m) = make_float4(acc[j][4 * e4], acc[j][4 * e4 + 1], acc[j][4 * e4 + 2], acc[j][4 * e4 + 3]);
+    for (int j = 0; j < NT; ++j) {
+        const int t = t0 + 32 * j + r;
+        if (t >= t_end) continue;
+#pragma unroll
+        for (int e4 = 0; e4 < 4; ++e4) {
+            const int m = mb0 + 32 * wave + 8 * e4 + 4 * hh;
+            if (m >= M) continue;              // M is a multiple of 4 for every projection
+            float4 o = make_float4(acc[j][4 * e4], acc[j][4 * e4 + 1], acc[j][4 * e4 + 2], acc[j][4 * e4 + 3]);
+            if (bias) {
+                const float4 b = *reinterpret_cast<const float4 *>(bias + m);
+                o.x += b.x; o.y += b.y; o.z += b.z; o.w += b.w;
             }
+            if (res) {
+                const float4 q = *reinterpret_cast<const float4 *>(res + (size_t)t * a.ldres + m);
+                o.x += q.x; o.y += q.y; o.z += q.z; o.w += q.w;
+            }
+            *reinterpret_cast<float4 *>(Y + (size_t)t * ldy + m) = o;
         }
     }
 }
 template <int TYPE>
-__global__ __launch_bounds__(EXPERT_THREADS, 2) void gemm_expert_kernel(GemmArgs a) {
+__global__ __launch_bounds__(256, 2) void gemm_expert_kernel(GemmArgs a) {
     __shared__ u32x4 xs[2 * 4 * 256];
     // workgroups go to the eight XCDs in turn: every row block of a tile on one of them, whose L2 fetches the tile's activations once
     const int g = (int)(blockIdx.y * gridDim.x + blockIdx.x), by = (g >> 3) / (int)gridDim.x * 8 + (g & 7), bx = (g >> 3) % (int)gridDim.x;
     if (by >= *a.n_tiles) return;
     const int4 tl = reinterpret_cast<const int4 *>(a.tiles)[by];
     const uint8_t *wp = static_cast<const uint8_t *>(a.Wp) + (size_t)tl.x * a.expert_stride;
+    const int n = a.K / GK;
     switch ((tl.z + 31) >> 5) {
-        case 1: return expert_tile<TYPE, 1>(a, wp, bx, tl.y, tl.y + tl.z, xs);
-        case 2: return expert_tile<TYPE, 2>(a, wp, bx, tl.y, tl.y + tl.z, xs);
-        case 3: return expert_tile<TYPE, 3>(a, wp, bx, tl.y, tl.y + tl.z, xs);
-        default: return expert_tile<TYPE, 4>(a, wp, bx, tl.y, tl.y + tl.z, xs);
+        case 1: return reg_tile<TYPE, 1, REG_EXPERT, 1>(a, wp, bx, tl.y, tl.y + tl.z, 0, n, xs);
+        case 2: return reg_tile<TYPE, 2, REG_EXPERT, 1>(a, wp, bx, tl.y, tl.y + tl.z, 0, n, xs);
+        case 3: return reg_tile<TYPE, 3, REG_EXPERT, 1>(a, wp, bx, tl.y, tl.y + tl.z, 0, n, xs);
+        default: return reg_tile<TYPE, 4, REG_EXPERT, 1>(a, wp, bx, tl.y, tl.y + tl.z, 0, n, xs);
     }
+}
+// Dense calls of at most 64 tokens, at most 32 or 64 columns.  A launch of few workgroups per CU needs its waves from K: four groups
+// (16 waves), two in a slice of a split launch, whose k range is short already.  Gate / up of 2 x 14336 rows x 4096 (q4_K, 66 MB):
+// 41 us at 40 tokens with the staging waves of gemm_kq_kernel, 31 with two groups, 28 with four; 22 at 20 tokens; down projection of
+// 4096 x 14336 (q6_K): 23 -> 18 us.  From 65 tokens on every wave reads every activation fragment, LDS gives out and the
+// 128-column tile is the better one (128 tokens: 45 us against 48 for gate / up, but 29 against 27 and 16 against 13 for the others).
+template <int TYPE, int NT, int MODE, int KG>
+__global__ __launch_bounds__(256 * KG, 4) void gemm_reg_kernel(GemmArgs a) {
+    __shared__ u32x4 lds[reg_lds_bytes(NT, KG) / 16];
+    const int n_all = a.K / GK, k0 = MODE == REG_SPLIT ? (int)blockIdx.z * a.k_per_split : 0;
+    const int n = MODE == REG_SPLIT && n_all - k0 > a.k_per_split ? a.k_per_split : n_all - k0;
+    reg_tile<TYPE, NT, MODE, KG>(a, static_cast<const uint8_t *>(a.Wp), (int)blockIdx.x, 0, a.T, k0, n, lds);
 }
 
 // ---- the same product on a 256 x 128 workgroup tile ----------------------------------------------------------
@@ -932,16 +1014,16 @@ int gemm_add_slices(const GemmArgs &k, int row_blocks, hipStream_t stream) {
     return MESH_OK;
 }
 
-template <int TYPE, bool PACKED, bool XDIRECT, bool SPLIT, bool NARROW>
+template <int TYPE, bool PACKED, bool XDIRECT, bool SPLIT>
 static int launch_gemm_kernel(const GemmArgs &k, dim3 grid, hipStream_t stream) {
     // two stages of the weight slab, and of the activation slab unless the activations bypass LDS: 73 728 / 36 864 B
     constexpr size_t smem = sizeof(_Float16) * 2 * (GM + (XDIRECT ? 0 : GN)) * LDS_LD;
     static bool attr_set = false;
     if (!attr_set) {
-        MESH_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_kq_kernel<TYPE, PACKED, XDIRECT, SPLIT, NARROW>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+        MESH_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_kq_kernel<TYPE, PACKED, XDIRECT, SPLIT>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
         attr_set = true;
     }
-    MESH_LAUNCH((gemm_kq_kernel<TYPE, PACKED, XDIRECT, SPLIT, NARROW>), grid, dim3(GEMM_THREADS), smem, stream, k);
+    MESH_LAUNCH((gemm_kq_kernel<TYPE, PACKED, XDIRECT, SPLIT>), grid, dim3(GEMM_THREADS), smem, stream, k);
     MESH_LAUNCH_CHECK();
     return SPLIT ? gemm_add_slices(k, (int)grid.x, stream) : MESH_OK;
 }
@@ -957,14 +1039,21 @@ static int gemm_n_cu() {
     return n;
 }
 
+template <int TYPE, int NT>
+static int launch_gemm_reg(const GemmArgs &k, dim3 grid, hipStream_t stream) {
+    if (k.ksplit > 1) MESH_LAUNCH((gemm_reg_kernel<TYPE, NT, REG_SPLIT, 2>), grid, dim3(512), 0, stream, k);
+    else MESH_LAUNCH((gemm_reg_kernel<TYPE, NT, REG_DENSE, 4>), grid, dim3(1024), 0, stream, k);
+    MESH_LAUNCH_CHECK();
+    return k.ksplit > 1 ? gemm_add_slices(k, (int)grid.x, stream) : MESH_OK;
+}
+
 template <int TYPE, bool PACKED, bool XDIRECT>
 static int launch_gemm(const GemmArgs &k, dim3 grid, hipStream_t stream) {
-    // calls of at most 64 tokens on the production layout (GEMM-layout weights, k8-major activations): narrow tile
+    // calls of at most 64 tokens on the production layout (GEMM-layout weights, k8-major activations)
     if constexpr (PACKED && XDIRECT) {
-        if (k.T <= GN / 2 && k.narrow_tile)
-            return k.ksplit > 1 ? launch_gemm_kernel<TYPE, true, true, true, true>(k, grid, stream) : launch_gemm_kernel<TYPE, true, true, false, true>(k, grid, stream);
+        if (k.T <= GN / 2 && k.narrow_tile) return k.T <= GN / 4 ? launch_gemm_reg<TYPE, 1>(k, grid, stream) : launch_gemm_reg<TYPE, 2>(k, grid, stream);
     }
-    return k.ksplit > 1 ? launch_gemm_kernel<TYPE, PACKED, XDIRECT, true, false>(k, grid, stream) : launch_gemm_kernel<TYPE, PACKED, XDIRECT, false, false>(k, grid, stream);
+    return k.ksplit > 1 ? launch_gemm_kernel<TYPE, PACKED, XDIRECT, true>(k, grid, stream) : launch_gemm_kernel<TYPE, PACKED, XDIRECT, false>(k, grid, stream);
 }
 
 // slices of K for a launch of row_blocks x t_blocks workgroups (1: not split); *k_per_split = k-steps per slice
@@ -1011,8 +1100,8 @@ int gemm_kquant(const GemmArgs &a, hipStream_t stream) {
             return fail(MESH_ERR_INVALID, "gemm: an expert launch needs the GEMM layout, k8-major activations and a plain or SwiGLU epilogue");
         if (a.type != MESH_Q4_K && a.type != MESH_Q6_K) return fail(MESH_ERR_UNSUPPORTED, "gemm: no MFMA kernel for ggml type %d", a.type);
         const dim3 g((unsigned)row_blocks, (unsigned)((a.max_tiles + 7) / 8 * 8));       // (the kernel deals them to the XCDs in eights)
-        if (a.type == MESH_Q4_K) MESH_LAUNCH(gemm_expert_kernel<MESH_Q4_K>, g, dim3(EXPERT_THREADS), 0, stream, k);
-        else MESH_LAUNCH(gemm_expert_kernel<MESH_Q6_K>, g, dim3(EXPERT_THREADS), 0, stream, k);
+        if (a.type == MESH_Q4_K) MESH_LAUNCH(gemm_expert_kernel<MESH_Q4_K>, g, dim3(256), 0, stream, k);
+        else MESH_LAUNCH(gemm_expert_kernel<MESH_Q6_K>, g, dim3(256), 0, stream, k);
         MESH_LAUNCH_CHECK();
         return MESH_OK;
     }

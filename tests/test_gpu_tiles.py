@@ -119,3 +119,33 @@ def test_expert_products_over_ragged_loads(tmp_path, n_embd, ff, tokens):
     # f16 activations: 11 bits in the inputs of the four products of each layer, and once more through the second layer
     assert np.linalg.norm((got[1] - want)[same]) / norm < 6e-3
     assert np.linalg.norm((got[1] - got[0])[same]) / norm < 6e-3
+
+
+@pytest.mark.parametrize("shape,tokens", [
+    ((256, 2, 1, 256), 17),         # four steps along K: one for each group of waves; padding columns
+    ((512, 4, 1, 768), 32),         # the full 32-column tile; 12 steps
+    ((512, 4, 1, 2816), 33),        # 44 steps in slices of eleven, six and five of them for a slice's two groups
+    ((1024, 8, 2, 2816), 64),       # the full 64-column tile
+    ((256, 2, 1, 33024), 47),       # more row blocks than compute units: K in one piece
+])
+def test_kquant_products_of_few_tokens(tmp_path, shape, tokens):
+    """A chunk of 17 to 64 tokens through one layer, against the oracle and against the 128-column tile."""
+    m = mesh()
+    cfg = kquant(*shape)
+    path = str(tmp_path / "model.gguf")
+    tensors = models.write_model(path, cfg, [0], seed=11)
+    x = np.random.Generator(np.random.PCG64(tokens)).standard_normal((tokens, cfg["n_embd"])).astype(np.float32)
+    want = StageOracle(cfg, tensors, 0, 1, 128, blas=True).forward(x, np.arange(tokens))
+    st = m.Stage(path, 0, 1, n_ctx=128, n_batch_max=128)
+    got = {}
+    for narrow in (0, 1):
+        ses = st.session(gemm_narrow=narrow)
+        got[narrow] = ses.decode(x, np.arange(tokens)).view(np.float32).reshape(want.shape)
+        assert ses.f16_saturations() == 0
+        ses.close()
+    st.close()
+    norm = np.linalg.norm(want)
+    # f16 activations over one layer: 11 bits in the inputs of four products
+    assert np.linalg.norm(got[1] - want) / norm < 3e-3, (shape, tokens)
+    # the same weights and inputs, sums along K met in another order
+    assert np.linalg.norm(got[1] - got[0]) / norm < 1e-3, (shape, tokens)
