@@ -523,8 +523,8 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_kq_kernel(GemmArgs a) {
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // KG groups of four waves, each over its own part of the k-steps; the partial products meet in LDS.
 // The k order of the sums is the 128-column tile's, within a group.
-// MODE: REG_DENSE, REG_SPLIT (raw sums of slice blockIdx.z to a.part), REG_EXPERT (one group).
-enum { REG_DENSE, REG_SPLIT, REG_EXPERT };
+// MODE: REG_DENSE, REG_SPLIT (raw sums of slice blockIdx.z to a.part), REG_EXPERT (one group), REG_NORM (a pair with a.norm_part).
+enum { REG_DENSE, REG_SPLIT, REG_EXPERT, REG_NORM };
 constexpr int reg_lds_bytes(int NT, int KG) { return KG * NT * 8192; }        // two buffers of activations per group; half the groups' sums
 template <int TYPE, int NT, int MODE, int KG>
 __device__ __forceinline__ void reg_tile(const GemmArgs &a, const uint8_t *wp, int bx, int t0, int t_end, int k0, int n_steps, u32x4 *lds) {
@@ -598,6 +598,16 @@ __device__ __forceinline__ void reg_tile(const GemmArgs &a, const uint8_t *wp, i
             lds_barrier();
         }
     }
+    float inv_rms = 1.0f;
+    float *const nrm = reinterpret_cast<float *>(lds) + reg_lds_bytes(NT, KG) / 4;     // [8 KG][32 columns]
+    if (MODE == REG_NORM && a.norm_part) {
+        // (after the weight stream: before it, the wave would wait for them ahead of its first tile loads)
+        const int cols = a.T > 16 ? 32 : 16;
+        float ss = 0.f;
+        if (r < cols)
+            for (int p = threadIdx.x >> 5; p < a.norm_parts; p += 8 * KG) ss += a.norm_part[(size_t)p * cols + r];
+        nrm[threadIdx.x] = ss;
+    }
     // the groups' sums, the upper half of them added to the lower until one is left
 #pragma unroll
     for (int half = KG / 2; half > 0; half /= 2) {
@@ -618,6 +628,11 @@ __device__ __forceinline__ void reg_tile(const GemmArgs &a, const uint8_t *wp, i
         if (half > 1) __syncthreads();
     }
     if (group > 0) return;
+    if (MODE == REG_NORM && a.norm_part) {
+        float ss = 0.f;
+        for (int q = 0; q < 8 * KG; ++q) ss += nrm[q * 32 + r];
+        inv_rms = 1.0f / sqrtf(ss / (float)a.K + a.norm_eps);
+    }
     if constexpr (MODE == REG_SPLIT) {
         // slice of a split launch: the raw sums go to part[slice][token][row of the launch]
         const size_t ld = (size_t)gridDim.x * GM;
@@ -645,7 +660,7 @@ __device__ __forceinline__ void reg_tile(const GemmArgs &a, const uint8_t *wp, i
                 float o[4];
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
-                    const float g = acc[j][4 * e4 + c], up = acc[j][8 + 4 * e4 + c];
+                    const float g = acc[j][4 * e4 + c] * inv_rms, up = acc[j][8 + 4 * e4 + c] * inv_rms;
                     o[c] = t < t_end ? g / (1.0f + expf(-g)) * up : 0.f;       // padding columns of the last token block hold zeros
                 }
                 note_f16_clamp(a.sat, o[0], o[1], o[2], o[3]);
@@ -711,7 +726,7 @@ __global__ __launch_bounds__(256, 2) void gemm_expert_kernel(GemmArgs a) {
 // 128-column tile is the better one (128 tokens: 45 us against 48 for gate / up, but 29 against 27 and 16 against 13 for the others).
 template <int TYPE, int NT, int MODE, int KG>
 __global__ __launch_bounds__(256 * KG, 4) void gemm_reg_kernel(GemmArgs a) {
-    __shared__ u32x4 lds[reg_lds_bytes(NT, KG) / 16];
+    __shared__ u32x4 lds[reg_lds_bytes(NT, KG) / 16 + (MODE == REG_NORM ? 64 * KG : 0)];
     const int n_all = a.K / GK, k0 = MODE == REG_SPLIT ? (int)blockIdx.z * a.k_per_split : 0;
     const int n = MODE == REG_SPLIT && n_all - k0 > a.k_per_split ? a.k_per_split : n_all - k0;
     reg_tile<TYPE, NT, MODE, KG>(a, static_cast<const uint8_t *>(a.Wp), (int)blockIdx.x, 0, a.T, k0, n, lds);
@@ -1039,10 +1054,12 @@ static int gemm_n_cu() {
     return n;
 }
 
-template <int TYPE, int NT>
+// groups of waves along K: four where a CU gets one workgroup (16 waves), two where it gets several or K is split already
+template <int TYPE, int NT, int MODE>
 static int launch_gemm_reg(const GemmArgs &k, dim3 grid, hipStream_t stream) {
     if (k.ksplit > 1) MESH_LAUNCH((gemm_reg_kernel<TYPE, NT, REG_SPLIT, 2>), grid, dim3(512), 0, stream, k);
-    else MESH_LAUNCH((gemm_reg_kernel<TYPE, NT, REG_DENSE, 4>), grid, dim3(1024), 0, stream, k);
+    else if ((int)grid.x > gemm_n_cu()) MESH_LAUNCH((gemm_reg_kernel<TYPE, NT, MODE, 2>), grid, dim3(512), 0, stream, k);
+    else MESH_LAUNCH((gemm_reg_kernel<TYPE, NT, MODE, 4>), grid, dim3(1024), 0, stream, k);
     MESH_LAUNCH_CHECK();
     return k.ksplit > 1 ? gemm_add_slices(k, (int)grid.x, stream) : MESH_OK;
 }
@@ -1051,7 +1068,7 @@ template <int TYPE, bool PACKED, bool XDIRECT>
 static int launch_gemm(const GemmArgs &k, dim3 grid, hipStream_t stream) {
     // calls of at most 64 tokens on the production layout (GEMM-layout weights, k8-major activations)
     if constexpr (PACKED && XDIRECT) {
-        if (k.T <= GN / 2 && k.narrow_tile) return k.T <= GN / 4 ? launch_gemm_reg<TYPE, 1>(k, grid, stream) : launch_gemm_reg<TYPE, 2>(k, grid, stream);
+        if (k.T <= GN / 2 && k.narrow_tile) return k.T <= GN / 4 ? launch_gemm_reg<TYPE, 1, REG_DENSE>(k, grid, stream) : launch_gemm_reg<TYPE, 2, REG_DENSE>(k, grid, stream);
     }
     return k.ksplit > 1 ? launch_gemm_kernel<TYPE, PACKED, XDIRECT, true>(k, grid, stream) : launch_gemm_kernel<TYPE, PACKED, XDIRECT, false>(k, grid, stream);
 }
@@ -1090,10 +1107,17 @@ int gemm_kquant(const GemmArgs &a, hipStream_t stream) {
     if (a.K % QK_K || a.M % 4 || a.ldx % 8 || a.ldy % 4 || (a.residual && a.ldres % 4))
         return fail(MESH_ERR_INVALID, "gemm: shape M=%d K=%d not supported (K %% 256, M %% 4)", a.M, a.K);
     if ((reinterpret_cast<uintptr_t>(a.X) | reinterpret_cast<uintptr_t>(a.Y)) & 15) return fail(MESH_ERR_INVALID, "gemm: X and Y must be 16-byte aligned");
-    if (gemm_tile_takes(a)) return gemm_tile(a, stream);
+    if (!a.norm_part && gemm_tile_takes(a)) return gemm_tile(a, stream);
     GemmArgs k = a;
     k.M_pad = (a.M + TILE_ROWS - 1) / TILE_ROWS * TILE_ROWS;
     const int row_blocks = a.y16_k8 ? (a.M + GM / 2 - 1) / (GM / 2) : (a.M + GM - 1) / GM;
+    if (a.norm_part) {
+        if (!a.y16_k8 || !a.Wp || !a.x_k8 || a.T > GN / 4 || a.tiles || a.norm_parts < 1) return fail(MESH_ERR_INVALID, "gemm: a norm hand-over needs a SwiGLU pair, the GEMM layout and at most 32 tokens");
+        if (a.type != MESH_Q4_K && a.type != MESH_Q6_K) return fail(MESH_ERR_UNSUPPORTED, "gemm: no MFMA kernel for ggml type %d", a.type);
+        k.ksplit = 1;
+        const dim3 g((unsigned)row_blocks);
+        return a.type == MESH_Q4_K ? launch_gemm_reg<MESH_Q4_K, 1, REG_NORM>(k, g, stream) : launch_gemm_reg<MESH_Q6_K, 1, REG_NORM>(k, g, stream);
+    }
     if (a.tiles) {
         // expert launch: one workgroup row per tile of the list (those past *n_tiles leave at once)
         if (!a.Wp || !a.x_k8 || !a.n_tiles || a.max_tiles <= 0 || a.n_seg > 1 || a.bias || a.residual || a.rope.pos || a.expert_stride % 16)

@@ -56,7 +56,14 @@ struct GemmArgs {
     const int32_t *tiles = nullptr, *n_tiles = nullptr;
     size_t expert_stride = 0;
     int max_tiles = 0;
+    // SwiGLU pair of a call of at most 32 tokens, x_k8: the consumer side of SkinnyF16Args' norm hand-over (X not yet divided by the
+    // token's rms, its sums of squares by [workgroup][16], from 17 tokens on [workgroup][32]).  Not split along K.
+    const float *norm_part = nullptr;
+    int norm_parts = 0;
+    float norm_eps = 0.f;
 };
+// workgroups of the launch of such a pair
+inline int gemm_pair_row_blocks(int64_t M) { return (int)((M + 63) / 64); }
 int gemm_kquant(const GemmArgs &a, hipStream_t stream);
 // Number of K slices gemm_kquant will use for this launch (1: not split).
 int gemm_split_count(const GemmArgs &a);

@@ -907,7 +907,20 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
         const bool next_fused = nf && Ln && layer_is_kquant_dense(*Ln) && Ln->w_gate.type == Ln->w_up.type &&
                                 gemm_skinny_f16_workgroups(da) >= 1 && gemm_skinny_f16_workgroups(da) <= SKINNY_F16_NORM_PARTS_MAX;
         ProfScope ps(s, MESH_PROF_GEMV);
-        if ((rc = gemm_skinny_f16(ga, stream)) != MESH_OK) return rc;
+        // From 17 tokens on the skinny GEMM walks two blocks of columns per weight tile; the register-formed tile has all 32 in its
+        // fragment.  Gate / up of 28672 x 4096 at 32 tokens 34 -> 24 us, of 55296 x 5120 70 -> 49; below (16 tokens) 23 against 23,
+        // and with the rest of the layer 691 against 684 us for eight layers.  Blocks: about one workgroup per CU; fewer would leave
+        // CUs idle, or split K and lose the epilogue.
+        if (ffn_norm_fused && L.gate_up_gemm && T >= s->tune.reg_min_tokens && T <= 32 && gemm_pair_row_blocks(FF) >= s->tune.reg_min_blocks) {
+            GemmArgs g;
+            g.Wp = L.gate_up_gemm; g.type = L.w_gate.type;
+            g.M = FF; g.K = E; g.T = T;
+            g.X = nx; g.x_k8 = true;
+            g.y16_k8 = f16ffn; g.sat = s->f16_sat;
+            g.norm_part = s->norm_part; g.norm_parts = s->norm_parts; g.norm_eps = hp.rms_eps;
+            rc = gemm_kquant(g, stream);
+        } else rc = gemm_skinny_f16(ga, stream);
+        if (rc != MESH_OK) return rc;
         if (next_fused) {
             da.norm_out.norm_w = static_cast<const float *>(Ln->attn_norm.data); da.norm_out.x16 = nx; da.norm_out.part = s->norm_part;
         }

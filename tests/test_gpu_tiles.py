@@ -149,3 +149,34 @@ def test_kquant_products_of_few_tokens(tmp_path, shape, tokens):
     assert np.linalg.norm(got[1] - want) / norm < 3e-3, (shape, tokens)
     # the same weights and inputs, sums along K met in another order
     assert np.linalg.norm(got[1] - got[0]) / norm < 1e-3, (shape, tokens)
+
+
+@pytest.mark.parametrize("shape,tokens", [
+    ((256, 2, 1, 256), 17),         # four steps along K, one per group; two columns' worth past the first block
+    ((768, 6, 2, 2816), 32),        # twelve steps; all columns
+    ((512, 4, 1, 33024), 23),       # more row blocks than compute units: two groups
+    ((512, 4, 1, 768), 5),          # one block of 16 columns
+])
+def test_gate_up_of_a_decode_batch(tmp_path, shape, tokens):
+    """A batch of single steps through two layers with gate / up on the register-formed tile, the norm before it handed over, against
+    the oracle and against the f16 skinny GEMM."""
+    m = mesh()
+    cfg = dict(kquant(*shape), n_layer=2)
+    path = str(tmp_path / "model.gguf")
+    tensors = models.write_model(path, cfg, [0, 1], seed=13)
+    x = np.random.Generator(np.random.PCG64(tokens)).standard_normal((tokens, cfg["n_embd"])).astype(np.float32)
+    pos, seq = np.zeros(tokens, np.int32), np.arange(tokens, dtype=np.int32)
+    want = StageOracle(cfg, tensors, 0, 2, 64, n_seq_max=tokens, blas=True).forward(x, pos, seq=seq)
+    st = m.Stage(path, 0, 2, n_ctx=64, n_seq_max=tokens, n_batch_max=32)
+    got = {}
+    for least in (1, 33):
+        ses = st.session(reg_min_tokens=least, reg_min_blocks=1)
+        got[least] = ses.decode(x, pos, seq=seq).view(np.float32).reshape(want.shape)
+        assert ses.f16_saturations() == 0
+        ses.close()
+    st.close()
+    norm = np.linalg.norm(want)
+    # f16 activations over two layers: 11 bits in the inputs of eight products
+    assert np.linalg.norm(got[1] - want) / norm < 4e-3, (shape, tokens)
+    # the same inputs and weights of one rounding each, formed in two ways and summed in two orders
+    assert np.linalg.norm(got[1] - got[33]) / norm < 2e-3, (shape, tokens)
