@@ -388,26 +388,15 @@ int hybrid_open(const char *folder, int layer_begin, int layer_end, const mesh_s
         }
         st->tok_embd.data = hm.embed; st->tok_embd.K = E; st->tok_embd.M = s.vocab;
     }
-    // second copies for the large tile
-    if (hm.act == ACT_BF16 && st->tune.tile_copies && st->n_batch_max >= st->tune.linear_tile_min_tokens) {
-        size_t total = 0;
-        auto each = [&](auto fn) -> int {
-            for (HybridLayer &L : hm.layers)
-                for (LinearWeight *w : {&L.in, &L.out, &L.up, &L.down, &L.side_gate, &L.side_proj, &L.uq, &L.ukv})
-                    if (w->present() && (rc = fn(*w)) != MESH_OK) return rc;
-            return MESH_OK;
-        };
-        (void)each([&](LinearWeight &w) -> int { total += linear_blocks_bytes(w); return MESH_OK; });
-        if (stage_copies_fit(total) &&
-            (rc = each([&](LinearWeight &w) -> int {
-                 void *p = nullptr;
-                 if ((rc = ld.dev_alloc(&p, linear_blocks_bytes(w))) != MESH_OK || (rc = linear_make_blocks(w, static_cast<uint16_t *>(p), nullptr)) != MESH_OK) return rc;
-                 w.blocks = static_cast<const uint16_t *>(p);
-                 return MESH_OK;
-             })) != MESH_OK)
-            return rc;
-    }
     MESH_HIP_TRY(hipDeviceSynchronize());
+    // weights in the large tile's layout
+    if (hm.act == ACT_BF16 && st->tune.tile_copies && st->n_batch_max >= st->tune.linear_tile_min_tokens) {
+        std::vector<SecondCopies::Item> items;
+        for (HybridLayer &L : hm.layers)
+            for (LinearWeight *w : {&L.in, &L.out, &L.up, &L.down, &L.side_gate, &L.side_proj, &L.uq, &L.ukv})
+                if (w->present()) items.push_back({&w->blocks, linear_blocks_bytes(*w), [w](void *p) { return linear_make_blocks(*w, static_cast<uint16_t *>(p), nullptr); }});
+        if ((rc = st->copies.make(items)) != MESH_OK) return rc;
+    }
     return MESH_OK;
 }
 

@@ -180,7 +180,7 @@ static int launch_tile_layout(const uint16_t *w, const LinearWeight &W, const vo
 }
 template <LinearOut OUT>
 static int launch_tile(const LinearWeight &W, const void *x, int T, void *y, int ldy, int M, const GtPlan &p, size_t stride, hipStream_t stream) {
-    return W.blocks ? launch_tile_layout<OUT, GT_BLOCKS>(W.blocks, W, x, T, y, ldy, M, p, stride, stream) : launch_tile_layout<OUT, GT_ROWS>(W.w, W, x, T, y, ldy, M, p, stride, stream);
+    return W.blocks ? launch_tile_layout<OUT, GT_BLOCKS>(static_cast<const uint16_t *>(W.blocks), W, x, T, y, ldy, M, p, stride, stream) : launch_tile_layout<OUT, GT_ROWS>(W.w, W, x, T, y, ldy, M, p, stride, stream);
 }
 
 static bool linear_ok(const LinearWeight &W, const void *x, int T, const void *y, int ldy) {

@@ -15,7 +15,7 @@ inline size_t act_bytes(ActType a) { return a == ACT_BF16 ? 2 : 4; }
 constexpr int LINEAR_ROW_PAD = 128, LINEAR_K_PAD = 64;
 struct LinearWeight {
     const uint16_t *w = nullptr;
-    const uint16_t *blocks = nullptr;      // optional second copy in the large tile's layout (gemm_tile.hpp: GT_BLOCKS)
+    void *blocks = nullptr;                // optional second copy in the large tile's layout (gemm_tile.hpp: GT_BLOCKS)
     int M = 0, K = 0, Mp = 0, Kp = 0;
     bool present() const { return w != nullptr; }
 };

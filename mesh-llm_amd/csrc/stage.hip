@@ -207,38 +207,30 @@ struct Loader {
         }
         return MESH_OK;
     }
-    // f16 copies for the large tile of what the dense layers hold in the GEMM layout: their bytes, or (bytes null) the copies.  The
-    // attention projections of mixture-of-experts layers keep the GEMM layout alone: the copies took 2-3% off their chunks.
-    int tile_copies(size_t *bytes) {
-        int rc;
-        auto one = [&](void **dst, size_t n, auto fill) -> int {
-            if (bytes) { *bytes += n; return MESH_OK; }
-            void *p = nullptr;
-            if ((rc = dev_alloc(&p, n)) != MESH_OK || (rc = fill(static_cast<uint8_t *>(p))) != MESH_OK) return rc;
-            *dst = p;
-            return MESH_OK;
-        };
-        auto copy = [&](const DevTensor &t, uint8_t *p) { return gemm_tile_copy(t.type, t.gemm, p, t.M, t.K, false, nullptr); };
+    // f16 copies for the large tile of what the dense layers hold in the GEMM layout.  The attention projections of
+    // mixture-of-experts layers keep the GEMM layout alone: the copies took 2-3% off their chunks.
+    std::vector<SecondCopies::Item> tile_copies() {
+        std::vector<SecondCopies::Item> items;
+        auto copy = [](const DevTensor *t, uint8_t *p) { return gemm_tile_copy(t->type, t->gemm, p, t->M, t->K, false, nullptr); };
         for (LayerWeights &L : st.layers) {
             if (!L.gate_up_gemm) continue;
-            const DevTensor &q = L.wq, &k = L.wk, &v = L.wv;
-            if (q.gemm && k.gemm && v.gemm && q.K == k.K && q.K == v.K && q.M % 128 == 0 && k.M % 128 == 0) {
-                const size_t qb = gemm_tile_bytes(q.M, q.K), kb = gemm_tile_bytes(k.M, k.K);
-                if ((rc = one(&L.qkv_tile, qb + kb + gemm_tile_bytes(v.M, v.K), [&](uint8_t *p) -> int {
-                         int r;
-                         if ((r = copy(q, p)) != MESH_OK || (r = copy(k, p + qb)) != MESH_OK) return r;
-                         return copy(v, p + qb + kb);
-                     })) != MESH_OK)
-                    return rc;
+            const DevTensor *q = &L.wq, *k = &L.wk, *v = &L.wv;
+            if (q->gemm && k->gemm && v->gemm && q->K == k->K && q->K == v->K && q->M % 128 == 0 && k->M % 128 == 0) {
+                const size_t qb = gemm_tile_bytes(q->M, q->K), kb = gemm_tile_bytes(k->M, k->K);
+                items.push_back({&L.qkv_tile, qb + kb + gemm_tile_bytes(v->M, v->K), [=](void *d) -> int {
+                                     uint8_t *p = static_cast<uint8_t *>(d);
+                                     int rc;
+                                     if ((rc = copy(q, p)) != MESH_OK || (rc = copy(k, p + qb)) != MESH_OK) return rc;
+                                     return copy(v, p + qb + kb);
+                                 }});
             }
             for (DevTensor *t : {&L.wo, &L.w_down})
-                if (t->gemm && (rc = one(&t->tile, gemm_tile_bytes(t->M, t->K), [&](uint8_t *p) -> int { return copy(*t, p); })) != MESH_OK) return rc;
-            if ((rc = one(&L.gate_up_tile, gemm_tile_pair_bytes(L.w_gate.M, L.w_gate.K), [&](uint8_t *p) -> int {
-                    return gemm_tile_copy(L.w_gate.type, L.gate_up_gemm, p, L.w_gate.M, L.w_gate.K, true, nullptr);
-                })) != MESH_OK)
-                return rc;
+                if (t->gemm) items.push_back({&t->tile, gemm_tile_bytes(t->M, t->K), [=](void *d) { return copy(t, static_cast<uint8_t *>(d)); }});
+            const LayerWeights *l = &L;
+            items.push_back({&L.gate_up_tile, gemm_tile_pair_bytes(L.w_gate.M, L.w_gate.K),
+                             [l](void *d) { return gemm_tile_copy(l->w_gate.type, l->gate_up_gemm, d, l->w_gate.M, l->w_gate.K, true, nullptr); }});
         }
-        return MESH_OK;
+        return items;
     }
     // the expert matrices of a mixture-of-experts layer, for prefill chunks (expert launches of the large-tile GEMM): every
     // expert's gate / up pair and down projection in the GEMM layout, experts back to back
@@ -273,14 +265,6 @@ int stage_select_device(const mesh_stage_opts *opts, mesh_stage *st) {
     if (mesh_device_count() < 1) return fail(MESH_ERR_DEVICE, "mesh_stage_open: no GPU available");
     MESH_HIP_TRY(hipGetDevice(&st->device));
     return MESH_OK;
-}
-
-// Second copies of the weights that the large tile reads faster are kept where they take at most an eighth of the memory that is
-// free once the stage is loaded: the rest belongs to the caller's sessions.
-bool stage_copies_fit(size_t bytes) {
-    size_t free_bytes = 0, total = 0;
-    if (hipMemGetInfo(&free_bytes, &total) != hipSuccess) { (void)hipGetLastError(); return false; }
-    return bytes <= free_bytes / 8;
 }
 
 // what every kind of model takes from the options
@@ -389,10 +373,6 @@ int stage_open(const char *path, int layer_begin, int layer_end, const mesh_stag
             if ((rc = ld.load("token_embd.weight", st->output, E, -1, 1, true, true, false)) != MESH_OK) return rc;
         }
     }
-    if (ld.gemm_layout && st->tune.tile_copies && st->n_batch_max >= st->tune.tile_min_tokens) {
-        size_t bytes = 0;
-        if ((rc = ld.tile_copies(&bytes)) != MESH_OK || (stage_copies_fit(bytes) && (rc = ld.tile_copies(nullptr)) != MESH_OK)) return rc;
-    }
     // inverse frequencies by ggml's f32 recurrence: theta_i = theta_{i-1} * base^(-2/n_rot)
     {
         std::vector<float> inv(hp.n_rot / 2);
@@ -405,6 +385,8 @@ int stage_open(const char *path, int layer_begin, int layer_end, const mesh_stag
         MESH_HIP_TRY(hipMemcpy(p, inv.data(), inv.size() * sizeof(float), hipMemcpyHostToDevice));
     }
     MESH_HIP_TRY(hipDeviceSynchronize());
+    // (last: what the stage cannot do without is allocated by now)
+    if (ld.gemm_layout && st->tune.tile_copies && st->n_batch_max >= st->tune.tile_min_tokens && (rc = st->copies.make(ld.tile_copies())) != MESH_OK) return rc;
     *out = st.release();
     return MESH_OK;
 }

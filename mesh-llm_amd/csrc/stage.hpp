@@ -10,6 +10,7 @@
 #include "hybrid.hpp"
 #include "mesh_common.hpp"
 #include "moe.hpp"
+#include "second_copies.hpp"
 #include "tuning.hpp"
 
 namespace mesh {
@@ -71,7 +72,6 @@ int session_attention(mesh_session *s, int layer, const float *d_q, const mesh_b
 int stage_decode_dev(mesh_session *s, const mesh_batch *b, const void *d_in, int in_fmt, void *d_out, int out_fmt, size_t out_cap, size_t *out_len);
 // shared by the runners
 int stage_select_device(const mesh_stage_opts *opts, mesh_stage *st);
-bool stage_copies_fit(size_t bytes);
 int sess_alloc(mesh_session *s, void **p, size_t bytes);
 int attn_splits_for(const Tuning &tune, int T, int n_kv, int max_keys, bool quantised);
 // names the kernel class of the launches made while it lives (mesh_session_profile)
@@ -96,6 +96,7 @@ struct mesh_stage {
     std::vector<void *> allocations;
     size_t gemm_layout_bytes = 0; // extra HBM held by the GEMM-layout copies
     size_t weight_bytes = 0;      // GGUF bytes of everything resident (the algorithmic weight traffic of one decode step)
+    mesh::SecondCopies copies;    // of the projections, for the large tile: what DevTensor::tile, LayerWeights::*_tile and LinearWeight::blocks point to
     float *rope_inv_freq = nullptr;   // [n_rot/2] f32, theta_scale^i by the f32 recurrence ggml uses
     ~mesh_stage();
 };
