@@ -278,7 +278,8 @@ int mesh_session_f16_saturations(mesh_session *session, uint64_t *count);
  *     skinny_min_tokens=0  calls of at least this many (and fewer than the above) run the skinny MFMA GEMM;
  *                          0 = 4 with skinny_f16, 5 without
  *     tile_copies=1        second copies of the projections for prefill-sized calls (bf16 models: as many bytes again; K-quant models:
- *                          2 bytes per weight, f16), where they take at most an eighth of the GPU's free memory
+ *                          2 bytes per weight, f16), where all of them take at most an eighth of the GPU's free memory; given back when
+ *                          a stage, session, weight or buffer that this process opens on the GPU finds no other room
  *   session level:
  *     gemm_splitk=1        GEMM launches too narrow to fill the chip split K over workgroups
  *     chunk_kv16=1         long prefill chunks over a quantised cache decode a layer's rows once into an f16 copy

@@ -5,6 +5,7 @@
 #include <mutex>
 
 #include "mesh_common.hpp"
+#include "second_copies.hpp"
 
 namespace mesh {
 
@@ -34,7 +35,7 @@ struct DevScratch {
     void *p = nullptr;
     ~DevScratch() { if (p) (void)hipFree(p); }
     int alloc(size_t bytes) {
-        hipError_t e = hipMalloc(&p, bytes ? bytes : 1);
+        hipError_t e = device_alloc(&p, bytes ? bytes : 1);
         if (e != hipSuccess) {
             p = nullptr;
             return fail(e == hipErrorOutOfMemory ? MESH_ERR_NOMEM : MESH_ERR_DEVICE, "hipMalloc(%zu) failed: %s", bytes,

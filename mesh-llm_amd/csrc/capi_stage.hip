@@ -28,7 +28,7 @@ int mesh_weight_upload(int type, const void *host_data, int64_t n_rows, int64_t 
     w->gguf_bytes = (size_t)(rb * n_rows);
     w->t.tiled = type_is_tiled(type);
     w->t.bytes = w->t.tiled ? (size_t)tiled_bytes(type, n_rows, row_len) : w->gguf_bytes;
-    hipError_t e = hipMalloc(&w->t.data, w->t.bytes);
+    hipError_t e = device_alloc(&w->t.data, w->t.bytes);
     if (e != hipSuccess) {
         const size_t wanted = w->t.bytes;
         delete w;
@@ -40,7 +40,7 @@ int mesh_weight_upload(int type, const void *host_data, int64_t n_rows, int64_t 
         if (e != hipSuccess) rc = fail(MESH_ERR_DEVICE, "mesh_weight_upload: copy failed: %s", hipGetErrorString(e));
     } else {
         void *tmp = nullptr;
-        e = hipMalloc(&tmp, w->gguf_bytes);
+        e = device_alloc(&tmp, w->gguf_bytes);
         if (e != hipSuccess) rc = fail(MESH_ERR_NOMEM, "mesh_weight_upload: hipMalloc(%zu) failed", w->gguf_bytes);
         if (rc == MESH_OK && (e = hipMemcpy(tmp, host_data, w->gguf_bytes, hipMemcpyHostToDevice)) != hipSuccess)
             rc = fail(MESH_ERR_DEVICE, "mesh_weight_upload: copy failed: %s", hipGetErrorString(e));
@@ -69,7 +69,7 @@ int mesh_weight_download(const mesh_weight *w, void *host_data) {
         return MESH_OK;
     }
     void *tmp = nullptr;
-    MESH_HIP_TRY(hipMalloc(&tmp, w->gguf_bytes));
+    MESH_HIP_TRY(device_alloc(&tmp, w->gguf_bytes));
     int rc = unpack_tiled(w->t.type, w->t.data, tmp, w->t.M, w->t.K, nullptr);
     if (rc == MESH_OK && hipMemcpy(host_data, tmp, w->gguf_bytes, hipMemcpyDeviceToHost) != hipSuccess)
         rc = fail(MESH_ERR_DEVICE, "mesh_weight_download: copy failed");
@@ -277,7 +277,7 @@ static int kv_xfer(mesh_session *s, int layer, int seq_id, int pos0, int n_pos, 
     const int hd = (int)hp.head_dim, nkv = (int)hp.n_head_kv;
     const size_t bytes = (size_t)n_pos * nkv * hd * 2;
     uint16_t *tmp = nullptr;
-    MESH_HIP_TRY(hipMalloc(reinterpret_cast<void **>(&tmp), bytes));
+    MESH_HIP_TRY(device_alloc(reinterpret_cast<void **>(&tmp), bytes));
     int rc = MESH_OK;
     for (int which = 0; which < 2 && rc == MESH_OK; ++which) {
         const size_t lb = which ? s->v_layer_bytes : s->k_layer_bytes;

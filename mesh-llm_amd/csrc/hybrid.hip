@@ -136,6 +136,7 @@ uint64_t hybrid_graph_key(const mesh_session *s, int T, int max_keys) {
         if (L.spec.mixer.kind == MIXER_ATTENTION) mix((uint64_t)layer_splits(s, L.spec.mixer, T, max_keys));
         if (L.spec.mixer.kind == MIXER_LATENT) mix((uint64_t)latent_layer_splits(s, L.latent, T, max_keys) << 1 | (s->chunk_pos0 >= 0 ? 1 : 0));
     }
+    mix(s->stage->copies.present() ? 1 : 0);
     if (s->stage->hybrid->has_chunks) mix(((uint64_t)s->hybrid->chunks.n_chunks << 32) | (uint64_t)s->hybrid->chunks.n_runs);
     return key;
 }

@@ -19,7 +19,7 @@ struct FolderLoader {
     mesh_stage &st;
 
     int dev_alloc(void **p, size_t bytes) {
-        hipError_t e = hipMalloc(p, bytes ? bytes : 16);
+        hipError_t e = device_alloc(p, bytes ? bytes : 16);
         if (e != hipSuccess) return fail(e == hipErrorOutOfMemory ? MESH_ERR_NOMEM : MESH_ERR_DEVICE, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
         st.allocations.push_back(*p);
         return MESH_OK;

@@ -4,6 +4,7 @@
 
 #include <cstdio>
 
+#include "../second_copies.hpp"
 #include "rpc_buffers.hpp"
 
 namespace mesh_rpc {
@@ -25,7 +26,7 @@ class HipBuffers final : public BufferBackend {
     bool device_memory(int dev, uint64_t *free_bytes, uint64_t *total_bytes) override {
         size_t f = 0, t = 0;
         if (!use(dev) || hipMemGetInfo(&f, &t) != hipSuccess) return false;
-        *free_bytes = f;
+        *free_bytes = f + mesh::second_copies_bytes(dev);        // (given back when an allocation needs the room)
         *total_bytes = t;
         return true;
     }
@@ -36,10 +37,7 @@ class HipBuffers final : public BufferBackend {
     }
     void *alloc(int dev, uint64_t size) override {
         void *p = nullptr;
-        if (!use(dev) || hipMalloc(&p, size ? size : 1) != hipSuccess) {
-            (void)hipGetLastError();
-            return nullptr;
-        }
+        if (!use(dev) || mesh::device_alloc(&p, size ? size : 1) != hipSuccess) return nullptr;
         return p;
     }
     void release(int dev, void *base) override {

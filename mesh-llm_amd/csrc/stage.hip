@@ -105,7 +105,7 @@ struct Loader {
     ~Loader() { if (staging) (void)hipFree(staging); }
 
     int dev_alloc(void **p, size_t bytes) {
-        hipError_t e = hipMalloc(p, bytes ? bytes : 16);
+        hipError_t e = device_alloc(p, bytes ? bytes : 16);
         if (e != hipSuccess) return fail(e == hipErrorOutOfMemory ? MESH_ERR_NOMEM : MESH_ERR_DEVICE, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
         st.allocations.push_back(*p);
         return MESH_OK;
@@ -144,7 +144,7 @@ struct Loader {
         if (staging_bytes < ti->nbytes) {
             if (staging) (void)hipFree(staging);
             staging = nullptr;
-            hipError_t e = hipMalloc(&staging, ti->nbytes);
+            hipError_t e = device_alloc(&staging, ti->nbytes);
             if (e != hipSuccess) { staging_bytes = 0; return fail(MESH_ERR_NOMEM, "hipMalloc(%llu) for load staging failed", (unsigned long long)ti->nbytes); }
             staging_bytes = ti->nbytes;
         }
@@ -395,7 +395,7 @@ static bool layer_is_kquant_dense(const LayerWeights &L);
 
 // ------------------------------------------------------------------------------------------------ session
 int sess_alloc(mesh_session *s, void **p, size_t bytes) {
-    hipError_t e = hipMalloc(p, bytes ? bytes : 16);
+    hipError_t e = device_alloc(p, bytes ? bytes : 16);
     if (e != hipSuccess) return fail(e == hipErrorOutOfMemory ? MESH_ERR_NOMEM : MESH_ERR_DEVICE, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
     s->allocations.push_back(*p);
     return MESH_OK;
@@ -1251,8 +1251,8 @@ static int validate_batch(const mesh_session *s, const mesh_batch *b, int *max_k
 }
 
 // run_layers, replayed from a captured graph for decode-sized batches.  The launches depend on T, on the KV split count
-// (a function of the deepest position) and on whether an expert mask is set; everything else they read is device
-// memory at fixed addresses (hidden state, positions, caches).  The first use of a key runs eagerly (which also
+// (a function of the deepest position), on whether an expert mask is set and on whether the stage holds second copies
+// of its weights; everything else they read is device memory at fixed addresses (hidden state, positions, caches).  The first use of a key runs eagerly (which also
 // finishes every lazy initialisation), the second is captured, later ones are replays.
 constexpr int GRAPH_MAX_TOKENS = 32;
 constexpr size_t GRAPH_MAX_ENTRIES = 96;
@@ -1264,7 +1264,7 @@ static int run_layers_graphed(mesh_session *s, int T, int max_keys) {
     const mesh_stage *st = s->stage;
     if (s->chunk_pos0 >= 0 && (T >= PREFILL_MIN_TOKENS || (st->hybrid && T >= s->tune.latent_chunk_min_tokens))) return run_layers(s, T, max_keys);
     const int n_splits = st->hybrid ? 0 : attn_splits_for(s->tune, T, (int)st->hp.n_head_kv, max_keys, st->k_type != MESH_F16);
-    const uint64_t key = st->hybrid ? hybrid_graph_key(s, T, max_keys) : (uint64_t)T | ((uint64_t)n_splits << 8) | ((uint64_t)(s->expert_mask_on ? 1 : 0) << 20);
+    const uint64_t key = st->hybrid ? hybrid_graph_key(s, T, max_keys) : (uint64_t)T | ((uint64_t)n_splits << 8) | ((uint64_t)(s->expert_mask_on ? 1 : 0) << 20) | ((uint64_t)(st->copies.present() ? 1 : 0) << 21);
     auto it = s->graphs.find(key);
     if (it == s->graphs.end()) {
         if (s->graphs.size() >= GRAPH_MAX_ENTRIES) return run_layers(s, T, max_keys);
@@ -1338,6 +1338,7 @@ static int decode_core(mesh_session *s, const mesh_batch *b, const int32_t *ids,
     if (out_cap < need) return fail(MESH_ERR_INVALID, "mesh_stage_decode: output needs %zu bytes, capacity is %zu", need, out_cap);
     MESH_HIP_TRY(hipSetDevice(st->device));
     hipStream_t stream = s->stream;
+    const auto copies_in_use = st->copies.in_use();
 
     // a run of consecutive positions of one sequence (a prefill chunk) can use the chunk attention kernel
     s->chunk_pos0 = b->pos[0];
