@@ -1,0 +1,106 @@
+"""Which kernels the calls of test_gpu_tiles.py and test_gpu_fullsize.py reach, as the built library launches them (host memory, no GPU)."""
+import os
+import sys
+import tempfile
+
+import numpy as np
+import pytest
+
+sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
+import models
+import nadosun_util as N
+import test_gpu_tiles as tiles
+from hip_host_util import call
+from util import mesh
+
+Q4_K, Q6_K = 12, 14
+ROWS, SWIGLU, PARTIAL = 0, 1, 2                     # gemm_f16_kernel's first argument
+DENSE, SPLIT, NORM = 0, 1, 3                        # gemm_reg_kernel's third
+
+
+def products(host):
+    return [(n, g) for n, g, _ in host.launches() if n.startswith(("gemm_", "linear_")) and "epilogue" not in n]
+
+
+def kquant_products(host, cfg, layers, tokens, decode=False, tuning=None, options=None):
+    m = mesh()
+    host.memory(1 << 37)
+    n_seq = tokens if decode else 1
+    with tempfile.TemporaryDirectory() as d:
+        path = os.path.join(d, "model.gguf")
+        models.write_model(path, cfg, layers, seed=1, fast=True)
+        st = m.Stage(path, layers[0], layers[-1] + 1, n_ctx=max(tokens, 64), n_seq_max=n_seq, n_batch_max=max(tokens, 32 if decode else 512), tuning=tuning)
+    ses = st.session(**(options or {}))
+    host.launches()
+    pos, seq = (np.zeros(tokens, np.int32), np.arange(tokens)) if decode else (np.arange(tokens), None)
+    ses.decode(np.zeros((tokens, cfg["n_embd"]), np.float32), pos, seq=seq)
+    return products(host)
+
+
+def bf16_products(host, width, ff, tokens, copies):
+    m = mesh()
+    host.memory(1 << 37)
+    cfg = N.config(64, width, 8, [N.attention(2, 1, 64, 50, ff=ff)])
+    with tempfile.TemporaryDirectory() as d:
+        st = m.Stage(N.write_folder(d, cfg, N.random_weights(cfg, 3)), 0, -1, n_ctx=512, n_seq_max=4, n_batch_max=512, tuning={"tile_copies": copies})
+    ses = st.session()
+    host.launches()
+    ses.decode(np.zeros(tokens, np.int32), np.arange(tokens), in_fmt=m.TOKENS)
+    return products(host)
+
+
+@pytest.mark.parametrize("copies", [0, 1])
+@pytest.mark.parametrize("case,up,down", tiles.BF16_CASES)
+def test_products_of_many_tokens(case, up, down, copies):
+    width, ff, tokens = case
+    got = call(bf16_products, width=width, ff=ff, tokens=tokens, copies=copies)
+    big = [(n, g) for n, g in got if n.startswith("linear_tile_kernel")]
+    # the feed-forward's: the one of most rows, and what follows it
+    at = max(range(len(big)), key=lambda i: big[i][1][0] * int(big[i][0][:-1].split(",")[2])) if ff > 200 else 2
+    for (name, grid), (wm, wt, slices), rows in zip(big[at:at + 2], (up, down), (ff, width)):
+        assert name == "linear_tile_kernel<0,%d,%d,%d>" % (0 if copies else 1, wm, wt)
+        assert grid[:2] == [-(-rows // (64 * wm)) * -(-tokens // (64 * wt)), slices]
+
+
+@pytest.mark.parametrize("case", tiles.KQUANT_MANY_CASES)
+def test_kquant_products_of_many_tokens(case):
+    (width, heads, kv, ff), tokens, *plans = case
+    got = call(kquant_products, cfg=tiles.kquant(*case[0]), layers=[0], tokens=tokens)
+    assert len(got) == 4
+    for i, ((name, grid), (wm, wt, slices), rows) in enumerate(zip(got, plans, ((heads + 2 * kv) * 128, width, 2 * ff, width))):
+        out = PARTIAL if slices > 1 else SWIGLU if i == 2 else ROWS
+        assert name == "gemm_f16_kernel<%d,%d,%d>" % (out, wm, wt), i
+        assert grid[:2] == [-(-rows // (64 * wm)) * -(-tokens // (64 * wt)), slices], i
+
+
+@pytest.mark.parametrize("case", tiles.KQUANT_FEW_CASES)
+def test_kquant_products_of_few_tokens(case):
+    (width, heads, kv, ff), tokens, gate_up, down = case
+    got = call(kquant_products, cfg=tiles.kquant(*case[0]), layers=[0], tokens=tokens)[-2:]
+    for (name, grid), (columns, groups, slices), type_, rows in zip(got, (gate_up, down), (Q4_K, Q6_K), (2 * ff, width)):
+        assert name == "gemm_reg_kernel<%d,%d,%d,%d>" % (type_, columns, SPLIT if slices > 1 else DENSE, groups)
+        assert grid == [rows // 128, 1, slices]
+    # (the other side of the test's comparison)
+    other = call(kquant_products, cfg=tiles.kquant(*case[0]), layers=[0], tokens=tokens, options={"gemm_narrow": 0})[-2:]
+    assert [n.split("<")[0] for n, _ in other] == ["gemm_kq_kernel"] * 2
+
+
+@pytest.mark.parametrize("case", tiles.DECODE_BATCH_CASES)
+def test_gate_up_of_a_decode_batch(case):
+    (width, heads, kv, ff), tokens, groups = case
+    cfg = dict(tiles.kquant(*case[0]), n_layer=2)
+    got = call(kquant_products, cfg=cfg, layers=[0, 1], tokens=tokens, decode=True, options={"reg_min_tokens": 1, "reg_min_blocks": 1})
+    assert [g for n, g in got if n == "gemm_reg_kernel<%d,1,%d,%d>" % (Q4_K, NORM, groups)] == [[ff // 64, 1, 1]] * 2
+    other = call(kquant_products, cfg=cfg, layers=[0, 1], tokens=tokens, decode=True, options={"reg_min_tokens": 33, "reg_min_blocks": 1})
+    assert not any(n.startswith("gemm_reg") for n, _ in other)
+
+
+@pytest.mark.parametrize("name,layers,tokens", [("llama3-8b", [3], 2048), ("qwen2.5-32b", [7], 1664)])
+def test_prefill_of_the_full_sizes(name, layers, tokens):
+    """Over the copies the large tile of gemm_f16.hip; without them the 256-row tile, or with gemm_big=0 the 128 x 128 one."""
+    cfg = models.CONFIGS[name]
+    kernels = [{n.split("<")[0] for n, _ in call(kquant_products, cfg=cfg, layers=layers, tokens=tokens, tuning=t, options=o)}
+               for t, o in ((None, None), ({"tile_copies": 0}, None), ({"tile_copies": 0}, {"gemm_big": 0}))]
+    assert kernels[0] == {"gemm_f16_kernel"}
+    assert "gemm_big_kernel" in kernels[1] and kernels[1] <= {"gemm_big_kernel", "gemm_kq_kernel"}
+    assert kernels[2] == {"gemm_kq_kernel"}

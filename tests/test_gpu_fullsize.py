@@ -88,6 +88,23 @@ def test_c3_sixteen_layer_stage_decode_at_kv_depth_4095(c3_model):
     ses.close(); st.close()
 
 
+def big_and_small_tiles_agree(path, begin, end, x, ref, what):
+    """A stage without f16 copies: launches that fill the chip with 256 x 128 tiles take the big-tile kernel, with gemm_big=0 all keep
+    the 128 x 128 one.  Same fragments, same order along K: the same bits; and the oracle's."""
+    m = mesh()
+    T, E = x.shape
+    st = m.Stage(path, begin, end, n_ctx=T + 8, n_seq_max=1, n_batch_max=T, tuning={"tile_copies": 0})
+    ses = st.session()
+    got = ses.decode(x, np.arange(T)).view(np.float32).reshape(T, E)
+    r = rel_l2(got, ref)
+    report(what, r)
+    assert r <= NORTH_STAR
+    assert max(rel_l2(got[i], ref[i]) for i in range(T)) <= NORTH_STAR
+    ses.set_option("gemm_big", 0)
+    assert np.array_equal(got, ses.decode(x, np.arange(T)).view(np.float32).reshape(T, E))
+    ses.close(); st.close()
+
+
 def test_c3_prefill_2048_tokens_two_layers(c3_model):
     m = mesh()
     cfg, tensors, path = c3_model
@@ -103,12 +120,7 @@ def test_c3_prefill_2048_tokens_two_layers(c3_model):
     report("C3 layers 3-4, prefill 2048 tokens", r)
     assert r <= NORTH_STAR
     assert max(rel_l2(got[i], ref[i]) for i in range(T)) <= NORTH_STAR
-    # launches that fill the chip with 256 x 128 tiles take the big-tile kernel; with gemm_big=0 all keep the
-    # 128 x 128 one.  Same fragments, same order along K: the same bits.
-    ses.set_option("gemm_big", 0)
-    small = ses.decode(x, np.arange(T)).view(np.float32).reshape(T, 4096)
-    ses.set_option("gemm_big", 1)
-    assert np.array_equal(got, small)
+    big_and_small_tiles_agree(path, 3, 5, x, ref, "C3 layers 3-4, prefill 2048 tokens over the GEMM layout")
     # one decode token on top of the 2048 cached positions
     x1 = rng.standard_normal((1, 4096)).astype(np.float32)
     r1 = rel_l2(ses.decode(x1, [T]).view(np.float32), orc.forward(x1, [T]))
@@ -140,16 +152,15 @@ def test_c3_prefill_256_tokens_sixteen_layers(c3_model):
 
 
 def test_c4_long_prefill_takes_the_big_tile_with_biases(tmp_path):
-    """1664 tokens through one Qwen2.5-32B-shaped layer: every projection launch has enough 256-row tiles to fill the chip,
-    so the fused q / k / v launch (three matrices, biases, 40 + 8 + 8 row blocks) and the q6_K down projection run on the
-    256 x 128 tile; against the oracle, and bit for bit against the 128 x 128 kernel."""
+    """1664 tokens through one Qwen2.5-32B-shaped layer, over f16 copies of the weights and without them.  Every projection launch but
+    v's has enough 256-row tiles to fill the chip, so without copies the fused q / k launch (biases, 40 + 8 row blocks), o, gate / up and
+    the q6_K down projection run on the 256 x 128 tile; against the oracle, and bit for bit against the 128 x 128 kernel."""
     m = mesh()
     cfg = models.CONFIGS["qwen2.5-32b"]
     path = os.path.join(str(tmp_path), "c4l.gguf")
     tensors = models.write_model(path, cfg, [7], seed=42, fast=True)
     T, E = 1664, 5120
     st = m.Stage(path, 7, 8, n_ctx=T, n_seq_max=1, n_batch_max=T)
-    os.unlink(path)
     ses = st.session()
     orc = StageOracle(cfg, tensors, 7, 8, T, blas=True)
     rng = np.random.Generator(np.random.PCG64(1664))
@@ -157,12 +168,11 @@ def test_c4_long_prefill_takes_the_big_tile_with_biases(tmp_path):
     got = ses.decode(x, np.arange(T)).view(np.float32).reshape(T, E)
     ref = orc.forward(x, np.arange(T))
     r = rel_l2(got, ref)
-    report("C4 layer 7, prefill 1664 tokens (big tile)", r)
+    report("C4 layer 7, prefill 1664 tokens", r)
     assert r <= NORTH_STAR
-    ses.set_option("gemm_big", 0)
-    small = ses.decode(x, np.arange(T)).view(np.float32).reshape(T, E)
-    assert np.array_equal(got, small)
     ses.close(); st.close()
+    big_and_small_tiles_agree(path, 7, 8, x, ref, "C4 layer 7, prefill 1664 tokens over the GEMM layout (big tile)")
+    os.unlink(path)
 
 
 @pytest.mark.parametrize("kv", ["f16", "q8_0/q4_0"])
@@ -201,7 +211,7 @@ def test_c4_qwen25_32b_layers_wide_batches_and_prefill(tmp_path, kv):
         r = rel_l2(got, ref)
         report("C4 layers 7-8, %s KV, prefill chunk of %d tokens at %d" % (kv, T, pos0), r)
         assert r <= NORTH_STAR
-    # decode batches of 24 and 32 single-token sequences at KV depth 100 / 101: large-tile GEMM, K split over workgroups
+    # decode batches of 24 and 32 single-token sequences at KV depth 100 / 101: f16 skinny GEMM, gate / up on the register-formed tile
     nxt = [420] + [depth] * (n_seq - 1)
     for seqs in (list(range(1, 25)), list(range(32))):
         T = len(seqs)

@@ -20,15 +20,26 @@ pytestmark = pytest.mark.gpu
 BF16_LIMIT = 2e-2
 
 
-@pytest.mark.parametrize("width,ff,tokens", [
-    (136, 130, 128),        # one tile of rows and a few rows more, one of tokens
-    (136, 1090, 129),       # a row of tokens past the tile; down projection of 34 steps, whole or in slices of 17
-    (320, 1160, 191),       # 38 steps: two left behind whole rounds of the stages
-    (256, 4100, 383),       # down projection in several slices, the last one shorter
-    (128, 28800, 250),      # enough tiles of 256 x 128 to fill the chip
-    (128, 28800, 300),      # 256 x 192: the second tile of tokens mostly empty
-    (128, 28804, 385),      # one token in the last tile, four rows in the last block
-])
+# What a case is for is which kernel it reaches: tile (of 64-row by 64-token waves) and slices along K.  test_dispatch.py holds the
+# launches of the built library against it.  Steps are of 32 elements of K (padded to 64), the tiles keep 5 (2 x 2), 4 (4 x 2) or 3 of them in LDS.
+#   (width, ff, tokens), tile and slices of the product up (K = width), and down (K = ff)
+BF16_CASES = [
+    # one tile of tokens, two of rows with a few rows in the second; six steps each: one behind a whole round
+    ((136, 130, 128), (2, 2, 1), (2, 2, 1)),
+    ((136, 1090, 129), (2, 2, 1), (2, 2, 4)),       # a token past the tile; down 36 steps: four slices of nine, four behind a round
+    ((320, 1160, 191), (2, 2, 1), (2, 2, 4)),       # ten steps, no remainder; down 38: slices of 10, 10, 10 and 8
+    ((256, 4100, 383), (2, 2, 1), (2, 2, 8)),       # eight steps: three behind a round; down 130: slices of 17, the last of 11
+    ((64, 8196, 385), (4, 2, 1), (2, 2, 8)),        # two steps, fewer than the stages; down 258: slices of 33, the last of 27
+    ((128, 28800, 250), (4, 2, 1), (2, 2, 8)),      # four steps; enough tiles of 256 x 128 to fill the chip; down 900: slices of 113, the last of 109
+    ((128, 28800, 300), (4, 3, 1), (2, 2, 8)),      # 256 x 192: the second tile of tokens mostly empty; four steps: one behind a round
+    ((64, 28804, 300), (4, 3, 1), (2, 2, 8)),       # two steps, four rows in the last block; down 902: slices of 113, the last of 111
+    ((192, 28800, 300), (4, 3, 1), (2, 2, 8)),      # six steps: whole rounds
+    ((128, 28804, 385), (4, 4, 1), (2, 2, 8)),      # one token in the last tile
+    ((64, 28800, 385), (4, 4, 1), (2, 2, 8)),       # two steps
+]
+
+
+@pytest.mark.parametrize("width,ff,tokens", [c[0] for c in BF16_CASES])
 def test_products_of_many_tokens(tmp_path, width, ff, tokens):
     """A feed-forward of `ff` behind attention over `tokens` tokens: products of (rows, K) = (ff, width) and (width, ff)."""
     cfg = N.config(64, width, 8, [N.attention(2, 1, 64, 50, ff=ff)])
@@ -55,14 +66,28 @@ def kquant(n_embd, n_head, n_kv, n_ff):
     return dict(arch="llama", n_layer=1, n_embd=n_embd, n_head=n_head, n_head_kv=n_kv, head_dim=128, n_ff=n_ff, n_vocab=256, eps=1e-5, rope=1e4)
 
 
-@pytest.mark.parametrize("shape,tokens", [
-    ((512, 4, 1, 768), 129),        # matrices of one launch that end inside a tile of 256 rows; slices along K; a token past the tile
-    ((512, 4, 1, 768), 143),        # the last block of 16 tokens one short
-    ((256, 2, 1, 28672), 140),      # 256 x 192, most of it empty
-    ((256, 2, 1, 14336), 256),      # 256 x 128
-    ((256, 2, 1, 28672), 256),      # 256 x 256
-    ((1024, 8, 2, 2816), 385),      # down projection of 88 steps in slices; three query heads' worth of rows in the last tile
-])
+#   (width, heads, kv heads, ff), tokens, tile and slices of q/k/v, o, gate/up and down
+KQUANT_MANY_CASES = [
+    ((512, 4, 1, 768), 129, (2, 2, 1), (2, 2, 1), (2, 2, 1), (2, 2, 1)),        # a token past the tile; 16 and 24 steps
+    ((512, 4, 1, 768), 143, (2, 2, 1), (2, 2, 1), (2, 2, 1), (2, 2, 1)),        # the last block of 16 tokens one short
+    ((256, 2, 1, 28672), 140, (2, 2, 1), (2, 2, 1), (4, 3, 1), (2, 2, 8)),      # 256 x 192, most of it empty
+    ((256, 2, 1, 14336), 256, (2, 2, 1), (2, 2, 1), (4, 2, 1), (2, 2, 8)),      # 256 x 128
+    ((256, 2, 1, 28672), 256, (2, 2, 1), (2, 2, 1), (4, 4, 1), (2, 2, 8)),      # 256 x 256
+    # down projection of 88 steps in slices of eleven; three query heads' worth of rows in the last tile
+    ((1024, 8, 2, 2816), 385, (2, 2, 1), (2, 2, 1), (2, 2, 1), (2, 2, 8)),
+    # every product in slices: rotation and append behind q/k/v, SwiGLU behind the slices of the pair; the tile of tokens full but for one, and whole
+    ((2048, 16, 4, 2048), 129, (2, 2, 4), (2, 2, 8), (2, 2, 4), (2, 2, 8)),
+    ((2048, 16, 4, 2048), 200, (2, 2, 4), (2, 2, 4), (2, 2, 4), (2, 2, 4)),
+    ((2304, 2, 1, 2304), 129, (2, 2, 8), (2, 2, 1), (4, 3, 8), (2, 2, 4)),      # the sliced pair on 256 x 192: nine steps a slice
+    ((3328, 2, 1, 768), 700, (2, 2, 8), (2, 2, 1), (4, 2, 4), (2, 2, 1)),       # ... on 256 x 128: 26 steps a slice
+    # q/k/v on tiles of 256 rows of which one holds k's last rows and v's first: in slices, on 256 x 128 and 256 x 192; in one piece
+    ((4096, 12, 3, 256), 129, (4, 2, 8), (2, 2, 4), (2, 2, 8), (2, 2, 1)),
+    ((2560, 30, 5, 256), 129, (4, 3, 8), (2, 2, 4), (2, 2, 8), (2, 2, 1)),
+    ((256, 22, 11, 256), 700, (4, 2, 1), (2, 2, 8), (2, 2, 1), (2, 2, 1)),
+]
+
+
+@pytest.mark.parametrize("shape,tokens", [c[:2] for c in KQUANT_MANY_CASES])
 def test_kquant_products_of_many_tokens(tmp_path, shape, tokens):
     """A chunk through one layer over f16 copies, against the oracle and against the GEMM that forms the same weights as it goes."""
     m = mesh()
@@ -70,10 +95,10 @@ def test_kquant_products_of_many_tokens(tmp_path, shape, tokens):
     path = str(tmp_path / "model.gguf")
     tensors = models.write_model(path, cfg, [0], seed=7)
     x = np.random.Generator(np.random.PCG64(tokens)).standard_normal((tokens, cfg["n_embd"])).astype(np.float32)
-    want = StageOracle(cfg, tensors, 0, 1, 512, blas=True).forward(x, np.arange(tokens))
+    want = StageOracle(cfg, tensors, 0, 1, 768, blas=True).forward(x, np.arange(tokens))
     got = {}
     for copies in (0, 1):
-        st = m.Stage(path, 0, 1, n_ctx=512, n_batch_max=512, tuning={"tile_copies": copies})
+        st = m.Stage(path, 0, 1, n_ctx=768, n_batch_max=768, tuning={"tile_copies": copies})
         ses = st.session()
         got[copies] = ses.decode(x, np.arange(tokens)).view(np.float32).reshape(want.shape)
         assert ses.f16_saturations() == 0
@@ -121,13 +146,20 @@ def test_expert_products_over_ragged_loads(tmp_path, n_embd, ff, tokens):
     assert np.linalg.norm((got[1] - got[0])[same]) / norm < 6e-3
 
 
-@pytest.mark.parametrize("shape,tokens", [
-    ((256, 2, 1, 256), 17),         # four steps along K: one for each group of waves; padding columns
-    ((512, 4, 1, 768), 32),         # the full 32-column tile; 12 steps
-    ((512, 4, 1, 2816), 33),        # 44 steps in slices of eleven, six and five of them for a slice's two groups
-    ((1024, 8, 2, 2816), 64),       # the full 64-column tile
-    ((256, 2, 1, 33024), 47),       # more row blocks than compute units: K in one piece
-])
+#   shape as above, tokens, (32-column groups, groups of waves, slices) of gate/up and down
+KQUANT_FEW_CASES = [
+    ((256, 2, 1, 256), 17, (1, 4, 1), (1, 4, 1)),       # four steps along K: one for each group of waves; padding columns
+    ((512, 4, 1, 768), 32, (1, 4, 1), (1, 4, 1)),       # the full 32-column tile; 12 steps
+    ((512, 4, 1, 2816), 33, (2, 4, 1), (2, 2, 4)),      # 44 steps in slices of eleven, six and five of them for a slice's two groups
+    ((1024, 8, 2, 2816), 64, (2, 2, 2), (2, 2, 4)),     # the full 64-column tile; the pair in slices
+    # more row blocks than compute units: two groups of waves, K in one piece (512 blocks and more: the 256-row tile takes those)
+    ((256, 2, 1, 20480), 20, (1, 2, 1), (1, 2, 16)),
+    ((256, 2, 1, 20480), 47, (2, 2, 1), (2, 2, 16)),
+    ((512, 4, 1, 32512), 33, (2, 2, 1), (2, 2, 16)),
+]
+
+
+@pytest.mark.parametrize("shape,tokens", [c[:2] for c in KQUANT_FEW_CASES])
 def test_kquant_products_of_few_tokens(tmp_path, shape, tokens):
     """A chunk of 17 to 64 tokens through one layer, against the oracle and against the 128-column tile."""
     m = mesh()
@@ -151,12 +183,16 @@ def test_kquant_products_of_few_tokens(tmp_path, shape, tokens):
     assert np.linalg.norm(got[1] - got[0]) / norm < 1e-3, (shape, tokens)
 
 
-@pytest.mark.parametrize("shape,tokens", [
-    ((256, 2, 1, 256), 17),         # four steps along K, one per group; two columns' worth past the first block
-    ((768, 6, 2, 2816), 32),        # twelve steps; all columns
-    ((512, 4, 1, 33024), 23),       # more row blocks than compute units: two groups
-    ((512, 4, 1, 768), 5),          # one block of 16 columns
-])
+#   shape as above, tokens, groups of waves of gate/up
+DECODE_BATCH_CASES = [
+    ((256, 2, 1, 256), 17, 4),          # four steps along K, one per group; two columns' worth past the first block
+    ((768, 6, 2, 2816), 32, 4),         # twelve steps; all columns
+    ((512, 4, 1, 33024), 23, 2),        # more row blocks than compute units: two groups
+    ((512, 4, 1, 768), 5, 4),           # one block of 16 columns
+]
+
+
+@pytest.mark.parametrize("shape,tokens", [c[:2] for c in DECODE_BATCH_CASES])
 def test_gate_up_of_a_decode_batch(tmp_path, shape, tokens):
     """A batch of single steps through two layers with gate / up on the register-formed tile, the norm before it handed over, against
     the oracle and against the f16 skinny GEMM."""
