@@ -292,7 +292,7 @@ int mesh_session_f16_saturations(mesh_session *session, uint64_t *count);
  *     gemm_fused=1         q/k/v and gate/up of a prefill call as one launch each
  *     gemm_xdirect=1       the prefill GEMM reads k8-major activations directly
  *     gemm_big=1           256-row tiles for wide projections of long calls
- *     gemm_narrow=1        tiles of 32 or 64 tokens for calls of at most 64
+ *     gemm_narrow=1        tiles of 32 or 64 tokens for calls of at most 64, where gemm_big does not take the projection
  *     attn_chunk_ksplit=1  a prefill chunk's key walks split over workgroups when the grid would not fill the chip
  *     attn_mma_min_tokens=1  decode attention on the matrix cores from this many tokens
  *     attn_split_target=0  workgroups a decode attention launch aims at (0 = 256, or 512 for quantised rows)

@@ -16,6 +16,7 @@
 // l%32, same k; accumulator register i of lane l = D[8*(i/4) + 4*(l/32) + i%4][l%32].
 
 #include "gemm.hpp"
+#include "gemm_tile.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -28,14 +29,6 @@ typedef float float16v __attribute__((ext_vector_type(16)));
 constexpr int GM = 128, GN = 128, GK = 64;     // workgroup tile: weight rows x tokens x k-step
 constexpr int LDS_LD = GK + 8;                 // f16 elements per LDS row (16-byte pad against bank conflicts)
 constexpr int GEMM_THREADS = 512;              // 4 matrix-core waves + 4 staging waves
-
-// f32 pair -> packed f16, saturating: a magnitude beyond the f16 range becomes +-65504 instead of an infinity that the
-// next layer's norm would turn into NaN for the whole token.
-__device__ __forceinline__ uint32_t pack_h2(float a, float b) {
-    a = __builtin_amdgcn_fmed3f(a, -65504.f, 65504.f);
-    b = __builtin_amdgcn_fmed3f(b, -65504.f, 65504.f);
-    return (uint32_t)__half_as_ushort(__float2half_rn(a)) | ((uint32_t)__half_as_ushort(__float2half_rn(b)) << 16);
-}
 
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 
@@ -1045,22 +1038,11 @@ static int launch_gemm_kernel(const GemmArgs &k, dim3 grid, hipStream_t stream) 
     return SPLIT ? gemm_add_slices(k, (int)grid.x, stream) : MESH_OK;
 }
 
-static int gemm_n_cu() {
-    static int n = 0;
-    if (!n) {
-        int dev = 0;
-        hipDeviceProp_t p;
-        if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&p, dev) == hipSuccess) n = p.multiProcessorCount;
-        if (n <= 0) n = 256;
-    }
-    return n;
-}
-
 // groups of waves along K: four where a CU gets one workgroup (16 waves), two where it gets several or K is split already
 template <int TYPE, int NT, int MODE>
 static int launch_gemm_reg(const GemmArgs &k, dim3 grid, hipStream_t stream) {
     if (k.ksplit > 1) MESH_LAUNCH((gemm_reg_kernel<TYPE, NT, REG_SPLIT, 2>), grid, dim3(512), 0, stream, k);
-    else if ((int)grid.x > gemm_n_cu()) MESH_LAUNCH((gemm_reg_kernel<TYPE, NT, MODE, 2>), grid, dim3(512), 0, stream, k);
+    else if ((int)grid.x > gt_n_cu()) MESH_LAUNCH((gemm_reg_kernel<TYPE, NT, MODE, 2>), grid, dim3(512), 0, stream, k);
     else MESH_LAUNCH((gemm_reg_kernel<TYPE, NT, MODE, 4>), grid, dim3(1024), 0, stream, k);
     MESH_LAUNCH_CHECK();
     return k.ksplit > 1 ? gemm_add_slices(k, (int)grid.x, stream) : MESH_OK;
@@ -1080,7 +1062,7 @@ static int split_plan(const GemmArgs &a, int row_blocks, int t_blocks, int *k_pe
     const int n_all = a.K / GK;
     *k_per_split = n_all;
     if (!a.part) return 1;
-    const int wgs = row_blocks * t_blocks, ncu = gemm_n_cu();
+    const int wgs = row_blocks * t_blocks, ncu = gt_n_cu();
     int ks = 1;
     while (ks < 16 && wgs * ks * 2 <= ncu && n_all / (ks * 2) >= 8 &&
            (size_t)(ks * 2) * a.T * row_blocks * GM * sizeof(float) <= a.part_bytes) ks *= 2;
@@ -1143,9 +1125,11 @@ int gemm_kquant(const GemmArgs &a, hipStream_t stream) {
         return fail(MESH_ERR_INVALID, "gemm: RoPE / KV append on a launch it does not fit");
     if (a.type != MESH_Q4_K && a.type != MESH_Q6_K) return fail(MESH_ERR_UNSUPPORTED, "gemm: no MFMA kernel for ggml type %d", a.type);
     const bool q4 = a.type == MESH_Q4_K, packed = a.Wp != nullptr;
-    // enough workgroups of the 256 x 128 tile to give every CU one: the big tile (gemm_big_kernel)
+    // enough workgroups of the 256 x 128 tile to give every CU one: the big tile (gemm_big_kernel).  A pair of 512 row blocks and more
+    // does at any token count: calls of 17 to 64 tokens over such a pair take it too, though the register-formed tile is the faster one
+    // there (two layers 4096 wide with 33024 feed-forward rows: 388 against 286 us at 17 tokens, 473 against 377 at 64).
     if (a.x_k8 && packed && k.ksplit <= 1 && !a.rope.pos && row_blocks % 2 == 0 && a.big_tile &&
-        (row_blocks / 2) * (int)grid.y >= gemm_n_cu())
+        (row_blocks / 2) * (int)grid.y >= gt_n_cu())
         return q4 ? launch_gemm_big<MESH_Q4_K>(k, row_blocks, (int)grid.y, stream) : launch_gemm_big<MESH_Q6_K>(k, row_blocks, (int)grid.y, stream);
     if (a.x_k8) {
         if (packed) return q4 ? launch_gemm<MESH_Q4_K, true, true>(k, grid, stream) : launch_gemm<MESH_Q6_K, true, true>(k, grid, stream);

@@ -14,12 +14,6 @@
 
 namespace mesh {
 
-__device__ __forceinline__ uint32_t tile_pack_h2(float a, float b) {
-    a = __builtin_amdgcn_fmed3f(a, -65504.f, 65504.f);
-    b = __builtin_amdgcn_fmed3f(b, -65504.f, 65504.f);
-    return (uint32_t)__half_as_ushort(__float2half_rn(a)) | ((uint32_t)__half_as_ushort(__float2half_rn(b)) << 16);
-}
-
 // TILE_ROWS_OUT: f32 rows with bias and residual, per matrix of the launch; TILE_SWIGLU: f16(silu(gate) up) in the k8-major layout;
 // TILE_PARTIAL: this slice's sums as they are.  SwiGLU holds tokens in the lanes (four weight rows of a lane are 8 bytes of the
 // output), the others weight rows (a store covers whole lines).
@@ -58,7 +52,7 @@ __global__ __launch_bounds__(64 * WM * WT, gt_waves_per_simd(WM, WT)) void gemm_
                 }
                 note_f16_clamp(a.sat, o[0], o[1], o[2], o[3]);
                 *reinterpret_cast<uint2 *>(a.y16_k8 + (size_t)(t >> 4) * 16 * a.M + ((size_t)(m >> 3) * 16 + (t & 15)) * 8 + (m & 7)) =
-                    make_uint2(tile_pack_h2(o[0], o[1]), tile_pack_h2(o[2], o[3]));
+                    make_uint2(pack_h2(o[0], o[1]), pack_h2(o[2], o[3]));
             }
         }
         return;

@@ -791,7 +791,7 @@ int moe_combine_quant16(float *x, const float *y, const float *w, int T, int n, 
 // Tokens are grouped in blocks of 16 columns, and within a block the 8 consecutive k of every column sit together:
 // element (t, k) of block b = t / 16 is at ((b * K/8 + k/8) * 16 + t % 16) * 8 + k % 8.
 typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
-// saturating, like gemm.hip's pack_h2; a clamped pair is noted in the caller's counter (mesh_common.hpp), if it has one
+// saturating, like pack_h2; a clamped pair is noted in the caller's counter (mesh_common.hpp), if it has one
 __device__ __forceinline__ uint32_t sk_pack_h2(unsigned *sat, float a, float b) {
     note_f16_clamp(sat, a, b);
     const h2_t h = {(_Float16)__builtin_amdgcn_fmed3f(a, -65504.f, 65504.f), (_Float16)__builtin_amdgcn_fmed3f(b, -65504.f, 65504.f)};

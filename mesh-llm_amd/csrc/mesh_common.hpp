@@ -122,6 +122,14 @@ __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
 }
 __device__ __forceinline__ float bf16_bits_to_f32(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
+// f32 pair -> packed f16, saturating: a magnitude beyond the f16 range becomes +-65504 instead of an infinity that the
+// next layer's norm would turn into NaN for the whole token.
+__device__ __forceinline__ uint32_t pack_h2(float a, float b) {
+    a = __builtin_amdgcn_fmed3f(a, -65504.f, 65504.f);
+    b = __builtin_amdgcn_fmed3f(b, -65504.f, 65504.f);
+    return (uint32_t)__half_as_ushort(__float2half_rn(a)) | ((uint32_t)__half_as_ushort(__float2half_rn(b)) << 16);
+}
+
 // The f16 producers of the batched paths clamp what f16 cannot hold to +-65504.  A caller can ask how often that happened
 // (mesh_session_f16_saturations): every producer that can meet such a value is handed the session's counter and notes each
 // group of values it clamps.  `sat` may be null (no counting).

@@ -489,7 +489,9 @@ static int kquant_session_alloc(mesh_session *s) {
             if ((rc = fbuf(&s->ffn_up, B * (size_t)hp.n_ff)) != MESH_OK) return rc;
         }
         if (B >= (size_t)PREFILL_MIN_TOKENS) {
-            // a split launch holds at most one 128 x 128 f32 tile per CU: 16.8 MB on 256 CUs
+            // Partial results of launches split along K.  A launch of the GEMM layout holds at most one 128 x 128 f32 tile per CU (16.8 MB on
+            // 256 CUs); over f16 copies a slice is a whole result (8.4 MB for the 8B down projection of 512 tokens), and it is this
+            // size that bounds the slices.
             s->gemm_part_bytes = (size_t)32 << 20;
             if ((rc = sess_alloc(s, &p, s->gemm_part_bytes)) != MESH_OK) return rc;
             s->gemm_part = static_cast<float *>(p);
@@ -891,8 +893,11 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
         ProfScope ps(s, MESH_PROF_GEMV);
         // From 17 tokens on the skinny GEMM walks two blocks of columns per weight tile; the register-formed tile has all 32 in its
         // fragment.  Gate / up of 28672 x 4096 at 32 tokens 34 -> 24 us, of 55296 x 5120 70 -> 49; below (16 tokens) 23 against 23,
-        // and with the rest of the layer 691 against 684 us for eight layers.  Blocks: about one workgroup per CU; fewer would leave
+        // and with the rest of the layer 691 against 684 us for eight layers.  Blocks: set near one workgroup per CU; fewer leave
         // CUs idle, or split K and lose the epilogue.
+        // Four layers at 32 tokens, time with the skinny GEMM over time with the tile: 144 blocks 1.15, 172 1.13, 192 1.10 (2048 wide 1.06),
+        // 224 1.07, 256 1.03, 260 1.12, 352 1.10, 432 1.13, 448 1.14.  144 and 172 show that the line could lie lower; nothing below them
+        // was measured.
         if (ffn_norm_fused && L.gate_up_gemm && T >= s->tune.reg_min_tokens && T <= 32 && gemm_pair_row_blocks(FF) >= s->tune.reg_min_blocks) {
             GemmArgs g;
             g.Wp = L.gate_up_gemm; g.type = L.w_gate.type;
@@ -1108,14 +1113,12 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
                     if ((rc = rmsnorm_f16_k8_gather(s->x, static_cast<const float *>(L.ffn_norm.data), hp.rms_eps, s->moe_sorted.pair_of_slot, k, slots, E,
                                                     reinterpret_cast<_Float16 *>(s->moe_x16), stream, s->f16_sat)) != MESH_OK) return rc;
                 }
-                const bool d_big = s->tune.gemm_big, d_narrow = s->tune.gemm_narrow;
                 GemmArgs g;
                 g.W = L.gate_exps.data; g.Wp = L.exps_gate_up_gemm; g.type = L.gate_exps.type;
                 g.M = ffe; g.K = E; g.T = slots;
                 g.X = reinterpret_cast<const _Float16 *>(s->moe_x16); g.ldx = E; g.x_k8 = true;
                 g.y16_k8 = reinterpret_cast<_Float16 *>(s->moe_ffn16);
                 g.sat = s->f16_sat;
-                g.big_tile = d_big; g.narrow_tile = d_narrow;
                 g.tiles = s->moe_sorted.tiles; g.n_tiles = s->moe_sorted.counts; g.max_tiles = max_tiles; g.expert_stride = L.exps_gate_up_stride;
                 { ProfScope ps(s, MESH_PROF_GEMV); rc = gemm_kquant(g, stream); }
                 if (rc != MESH_OK) return rc;
@@ -1124,7 +1127,6 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
                 d.M = E; d.K = ffe; d.T = slots;
                 d.X = reinterpret_cast<const _Float16 *>(s->moe_ffn16); d.ldx = ffe; d.x_k8 = true;
                 d.Y = s->moe_out_slots; d.ldy = E;
-                d.big_tile = d_big; d.narrow_tile = d_narrow;
                 d.tiles = s->moe_sorted.tiles; d.n_tiles = s->moe_sorted.counts; d.max_tiles = max_tiles; d.expert_stride = L.exps_down_stride;
                 { ProfScope ps(s, MESH_PROF_GEMV); rc = gemm_kquant(d, stream); }
                 if (rc != MESH_OK) return rc;

@@ -31,7 +31,7 @@ struct Tuning {
     int gemm_fused = 1;            // q/k/v and gate/up of a prefill call as one GEMM launch each
     int gemm_xdirect = 1;          // the prefill GEMM reads k8-major activations directly (0: row-major staged through LDS)
     int gemm_big = 1;              // the 256-row tile for wide projections of long calls
-    int gemm_narrow = 1;           // the register-formed tile of 32 or 64 columns for calls of at most 64 tokens
+    int gemm_narrow = 1;           // the register-formed tile of 32 or 64 columns for calls of at most 64 tokens that gemm_big leaves
     int attn_chunk_ksplit = 1;     // a prefill chunk's key walks split over workgroups when the grid would not fill the chip
     int attn_mma_min_tokens = 1;   // decode attention on the matrix cores from this many tokens (below: the all-f32 kernel)
     int attn_split_target = 0;     // workgroups a decode attention launch aims at; 0 = 256, 512 for quantised rows of 64+ (token, head) pairs

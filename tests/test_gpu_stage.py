@@ -642,7 +642,8 @@ def test_skinny_gemm_norms_ride_in_the_neighbouring_launches(tmp_path):
 def test_decode_batches_of_17_to_32_stay_on_the_skinny_gemm(tmp_path):
     """Batches of 17 to 32 decode steps: one pass of the f16 skinny GEMM over the weights multiplies with two blocks of 16
     activation columns (the activation fragments of one super-block are held and refilled behind the MFMAs that used
-    them), RoPE / KV append and the norm hand-over as for smaller batches.  Three real-shape layers (the middle one
+    them), RoPE / KV append and the norm hand-over as for smaller batches; gate / up, its norm handed over, on the
+    register-formed tile (on the skinny GEMM with skinny_norm_fused=0).  Three real-shape layers (the middle one
     with q6_K attn_v / ffn_down) at ragged KV depths, a x40 outlier channel in one step: against the oracle, against the
     large-tile GEMM (skinny_f16_wide=0) and against norm launches of their own (skinny_norm_fused=0); then a smaller batch
     on the same sessions, so that the hand-over buffers of a 32-column call are followed by a 16-column one."""
