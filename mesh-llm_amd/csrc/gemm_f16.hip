@@ -6,7 +6,7 @@
 // per weight of memory and, for calls of few tokens, their reading, which is why those stay with the quantised layouts
 // (tile_min_tokens).  A chunk through eight 8B-shaped layers, us, quantised layouts / copies: 64 tokens 1122 / 1241, 128 1326 / 1328,
 // 192 1770 / 1635, 333 2577 / 2030, 512 2965 / 2600, 1024 5061 / 4245, 2048 9002 / 7654; four 32B-shaped layers: 128 1128 / 1194,
-// 192 1715 / 1381, 1024 5452 / 4545.  gate/up of the 8B shape at 2048 tokens: 531 -> 410 us (1170 TFLOP/s).
+// 192 1715 / 1381, 1024 5452 / 4545.  gate/up of the 8B shape at 2048 tokens: 531 -> 410 us (1170 TFLOP/s) on one box, 410 to 434 over several.
 #include <algorithm>
 
 #include "gemm.hpp"

@@ -39,7 +39,7 @@ __device__ __forceinline__ gt_f16v gt_mma(gt_b8 a, gt_b8 b, gt_f16v c) { return 
 //   GT_ROWS:   plain rows of K elements.  A chunk is 64 bytes of each of 16 rows, kept in LDS as 16-byte piece p of row r at
 //              position p ^ ((r / 4) % 4), so that 16 rows' same piece falls on all 64 banks; the swizzle is
 //              applied to the source address, because the destination of such a load is linear in the lane.
-// Half lines of 16 rows cost the address path four times a contiguous chunk's lines: M 28672, K 4096, 2048 tokens take 410 us with
+// Half lines of 16 rows cost the address path four times a contiguous chunk's lines: M 28672, K 4096, 2048 tokens take (on one box) 410 us with
 // both operands in blocks, 465 with only the weights, 530 with plain rows (M 4096, K 14336: 187, 192, 233).
 enum GtLayout { GT_BLOCKS = 0, GT_ROWS = 1 };
 
