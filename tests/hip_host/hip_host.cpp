@@ -57,7 +57,8 @@ hipError_t hipMalloc(void **p, size_t bytes) {
     std::lock_guard<std::mutex> l(mu);
     *p = nullptr;
     if (bytes > free_bytes()) return result(hipErrorOutOfMemory);
-    *p = calloc(1, bytes ? bytes : 1);
+    *p = aligned_alloc(256, (bytes + 255) / 256 * 256 + 256);        // (what the runtime promises)
+    memset(*p, 0, bytes);
     blocks[*p] = bytes;
     used_bytes += bytes;
     return hipSuccess;
