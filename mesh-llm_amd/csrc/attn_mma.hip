@@ -7,73 +7,126 @@
 // cost per key does not depend on the group size (up to 16), and the cache rows cross the vector ALUs only to be
 // converted (quantised rows) and transposed (V).
 //
-// A workgroup takes one (split, kv head, token); each of its 4 waves walks its own 16-key blocks of the range and
+// A workgroup takes one (split, kv head, token); each of its 4 waves walks its own 32-key blocks of the range and
 // keeps its own running softmax, merged at the end:
-//   S^T (16 keys x 16 heads)  = K . Q^T      v_mfma_f32_16x16x32_f16 per 32 dims; the K operand is the cache row as it
+//   S^T (2 x 16 keys x 16 heads) = K . Q^T   v_mfma_f32_16x16x32_f16 per 32 dims; the K operand is the cache row as it
 //                                             lies in memory (lane = key, 8 consecutive dims), loaded straight from HBM
-//   O^T (16 dims x 16 heads) += V^T . P^T     v_mfma_f32_16x16x16_f16 per 16 dims; the result registers of S^T (4 keys of
-//                                             one head per lane) are the P^T operand as they are; V^T needs the keys
-//                                             along a lane, so V rows are transposed through a wave-private LDS tile
-// A lane owns one head column throughout: softmax maximum and sum are reductions over its 4 registers and the 4
-// lane groups, the rescale of O is a per-lane scalar.
+//   O^T (16 dims x 16 heads) += V^T . P^T     v_mfma_f32_16x16x32_f16 per 16 dims and 32 keys; the result registers of
+//                                             S^T (4 keys of one head per lane and half) are the P^T operand as they are;
+//                                             V^T needs the keys along a lane: V rows pass a wave-private LDS tile as
+//                                             they are, and ds_read_b64_tr_b16 hands them back transposed
+// A lane owns one head column throughout: the softmax maximum is a reduction over its 8 registers and the 4 lane
+// groups, the rescale of O is a per-lane scalar, and its share of the sum meets the others' once, at the end.
 // Q and the probabilities are rounded to f16 for the matrix cores; sums are f32.
+//
+// What bounds it: the walk of a workgroup is a chain of row loads (29 GB/s per workgroup), beside it the conversion of
+// quantised rows (~430 vector instructions per 32 keys).  Against blocks of 16 keys with V scattered into the transposed
+// tile by 32 two-byte stores a lane: 64.4 -> 55.9 us (32 sequences of 2000 to 6000 keys, 8 heads, q8_0 / q4_0: 213 MB),
+// 17.4 -> 15.4 (16 sequences, 4 heads), f16 rows 41.4 -> 39.5 (16 sequences, 179 MB: 4.5 TB/s), 7.3 -> 6.8 (one).
 
 #include "attn.hpp"
 #include "q16.hpp"
 
 namespace mesh {
 
-constexpr int MMA_THREADS = 256, MMA_WAVES = 4, MMA_KEYS = 16;
+constexpr int MMA_THREADS = 256, MMA_WAVES = 4, MMA_KEYS = 32;
 constexpr float MMA_RESCALE_STEP = 8.f;  // log2 units
-constexpr int MMA_VPITCH = 20;          // halfs per dim row of the transposed V tile (16 keys + padding, 8-byte aligned)
+// Blocks in flight per wave.  A block of f16 rows is 16 KB, of quantised rows 4.6 - 6.7 KB: a second one of those covers the
+// latency of the walk (61.6 -> 55.9 us at 32 tokens), a third one and a second one of f16 rows cost more waves than they
+// bring (step of eight 8B-shaped layers at 16 tokens 910 -> 920 us).
+constexpr int MMA_DEPTH_F16 = 1, MMA_DEPTH_Q = 2;
+// halfs added to a key row of the V tile: rows of 272 (144) bytes put the 16 rows of a wave's stores on different banks
+constexpr int MMA_VPAD = 8;
 
 typedef _Float16 mm_h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 mm_h4 __attribute__((ext_vector_type(4)));
 typedef _Float16 mm_h2 __attribute__((ext_vector_type(2)));
 typedef float mm_f4 __attribute__((ext_vector_type(4)));
 typedef uint32_t mm_u4 __attribute__((ext_vector_type(4)));
 typedef uint32_t mm_u2 __attribute__((ext_vector_type(2)));
+typedef uint32_t mm_u4a8 __attribute__((ext_vector_type(4), aligned(8)));
+typedef short mm_s4 __attribute__((ext_vector_type(4)));
+
+// Four halves of one column of a 4-row x 16-column tile: lane i of a group of 16 lanes hands in the address of row i / 4,
+// columns 4 (i % 4) .. + 4, and receives column i of the four rows.
+__device__ __forceinline__ mm_u2 mm_read_transposed(const _Float16 *p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_bit_cast(mm_u2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) mm_s4 *)p));
+#else
+    return mm_u2{0, 0};
+#endif
+}
 
 __device__ __forceinline__ uint32_t mm_pack(float a, float b) {
     const mm_h2 h = {(_Float16)a, (_Float16)b};
     return __builtin_bit_cast(uint32_t, h);
 }
 
-// Bytes / nibbles -> f16 without conversions: 0x6400 | u is the half 1024 + u, so one packed subtraction of
-// 1024 + offset leaves the signed quant exactly, and one packed multiply by the block scale (an f16 in the cache)
-// gives d * q rounded to f16 -- the same value as the f32 product rounded once.
-__device__ __forceinline__ uint32_t mm_scale_pair(uint32_t biased, _Float16 bias, mm_h2 d2) {
-    const mm_h2 v = (__builtin_bit_cast(mm_h2, biased) - mm_h2{bias, bias}) * d2;
+// Bytes / nibbles -> f16 without conversions: 0x6400 | u is the half 1024 + u (0x5400 | u << 4 the half 64 + u), so one
+// packed subtraction of that and the offset leaves the signed quant exactly, and one packed multiply by the block scale
+// (an f16 in the cache) gives d * q rounded to f16 -- the same value as the f32 product rounded once.
+__device__ __forceinline__ uint32_t mm_scale_pair(uint32_t biased, float bias, mm_h2 d2) {
+    const mm_h2 v = (__builtin_bit_cast(mm_h2, biased) - mm_h2{(_Float16)bias, (_Float16)bias}) * d2;
     return __builtin_bit_cast(uint32_t, v);
 }
 
-// the 8 values a lane fetched from a cache row as packed f16 (quantised rows are dequantised in f16, exactly as above)
-template <int TYPE>
-__device__ __forceinline__ uint4 mm_piece_f16(const KvRaw<TYPE> &r) {
-    if constexpr (TYPE == MESH_F16) {
-        return r.v;
-    } else {
-        const _Float16 d = __builtin_bit_cast(_Float16, r.d);
-        const mm_h2 d2 = {d, d};
-        if constexpr (TYPE == MESH_Q8_0) {
-            const uint32_t a = r.v.x ^ 0x80808080u, b = r.v.y ^ 0x80808080u;       // int8 -> biased uint8
-            const _Float16 bias = (_Float16)(1024.f + 128.f);
-            return make_uint4(mm_scale_pair(__builtin_amdgcn_perm(0x64646464u, a, 0x04010400u), bias, d2),
-                              mm_scale_pair(__builtin_amdgcn_perm(0x64646464u, a, 0x04030402u), bias, d2),
-                              mm_scale_pair(__builtin_amdgcn_perm(0x64646464u, b, 0x04010400u), bias, d2),
-                              mm_scale_pair(__builtin_amdgcn_perm(0x64646464u, b, 0x04030402u), bias, d2));
+// What a lane (key row c, lane group g) holds of a cache row: HD / 4 values as HD / 32 pieces of 8.
+//   f16         piece cc is dims 32 cc + 8 g .. + 8: the four groups of a row read 64 consecutive bytes per load
+//   quantised   piece cc is dims (HD / 4) g + 8 cc .. + 8: whole 16-byte loads, and one block scale per lane
+// q4_0 pieces come out with their dims in the order 0 4 1 5 2 6 3 7 (mm_dim_slot), which takes one shift per eight
+// nibbles; Q is packed in the same order for K, and the merge undoes it for V.
+template <int TYPE, int HD>
+struct RowShare {
+    static constexpr int NC = HD / 32;
+    static constexpr int BYTES = TYPE == MESH_F16 ? HD / 2 : TYPE == MESH_Q8_0 ? HD / 4 : HD / 8;
+    uint32_t w[BYTES / 4];
+    uint16_t d;
+    __device__ __forceinline__ void load(const uint8_t *row, int g) {
+        if constexpr (TYPE == MESH_F16) {
+#pragma unroll
+            for (int cc = 0; cc < NC; ++cc) {
+                const uint4 v = *reinterpret_cast<const uint4 *>(row + 64 * cc + 16 * g);
+                w[4 * cc] = v.x; w[4 * cc + 1] = v.y; w[4 * cc + 2] = v.z; w[4 * cc + 3] = v.w;
+            }
         } else {
-            // byte i of the word holds elements 2i (low nibble) and 2i + 1 (high nibble)
-            const uint32_t lo = r.v & 0x0F0F0F0Fu, hi = (r.v >> 4) & 0x0F0F0F0Fu;
-            const _Float16 bias = (_Float16)(1024.f + 8.f);
-            // pair k = elements (2k, 2k + 1) = (byte k of lo, byte k of hi); selector bytes 0-3 address hi, 4-7 address lo
-            return make_uint4(mm_scale_pair(__builtin_amdgcn_perm(lo, hi, 0x0c000c04u) | 0x64006400u, bias, d2),
-                              mm_scale_pair(__builtin_amdgcn_perm(lo, hi, 0x0c010c05u) | 0x64006400u, bias, d2),
-                              mm_scale_pair(__builtin_amdgcn_perm(lo, hi, 0x0c020c06u) | 0x64006400u, bias, d2),
-                              mm_scale_pair(__builtin_amdgcn_perm(lo, hi, 0x0c030c07u) | 0x64006400u, bias, d2));
+            // (rows are multiples of 8 bytes, not of 16)
+            const uint8_t *p = row + BYTES * g;
+            if constexpr (BYTES >= 16) {
+#pragma unroll
+                for (int i = 0; i < BYTES / 16; ++i) {
+                    const mm_u4a8 v = *reinterpret_cast<const mm_u4a8 *>(p + 16 * i);
+                    w[4 * i] = v[0]; w[4 * i + 1] = v[1]; w[4 * i + 2] = v[2]; w[4 * i + 3] = v[3];
+                }
+            } else {
+                const uint2 v = *reinterpret_cast<const uint2 *>(p);
+                w[0] = v.x; w[1] = v.y;
+            }
+            d = *reinterpret_cast<const uint16_t *>(row + kv_quant_bytes(TYPE, HD) + (HD / 4 * g >> 5) * 2);
         }
     }
-}
+    __device__ __forceinline__ mm_u4 piece(int cc) const {
+        if constexpr (TYPE == MESH_F16) {
+            return mm_u4{w[4 * cc], w[4 * cc + 1], w[4 * cc + 2], w[4 * cc + 3]};
+        } else {
+            const _Float16 dh = __builtin_bit_cast(_Float16, d);
+            const mm_h2 d2 = {dh, dh};
+            if constexpr (TYPE == MESH_Q8_0) {
+                const uint32_t a = w[2 * cc] ^ 0x80808080u, b = w[2 * cc + 1] ^ 0x80808080u;       // int8 -> biased uint8
+                return mm_u4{mm_scale_pair(__builtin_amdgcn_perm(0x64646464u, a, 0x04010400u), 1024.f + 128.f, d2),
+                             mm_scale_pair(__builtin_amdgcn_perm(0x64646464u, a, 0x04030402u), 1024.f + 128.f, d2),
+                             mm_scale_pair(__builtin_amdgcn_perm(0x64646464u, b, 0x04010400u), 1024.f + 128.f, d2),
+                             mm_scale_pair(__builtin_amdgcn_perm(0x64646464u, b, 0x04030402u), 1024.f + 128.f, d2)};
+            } else {
+                const uint32_t x = w[cc], y = x >> 8;
+                return mm_u4{mm_scale_pair((x & 0x000F000Fu) | 0x64006400u, 1024.f + 8.f, d2), mm_scale_pair((x & 0x00F000F0u) | 0x54005400u, 64.f + 8.f, d2),
+                             mm_scale_pair((y & 0x000F000Fu) | 0x64006400u, 1024.f + 8.f, d2), mm_scale_pair((y & 0x00F000F0u) | 0x54005400u, 64.f + 8.f, d2)};
+            }
+        }
+    }
+    // first dim of piece cc
+    static __device__ __forceinline__ int dim0(int cc, int g) { return TYPE == MESH_F16 ? 32 * cc + 8 * g : HD / 4 * g + 8 * cc; }
+};
+// place, within its eight, of dim dd of a q4_0 piece
+__device__ __forceinline__ int mm_dim_slot(int dd) { return (dd & ~7) | ((dd & 3) << 1) | ((dd >> 2) & 1); }
 
 __device__ __forceinline__ void mm_wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -89,13 +142,14 @@ __global__ __launch_bounds__(MMA_THREADS) void attn_mma_kernel(const float *p_q,
                                                                const uint8_t *p_kcache, const uint8_t *p_vcache, int p_n_splits,
                                                                int p_n_ctx, int p_n_kv, int p_group, int p_n_head, float p_scale, int p_window,
                                                                const AttnArgs a) {
-    constexpr int NC = HD / 32;             // 32-dim chunks of the score product
+    constexpr int NC = HD / 32;             // steps of the score product
     constexpr int NDB = HD / 16;            // 16-dim blocks of the output
     constexpr int KRB = kv_row_bytes(KT, HD), VRB = kv_row_bytes(VT, HD);
-    // the transposed V tiles (one per wave) and, after the key loop, the per-wave results share this memory
-    constexpr int STAGE_HALFS = MMA_WAVES * HD * MMA_VPITCH;
-    constexpr int MERGE_FLOATS = MMA_WAVES * HD * 16;
-    constexpr int SH_BYTES = STAGE_HALFS * 2 > MERGE_FLOATS * 4 ? STAGE_HALFS * 2 : MERGE_FLOATS * 4;
+    constexpr int VPITCH = HD + MMA_VPAD;   // halfs per key row of the V tile
+    constexpr int OPITCH = HD + 4;          // floats per head row of the merge buffer
+    // the V tiles (one per wave) and, after the key loop, the per-wave results share this memory
+    constexpr int STAGE_BYTES = MMA_WAVES * MMA_KEYS * VPITCH * 2, MERGE_BYTES = MMA_WAVES * 16 * OPITCH * 4;
+    constexpr int SH_BYTES = STAGE_BYTES > MERGE_BYTES ? STAGE_BYTES : MERGE_BYTES;
     __shared__ __align__(16) uint8_t s_raw[SH_BYTES];
     __shared__ float s_m[MMA_WAVES][16], s_l[MMA_WAVES][16];
 
@@ -110,80 +164,88 @@ __global__ __launch_bounds__(MMA_THREADS) void attn_mma_kernel(const float *p_q,
     const int j0 = first + split * per;
     const int j1 = j0 + per < n_keys ? j0 + per : n_keys;
 
-    // Q^T operand: head column c, dims 32*cc + 8*g + j, in log2 units
+    // Q^T operand: head column c, the dims a lane of the K operand has, in log2 units
     mm_h8 qf[NC];
     {
         const float qs = c < G ? p_scale * 1.44269504088896341f : 0.f;
-        const float *qp = p_q + ((size_t)t * p_n_head + (size_t)kvh * G + (c < G ? c : 0)) * HD + 8 * g;
+        const float *qp = p_q + ((size_t)t * p_n_head + (size_t)kvh * G + (c < G ? c : 0)) * HD;
 #pragma unroll
         for (int cc = 0; cc < NC; ++cc) {
-            const float4 v0 = *reinterpret_cast<const float4 *>(qp + 32 * cc), v1 = *reinterpret_cast<const float4 *>(qp + 32 * cc + 4);
-            const mm_u4 p = {mm_pack(v0.x * qs, v0.y * qs), mm_pack(v0.z * qs, v0.w * qs), mm_pack(v1.x * qs, v1.y * qs), mm_pack(v1.z * qs, v1.w * qs)};
+            const float *qd = qp + RowShare<KT, HD>::dim0(cc, g);
+            const float4 v0 = *reinterpret_cast<const float4 *>(qd), v1 = *reinterpret_cast<const float4 *>(qd + 4);
+            const mm_u4 p = KT == MESH_Q4_0
+                                ? mm_u4{mm_pack(v0.x * qs, v1.x * qs), mm_pack(v0.y * qs, v1.y * qs), mm_pack(v0.z * qs, v1.z * qs), mm_pack(v0.w * qs, v1.w * qs)}
+                                : mm_u4{mm_pack(v0.x * qs, v0.y * qs), mm_pack(v0.z * qs, v0.w * qs), mm_pack(v1.x * qs, v1.y * qs), mm_pack(v1.z * qs, v1.w * qs)};
             qf[cc] = __builtin_bit_cast(mm_h8, p);
         }
     }
     mm_f4 o[NDB];
 #pragma unroll
     for (int db = 0; db < NDB; ++db) o[db] = mm_f4{0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, l = 0.f;
+    float m = -INFINITY, l = 0.f;           // l: of this lane's keys only
 
-    _Float16 *sV = reinterpret_cast<_Float16 *>(s_raw) + wave * HD * MMA_VPITCH;
+    _Float16 *const sV = reinterpret_cast<_Float16 *>(s_raw) + wave * MMA_KEYS * VPITCH;
+    _Float16 *const v_put = sV + c * VPITCH;                                              // rows c and 16 + c of the tile
+    const _Float16 *const v_get = sV + (4 * g + (c >> 2)) * VPITCH + 4 * (c & 3);         // (mm_read_transposed: rows 4 g .. + 4)
     const size_t base = ((size_t)seq * p_n_kv + kvh) * p_n_ctx;
-    // what a lane fetches of a 16-key block: its key row c, dims 32*cc + 8*g .. + 8 of K and of V; rows past the range
-    // are clamped to its last key (and masked below), so the fetch of the block after the last one is harmless
-    // Blocks in flight per wave: quantised rows are 2.5 - 3.5 times smaller than f16 rows, so one block ahead leaves
-    // too few bytes in flight to cover the memory latency; they run two ahead (20 more registers).
-    constexpr int DEPTH = (KT == MESH_F16 && VT == MESH_F16) ? 1 : 2;
+    // what a lane fetches of a 32-key block: its shares of key rows c and 16 + c; rows past the range are clamped to its
+    // last key (and masked below)
     constexpr int STEP = MMA_WAVES * MMA_KEYS;
-    KvRaw<KT> kraw[DEPTH][NC];
-    KvRaw<VT> vraw[DEPTH][NC];
-    auto fetch = [&](KvRaw<KT> (&kr_)[NC], KvRaw<VT> (&vr_)[NC], int kb) {
-        int kr = kb + c;
-        kr = kr < j1 ? kr : j1 - 1;
-        const uint8_t *krow = p_kcache + (base + kr) * KRB, *vrow = p_vcache + (base + kr) * VRB;
+    constexpr int DEPTH = KT == MESH_F16 && VT == MESH_F16 ? MMA_DEPTH_F16 : MMA_DEPTH_Q;
+    RowShare<KT, HD> krs[DEPTH][2];
+    RowShare<VT, HD> vrs[DEPTH][2];
+    auto fetch = [&](RowShare<KT, HD> (&kr)[2], RowShare<VT, HD> (&vr)[2], int kb) {
 #pragma unroll
-        for (int cc = 0; cc < NC; ++cc) kr_[cc] = kv_load<KT, HD>(krow, 32 * cc + 8 * g);
+        for (int h = 0; h < 2; ++h) {
+            int key = kb + 16 * h + c;
+            key = key < j1 ? key : j1 - 1;
+            kr[h].load(p_kcache + (base + key) * KRB, g);
+        }
 #pragma unroll
-        for (int cc = 0; cc < NC; ++cc) vr_[cc] = kv_load<VT, HD>(vrow, 32 * cc + 8 * g);
+        for (int h = 0; h < 2; ++h) {
+            int key = kb + 16 * h + c;
+            key = key < j1 ? key : j1 - 1;
+            vr[h].load(p_vcache + (base + key) * VRB, g);
+        }
     };
-    const int kb0 = j0 + wave * MMA_KEYS;
+    const int kb0 = j0 + __builtin_amdgcn_readfirstlane(wave) * MMA_KEYS;
     if (kb0 < j1) {
 #pragma unroll
-        for (int d = 0; d < DEPTH; ++d) fetch(kraw[d], vraw[d], kb0 + d * STEP);
+        for (int d = 0; d < DEPTH; ++d) fetch(krs[d], vrs[d], kb0 + d * STEP);
     }
     for (int kbb = kb0; kbb < j1; kbb += DEPTH * STEP) {
 #pragma unroll
       for (int d = 0; d < DEPTH; ++d) {
         const int kb = kbb + d * STEP;
         if (kb >= j1) break;
-        uint4 kf[NC], vf[NC];
+        RowShare<KT, HD> (&kr)[2] = krs[d];
+        RowShare<VT, HD> (&vr)[2] = vrs[d];
+        // S^T = K . Q^T : register i of half h is key kb + 16 h + 4 g + i for head c
+        mm_f4 s[2];
 #pragma unroll
-        for (int cc = 0; cc < NC; ++cc) kf[cc] = mm_piece_f16<KT>(kraw[d][cc]);
+        for (int h = 0; h < 2; ++h) {
+            s[h] = mm_f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int cc = 0; cc < NC; ++cc) vf[cc] = mm_piece_f16<VT>(vraw[d][cc]);
-        fetch(kraw[d], vraw[d], kb + DEPTH * STEP);      // rows of a later block travel while this one is worked on
-
-        // S^T = K . Q^T : register i is key kb + 4*g + i for head c
-        mm_f4 s = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int cc = 0; cc < NC; ++cc)
-            s = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(mm_h8, kf[cc]), qf[cc], s, 0, 0, 0);
-
-        // V rows -> transposed tile: sV[dim][key]
-#pragma unroll
-        for (int cc = 0; cc < NC; ++cc) {
-            const uint32_t w[4] = {vf[cc].x, vf[cc].y, vf[cc].z, vf[cc].w};
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-                reinterpret_cast<uint16_t *>(sV)[(32 * cc + 8 * g + e) * MMA_VPITCH + c] = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
+            for (int cc = 0; cc < NC; ++cc) s[h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(mm_h8, kr[h].piece(cc)), qf[cc], s[h], 0, 0, 0);
         }
+        // V rows as they are: sV[key][dim]
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int cc = 0; cc < NC; ++cc) *reinterpret_cast<mm_u4 *>(v_put + 16 * h * VPITCH + RowShare<VT, HD>::dim0(cc, g)) = vr[h].piece(cc);
+        // rows of a later block travel while this one is worked on (two blocks deep without a branch: the compiler then
+        // counts the loads in flight exactly, 56 against 60 us; one block deep waits for all of them anyway, and the walks
+        // of one block save the fetch)
+        if (DEPTH > 1 || kb + DEPTH * STEP < j1) fetch(kr, vr, kb + DEPTH * STEP);
 
         float mx = -INFINITY;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            s[i] = kb + 4 * g + i < j1 ? s[i] : -INFINITY;
-            mx = fmaxf(mx, s[i]);
-        }
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                s[h][i] = kb + 16 * h + 4 * g + i < j1 ? s[h][i] : -INFINITY;
+                mx = fmaxf(mx, s[h][i]);
+            }
         mx = fmaxf(mx, __shfl_xor(mx, 16));
         mx = fmaxf(mx, __shfl_xor(mx, 32));
         // The reference point m of the exponentials only moves when a score exceeds it by more than 2^RESCALE_STEP
@@ -199,38 +261,40 @@ __global__ __launch_bounds__(MMA_THREADS) void attn_mma_kernel(const float *p_q,
                 for (int i = 0; i < 4; ++i) o[db][i] *= corr;
             m = m_new;
         }
-        float p[4], ps = 0.f;
+        float p[8];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) { p[i] = __builtin_amdgcn_exp2f(s[i] - m); ps += p[i]; }
-        ps += __shfl_xor(ps, 16);
-        ps += __shfl_xor(ps, 32);
-        l += ps;
-        const mm_u2 pu = {mm_pack(p[0], p[1]), mm_pack(p[2], p[3])};
-        const mm_h4 pf = __builtin_bit_cast(mm_h4, pu);      // P^T operand: head column c, keys 4*g + j
+        for (int i = 0; i < 8; ++i) p[i] = __builtin_amdgcn_exp2f(s[i >> 2][i & 3] - m);
+        l += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+        // P^T operand: head column c, keys 4 g + j, then 16 + 4 g + j
+        const mm_u4 pu = {mm_pack(p[0], p[1]), mm_pack(p[2], p[3]), mm_pack(p[4], p[5]), mm_pack(p[6], p[7])};
+        const mm_h8 pf = __builtin_bit_cast(mm_h8, pu);
 
         mm_wave_lds_sync();
-        // O^T += V^T . P^T : the V^T operand is dim row 16*db + c, keys 4*g + j
+        // O^T += V^T . P^T : the V^T operand is place 16 db + c of the rows, keys in the order of P^T
 #pragma unroll
         for (int db = 0; db < NDB; ++db) {
-            const mm_u2 vv = *reinterpret_cast<const mm_u2 *>(sV + (16 * db + c) * MMA_VPITCH + 4 * g);
-            o[db] = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(mm_h4, vv), pf, o[db], 0, 0, 0);
+            const mm_u2 v0 = mm_read_transposed(v_get + 16 * db), v1 = mm_read_transposed(v_get + 16 * VPITCH + 16 * db);
+            const mm_u4 vv = {v0[0], v0[1], v1[0], v1[1]};
+            o[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(mm_h8, vv), pf, o[db], 0, 0, 0);
         }
         mm_wave_lds_sync();        // the tile is rewritten by the next block
       }
     }
 
-    // merge the waves: o[db][i] is dim 16*db + 4*g + i of head c
+    // merge the waves: o[db][i] is place 16 db + 4 g + i of head c
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
     __syncthreads();               // every wave is done with its V tile: the memory becomes the merge buffer
-    float *s_o = reinterpret_cast<float *>(s_raw);          // [wave][dim][16 heads]
+    float *s_o = reinterpret_cast<float *>(s_raw);          // [wave][16 heads][place]
     if (g == 0) { s_m[wave][c] = m; s_l[wave][c] = l; }
+    if (c < G) {
 #pragma unroll
-    for (int db = 0; db < NDB; ++db)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) s_o[(wave * HD + 16 * db + 4 * g + i) * 16 + c] = o[db][i];
+        for (int db = 0; db < NDB; ++db) *reinterpret_cast<mm_f4 *>(s_o + (wave * 16 + c) * OPITCH + 16 * db + 4 * g) = o[db];
+    }
     __syncthreads();
     const bool single = p_n_splits == 1;
     for (int idx = tid; idx < G * HD; idx += MMA_THREADS) {
-        const int h = idx / HD, dd = idx % HD;
+        const int h = idx / HD, dd = idx % HD, slot = VT == MESH_Q4_0 ? mm_dim_slot(dd) : dd;
         float mh = -INFINITY;
 #pragma unroll
         for (int w = 0; w < MMA_WAVES; ++w) mh = fmaxf(mh, s_m[w][h]);
@@ -239,7 +303,7 @@ __global__ __launch_bounds__(MMA_THREADS) void attn_mma_kernel(const float *p_q,
         for (int w = 0; w < MMA_WAVES; ++w) {
             const float mw = s_m[w][h];
             const float wgt = mw == -INFINITY ? 0.f : exp2f(mw - mh);
-            sum = fmaf(s_o[(w * HD + dd) * 16 + h], wgt, sum);
+            sum = fmaf(s_o[(w * 16 + h) * OPITCH + slot], wgt, sum);
             ll = fmaf(s_l[w][h], wgt, ll);
         }
         const size_t row = (size_t)t * p_n_head + (size_t)kvh * G + h;

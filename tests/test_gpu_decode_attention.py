@@ -1,0 +1,57 @@
+"""Decode attention over the session's cache rows at the edges of its key blocks (32 keys a wave, 128 a workgroup), both head
+sizes, every cache tier, alone and split, against a float64 softmax over the rows as the cache holds them."""
+import os
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+import models
+import oracle
+from util import mesh
+
+pytestmark = pytest.mark.gpu
+
+TIERS = [(oracle.F16, oracle.F16), (oracle.Q8_0, oracle.Q4_0), (oracle.Q4_0, oracle.Q4_0)]
+KEYS = [1, 2, 31, 32, 33, 64, 95, 127, 128, 129, 160, 255, 257, 384, 513]
+# Q and the probabilities are rounded to f16 (2^-12 of themselves, root mean square), a quantised row's product with its block
+# scale once more: independent errors of three roundings on weights that sum to one stay below 2^-11 of the result; four times that
+TOL = 4 * 2.0 ** -11
+
+
+@pytest.mark.parametrize("kv_types", TIERS)
+@pytest.mark.parametrize("name", ["tiny-llama", "tiny-g5", "tiny-g8"])      # head_dim 64; 128 with groups of 5 and 8
+def test_key_block_edges(tmp_path, name, kv_types):
+    m, cfg = mesh(), models.CONFIGS[name]
+    path = os.path.join(str(tmp_path), name + ".gguf")
+    models.write_model(path, cfg, [0], seed=3)
+    st = m.Stage(path, 0, 1, n_ctx=max(KEYS), n_seq_max=len(KEYS), n_batch_max=32, kv_types=kv_types)
+    H, HK, D = cfg["n_head"], cfg["n_head_kv"], cfg["head_dim"]
+    rng = np.random.Generator(np.random.PCG64(9))
+    ses = st.session()
+    for i, n in enumerate(KEYS):
+        # (every other sequence's rows past its keys hold large values: a key block reaches past the last key)
+        rows = max(KEYS)
+        k, v = rng.standard_normal((rows, HK, D)), rng.standard_normal((rows, HK, D))
+        k[n:] *= 50.0 * (i % 2)
+        v[n:] *= 1000.0 * (i % 2)
+        ses.kv_write(0, i, 0, k.astype(np.float16).view(np.uint16), v.astype(np.float16).view(np.uint16))
+    q = rng.standard_normal((len(KEYS), H, D)).astype(np.float32) * 1.5
+    qd = torch.from_numpy(q).cuda()
+    for batch in ([[i] for i in range(len(KEYS))] + [list(range(len(KEYS)))]):
+        part = qd[batch].contiguous()
+        out = torch.full_like(part, float("nan"))
+        torch.cuda.synchronize()
+        ses.attn_dev(0, part.data_ptr(), [KEYS[i] - 1 for i in batch], out.data_ptr(), seq=batch)
+        ses.synchronize()
+        got = out.cpu().numpy().astype(np.float64)
+        for j, i in enumerate(batch):
+            kd, vd = (r.view(np.float16).astype(np.float64).repeat(H // HK, axis=1) for r in ses.kv_read(0, i, 0, KEYS[i]))
+            s = np.einsum("hd,nhd->hn", q[i].astype(np.float64), kd) / np.sqrt(D)
+            p = np.exp(s - s.max(1, keepdims=True))
+            want = np.einsum("hn,nhd->hd", p / p.sum(1, keepdims=True), vd)
+            rel = np.linalg.norm(got[j] - want) / np.linalg.norm(want)
+            assert rel <= TOL, (name, kv_types, KEYS[i], len(batch), rel)
+    ses.close()
+    st.close()
