@@ -3,15 +3,19 @@
 //
 // The alternative to the integer kernel of gemm_skinny.hip for the same launches: the weight stream is organised as in
 // the mat-vec kernel -- a workgroup owns a few tile-rows (16 rows each), its waves split K and each keeps two
-// weight tiles in flight -- and a tile is dequantised in registers to f16 and multiplied with 16 activation columns at
-// once (v_mfma_f32_16x16x32_f16).  It issues about a third of the integer kernel's vector instructions per tile, so it
-// streams weights faster; what it gives up is precision: activations are rounded to f16 (11 significant bits against the
-// integer kernel's 16-bit fixed point), and so is every weight, ONCE: a weight is formed as ((q - offset) * sc) * d + c
-// with q - offset and the integer sub-block scale sc exact in f16, d the super-block's own f16 scale, and c = 8 d sc -
-// dmin m the sub-block's centre (q4_K; 0 for q6_K) -- the formation the prefill GEMM uses (gemm.hip).  The first version
-// of this kernel multiplied by the products d * sc and dmin * m rounded to f16, an error shared by all 32 weights of a
-// sub-block that does not average out over K and put a 16-layer stage at 1.2e-2 from the oracle; with one rounding per
-// weight the same stage measures what the prefill path does (1-2e-3).
+// weight tiles in flight -- and a tile is formed in registers as f16 and multiplied with 16 activation columns at
+// once (v_mfma_f32_16x16x32_f16).  Activations are f16 (11 significant bits against the integer kernel's 16-bit fixed point);
+// weights are exact: a fragment holds the integers q * sc (q4_K, at most 945) or (q - 32) * sc (q6_K), the sub-block minimum's
+// integers go through MFMAs of their own, and the super-block's d and dmin multiply the tile's sums in f32.  (Before, a weight
+// was rounded to f16 once; a first version multiplied by d * sc rounded to f16, which does not average out over K.)
+//
+// What bounds it.  By time stamps (gate / up of 28672 x 4096, 5 tokens): first loads requested at 2.3 us, weight stream done at 11.2
+// (66 MB in 8.5 us, the memory's rate), the slowest wave at 14.9, end 16.1 (20.3 with the last workgroup).  The stream before was
+// as fast, but every round waited for all it had requested (a branch around a tile makes the compiler assume the worst), the
+// norm's partial sums were fetched behind it (2.9 us) and the epilogue's operands behind the barrier (1.5 - 2).
+// Now / before, us: 5 tokens gate / up 20.4 / 22.4, q/k/v 10.1 - 10.8 / 11.6 - 12.0, output and q4_K down 9.8 / 10.4, q6_K down
+// 17.0 / 19.1; 16 tokens 21.1 / 23.4, 10.8 - 11.1 / 12.5 - 12.7, 10.2 / 11.1, 17.7 / 19.7; 32 tokens of the 32B shape (160 workgroups
+// of two tile-rows) q6_K down 52.3 / 55.0, q4_K down and output 24.5 / 27.9, q/k/v 15.6 / 16.1.
 //
 // Register dequantisation: lane (m = l % 16, g = l / 16) loads what lane 4m + g of the mat-vec kernel loads, i.e.
 // quarter g of row m of the super-block (gemv.hpp).  An MFMA's k-slots of lane group g are then 8 consecutive
@@ -31,8 +35,7 @@ namespace f16sk {
 
 constexpr int SK_THREADS = 512;
 constexpr int SK_WAVES = SK_THREADS / 64;
-constexpr int SK_DEPTH_Q4 = 2;            // weight tiles a wave keeps in flight (2304 B each; three and four measured 8% slower)
-constexpr int SK_DEPTH_Q6 = 2;            // q6_K tiles are 3360 B and their fragments need more registers
+constexpr int SK_DEPTH = 2;               // weight tiles a wave keeps in flight (three or four: 1-5% of a step slower)
 constexpr int SK_NT = 16;                 // activation columns of one MFMA (a launch takes one or two such blocks)
 constexpr int SK_SEGS_MAX = 4;            // (tile-row, matrix) segments one wave may own (8 spills registers)
 constexpr size_t SK_LDS_LIMIT = 160 * 1024;
@@ -69,84 +72,88 @@ struct SkinnyKernelArgs {
     float ni_eps;
 };
 
-// four bytes (values < 64) -> four f16 holding 1024 + value
-__device__ __forceinline__ void bytes_to_h1024(uint32_t v, h2_t &lo, h2_t &hi) {
-    lo = __builtin_bit_cast(h2_t, __builtin_amdgcn_perm(0x64646464u, v, 0x04010400u));
-    hi = __builtin_bit_cast(h2_t, __builtin_amdgcn_perm(0x64646464u, v, 0x04030402u));
-}
-
-// Eight weights as an MFMA A fragment: bytes of v0, v1 hold the quants; w = ((q - off) * sc) * d + c, where (q - off) * sc
-// is an exact integer in f16 and the fma rounds once.
-__device__ __forceinline__ h8_t dequant8(uint32_t v0, uint32_t v1, h2_t off, h2_t sc, h2_t d, h2_t c) {
-    h2_t p[4];
-    bytes_to_h1024(v0, p[0], p[1]);
-    bytes_to_h1024(v1, p[2], p[3]);
-    u4_t a;                                                          // built as four dwords: no half-register moves
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const h2_t q = (p[i] - off) * sc;                            // exact
-        a[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(q, d, c));
-    }
-    return __builtin_bit_cast(h8_t, a);
-}
-
 __device__ __forceinline__ h2_t h2_of(float v) {
     const _Float16 h = (_Float16)v;
     return h2_t{h, h};
 }
+__device__ __forceinline__ h2_t h2_bits(uint32_t v) { return __builtin_bit_cast(h2_t, v); }
+__device__ __forceinline__ uint32_t h2_bits(h2_t v) { return __builtin_bit_cast(uint32_t, v); }
 
-// A fragments of one tile, MFMA by MFMA.  frag(t, ...) returns the fragment of MFMA t (0..7) and the element
-// offset within the super-block of this lane's 8 k-slots.
+// A choice between two values by lane, as arithmetic: written as `lane ? a : b`, the two formulas of a tile's scales are compiled
+// into branches.
+__device__ __forceinline__ uint32_t lanes_mask(bool b) {
+    uint32_t m = b ? 0xFFFFFFFFu : 0u;
+    asm("" : "+v"(m));          // (or the compiler turns the arithmetic back into the choice)
+    return m;
+}
+__device__ __forceinline__ uint32_t bits_of(uint32_t mask, uint32_t a, uint32_t b) { return (a & mask) | (b & ~mask); }
+
+// Weight fragments of one tile, MFMA by MFMA.  frag(t) returns the fragment of MFMA t (0..7), integers exact in f16 (see below for
+// q6_K): the sum of the tile's products times `d` is what the weights without their minimum contribute.  minimum(high), where a
+// type has one, is the same for all MFMAs of a sub-block: its products times `ndmin` complete the sum.
 template <int TYPE> struct TileFrags;
 
 template <> struct TileFrags<MESH_Q4_K> {
+    static constexpr bool MINIMUM = true;
     uint32_t w[8];
-    h2_t s_lo, s_hi, c_lo, c_hi, d2;
-    int kbase;
+    h2_t s_lo, s_hi, o_lo, o_hi;
+    uint32_t m_lo, m_hi, mask_lo, mask_hi, base_lo, base_hi;
+    float d, ndmin;
     __device__ __forceinline__ void prepare(const TileRegs<MESH_Q4_K> &R, int g) {
-        const float d = f16_bits_to_f32((uint16_t)(R.hdr.x & 0xFFFFu));
-        const float dmin = f16_bits_to_f32((uint16_t)(R.hdr.x >> 16));
+        d = f16_bits_to_f32((uint16_t)(R.hdr.x & 0xFFFFu));
+        ndmin = -f16_bits_to_f32((uint16_t)(R.hdr.x >> 16));
         // 6-bit (scale, min) of sub-blocks 2g and 2g+1 (get_scale_min_k4 of ggml-quants.c)
-        const uint32_t scw = g < 2 ? (R.hdr.y & 0x3F3F3F3Fu) : ((R.hdr.w & 0x0F0F0F0Fu) | ((R.hdr.y >> 2) & 0x30303030u));
-        const uint32_t mnw = g < 2 ? (R.hdr.z & 0x3F3F3F3Fu) : (((R.hdr.w >> 4) & 0x0F0F0F0Fu) | ((R.hdr.z >> 2) & 0x30303030u));
+        const uint32_t first = lanes_mask(g < 2);
+        const uint32_t scw = bits_of(first, R.hdr.y & 0x3F3F3F3Fu, (R.hdr.w & 0x0F0F0F0Fu) | ((R.hdr.y >> 2) & 0x30303030u));
+        const uint32_t mnw = bits_of(first, R.hdr.z & 0x3F3F3F3Fu, ((R.hdr.w >> 4) & 0x0F0F0F0Fu) | ((R.hdr.z >> 2) & 0x30303030u));
         const int sh = (g & 1) * 16;
-        const float sa = (float)((scw >> sh) & 0xFFu), sb = (float)((scw >> (sh + 8)) & 0xFFu);
-        s_lo = h2_of(sa);                                            // integers below 64: exact
-        s_hi = h2_of(sb);
-        c_lo = h2_of(8.0f * d * sa - dmin * (float)((mnw >> sh) & 0xFFu));
-        c_hi = h2_of(8.0f * d * sb - dmin * (float)((mnw >> (sh + 8)) & 0xFFu));
-        d2 = h2_of(d);                                               // d is an f16 in the block: exact
-        w[0] = R.qa.x; w[1] = R.qa.y; w[2] = R.qa.z; w[3] = R.qa.w;
-        w[4] = R.qb.x; w[5] = R.qb.y; w[6] = R.qb.z; w[7] = R.qb.w;
-        kbase = 64 * g;
+        s_lo = h2_of((float)((scw >> sh) & 0xFFu));                  // integers below 64: exact
+        s_hi = h2_of((float)((scw >> (sh + 8)) & 0xFFu));
+        o_lo = s_lo * h2_of(-1024.f);                                // (powers of two times them: exact too)
+        o_hi = s_hi * h2_of(-64.f);
+        m_lo = h2_bits(h2_of((float)((mnw >> sh) & 0xFFu)));
+        m_hi = h2_bits(h2_of((float)((mnw >> (sh + 8)) & 0xFFu)));
+        // (values the compiler cannot see make mask and base one and-or; with literals it forms an and, then an or)
+        mask_lo = 0x000F000Fu; mask_hi = 0x00F000F0u; base_lo = 0x64006400u; base_hi = 0x54005400u;
+        asm("" : "+s"(mask_lo), "+s"(mask_hi), "+v"(base_lo), "+v"(base_hi));
+        const uint32_t q[8] = {R.qa.x, R.qa.y, R.qa.z, R.qa.w, R.qb.x, R.qb.y, R.qb.z, R.qb.w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w[i] = __builtin_amdgcn_perm(0u, q[i], 0x03010200u);      // bytes 0 2 1 3: neighbours 16 bits apart
     }
-    // MFMA t: t < 4 low nibbles (sub-block 2g), bytes 8t..8t+7; t >= 4 high nibbles (sub-block 2g+1)
+    // MFMA t: t < 4 low nibbles (sub-block 2g), bytes 8t..8t+7; t >= 4 high nibbles (sub-block 2g+1).  0x6400 | q is 1024 + q, and
+    // 0x5400 | q << 4 is 64 + q; one fma takes the offset off and multiplies by the sub-block's integer scale: q * sc <= 945.
     __device__ __forceinline__ h8_t frag(int t) const {
         const int tt = t & 3;
-        const bool high = t >= 4;
-        const uint32_t v0 = (high ? w[2 * tt] >> 4 : w[2 * tt]) & 0x0F0F0F0Fu;
-        const uint32_t v1 = (high ? w[2 * tt + 1] >> 4 : w[2 * tt + 1]) & 0x0F0F0F0Fu;
-        const h2_t off = {(_Float16)1032.f, (_Float16)1032.f};       // 1024 + 8: the centred quant q - 8
-        return dequant8(v0, v1, off, high ? s_hi : s_lo, d2, high ? c_hi : c_lo);
+        u4_t a;                                                      // built as four dwords: no half-register moves
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t v = i & 1 ? w[2 * tt + (i >> 1)] >> 8 : w[2 * tt + (i >> 1)];
+            a[i] = t < 4 ? h2_bits(__builtin_elementwise_fma(h2_bits((v & mask_lo) | base_lo), s_lo, o_lo))
+                         : h2_bits(__builtin_elementwise_fma(h2_bits((v & mask_hi) | base_hi), s_hi, o_hi));
+        }
+        return __builtin_bit_cast(h8_t, a);
     }
-    __device__ __forceinline__ int koff(int t) const { return kbase + 32 * (t >> 2) + 8 * (t & 3); }
+    __device__ __forceinline__ h8_t minimum(int t) const {
+        const uint32_t v = t < 4 ? m_lo : m_hi;
+        return __builtin_bit_cast(h8_t, u4_t{v, v, v, v});
+    }
 };
 
 template <> struct TileFrags<MESH_Q6_K> {
+    static constexpr bool MINIMUM = false;
     uint32_t v[4][4];      // [t4][dword]: six-bit quants in bytes, elements 128n + 32 t4 + 16u + 4 dword + byte
-    h2_t s[4], d2;
-    int kbase;
+    h2_t s[4];
+    float d;
     __device__ __forceinline__ void prepare(const TileRegs<MESH_Q6_K> &R, int g) {
         const int n = g >> 1, u = g & 1;
-        const float d = f16_bits_to_f32((uint16_t)R.d);
+        d = f16_bits_to_f32((uint16_t)R.d);
         const uint32_t la[4] = {R.qla.x, R.qla.y, R.qla.z, R.qla.w}, lb[4] = {R.qlb.x, R.qlb.y, R.qlb.z, R.qlb.w};
         const uint32_t qh[4] = {R.qh.x, R.qh.y, R.qh.z, R.qh.w};
-        const uint32_t scw0 = n ? R.sc.z : R.sc.x, scw1 = n ? R.sc.w : R.sc.y;
+        const uint32_t upper = lanes_mask(n != 0), scw0 = bits_of(upper, R.sc.z, R.sc.x), scw1 = bits_of(upper, R.sc.w, R.sc.y);
         s[0] = h2_of((float)(int8_t)((scw0 >> (8 * u)) & 0xFFu));     // int8: exact
         s[1] = h2_of((float)(int8_t)((scw0 >> (16 + 8 * u)) & 0xFFu));
         s[2] = h2_of((float)(int8_t)((scw1 >> (8 * u)) & 0xFFu));
         s[3] = h2_of((float)(int8_t)((scw1 >> (16 + 8 * u)) & 0xFFu));
-        d2 = h2_of(d);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             v[0][j] = (la[j] & 0x0F0F0F0Fu) | ((qh[j] << 4) & 0x30303030u);
@@ -154,18 +161,18 @@ template <> struct TileFrags<MESH_Q6_K> {
             v[2][j] = ((la[j] >> 4) & 0x0F0F0F0Fu) | (qh[j] & 0x30303030u);
             v[3][j] = ((lb[j] >> 4) & 0x0F0F0F0Fu) | ((qh[j] >> 2) & 0x30303030u);
         }
-        kbase = 128 * n + 16 * u;
     }
-    // MFMA t = 2 t4 + h: elements 8h..8h+7 of the 16-element scale group t4
+    // MFMA t = 2 t4 + h: elements 8h..8h+7 of the 16-element scale group t4.  (q - 32) * sc reaches 32 * 128 = 4096, one bit more
+    // than f16 holds exactly: products above 2048 with an odd value round by 2^-12 of themselves.
     __device__ __forceinline__ h8_t frag(int t) const {
         const int t4 = t >> 1, h = t & 1;
         const h2_t off = {(_Float16)1056.f, (_Float16)1056.f};       // 1024 + 32: quants are stored with a bias of 32
-        const h2_t zero = {(_Float16)0.f, (_Float16)0.f};
-        // ((q - 32) * sc reaches 32 * 128 = 4096, one bit more than f16 holds exactly: products above 2048 with an odd value
-        // round by 2^-12 of themselves, below the rounding of the multiplication by d that follows)
-        return dequant8(v[t4][2 * h], v[t4][2 * h + 1], off, s[t4], d2, zero);
+        u4_t a;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            a[i] = h2_bits((h2_bits(__builtin_amdgcn_perm(0x64646464u, v[t4][2 * h + (i >> 1)], i & 1 ? 0x04030402u : 0x04010400u)) - off) * s[t4]);
+        return __builtin_bit_cast(h8_t, a);
     }
-    __device__ __forceinline__ int koff(int t) const { return kbase + 32 * (t >> 1) + 8 * (t & 1); }
 };
 
 // B fragments of one super-block for this lane: 8 MFMAs x 8 f16
@@ -209,6 +216,22 @@ __device__ __forceinline__ void to_mfma_lanes(TileRegs<MESH_Q6_K> &R, int src_la
 // element (row k, column t) of k8-major f16 activations with K rows per column: block t / 16 of 16 * K halfs
 __device__ __forceinline__ size_t k8_at(int K, int k, int t) { return (size_t)(t >> 4) * 16 * K + ((size_t)(k >> 3) * 16 + (t & 15)) * 8 + (k & 7); }
 
+// 1 KB from memory to LDS without passing registers: the 16 bytes at base + off (bytes, a lane's own) go to dst + 4 lane (dst
+// uniform).  As text: behind the builtin the compiler waits for every load in flight at the next cross-lane move, which counts as
+// an LDS access.  Its own counts stay right, a load it does not know of only makes a wait stricter; the reader waits itself.
+__device__ __forceinline__ void load_to_lds_16(const float *base, int off, float *dst) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const unsigned place = (unsigned)(unsigned long long)(__attribute__((address_space(3))) float *)dst;
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"         // (m0 is reserved: named so that the compiler keeps its own uses away)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(place)), "v"(off), "s"(base) : "memory", "m0");
+#pragma clang diagnostic pop
+#endif
+}
+// KB per wave and column block that hold a wave's share of the partial sums
+constexpr int NORM_CHUNKS = SKINNY_F16_NORM_PARTS_MAX / SK_WAVES * SK_NT / 256;
+static_assert(NORM_CHUNKS * 256 * SK_WAVES == SKINNY_F16_NORM_PARTS_MAX * SK_NT, "shares of whole KB");
+
 // most tile-rows a workgroup of the launch has (p_split = tile-rows per workgroup | workgroups with one more << 16)
 __device__ __forceinline__ int rows_here_max(unsigned p_split) { return (int)(p_split & 0xFFFFu) + ((p_split >> 16) ? 1 : 0); }
 
@@ -224,7 +247,6 @@ __device__ __forceinline__ void skinny_workgroup(int bx, const _Float16 *p_x, co
     extern __shared__ __align__(16) uint8_t smem[];
     float *red = reinterpret_cast<float *>(smem);         // [KS][rows_here][NU][16 rows][16 NC columns]
     constexpr int TB = TileRegs<TYPE>::BYTES;
-    constexpr int SK_DEPTH = TYPE == MESH_Q4_K ? SK_DEPTH_Q4 : SK_DEPTH_Q6;
     const int K = p_K, nsb = K / QK_K;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);       // scalar: tile addresses become SGPR base + lane offset
@@ -239,10 +261,11 @@ __device__ __forceinline__ void skinny_workgroup(int bx, const _Float16 *p_x, co
     const size_t row_stride = (size_t)nsb * TB;
     // B fragments: lane (n = m, g) supplies column n, quarter g (columns beyond T hold zeros)
     const int lane_off = (TYPE == MESH_Q4_K ? 64 * g : 128 * (g >> 1) + 16 * (g & 1)) * 16 + m * 8;
-    // flat tile index f -> (ii, seg); seg -> (local tile-row j, matrix u)
+    // flat tile index f = ii * SEGS + seg; seg -> (local tile-row j, matrix u).  A segment past the workgroup's rows reads the wave's
+    // first one again and is dropped at the end: the walk has no branch (see below).
     auto seg_valid = [&](int seg) { return rs + RS * (seg / NU) < rows_here; };
     auto tile_ptr = [&](int ii, int seg) -> const uint8_t * {
-        const int tr = tr0 + rs + RS * (seg / NU);
+        const int tr = tr0 + rs + (seg_valid(seg) ? RS * (seg / NU) : 0);
         int mi = seg % NU;
         if (NU == 1) mi = (tr >= p_begin1 ? 1 : 0) + (tr >= p_begin2 ? 1 : 0);
         // (offsets added under conditions: an indexed kernel-argument array is fetched with a load, and a three-way
@@ -250,9 +273,10 @@ __device__ __forceinline__ void skinny_workgroup(int bx, const _Float16 *p_x, co
         const uint8_t *wb = p_w0 + (mi >= 1 ? p_w1 - p_w0 : (ptrdiff_t)0) + (mi >= 2 ? p_w2 - p_w1 : (ptrdiff_t)0);
         return wb + (size_t)tr * row_stride + (size_t)(ks + KS * ii) * TB;
     };
-    // flat tile index f = ii * SEGS + seg, invalid segments included as bubbles; a wave without a valid first
-    // segment has nothing at all
-    const int total = seg_valid(0) ? n_i * SEGS : 0;
+    // a wave without a valid first segment has nothing at all
+    const bool any = n_i > 0 && seg_valid(0);
+    constexpr int RB = SEGS % SK_DEPTH == 0 ? 1 : SK_DEPTH;      // super-blocks per round: ring slots static inside it
+    static_assert(RB <= 2 && RB * SEGS % SK_DEPTH == 0, "ring slots must be static inside a round, and at most one super-block left over");
 
     constexpr int NT = SK_NT * NC;                        // activation columns of this launch
     TileRegs<TYPE> ring[SK_DEPTH];
@@ -262,104 +286,155 @@ __device__ __forceinline__ void skinny_workgroup(int bx, const _Float16 *p_x, co
 #pragma unroll
         for (int c = 0; c < NC; ++c) D[s][c] = f4_t{0.f, 0.f, 0.f, 0.f};
 
-    // Loads are never under a branch of their own: an index past the end or an invalid segment is clamped to a tile
-    // the wave owns (a cache hit).  The compiler then knows exactly how many loads are in flight at every point
-    // and waits for one tile without draining the others; a load under a branch makes it assume the worst at the
-    // join, which in an unrolled pipeline degenerates to waiting for everything.
-    auto load_tile = [&](TileRegs<TYPE> &dst, int f, int seg) {
-        const bool ok = f < total && seg_valid(seg);
-        dst.load(tile_ptr(ok ? f / SEGS : n_i - 1, ok ? seg : 0), lane);
-    };
+    // The walk has no branch inside a round of tiles: a tile past the end is the wave's last one again (a cache hit).  The compiler
+    // then knows how many loads are in flight at every point and waits for one tile without draining the others; with a branch
+    // around a tile or a load it assumes the worst at the join, and every round waited for everything it had just requested.
+    auto load_tile = [&](TileRegs<TYPE> &dst, int ii, int seg) { dst.load(tile_ptr(ii < n_i ? ii : n_i - 1, seg), lane); };
     // Activation fragments: 8 KB per super-block, column block and wave.  Only ONE super-block is held (32 registers per
     // column block) and every fragment is fetched again, for the next super-block, right behind the last MFMAs that read
     // it: one tile's time ahead of its use, enough for a hit in L2.  (Two whole super-blocks in registers, fetched a
-    // super-block ahead, cost 32 more registers per column block and measured 6% slower at 16 columns.)  A tile that
-    // is not computed (past the end, invalid segment) issues the same loads in the same order, so that the compiler's
-    // count of loads in flight is the same along both paths.
+    // super-block ahead, cost 32 more registers per column block and measured 6% slower at 16 columns.)
     BFrags<TYPE> Bw[NC];
     auto frag_koff = [](int t) { return (TYPE == MESH_Q4_K ? 32 * (t >> 2) + 8 * (t & 3) : 32 * (t >> 1) + 8 * (t & 1)) * 16; };
-    auto b_base = [&](int sb, int c) { return p_x + (size_t)c * SK_NT * K + (size_t)sb * (QK_K * 16) + lane_off; };
-    auto step = [&](const TileRegs<TYPE> &loaded, f4_t (&acc)[NC], bool valid, bool refill, int next_sb) {
-        const _Float16 *nb[NC];
+    auto step = [&](const TileRegs<TYPE> &loaded, f4_t (&acc)[NC], bool refill, int next_ii) {
+        const _Float16 *nb = p_x + (size_t)(ks + KS * (next_ii < n_i ? next_ii : n_i - 1)) * (QK_K * 16);
+        TileRegs<TYPE> tile = loaded;
+        to_mfma_lanes(tile, src_lane4);
+        TileFrags<TYPE> F;
+        F.prepare(tile, g);
+        f4_t sum[NC];
+        [[maybe_unused]] f4_t low[NC];
 #pragma unroll
-        for (int c = 0; c < NC; ++c) nb[c] = b_base(next_sb, c);
-        if (valid) {
-            TileRegs<TYPE> tile = loaded;
-            to_mfma_lanes(tile, src_lane4);
-            TileFrags<TYPE> F;
-            F.prepare(tile, g);
+        for (int c = 0; c < NC; ++c) sum[c] = low[c] = f4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                const h8_t af = F.frag(t);
+        for (int t = 0; t < 8; ++t) {
+            const h8_t wf = F.frag(t);
 #pragma unroll
-                for (int c = 0; c < NC; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, __builtin_bit_cast(h8_t, Bw[c].b[t]), acc[c], 0, 0, 0);
-                if (refill) {
-#pragma unroll
-                    for (int c = 0; c < NC; ++c) Bw[c].b[t] = ldg<uint4>(nb[c] + frag_koff(t));
-                }
+            for (int c = 0; c < NC; ++c) {
+                sum[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, Bw[c].b[t]), wf, sum[c], 0, 0, 0);
+                if constexpr (TileFrags<TYPE>::MINIMUM)
+                    low[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, Bw[c].b[t]), F.minimum(t), low[c], 0, 0, 0);
             }
-        } else if (refill) {
+            if (refill) {
 #pragma unroll
-            for (int t = 0; t < 8; ++t)
-#pragma unroll
-                for (int c = 0; c < NC; ++c) Bw[c].b[t] = ldg<uint4>(nb[c] + frag_koff(t));
+                for (int c = 0; c < NC; ++c) Bw[c].b[t] = ldg<uint4>(nb + (size_t)c * SK_NT * K + lane_off + frag_koff(t));
+            }
         }
-    };
-    if (total > 0) {
+        // a lane's outputs are all of weight row m, whose scales it holds
 #pragma unroll
-        for (int f = 0; f < SK_DEPTH; ++f) load_tile(ring[f], f, f % SEGS);
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                acc[c][i] = fmaf(F.d, sum[c][i], acc[c][i]);
+                if constexpr (TileFrags<TYPE>::MINIMUM) acc[c][i] = fmaf(F.ndmin, low[c][i], acc[c][i]);
+            }
+    };
+    if (any) {
+#pragma unroll
+        for (int f = 0; f < SK_DEPTH; ++f) load_tile(ring[f], f / SEGS, f % SEGS);
 #pragma unroll
         for (int c = 0; c < NC; ++c) Bw[c].load(p_x + (size_t)c * SK_NT * K, lane_off, ks);
-        constexpr int RB = SEGS % SK_DEPTH == 0 ? 1 : SK_DEPTH;      // rounds per unrolled block: ring slots static inside it
-        constexpr int UB = RB * SEGS;
-        static_assert(UB % SK_DEPTH == 0, "ring slots must be static inside a block");
-        for (int blk = 0; blk * RB < n_i; ++blk) {
+    }
+    // What the tail of the workgroup reads is requested here, behind the first tiles: fetched where it is used, the norm's
+    // partial sums cost 2.9 us behind the weight stream, the residual or the rotation's operands 1.5 - 2.
+    // (Branch-free: a launch or thread that has no use for an operand reads the first activations instead.)
+    const float *const idle = reinterpret_cast<const float *>(p_x);
+    float *const nrm = red + (size_t)KS * rows_here_max(p_split) * NU * 16 * NT;        // [SK_WAVES][NT] sums of the consumer side
+    float *const wsum = nrm + SK_WAVES * NT;                                            // [SK_WAVES][NT] of the producer side
+    float *const my_parts = wsum + SK_WAVES * NT + wave * (NORM_CHUNKS * NC * 256);     // this wave's share of the partial sums
+    const int parts_per = a.ni_part ? (a.ni_parts + SK_WAVES - 1) / SK_WAVES : 0, parts_end = a.ni_part ? a.ni_parts : 0;
+    {
+        const float *src = a.ni_part ? a.ni_part : idle;
+        const int last = a.ni_part ? a.ni_parts * NT - 4 : 4 * 63;
 #pragma unroll
-            for (int q = 0; q < UB; ++q) {
-                const int r = q / SEGS, seg = q % SEGS, slot = q % SK_DEPTH;
-                const int ii = blk * RB + r, f = ii * SEGS + seg;
-                step(ring[slot], D[seg], ii < n_i && seg_valid(seg), seg == SEGS - 1, ks + KS * (ii + 1 < n_i ? ii + 1 : n_i - 1));
-                load_tile(ring[slot], f + SK_DEPTH, (q + SK_DEPTH) % SEGS);
+        for (int i = 0; i < NORM_CHUNKS * NC; ++i) {
+            const int at = wave * parts_per * NT + i * 256 + lane * 4;
+            load_to_lds_16(src, 4 * (at < last ? at : last), my_parts + i * 256);
+        }
+    }
+    // outputs of a thread: column tid % NT and row (tid / NT) % 16 of the tile-rows out_j, out_j + OUT_STEP, ...
+    constexpr int OUT_STEP = SK_THREADS / (16 * NT), OUT_PRE = 2;
+    // (a wave's outputs lie in one tile-row: which matrix that is of stays a scalar)
+    const int out_t = tid % NT, out_r = (tid / NT) % 16, out_j = __builtin_amdgcn_readfirstlane(tid / (16 * NT));
+    const bool roped = NU == 1 && a.rope.pos;
+    [[maybe_unused]] float pre_res[OUT_PRE], pre_w[OUT_PRE], pre_freq[OUT_PRE];
+    [[maybe_unused]] bool pre_rot[OUT_PRE];
+    [[maybe_unused]] int pre_pos = 0;
+    auto matrix_of = [&](int tr) { return NU == 1 ? (tr >= a.tile_begin[1] ? 1 : 0) + (tr >= a.tile_begin[2] ? 1 : 0) : 0; };
+    if constexpr (NU == 1) {
+        pre_pos = *(roped && out_t < a.T ? a.rope.pos + out_t : reinterpret_cast<const int32_t *>(idle));
+#pragma unroll
+        for (int k = 0; k < OUT_PRE; ++k) {
+            const int tr = tr0 + out_j + k * OUT_STEP, mi = matrix_of(tr), row = (tr - a.tile_begin[mi]) * TILE_ROWS + out_r;
+            const bool ok = out_j + k * OUT_STEP < rows_here && row < a.M[mi] && out_t < a.T;
+            pre_res[k] = *(ok && a.epi == EPI_RESIDUAL ? a.residual + (size_t)out_t * a.ldres + row : idle);
+            pre_w[k] = *(ok && a.no_x16 ? a.no_w + row : idle);
+            const int dd = roped ? row % a.rope.head_dim : 0;
+            pre_rot[k] = ok && roped && dd < a.rope.n_rot && (a.kind[mi] == GEMV_KIND_Q || a.kind[mi] == GEMV_KIND_K);
+            pre_freq[k] = *(pre_rot[k] ? a.rope.inv_freq + (dd >> 1) : idle);
+        }
+    }
+    if (any) {
+        int ii = 0;
+        for (; ii + RB <= n_i; ii += RB) {
+#pragma unroll
+            for (int q = 0; q < RB * SEGS; ++q) {
+                const int seg = q % SEGS, slot = q % SK_DEPTH;
+                step(ring[slot], D[seg], seg == SEGS - 1, ii + q / SEGS + 1);
+                // (the tile goes out behind the fragments, which are needed first: loads return in order)
+                __builtin_amdgcn_sched_barrier(0);
+                load_tile(ring[slot], ii + (q + SK_DEPTH) / SEGS, (q + SK_DEPTH) % SEGS);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-    }
-    // partial sums of this wave: D[seg] holds rows 4g..4g+3, column m of segment seg
+        if (RB > 1 && ii < n_i) {
 #pragma unroll
-    for (int seg = 0; seg < SEGS; ++seg) {
-        if (total > 0 && seg_valid(seg)) {
-            const int j = rs + RS * (seg / NU), u = seg % NU;
-#pragma unroll
-            for (int c = 0; c < NC; ++c)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) red[((((size_t)ks * rows_here + j) * NU + u) * 16 + 4 * g + i) * NT + c * SK_NT + m] = D[seg][c][i];
+            for (int seg = 0; seg < SEGS; ++seg) step(ring[seg % SK_DEPTH], D[seg], false, 0);
         }
     }
-    // (after the reduction buffer: [NORM_GROUPS][NT] sums of the consumer side, [SK_WAVES][NT] of the producer side)
-    constexpr int NORM_GROUPS = SK_THREADS / NT;          // threads sharing a token column in the epilogue
-    float *nrm = red + (size_t)KS * rows_here_max(p_split) * NU * 16 * NT;
+    // partial sums of this wave: D[seg] holds row m, columns 4g..4g+3 of segment seg
+#pragma unroll
+    for (int seg = 0; seg < SEGS; ++seg) {
+        if (any && seg_valid(seg)) {
+            const int j = rs + RS * (seg / NU), u = seg % NU;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) *reinterpret_cast<f4_t *>(red + ((((size_t)ks * rows_here + j) * NU + u) * 16 + m) * NT + c * SK_NT + 4 * g) = D[seg][c];
+        }
+    }
+    // norm hand-over, consumer side: this wave's share of the partial sums of squares of every column, in order
     if (a.ni_part) {
-        // norm hand-over, consumer side: this thread's share of the partial sums of squares of its epilogue column
-        // (fetched after the weight stream: before it, the wave would wait for them ahead of its first tile loads)
-        float ni_sum = 0.f;
-        for (int p = tid / NT; p < a.ni_parts; p += NORM_GROUPS) ni_sum += a.ni_part[(size_t)p * NT + tid % NT];
-        nrm[tid] = ni_sum;                             // tid = group * NT + column
+        // (a wave that went through a round has requested the last round's fragments and SK_DEPTH tiles behind them: loads return in
+        // order, and those nobody waits for)
+        if (any && n_i >= RB) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 * NC + SK_DEPTH * (TYPE == MESH_Q4_K ? 3 : 5)) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        float ss = 0.f;
+        for (int p = lane / NT; p < parts_per; p += 64 / NT) ss += wave * parts_per + p < parts_end ? my_parts[p * NT + lane % NT] : 0.f;
+        if (NT == 16) ss += __shfl_xor(ss, 16);
+        ss += __shfl_xor(ss, 32);
+        if (lane < NT) nrm[wave * NT + lane] = ss;
+    }
+    [[maybe_unused]] float pre_sin[OUT_PRE], pre_cos[OUT_PRE];
+    if constexpr (NU == 1) {
+#pragma unroll
+        for (int k = 0; k < OUT_PRE; ++k) {
+            pre_sin[k] = pre_cos[k] = 0.f;
+            if (pre_rot[k]) sincosf((float)pre_pos * pre_freq[k], &pre_sin[k], &pre_cos[k]);
+        }
     }
     __syncthreads();
-    // 1 / rms of this thread's column (every output of a thread is of column tid % NT): groups added in order
+    // 1 / rms of this thread's column (every output of a thread is of column tid % NT): waves added in order
     float inv_rms = 1.0f;
     if (a.ni_part) {
         float ss = 0.f;
-        for (int q = 0; q < NORM_GROUPS; ++q) ss += nrm[q * NT + tid % NT];
+#pragma unroll
+        for (int q = 0; q < SK_WAVES; ++q) ss += nrm[q * NT + out_t];
         inv_rms = 1.0f / sqrtf(ss / (float)K + a.ni_eps);
     }
     float no_ss = 0.f;         // producer side: sum of squares of this thread's outputs (one column)
     // outputs of this workgroup: rows_here x 16 rows x T columns; column t is column t % 16 of the f16 layouts' block t / 16
-    for (int o = tid; o < rows_here * 16 * NT; o += SK_THREADS) {
-        const int t = o % NT, r = (o / NT) % 16, j = o / (NT * 16);
-        const int tr = tr0 + j;
-        int mi = 0;
-        if (NU == 1) mi = (tr >= a.tile_begin[1] ? 1 : 0) + (tr >= a.tile_begin[2] ? 1 : 0);
+    const int t = out_t, r = out_r;
+    for (int j = out_j, k = 0; j < rows_here; j += OUT_STEP, ++k) {
+        const int tr = tr0 + j, mi = matrix_of(tr);
         const int row = (tr - a.tile_begin[mi]) * TILE_ROWS + r;
         if (row >= a.M[mi]) continue;
         if (t >= a.T) {                                    // unused columns of the f16 output block stay finite
@@ -379,15 +454,15 @@ __device__ __forceinline__ void skinny_workgroup(int bx, const _Float16 *p_x, co
             // q / k / v row of a token (see gemv.hpp): rotate q and k with the neighbouring row, k and v go to the cache
             const int kind = a.kind[mi], hd = a.rope.head_dim;
             const int head = row / hd, dd = row - head * hd;
-            const int pos = a.rope.pos[t];
+            const int pos = pre_pos;
             float val = s0;
             if (kind != GEMV_KIND_V && dd < a.rope.n_rot) {
                 float sp = 0.f;
                 for (int k2 = 0; k2 < KS; ++k2) sp += red[((((size_t)k2 * rows_here + j) * NU + 0) * 16 + (r ^ 1)) * NT + t];
                 sp *= inv_rms;
                 if (a.bias[mi]) sp += a.bias[mi][row ^ 1];
-                float sn, cs;
-                sincosf((float)pos * a.rope.inv_freq[dd >> 1], &sn, &cs);
+                float sn = k == 0 ? pre_sin[0] : pre_sin[1], cs = k == 0 ? pre_cos[0] : pre_cos[1];
+                if (k >= OUT_PRE) sincosf((float)pos * a.rope.inv_freq[dd >> 1], &sn, &cs);
                 val = (dd & 1) ? sp * sn + s0 * cs : s0 * cs - sp * sn;
             }
             if (kind == GEMV_KIND_Q) {
@@ -403,7 +478,8 @@ __device__ __forceinline__ void skinny_workgroup(int bx, const _Float16 *p_x, co
             if (a.bias[1]) s1 += a.bias[1][row];
             out = (s0 / (1.0f + expf(-s0))) * s1;
         } else if (a.epi == EPI_RESIDUAL) {
-            out = a.residual[(size_t)t * a.ldres + row] + s0;
+            if constexpr (NU == 1) out = (k == 0 ? pre_res[0] : k == 1 ? pre_res[1] : a.residual[(size_t)t * a.ldres + row]) + s0;
+            else out = s0;
         } else {
             out = s0;
         }
@@ -414,7 +490,8 @@ __device__ __forceinline__ void skinny_workgroup(int bx, const _Float16 *p_x, co
             a.y16[k8_at(a.M16, row, t)] = (_Float16)__builtin_amdgcn_fmed3f(out, -65504.f, 65504.f);
         }
         if (a.no_x16) {
-            const float v = out * a.no_w[row];
+            float v = out;
+            if constexpr (NU == 1) v *= k == 0 ? pre_w[0] : k == 1 ? pre_w[1] : a.no_w[row];
             note_f16_clamp(a.sat, v, 0.f);
             a.no_x16[k8_at(a.M[0], row, t)] = (_Float16)__builtin_amdgcn_fmed3f(v, -65504.f, 65504.f);
             no_ss = fmaf(out, out, no_ss);
@@ -424,7 +501,6 @@ __device__ __forceinline__ void skinny_workgroup(int bx, const _Float16 *p_x, co
         // this workgroup's sum of squares per column: the lanes of a wave that share a column, then the waves in order
         if (NT == 16) no_ss += __shfl_xor(no_ss, 16);
         no_ss += __shfl_xor(no_ss, 32);
-        float *wsum = nrm + NORM_GROUPS * NT;
         if (lane < NT) wsum[wave * NT + lane] = no_ss;
         __syncthreads();
         if (tid < NT) {
@@ -512,7 +588,7 @@ static int skinny_grid(int total_rows, int NU, int KS) {
 struct SkinnyLaunch {
     SkinnyKernelArgs ka;
     int type, NU, KS, total_rows, grid, rows_max, segs;
-    size_t smem(int nt) const { return sizeof(float) * ((size_t)KS * rows_max * NU * 16 * nt + (size_t)SK_THREADS + (size_t)SK_WAVES * nt); }
+    size_t smem(int nt) const { return sizeof(float) * ((size_t)KS * rows_max * NU * 16 * nt + 2 * (size_t)SK_WAVES * nt + (size_t)SKINNY_F16_NORM_PARTS_MAX * nt); }
 };
 static int skinny_prepare(const SkinnyF16Args &a, SkinnyLaunch &L) {
     L.type = a.mat[0].type;

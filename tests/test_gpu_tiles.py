@@ -216,3 +216,29 @@ def test_gate_up_of_a_decode_batch(tmp_path, shape, tokens):
     assert np.linalg.norm(got[1] - want) / norm < 4e-3, (shape, tokens)
     # the same inputs and weights of one rounding each, formed in two ways and summed in two orders
     assert np.linalg.norm(got[1] - got[33]) / norm < 2e-3, (shape, tokens)
+
+
+# super-blocks of 256 along K per wave of the f16 skinny GEMM: rounds of two, one left over, waves with one more than others, fewer
+# super-blocks than waves
+@pytest.mark.parametrize("width,ff", [(256, 256), (512, 1280), (768, 3840), (1280, 5376), (2048, 6400)])
+def test_batches_of_decode_steps_along_k(tmp_path, width, ff):
+    """Every product of two layers (q6_K v and down projections in the first) for 4 to 32 decode steps, at K of `width` and `ff`."""
+    m = mesh()
+    cfg = dict(arch="llama", n_layer=2, n_embd=width, n_head=width // 128, n_head_kv=width // 256, head_dim=128, n_ff=ff, n_vocab=256, eps=1e-5, rope=1e4)
+    path = os.path.join(str(tmp_path), "model.gguf")
+    tensors = models.write_model(path, cfg, [0, 1], seed=4)
+    st = m.Stage(path, 0, 2, n_ctx=16, n_seq_max=32, n_batch_max=32)
+    ses = st.session()
+    orc = StageOracle(cfg, tensors, 0, 2, 16, n_seq_max=32)
+    rng = np.random.Generator(np.random.PCG64(5))
+    done = np.zeros(32, np.int32)
+    for T in (4, 11, 16, 17, 32):
+        x = rng.standard_normal((T, width)).astype(np.float32)
+        pos, seq = done[:T].copy(), list(range(T))
+        done[:T] += 1
+        got = ses.decode(x, pos, seq=seq).view(np.float32).reshape(T, width).astype(np.float64)
+        want = orc.forward(x, pos, seq=seq).astype(np.float64)
+        # activations rounded to f16 in front of every product (2^-12 root mean square, seven products and the attention): 4 * 2^-12 * sqrt(8)
+        assert np.linalg.norm(got - want) <= 2.8e-3 * np.linalg.norm(want), (T, np.linalg.norm(got - want) / np.linalg.norm(want))
+    ses.close()
+    st.close()
