@@ -10,17 +10,25 @@
 //   O^T += V^T . P^T     (128 dims x 32 queries, contraction over the 32 keys)
 // Both products are arranged transposed so that a lane owns ONE query column: the softmax maximum and sum of a
 // query are reductions over the lane's own 16 registers plus one cross-half shuffle, and the rescale of O is a
-// per-lane scalar.  K and V tiles are staged once per workgroup in LDS (all heads of the group share them), V
-// transposed on the way in because the contraction index (keys) has to be contiguous in an MFMA operand.
+// per-lane scalar.  K and V tiles are staged once per workgroup in LDS (all heads of the group share them), as rows; the
+// contraction index (keys) has to be contiguous in an MFMA operand, so V is read back with ds_read_b64_tr_b16, which
+// transposes.  f16 rows go from memory to LDS without passing registers, into the buffer the step before has left: the
+// loads of a step have the whole step before it to arrive, and a step costs one barrier.
 // The MFMA k-slots of the second product are the lane's own S^T registers, in the order the hardware leaves them:
 // slot (half, j) of the first MFMA is key 4*half + j (j < 4) or 8 + 4*half + j - 4; the V^T operand is read from LDS
 // with the same key order, so no data moves between lanes.
+//
+// What bounds it: a step of a wave is 32 MFMAs of 32 cycles and ~180 vector instructions with 33 exponentials (~1 200 cycles), two waves
+// to a SIMD.  Llama-3-8B shape, a layer: 2048 tokens 78.7 -> 59.3 us (padded tiles with V transposed on the way in, two barriers a step,
+// four waves a workgroup; of that 74 with rows by direct loads, 63 with two key groups, the rest by the order of pieces and addresses
+// that are constants), 333 tokens behind 1500 36.7 -> 29.5; expert shard 600 tokens 24.2 -> 19.6.
 //
 // Same result as the per-token kernel of attn.hip (ggml's soft_max + mul_mat of the attention block, reached from
 // rpc_server::graph_compute, third_party/llama.cpp/patches/0002-rpc-add-direct-peer-tensor-transfers.patch:443-451)
 // except that Q and the probabilities are rounded to f16 for the matrix cores; sums are f32.
 
 #include <algorithm>
+#include <type_traits>
 
 #include "act_math.hpp"
 #include "attn.hpp"
@@ -29,10 +37,10 @@ namespace mesh {
 
 constexpr int PF_TILE = 32;                 // queries per workgroup
 
-// Column (dword) of key pair kp in dim row `dim` of the transposed V tile.  Rows 32 apart start on the same LDS bank
-// (32 rows of 18 or 34 dwords are a multiple of the 64 banks), and the staging writes of a wave touch four such rows at once; the
-// XOR moves them onto different banks.  It keeps dwords 2j, 2j + 1 neighbours, which the 8-byte fragment reads need.
-__device__ __forceinline__ int pf_vcol(int dim, int kp) { return kp ^ ((dim >> 5) << 2); }
+// Rows of a tile lie in LDS without padding (a load to LDS writes 1 KB in one piece), the 16-byte pieces of row r in the order
+// piece ^ pf_swizzle(r): equal pieces of the 16 rows that a read of K touches at once, and equal 64-byte runs of the 4 rows that a
+// transposing read touches, lie on different banks.  (Rows of 128 halfs all start on bank 0, rows of 64 and 192 on 0 and 32 in turn.)
+template <int D> __host__ __device__ constexpr int pf_swizzle(int row) { return D == 128 ? (row & 3) << 2 | (row >> 2 & 3) : (row & 2) << 1 | (row >> 2 & 3); }
 constexpr int PF_EXPAND_HD = 128;            // kv_expand_kernel's head_dim
 constexpr int PF_EXPAND_MIN_T = 128;         // chunks from this many tokens decode a quantised cache to f16 once, ahead of the walk
 constexpr float PF_RESCALE_STEP = 8.f;      // the softmax reference moves only when the running maximum exceeds it by this (log2)
@@ -41,6 +49,34 @@ typedef _Float16 pf_h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 pf_h2 __attribute__((ext_vector_type(2)));
 typedef float pf_f16v __attribute__((ext_vector_type(16)));
 typedef uint32_t pf_u4 __attribute__((ext_vector_type(4)));
+typedef uint32_t pf_u2 __attribute__((ext_vector_type(2)));
+typedef short pf_s4 __attribute__((ext_vector_type(4)));
+
+// Four halves of one column of a 4-row x 16-column tile: lane i of a group of 16 lanes hands in the address of row i / 4,
+// columns 4 (i % 4) .. + 4, and receives column i of the four rows.
+__device__ __forceinline__ pf_u2 pf_read_transposed(const _Float16 *p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_bit_cast(pf_u2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) pf_s4 *)p));
+#else
+    return pf_u2{0, 0};
+#endif
+}
+// 1 KB from memory to LDS: the 16 bytes at base + off (a lane's own) go to dst + 16 lane (bytes, dst uniform).  As text: the compiler
+// would wait for them at the next access to LDS, the step after waits itself.
+__device__ __forceinline__ void pf_load_to_lds(const uint8_t *base, uint32_t off, const _Float16 *dst) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const unsigned place = (unsigned)(unsigned long long)(__attribute__((address_space(3))) const _Float16 *)dst;
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"         // (m0 is reserved: named so that the compiler keeps its own uses away)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(place)), "v"(off), "s"(base) : "memory", "m0");
+#pragma clang diagnostic pop
+#endif
+}
+__device__ __forceinline__ void pf_step_barrier() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#endif
+}
 
 __device__ __forceinline__ uint32_t pf_pack(float a, float b) {
     const pf_h2 h = {(_Float16)a, (_Float16)b};
@@ -48,9 +84,8 @@ __device__ __forceinline__ uint32_t pf_pack(float a, float b) {
 }
 
 // the 8 values a (key, piece) pair contributes to a tile, as packed f16
-template <int TYPE, int HD>
-__device__ __forceinline__ uint4 pf_row_piece(const uint8_t *row, int piece) {
-    const KvRaw<TYPE> r = kv_load<TYPE, HD>(row, piece * 8);
+template <int TYPE>
+__device__ __forceinline__ uint4 pf_decode(const KvRaw<TYPE> &r) {
     if constexpr (TYPE == MESH_F16) {
         return r.v;
     } else {
@@ -61,35 +96,39 @@ __device__ __forceinline__ uint4 pf_row_piece(const uint8_t *row, int piece) {
         return make_uint4(pf_pack(u[0], u[1]), pf_pack(u[2], u[3]), pf_pack(u[4], u[5]), pf_pack(u[6], u[7]));
     }
 }
+template <int TYPE, int HD>
+__device__ __forceinline__ uint4 pf_row_piece(const uint8_t *row, int piece) { return pf_decode<TYPE>(kv_load<TYPE, HD>(row, piece * 8)); }
 
-// HD, VD: entries of a key and of a value row.  NT: tiles of 32 keys per step (1 or 2; two give the wave two independent score chains and half the barriers per key, at
-// ~50 more registers).  NP: (key, 8-dim piece) pairs of a step one thread carries in registers, at least 4 HD NT /
-// (threads of the workgroup); 0 for small workgroups, which load each step's rows where they write them.
-template <int HD, int VD, int KT, int VT, int NP, int NT>
-__global__ __launch_bounds__(512) void attn_chunk_kernel(const AttnArgs a, int T, int pos0, int seq, int hpw, int fwd_from, int qtiles, int n_ksplit) {
+// HD, VD: entries of a key and of a value row.  NP: KB of a step's keys (and at most as many of its values) that a wave brings, at least
+// HD / 8 / (waves of the workgroup); for quantised rows (key, 8-dim piece) pairs of a thread, which are as many.
+template <int HD, int VD, int KT, int VT, int NP, int KG>
+__global__ __launch_bounds__(512) void attn_chunk_kernel(const AttnArgs a, int T, int pos0, int seq, int hpw, int qtiles, int n_ksplit) {
     constexpr int KRB = kv_row_bytes(KT, HD), VRB = kv_row_bytes(VT, VD);
     constexpr int PIECES = HD / 8, VPIECES = VD / 8;      // 8-dim pieces of a row
     constexpr int NKC = HD / 16, NDB = VD / 32;     // steps of the score product along the dims, 32-dim blocks of the output
-    constexpr int PF_KPITCH = HD + 8;               // halfs per key row of the K tile in LDS (bank-conflict padding)
+    constexpr int NT = 2;                           // tiles of 32 keys per step: two independent score chains
     constexpr int PF_KEYS = 32 * NT;                // keys per step
-    constexpr int PF_VPITCH = PF_KEYS / 2 + 2;      // dwords (key pairs) per dim row of the transposed V tile
-    __shared__ __align__(16) _Float16 sK[PF_KEYS * PF_KPITCH];
-    __shared__ __align__(16) uint32_t sVt[VD * PF_VPITCH];
+    constexpr bool DIRECT = KT == MESH_F16 && VT == MESH_F16;
+    static_assert(!DIRECT || (KRB == HD * 2 && VRB == VD * 2), "f16 rows without gaps");
+    constexpr int PF_STAGE = PF_KEYS * KG;          // keys brought at a time
+    __shared__ __align__(16) _Float16 sK[2][PF_STAGE * HD];
+    __shared__ __align__(16) _Float16 sV[2][PF_STAGE * VD];
     const int tid = threadIdx.x, lane = tid & 63, nthreads = blockDim.x;
     // wave -> (head of the workgroup, one of its `qtiles` consecutive query tiles): groups of fewer than four heads fill the
     // workgroup with several query tiles of the same heads, which share the K / V tiles like heads do
-    const int wave = (tid >> 6) % hpw, qtl = (tid >> 6) / hpw;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), n_waves = nthreads >> 6, own = wv % (hpw * qtiles), kg = wv / (hpw * qtiles);
+    const int wave = own % hpw, qtl = own / hpw;
     const int qcol = lane & 31, half = lane >> 5;
     // the last query tile of a chunk walks the most keys: the launch hands the tiles out from the last one backwards, so
     // that the longest walks start first when the workgroups do not all fit on the chip at once
-    // (a launch whose workgroups all fit at once, two per CU, runs its second half forwards: see attention_chunk)
-    const int lin = (int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
-    const int qg = lin >= fwd_from ? (int)blockIdx.x : (int)(gridDim.x - 1 - blockIdx.x), kvh = blockIdx.y;
+    const int lin = (int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z)), across = (int)(gridDim.y * gridDim.z);
+    const int qg = (int)gridDim.x - 1 - (KG > 1 ? lin / across : (int)blockIdx.x);
+    const int kvh = KG > 1 ? lin % across % (int)gridDim.y : (int)blockIdx.y, bz = KG > 1 ? lin % across / (int)gridDim.y : (int)blockIdx.z;
     const int qt = qg * qtiles + qtl;           // (past the last tile of the chunk: a wave without queries, q_live false)
-    // blockIdx.z = (head group, key split): with n_ksplit > 1 the workgroup walks one n_ksplit-th of the keys and leaves
+    // bz = (head group, key split): with n_ksplit > 1 the workgroup walks one n_ksplit-th of the keys and leaves
     // an un-normalised partial for attn_combine_kernel (short chunks on a long history, which have few query tiles)
-    const int ks = (int)blockIdx.z % n_ksplit;
-    const int h = kvh * a.group + ((int)blockIdx.z / n_ksplit) * hpw + wave;
+    const int ks = bz % n_ksplit;
+    const int h = kvh * a.group + (bz / n_ksplit) * hpw + wave;
     const int tq = qt * PF_TILE + qcol;
     const bool q_live = tq < T;
     const int pos_q = pos0 + tq;
@@ -128,67 +167,58 @@ __global__ __launch_bounds__(512) void attn_chunk_kernel(const AttnArgs a, int T
     const int k_lo = wg_first + ks * per_split;
     const int n_keys = k_lo + per_split < n_keys_wg ? k_lo + per_split : n_keys_wg;   // end of this workgroup's walk
     const int n_keys_mine = n_keys_own < n_keys ? n_keys_own : n_keys;              // and of this wave's
-    // K is staged as it is: (key, 8-dim piece) pairs, 16 bytes each.  V is staged transposed: an item is the same 8 dims
-    // of two neighbouring keys, written as 8 dwords, one per dim, each holding the pair of keys.  Rows past the context
-    // end are clamped (masked below).
-    auto k_row = [&](int k0, int p) {
-        int kr = k0 + p / PIECES;
-        kr = kr < a.n_ctx ? kr : a.n_ctx - 1;
-        return pf_row_piece<KT, HD>(a.kcache + (base + kr) * KRB, p % PIECES);
-    };
-    auto v_row = [&](int k0, int p, int second) {
-        int kr = k0 + 2 * (p / VPIECES) + second;
-        kr = kr < a.n_ctx ? kr : a.n_ctx - 1;
-        return pf_row_piece<VT, VD>(a.vcache + (base + kr) * VRB, p % VPIECES);
-    };
-    auto k_put = [&](int p, const uint4 &r) { *reinterpret_cast<uint4 *>(sK + (p / PIECES) * PF_KPITCH + (p % PIECES) * 8) = r; };
-    auto v_put = [&](int p, const uint4 &r0, const uint4 &r1) {
-        const int kp = p / VPIECES, piece = p % VPIECES;
-        const uint32_t w0[4] = {r0.x, r0.y, r0.z, r0.w}, w1[4] = {r1.x, r1.y, r1.z, r1.w};
-        uint32_t *dst = sVt + piece * 8 * PF_VPITCH + pf_vcol(piece * 8, kp);
+    // Staging.  Rows past the context end are clamped (masked below).
+    const uint8_t *const k_rows = a.kcache + base * KRB, *const v_rows = a.vcache + base * VRB;
+    auto row_of = [&](int key) { return (uint32_t)(key < a.n_ctx ? key : a.n_ctx - 1); };
+    // f16: a wave brings every n_waves-th KB of the tiles
+    auto bring = [&](int k0, int buf) {
 #pragma unroll
-        for (int e2 = 0; e2 < 4; ++e2) {
-            dst[(2 * e2) * PF_VPITCH] = (w0[e2] & 0xffffu) | (w1[e2] << 16);
-            dst[(2 * e2 + 1) * PF_VPITCH] = (w0[e2] >> 16) | (w1[e2] & 0xffff0000u);
+        for (int i = 0; i < NP; ++i) {
+            const int kb = wv + i * n_waves, at = kb * 64 + lane, row = at / PIECES, piece = (at % PIECES) ^ pf_swizzle<HD>(row);
+            if (kb < PF_STAGE * HD / 512) pf_load_to_lds(k_rows, row_of(k0 + row) * KRB + piece * 16, sK[buf] + kb * 512);
+        }
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            const int kb = wv + i * n_waves, at = kb * 64 + lane, row = at / VPIECES, piece = (at % VPIECES) ^ pf_swizzle<VD>(row);
+            if (kb < PF_STAGE * VD / 512) pf_load_to_lds(v_rows, row_of(k0 + row) * VRB + piece * 16, sV[buf] + kb * 512);
         }
     };
-    // With NP > 0 the rows of a step travel through registers: a thread fetches its share of step k0 + 64 right after it
-    // has written that of step k0 to LDS, so the loads are in flight while the step is multiplied.
-    constexpr int NPK = NP > 0 ? NP : 1, NPV = NP > 0 ? (NP + 1) / 2 : 1;
-    uint4 rk[NPK], rv[NPV][2];
-    auto fetch_step = [&](int k0) {
+    // quantised rows travel through registers: requested ahead of a step's products, decoded and written behind them
+    KvRaw<KT> rk[DIRECT ? 1 : NP];
+    KvRaw<VT> rv[DIRECT ? 1 : NP];
+    auto fetch = [&](int k0) {
 #pragma unroll
-        for (int i = 0; i < NPK; ++i) {
+        for (int i = 0; i < NP; ++i) {
             const int p = tid + i * nthreads;
-            if (p < PF_KEYS * PIECES) rk[i] = k_row(k0, p);
-        }
-#pragma unroll
-        for (int i = 0; i < NPV; ++i) {
-            const int p = tid + i * nthreads;
-            if (p < PF_KEYS * VPIECES / 2) { rv[i][0] = v_row(k0, p, 0); rv[i][1] = v_row(k0, p, 1); }
+            if (p < PF_STAGE * PIECES) rk[i] = kv_load<KT, HD>(k_rows + (size_t)row_of(k0 + p / PIECES) * KRB, p % PIECES * 8);
+            if (p < PF_STAGE * VPIECES) rv[i] = kv_load<VT, VD>(v_rows + (size_t)row_of(k0 + p / VPIECES) * VRB, p % VPIECES * 8);
         }
     };
-    if constexpr (NP > 0) fetch_step(k_lo);
-    for (int k0 = k_lo; k0 < n_keys; k0 += PF_KEYS) {
-        if constexpr (NP > 0) {
+    auto put = [&](int buf) {
 #pragma unroll
-            for (int i = 0; i < NPK; ++i) {
-                const int p = tid + i * nthreads;
-                if (p < PF_KEYS * PIECES) k_put(p, rk[i]);
-            }
-#pragma unroll
-            for (int i = 0; i < NPV; ++i) {
-                const int p = tid + i * nthreads;
-                if (p < PF_KEYS * VPIECES / 2) v_put(p, rv[i][0], rv[i][1]);
-            }
-        } else {
-            for (int p = tid; p < PF_KEYS * PIECES; p += nthreads) k_put(p, k_row(k0, p));
-            for (int p = tid; p < PF_KEYS * VPIECES / 2; p += nthreads) v_put(p, v_row(k0, p, 0), v_row(k0, p, 1));
+        for (int i = 0; i < NP; ++i) {
+            const int p = tid + i * nthreads;
+            if (p < PF_STAGE * PIECES) *reinterpret_cast<uint4 *>(sK[buf] + (p / PIECES) * HD + ((p % PIECES) ^ pf_swizzle<HD>(p / PIECES)) * 8) = pf_decode<KT>(rk[i]);
+            if (p < PF_STAGE * VPIECES) *reinterpret_cast<uint4 *>(sV[buf] + (p / VPIECES) * VD + ((p % VPIECES) ^ pf_swizzle<VD>(p / VPIECES)) * 8) = pf_decode<VT>(rv[i]);
         }
-        __syncthreads();
-        if constexpr (NP > 0) {
-            if (k0 + PF_KEYS < n_keys) fetch_step(k0 + PF_KEYS);
+    };
+    // V^T operand: dim 32 db + lane % 32, keys of a 32-key tile 8 quad + 4 half .. + 4 (pf_read_transposed: this lane hands in row
+    // (lane % 16) / 4 of the four, 4 dims)
+    const int tr_row = 4 * half + ((lane & 15) >> 2), tr_piece = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1), tr_at = 4 * (lane & 1);
+    if (k_lo < n_keys) {
+        if constexpr (DIRECT) bring(k_lo, 0);
+        else { fetch(k_lo); put(0); }
+    }
+    // (which buffer is known when compiling: with a switch in a register every LDS address of a step is an addition)
+    auto stage = [&](int ks0, auto which) {
+        constexpr int buf = decltype(which)::value;
+        pf_step_barrier();          // the step's tiles are there, and every wave is done with the other buffer
+        if (ks0 + PF_STAGE < n_keys) {
+            if constexpr (DIRECT) bring(ks0 + PF_STAGE, buf ^ 1);
+            else fetch(ks0 + PF_STAGE);
         }
+        const int k0 = ks0 + kg * PF_KEYS;          // this wave's keys of the step
+        const _Float16 *const tK = sK[buf] + kg * (PF_KEYS * HD), *const tV = sV[buf] + kg * (PF_KEYS * VD);
         // (an earlier query tile of the workgroup is done before the last one, and with a window starts before it)
         if (k0 < n_keys_mine && k0 + PF_KEYS > own_first) {
         // the second 32 keys of the step lie past every query of the tile at the end of the walk
@@ -206,13 +236,13 @@ __global__ __launch_bounds__(512) void attn_chunk_kernel(const AttnArgs a, int T
             for (int kc = 0; kc < NKC; ++kc)
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
-                    const pf_h8 kf = *reinterpret_cast<const pf_h8 *>(sK + (32 * t + qcol) * PF_KPITCH + kc * 16 + 8 * half);
+                    const pf_h8 kf = *reinterpret_cast<const pf_h8 *>(tK + (32 * t + qcol) * HD + ((2 * kc + half) ^ pf_swizzle<HD>(qcol)) * 8);
                     s[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[kc], s[t], 0, 0, 0);
                 }
         } else {
 #pragma unroll
             for (int kc = 0; kc < NKC; ++kc) {
-                const pf_h8 kf = *reinterpret_cast<const pf_h8 *>(sK + qcol * PF_KPITCH + kc * 16 + 8 * half);
+                const pf_h8 kf = *reinterpret_cast<const pf_h8 *>(tK + qcol * HD + ((2 * kc + half) ^ pf_swizzle<HD>(qcol)) * 8);
                 s[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[kc], s[0], 0, 0, 0);
             }
         }
@@ -275,20 +305,54 @@ __global__ __launch_bounds__(512) void attn_chunk_kernel(const AttnArgs a, int T
         l += ps;
 #pragma unroll
         for (int db = 0; db < NDB; ++db) {
-            // dim row db * 32 + qcol, this half's keys of tile t: key pairs 16 * t + 2 * half + 4 * j (+ 1), j = 0 .. 3
-            const uint32_t *vrow = sVt + (db * 32 + qcol) * PF_VPITCH + 2 * half;
+            // keys 8 quad + 4 half .. + 4 of tile t, quad = 0 .. 3: the order of P^T's registers
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
                 if (t == 1 && !two) break;
-                const uint2 a0 = *reinterpret_cast<const uint2 *>(vrow + 16 * t + 4 * (0 ^ db)), a1 = *reinterpret_cast<const uint2 *>(vrow + 16 * t + 4 * (1 ^ db));
-                const uint2 a2 = *reinterpret_cast<const uint2 *>(vrow + 16 * t + 4 * (2 ^ db)), a3 = *reinterpret_cast<const uint2 *>(vrow + 16 * t + 4 * (3 ^ db));
-                const pf_u4 v1 = {a0.x, a0.y, a1.x, a1.y}, v2 = {a2.x, a2.y, a3.x, a3.y};
+                pf_u2 v[4];
+#pragma unroll
+                for (int quad = 0; quad < 4; ++quad) {
+                    const int row = 32 * t + 8 * quad + tr_row;
+                    v[quad] = pf_read_transposed(tV + row * VD + ((4 * db + tr_piece) ^ pf_swizzle<VD>(row)) * 8 + tr_at);
+                }
+                const pf_u4 v1 = {v[0][0], v[0][1], v[1][0], v[1][1]}, v2 = {v[2][0], v[2][1], v[3][0], v[3][1]};
                 o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(pf_h8, v1), pf[t][0], o[db], 0, 0, 0);
                 o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(pf_h8, v2), pf[t][1], o[db], 0, 0, 0);
             }
         }
         }
-        __syncthreads();        // the tiles are overwritten by the next step
+        if constexpr (!DIRECT) {
+            if (ks0 + PF_STAGE < n_keys) put(buf ^ 1);
+        }
+    };
+    for (int ks0 = k_lo; ks0 < n_keys; ks0 += 2 * PF_STAGE) {
+        stage(ks0, std::integral_constant<int, 0>{});
+        if (ks0 + PF_STAGE < n_keys) stage(ks0 + PF_STAGE, std::integral_constant<int, 1>{});
+    }
+    if constexpr (KG > 1) {
+        // the second key group's result joins the first's, through the tiles' memory
+        static_assert(KG == 2 && sizeof(sK) >= 4 * 64 * (VD / 2) * sizeof(float) && sizeof(sV) >= 2 * 4 * 64 * sizeof(float), "four waves' results");
+        float *const s_m = reinterpret_cast<float *>(&sV[0][0]) + own * 64 + lane, *const s_l = s_m + 4 * 64;
+        float *const s_o = reinterpret_cast<float *>(&sK[0][0]) + (size_t)own * 64 * (VD / 2) + lane;
+        __syncthreads();
+        if (kg == 1) {
+            *s_m = m;
+            *s_l = l;
+#pragma unroll
+            for (int db = 0; db < NDB; ++db)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) s_o[(db * 16 + i) * 64] = o[db][i];
+        }
+        __syncthreads();
+        if (kg == 1) return;
+        // (a group that has seen no key has m = -inf, l = 0 and o = 0)
+        const float m1 = *s_m, mm = fmaxf(m, m1), w0 = m == -INFINITY ? 0.f : exp2f(m - mm), w1 = m1 == -INFINITY ? 0.f : exp2f(m1 - mm);
+        l = l * w0 + *s_l * w1;
+        m = mm;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) o[db][i] = o[db][i] * w0 + s_o[(db * 16 + i) * 64] * w1;
     }
     if (n_ksplit > 1) {
         // un-normalised partial and (maximum, sum) of this key split, in the layout of the split-KV decode kernels
@@ -409,7 +473,10 @@ int attention_chunk(const AttnArgs &a_in, int T, int pos0, int seq, hipStream_t 
     const int qtiles = hpw >= 4 ? 1 : hpw == 1 ? 4 : 2;
     const int waves = hpw * qtiles, n_tiles = (T + PF_TILE - 1) / PF_TILE;
     dim3 grid((unsigned)((n_tiles + qtiles - 1) / qtiles), (unsigned)a.n_kv, (unsigned)(a.group / hpw));
-    const dim3 block((unsigned)(64 * waves));
+    // Workgroups of four waves leave a SIMD one wave, whose products wait for its softmax and the other way round (two workgroups fit
+    // a CU, but the longest walks end alone): a second group of four waves takes every other step of 64 keys of the same walks.
+    const int key_groups = waves == 4 ? 2 : 1;
+    const dim3 block((unsigned)(64 * waves * key_groups));
     // A short chunk on a long history has few query tiles, each with a long walk: split the keys of every walk over
     // several workgroups (partials in the caller's split buffers, merged by attn_combine_kernel) until the launch has a
     // workgroup per CU, at most 8 ways, at least 256 keys each, within the buffers' rows of (token, split).
@@ -421,24 +488,19 @@ int attention_chunk(const AttnArgs &a_in, int T, int pos0, int seq, hipStream_t 
         if (n_ksplit > ATTN_SPLITS_CAP) n_ksplit = ATTN_SPLITS_CAP;
     }
     grid.z *= (unsigned)n_ksplit;
-    // When the whole launch is resident at once with two workgroups per CU, the hardware has been seen to give a CU
-    // workgroups i and i + (half the launch): handing the second half its query tiles in forward order pairs a long
-    // walk with a short one on every CU.  (A guess about placement costs nothing when wrong: the tiles are the same.)
-    const int total = (int)(grid.x * grid.y * grid.z);
-    // (half the launch has to be whole rows of query tiles: an even number of (KV head, head group) rows)
-    const int fwd_from = (n_ksplit == 1 && waves <= 4 && (grid.y * grid.z) % 2 == 0 && total <= 2 * pf_n_cu() && total > pf_n_cu()) ? total / 2 : INT32_MAX;
     // (Two tiles per step everywhere.  With 5 heads per KV head one tile per step keeps the kernel under 170 registers, so
     // that two 5-wave workgroups share a CU instead of one: measured slower, 16.5 against 14.8 ms over 32 layers of 4096 tokens.)
     // NP by the threads of the workgroup: 1024 / threads pairs each, rounded up
 #define MESH_CHUNK_LAUNCH(HD, KT, VT)                                                                                     \
     do {                                                                                                                  \
-        if (waves == 8) MESH_LAUNCH((attn_chunk_kernel<HD, HD, KT, VT, 2, 2>), grid, block, 0, stream, a, T, pos0, seq, hpw, fwd_from, qtiles, n_ksplit);      \
-        else if (waves == 6) MESH_LAUNCH((attn_chunk_kernel<HD, HD, KT, VT, 3, 2>), grid, block, 0, stream, a, T, pos0, seq, hpw, fwd_from, qtiles, n_ksplit); \
-        else MESH_LAUNCH((attn_chunk_kernel<HD, HD, KT, VT, 4, 2>), grid, block, 0, stream, a, T, pos0, seq, hpw, fwd_from, qtiles, n_ksplit);                  \
+        if (waves == 8) MESH_LAUNCH((attn_chunk_kernel<HD, HD, KT, VT, 2, 1>), grid, block, 0, stream, a, T, pos0, seq, hpw, qtiles, n_ksplit);      \
+        else if (waves == 6) MESH_LAUNCH((attn_chunk_kernel<HD, HD, KT, VT, 3, 1>), grid, block, 0, stream, a, T, pos0, seq, hpw, qtiles, n_ksplit); \
+        else if (key_groups == 2) MESH_LAUNCH((attn_chunk_kernel<HD, HD, KT, VT, 4, 2>), grid, block, 0, stream, a, T, pos0, seq, hpw, qtiles, n_ksplit); \
+        else MESH_LAUNCH((attn_chunk_kernel<HD, HD, KT, VT, 4, 1>), grid, block, 0, stream, a, T, pos0, seq, hpw, qtiles, n_ksplit);                  \
     } while (0)
     // (a group of one: four waves)
-    if (apart && a.head_dim == 192) MESH_LAUNCH((attn_chunk_kernel<192, 128, MESH_F16, MESH_F16, 6, 2>), grid, block, 0, stream, a, T, pos0, seq, hpw, fwd_from, qtiles, n_ksplit);
-    else if (apart) MESH_LAUNCH((attn_chunk_kernel<128, 64, MESH_F16, MESH_F16, 4, 2>), grid, block, 0, stream, a, T, pos0, seq, hpw, fwd_from, qtiles, n_ksplit);
+    if (apart && a.head_dim == 192) MESH_LAUNCH((attn_chunk_kernel<192, 128, MESH_F16, MESH_F16, 6, 2>), grid, block, 0, stream, a, T, pos0, seq, hpw, qtiles, n_ksplit);
+    else if (apart) MESH_LAUNCH((attn_chunk_kernel<128, 64, MESH_F16, MESH_F16, 4, 2>), grid, block, 0, stream, a, T, pos0, seq, hpw, qtiles, n_ksplit);
     else if (a.head_dim == 64) MESH_CHUNK_LAUNCH(64, MESH_F16, MESH_F16);
     else if (a.k_type == MESH_F16 && a.v_type == MESH_F16) MESH_CHUNK_LAUNCH(128, MESH_F16, MESH_F16);
     else if (a.k_type == MESH_Q8_0 && a.v_type == MESH_Q4_0) MESH_CHUNK_LAUNCH(128, MESH_Q8_0, MESH_Q4_0);

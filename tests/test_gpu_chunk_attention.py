@@ -1,0 +1,45 @@
+"""Attention of prompt chunks at the edges of its steps: 64 keys a wave, 128 a workgroup of two key groups, over cached positions
+that end anywhere in a step, for the head sizes and query heads per KV head that choose its launches."""
+import os
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+import models
+from oracle.stage import StageOracle
+from util import mesh
+
+pytestmark = pytest.mark.gpu
+
+CHUNKS = [(0, 17), (0, 64), (0, 65), (1, 127), (0, 129), (63, 40), (64, 64), (127, 33), (128, 192), (300, 97), (190, 257)]
+# f16 queries, probabilities and activations of one layer's products (2^-12 of themselves, root mean square, ten roundings on the
+# way through the layer, weights of the large tile rounded once more): 4 * 2^-12 * sqrt(12)
+TOL = 3.4e-3
+
+
+# four heads a workgroup; one head and four query tiles; head_dim 64 with two heads and two query tiles; five waves; eight heads
+@pytest.mark.parametrize("name", ["tiny-kv3", "tiny-mha", "tiny-llama", "tiny-g5", "tiny-g8"])
+def test_chunks_end_anywhere_in_a_step(tmp_path, name):
+    m, cfg = mesh(), models.CONFIGS[name]
+    path = os.path.join(str(tmp_path), name + ".gguf")
+    tensors = models.write_model(path, cfg, [0], seed=6)
+    st = m.Stage(path, 0, 1, n_ctx=512, n_seq_max=len(CHUNKS), n_batch_max=320)
+    E, HK, D = cfg["n_embd"], cfg["n_head_kv"], cfg["head_dim"]
+    rng = np.random.Generator(np.random.PCG64(8))
+    ses = st.session()
+    orc = StageOracle(cfg, tensors, 0, 1, 512, n_seq_max=len(CHUNKS), blas=True)
+    for i, (past, T) in enumerate(CHUNKS):
+        if past:
+            k, v = (rng.standard_normal((past, HK, D)).astype(np.float16).view(np.uint16) for _ in "kv")
+            ses.kv_write(0, i, 0, k, v)
+            orc.k[0, i, :, :past], orc.v[0, i, :, :past] = k.transpose(1, 0, 2), v.transpose(1, 0, 2)
+        x = rng.standard_normal((T, E)).astype(np.float32)
+        pos, seq = np.arange(past, past + T), np.full(T, i, np.int32)
+        got = ses.decode(x, pos, seq=seq).view(np.float32).reshape(T, E).astype(np.float64)
+        want = orc.forward(x, pos, seq=seq).astype(np.float64)
+        worst = np.max(np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1))
+        assert np.linalg.norm(got - want) <= TOL * np.linalg.norm(want) and worst <= 2 * TOL, (name, past, T, worst)
+    ses.close()
+    st.close()
