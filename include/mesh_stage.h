@@ -289,6 +289,7 @@ int mesh_session_f16_saturations(mesh_session *session, uint64_t *count);
  *     skinny_norm_fused=1  f16 skinny GEMM: the RMS norms ride in the launches around them
  *     skinny_pair=1        skinny GEMMs: q4_K q/k and a q6_K v projection as one launch (0: one launch per type)
  *     skinny_f16_wide=1    batches of gemm_min_tokens..32 decode steps stay on the f16 skinny GEMM (0: large-tile GEMM)
+ *     gemm_norm_rides=1    split output and down projections of a prefill call write the next norm's rows with their sums
  *     gemm_fused=1         q/k/v and gate/up of a prefill call as one launch each
  *     gemm_xdirect=1       the prefill GEMM reads k8-major activations directly
  *     gemm_big=1           256-row tiles for wide projections of long calls

@@ -1046,7 +1046,101 @@ __global__ __launch_bounds__(256) void gemm_splitk_epilogue_kernel(GemmArgs a, i
     }
 }
 
+// The same for one matrix whose result is the hidden state, with the RMS norm of the next launch's input: a workgroup per token holds
+// the row, so the norm costs a reduction over the workgroup instead of a launch that reads the row again.  The sums are those of
+// the kernel above, in its order.  Bound by the latency of its loads, all of a row's in flight at once; two launches of 5 to 8 us
+// become one of about that.  Chunks through eight 8B-shaped layers, us with it / without: 20 tokens 795 / 841, 40 921 / 970, 64 963 / 1082,
+// 100 1157 / 1273, 200 1596 / 1704, 333 behind 1500 2137 / 2210, 512 2500 / 2625, 800 3849 / 3876; four 32B-shaped layers 40 tokens
+// 734 / 754, 150 1296 / 1338, 400 2217 / 2274: at every count that splits.
+constexpr int SN_THREADS = 512;
+template <int NG>              // groups of 8 elements a thread has: rows of up to NG * 4096
+__global__ __launch_bounds__(SN_THREADS) void gemm_splitk_norm_kernel(GemmArgs a, int row_blocks) {
+    __shared__ float s_ss[SN_THREADS / 64];
+    const size_t ld = (size_t)row_blocks * GM;
+    const int t = blockIdx.x, tid = threadIdx.x;
+    const bool live = t < a.T;
+    float4 v[NG][2], w[NG][2], res[NG][2];
+    float ss = 0.f;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        const int i = 8 * (tid + SN_THREADS * g);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            v[g][h] = w[g][h] = res[g][h] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (!live || i >= a.M) continue;
+            w[g][h] = *reinterpret_cast<const float4 *>(a.next_w + i + 4 * h);
+            res[g][h] = *reinterpret_cast<const float4 *>(a.residual + (size_t)t * a.ldres + i + 4 * h);
+        }
+    }
+    for (int z0 = 0; z0 < a.ksplit; z0 += 4) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            const int i = 8 * (tid + SN_THREADS * g);
+            if (!live || i >= a.M) continue;
+            float4 p[4][2];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int z = z0 + u < a.ksplit ? z0 + u : a.ksplit - 1;
+                const float *src = a.part + ((size_t)z * a.T + t) * ld + i;
+                p[u][0] = *reinterpret_cast<const float4 *>(src);
+                p[u][1] = *reinterpret_cast<const float4 *>(src + 4);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (z0 + u < a.ksplit)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) { v[g][h].x += p[u][h].x; v[g][h].y += p[u][h].y; v[g][h].z += p[u][h].z; v[g][h].w += p[u][h].w; }
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        const int i = 8 * (tid + SN_THREADS * g);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            float4 &o = v[g][h];
+            o.x += res[g][h].x; o.y += res[g][h].y; o.z += res[g][h].z; o.w += res[g][h].w;
+            if (live && i < a.M) *reinterpret_cast<float4 *>(a.Y + (size_t)t * a.ldy + i + 4 * h) = o;
+            ss += (o.x * o.x + o.y * o.y) + (o.z * o.z + o.w * o.w);
+        }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+    if ((tid & 63) == 0) s_ss[tid >> 6] = ss;
+    __syncthreads();
+    float tot = 0.f;
+#pragma unroll
+    for (int k = 0; k < SN_THREADS / 64; ++k) tot += s_ss[k];
+    const float sc = 1.0f / sqrtf(tot / (float)a.M + a.next_eps);
+    _Float16 *yb = a.next_x16 + (size_t)(t >> 4) * 16 * a.M + (size_t)(t & 15) * 8;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        const int i = 8 * (tid + SN_THREADS * g);
+        if (i >= a.M) continue;
+        float o[8];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            o[4 * h] = v[g][h].x * sc * w[g][h].x; o[4 * h + 1] = v[g][h].y * sc * w[g][h].y;
+            o[4 * h + 2] = v[g][h].z * sc * w[g][h].z; o[4 * h + 3] = v[g][h].w * sc * w[g][h].w;
+        }
+#pragma unroll
+        for (int h = 0; h < 4; ++h) note_f16_clamp(a.sat, o[2 * h], o[2 * h + 1]);
+        *reinterpret_cast<uint4 *>(yb + (size_t)(i >> 3) * 128) = make_uint4(pack_h2(o[0], o[1]), pack_h2(o[2], o[3]), pack_h2(o[4], o[5]), pack_h2(o[6], o[7]));
+    }
+}
+
+bool gemm_norm_rides(const GemmArgs &a) {
+    return a.n_seg <= 1 && !a.y16_k8 && !a.bias && a.residual && !a.tiles && a.M % 8 == 0 && a.M <= 2 * 8 * SN_THREADS &&
+           a.ldy % 4 == 0 && a.ldres % 4 == 0 && gemm_split_count(a) > 1;
+}
+
 int gemm_add_slices(const GemmArgs &k, int row_blocks, hipStream_t stream) {
+    if (k.next_x16) {
+        const dim3 grid((unsigned)((k.T + 15) & ~15)), block(SN_THREADS);
+        if (k.M <= 8 * SN_THREADS) MESH_LAUNCH(gemm_splitk_norm_kernel<1>, grid, block, 0, stream, k, row_blocks);
+        else MESH_LAUNCH(gemm_splitk_norm_kernel<2>, grid, block, 0, stream, k, row_blocks);
+        MESH_LAUNCH_CHECK();
+        return MESH_OK;
+    }
     const int t_pad = k.y16_k8 ? (k.T + 15) & ~15 : k.T;
     const size_t n = (size_t)t_pad * row_blocks * (k.y16_k8 ? GM / 8 : GM / 4);
     const unsigned blocks = (unsigned)std::min<size_t>((n + 255) / 256, 4096);
@@ -1111,6 +1205,7 @@ int gemm_split_count(const GemmArgs &a) {
 }
 
 int gemm_kquant(const GemmArgs &a, hipStream_t stream) {
+    if (a.next_x16 && !gemm_norm_rides(a)) return fail(MESH_ERR_INVALID, "gemm: the next norm on a launch it does not fit");
     if (!a.X || a.M <= 0 || a.K <= 0 || a.T <= 0) return fail(MESH_ERR_INVALID, "gemm: null pointer or empty shape");
     if (a.y16_k8 || a.n_seg > 1) {
         if ((!a.Wp && !gemm_tile_takes(a)) || (a.y16_k8 && (a.n_seg > 1 || a.bias || a.residual)) || a.n_seg > 3)

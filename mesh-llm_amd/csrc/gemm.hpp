@@ -48,6 +48,11 @@ struct GemmArgs {
     // the f16 KV cache instead of storing them to their outputs, like the projection epilogues of the decode kernels.
     GemvRope rope;
     int kind[3] = {GEMV_KIND_PLAIN, GEMV_KIND_PLAIN, GEMV_KIND_PLAIN};
+    // Optional, where gemm_norm_rides() says so: the second kernel of a split launch also writes f16(rms_norm(Y) * next_w), k8-major with
+    // T padded to 16 by zeros, to next_x16 (which may be X).
+    const float *next_w = nullptr;
+    float next_eps = 0.f;
+    _Float16 *next_x16 = nullptr;
     // Expert launch (mixture of experts; GEMM layout and k8-major activations only, plain store or SwiGLU): X holds the
     // (token, slot) pairs sorted by expert (moe.hpp: moe_sort), T is its capacity in pair slots, and tile i of `tiles` =
     // {expert, first slot, slots, 0} multiplies slots [first, first + slots) (at most 128; first a multiple of 16) by the
@@ -67,6 +72,8 @@ inline int gemm_pair_row_blocks(int64_t M) { return (int)((M + 63) / 64); }
 int gemm_kquant(const GemmArgs &a, hipStream_t stream);
 // Number of K slices gemm_kquant will use for this launch (1: not split).
 int gemm_split_count(const GemmArgs &a);
+// Whether the launch adds slices in a second kernel that can take the next norm along (one matrix and a residual).
+bool gemm_norm_rides(const GemmArgs &a);
 
 // GEMM layout of a K-quant matrix: a second copy for the prefill GEMM, arranged by the workgroup tile that consumes it.
 // One chunk per (128-row block, 64-element k-step), chunks of a row block consecutive in k.  A chunk holds, for each of

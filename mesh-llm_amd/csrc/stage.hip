@@ -696,9 +696,17 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
     _Float16 *const nx = reinterpret_cast<_Float16 *>(s->norm16);
     const bool norm_ready = nf && s->norm_layer == (int)il;
     s->norm_layer = -1;
+    // split products of a chunk: the launch that adds the slices of the output or the down projection writes the next norm's rows
+    // too, in place of a launch that reads the hidden state again (xn is free by then: its readers are behind)
+    auto norm_rides = [&](GemmArgs &g, const DevTensor &w) {
+        if (!k8 || skinny || !s->tune.gemm_norm_rides || !gemm_norm_rides(g)) return false;
+        g.next_w = static_cast<const float *>(w.data); g.next_eps = hp.rms_eps; g.next_x16 = xn;
+        return true;
+    };
+    bool ffn_norm_rode = false;
     {
         ProfScope ps(s, MESH_PROF_PREP);
-        if (norm_ready) rc = MESH_OK;                        // the previous layer's down projection has left them in norm16
+        if (norm_ready || (!sk8 && s->xn_layer == (int)il)) rc = MESH_OK;    // the previous layer's down projection has left them in norm16
         else if (sk8 && s->xq_layer == (int)il) rc = MESH_OK;     // the previous layer's combine step has left them in s->xq
         else if (sk8) rc = quant16_k8(s->x, static_cast<const float *>(L.attn_norm.data), hp.rms_eps, T, E, s->xq, stream);
         else if (k8) rc = rmsnorm_f16_k8(s->x, static_cast<const float *>(L.attn_norm.data), hp.rms_eps, T, E, xn, stream, s->f16_sat);
@@ -856,12 +864,13 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
         ProfScope ps(s, MESH_PROF_GEMV);
         GemmArgs go = gemm_k8(gemm_of(L.wo, s->xn16, QD, T, s->x, E, nullptr));
         go.residual = s->x; go.ldres = E;
+        ffn_norm_rode = !attn_only && norm_rides(go, L.ffn_norm);
         if ((rc = gemm_kquant(go, stream)) != MESH_OK) return rc;
     }
     if (attn_only) return MESH_OK;
     {
         ProfScope ps(s, MESH_PROF_PREP);
-        if (ffn_norm_fused) rc = MESH_OK;
+        if (ffn_norm_fused || ffn_norm_rode) rc = MESH_OK;
         else if (sk8) rc = quant16_k8(s->x, static_cast<const float *>(L.ffn_norm.data), hp.rms_eps, T, E, s->xq, stream);
         else if (k8) rc = rmsnorm_f16_k8(s->x, static_cast<const float *>(L.ffn_norm.data), hp.rms_eps, T, E, xn, stream, s->f16_sat);
         else rc = rmsnorm_f16(s->x, static_cast<const float *>(L.ffn_norm.data), hp.rms_eps, T, E, xn, E, stream, s->f16_sat);
@@ -960,6 +969,9 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
         ProfScope ps(s, MESH_PROF_GEMV);
         GemmArgs gd = gemm_k8(gemm_of(L.w_down, s->ffn16, FF, T, s->x, E, nullptr));
         gd.residual = s->x; gd.ldres = E;
+        // (the next layer takes this path at this token count if its matrices allow it, see run_layers)
+        const LayerWeights *Ln = il + 1 < st->layers.size() ? &st->layers[il + 1] : nullptr;
+        if (Ln && layer_is_kquant_dense(*Ln) && norm_rides(gd, Ln->attn_norm)) s->xn_layer = (int)il + 1;
         if ((rc = gemm_kquant(gd, stream)) != MESH_OK) return rc;
     }
     return MESH_OK;
@@ -975,6 +987,7 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
     int rc;
     s->xq_layer = -1;
     s->norm_layer = -1;
+    s->xn_layer = -1;
     // a mixture-of-experts layer whose attention block runs on the batched-decode (integer matrix-core) path
     auto moe_attn_skinny = [&](const LayerWeights &Ln) {
         return !Ln.w_gate.present() && T >= std::min(PREFILL_MIN_TOKENS, s->tune.skinny_from()) && T < PREFILL_MIN_TOKENS && s->xn16 && layer_attn_is_kquant(Ln) &&

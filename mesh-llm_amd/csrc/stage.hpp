@@ -126,6 +126,7 @@ struct mesh_session {
     float *norm_part = nullptr;
     int norm_parts = 0;              // partial sums per token the last producer wrote
     int norm_layer = -1;             // layer whose attention norm norm16 / norm_part hold (-1: none)
+    int xn_layer = -1;               // layer whose normalised attention input the down projection before it has left in xn16 (-1: none)
     uint16_t *chunk_kv16 = nullptr;      // quantised KV caches: f16 rows of one sequence and layer for long prefill chunks (attn.hpp)
     size_t xq_tokens = 0;               // tokens the q16 buffer below is sized for
     uint8_t *xq = nullptr;               // 16-bit fixed-point activations of the skinny GEMM (gemm.hpp: q16 layout)

@@ -242,3 +242,32 @@ def test_batches_of_decode_steps_along_k(tmp_path, width, ff):
         assert np.linalg.norm(got - want) <= 2.8e-3 * np.linalg.norm(want), (T, np.linalg.norm(got - want) / np.linalg.norm(want))
     ses.close()
     st.close()
+
+
+# rows of one and two groups of eight a thread, whole and with idle threads; token counts of every tile that splits
+@pytest.mark.parametrize("width,heads", [(768, 6), (2048, 16), (4096, 32), (5120, 40)])
+def test_norms_ride_with_the_sums_of_slices(tmp_path, width, heads):
+    """Chunks whose output and down projections are split: the next norm's rows from the launch that adds the slices against a norm launch of
+    their own, and against the oracle."""
+    m = mesh()
+    cfg = dict(arch="llama", n_layer=3, n_embd=width, n_head=heads, n_head_kv=2, head_dim=128, n_ff=1280, n_vocab=256, eps=1e-5, rope=1e4)
+    path = os.path.join(str(tmp_path), "model.gguf")
+    tensors = models.write_model(path, cfg, [0, 1, 2], seed=4)
+    st = m.Stage(path, 0, 3, n_ctx=256, n_seq_max=1, n_batch_max=256)
+    rng = np.random.Generator(np.random.PCG64(5))
+    for T in (17, 33, 70, 130, 200):
+        x = rng.standard_normal((T, width)).astype(np.float32)
+        x[:, 3] *= 20.0
+        out = []
+        for rides in (1, 0):
+            ses = st.session(gemm_norm_rides=rides)
+            out.append(ses.decode(x, np.arange(T)).view(np.float32).reshape(T, width).astype(np.float64))
+            ses.close()
+        want = StageOracle(cfg, tensors, 0, 3, 256, blas=True).forward(x, np.arange(T)).astype(np.float64)
+        size = np.linalg.norm(want)
+        # the two norms add a row's squares in another order (2^-24 of the scale), which moves a value of f16 where it sits next to a
+        # rounding point: fewer than one in 2^10, by 2^-11 of itself
+        assert np.linalg.norm(out[0] - out[1]) <= 2.0 ** -11 * size, (width, T, np.linalg.norm(out[0] - out[1]) / size)
+        # f16 inputs of seven products a layer and weights rounded once (2^-12 root mean square each): 4 * 2^-12 * sqrt(3 * 10)
+        assert np.linalg.norm(out[0] - want) <= 5.4e-3 * size, (width, T, np.linalg.norm(out[0] - want) / size)
+    st.close()
