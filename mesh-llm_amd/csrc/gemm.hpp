@@ -178,8 +178,9 @@ constexpr int SKINNY_F16_NORM_TOKENS_MAX = 32;
 int rmsnorm_f16_k8(const float *x, const float *w, float eps, int T, int n, _Float16 *y, hipStream_t stream, unsigned *sat = nullptr);
 int pack_f16_k8(const float *x, int T, int n, _Float16 *y, hipStream_t stream, unsigned *sat = nullptr);
 // the same as rmsnorm_f16_k8 for n_slots (a multiple of 16) gathered rows: slot i holds row row_of_slot[i] / row_div of x, zeros when negative
+// (scale: optional 1 / rms of the rows of x)
 int rmsnorm_f16_k8_gather(const float *x, const float *w, float eps, const int32_t *row_of_slot, int row_div, int n_slots, int n, _Float16 *y, hipStream_t stream,
-                          unsigned *sat = nullptr);
+                          unsigned *sat = nullptr, const float *scale = nullptr);
 int swiglu_f16_k8(const float *gate, const float *up, int T, int n, _Float16 *y, hipStream_t stream, unsigned *sat = nullptr);
 
 int rmsnorm_f16(const float *x, const float *w, float eps, int T, int n, _Float16 *y, int ldy, hipStream_t stream, unsigned *sat = nullptr);

@@ -944,18 +944,22 @@ int rmsnorm_f16_k8(const float *x, const float *w, float eps, int T, int n, _Flo
 // The gathered form with one workgroup per block of 16 slots: each wave first sums the squares of four of the block's rows,
 // then thread (k8 group, slot) converts 8 values at a time, so that 16 neighbouring threads write one contiguous 256-byte
 // run of the block.  The sum of squares is taken in another order than in to_k8_kernel (one wave per row instead of four),
-// so the scale can differ from that kernel's in its last bit.
+// so the scale can differ from that kernel's in its last bit; scale, when the router before has it, spares the pass over the rows.
+// Bound by the latency of its loads (4800 slots x 2048, 600 tokens with 8 experts each: 20.1 us when every workgroup added the
+// squares first and a branch kept one piece in flight, 14.1 us so).
 __global__ __launch_bounds__(256) void gather_k8_kernel(const float *__restrict__ x, const float *__restrict__ w, float eps, int n,
-                                                        _Float16 *__restrict__ y, const int32_t *__restrict__ row_of_slot, int row_div, unsigned *sat) {
+                                                        _Float16 *__restrict__ y, const int32_t *__restrict__ row_of_slot, int row_div, unsigned *sat,
+                                                        const float *__restrict__ scale) {
     __shared__ float s_scale[16];
     __shared__ int s_row[16];
     const int blk = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     if (tid < 16) {
         const int r = row_of_slot[blk * 16 + tid];
         s_row[tid] = r < 0 ? -1 : r / row_div;
+        if (scale) s_scale[tid] = r < 0 ? 0.f : scale[r / row_div];
     }
     __syncthreads();
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < 4 && !scale; ++i) {
         const int sl = wave * 4 + i, row = s_row[sl];
         float ss = 0.f;
         if (row >= 0) {
@@ -974,24 +978,24 @@ __global__ __launch_bounds__(256) void gather_k8_kernel(const float *__restrict_
     const int sl = tid & 15, row = s_row[sl];
     const float sc = s_scale[sl];
     _Float16 *yb = y + (size_t)blk * 16 * n + (size_t)sl * 8;
+#pragma unroll 4
     for (int k8 = tid >> 4; k8 < n / 8; k8 += 16) {
-        uint4 o = make_uint4(0u, 0u, 0u, 0u);
-        if (row >= 0) {
-            const float *xt = x + (size_t)row * n + k8 * 8;
-            const float4 v0 = *reinterpret_cast<const float4 *>(xt), v1 = *reinterpret_cast<const float4 *>(xt + 4);
-            const float4 g0 = *reinterpret_cast<const float4 *>(w + k8 * 8), g1 = *reinterpret_cast<const float4 *>(w + k8 * 8 + 4);
-            o = make_uint4(sk_pack_h2(sat, v0.x * sc * g0.x, v0.y * sc * g0.y), sk_pack_h2(sat, v0.z * sc * g0.z, v0.w * sc * g0.w),
-                           sk_pack_h2(sat, v1.x * sc * g1.x, v1.y * sc * g1.y), sk_pack_h2(sat, v1.z * sc * g1.z, v1.w * sc * g1.w));
-        }
+        const float *xt = x + (size_t)(row < 0 ? 0 : row) * n + k8 * 8;       // (no branch around the loads: several pieces travel at once)
+        const float4 v0 = *reinterpret_cast<const float4 *>(xt), v1 = *reinterpret_cast<const float4 *>(xt + 4);
+        const float4 g0 = *reinterpret_cast<const float4 *>(w + k8 * 8), g1 = *reinterpret_cast<const float4 *>(w + k8 * 8 + 4);
+        unsigned *st = row < 0 ? nullptr : sat;        // (an empty slot's zeros come from no value)
+        uint4 o = make_uint4(sk_pack_h2(st, v0.x * sc * g0.x, v0.y * sc * g0.y), sk_pack_h2(st, v0.z * sc * g0.z, v0.w * sc * g0.w),
+                             sk_pack_h2(st, v1.x * sc * g1.x, v1.y * sc * g1.y), sk_pack_h2(st, v1.z * sc * g1.z, v1.w * sc * g1.w));
+        if (row < 0) o = make_uint4(0u, 0u, 0u, 0u);
         *reinterpret_cast<uint4 *>(yb + (size_t)k8 * 128) = o;
     }
 }
 
 int rmsnorm_f16_k8_gather(const float *x, const float *w, float eps, const int32_t *row_of_slot, int row_div, int n_slots, int n, _Float16 *y, hipStream_t stream,
-                          unsigned *sat) {
+                          unsigned *sat, const float *scale) {
     if (n_slots <= 0) return MESH_OK;
     if (n % 8 || n_slots % 16 || !row_of_slot || row_div < 1 || !w) return fail(MESH_ERR_INVALID, "rmsnorm_f16_k8_gather: bad arguments (row length %d, %d slots)", n, n_slots);
-    MESH_LAUNCH(gather_k8_kernel, dim3((unsigned)(n_slots / 16)), dim3(256), 0, stream, x, w, eps, n, y, row_of_slot, row_div, sat);
+    MESH_LAUNCH(gather_k8_kernel, dim3((unsigned)(n_slots / 16)), dim3(256), 0, stream, x, w, eps, n, y, row_of_slot, row_div, sat, scale);
     MESH_LAUNCH_CHECK();
     return MESH_OK;
 }

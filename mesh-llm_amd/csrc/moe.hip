@@ -139,7 +139,8 @@ constexpr int ROUTER_THREADS_WIDE = 256, ROUTER_WIDE_MIN_TOKENS = 512;
 // the logits of this workgroup's token and expert slice (blockIdx.y of gridDim.y), into s_logits and logits_out
 template <int NV, int RT>      // float4 groups per lane = E / 256
 __device__ __forceinline__ void router_logits(const float *__restrict__ x, const float *__restrict__ norm_w, const float *__restrict__ W,
-                                              float *__restrict__ logits_out, int ldx, float eps, int p_n_expert, float *s_logits) {
+                                              float *__restrict__ logits_out, int ldx, float eps, int p_n_expert, float *s_logits,
+                                              float *__restrict__ scale_out = nullptr) {
     constexpr int E = NV * 256, ROUTER_WAVES = RT / 64;
     const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     // element index of a lane's values: 4 * (lane + 64 * i) + c
@@ -154,6 +155,7 @@ __device__ __forceinline__ void router_logits(const float *__restrict__ x, const
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
     const float scale = 1.0f / sqrtf(ss / (float)E + eps);
+    if (scale_out && blockIdx.y == 0 && threadIdx.x == 0) scale_out[t] = scale;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const float4 w = *reinterpret_cast<const float4 *>(norm_w + 4 * (lane + 64 * i));
@@ -196,9 +198,9 @@ template <int NV, int RT = ROUTER_THREADS>
 // (scalar arguments first: preloaded into SGPRs, see gemv.hip)
 __global__ __launch_bounds__(RT) void moe_router_fused_kernel(const float *__restrict__ x, const float *__restrict__ norm_w,
                                                                           const float *__restrict__ W, float *__restrict__ logits_out,
-                                                                          int ldx, float eps, int p_n_expert, const MoeRouteArgs a) {
+                                                                          int ldx, float eps, int p_n_expert, const MoeRouteArgs a, float *__restrict__ scale_out) {
     __shared__ float s_logits[64 * ROUTE_MAX_PER_LANE];
-    router_logits<NV, RT>(x, norm_w, W, logits_out, ldx, eps, p_n_expert, s_logits);
+    router_logits<NV, RT>(x, norm_w, W, logits_out, ldx, eps, p_n_expert, s_logits, scale_out);
     if (gridDim.y > 1) return;
     __syncthreads();
     if ((threadIdx.x >> 6) == 0) route_wave_any(s_logits, a, blockIdx.x, threadIdx.x & 63);
@@ -212,11 +214,12 @@ constexpr int CHUNK_TOKENS = 4, CHUNK_WAVES = 8, CHUNK_THREADS = 64 * CHUNK_WAVE
 template <int NV>
 __global__ __launch_bounds__(CHUNK_THREADS) void moe_router_chunk_kernel(const float *__restrict__ x, const float *__restrict__ norm_w,
                                                                          const float *__restrict__ W, float *__restrict__ logits_out,
-                                                                         int ldx, float eps, int T, const MoeRouteArgs a) {
+                                                                         int ldx, float eps, int T, const MoeRouteArgs a, float *__restrict__ scale_out) {
     constexpr int E = NV * 256;
     __shared__ float s_logits[CHUNK_TOKENS][64 * ROUTE_MAX_PER_LANE];
     const int t0 = blockIdx.x * CHUNK_TOKENS, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     float4 xr[CHUNK_TOKENS][NV];
+    float sc[CHUNK_TOKENS];
 #pragma unroll
     for (int k = 0; k < CHUNK_TOKENS; ++k) {
         const int t = t0 + k < T ? t0 + k : T - 1;
@@ -230,6 +233,7 @@ __global__ __launch_bounds__(CHUNK_THREADS) void moe_router_chunk_kernel(const f
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
         const float scale = 1.0f / sqrtf(ss / (float)E + eps);
+        sc[k] = scale;
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
             const float4 w = *reinterpret_cast<const float4 *>(norm_w + 4 * (lane + 64 * i));
@@ -264,21 +268,25 @@ __global__ __launch_bounds__(CHUNK_THREADS) void moe_router_chunk_kernel(const f
             }
         }
     }
+    if (scale_out && wave == 0 && lane == 0)
+#pragma unroll
+        for (int k = 0; k < CHUNK_TOKENS; ++k)
+            if (t0 + k < T) scale_out[t0 + k] = sc[k];
     __syncthreads();
     if (wave < CHUNK_TOKENS && t0 + wave < T) route_wave_any(s_logits[wave], a, t0 + wave, lane);
 }
 
 int moe_router_fused(const MoeRouteArgs &a, const float *x, int ldx, const float *norm_w, float eps, const float *W, int E,
-                     float *logits_out, int T, hipStream_t stream) {
+                     float *logits_out, int T, hipStream_t stream, float *scale_out) {
     if (T <= 0) return MESH_OK;
     if (!moe_router_fused_supported(E, a.n_expert, a.top_k)) return fail(MESH_ERR_UNSUPPORTED, "moe: fused router for hidden size %d / %d experts", E, a.n_expert);
     const dim3 grid((unsigned)T);
     if (T >= ROUTER_WIDE_MIN_TOKENS && E <= 2048) {
         const dim3 cgrid((unsigned)((T + CHUNK_TOKENS - 1) / CHUNK_TOKENS)), cblock(CHUNK_THREADS);
         switch (E / 256) {
-            case 2: MESH_LAUNCH(moe_router_chunk_kernel<2>, cgrid, cblock, 0, stream, x, norm_w, W, logits_out, ldx, eps, T, a); break;
-            case 4: MESH_LAUNCH(moe_router_chunk_kernel<4>, cgrid, cblock, 0, stream, x, norm_w, W, logits_out, ldx, eps, T, a); break;
-            default: MESH_LAUNCH(moe_router_chunk_kernel<8>, cgrid, cblock, 0, stream, x, norm_w, W, logits_out, ldx, eps, T, a); break;
+            case 2: MESH_LAUNCH(moe_router_chunk_kernel<2>, cgrid, cblock, 0, stream, x, norm_w, W, logits_out, ldx, eps, T, a, scale_out); break;
+            case 4: MESH_LAUNCH(moe_router_chunk_kernel<4>, cgrid, cblock, 0, stream, x, norm_w, W, logits_out, ldx, eps, T, a, scale_out); break;
+            default: MESH_LAUNCH(moe_router_chunk_kernel<8>, cgrid, cblock, 0, stream, x, norm_w, W, logits_out, ldx, eps, T, a, scale_out); break;
         }
         MESH_LAUNCH_CHECK();
         return MESH_OK;
@@ -286,10 +294,10 @@ int moe_router_fused(const MoeRouteArgs &a, const float *x, int ldx, const float
     if (T >= ROUTER_WIDE_MIN_TOKENS) {
         const dim3 block(ROUTER_THREADS_WIDE);
         switch (E / 256) {
-            case 2: MESH_LAUNCH((moe_router_fused_kernel<2, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a); break;
-            case 4: MESH_LAUNCH((moe_router_fused_kernel<4, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a); break;
-            case 8: MESH_LAUNCH((moe_router_fused_kernel<8, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a); break;
-            case 16: MESH_LAUNCH((moe_router_fused_kernel<16, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a); break;
+            case 2: MESH_LAUNCH((moe_router_fused_kernel<2, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
+            case 4: MESH_LAUNCH((moe_router_fused_kernel<4, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
+            case 8: MESH_LAUNCH((moe_router_fused_kernel<8, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
+            case 16: MESH_LAUNCH((moe_router_fused_kernel<16, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
             default: return fail(MESH_ERR_UNSUPPORTED, "moe: fused router for hidden size %d", E);
         }
         MESH_LAUNCH_CHECK();
@@ -297,10 +305,10 @@ int moe_router_fused(const MoeRouteArgs &a, const float *x, int ldx, const float
     }
     const dim3 block(ROUTER_THREADS);
     switch (E / 256) {
-        case 2: MESH_LAUNCH(moe_router_fused_kernel<2>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a); break;
-        case 4: MESH_LAUNCH(moe_router_fused_kernel<4>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a); break;
-        case 8: MESH_LAUNCH(moe_router_fused_kernel<8>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a); break;
-        case 16: MESH_LAUNCH(moe_router_fused_kernel<16>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a); break;
+        case 2: MESH_LAUNCH(moe_router_fused_kernel<2>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
+        case 4: MESH_LAUNCH(moe_router_fused_kernel<4>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
+        case 8: MESH_LAUNCH(moe_router_fused_kernel<8>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
+        case 16: MESH_LAUNCH(moe_router_fused_kernel<16>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
         default: return fail(MESH_ERR_UNSUPPORTED, "moe: fused router for hidden size %d", E);
     }
     MESH_LAUNCH_CHECK();
@@ -471,10 +479,10 @@ int moe_router_group(const MoeRouteArgs &a, const float *x, int ldx, const float
         return MESH_OK;
     }
     switch (E / 256) {
-        case 2: MESH_LAUNCH(moe_router_fused_kernel<2>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la); break;
-        case 4: MESH_LAUNCH(moe_router_fused_kernel<4>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la); break;
-        case 8: MESH_LAUNCH(moe_router_fused_kernel<8>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la); break;
-        case 16: MESH_LAUNCH(moe_router_fused_kernel<16>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la); break;
+        case 2: MESH_LAUNCH(moe_router_fused_kernel<2>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, static_cast<float *>(nullptr)); break;
+        case 4: MESH_LAUNCH(moe_router_fused_kernel<4>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, static_cast<float *>(nullptr)); break;
+        case 8: MESH_LAUNCH(moe_router_fused_kernel<8>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, static_cast<float *>(nullptr)); break;
+        case 16: MESH_LAUNCH(moe_router_fused_kernel<16>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, static_cast<float *>(nullptr)); break;
         default: return fail(MESH_ERR_UNSUPPORTED, "moe: fused router for hidden size %d", E);
     }
     MESH_LAUNCH_CHECK();

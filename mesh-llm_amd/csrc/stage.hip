@@ -500,7 +500,7 @@ static int kquant_session_alloc(mesh_session *s) {
     if (hp.n_expert_used > 0 && !st->layers.empty() && st->layers[0].gate_inp.present()) {
         const size_t ne = (size_t)st->layers[0].gate_inp.M, k = hp.n_expert_used;
         if ((rc = fbuf(&s->moe_logits, B * ne)) || (rc = fbuf(&s->moe_w, B * k)) || (rc = fbuf(&s->moe_out, B * k * hp.n_embd)) ||
-            (rc = fbuf(&s->expert_mask, ne)))
+            (rc = fbuf(&s->expert_mask, ne)) || (rc = fbuf(&s->moe_scale, B)))
             return rc;
         if ((rc = sess_alloc(s, &p, B * k * sizeof(int32_t))) != MESH_OK) return rc;
         s->moe_ids = static_cast<int32_t *>(p);
@@ -1105,10 +1105,12 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
             const bool big = s->moe_sorted.tiles && s->tune.moe_group && (size_t)T * k >= (size_t)MOE_GEMM_MIN_PAIRS_PER_EXPERT * ne &&
                              s->tune.moe_gemm && E % 256 == 0 && ffe % 256 == 0;
             if (big) {
+                const float *scale = nullptr;
                 if (L.gate_inp.type == MESH_F32 && moe_router_fused_supported(E, ne, k)) {
                     ProfScope ps(s, MESH_PROF_GEMV);
                     if ((rc = moe_router_fused(mr, s->x, E, static_cast<const float *>(L.ffn_norm.data), hp.rms_eps,
-                                               static_cast<const float *>(L.gate_inp.data), E, s->moe_logits, T, stream)) != MESH_OK) return rc;
+                                               static_cast<const float *>(L.gate_inp.data), E, s->moe_logits, T, stream, s->moe_scale)) != MESH_OK) return rc;
+                    scale = s->moe_scale;           // (the router has normalised the rows: the gather need not add their squares again)
                 } else {
                     GemvArgs ra2;
                     ra2.n_mat = 1;
@@ -1124,7 +1126,7 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
                     ProfScope ps(s, MESH_PROF_PREP);
                     if ((rc = moe_sort(s->moe_ids, T * k, ne, s->moe_sorted, stream)) != MESH_OK) return rc;
                     if ((rc = rmsnorm_f16_k8_gather(s->x, static_cast<const float *>(L.ffn_norm.data), hp.rms_eps, s->moe_sorted.pair_of_slot, k, slots, E,
-                                                    reinterpret_cast<_Float16 *>(s->moe_x16), stream, s->f16_sat)) != MESH_OK) return rc;
+                                                    reinterpret_cast<_Float16 *>(s->moe_x16), stream, s->f16_sat, scale)) != MESH_OK) return rc;
                 }
                 GemmArgs g;
                 g.W = L.gate_exps.data; g.Wp = L.exps_gate_up_gemm; g.type = L.gate_exps.type;

@@ -133,7 +133,7 @@ struct mesh_session {
     float *gemm_part = nullptr;          // partial tiles of large-tile GEMM launches that split K (gemm.hpp)
     size_t gemm_part_bytes = 0;
     float *ffn_up = nullptr;
-    float *moe_logits = nullptr, *moe_w = nullptr, *moe_out = nullptr, *expert_mask = nullptr;
+    float *moe_logits = nullptr, *moe_w = nullptr, *moe_out = nullptr, *expert_mask = nullptr, *moe_scale = nullptr;
     bool expert_mask_on = false;
     int32_t *moe_ids = nullptr;
     int32_t *moe_items = nullptr, *moe_n_items = nullptr;      // (token, slot) pairs grouped by expert, see moe_group
