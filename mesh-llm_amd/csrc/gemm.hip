@@ -581,15 +581,21 @@ __device__ __forceinline__ void reg_tile(const GemmArgs &a, const uint8_t *wp, i
     if (n <= 0) { wp -= (size_t)k0 * PackedSub<TYPE>::CHUNK; }
     const u32x4 *const xb = n > 0 ? xbase : xbase - (size_t)k0 * 128;
     PackedSub<TYPE> rw[AHEAD];
-    u32x4 rx[NT];
+    // Loads return in order: activations stored a step after they were asked for would have the weights asked for before them arrive
+    // by then too, two chunks ahead instead of AHEAD.  Activations asked for XA steps before, against one: a batch of 32 decode steps of
+    // four layers 5120 wide 821 -> 809 us, eight layers of a 40-token chunk 4096 wide 971 -> 953, a 600-token chunk of 128 experts
+    // 2175 -> 2151.  Two columns of tiles in a dense call with AHEAD spill (40 tokens: 995).
+    constexpr int XA = NT == 1 ? AHEAD : NT > 2 ? 1 : MODE == REG_EXPERT ? AHEAD : 2;       // (the registers that are left at the occupancy)
+    u32x4 rx[XA][NT];
 #pragma unroll
-    for (int i = 0; i < NT; ++i) rx[i] = xb[xo[i]];
+    for (int i = 0; i < NT; ++i) xs[i * 256 + tid] = xb[xo[i]];
+#pragma unroll
+    for (int v = 1; v <= XA; ++v)
+#pragma unroll
+        for (int i = 0; i < NT; ++i) rx[v % XA][i] = (xb + (size_t)(v < last ? v : last) * 128)[xo[i]];
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < AHEAD; ++u) rw[u].load(wp + (size_t)(MODE == REG_EXPERT || u < last ? u : last) * PackedSub<TYPE>::CHUNK, slot);
-#pragma unroll
-    for (int i = 0; i < NT; ++i) xs[i * 256 + tid] = rx[i];
-#pragma unroll
-    for (int i = 0; i < NT; ++i) rx[i] = (xb + (size_t)(1 < last ? 1 : last) * 128)[xo[i]];
     lds_barrier();
     const int at = (lane & 15) + ((lane >> 4) & 1) * 128 + hh * 16;
     for (int kc0 = 0; kc0 < per; kc0 += AHEAD) {
@@ -598,9 +604,9 @@ __device__ __forceinline__ void reg_tile(const GemmArgs &a, const uint8_t *wp, i
             const int kc = kc0 + u;
             // (the other buffer was read a step ago; the step's barrier hands it over)
 #pragma unroll
-            for (int i = 0; i < NT; ++i) xs[((u + 1) & 1) * STEP + i * 256 + tid] = rx[i];
+            for (int i = 0; i < NT; ++i) xs[((u + 1) & 1) * STEP + i * 256 + tid] = rx[(u + 1) % XA][i];
 #pragma unroll
-            for (int i = 0; i < NT; ++i) rx[i] = (xb + (size_t)(kc + 2 < last ? kc + 2 : last) * 128)[xo[i]];
+            for (int i = 0; i < NT; ++i) rx[(u + 1) % XA][i] = (xb + (size_t)(kc + 1 + XA < last ? kc + 1 + XA : last) * 128)[xo[i]];
             const u32x4 *x = xs + (u & 1) * STEP + at;
             if (MODE == REG_EXPERT || kc < n) {                // (an expert's K is a multiple of 256)
                 u32x4 f[2][NT];
