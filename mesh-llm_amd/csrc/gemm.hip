@@ -102,8 +102,10 @@ template <> struct RawSub<MESH_Q4_K> {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             *reinterpret_cast<uint32_t *>(chunk + (s - h + (j & 1)) * 16 + (2 * h + (j >> 1)) * 4) = pair_nibbles((w[2 * j] >> (4 * h)) & 0x0F0F0F0Fu, (w[2 * j + 1] >> (4 * h)) & 0x0F0F0F0Fu);
-        *reinterpret_cast<uint2 *>(chunk + 4096 + s * 8) =
-            make_uint2(__builtin_bit_cast(uint32_t, sc_c), (hdr.x & 0xFFFFu) | (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(-72.f * (float)sc_c[0])) << 16);
+        uint8_t *row = chunk + 4096 + (s >> 1) * 8;
+        row[h] = (uint8_t)(scw >> sh);
+        *reinterpret_cast<uint16_t *>(row + 4 + 2 * h) = (uint16_t)(__builtin_bit_cast(uint32_t, sc_c) >> 16);
+        if (h == 0) *reinterpret_cast<uint16_t *>(row + 2) = (uint16_t)hdr.x;
     }
 };
 
@@ -146,7 +148,6 @@ template <> struct RawSub<MESH_Q6_K> {
     }
     __device__ __forceinline__ void pack(int c, int h, uint8_t *chunk, int s) const {
         const int t4 = 2 * (c & 1) + h;
-        const half2v s01 = {(_Float16)(float)(int8_t)(sc & 0xFFu), (_Float16)(float)(int8_t)(sc >> 8)};
         const uint32_t lw[8] = {la.x, la.y, la.z, la.w, lb.x, lb.y, lb.z, lb.w};
         const uint32_t hw[8] = {ha.x, ha.y, ha.z, ha.w, hb.x, hb.y, hb.z, hb.w};
         uint32_t q[8];
@@ -166,7 +167,9 @@ template <> struct RawSub<MESH_Q6_K> {
         }
 #pragma unroll
         for (int j = 0; j < 2; ++j) *reinterpret_cast<uint32_t *>(chunk + 4096 + (s - h + j) * 8 + h * 4) = hb2[j];
-        *reinterpret_cast<uint2 *>(chunk + 6144 + s * 8) = make_uint2(__builtin_bit_cast(uint32_t, s01), d & 0xFFFFu);
+        uint8_t *row = chunk + 6144 + (s >> 1) * 8;
+        *reinterpret_cast<uint16_t *>(row + 2 * h) = (uint16_t)(sc ^ 0x8080u);
+        *reinterpret_cast<uint16_t *>(row + 4 + 2 * h) = (uint16_t)d;
     }
 };
 
@@ -175,14 +178,15 @@ template <> struct RawSub<MESH_Q6_K> {
 // Eight weights of it are a dword of nibbles, element e at nibble e / 2 + 4 (e % 2): one shift puts a pair into bits 4..7 and
 // 20..23, where or-ing 0x5400 makes two f16 of exactly 64 + q (64 to 127: sixteenths in the lowest bits), and one packed fma with
 // the scale then takes the offset off: (64 + q) sc - (64 + off) sc is (q - off) sc, exactly or rounded once, as (q - off)
-// times sc is; 72 sc (off 8, sc <= 63) and 96 sc (off 32, |sc| <= 128) are f16.  15 instructions for 8 weights of q4_K, 23 of q6_K.
+// times sc is; 72 sc (off 8, sc <= 63) and 96 sc (off 32, |sc| <= 128) are f16.  15 instructions for 8 weights of q4_K, 23 of q6_K,
+// and up to two a scale to make it an f16.
 template <int TYPE> struct PackedSub;
 // Loads of a staging wave's loop (load_staged), from a uniform base plus a 32-bit offset of the lane that stays in its register.  Left to
 // itself the compiler adds 64-bit addresses in the loop, into registers of loads under way, and waits for those.  Down projection of
 // 4096 x 14336, q6_K: 25.6 -> 23.5 us at 100 tokens, 76.4 -> 70.8 at 512, on the 256-row tile at 2048 tokens 258 -> 248 (with the stores of
 // staged_slot); gate / up, q4_K: 48.3 -> 46.6 at 100 tokens, 478 -> 466 at 2048.
 struct StagedSlot { unsigned quants, bits, scales; };
-__device__ __forceinline__ StagedSlot staged_offsets(unsigned s) { return StagedSlot{s * 16, s * 8, (s >> 1) * 16}; }
+__device__ __forceinline__ StagedSlot staged_offsets(unsigned s) { return StagedSlot{s * 16, s * 8, (s >> 1) * 8}; }
 template <class V> __device__ __forceinline__ V load_section(const uint8_t *chunk, int at, unsigned &off) {
     uint64_t base = reinterpret_cast<uint64_t>(chunk) + at;
     asm volatile("" : "+s"(base), "+v"(off));
@@ -199,23 +203,25 @@ __device__ __forceinline__ uint32_t and_or(uint32_t x, uint32_t mask, uint32_t y
     return r;
 }
 __device__ __forceinline__ uint32_t nibble_pair(uint32_t w, int p) { return and_or(p == 0 ? w << 4 : w >> (4 * (p - 1)), 0x00F000F0u, 0x54005400u); }
+// 1024 + byte i of w, twice, exactly
+__device__ __forceinline__ half2v byte_pair(uint32_t w, int i) { return __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, w, 0x04000400u + 0x00010001u * i)); }
 template <> struct PackedSub<MESH_Q4_K> {
-    static constexpr int CHUNK = 6144;
+    static constexpr int CHUNK = 5120;
     uint4 q;
-    uint4 sm;          // per 32 elements: {f16 sc, f16 c}, {f16 d, f16 -72 sc}
+    uint2 sm;          // {byte sc of elements 0..31, of 32..63, f16 d}, {f16 c of elements 0..31, of 32..63}
     __device__ __forceinline__ void load(const uint8_t *__restrict__ chunk, unsigned s) {
         q = *reinterpret_cast<const uint4 *>(chunk + s * 16);
-        sm = *reinterpret_cast<const uint4 *>(chunk + 4096 + (s >> 1) * 16);
+        sm = *reinterpret_cast<const uint2 *>(chunk + 4096 + (s >> 1) * 8);
     }
     __device__ __forceinline__ void load_staged(const uint8_t *chunk, StagedSlot &s) {
         q = load_section<uint4>(chunk, 0, s.quants);
-        sm = load_section<uint4>(chunk, 4096, s.scales);
+        sm = load_section<uint2>(chunk, 4096, s.scales);
     }
     // the eight weights of step j (known at compile time)
     __device__ __forceinline__ uint4 form(int j) const {
-        const uint32_t a = j < 2 ? sm.x : sm.z, b = j < 2 ? sm.y : sm.w;
-        const half2v sc = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(a, a, 0x01000100u)), cc = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(a, a, 0x03020302u));
-        const half2v dd = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(b, b, 0x01000100u)), off = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(b, b, 0x03020302u));
+        const half2v sc = byte_pair(sm.x, j >> 1) - half2v{(_Float16)1024.f, (_Float16)1024.f}, off = sc * half2v{(_Float16)-72.f, (_Float16)-72.f};
+        const half2v dd = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(sm.x, sm.x, 0x03020302u));
+        const half2v cc = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(sm.y, sm.y, j < 2 ? 0x01000100u : 0x03020302u));
         const uint32_t w = j == 0 ? q.x : j == 1 ? q.y : j == 2 ? q.z : q.w;
         uint32_t o[4];
 #pragma unroll
@@ -224,24 +230,24 @@ template <> struct PackedSub<MESH_Q4_K> {
     }
 };
 template <> struct PackedSub<MESH_Q6_K> {
-    static constexpr int CHUNK = 8192;
+    static constexpr int CHUNK = 7168;
     uint4 q;
     uint2 hb;
-    uint4 sc;          // f16 sc of elements 0..15, of 16..31, f16 d, -, f16 sc of elements 32..47, of 48..63, f16 d, -
+    uint2 sc;          // bytes 128 + sc of elements 0..15, 16..31, 32..47, 48..63; f16 d, twice
     __device__ __forceinline__ void load(const uint8_t *__restrict__ chunk, unsigned s) {
         q = *reinterpret_cast<const uint4 *>(chunk + s * 16);
         hb = *reinterpret_cast<const uint2 *>(chunk + 4096 + s * 8);
-        sc = *reinterpret_cast<const uint4 *>(chunk + 6144 + (s >> 1) * 16);
+        sc = *reinterpret_cast<const uint2 *>(chunk + 6144 + (s >> 1) * 8);
     }
     __device__ __forceinline__ void load_staged(const uint8_t *chunk, StagedSlot &s) {
         q = load_section<uint4>(chunk, 0, s.quants);
         hb = load_section<uint2>(chunk, 4096, s.bits);
-        sc = load_section<uint4>(chunk, 6144, s.scales);
+        sc = load_section<uint2>(chunk, 6144, s.scales);
     }
     __device__ __forceinline__ uint4 form(int j) const {
-        const half2v s = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(j < 2 ? sc.x : sc.z, j < 2 ? sc.x : sc.z, j & 1 ? 0x03020302u : 0x01000100u));
+        const half2v s = byte_pair(sc.x, j) - half2v{(_Float16)1152.f, (_Float16)1152.f};
         const half2v off = s * half2v{(_Float16)-96.f, (_Float16)-96.f};
-        const half2v dd = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(sc.y, sc.y, 0x01000100u)), zero = {(_Float16)0.f, (_Float16)0.f};
+        const half2v dd = __builtin_bit_cast(half2v, sc.y), zero = {(_Float16)0.f, (_Float16)0.f};
         const uint32_t w = j == 0 ? q.x : j == 1 ? q.y : j == 2 ? q.z : q.w, hw = j < 2 ? hb.x : hb.y;
         uint32_t o[4];
 #pragma unroll
@@ -1291,7 +1297,7 @@ __global__ __launch_bounds__(256) void gemm_pack_kernel(const uint8_t *__restric
     if (wrow >= M_pad) {
         *reinterpret_cast<uint4 *>(chunk + s * 16) = make_uint4(0, 0, 0, 0);
         if (TYPE == MESH_Q6_K) *reinterpret_cast<uint2 *>(chunk + 4096 + s * 8) = make_uint2(0, 0);
-        *reinterpret_cast<uint2 *>(chunk + (TYPE == MESH_Q6_K ? 6144 : 4096) + s * 8) = make_uint2(0u, 0u);
+        *reinterpret_cast<uint32_t *>(chunk + (TYPE == MESH_Q6_K ? 6144 : 4096) + s * 4) = 0u;
         return;
     }
     RawSub<TYPE> r;

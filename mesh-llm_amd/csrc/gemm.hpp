@@ -79,14 +79,17 @@ bool gemm_norm_rides(const GemmArgs &a);
 // One chunk per (128-row block, 64-element k-step), chunks of a row block consecutive in k.  A chunk holds, for each of
 // the 256 slots s = 2 * row + h (elements 16 j + 8 h .. + 7, j = 0..3, of the row's 64), what a thread that forms them
 // needs, at s * stride of each section, and per row the scales; a load of a wave covers whole lines:
-//   q4_K (6144 B): [256 x 16 B quants: dword j, element e of its eight at nibble e / 2 + 4 (e % 2)]
-//                  [128 x 16 B, per 32 elements: f16 sc (the integer block scale), f16 c = 8 d sc - dmin m, f16 d, f16 -72 sc]
-//   q6_K (8192 B): [256 x 16 B low nibbles, same order][256 x 8 B upper two bits: those of element e of dword j in dword j / 2
+//   q4_K (5120 B): [256 x 16 B quants: dword j, element e of its eight at nibble e / 2 + 4 (e % 2)]
+//                  [128 x 8 B: byte sc (the integer block scale) of the first 32 elements, of the others, f16 d, f16 c = 8 d sc - dmin m
+//                  of the first 32, of the others]
+//   q6_K (7168 B): [256 x 16 B low nibbles, same order][256 x 8 B upper two bits: those of element e of dword j in dword j / 2
 //                  at bit 2 P + 16 (e % 2), P = 4 (j % 2) + e / 2]
-//                  [128 x 16 B, per 32 elements: f16 sc of the first 16, f16 sc of the others, f16 d, unused]
+//                  [128 x 8 B: byte 128 + sc of each 16 elements, f16 d, twice]
 // The kernel forms a weight as ((q - offset) * sc) * d + c: an exact small integer times the super-block's own f16
 // scale, rounded once.  The fields are the ones the kernel would otherwise derive from the block headers, so both
-// layouts give the same bits.  Rows beyond M are zero.
+// layouts give the same bits; the integer scales are bytes, 1024 + byte being an f16 that one permutation makes (five bits a weight
+// of q4_K, seven of q6_K; as f16 they made it six and eight: batches of 32 decode steps of four layers 5120 wide 1.0% slower, the
+// copies a sixth and an eighth larger).  Rows beyond M are zero.
 size_t gemm_packed_bytes(int type, int64_t M, int64_t K);
 int gemm_pack(int type, const void *tiled, void *packed, int64_t M, int64_t K, hipStream_t stream);
 // gate / up pair for the SwiGLU launch: row block b = gate rows [64b, 64b + 64) followed by up rows [64b, 64b + 64)
