@@ -214,6 +214,28 @@ def test_unequal_requests_in_one_call_equal_each_alone(tmp_path, prec):
 
 
 @BOTH
+@pytest.mark.parametrize("lens", [[7, 8, 9, 1, 31, 33, 2, 5], [32, 32, 64, 3], [3, 90, 1, 1, 24, 41], [40, 8, 8, 8, 8]])
+def test_recurrences_of_sequences_that_start_anywhere_in_a_window(tmp_path, lens, prec):
+    """Sequences that begin and end at the edges of the recurrence's runs of 8 tokens and windows of 32, inside them, and across
+    several, from a zero state and then from the state they left."""
+    m = mesh()
+    cfg, w, folder, orc = made(tmp_path, "recurrent-only")
+    st = open_stage(folder, prec, n_seq=len(lens), batch=256)
+    toks, want = [N.prompt(cfg, 2 * n, 60 + i) for i, n in enumerate(lens)], []
+    for t in toks:
+        orc.reset()
+        want.append(orc.forward(t))
+    ses = st.session()
+    for half in (0, 1):
+        cut = [slice(half * n, (half + 1) * n) for n in lens]
+        got = ses.decode(np.concatenate([t[c] for t, c in zip(toks, cut)]), np.concatenate([np.arange(c.start, c.stop) for c in cut]).astype(np.int32),
+                         seq=np.repeat(np.arange(len(lens), dtype=np.int32), lens), in_fmt=m.TOKENS, out_fmt=m.LOGITS).view(np.float32).reshape(sum(lens), -1)
+        assert N.error(got, np.concatenate([x[c] for x, c in zip(want, cut)])) < LIMIT[prec], half
+    ses.close()
+    st.close()
+
+
+@BOTH
 def test_a_sequence_given_back_starts_clean(tmp_path, prec):
     m = mesh()
     cfg, w, folder, orc = made(tmp_path, "mixed")
