@@ -3,12 +3,20 @@
 // A wave takes R rows at a time; its 64 lanes cover 512 consecutive k per 16-byte load and R * U loads are in flight while
 // the R * U before them are multiplied.  The input vector sits in LDS as f32.  Every workgroup derives it itself from what
 // the launch before left (residual update with its output norm, polynomial activation: linear.hpp), which saves a launch
-// between two products; the first weight loads go out before that work and travel behind it.  Sums of squares a later norm
-// needs are left per workgroup and added in workgroup order by the consumer, so the result does not depend on timing.
+// between two products.  Loads return in order, so the vectors it is derived from are requested first, the first weights
+// right behind them, and no branch lies around a weight load (the compiler would wait for all of them at its join): the
+// weights travel while norms are worked out.  What an epilogue reads (state, biases, side embedding) is requested with the
+// weights of its rows.
+// 8192 x 2048 behind two layer norms 12.5 -> 11.3 us (as long where the weights wait for the vectors to arrive: the norms' four sums
+// and the start of the stream are what is left), behind an RMS norm 10.7 -> 9.6, three of 2048 x 2048 with the recurrence's update
+// 9.7 -> 8.2, 2048 x 2048 5.0 -> 4.6 in a model that cycles through its weights.
+// Sums of squares a later norm needs are left per workgroup and added in workgroup order by the consumer, so the result does
+// not depend on timing.
 #include "act_math.hpp"
 #include "linear.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace mesh {
 
@@ -26,16 +34,29 @@ __device__ __forceinline__ float step_wave_sum(float v) {
     v += __shfl_xor(v, 32);
     return v;
 }
-// sum over the workgroup in a fixed order, the same in every thread
-__device__ __forceinline__ float step_block_sum(float v, float *scratch, int lane, int wave) {
-    v = step_wave_sum(v);
-    __syncthreads();
-    if (lane == 0) scratch[wave] = v;
-    __syncthreads();
-    float s = 0.f;
+// N sums over the workgroup in a fixed order, the same in every thread.  Two sums in a row use different slots: the barrier of the
+// second is what keeps a third from overwriting what the first's readers still need.
+typedef float StepScratch[2][STEP_WAVES][4];
+template <int SLOT, int N>
+__device__ __forceinline__ void step_block_sums(float (&v)[N], StepScratch &scratch, int lane, int wave) {
 #pragma unroll
-    for (int w = 0; w < STEP_WAVES; ++w) s += scratch[w];
-    return s;
+    for (int i = 0; i < N; ++i) v[i] = step_wave_sum(v[i]);
+    if (lane == 0)
+#pragma unroll
+        for (int i = 0; i < N; ++i) scratch[SLOT][wave][i] = v[i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        v[i] = 0.f;
+#pragma unroll
+        for (int w = 0; w < STEP_WAVES; ++w) v[i] += scratch[SLOT][w][i];
+    }
+}
+template <int SLOT>
+__device__ __forceinline__ float step_block_sum(float v, StepScratch &scratch, int lane, int wave) {
+    float s[1] = {v};
+    step_block_sums<SLOT>(s, scratch, lane, wave);
+    return s[0];
 }
 
 // four elements of a vector of K, zeros behind its end
@@ -43,73 +64,120 @@ __device__ __forceinline__ float4 ln_load4(const float *p, int k, int K) {
     if (k + 4 <= K) return *reinterpret_cast<const float4 *>(p + k);
     return make_float4(k < K ? p[k] : 0.f, k + 1 < K ? p[k + 1] : 0.f, k + 2 < K ? p[k + 2] : 0.f, 0.f);
 }
-// xs[k .. k + 3] = map(k, load(k)) over [0, Kp), four loads of a thread in flight
-template <typename Load, typename Map>
-__device__ __forceinline__ void step_vec(int K, int Kp, int tid, Load load, Map map, float *xs) {
-    constexpr int N = 4;
-    for (int k0 = tid * 4; k0 < Kp; k0 += N * STEP_THREADS * 4) {
-        float4 v[N];
-#pragma unroll
-        for (int i = 0; i < N; ++i) v[i] = load(k0 + i * STEP_THREADS * 4);
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            const int k = k0 + i * STEP_THREADS * 4;
-            if (k < Kp) *reinterpret_cast<float4 *>(xs + k) = map(k, v[i]);
-        }
-    }
+// The same requested ahead, in two parts: a load that no branch lies around where K is a multiple of four (`whole`, the same for
+// all threads), and, once it is needed, its zeros.
+template <bool WHOLE> __device__ __forceinline__ float4 ln_request4(const float *p, int k, int K) {
+    if constexpr (WHOLE) return *reinterpret_cast<const float4 *>(p + (k < K ? k : K - 4));
+    return ln_load4(p, k, K);
+}
+__device__ __forceinline__ void ln_settle4(float4 &v, int k, int K) {
+    if (k >= K) v = make_float4(0.f, 0.f, 0.f, 0.f);
+}
+template <typename Request> __device__ __forceinline__ void ln_request(int K, Request request) {
+    if (K & 3) request(std::false_type{});
+    else request(std::true_type{});
 }
 
+// A thread's first N groups of four elements of a vector, requested ahead; xs[k .. k + 3] = map(k, them) over [0, Kp), the groups
+// behind them loaded on the way.
+template <int N> struct StepVec {
+    static constexpr int STRIDE = STEP_THREADS * 4;
+    float4 v[N];
+    template <typename Whole> __device__ __forceinline__ void load(Whole, const float *p, int tid, int K) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = ln_request4<Whole::value>(p, tid * 4 + i * STRIDE, K);
+    }
+    template <typename Map> __device__ __forceinline__ void put(const float *p, int tid, int K, int Kp, Map map, float *xs) {
+        for (int k0 = tid * 4; k0 < Kp; k0 += N * STRIDE) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                if (k0 == tid * 4) ln_settle4(v[i], k0 + i * STRIDE, K);
+                else v[i] = ln_load4(p, k0 + i * STRIDE, K);
+            }
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                const int k = k0 + i * STRIDE;
+                if (k < Kp) *reinterpret_cast<float4 *>(xs + k) = map(k, v[i]);
+            }
+        }
+    }
+};
+
 template <int R, int U, StepIn IN, StepOut OUT>
-__global__ __launch_bounds__(STEP_THREADS) void linear_step_kernel(const uint16_t *p_w, int p_Kp, int p_groups, int p_width, int p_K, const StepArgs a) {
+__global__ __launch_bounds__(STEP_THREADS, 4) void linear_step_kernel(const uint16_t *p_w, int p_Kp, int p_groups, int p_width, int p_K, const StepArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
-    __shared__ float scratch[STEP_WAVES][4];
+    __shared__ StepScratch scratch;
     float *xs = reinterpret_cast<float *>(smem);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int K = p_K, Kp = p_Kp;
     const int batches = (Kp + 512 * U - 1) / (512 * U);
     const int g_step = gridDim.x * STEP_WAVES;
-    int grp = blockIdx.x * STEP_WAVES + wave, batch = 0;
     auto row_of = [&](int gr, int r) { return OUT == STEP_OUT_MIN_GRU ? r * p_width + gr : gr * R + r; };
-    auto fetch = [&](uint4 (&b)[R][U], int gr, int bt) {
+    // a batch of weights and what the epilogue of their rows reads
+    struct Batch {
+        uint4 w[R][U];
+        float e[3];
+    };
+    static_assert(R <= 3, "e holds one number a row");
+    int seq0 = 0, pos0 = 0, tok0 = 0;
+    if constexpr (OUT == STEP_OUT_MIN_GRU) { seq0 = a.seq[0]; pos0 = a.pos[0]; }
+    if constexpr (OUT == STEP_OUT_SIDE) tok0 = a.tok[0];
+    auto fetch = [&](Batch &b, int gr, int bt) {
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const uint16_t *wr = p_w + (size_t)row_of(gr, r) * Kp;
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const int k = (bt * U + u) * 512 + lane * 8;
-                b[r][u] = make_uint4(0, 0, 0, 0);
-                if (k < Kp) b[r][u] = *reinterpret_cast<const uint4 *>(wr + k);
+                b.w[r][u] = *reinterpret_cast<const uint4 *>(wr + (k < Kp ? k : Kp - 8));       // (past the row's end: not used)
             }
         }
+        if constexpr (OUT == STEP_OUT_MIN_GRU) { b.e[0] = a.bias_z[gr]; b.e[1] = a.bias_x[gr]; b.e[2] = a.state[(size_t)seq0 * p_width + gr]; }
+        if constexpr (OUT == STEP_OUT_SIDE) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) b.e[r] = bf16_bits_to_f32(a.side[(size_t)tok0 * a.side_stride + a.side_offset + (gr * R + r < a.W.M ? gr * R + r : a.W.M - 1)]);
+        }
     };
-    uint4 b0[R][U], b1[R][U];
-    if (grp < p_groups) fetch(b0, grp, 0);
+    Batch b0, b1;
+    const int first = blockIdx.x * STEP_WAVES + wave;
+    const int turns = first < p_groups ? (p_groups - first + g_step - 1) / g_step : 0;
+    auto fetch_first = [&]() { fetch(b0, turns ? first : p_groups - 1, 0); };
 
     // ---- the input vector
-    if constexpr (IN == STEP_IN_VEC) {
-        step_vec(K, Kp, tid, [&](int k) { return ln_load4(a.in, k, K); }, [&](int k, const float4 &v) { return v; }, xs);
-    } else if constexpr (IN == STEP_IN_POLY) {
-        float p2 = 0.f, p4 = 0.f, p6 = 0.f;
-        for (int i = tid; i < a.n_part; i += STEP_THREADS) { p2 += a.part[i]; p4 += a.part[a.n_part + i]; p6 += a.part[2 * a.n_part + i]; }
-        p2 = step_block_sum(p2, &scratch[0][0], lane, wave);
-        p4 = step_block_sum(p4, &scratch[0][0], lane, wave);
-        p6 = step_block_sum(p6, &scratch[0][0], lane, wave);
-        const float c1 = a.coef[0] / sqrtf(p2 / (float)K + a.eps), c2 = a.coef[1] / sqrtf(p4 / (float)K + a.eps), c3 = a.coef[2] / sqrtf(p6 / (float)K + a.eps);
-        const float c0 = a.coef[3];
-        auto poly = [&](float u) { return ((c3 * u + c2) * u + c1) * u + c0; };
-        step_vec(K, Kp, tid, [&](int k) { return ln_load4(a.in, k, K); },
-                 [&](int k, const float4 &u) {
-                     return make_float4(k < K ? poly(u.x) : 0.f, k + 1 < K ? poly(u.y) : 0.f, k + 2 < K ? poly(u.z) : 0.f, k + 3 < K ? poly(u.w) : 0.f);
-                 }, xs);
-    } else if constexpr (IN == STEP_IN_RELU2) {
+    static_assert(STEP_PARTS_MAX <= STEP_THREADS, "a partial sum per thread");
+    if constexpr (IN == STEP_IN_VEC || IN == STEP_IN_RELU2) {
+        StepVec<4> in;
+        ln_request(K, [&](auto whole) { in.load(whole, a.in, tid, K); });
+        fetch_first();
         auto sq = [](float v) { const float p = fmaxf(v, 0.f); return p * p; };
-        step_vec(K, Kp, tid, [&](int k) { return ln_load4(a.in, k, K); }, [&](int k, const float4 &v) { return make_float4(sq(v.x), sq(v.y), sq(v.z), sq(v.w)); }, xs);
+        in.put(a.in, tid, K, Kp, [&](int, const float4 &v) { return IN == STEP_IN_VEC ? v : make_float4(sq(v.x), sq(v.y), sq(v.z), sq(v.w)); }, xs);
+    } else if constexpr (IN == STEP_IN_POLY) {
+        float p[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) p[i] = tid < a.n_part ? a.part[i * a.n_part + tid] : 0.f;
+        const float f1 = a.coef[0], f2 = a.coef[1], f3 = a.coef[2], c0 = a.coef[3];
+        StepVec<4> in;
+        ln_request(K, [&](auto whole) { in.load(whole, a.in, tid, K); });
+        fetch_first();
+        step_block_sums<0>(p, scratch, lane, wave);
+        const float c1 = f1 / sqrtf(p[0] / (float)K + a.eps), c2 = f2 / sqrtf(p[1] / (float)K + a.eps), c3 = f3 / sqrtf(p[2] / (float)K + a.eps);
+        auto poly = [&](float u) { return ((c3 * u + c2) * u + c1) * u + c0; };
+        in.put(a.in, tid, K, Kp,
+               [&](int k, const float4 &u) {
+                   return make_float4(k < K ? poly(u.x) : 0.f, k + 1 < K ? poly(u.y) : 0.f, k + 2 < K ? poly(u.z) : 0.f, k + 3 < K ? poly(u.w) : 0.f);
+               }, xs);
     } else if constexpr (IN == STEP_IN_UNIT_RMS) {
+        StepVec<1> in, gain;
+        ln_request(K, [&](auto whole) { in.load(whole, a.in, tid, K); gain.load(whole, a.gain, tid, K); });
+        fetch_first();
         float ss = 0.f;
-        step_vec(K, Kp, tid, [&](int k) { return ln_load4(a.in, k, K); },
-                 [&](int k, const float4 &v) { ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w; return v; }, xs);
-        const float rinv = 1.0f / sqrtf(step_block_sum(ss, &scratch[0][0], lane, wave) / (float)K + a.eps);
-        for (int k = tid; k < K; k += STEP_THREADS) xs[k] *= rinv * a.gain[k];
+        in.put(a.in, tid, K, Kp, [&](int, const float4 &v) { ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w; return v; }, xs);
+        const float rinv = 1.0f / sqrtf(step_block_sum<0>(ss, scratch, lane, wave) / (float)K + a.eps);
+        gain.put(a.gain, tid, K, Kp,
+                 [&](int k, const float4 &g) {
+                     const float4 v = *reinterpret_cast<const float4 *>(xs + k);
+                     return make_float4(v.x * (rinv * g.x), v.y * (rinv * g.y), v.z * (rinv * g.z), v.w * (rinv * g.w));
+                 }, xs);
     } else if constexpr (IN == STEP_IN_LAYER) {
         // a thread's first AHEAD groups of four, of every vector, are requested before the first sum; means first, then squared
         // deviations
@@ -117,12 +185,23 @@ __global__ __launch_bounds__(STEP_THREADS) void linear_step_kernel(const uint16_
         const int k0 = tid * 4;
         const float inv_n = 1.0f / (float)K;
         float4 x4[AHEAD], y4[AHEAD], g4[AHEAD], b4[AHEAD], ng4[AHEAD], nb4[AHEAD];
+        ln_request(K, [&](auto whole) {
+#pragma unroll
+            for (int i = 0; i < AHEAD; ++i) {
+                const int k = k0 + i * STRIDE;
+                auto get = [&](const float *p) { return ln_request4<decltype(whole)::value>(p, k, K); };
+                x4[i] = get(a.in);
+                if (a.y) { y4[i] = get(a.y); g4[i] = get(a.gain); b4[i] = get(a.bias); }
+                ng4[i] = get(a.norm_gain); nb4[i] = get(a.norm_bias);
+            }
+        });
+        fetch_first();
 #pragma unroll
         for (int i = 0; i < AHEAD; ++i) {
             const int k = k0 + i * STRIDE;
-            x4[i] = ln_load4(a.in, k, K);
-            if (a.y) { y4[i] = ln_load4(a.y, k, K); g4[i] = ln_load4(a.gain, k, K); b4[i] = ln_load4(a.bias, k, K); }
-            ng4[i] = ln_load4(a.norm_gain, k, K); nb4[i] = ln_load4(a.norm_bias, k, K);
+            ln_settle4(x4[i], k, K);
+            if (a.y) { ln_settle4(y4[i], k, K); ln_settle4(g4[i], k, K); ln_settle4(b4[i], k, K); }
+            ln_settle4(ng4[i], k, K); ln_settle4(nb4[i], k, K);
         }
         auto sum4 = [](const float4 &v) { return (v.x + v.y) + (v.z + v.w); };
         auto dev4 = [&](int k, const float4 &v, float mean) {
@@ -137,12 +216,12 @@ __global__ __launch_bounds__(STEP_THREADS) void linear_step_kernel(const uint16_
 #pragma unroll
             for (int i = 0; i < AHEAD; ++i) s += sum4(y4[i]);
             for (int k = k0 + AHEAD * STRIDE; k < K; k += STRIDE) s += sum4(ln_load4(a.y, k, K));
-            const float mean = step_block_sum(s, &scratch[0][0], lane, wave) * inv_n;
+            const float mean = step_block_sum<0>(s, scratch, lane, wave) * inv_n;
             s = 0.f;
 #pragma unroll
             for (int i = 0; i < AHEAD; ++i) s += dev4(k0 + i * STRIDE, y4[i], mean);
             for (int k = k0 + AHEAD * STRIDE; k < K; k += STRIDE) s += dev4(k, ln_load4(a.y, k, K), mean);
-            const float rs = 1.0f / sqrtf(step_block_sum(s, &scratch[0][0], lane, wave) * inv_n + a.eps);
+            const float rs = 1.0f / sqrtf(step_block_sum<1>(s, scratch, lane, wave) * inv_n + a.eps);
             auto update = [&](int k, const float4 &x, const float4 &y, const float4 &g, const float4 &b) {
                 const float4 v = make_float4(x.x + ((y.x - mean) * rs * g.x + b.x), x.y + ((y.y - mean) * rs * g.y + b.y), x.z + ((y.z - mean) * rs * g.z + b.z),
                                              x.w + ((y.w - mean) * rs * g.w + b.w));
@@ -166,12 +245,12 @@ __global__ __launch_bounds__(STEP_THREADS) void linear_step_kernel(const uint16_
 #pragma unroll
         for (int i = 0; i < AHEAD; ++i) s += sum4(x4[i]);
         for (int k = k0 + AHEAD * STRIDE; k < Kp; k += STRIDE) s += sum4(*reinterpret_cast<const float4 *>(xs + k));
-        const float mean = step_block_sum(s, &scratch[0][0], lane, wave) * inv_n;
+        const float mean = step_block_sum<0>(s, scratch, lane, wave) * inv_n;
         s = 0.f;
 #pragma unroll
         for (int i = 0; i < AHEAD; ++i) s += dev4(k0 + i * STRIDE, x4[i], mean);
         for (int k = k0 + AHEAD * STRIDE; k < Kp; k += STRIDE) s += dev4(k, *reinterpret_cast<const float4 *>(xs + k), mean);
-        const float rs = 1.0f / sqrtf(step_block_sum(s, &scratch[0][0], lane, wave) * inv_n + a.eps);
+        const float rs = 1.0f / sqrtf(step_block_sum<1>(s, scratch, lane, wave) * inv_n + a.eps);
         auto put = [&](int k, const float4 &v, const float4 &g, const float4 &b) {
             if (k < Kp) *reinterpret_cast<float4 *>(xs + k) = make_float4((v.x - mean) * rs * g.x + b.x, (v.y - mean) * rs * g.y + b.y, (v.z - mean) * rs * g.z + b.z, (v.w - mean) * rs * g.w + b.w);
         };
@@ -179,17 +258,19 @@ __global__ __launch_bounds__(STEP_THREADS) void linear_step_kernel(const uint16_
         for (int i = 0; i < AHEAD; ++i) put(k0 + i * STRIDE, x4[i], ng4[i], nb4[i]);
         for (int k = k0 + AHEAD * STRIDE; k < Kp; k += STRIDE) put(k, *reinterpret_cast<const float4 *>(xs + k), ln_load4(a.norm_gain, k, K), ln_load4(a.norm_bias, k, K));
     } else {
-        float ss = 0.f;
-        for (int i = tid; i < a.n_part; i += STEP_THREADS) ss += a.part[i];
-        // the vectors' loads go out before the partial sums are added up
+        float ss = tid < a.n_part ? a.part[tid] : 0.f;
         constexpr int AHEAD = 2;
         float4 x4[AHEAD], y4[AHEAD], g4[AHEAD];
+        ln_request(K, [&](auto whole) {
 #pragma unroll
-        for (int i = 0; i < AHEAD; ++i) {
-            const int k = (tid + i * STEP_THREADS) * 4;
-            x4[i] = ln_load4(a.in, k, K); y4[i] = ln_load4(a.y, k, K); g4[i] = ln_load4(a.gain, k, K);
-        }
-        ss = step_block_sum(ss, &scratch[0][0], lane, wave);
+            for (int i = 0; i < AHEAD; ++i) {
+                const int k = (tid + i * STEP_THREADS) * 4;
+                auto get = [&](const float *p) { return ln_request4<decltype(whole)::value>(p, k, K); };
+                x4[i] = get(a.in); y4[i] = get(a.y); g4[i] = get(a.gain);
+            }
+        });
+        fetch_first();
+        ss = step_block_sum<0>(ss, scratch, lane, wave);
         const float rinv = 1.0f / sqrtf(ss / (float)K + a.eps);
         float sx = 0.f;
         auto update = [&](int k, const float4 &x, const float4 &y, const float4 &g) {
@@ -205,10 +286,14 @@ __global__ __launch_bounds__(STEP_THREADS) void linear_step_kernel(const uint16_
             }
         };
 #pragma unroll
-        for (int i = 0; i < AHEAD; ++i) update((tid + i * STEP_THREADS) * 4, x4[i], y4[i], g4[i]);
+        for (int i = 0; i < AHEAD; ++i) {
+            const int k = (tid + i * STEP_THREADS) * 4;
+            ln_settle4(x4[i], k, K); ln_settle4(y4[i], k, K); ln_settle4(g4[i], k, K);
+            update(k, x4[i], y4[i], g4[i]);
+        }
         for (int k = (tid + AHEAD * STEP_THREADS) * 4; k < Kp; k += STEP_THREADS * 4) update(k, ln_load4(a.in, k, K), ln_load4(a.y, k, K), ln_load4(a.gain, k, K));
         if constexpr (IN == STEP_IN_RESIDUAL_NORM) {
-            sx = step_block_sum(sx, &scratch[0][0], lane, wave);
+            sx = step_block_sum<1>(sx, scratch, lane, wave);
             const float z = a.norm_gain[0] / sqrtf(sx / (float)K + a.eps);
             for (int k = tid; k < Kp; k += STEP_THREADS) xs[k] *= z;
         }
@@ -219,16 +304,15 @@ __global__ __launch_bounds__(STEP_THREADS) void linear_step_kernel(const uint16_
     float acc[R], s2 = 0.f, s4 = 0.f, s6 = 0.f;
 #pragma unroll
     for (int r = 0; r < R; ++r) acc[r] = 0.f;
-    auto finish = [&](int gr) {
+    auto finish = [&](int gr, const float (&e)[3]) {
         float v[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) { v[r] = step_wave_sum(acc[r]); acc[r] = 0.f; }
         if constexpr (OUT == STEP_OUT_MIN_GRU) {
             if (lane == 0) {
-                const MinGruGate g = min_gru_gate(v[0] + a.bias_z[gr], v[1] + a.bias_x[gr]);
-                float *st = a.state + (size_t)a.seq[0] * p_width + gr;
-                const float s = a.pos[0] == 0 ? g.in : fmaf(g.keep, *st, g.in);
-                *st = s;
+                const MinGruGate g = min_gru_gate(v[0] + e[0], v[1] + e[1]);
+                const float s = pos0 == 0 ? g.in : fmaf(g.keep, e[2], g.in);
+                a.state[(size_t)seq0 * p_width + gr] = s;
                 a.out[gr] = s * act_silu(v[2]);
             }
         } else {
@@ -237,10 +321,7 @@ __global__ __launch_bounds__(STEP_THREADS) void linear_step_kernel(const uint16_
                 const int m = gr * R + r;
                 if (m >= a.W.M) continue;
                 float o = v[r];
-                if constexpr (OUT == STEP_OUT_SIDE) {
-                    const float e = bf16_bits_to_f32(a.side[(size_t)a.tok[0] * a.side_stride + a.side_offset + m]);
-                    o = act_gelu_tanh(o) * e;
-                }
+                if constexpr (OUT == STEP_OUT_SIDE) o = act_gelu_tanh(o) * e[r];
                 if (lane == 0) a.out[m] = o;
                 const float q = o * o;
                 if constexpr (OUT == STEP_OUT_SUMSQ || OUT == STEP_OUT_POWERS) s2 += q;
@@ -248,7 +329,7 @@ __global__ __launch_bounds__(STEP_THREADS) void linear_step_kernel(const uint16_
             }
         }
     };
-    auto use = [&](const uint4 (&b)[R][U], int bt) {
+    auto use = [&](const Batch &b, int gr, int bt) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int k = (bt * U + u) * 512 + lane * 8;
@@ -257,34 +338,46 @@ __global__ __launch_bounds__(STEP_THREADS) void linear_step_kernel(const uint16_
                 const float xf[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
-                    const uint32_t w[4] = {b[r][u].x, b[r][u].y, b[r][u].z, b[r][u].w};
+                    const uint32_t w[4] = {b.w[r][u].x, b.w[r][u].y, b.w[r][u].z, b.w[r][u].w};
 #pragma unroll
                     for (int j = 0; j < 8; ++j) acc[r] = fmaf(__uint_as_float((j & 1) ? (w[j >> 1] & 0xFFFF0000u) : (w[j >> 1] << 16)), xf[j], acc[r]);
                 }
             }
         }
+        if (bt == batches - 1) finish(gr, b.e);
     };
     // (group, batch) pairs in order; each is fetched while the one before it is used
-    auto step = [&](uint4 (&cur)[R][U], uint4 (&next)[R][U]) {
-        const int gr = grp, bt = batch;
-        if (++batch == batches) { batch = 0; grp += g_step; }
-        if (grp < p_groups) fetch(next, grp, batch);
-        use(cur, bt);
-        if (bt == batches - 1) finish(gr);
+    int gr0 = first, bt0 = 0, gr1, bt1;
+    auto after = [&](int gr, int bt, int &gr_next, int &bt_next) {
+        const bool turn = bt + 1 == batches;
+        bt_next = turn ? 0 : bt + 1;
+        gr_next = turn ? gr + g_step : gr;
     };
-    while (grp < p_groups) {
-        step(b0, b1);
-        if (grp >= p_groups) break;
-        step(b1, b0);
+    int left = turns * batches;
+    for (; left > 2; left -= 2) {
+        after(gr0, bt0, gr1, bt1);
+        fetch(b1, gr1, bt1);
+        use(b0, gr0, bt0);
+        after(gr1, bt1, gr0, bt0);
+        fetch(b0, gr0, bt0);
+        use(b1, gr1, bt1);
+    }
+    if (left == 2) {
+        after(gr0, bt0, gr1, bt1);
+        fetch(b1, gr1, bt1);
+        use(b0, gr0, bt0);
+        use(b1, gr1, bt1);
+    } else if (left == 1) {
+        use(b0, gr0, bt0);
     }
     if constexpr (OUT == STEP_OUT_SUMSQ || OUT == STEP_OUT_POWERS) {
         // (every lane of a wave holds the wave's sums)
         __syncthreads();
-        if (lane == 0) { scratch[wave][0] = s2; scratch[wave][1] = s4; scratch[wave][2] = s6; }
+        if (lane == 0) { scratch[0][wave][0] = s2; scratch[0][wave][1] = s4; scratch[0][wave][2] = s6; }
         __syncthreads();
         if (tid < (OUT == STEP_OUT_POWERS ? 3 : 1)) {
             float s = 0.f;
-            for (int w = 0; w < STEP_WAVES; ++w) s += scratch[w][tid];
+            for (int w = 0; w < STEP_WAVES; ++w) s += scratch[0][w][tid];
             a.out_part[(size_t)tid * gridDim.x + blockIdx.x] = s;
         }
     }
