@@ -44,19 +44,24 @@ __device__ __forceinline__ float row_sum(float v, float *scratch) {
     return scratch[0] + scratch[1] + scratch[2] + scratch[3];
 }
 
+// Grid (tokens, groups of ROW_THREADS pairs): a thread takes the sine and the cosine of one frequency, so that a wave walks the
+// range reduction of an angle once and a single token's row is not one workgroup's serial work.  One row of 2048: 10.3 -> 4.4 us,
+// 900 rows: 13.4 -> 9.1.
 __global__ __launch_bounds__(ROW_THREADS) void embed_rows_kernel(const uint16_t *table, int ldt, const int32_t *tok, const int32_t *pos, const float *freq, float scale,
                                                                  int n, float *x) {
-    const int t = blockIdx.x;
-    const uint16_t *e = table + (size_t)tok[t] * ldt;
-    const float p = (float)pos[t];
-    for (int i = threadIdx.x; i < n; i += ROW_THREADS) {
-        float v = bf16_bits_to_f32(e[i]) * scale;
-        if (freq) {
-            const float angle = p * freq[i >> 1];
-            v += (i & 1) ? cosf(angle) : sinf(angle);
-        }
-        x[(size_t)t * n + i] = v;
+    const int t = blockIdx.x, pair = blockIdx.y * ROW_THREADS + threadIdx.x, i = 2 * pair;
+    if (i >= n) return;
+    const bool both = i + 1 < n;
+    const uint16_t *e = table + (size_t)tok[t] * ldt + i;
+    float v0 = bf16_bits_to_f32(e[0]) * scale, v1 = both ? bf16_bits_to_f32(e[1]) * scale : 0.f;
+    if (freq) {
+        const float angle = (float)pos[t] * freq[pair];
+        v0 += sinf(angle);
+        v1 += cosf(angle);
     }
+    float *o = x + (size_t)t * n + i;
+    o[0] = v0;
+    if (both) o[1] = v1;
 }
 
 // y as its producer left it: partial products `stride` floats apart, added in order
@@ -321,7 +326,7 @@ __global__ __launch_bounds__(ROW_THREADS) void qk_norm_append_kernel(const QkApp
 
 int embed_rows(const uint16_t *table, int ldt, const int32_t *tok, const int32_t *pos, const float *freq, float scale, int T, int n, float *x, hipStream_t stream) {
     if (T <= 0) return MESH_OK;
-    MESH_LAUNCH(embed_rows_kernel, dim3((unsigned)T), dim3(ROW_THREADS), 0, stream, table, ldt, tok, pos, freq, scale, n, x);
+    MESH_LAUNCH(embed_rows_kernel, dim3((unsigned)T, (unsigned)((n + 2 * ROW_THREADS - 1) / (2 * ROW_THREADS))), dim3(ROW_THREADS), 0, stream, table, ldt, tok, pos, freq, scale, n, x);
     MESH_LAUNCH_CHECK();
     return MESH_OK;
 }
