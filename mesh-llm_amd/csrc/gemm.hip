@@ -1066,7 +1066,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_epilogue_kernel(GemmArgs a, i
 // 734 / 754, 150 1296 / 1338, 400 2217 / 2274: at every count that splits.
 constexpr int SN_THREADS = 512;
 template <int NG>              // groups of 8 elements a thread has: rows of up to NG * 4096
-__global__ __launch_bounds__(SN_THREADS) void gemm_splitk_norm_kernel(GemmArgs a, int row_blocks) {
+__global__ __launch_bounds__(SN_THREADS) void gemm_splitk_epilogue_norm_kernel(GemmArgs a, int row_blocks) {
     __shared__ float s_ss[SN_THREADS / 64];
     const size_t ld = (size_t)row_blocks * GM;
     const int t = blockIdx.x, tid = threadIdx.x;
@@ -1148,8 +1148,8 @@ bool gemm_norm_rides(const GemmArgs &a) {
 int gemm_add_slices(const GemmArgs &k, int row_blocks, hipStream_t stream) {
     if (k.next_x16) {
         const dim3 grid((unsigned)((k.T + 15) & ~15)), block(SN_THREADS);
-        if (k.M <= 8 * SN_THREADS) MESH_LAUNCH(gemm_splitk_norm_kernel<1>, grid, block, 0, stream, k, row_blocks);
-        else MESH_LAUNCH(gemm_splitk_norm_kernel<2>, grid, block, 0, stream, k, row_blocks);
+        if (k.M <= 8 * SN_THREADS) MESH_LAUNCH(gemm_splitk_epilogue_norm_kernel<1>, grid, block, 0, stream, k, row_blocks);
+        else MESH_LAUNCH(gemm_splitk_epilogue_norm_kernel<2>, grid, block, 0, stream, k, row_blocks);
         MESH_LAUNCH_CHECK();
         return MESH_OK;
     }
