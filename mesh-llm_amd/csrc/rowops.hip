@@ -255,18 +255,25 @@ __global__ __launch_bounds__(ROW_THREADS) void poly_norm_kernel(const float *u, 
     }
 }
 
+// A thread's slices travel GROUP at a time (past the last one it is that one again): 900 rows of 128 in eight slices 7.6 -> 4.4 us.
+constexpr int SIDE_THREADS = 128;
 template <ActType ACT>
-__global__ __launch_bounds__(64) void side_gate_kernel(const float *g, int slices, size_t slice_stride, const uint16_t *side, const int32_t *tok, int stride, int offset, int n, void *out, int ld) {
+__global__ __launch_bounds__(SIDE_THREADS) void side_gate_kernel(const float *g, int slices, size_t slice_stride, const uint16_t *side, const int32_t *tok, int stride, int offset, int n, void *out, int ld) {
+    constexpr int GROUP = 8;
     const int t = blockIdx.x;
     const uint16_t *e = side + (size_t)tok[t] * stride + offset;
-    for (int i = threadIdx.x; i < ld; i += 64) {
-        float v = 0.f;
-        if (i < n) {
-            float z = 0.f;
-            for (int s = 0; s < slices; ++s) z += g[s * slice_stride + (size_t)t * n + i];
-            v = act_gelu_tanh(z) * bf16_bits_to_f32(e[i]);
+    for (int i = threadIdx.x; i < ld; i += SIDE_THREADS) {
+        const int ic = i < n ? i : n - 1;
+        const float ei = bf16_bits_to_f32(e[ic]);
+        float z = 0.f;
+        for (int s = 0; s < slices; s += GROUP) {
+            float p[GROUP];
+#pragma unroll
+            for (int k = 0; k < GROUP; ++k) p[k] = g[(s + k < slices ? s + k : slices - 1) * slice_stride + (size_t)t * n + ic];
+#pragma unroll
+            for (int k = 0; k < GROUP; ++k) z = s + k < slices ? z + p[k] : z;
         }
-        act_store<ACT>(out, (size_t)t * ld + i, v);
+        act_store<ACT>(out, (size_t)t * ld + i, i < n ? act_gelu_tanh(z) * ei : 0.f);
     }
 }
 
@@ -382,7 +389,7 @@ int poly_norm_rows(const float *u, const float *coef, float eps, int T, int n, v
 int side_gate_rows(const float *g, int slices, size_t slice_stride, const uint16_t *side, const int32_t *tok, int stride, int offset, int T, int n, void *out, ActType act, int ld, hipStream_t stream) {
     if (T <= 0) return MESH_OK;
     if (ld < n || offset + n > stride) return fail(MESH_ERR_INVALID, "side_gate_rows: bad operands");
-    MESH_ACT_LAUNCH(side_gate_kernel, act, dim3((unsigned)T), dim3(64), g, slices, slice_stride, side, tok, stride, offset, n, out, ld);
+    MESH_ACT_LAUNCH(side_gate_kernel, act, dim3((unsigned)T), dim3(SIDE_THREADS), g, slices, slice_stride, side, tok, stride, offset, n, out, ld);
     return MESH_OK;
 }
 
