@@ -2,7 +2,7 @@
 // runs, one for each wave of a workgroup of 64 channels.
 //
 // The first launch composes each window's steps into (A, B), S_out = A S_in + B, or, when a sequence starts inside the window,
-// into the state its last sequence leaves (A = 0).  The second composes the windows before its own, a quarter a wave, and the
+// into the state its last sequence leaves (a restart: S_out = B).  The second composes the windows before its own, a quarter a wave, and the
 // runs before its own, and walks its run from there.  A call of one window (decode batches) needs the second launch only.
 //
 // Bound by memory.  A thread requests all its projections (16 in the first launch, 24 in the second) before it uses one: a loop
@@ -19,10 +19,15 @@ namespace mesh {
 
 constexpr int GRU_RUN = 8, GRU_WAVES = 4, GRU_WINDOW = GRU_RUN * GRU_WAVES, GRU_THREADS = 64 * GRU_WAVES;
 
-// a step or a row of them: S -> A S + B; A = 0 forgets S whatever it holds (another sequence's infinity, say)
+// A step or a row of them: S -> A S + B, or, where a sequence starts in the row, S -> B whatever S holds (another sequence's
+// infinity, say): A is GRU_RESTART then, which no product of keeps is.  (A product that has underflowed to 0 is no restart: a NaN or
+// an infinity of the sequence's own state stays in it, as it does token by token.)
+constexpr float GRU_RESTART = -1.f;
 struct GruStep { float A, B; };
-__device__ __forceinline__ float gru_apply(const GruStep &s, float S) { return s.A == 0.f ? s.B : fmaf(s.A, S, s.B); }
-__device__ __forceinline__ GruStep gru_then(const GruStep &first, const GruStep &s) { return {first.A * s.A, gru_apply(s, first.B)}; }
+__device__ __forceinline__ float gru_apply(const GruStep &s, float S) { return s.A == GRU_RESTART ? s.B : fmaf(s.A, S, s.B); }
+__device__ __forceinline__ GruStep gru_then(const GruStep &first, const GruStep &s) {
+    return {first.A == GRU_RESTART || s.A == GRU_RESTART ? GRU_RESTART : first.A * s.A, gru_apply(s, first.B)};
+}
 
 // The steps of tokens t0 .. t0 + GRU_RUN - 1 of channel c (identities from T on) and where sequences start among them.
 struct GruRun {
@@ -33,7 +38,7 @@ struct GruRun {
         GruStep r{1.f, 0.f};
 #pragma unroll
         for (int i = 0; i < GRU_RUN; ++i) {
-            if (starts >> i & 1) r = {0.f, init[i]};
+            if (starts >> i & 1) r = {GRU_RESTART, init[i]};
             r = gru_then(r, step[i]);
         }
         return r;

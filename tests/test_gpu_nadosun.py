@@ -236,6 +236,45 @@ def test_recurrences_of_sequences_that_start_anywhere_in_a_window(tmp_path, lens
 
 
 @BOTH
+def test_a_broken_state_stays_broken_and_stays_its_own(tmp_path, prec):
+    """A token that drives one channel of the state to infinity, then many under gates that keep 2e-9 of it: the recurrence of a whole
+    prompt carries it on over its runs and windows, and into the next call, as single tokens do; the sequences beside it never see it."""
+    m, bad = mesh(), 5
+
+    def broken(w, cfg):
+        w = {k: v.copy() for k, v in w.items()}
+        w["embed"][:, 3], w["embed"][bad, 3] = -2.0, 48.0       # (below the position vector's reach for every other token)
+        w["l0.mix.x"][7, 3] = N.bf16([3e38])[0]
+        for i in range(len(cfg["layers"])):
+            w["l%d.mix.z.b" % i][:] = 20.0
+        return w
+
+    cfg, w, folder, orc = made(tmp_path, "recurrent-only", change=broken)
+    lens = [20, 75, 30]
+    toks = [N.prompt(cfg, 2 * n, 80 + i, avoid=(bad,)) for i, n in enumerate(lens)]
+    toks[1][2] = bad
+    st = open_stage(folder, prec, n_seq=len(lens))
+    ses = st.session()
+    for half in (0, 1):
+        cut = [slice(half * n, (half + 1) * n) for n in lens]
+        got = ses.decode(np.concatenate([t[c] for t, c in zip(toks, cut)]), np.concatenate([np.arange(c.start, c.stop) for c in cut]).astype(np.int32),
+                         seq=np.repeat(np.arange(len(lens), dtype=np.int32), lens), in_fmt=m.TOKENS, out_fmt=m.LOGITS).view(np.float32).reshape(sum(lens), -1)
+        rows = np.split(got, np.cumsum(lens)[:-1])
+        for i in (0, 2):
+            orc.reset()
+            assert N.error(rows[i], orc.forward(toks[i])[cut[i]]) < LIMIT[prec], (half, i)
+        assert np.isfinite(rows[1][:2]).all() == (half == 0)
+        assert not np.isfinite(rows[1][2 if half == 0 else 0:]).any(), half
+    ses.close()
+    ses = st.session()
+    s = Seq(st, ses)
+    alone = np.concatenate([s.feed(toks[1][i:i + 1]) for i in range(12)])
+    assert np.isfinite(alone[:2]).all() and not np.isfinite(alone[2:]).any()
+    ses.close()
+    st.close()
+
+
+@BOTH
 def test_a_sequence_given_back_starts_clean(tmp_path, prec):
     m = mesh()
     cfg, w, folder, orc = made(tmp_path, "mixed")
