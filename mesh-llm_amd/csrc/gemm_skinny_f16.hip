@@ -218,7 +218,8 @@ __device__ __forceinline__ size_t k8_at(int K, int k, int t) { return (size_t)(t
 
 // 1 KB from memory to LDS without passing registers: the 16 bytes at base + off (bytes, a lane's own) go to dst + 4 lane (dst
 // uniform).  As text: behind the builtin the compiler waits for every load in flight at the next cross-lane move, which counts as
-// an LDS access.  Its own counts stay right, a load it does not know of only makes a wait stricter; the reader waits itself.
+// an LDS access.  Its own counts stay right, a load it does not know of only makes a wait stricter; the reader sees to it itself that
+// they have arrived.
 __device__ __forceinline__ void load_to_lds_16(const float *base, int off, float *dst) {
 #if defined(__HIP_DEVICE_COMPILE__)
     const unsigned place = (unsigned)(unsigned long long)(__attribute__((address_space(3))) float *)dst;
@@ -403,9 +404,9 @@ __device__ __forceinline__ void skinny_workgroup(int bx, const _Float16 *p_x, co
     }
     // norm hand-over, consumer side: this wave's share of the partial sums of squares of every column, in order
     if (a.ni_part) {
-        // (a wave that went through a round has requested the last round's fragments and SK_DEPTH tiles behind them: loads return in
-        // order, and those nobody waits for)
-        if (any && n_i >= RB) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 * NC + SK_DEPTH * (TYPE == MESH_Q4_K ? 3 : 5)) : "memory");
+        // (loads return in order: a wave that has walked a second super-block has used activations that it requested behind the
+        // partial sums, and its sums with them stand before this in memory's order; any other waits for all it has requested)
+        if (any && n_i >= 2) asm volatile("" ::: "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         float ss = 0.f;
         for (int p = lane / NT; p < parts_per; p += 64 / NT) ss += wave * parts_per + p < parts_end ? my_parts[p * NT + lane % NT] : 0.f;

@@ -244,6 +244,33 @@ def test_batches_of_decode_steps_along_k(tmp_path, width, ff):
     st.close()
 
 
+# super-blocks of a wave of the launches behind a norm: one; two; two or three; one, and none for some waves
+@pytest.mark.parametrize("width", [2048, 4096, 5120, 1280])
+def test_norms_handed_over_to_short_walks(tmp_path, width):
+    """The partial sums of a norm that reach a launch behind its weights, where its walk is too short to cover them: against norm launches
+    of their own, and the same bits call after call."""
+    m = mesh()
+    cfg = dict(arch="llama", n_layer=3, n_embd=width, n_head=width // 128, n_head_kv=width // 256, head_dim=128, n_ff=1280, n_vocab=256, eps=1e-5, rope=1e4)
+    path = os.path.join(str(tmp_path), "model.gguf")
+    models.write_model(path, cfg, [0, 1, 2], seed=4)
+    st = m.Stage(path, 0, 3, n_ctx=16, n_seq_max=32, n_batch_max=32)
+    ses = [st.session(skinny_norm_fused=on) for on in (1, 0)]
+    rng = np.random.Generator(np.random.PCG64(5))
+    for T in (4, 16, 17, 32):
+        x = rng.standard_normal((T, width)).astype(np.float32) * (10.0 ** rng.uniform(-2, 2, (T, 1))).astype(np.float32)
+        pos, seq = np.zeros(T, np.int32), list(range(T))
+        outs = [s.decode(x, pos, seq=seq).view(np.float32).reshape(T, width).astype(np.float64) for s in ses]
+        for _ in range(8):
+            assert np.array_equal(ses[0].decode(x, pos, seq=seq).view(np.float32).reshape(T, width), outs[0]), (width, T)
+        # a norm of its own rounds scaled rows to f16, the hand-over rows before their scale (2^-12 of themselves each, root mean
+        # square): six products behind one; 4 * 2^-12 * sqrt(2 * 6)
+        worst = np.max(np.linalg.norm(outs[0] - outs[1], axis=1) / np.linalg.norm(outs[1], axis=1))
+        assert worst <= 3.4e-3, (width, T, worst)
+    for s in ses:
+        s.close()
+    st.close()
+
+
 # rows of one and two groups of eight a thread, whole and with idle threads; token counts of every tile that splits
 @pytest.mark.parametrize("width,heads", [(768, 6), (2048, 16), (4096, 32), (5120, 40)])
 def test_norms_ride_with_the_sums_of_slices(tmp_path, width, heads):
