@@ -506,7 +506,9 @@ __global__ __launch_bounds__(PREP_THREADS) void gla_prepare_kernel(const GatedSt
 static size_t gla_prepare_lds(int dim, int rank) { return ((size_t)C * (3 * (gs_pad64(dim) + 4) + rank) + gs_pad64(dim)) * sizeof(float); }
 
 // grid (heads, 16-column slices of the values, sequences of the call).  Wave w owns rows [16 NT w, 16 NT (w + 1)) of the state.
-template <bool DELTA, int NT>
+// PIPED: a chunk is worked on while the next ones travel, which takes the registers of one workgroup a CU; without, as many of them as fit
+// hide each other's waits (launch_scan).
+template <bool DELTA, int NT, bool PIPED>
 __global__ __launch_bounds__(256) void state_scan_kernel(const GatedStateArgs a) {
     constexpr int Dp = 64 * NT;
     __shared__ __align__(16) float red[2][4][DELTA ? 4 : 2][64][4];        // by chunk parity, wave: partial W S and Q S of the two row tiles
@@ -534,11 +536,11 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const GatedStateArgs a)
     // (every chunk of a run but its last is whole)
     const int t_end = a.chunks.chunk[c1], col_in = col < V ? col : V - 1;
     // No branch lies around a load: the compiler waits for everything in flight at the join of one, the chunks just asked for among
-    // them.  What lies past the end is the last chunk, token or column again and is left out where it is used.
-    // 29 chunks x 16 heads of 128 x 128: 70.6 -> 64.2 us with the delta rule, 63.3 -> 44.3 without (the chains of matrix
+    // them.  What lies past the end is the last chunk (PIPED), token or column again and is left out where it is used.
+    // PIPED, 29 chunks x 16 heads of 128 x 128: 70.6 -> 64.2 us with the delta rule, 63.3 -> 44.3 without (the chains of matrix
     // instructions taking turns instead of one after another: 69.6 and 46.2).
     auto load = [&](int ci, Frag &f) {
-        if (ci >= c1) ci = c1 - 1;
+        if (PIPED && ci >= c1) ci = c1 - 1;
         const GsMats m(a.ws, (size_t)ci * a.heads + h, Dp, Vp, DELTA);
 #pragma unroll
         for (int k = 0; k < NT; ++k) {
@@ -564,10 +566,7 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const GatedStateArgs a)
                 else f.u[r][i] = a.in[(size_t)(t0 + tk < t_end ? t0 + tk : t_end - 1) * a.ld + a.at_v + h * V + col_in];
             }
     };
-    // the chunk in `cur`, while the one AHEAD behind it is fetched into `ahead` (as many as the registers hold)
-    constexpr int AHEAD = NT < 4 ? 2 : 1;
-    auto step = [&](int ci, const Frag &cur, Frag &ahead) {
-        load(ci + AHEAD, ahead);
+    auto step = [&](int ci, const Frag &cur) {
         float (*rd)[DELTA ? 4 : 2][64][4] = red[(ci - c0) & 1];
         gs_f4 ws[2], qs[2];
 #pragma unroll
@@ -616,26 +615,30 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const GatedStateArgs a)
             S[k] = gs_mma(cur.k[k][1], u[1], s);
         }
     };
-    Frag f0, f1;
-    load(c0, f0);
-    if constexpr (AHEAD == 2) {
-        Frag f2;
+    Frag f0;
+    if constexpr (!PIPED) {
+        for (int ci = c0; ci < c1; ++ci) { load(ci, f0); step(ci, f0); }
+    } else if constexpr (NT < 4) {          // (two chunks ahead, as many as the registers hold)
+        Frag f1, f2;
+        load(c0, f0);
         load(c0 + 1, f1);
         int ci = c0;
         for (; ci + 3 <= c1; ci += 3) {
-            step(ci, f0, f2);
-            step(ci + 1, f1, f0);
-            step(ci + 2, f2, f1);
+            load(ci + 2, f2); step(ci, f0);
+            load(ci + 3, f0); step(ci + 1, f1);
+            load(ci + 4, f1); step(ci + 2, f2);
         }
-        if (ci < c1) step(ci, f0, f2);
-        if (ci + 1 < c1) step(ci + 1, f1, f0);
+        if (ci < c1) { load(ci + 2, f2); step(ci, f0); }
+        if (ci + 1 < c1) { load(ci + 3, f0); step(ci + 1, f1); }
     } else {
+        Frag f1;
+        load(c0, f0);
         int ci = c0;
         for (; ci + 2 <= c1; ci += 2) {
-            step(ci, f0, f1);
-            step(ci + 1, f1, f0);
+            load(ci + 1, f1); step(ci, f0);
+            load(ci + 2, f0); step(ci + 1, f1);
         }
-        if (ci < c1) step(ci, f0, f1);
+        if (ci < c1) { load(ci + 1, f1); step(ci, f0); }
     }
 #pragma unroll
     for (int k = 0; k < NT; ++k)
@@ -705,17 +708,27 @@ int gated_state_step(const GatedStateArgs &a, int T, hipStream_t stream) {
     return MESH_OK;
 }
 
-template <bool DELTA>
-static int launch_scan(const GatedStateArgs &a, hipStream_t stream) {
+template <bool DELTA, bool PIPED>
+static int launch_scan_of(const GatedStateArgs &a, hipStream_t stream) {
     const dim3 grid((unsigned)a.heads, (unsigned)(gs_pad16(a.vdim) / 16), (unsigned)a.chunks.n_runs), block(256);
     switch (gs_pad64(a.dim) / 64) {
-        case 1: MESH_LAUNCH((state_scan_kernel<DELTA, 1>), grid, block, 0, stream, a); break;
-        case 2: MESH_LAUNCH((state_scan_kernel<DELTA, 2>), grid, block, 0, stream, a); break;
-        case 3: MESH_LAUNCH((state_scan_kernel<DELTA, 3>), grid, block, 0, stream, a); break;
-        default: MESH_LAUNCH((state_scan_kernel<DELTA, 4>), grid, block, 0, stream, a); break;
+        case 1: MESH_LAUNCH((state_scan_kernel<DELTA, 1, PIPED>), grid, block, 0, stream, a); break;
+        case 2: MESH_LAUNCH((state_scan_kernel<DELTA, 2, PIPED>), grid, block, 0, stream, a); break;
+        case 3: MESH_LAUNCH((state_scan_kernel<DELTA, 3, PIPED>), grid, block, 0, stream, a); break;
+        default: MESH_LAUNCH((state_scan_kernel<DELTA, 4, PIPED>), grid, block, 0, stream, a); break;
     }
     MESH_LAUNCH_CHECK();
     return MESH_OK;
+}
+
+// Pipelined where a CU has one workgroup at most and a sequence more than one chunk.  Layers of 16 heads of 128 x 128, us of a call of six
+// layers, two of them scans, pipelined / not (a sequence makes 128 workgroups): one sequence of 900 tokens 1417 / 1464, of 300 870 / 878, two
+// of 300 1520 / 1528; four of 300 2276 / 2252, 16 of 96 2774 / 2674, 32 of 32 1979 / 1830, 60 of 8 and four of 40 2094 / 1787.
+constexpr int SCAN_PIPED_WORKGROUPS_MAX = 256;
+template <bool DELTA>
+static int launch_scan(const GatedStateArgs &a, hipStream_t stream) {
+    const long workgroups = (long)a.heads * (gs_pad16(a.vdim) / 16) * a.chunks.n_runs;
+    return workgroups <= SCAN_PIPED_WORKGROUPS_MAX && a.chunks.n_chunks > a.chunks.n_runs ? launch_scan_of<DELTA, true>(a, stream) : launch_scan_of<DELTA, false>(a, stream);
 }
 
 int gated_state_chunks(const GatedStateArgs &a, int T, hipStream_t stream) {

@@ -254,6 +254,28 @@ def test_unequal_requests_in_one_call_equal_each_alone(tmp_path, prec):
     st.close()
 
 
+# workgroups of a scan on both sides of one a CU, sequences of one to three chunks of 32 tokens and parts of them
+@BOTH
+@pytest.mark.parametrize("name,lens", [("wide-states", [70, 1, 32, 33] * 5), ("wide-states", [64, 65, 96]), ("states-only", [40, 33, 8] * 14), ("states-only", [8, 97, 31])])
+def test_scans_of_many_sequences_in_one_call(tmp_path, name, lens, prec):
+    m = mesh()
+    cfg, w, folder, orc = made(tmp_path, name)
+    st = open_stage(folder, prec, n_ctx=128, n_seq=len(lens), batch=1280)
+    toks, want = [prompt(cfg, n + 9, 70 + i) for i, n in enumerate(lens)], []
+    for t in toks:
+        orc.reset()
+        want.append(orc.forward(t))
+    ses = st.session()
+    for part in (0, 1):         # the prompts, then nine tokens more of each: chunks that start from a state
+        cut = [slice(0, n) if part == 0 else slice(n, n + 9) for n in lens]
+        ends = np.concatenate([np.arange(c.start, c.stop) == c.stop - 1 for c in cut])
+        got = ses.decode(np.concatenate([t[c] for t, c in zip(toks, cut)]), np.concatenate([np.arange(c.start, c.stop) for c in cut]).astype(np.int32),
+                         seq=np.repeat(np.arange(len(lens), dtype=np.int32), [c.stop - c.start for c in cut]), in_fmt=m.TOKENS, out_fmt=m.LOGITS, want=ends)
+        assert off(got.view(np.float32).reshape(len(lens), -1), np.stack([x[c.stop - 1] for x, c in zip(want, cut)]), prec) < 1, part
+    ses.close()
+    st.close()
+
+
 @BOTH
 def test_a_sequence_given_back_starts_clean(tmp_path, prec):
     m = mesh()
