@@ -41,6 +41,7 @@ constexpr int PF_TILE = 32;                 // queries per workgroup
 // piece ^ pf_swizzle(r): equal pieces of the 16 rows that a read of K touches at once, and equal 64-byte runs of the 4 rows that a
 // transposing read touches, lie on different banks.  (Rows of 128 halfs all start on bank 0, rows of 64 and 192 on 0 and 32 in turn.)
 template <int D> __host__ __device__ constexpr int pf_swizzle(int row) { return D == 128 ? (row & 3) << 2 | (row >> 2 & 3) : (row & 2) << 1 | (row >> 2 & 3); }
+constexpr int PF_TWO_GROUPS_WALK = 320;      // two groups of waves share walks of more keys than this
 constexpr int PF_EXPAND_HD = 128;            // kv_expand_kernel's head_dim
 constexpr int PF_EXPAND_MIN_T = 128;         // chunks from this many tokens decode a quantised cache to f16 once, ahead of the walk
 constexpr float PF_RESCALE_STEP = 8.f;      // the softmax reference moves only when the running maximum exceeds it by this (log2)
@@ -473,21 +474,25 @@ int attention_chunk(const AttnArgs &a_in, int T, int pos0, int seq, hipStream_t 
     const int qtiles = hpw >= 4 ? 1 : hpw == 1 ? 4 : 2;
     const int waves = hpw * qtiles, n_tiles = (T + PF_TILE - 1) / PF_TILE;
     dim3 grid((unsigned)((n_tiles + qtiles - 1) / qtiles), (unsigned)a.n_kv, (unsigned)(a.group / hpw));
-    // Workgroups of four waves leave a SIMD one wave, whose products wait for its softmax and the other way round (two workgroups fit
-    // a CU, but the longest walks end alone): a second group of four waves takes every other step of 64 keys of the same walks.
-    const int key_groups = waves == 4 ? 2 : 1;
-    const dim3 block((unsigned)(64 * waves * key_groups));
     // A short chunk on a long history has few query tiles, each with a long walk: split the keys of every walk over
     // several workgroups (partials in the caller's split buffers, merged by attn_combine_kernel) until the launch has a
     // workgroup per CU, at most 8 ways, at least 256 keys each, within the buffers' rows of (token, split).
     int n_ksplit = 1;
+    const int n_keys = a.window > 0 ? std::min(pos0 + T, a.window + PF_TILE) : pos0 + T;
     {
-        const int wgs = (int)(grid.x * grid.y * grid.z), n_keys = a.window > 0 ? std::min(pos0 + T, a.window + PF_TILE) : pos0 + T;
+        const int wgs = (int)(grid.x * grid.y * grid.z);
         if (a.part && a.ml && a.part_rows > 0 && wgs < pf_n_cu())
             n_ksplit = std::max(1, std::min(std::min(pf_n_cu() / wgs, 8), std::min(n_keys / 256, (int)(a.part_rows / (size_t)T))));
         if (n_ksplit > ATTN_SPLITS_CAP) n_ksplit = ATTN_SPLITS_CAP;
     }
     grid.z *= (unsigned)n_ksplit;
+    // Workgroups of four waves leave a SIMD one wave, whose products wait for its softmax and the other way round (two workgroups fit
+    // a CU, but the longest walks end alone): a second group of four waves takes every other step of 64 keys of the same walks.  Short
+    // walks have few steps to share and pay for the larger workgroup and the merge.  One group / two, us, 8B shape: 17 tokens alone 6.7 /
+    // 10.5, 200 12.6 / 13.8, 128 behind 500 (walks of 314) 15.3 / 16.7, 333 16.1 / 16.1, 17 behind 1000 (339) 15.0 / 14.7, 1024 32.4 / 27.3,
+    // 2048 75.7 / 57.8; quantised rows 17 behind 1000 18.9 / 17.2; 16 heads of 192 with values of 128 320 tokens 18.7 / 19.3, 400 21.2 / 20.6.
+    const int key_groups = waves == 4 && (n_keys + n_ksplit - 1) / n_ksplit > PF_TWO_GROUPS_WALK ? 2 : 1;
+    const dim3 block((unsigned)(64 * waves * key_groups));
     // (Two tiles per step everywhere.  With 5 heads per KV head one tile per step keeps the kernel under 170 registers, so
     // that two 5-wave workgroups share a CU instead of one: measured slower, 16.5 against 14.8 ms over 32 layers of 4096 tokens.)
     // NP by the threads of the workgroup: 1024 / threads pairs each, rounded up
@@ -499,8 +504,13 @@ int attention_chunk(const AttnArgs &a_in, int T, int pos0, int seq, hipStream_t 
         else MESH_LAUNCH((attn_chunk_kernel<HD, HD, KT, VT, 4, 1>), grid, block, 0, stream, a, T, pos0, seq, hpw, qtiles, n_ksplit);                  \
     } while (0)
     // (a group of one: four waves)
-    if (apart && a.head_dim == 192) MESH_LAUNCH((attn_chunk_kernel<192, 128, MESH_F16, MESH_F16, 6, 2>), grid, block, 0, stream, a, T, pos0, seq, hpw, qtiles, n_ksplit);
-    else if (apart) MESH_LAUNCH((attn_chunk_kernel<128, 64, MESH_F16, MESH_F16, 4, 2>), grid, block, 0, stream, a, T, pos0, seq, hpw, qtiles, n_ksplit);
+    if (apart && a.head_dim == 192) {
+        if (key_groups == 2) MESH_LAUNCH((attn_chunk_kernel<192, 128, MESH_F16, MESH_F16, 6, 2>), grid, block, 0, stream, a, T, pos0, seq, hpw, qtiles, n_ksplit);
+        else MESH_LAUNCH((attn_chunk_kernel<192, 128, MESH_F16, MESH_F16, 6, 1>), grid, block, 0, stream, a, T, pos0, seq, hpw, qtiles, n_ksplit);
+    } else if (apart) {
+        if (key_groups == 2) MESH_LAUNCH((attn_chunk_kernel<128, 64, MESH_F16, MESH_F16, 4, 2>), grid, block, 0, stream, a, T, pos0, seq, hpw, qtiles, n_ksplit);
+        else MESH_LAUNCH((attn_chunk_kernel<128, 64, MESH_F16, MESH_F16, 4, 1>), grid, block, 0, stream, a, T, pos0, seq, hpw, qtiles, n_ksplit);
+    }
     else if (a.head_dim == 64) MESH_CHUNK_LAUNCH(64, MESH_F16, MESH_F16);
     else if (a.k_type == MESH_F16 && a.v_type == MESH_F16) MESH_CHUNK_LAUNCH(128, MESH_F16, MESH_F16);
     else if (a.k_type == MESH_Q8_0 && a.v_type == MESH_Q4_0) MESH_CHUNK_LAUNCH(128, MESH_Q8_0, MESH_Q4_0);

@@ -43,3 +43,30 @@ def test_chunks_end_anywhere_in_a_step(tmp_path, name):
         assert np.linalg.norm(got - want) <= TOL * np.linalg.norm(want) and worst <= 2 * TOL, (name, past, T, worst)
     ses.close()
     st.close()
+
+
+# one and two key groups: walks of 320 keys and the next, walks that are split (533 and 900 keys in two and three), and short ones
+@pytest.mark.parametrize("name", ["tiny-kv3", "tiny-mha"])
+def test_walks_of_one_and_two_key_groups(tmp_path, name):
+    m, cfg = mesh(), models.CONFIGS[name]
+    path = os.path.join(str(tmp_path), name + ".gguf")
+    tensors = models.write_model(path, cfg, [0], seed=6)
+    chunks = [(0, 319), (0, 320), (0, 321), (280, 40), (281, 40), (500, 33), (870, 30), (0, 20)]
+    st = m.Stage(path, 0, 1, n_ctx=1024, n_seq_max=len(chunks), n_batch_max=336)
+    E, HK, D = cfg["n_embd"], cfg["n_head_kv"], cfg["head_dim"]
+    rng = np.random.Generator(np.random.PCG64(18))
+    ses = st.session()
+    orc = StageOracle(cfg, tensors, 0, 1, 1024, n_seq_max=len(chunks), blas=True)
+    for i, (past, T) in enumerate(chunks):
+        if past:
+            k, v = (rng.standard_normal((past, HK, D)).astype(np.float16).view(np.uint16) for _ in "kv")
+            ses.kv_write(0, i, 0, k, v)
+            orc.k[0, i, :, :past], orc.v[0, i, :, :past] = k.transpose(1, 0, 2), v.transpose(1, 0, 2)
+        x = rng.standard_normal((T, E)).astype(np.float32)
+        pos, seq = np.arange(past, past + T), np.full(T, i, np.int32)
+        got = ses.decode(x, pos, seq=seq).view(np.float32).reshape(T, E).astype(np.float64)
+        want = orc.forward(x, pos, seq=seq).astype(np.float64)
+        worst = np.max(np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1))
+        assert np.linalg.norm(got - want) <= TOL * np.linalg.norm(want) and worst <= 2 * TOL, (name, past, T, worst)
+    ses.close()
+    st.close()
