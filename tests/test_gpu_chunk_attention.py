@@ -8,6 +8,7 @@ import pytest
 torch = pytest.importorskip("torch")
 
 import models
+import oracle
 from oracle.stage import StageOracle
 from util import mesh
 
@@ -68,5 +69,47 @@ def test_walks_of_one_and_two_key_groups(tmp_path, name):
         want = orc.forward(x, pos, seq=seq).astype(np.float64)
         worst = np.max(np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1))
         assert np.linalg.norm(got - want) <= TOL * np.linalg.norm(want) and worst <= 2 * TOL, (name, past, T, worst)
+    ses.close()
+    st.close()
+
+
+def half(x):
+    return x.view(np.float16).astype(np.float32)
+
+
+# heads per KV head, KV heads and the shape of the workgroup: four and five waves, six of six heads and of three heads and two query tiles,
+# one head and four query tiles, eight
+QUANT = {"four": (4, 3), "five": (5, 2), "six": (6, 2), "three": (3, 2), "one": (1, 4), "eight": (8, 32)}
+
+
+@pytest.mark.parametrize("kv_types", [(oracle.Q8_0, oracle.Q4_0), (oracle.Q4_0, oracle.Q4_0)])
+@pytest.mark.parametrize("shape", sorted(QUANT))
+def test_chunks_over_quantised_rows(tmp_path, shape, kv_types):
+    """Chunks whose workgroups decode the cache rows themselves, at the edges of their steps, one and two key groups, against the oracle over
+    the rows that the device's cache holds."""
+    group, n_kv = QUANT[shape]
+    # (eight waves a workgroup from 256 workgroups of 32 queries on)
+    chunks = [(0, 225), (100, 230)] if shape == "eight" else [(0, 17), (0, 65), (63, 40), (64, 64), (127, 33), (0, 127), (300, 97), (190, 150)]
+    m = mesh()
+    cfg = dict(arch="llama", n_layer=1, n_embd=512, n_head=group * n_kv, n_head_kv=n_kv, head_dim=128, n_ff=512, n_vocab=256, eps=1e-5, rope=1e4)
+    path = os.path.join(str(tmp_path), "model.gguf")
+    tensors = models.write_model(path, cfg, [0], seed=6)
+    st = m.Stage(path, 0, 1, n_ctx=512, n_seq_max=len(chunks), n_batch_max=256, kv_types=kv_types)
+    rng = np.random.Generator(np.random.PCG64(28))
+    ses = st.session(chunk_kv16=0)
+    orc = StageOracle(cfg, tensors, 0, 1, 512, n_seq_max=len(chunks), blas=True, kv_types=kv_types)
+    for i, (past, T) in enumerate(chunks):
+        if past:
+            k, v = (rng.standard_normal((past, n_kv, 128)).astype(np.float16).view(np.uint16) for _ in "kv")
+            ses.kv_write(0, i, 0, k, v)
+            orc.k[0, i, :, :past], orc.v[0, i, :, :past] = (half(r).transpose(1, 0, 2) for r in ses.kv_read(0, i, 0, past))
+        x = rng.standard_normal((T, 512)).astype(np.float32)
+        pos, seq = np.arange(past, past + T), np.full(T, i, np.int32)
+        got = ses.decode(x, pos, seq=seq).view(np.float32).reshape(T, 512).astype(np.float64)
+        rows = tuple(half(r) for r in ses.kv_read(0, i, past, T))
+        want = orc.forward(x, pos, seq=seq, kv_rows={0: rows}).astype(np.float64)
+        worst = np.max(np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1))
+        # (kv_read rounds a row's values to f16, as the kernel that multiplies them does)
+        assert np.linalg.norm(got - want) <= TOL * np.linalg.norm(want) and worst <= 2 * TOL, (shape, past, T, worst)
     ses.close()
     st.close()
