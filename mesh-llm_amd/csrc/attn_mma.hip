@@ -22,7 +22,9 @@
 // What bounds it: the walk of a workgroup is a chain of row loads (29 GB/s per workgroup), beside it the conversion of
 // quantised rows (~430 vector instructions per 32 keys).  Against blocks of 16 keys with V scattered into the transposed
 // tile by 32 two-byte stores a lane: 64.4 -> 55.9 us (32 sequences of 2000 to 6000 keys, 8 heads, q8_0 / q4_0: 213 MB),
-// 17.4 -> 15.4 (16 sequences, 4 heads), f16 rows 41.4 -> 39.5 (16 sequences, 179 MB: 4.5 TB/s), 7.3 -> 6.8 (one).
+// 17.4 -> 15.4 (16 sequences, 4 heads), f16 rows 41.4 -> 39.5 (16 sequences, 179 MB: 4.5 TB/s), 7.3 -> 6.8 (one); f16 rows and whole
+// lines of V (ValueBlock) against those blocks of 16 keys, 8 heads of 128, 4000 keys, with the merge: 64 sequences 177 -> 177, 33 140 -> 129,
+// 20 69 -> 59, 5 23.6 -> 22.6, one 11.5 -> 10.9; of 64: 128 sequences 180 -> 172, 33 62 -> 62, 40 66 -> 69, 20 49 -> 33.
 
 #include "attn.hpp"
 #include "q16.hpp"
@@ -125,6 +127,47 @@ struct RowShare {
     // first dim of piece cc
     static __device__ __forceinline__ int dim0(int cc, int g) { return TYPE == MESH_F16 ? 32 * cc + 8 * g : HD / 4 * g + 8 * cc; }
 };
+// What a lane holds of the value rows of a 32-key block on their way to the wave's LDS tile [key][dim]; rows past the range are
+// clamped to its last key (their probabilities are zero).  Quantised rows: a lane's shares of rows c and 16 + c, as above.  f16 rows
+// pass as they are, so a load takes whole rows: the 16 lanes that the memory pipe works on at a time lie in two cache lines instead
+// of 16.  Looking lines up is what bounds a CU that walks two ranges at once: 33 sequences of 4000 keys, 8 KV heads, as shares of
+// rows / whole rows 69.5 / 61.9 us (rows of 64), 143 / 129 (128); 16 sequences 29.3 / 29.1 and 52.1 / 51.6.
+template <int TYPE, int HD, int PITCH>
+struct ValueBlock {
+    RowShare<TYPE, HD> r[2];
+    __device__ __forceinline__ void load(const uint8_t *rows, int kb, int j1, int lane) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            int key = kb + 16 * h + (lane & 15);
+            key = key < j1 ? key : j1 - 1;
+            r[h].load(rows + (size_t)key * kv_row_bytes(TYPE, HD), lane >> 4);
+        }
+    }
+    __device__ __forceinline__ void put(_Float16 *tile, int lane) const {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int cc = 0; cc < RowShare<TYPE, HD>::NC; ++cc)
+                *reinterpret_cast<mm_u4 *>(tile + (16 * h + (lane & 15)) * PITCH + RowShare<TYPE, HD>::dim0(cc, lane >> 4)) = r[h].piece(cc);
+    }
+};
+template <int HD, int PITCH>
+struct ValueBlock<MESH_F16, HD, PITCH> {
+    static constexpr int PIECES = HD / 8, ROWS = 64 / PIECES;       // 16-byte pieces of a row, rows of a load
+    mm_u4 v[MMA_KEYS / ROWS];
+    __device__ __forceinline__ void load(const uint8_t *rows, int kb, int j1, int lane) {
+#pragma unroll
+        for (int i = 0; i < MMA_KEYS / ROWS; ++i) {
+            int key = kb + i * ROWS + lane / PIECES;
+            key = key < j1 ? key : j1 - 1;
+            v[i] = *reinterpret_cast<const mm_u4 *>(rows + (size_t)key * (HD * 2) + lane % PIECES * 16);
+        }
+    }
+    __device__ __forceinline__ void put(_Float16 *tile, int lane) const {
+#pragma unroll
+        for (int i = 0; i < MMA_KEYS / ROWS; ++i) *reinterpret_cast<mm_u4 *>(tile + (i * ROWS + lane / PIECES) * PITCH + lane % PIECES * 8) = v[i];
+    }
+};
 // place, within its eight, of dim dd of a q4_0 piece
 __device__ __forceinline__ int mm_dim_slot(int dd) { return (dd & ~7) | ((dd & 3) << 1) | ((dd >> 2) & 1); }
 
@@ -185,28 +228,22 @@ __global__ __launch_bounds__(MMA_THREADS) void attn_mma_kernel(const float *p_q,
     float m = -INFINITY, l = 0.f;           // l: of this lane's keys only
 
     _Float16 *const sV = reinterpret_cast<_Float16 *>(s_raw) + wave * MMA_KEYS * VPITCH;
-    _Float16 *const v_put = sV + c * VPITCH;                                              // rows c and 16 + c of the tile
     const _Float16 *const v_get = sV + (4 * g + (c >> 2)) * VPITCH + 4 * (c & 3);         // (mm_read_transposed: rows 4 g .. + 4)
     const size_t base = ((size_t)seq * p_n_kv + kvh) * p_n_ctx;
-    // what a lane fetches of a 32-key block: its shares of key rows c and 16 + c; rows past the range are clamped to its
-    // last key (and masked below)
+    // what a lane fetches of a 32-key block: its shares of key rows c and 16 + c (rows past the range are clamped to its
+    // last key, and masked below), and of the value rows
     constexpr int STEP = MMA_WAVES * MMA_KEYS;
     constexpr int DEPTH = KT == MESH_F16 && VT == MESH_F16 ? MMA_DEPTH_F16 : MMA_DEPTH_Q;
     RowShare<KT, HD> krs[DEPTH][2];
-    RowShare<VT, HD> vrs[DEPTH][2];
-    auto fetch = [&](RowShare<KT, HD> (&kr)[2], RowShare<VT, HD> (&vr)[2], int kb) {
+    ValueBlock<VT, HD, VPITCH> vrs[DEPTH];
+    auto fetch = [&](RowShare<KT, HD> (&kr)[2], ValueBlock<VT, HD, VPITCH> &vr, int kb) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             int key = kb + 16 * h + c;
             key = key < j1 ? key : j1 - 1;
             kr[h].load(p_kcache + (base + key) * KRB, g);
         }
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            int key = kb + 16 * h + c;
-            key = key < j1 ? key : j1 - 1;
-            vr[h].load(p_vcache + (base + key) * VRB, g);
-        }
+        vr.load(p_vcache + base * VRB, kb, j1, lane);
     };
     const int kb0 = j0 + __builtin_amdgcn_readfirstlane(wave) * MMA_KEYS;
     if (kb0 < j1) {
@@ -219,7 +256,7 @@ __global__ __launch_bounds__(MMA_THREADS) void attn_mma_kernel(const float *p_q,
         const int kb = kbb + d * STEP;
         if (kb >= j1) break;
         RowShare<KT, HD> (&kr)[2] = krs[d];
-        RowShare<VT, HD> (&vr)[2] = vrs[d];
+        ValueBlock<VT, HD, VPITCH> &vr = vrs[d];
         // S^T = K . Q^T : register i of half h is key kb + 16 h + 4 g + i for head c
         mm_f4 s[2];
 #pragma unroll
@@ -229,10 +266,7 @@ __global__ __launch_bounds__(MMA_THREADS) void attn_mma_kernel(const float *p_q,
             for (int cc = 0; cc < NC; ++cc) s[h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(mm_h8, kr[h].piece(cc)), qf[cc], s[h], 0, 0, 0);
         }
         // V rows as they are: sV[key][dim]
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int cc = 0; cc < NC; ++cc) *reinterpret_cast<mm_u4 *>(v_put + 16 * h * VPITCH + RowShare<VT, HD>::dim0(cc, g)) = vr[h].piece(cc);
+        vr.put(sV, lane);
         // rows of a later block travel while this one is worked on (two blocks deep without a branch: the compiler then
         // counts the loads in flight exactly, 56 against 60 us; one block deep waits for all of them anyway, and the walks
         // of one block save the fetch)
