@@ -16,7 +16,6 @@
 #include "linear.hpp"
 
 #include <algorithm>
-#include <type_traits>
 
 namespace mesh {
 
@@ -64,34 +63,33 @@ __device__ __forceinline__ float4 ln_load4(const float *p, int k, int K) {
     if (k + 4 <= K) return *reinterpret_cast<const float4 *>(p + k);
     return make_float4(k < K ? p[k] : 0.f, k + 1 < K ? p[k + 1] : 0.f, k + 2 < K ? p[k + 2] : 0.f, 0.f);
 }
-// The same requested ahead, in two parts: a load that no branch lies around where K is a multiple of four (`whole`, the same for
-// all threads), and, once it is needed, its zeros.
+// The same requested ahead, in two parts: loads that no branch lies around, of 16 bytes where K is a multiple of four (WHOLE) and of 4
+// each otherwise, and, once they are needed, their zeros.  (With a branch for a row's last elements the weights wait for the vectors:
+// products of rows of 1031 0.6 us later each; both kinds in one kernel cost rows of 4096 as much.)
 template <bool WHOLE> __device__ __forceinline__ float4 ln_request4(const float *p, int k, int K) {
     if constexpr (WHOLE) return *reinterpret_cast<const float4 *>(p + (k < K ? k : K - 4));
-    return ln_load4(p, k, K);
+    auto at = [&](int i) { return p[i < K ? i : K - 1]; };
+    return make_float4(at(k), at(k + 1), at(k + 2), at(k + 3));
 }
-__device__ __forceinline__ void ln_settle4(float4 &v, int k, int K) {
-    if (k >= K) v = make_float4(0.f, 0.f, 0.f, 0.f);
-}
-template <typename Request> __device__ __forceinline__ void ln_request(int K, Request request) {
-    if (K & 3) request(std::false_type{});
-    else request(std::true_type{});
+template <bool WHOLE> __device__ __forceinline__ void ln_settle4(float4 &v, int k, int K) {
+    if constexpr (!WHOLE) v = make_float4(k < K ? v.x : 0.f, k + 1 < K ? v.y : 0.f, k + 2 < K ? v.z : 0.f, k + 3 < K ? v.w : 0.f);
+    else if (k >= K) v = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
 // A thread's first N groups of four elements of a vector, requested ahead; xs[k .. k + 3] = map(k, them) over [0, Kp), the groups
 // behind them loaded on the way.
-template <int N> struct StepVec {
+template <int N, bool WHOLE> struct StepVec {
     static constexpr int STRIDE = STEP_THREADS * 4;
     float4 v[N];
-    template <typename Whole> __device__ __forceinline__ void load(Whole, const float *p, int tid, int K) {
+    __device__ __forceinline__ void load(const float *p, int tid, int K) {
 #pragma unroll
-        for (int i = 0; i < N; ++i) v[i] = ln_request4<Whole::value>(p, tid * 4 + i * STRIDE, K);
+        for (int i = 0; i < N; ++i) v[i] = ln_request4<WHOLE>(p, tid * 4 + i * STRIDE, K);
     }
     template <typename Map> __device__ __forceinline__ void put(const float *p, int tid, int K, int Kp, Map map, float *xs) {
         for (int k0 = tid * 4; k0 < Kp; k0 += N * STRIDE) {
 #pragma unroll
             for (int i = 0; i < N; ++i) {
-                if (k0 == tid * 4) ln_settle4(v[i], k0 + i * STRIDE, K);
+                if (k0 == tid * 4) ln_settle4<WHOLE>(v[i], k0 + i * STRIDE, K);
                 else v[i] = ln_load4(p, k0 + i * STRIDE, K);
             }
 #pragma unroll
@@ -103,7 +101,7 @@ template <int N> struct StepVec {
     }
 };
 
-template <int R, int U, StepIn IN, StepOut OUT>
+template <int R, int U, StepIn IN, StepOut OUT, bool WHOLE>
 __global__ __launch_bounds__(STEP_THREADS, 4) void linear_step_kernel(const uint16_t *p_w, int p_Kp, int p_groups, int p_width, int p_K, const StepArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
     __shared__ StepScratch scratch;
@@ -146,8 +144,8 @@ __global__ __launch_bounds__(STEP_THREADS, 4) void linear_step_kernel(const uint
     // ---- the input vector
     static_assert(STEP_PARTS_MAX <= STEP_THREADS, "a partial sum per thread");
     if constexpr (IN == STEP_IN_VEC || IN == STEP_IN_RELU2) {
-        StepVec<4> in;
-        ln_request(K, [&](auto whole) { in.load(whole, a.in, tid, K); });
+        StepVec<4, WHOLE> in;
+        in.load(a.in, tid, K);
         fetch_first();
         auto sq = [](float v) { const float p = fmaxf(v, 0.f); return p * p; };
         in.put(a.in, tid, K, Kp, [&](int, const float4 &v) { return IN == STEP_IN_VEC ? v : make_float4(sq(v.x), sq(v.y), sq(v.z), sq(v.w)); }, xs);
@@ -156,8 +154,8 @@ __global__ __launch_bounds__(STEP_THREADS, 4) void linear_step_kernel(const uint
 #pragma unroll
         for (int i = 0; i < 3; ++i) p[i] = tid < a.n_part ? a.part[i * a.n_part + tid] : 0.f;
         const float f1 = a.coef[0], f2 = a.coef[1], f3 = a.coef[2], c0 = a.coef[3];
-        StepVec<4> in;
-        ln_request(K, [&](auto whole) { in.load(whole, a.in, tid, K); });
+        StepVec<4, WHOLE> in;
+        in.load(a.in, tid, K);
         fetch_first();
         step_block_sums<0>(p, scratch, lane, wave);
         const float c1 = f1 / sqrtf(p[0] / (float)K + a.eps), c2 = f2 / sqrtf(p[1] / (float)K + a.eps), c3 = f3 / sqrtf(p[2] / (float)K + a.eps);
@@ -167,8 +165,9 @@ __global__ __launch_bounds__(STEP_THREADS, 4) void linear_step_kernel(const uint
                    return make_float4(k < K ? poly(u.x) : 0.f, k + 1 < K ? poly(u.y) : 0.f, k + 2 < K ? poly(u.z) : 0.f, k + 3 < K ? poly(u.w) : 0.f);
                }, xs);
     } else if constexpr (IN == STEP_IN_UNIT_RMS) {
-        StepVec<1> in, gain;
-        ln_request(K, [&](auto whole) { in.load(whole, a.in, tid, K); gain.load(whole, a.gain, tid, K); });
+        StepVec<1, WHOLE> in, gain;
+        in.load(a.in, tid, K);
+        gain.load(a.gain, tid, K);
         fetch_first();
         float ss = 0.f;
         in.put(a.in, tid, K, Kp, [&](int, const float4 &v) { ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w; return v; }, xs);
@@ -185,23 +184,21 @@ __global__ __launch_bounds__(STEP_THREADS, 4) void linear_step_kernel(const uint
         const int k0 = tid * 4;
         const float inv_n = 1.0f / (float)K;
         float4 x4[AHEAD], y4[AHEAD], g4[AHEAD], b4[AHEAD], ng4[AHEAD], nb4[AHEAD];
-        ln_request(K, [&](auto whole) {
 #pragma unroll
-            for (int i = 0; i < AHEAD; ++i) {
-                const int k = k0 + i * STRIDE;
-                auto get = [&](const float *p) { return ln_request4<decltype(whole)::value>(p, k, K); };
-                x4[i] = get(a.in);
-                if (a.y) { y4[i] = get(a.y); g4[i] = get(a.gain); b4[i] = get(a.bias); }
-                ng4[i] = get(a.norm_gain); nb4[i] = get(a.norm_bias);
-            }
-        });
+        for (int i = 0; i < AHEAD; ++i) {
+            const int k = k0 + i * STRIDE;
+            auto get = [&](const float *p) { return ln_request4<WHOLE>(p, k, K); };
+            x4[i] = get(a.in);
+            if (a.y) { y4[i] = get(a.y); g4[i] = get(a.gain); b4[i] = get(a.bias); }
+            ng4[i] = get(a.norm_gain); nb4[i] = get(a.norm_bias);
+        }
         fetch_first();
 #pragma unroll
         for (int i = 0; i < AHEAD; ++i) {
             const int k = k0 + i * STRIDE;
-            ln_settle4(x4[i], k, K);
-            if (a.y) { ln_settle4(y4[i], k, K); ln_settle4(g4[i], k, K); ln_settle4(b4[i], k, K); }
-            ln_settle4(ng4[i], k, K); ln_settle4(nb4[i], k, K);
+            ln_settle4<WHOLE>(x4[i], k, K);
+            if (a.y) { ln_settle4<WHOLE>(y4[i], k, K); ln_settle4<WHOLE>(g4[i], k, K); ln_settle4<WHOLE>(b4[i], k, K); }
+            ln_settle4<WHOLE>(ng4[i], k, K); ln_settle4<WHOLE>(nb4[i], k, K);
         }
         auto sum4 = [](const float4 &v) { return (v.x + v.y) + (v.z + v.w); };
         auto dev4 = [&](int k, const float4 &v, float mean) {
@@ -261,14 +258,12 @@ __global__ __launch_bounds__(STEP_THREADS, 4) void linear_step_kernel(const uint
         float ss = tid < a.n_part ? a.part[tid] : 0.f;
         constexpr int AHEAD = 2;
         float4 x4[AHEAD], y4[AHEAD], g4[AHEAD];
-        ln_request(K, [&](auto whole) {
 #pragma unroll
-            for (int i = 0; i < AHEAD; ++i) {
-                const int k = (tid + i * STEP_THREADS) * 4;
-                auto get = [&](const float *p) { return ln_request4<decltype(whole)::value>(p, k, K); };
-                x4[i] = get(a.in); y4[i] = get(a.y); g4[i] = get(a.gain);
-            }
-        });
+        for (int i = 0; i < AHEAD; ++i) {
+            const int k = (tid + i * STEP_THREADS) * 4;
+            auto get = [&](const float *p) { return ln_request4<WHOLE>(p, k, K); };
+            x4[i] = get(a.in); y4[i] = get(a.y); g4[i] = get(a.gain);
+        }
         fetch_first();
         ss = step_block_sum<0>(ss, scratch, lane, wave);
         const float rinv = 1.0f / sqrtf(ss / (float)K + a.eps);
@@ -288,7 +283,7 @@ __global__ __launch_bounds__(STEP_THREADS, 4) void linear_step_kernel(const uint
 #pragma unroll
         for (int i = 0; i < AHEAD; ++i) {
             const int k = (tid + i * STEP_THREADS) * 4;
-            ln_settle4(x4[i], k, K); ln_settle4(y4[i], k, K); ln_settle4(g4[i], k, K);
+            ln_settle4<WHOLE>(x4[i], k, K); ln_settle4<WHOLE>(y4[i], k, K); ln_settle4<WHOLE>(g4[i], k, K);
             update(k, x4[i], y4[i], g4[i]);
         }
         for (int k = (tid + AHEAD * STEP_THREADS) * 4; k < Kp; k += STEP_THREADS * 4) update(k, ln_load4(a.in, k, K), ln_load4(a.y, k, K), ln_load4(a.gain, k, K));
@@ -395,17 +390,21 @@ int linear_step_grid(const StepArgs &a) {
     return (wgs + turns - 1) / turns;
 }
 
-template <int R, int U, StepIn IN, StepOut OUT>
-static int launch_step(const StepArgs &a, hipStream_t stream) {
+template <int R, int U, StepIn IN, StepOut OUT, bool WHOLE>
+static int launch_step_of(const StepArgs &a, hipStream_t stream) {
     const size_t lds = (size_t)a.W.Kp * sizeof(float);
     static bool ready = false;        // (hosts are single-threaded per session; a second thread sets the same attribute)
     if (!ready) {
-        MESH_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(linear_step_kernel<R, U, IN, OUT>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)STEP_LDS_MAX));
+        MESH_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(linear_step_kernel<R, U, IN, OUT, WHOLE>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)STEP_LDS_MAX));
         ready = true;
     }
-    MESH_LAUNCH((linear_step_kernel<R, U, IN, OUT>), dim3((unsigned)linear_step_grid(a)), dim3(STEP_THREADS), lds, stream, a.W.w, a.W.Kp, step_groups(a), a.width, a.W.K, a);
+    MESH_LAUNCH((linear_step_kernel<R, U, IN, OUT, WHOLE>), dim3((unsigned)linear_step_grid(a)), dim3(STEP_THREADS), lds, stream, a.W.w, a.W.Kp, step_groups(a), a.width, a.W.K, a);
     MESH_LAUNCH_CHECK();
     return MESH_OK;
+}
+template <int R, int U, StepIn IN, StepOut OUT>
+static int launch_step(const StepArgs &a, hipStream_t stream) {
+    return a.W.K % 4 ? launch_step_of<R, U, IN, OUT, false>(a, stream) : launch_step_of<R, U, IN, OUT, true>(a, stream);
 }
 template <StepIn IN, StepOut OUT>
 static int launch_step_rows(const StepArgs &a, hipStream_t stream) {
