@@ -139,7 +139,10 @@ __global__ __launch_bounds__(STEP_THREADS, 4) void linear_step_kernel(const uint
     Batch b0, b1;
     const int first = blockIdx.x * STEP_WAVES + wave;
     const int turns = first < p_groups ? (p_groups - first + g_step - 1) / g_step : 0;
-    auto fetch_first = [&]() { fetch(b0, turns ? first : p_groups - 1, 0); };
+    auto fetch_first = [&]() {
+        asm volatile("" ::: "memory");          // (or the compiler moves the vectors' loads to where they are used, behind these)
+        fetch(b0, turns ? first : p_groups - 1, 0);
+    };
 
     // ---- the input vector
     static_assert(STEP_PARTS_MAX <= STEP_THREADS, "a partial sum per thread");
