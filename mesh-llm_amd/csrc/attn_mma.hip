@@ -27,6 +27,7 @@
 // 20 69 -> 59, 5 23.6 -> 22.6, one 11.5 -> 10.9; of 64: 128 sequences 180 -> 172, 33 62 -> 62, 40 66 -> 69, 20 49 -> 33.
 
 #include "attn.hpp"
+#include "lds_ops.hpp"
 #include "q16.hpp"
 
 namespace mesh {
@@ -44,19 +45,7 @@ typedef _Float16 mm_h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 mm_h2 __attribute__((ext_vector_type(2)));
 typedef float mm_f4 __attribute__((ext_vector_type(4)));
 typedef uint32_t mm_u4 __attribute__((ext_vector_type(4)));
-typedef uint32_t mm_u2 __attribute__((ext_vector_type(2)));
 typedef uint32_t mm_u4a8 __attribute__((ext_vector_type(4), aligned(8)));
-typedef short mm_s4 __attribute__((ext_vector_type(4)));
-
-// Four halves of one column of a 4-row x 16-column tile: lane i of a group of 16 lanes hands in the address of row i / 4,
-// columns 4 (i % 4) .. + 4, and receives column i of the four rows.
-__device__ __forceinline__ mm_u2 mm_read_transposed(const _Float16 *p) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    return __builtin_bit_cast(mm_u2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) mm_s4 *)p));
-#else
-    return mm_u2{0, 0};
-#endif
-}
 
 __device__ __forceinline__ uint32_t mm_pack(float a, float b) {
     const mm_h2 h = {(_Float16)a, (_Float16)b};
@@ -228,7 +217,7 @@ __global__ __launch_bounds__(MMA_THREADS) void attn_mma_kernel(const float *p_q,
     float m = -INFINITY, l = 0.f;           // l: of this lane's keys only
 
     _Float16 *const sV = reinterpret_cast<_Float16 *>(s_raw) + wave * MMA_KEYS * VPITCH;
-    const _Float16 *const v_get = sV + (4 * g + (c >> 2)) * VPITCH + 4 * (c & 3);         // (mm_read_transposed: rows 4 g .. + 4)
+    const _Float16 *const v_get = sV + (4 * g + (c >> 2)) * VPITCH + 4 * (c & 3);         // (lds_read_transposed: rows 4 g .. + 4)
     const size_t base = ((size_t)seq * p_n_kv + kvh) * p_n_ctx;
     // what a lane fetches of a 32-key block: its shares of key rows c and 16 + c (rows past the range are clamped to its
     // last key, and masked below), and of the value rows
@@ -307,7 +296,7 @@ __global__ __launch_bounds__(MMA_THREADS) void attn_mma_kernel(const float *p_q,
         // O^T += V^T . P^T : the V^T operand is place 16 db + c of the rows, keys in the order of P^T
 #pragma unroll
         for (int db = 0; db < NDB; ++db) {
-            const mm_u2 v0 = mm_read_transposed(v_get + 16 * db), v1 = mm_read_transposed(v_get + 16 * VPITCH + 16 * db);
+            const lds_u2 v0 = lds_read_transposed(v_get + 16 * db), v1 = lds_read_transposed(v_get + 16 * VPITCH + 16 * db);
             const mm_u4 vv = {v0[0], v0[1], v1[0], v1[1]};
             o[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(mm_h8, vv), pf, o[db], 0, 0, 0);
         }

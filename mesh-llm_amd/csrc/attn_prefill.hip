@@ -32,6 +32,7 @@
 
 #include "act_math.hpp"
 #include "attn.hpp"
+#include "lds_ops.hpp"
 
 namespace mesh {
 
@@ -50,29 +51,7 @@ typedef _Float16 pf_h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 pf_h2 __attribute__((ext_vector_type(2)));
 typedef float pf_f16v __attribute__((ext_vector_type(16)));
 typedef uint32_t pf_u4 __attribute__((ext_vector_type(4)));
-typedef uint32_t pf_u2 __attribute__((ext_vector_type(2)));
-typedef short pf_s4 __attribute__((ext_vector_type(4)));
 
-// Four halves of one column of a 4-row x 16-column tile: lane i of a group of 16 lanes hands in the address of row i / 4,
-// columns 4 (i % 4) .. + 4, and receives column i of the four rows.
-__device__ __forceinline__ pf_u2 pf_read_transposed(const _Float16 *p) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    return __builtin_bit_cast(pf_u2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) pf_s4 *)p));
-#else
-    return pf_u2{0, 0};
-#endif
-}
-// 1 KB from memory to LDS: the 16 bytes at base + off (a lane's own) go to dst + 16 lane (bytes, dst uniform).  As text: the compiler
-// would wait for them at the next access to LDS, the step after waits itself.
-__device__ __forceinline__ void pf_load_to_lds(const uint8_t *base, uint32_t off, const _Float16 *dst) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    const unsigned place = (unsigned)(unsigned long long)(__attribute__((address_space(3))) const _Float16 *)dst;
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"         // (m0 is reserved: named so that the compiler keeps its own uses away)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(place)), "v"(off), "s"(base) : "memory", "m0");
-#pragma clang diagnostic pop
-#endif
-}
 __device__ __forceinline__ void pf_step_barrier() {
 #if defined(__HIP_DEVICE_COMPILE__)
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -176,12 +155,12 @@ __global__ __launch_bounds__(512) void attn_chunk_kernel(const AttnArgs a, int T
 #pragma unroll
         for (int i = 0; i < NP; ++i) {
             const int kb = wv + i * n_waves, at = kb * 64 + lane, row = at / PIECES, piece = (at % PIECES) ^ pf_swizzle<HD>(row);
-            if (kb < PF_STAGE * HD / 512) pf_load_to_lds(k_rows, row_of(k0 + row) * KRB + piece * 16, sK[buf] + kb * 512);
+            if (kb < PF_STAGE * HD / 512) load_to_lds_16(k_rows, row_of(k0 + row) * KRB + piece * 16, lds_place(sK[buf] + kb * 512));
         }
 #pragma unroll
         for (int i = 0; i < NP; ++i) {
             const int kb = wv + i * n_waves, at = kb * 64 + lane, row = at / VPIECES, piece = (at % VPIECES) ^ pf_swizzle<VD>(row);
-            if (kb < PF_STAGE * VD / 512) pf_load_to_lds(v_rows, row_of(k0 + row) * VRB + piece * 16, sV[buf] + kb * 512);
+            if (kb < PF_STAGE * VD / 512) load_to_lds_16(v_rows, row_of(k0 + row) * VRB + piece * 16, lds_place(sV[buf] + kb * 512));
         }
     };
     // quantised rows travel through registers: requested ahead of a step's products, decoded and written behind them
@@ -203,7 +182,7 @@ __global__ __launch_bounds__(512) void attn_chunk_kernel(const AttnArgs a, int T
             if (p < PF_STAGE * VPIECES) *reinterpret_cast<uint4 *>(sV[buf] + (p / VPIECES) * VD + ((p % VPIECES) ^ pf_swizzle<VD>(p / VPIECES)) * 8) = pf_decode<VT>(rv[i]);
         }
     };
-    // V^T operand: dim 32 db + lane % 32, keys of a 32-key tile 8 quad + 4 half .. + 4 (pf_read_transposed: this lane hands in row
+    // V^T operand: dim 32 db + lane % 32, keys of a 32-key tile 8 quad + 4 half .. + 4 (lds_read_transposed: this lane hands in row
     // (lane % 16) / 4 of the four, 4 dims)
     const int tr_row = 4 * half + ((lane & 15) >> 2), tr_piece = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1), tr_at = 4 * (lane & 1);
     if (k_lo < n_keys) {
@@ -310,11 +289,11 @@ __global__ __launch_bounds__(512) void attn_chunk_kernel(const AttnArgs a, int T
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
                 if (t == 1 && !two) break;
-                pf_u2 v[4];
+                lds_u2 v[4];
 #pragma unroll
                 for (int quad = 0; quad < 4; ++quad) {
                     const int row = 32 * t + 8 * quad + tr_row;
-                    v[quad] = pf_read_transposed(tV + row * VD + ((4 * db + tr_piece) ^ pf_swizzle<VD>(row)) * 8 + tr_at);
+                    v[quad] = lds_read_transposed(tV + row * VD + ((4 * db + tr_piece) ^ pf_swizzle<VD>(row)) * 8 + tr_at);
                 }
                 const pf_u4 v1 = {v[0][0], v[0][1], v[1][0], v[1][1]}, v2 = {v[2][0], v[2][1], v[3][0], v[3][1]};
                 o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(pf_h8, v1), pf[t][0], o[db], 0, 0, 0);

@@ -29,6 +29,7 @@
 
 #include "gemm.hpp"
 #include "gemv_device.hpp"
+#include "lds_ops.hpp"
 
 namespace mesh {
 namespace f16sk {
@@ -216,19 +217,6 @@ __device__ __forceinline__ void to_mfma_lanes(TileRegs<MESH_Q6_K> &R, int src_la
 // element (row k, column t) of k8-major f16 activations with K rows per column: block t / 16 of 16 * K halfs
 __device__ __forceinline__ size_t k8_at(int K, int k, int t) { return (size_t)(t >> 4) * 16 * K + ((size_t)(k >> 3) * 16 + (t & 15)) * 8 + (k & 7); }
 
-// 1 KB from memory to LDS without passing registers: the 16 bytes at base + off (bytes, a lane's own) go to dst + 4 lane (dst
-// uniform).  As text: behind the builtin the compiler waits for every load in flight at the next cross-lane move, which counts as
-// an LDS access.  Its own counts stay right, a load it does not know of only makes a wait stricter; the reader sees to it itself that
-// they have arrived.
-__device__ __forceinline__ void load_to_lds_16(const float *base, int off, float *dst) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    const unsigned place = (unsigned)(unsigned long long)(__attribute__((address_space(3))) float *)dst;
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"         // (m0 is reserved: named so that the compiler keeps its own uses away)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(place)), "v"(off), "s"(base) : "memory", "m0");
-#pragma clang diagnostic pop
-#endif
-}
 // KB per wave and column block that hold a wave's share of the partial sums
 constexpr int NORM_CHUNKS = SKINNY_F16_NORM_PARTS_MAX / SK_WAVES * SK_NT / 256;
 static_assert(NORM_CHUNKS * 256 * SK_WAVES == SKINNY_F16_NORM_PARTS_MAX * SK_NT, "shares of whole KB");
@@ -350,7 +338,7 @@ __device__ __forceinline__ void skinny_workgroup(int bx, const _Float16 *p_x, co
 #pragma unroll
         for (int i = 0; i < NORM_CHUNKS * NC; ++i) {
             const int at = wave * parts_per * NT + i * 256 + lane * 4;
-            load_to_lds_16(src, 4 * (at < last ? at : last), my_parts + i * 256);
+            load_to_lds_16(src, 4u * (at < last ? at : last), lds_place(my_parts + i * 256));
         }
     }
     // outputs of a thread: column tid % NT and row (tid / NT) % 16 of the tile-rows out_j, out_j + OUT_STEP, ...

@@ -21,6 +21,7 @@
 
 #include <type_traits>
 
+#include "lds_ops.hpp"
 #include "mesh_common.hpp"
 
 namespace mesh {
@@ -124,13 +125,8 @@ __device__ __forceinline__ void gt_multiply(char *smem, gt_f16v (&acc)[2][2], co
     }
     auto load = [&](int stage, int k) {
         const uint32_t at = (uint32_t)(k < n_steps ? k : n_steps - 1);        // (past the end: the last step again, read by nobody)
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"         // (m0 is reserved: named so that the compiler keeps its own uses away)
 #pragma unroll
-        for (int j = 0; j < PER; ++j)
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(place[j] + stage * STAGE)), "v"(off[j] + at * step_bytes[j]), "s"(src[j])
-                         : "memory", "m0");
-#pragma clang diagnostic pop
+        for (int j = 0; j < PER; ++j) load_to_lds_16(src[j], off[j] + at * step_bytes[j], place[j] + stage * STAGE);
     };
     // fragments of this wave's 64 rows: lane -> row lane % 32 of a 32-row half, 8 elements from 8 * (lane / 32) of a k16 step
     const int r16 = lane & 15, half = lane >> 5;
