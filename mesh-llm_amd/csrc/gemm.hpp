@@ -144,8 +144,9 @@ bool moe_combine_quant16_supported(int n);
 int moe_combine_quant16(float *x, const float *y, const float *w, int T, int n, int top_k, const float *norm_w, float eps, uint8_t *yq, hipStream_t stream);
 // The "k8-major" f16 layout the large-tile GEMM reads: blocks of 16 tokens, element (t, k) of block t / 16 at
 // ((k / 8) * 16 + t % 16) * 8 + k % 8 within the block of 16 * K halfs; columns beyond T hold zeros.
-// The same launches on the f16 matrix cores (gemm_skinny_f16.hip): activations in the k8-major f16 layout below, weights
-// dequantised to f16 with one rounding each.  Faster than the integer kernel, less precise (f16 activations).
+// The same launches on the f16 matrix cores (gemm_skinny_f16.hip): activations in the k8-major f16 layout above, weights as the
+// integers of their quants and scales in f16, the super-blocks' factors on the f32 sums.  Faster than the integer kernel, less
+// precise (f16 activations).
 struct SkinnyF16Args {
     GemvMat mat[3];
     int n_mat = 1;                   // for EPI_SWIGLU exactly 2 (gate, up), written through mat[0].y and/or y16

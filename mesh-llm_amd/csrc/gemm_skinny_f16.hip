@@ -4,15 +4,17 @@
 // The alternative to the integer kernel of gemm_skinny.hip for the same launches: the weight stream is organised as in
 // the mat-vec kernel -- a workgroup owns a few tile-rows (16 rows each), its waves split K and each keeps two
 // weight tiles in flight -- and a tile is formed in registers as f16 and multiplied with 16 activation columns at
-// once (v_mfma_f32_16x16x32_f16).  Activations are f16 (11 significant bits against the integer kernel's 16-bit fixed point);
-// weights are exact: a fragment holds the integers q * sc (q4_K, at most 945) or (q - 32) * sc (q6_K), the sub-block minimum's
-// integers go through MFMAs of their own, and the super-block's d and dmin multiply the tile's sums in f32.  (Before, a weight
-// was rounded to f16 once; a first version multiplied by d * sc rounded to f16, which does not average out over K.)
+// once (v_mfma_f32_16x16x32_f16).  Activations are f16 (11 significant bits against the integer kernel's 16-bit fixed point).
+// A fragment holds the integers q * sc of q4_K (at most 945, exact) or (q - 32) * sc of q6_K (exact up to 2048; odd ones above, up
+// to 4096, are rounded by 2^-12 of themselves), the sub-block minimum's integers go through MFMAs of their own, and the super-block's
+// d and dmin multiply the tile's sums in f32.  (Before, every weight was rounded to f16 once; a first version multiplied by d * sc
+// rounded to f16, which does not average out over K.)
 //
-// What bounds it.  By time stamps (gate / up of 28672 x 4096, 5 tokens): first loads requested at 2.3 us, weight stream done at 11.2
-// (66 MB in 8.5 us, the memory's rate), the slowest wave at 14.9, end 16.1 (20.3 with the last workgroup).  The stream before was
-// as fast, but every round waited for all it had requested (a branch around a tile makes the compiler assume the worst), the
-// norm's partial sums were fetched behind it (2.9 us) and the epilogue's operands behind the barrier (1.5 - 2).
+// What bounds it.  By time stamps (gate / up of 28672 x 4096, 66 MB, 5 tokens): first loads requested at 2.3 us, a workgroup's weight
+// stream done at 11.2, its slowest wave at 14.9, its end 16.1; the last workgroup ends at 20.3, so the launch as a whole streams at
+// 3.2 TB/s of the 5.9 - 6.1 that reads reach.  Before, every round waited for all it had requested (a branch around
+// a tile makes the compiler assume the worst), the norm's partial sums were fetched behind it (2.9 us) and the epilogue's operands
+// behind the barrier (1.5 - 2).
 // Now / before, us: 5 tokens gate / up 20.4 / 22.4, q/k/v 10.1 - 10.8 / 11.6 - 12.0, output and q4_K down 9.8 / 10.4, q6_K down
 // 17.0 / 19.1; 16 tokens 21.1 / 23.4, 10.8 - 11.1 / 12.5 - 12.7, 10.2 / 11.1, 17.7 / 19.7; 32 tokens of the 32B shape (160 workgroups
 // of two tile-rows) q6_K down 52.3 / 55.0, q4_K down and output 24.5 / 27.9, q/k/v 15.6 / 16.1.
@@ -462,15 +464,12 @@ __device__ __forceinline__ void skinny_workgroup(int bx, const _Float16 *p_x, co
             }
             continue;
         }
-        float out;
-        if (NU == 2) {
+        float out = s0;
+        if constexpr (NU == 2) {
             if (a.bias[1]) s1 += a.bias[1][row];
             out = (s0 / (1.0f + expf(-s0))) * s1;
         } else if (a.epi == EPI_RESIDUAL) {
-            if constexpr (NU == 1) out = (k == 0 ? pre_res[0] : k == 1 ? pre_res[1] : a.residual[(size_t)t * a.ldres + row]) + s0;
-            else out = s0;
-        } else {
-            out = s0;
+            out = (k == 0 ? pre_res[0] : k == 1 ? pre_res[1] : a.residual[(size_t)t * a.ldres + row]) + s0;
         }
         if (a.y[mi]) a.y[mi][(size_t)t * a.ldy[mi] + row] = out;
         // (saturating: a SwiGLU product beyond the f16 range becomes +-65504, not an infinity the next GEMM would spread)

@@ -586,7 +586,11 @@ int attn_splits_for(const Tuning &tune, int T, int n_kv, int max_keys, bool quan
     // workgroups stream at the memory's rate.  Quantised rows are bound by the instructions that decode them, and two
     // workgroups per CU hide each other's waits: 3-7% of the step at batch 8-32 (Qwen2.5-32B shape, q8_0 / q4_0 cache:
     // 9.86 -> 9.18 ms at batch 32, which otherwise runs unsplit); four per CU lose again, and so do 64 splits of a single
-    // token's walk (from 64 (token, KV head) pairs on).
+    // token's walk (from 64 (token, KV head) pairs on).  (Those of a kernel whose waves took 16 keys a step.)
+    // 64 keys a split at least, which gives two of the matrix-core kernel's four waves work (32 keys a wave step); against 128 keys,
+    // attention and merge, us, 8 KV heads, f16 rows: one token 128 keys 7.8 / 6.6 (unsplit), 256 8.4 / 8.7, 400 9.4 / 9.1, 512 7.8 /
+    // 9.3, 1000 8.3 / 8.8, 2000 9.4 / 9.2; 5 tokens 128 8.1 / 5.8, 256 8.8 / 8.9, 512 11.0 / 9.6, from 700 on the same splits; 16 tokens
+    // 128 8.6 / 6.2, from 192 on the same; q8_0 / q4_0 rows 128 8.4 / 6.6, 512 8.0 / 9.1, 1000 8.6 / 8.5 (one token).
     // (attn_split_target: the workgroup count aimed at, for experiments)
     const int forced = tune.attn_split_target;
     const int target = forced ? forced : (quantised && T * n_kv >= 64) ? 512 : 256;
