@@ -15,9 +15,9 @@
 // 3.2 TB/s of the 5.9 - 6.1 that reads reach.  Before, every round waited for all it had requested (a branch around
 // a tile makes the compiler assume the worst), the norm's partial sums were fetched behind it (2.9 us) and the epilogue's operands
 // behind the barrier (1.5 - 2).
-// Now / before, us: 5 tokens gate / up 20.4 / 22.4, q/k/v 10.1 - 10.8 / 11.6 - 12.0, output and q4_K down 9.8 / 10.4, q6_K down
-// 17.0 / 19.1; 16 tokens 21.1 / 23.4, 10.8 - 11.1 / 12.5 - 12.7, 10.2 / 11.1, 17.7 / 19.7; 32 tokens of the 32B shape (160 workgroups
-// of two tile-rows) q6_K down 52.3 / 55.0, q4_K down and output 24.5 / 27.9, q/k/v 15.6 / 16.1.
+// Before / now, us: 5 tokens gate / up 22.6 / 20.5, q/k/v 11.8 - 12.0 / 10.1 - 10.7, output 7.4 / 7.6, q4_K down 16.4 / 14.4, q6_K down
+// 19.4 / 17.2; 16 tokens 23.3 / 21.0, 12.6 - 12.9 / 10.8 - 11.6, 7.9 / 7.6, 16.7 / 14.8, 19.7 / 17.7; 32 tokens of the 32B shape (160
+// workgroups of two tile-rows) q6_K down 59.0 / 52.4, q4_K down 57.4 / 44.8, output 17.0 / 14.5, q/k/v 16.7 - 18.4 / 15.8 - 16.2.
 //
 // Register dequantisation: lane (m = l % 16, g = l / 16) loads what lane 4m + g of the mat-vec kernel loads, i.e.
 // quarter g of row m of the super-block (gemv.hpp).  An MFMA's k-slots of lane group g are then 8 consecutive
