@@ -101,8 +101,10 @@ size_t hybrid_chunk_table(mesh_session *s, const mesh_batch *b, int32_t *table, 
     HybridSession &h = *s->hybrid;
     if (!s->stage->hybrid->has_chunks) return 0;
     const size_t B = (size_t)s->stage->n_batch_max;
-    int32_t *chunk = table, *first = chunk + B + 1, *run = first + B;
+    int32_t one[5];            // (a single token: nothing reads the tables)
+    int32_t *chunk = table ? table : one, *first = table ? chunk + B + 1 : one + 2, *run = table ? first + B : one + 3;
     int nc = 0, nr = 0, start = 0;
+    if (!table && b->n_tokens != 1) return 0;
     for (int i = 0; i < b->n_tokens; ++i) {
         const bool opens = i == 0 || (b->seq_id && b->seq_id[i] != b->seq_id[i - 1]);
         if (opens) { start = i; run[nr++] = nc; }
@@ -141,10 +143,10 @@ uint64_t hybrid_graph_key(const mesh_session *s, int T, int max_keys) {
     return key;
 }
 
-int hybrid_embed(mesh_session *s, int T) {
+int hybrid_embed(mesh_session *s, int T, const EmbedToken *one) {
     const HybridModel &hm = *s->stage->hybrid;
     ProfScope ps(s, MESH_PROF_CODEC);
-    return embed_rows(hm.embed, hm.embed_ld, s->d_tok, s->d_pos, hm.freq, hm.spec.embed_scale, T, hm.spec.width, s->x, s->stream);
+    return embed_rows(hm.embed, hm.embed_ld, s->d_tok, s->d_pos, hm.freq, hm.spec.embed_scale, T, hm.spec.width, s->x, one, s->stream);
 }
 
 // q, k of the call in h.big -> attention output in h.acta: f32 rows for the single-token step, else the product's activations

@@ -87,11 +87,12 @@ void hybrid_note_batch(mesh_session *s, const mesh_batch *b, bool ok);
 // Layers that read the token ids of the call.
 bool hybrid_needs_ids(const mesh_stage *st);
 // The tables of StateChunks for a call, into `table` (3 * n_batch_max + 2 entries; the device copy is at d_table); entries used,
-// 0 if the call needs none.
+// 0 if the call needs none (every token a run of its own; a single token's table may be null).
 size_t hybrid_chunk_table(mesh_session *s, const mesh_batch *b, int32_t *table, const int32_t *d_table);
 bool hybrid_single_step(const mesh_session *s, int T);
 uint64_t hybrid_graph_key(const mesh_session *s, int T, int max_keys);
-int hybrid_embed(mesh_session *s, int T);
+// one: the token of a call of one whose position, sequence and id are not on the device yet (embed_rows leaves them there)
+int hybrid_embed(mesh_session *s, int T, const EmbedToken *one);
 int hybrid_run_layers(mesh_session *s, int T, int max_keys);
 // after the layers: the residual stream complete (returned in *x), or logits of n_rows rows (rows null: the first n_rows)
 int hybrid_finish(mesh_session *s, int T, float **x);

@@ -515,26 +515,26 @@ int moe_group(const int32_t *ids, int n_pairs, int n_expert, int32_t *items, int
     return MESH_OK;
 }
 
-// x[t][i] += sum_s w[t][s] * y[(t*top_k + s)][i]
-__global__ __launch_bounds__(256) void moe_combine_kernel(float *__restrict__ x, const float *__restrict__ y,
+// out[t][i] = x[t][i] + sum_s w[t][s] * y[(t*top_k + s)][i]; out may be x
+__global__ __launch_bounds__(256) void moe_combine_kernel(const float *x, float *out, const float *__restrict__ y,
                                                           const float *__restrict__ w, int n_embd, int top_k) {
     const int t = blockIdx.y;
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n_embd) return;
     float acc = x[(size_t)t * n_embd + i];
     for (int s = 0; s < top_k; ++s) acc = fmaf(w[(size_t)t * top_k + s], y[((size_t)t * top_k + s) * n_embd + i], acc);
-    x[(size_t)t * n_embd + i] = acc;
+    out[(size_t)t * n_embd + i] = acc;
 }
 
-int moe_combine(float *x, const float *y, const float *w, int T, int n_embd, int top_k, hipStream_t stream) {
+int moe_combine(const float *x, float *out, const float *y, const float *w, int T, int n_embd, int top_k, hipStream_t stream) {
     if (T <= 0) return MESH_OK;
-    MESH_LAUNCH(moe_combine_kernel, dim3((unsigned)((n_embd + 255) / 256), (unsigned)T), dim3(256), 0, stream, x, y, w, n_embd, top_k);
+    MESH_LAUNCH(moe_combine_kernel, dim3((unsigned)((n_embd + 255) / 256), (unsigned)T), dim3(256), 0, stream, x, out, y, w, n_embd, top_k);
     MESH_LAUNCH_CHECK();
     return MESH_OK;
 }
 
-// the same with the rows of y at the slots of moe_sort: x[t][i] += sum_s w[t][s] * y[slot_of_pair[t*top_k + s]][i], four columns a thread
-__global__ __launch_bounds__(256) void moe_combine_slots_kernel(float *__restrict__ x, const float *__restrict__ y, const float *__restrict__ w,
+// the same with the rows of y at the slots of moe_sort: out[t][i] = x[t][i] + sum_s w[t][s] * y[slot_of_pair[t*top_k + s]][i], four columns a thread
+__global__ __launch_bounds__(256) void moe_combine_slots_kernel(const float *x, float *out, const float *__restrict__ y, const float *__restrict__ w,
                                                                 const int32_t *__restrict__ slot_of_pair, int n_embd, int top_k) {
     const int t = blockIdx.y;
     const int i = (blockIdx.x * 256 + threadIdx.x) * 4;
@@ -545,13 +545,13 @@ __global__ __launch_bounds__(256) void moe_combine_slots_kernel(float *__restric
         const float4 v = *reinterpret_cast<const float4 *>(y + (size_t)slot_of_pair[(size_t)t * top_k + s] * n_embd + i);
         acc.x = fmaf(ws, v.x, acc.x); acc.y = fmaf(ws, v.y, acc.y); acc.z = fmaf(ws, v.z, acc.z); acc.w = fmaf(ws, v.w, acc.w);
     }
-    *reinterpret_cast<float4 *>(x + (size_t)t * n_embd + i) = acc;
+    *reinterpret_cast<float4 *>(out + (size_t)t * n_embd + i) = acc;
 }
 
-int moe_combine_slots(float *x, const float *y, const float *w, const int32_t *slot_of_pair, int T, int n_embd, int top_k, hipStream_t stream) {
+int moe_combine_slots(const float *x, float *out, const float *y, const float *w, const int32_t *slot_of_pair, int T, int n_embd, int top_k, hipStream_t stream) {
     if (T <= 0) return MESH_OK;
     if (n_embd % 4) return fail(MESH_ERR_INVALID, "moe_combine_slots: row length %d not a multiple of 4", n_embd);
-    MESH_LAUNCH(moe_combine_slots_kernel, dim3((unsigned)((n_embd / 4 + 255) / 256), (unsigned)T), dim3(256), 0, stream, x, y, w, slot_of_pair, n_embd, top_k);
+    MESH_LAUNCH(moe_combine_slots_kernel, dim3((unsigned)((n_embd / 4 + 255) / 256), (unsigned)T), dim3(256), 0, stream, x, out, y, w, slot_of_pair, n_embd, top_k);
     MESH_LAUNCH_CHECK();
     return MESH_OK;
 }

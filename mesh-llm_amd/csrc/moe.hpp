@@ -32,11 +32,11 @@ int moe_group(const int32_t *ids, int n_pairs, int n_expert, int32_t *items, int
 // ([T][n_expert]) is required.
 bool moe_router_group_supported(int E, int n_expert, int top_k, int T);
 // arrive (optional): a device int that is zero between launches; with it the two launches become one, whose last-arriving
-// workgroup routes and groups (same results)
+// workgroup routes and groups (same results).
 int moe_router_group(const MoeRouteArgs &a, const float *x, int ldx, const float *norm_w, float eps, const float *W, int E,
                      float *logits, int T, int32_t *items, int32_t *n_items, int item_pairs, hipStream_t stream, int *arrive = nullptr);
-// x[t] += sum_s weights[t][s] * y[t*top_k + s]
-int moe_combine(float *x, const float *y, const float *w, int T, int n_embd, int top_k, hipStream_t stream);
+// out[t] = x[t] + sum_s weights[t][s] * y[t*top_k + s]; out may be x
+int moe_combine(const float *x, float *out, const float *y, const float *w, int T, int n_embd, int top_k, hipStream_t stream);
 
 // The pairs sorted by expert, for the expert launches of the large-tile GEMM (gemm.hpp): the pairs of an expert take
 // consecutive slots from a multiple of 16 on (padding slots in between hold no pair), experts in ascending order, and
@@ -50,7 +50,7 @@ struct MoeSorted {
 int moe_sort_slots(int n_pairs, int n_expert);         // slot capacity for any routing
 int moe_sort_max_tiles(int n_pairs, int n_expert);
 int moe_sort(const int32_t *ids, int n_pairs, int n_expert, const MoeSorted &out, hipStream_t stream);
-// x[t] += sum_s weights[t][s] * y[slot_of_pair[t*top_k + s]]
-int moe_combine_slots(float *x, const float *y, const float *w, const int32_t *slot_of_pair, int T, int n_embd, int top_k, hipStream_t stream);
+// out[t] = x[t] + sum_s weights[t][s] * y[slot_of_pair[t*top_k + s]]; out may be x
+int moe_combine_slots(const float *x, float *out, const float *y, const float *w, const int32_t *slot_of_pair, int T, int n_embd, int top_k, hipStream_t stream);
 
 }  // namespace mesh

@@ -47,15 +47,19 @@ __device__ __forceinline__ float row_sum(float v, float *scratch) {
 // Grid (tokens, groups of ROW_THREADS pairs): a thread takes the sine and the cosine of one frequency, so that a wave walks the
 // range reduction of an angle once and a single token's row is not one workgroup's serial work.  One row of 2048: 10.3 -> 4.4 us,
 // 900 rows: 13.4 -> 9.1.
-__global__ __launch_bounds__(ROW_THREADS) void embed_rows_kernel(const uint16_t *table, int ldt, const int32_t *tok, const int32_t *pos, const float *freq, float scale,
-                                                                 int n, float *x) {
+// ONE: a call of a single token, whose position, sequence and id come as arguments and are left where the launches behind read them
+// (a launch of its own for that: 4 us of a step's 190).
+template <bool ONE>
+__global__ __launch_bounds__(ROW_THREADS) void embed_rows_kernel(const uint16_t *table, int ldt, int32_t *tok, int32_t *pos, const float *freq, float scale,
+                                                                 int n, float *x, const EmbedToken one) {
     const int t = blockIdx.x, pair = blockIdx.y * ROW_THREADS + threadIdx.x, i = 2 * pair;
+    if (ONE && pair == 0) { pos[0] = one.pos; one.d_seq[0] = one.seq; tok[0] = one.id; }
     if (i >= n) return;
     const bool both = i + 1 < n;
-    const uint16_t *e = table + (size_t)tok[t] * ldt + i;
+    const uint16_t *e = table + (size_t)(ONE ? one.id : tok[t]) * ldt + i;
     float v0 = bf16_bits_to_f32(e[0]) * scale, v1 = both ? bf16_bits_to_f32(e[1]) * scale : 0.f;
     if (freq) {
-        const float angle = (float)pos[t] * freq[pair];
+        const float angle = (float)(ONE ? one.pos : pos[t]) * freq[pair];
         v0 += sinf(angle);
         v1 += cosf(angle);
     }
@@ -331,9 +335,11 @@ __global__ __launch_bounds__(ROW_THREADS) void qk_norm_append_kernel(const QkApp
         MESH_LAUNCH_CHECK();                                                                               \
     } while (0)
 
-int embed_rows(const uint16_t *table, int ldt, const int32_t *tok, const int32_t *pos, const float *freq, float scale, int T, int n, float *x, hipStream_t stream) {
+int embed_rows(const uint16_t *table, int ldt, int32_t *tok, int32_t *pos, const float *freq, float scale, int T, int n, float *x, const EmbedToken *one, hipStream_t stream) {
     if (T <= 0) return MESH_OK;
-    MESH_LAUNCH(embed_rows_kernel, dim3((unsigned)T, (unsigned)((n + 2 * ROW_THREADS - 1) / (2 * ROW_THREADS))), dim3(ROW_THREADS), 0, stream, table, ldt, tok, pos, freq, scale, n, x);
+    const dim3 grid((unsigned)T, (unsigned)((n + 2 * ROW_THREADS - 1) / (2 * ROW_THREADS))), block(ROW_THREADS);
+    if (one && T == 1) MESH_LAUNCH(embed_rows_kernel<true>, grid, block, 0, stream, table, ldt, tok, pos, freq, scale, n, x, *one);
+    else MESH_LAUNCH(embed_rows_kernel<false>, grid, block, 0, stream, table, ldt, tok, pos, freq, scale, n, x, EmbedToken{});
     MESH_LAUNCH_CHECK();
     return MESH_OK;
 }

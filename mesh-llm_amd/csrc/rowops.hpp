@@ -14,9 +14,14 @@ struct RowNorm {
     const float *gain = nullptr, *bias = nullptr;
 };
 
+// A single token by value, and where its sequence id goes.
+struct EmbedToken {
+    int32_t id = 0, pos = 0, seq = 0;
+    int32_t *d_seq = nullptr;
+};
 // x[t] = table[tok[t]] * scale, table rows of ldt, plus (freq set) the position vector of pos[t]: entries 2i and 2i + 1 are
-// sin and cos of pos * freq[i]
-int embed_rows(const uint16_t *table, int ldt, const int32_t *tok, const int32_t *pos, const float *freq, float scale, int T, int n, float *x, hipStream_t stream);
+// sin and cos of pos * freq[i].  one (T == 1): tok, pos and one->d_seq are written from it instead of read.
+int embed_rows(const uint16_t *table, int ldt, int32_t *tok, int32_t *pos, const float *freq, float scale, int T, int n, float *x, const EmbedToken *one, hipStream_t stream);
 
 // x[t] += post(y[t]) (y null: x as it is), and act[t] = pre(x[t]): post RMS with pre NONE, or both LAYER; y as the sum of
 // `slices` partial products (linear_sliced)

@@ -667,6 +667,12 @@ static GemmArgs gemm_of(const DevTensor &w, const uint16_t *x16, int ldx, int T,
     return g;
 }
 
+// Where a layer's hidden state comes from and goes to: the caller's own f32 buffers at the ends of a call that has them
+// (decode_core), the session's in between.  The attention block reads the input alone, the last launch of a layer writes the
+// output, so the caller's two may overlap.
+static const float *layer_input(const mesh_session *s, size_t il) { return il == 0 && s->x_in ? s->x_in : s->x; }
+static float *layer_output(const mesh_session *s, size_t il) { return il + 1 == s->stage->layers.size() && s->x_out ? s->x_out : s->x; }
+
 // One layer over many tokens: norms and activations are materialised in f16 and every projection is an MFMA GEMM.
 // One dense K-quant layer over f16 activations on the matrix cores: `skinny` selects the batched-decode GEMM (few
 // tokens, weight-streaming bound) instead of the large-tile prefill GEMM.
@@ -676,6 +682,8 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
     const HParams &hp = st->hp;
     hipStream_t stream = s->stream;
     const int E = (int)hp.n_embd, QD = (int)(hp.n_head * hp.head_dim), KD = (int)(hp.n_head_kv * hp.head_dim), FF = (int)hp.n_ff;
+    const float *x_in = layer_input(s, il);
+    float *x_out = layer_output(s, il);
     _Float16 *xn = reinterpret_cast<_Float16 *>(s->xn16), *f16ffn = reinterpret_cast<_Float16 *>(s->ffn16);
     int rc;
     bool rope_fused = false, attn_is_k8 = false, ffn_norm_fused = false;
@@ -712,9 +720,9 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
         ProfScope ps(s, MESH_PROF_PREP);
         if (norm_ready || (!sk8 && s->xn_layer == (int)il)) rc = MESH_OK;    // the previous layer's down projection has left them in norm16
         else if (sk8 && s->xq_layer == (int)il) rc = MESH_OK;     // the previous layer's combine step has left them in s->xq
-        else if (sk8) rc = quant16_k8(s->x, static_cast<const float *>(L.attn_norm.data), hp.rms_eps, T, E, s->xq, stream);
-        else if (k8) rc = rmsnorm_f16_k8(s->x, static_cast<const float *>(L.attn_norm.data), hp.rms_eps, T, E, xn, stream, s->f16_sat);
-        else rc = rmsnorm_f16(s->x, static_cast<const float *>(L.attn_norm.data), hp.rms_eps, T, E, xn, E, stream, s->f16_sat);
+        else if (sk8) rc = quant16_k8(x_in, static_cast<const float *>(L.attn_norm.data), hp.rms_eps, T, E, s->xq, stream);
+        else if (k8) rc = rmsnorm_f16_k8(x_in, static_cast<const float *>(L.attn_norm.data), hp.rms_eps, T, E, xn, stream, s->f16_sat);
+        else rc = rmsnorm_f16(x_in, static_cast<const float *>(L.attn_norm.data), hp.rms_eps, T, E, xn, E, stream, s->f16_sat);
     }
     if (rc != MESH_OK) return rc;
     if (sk16) {
@@ -847,7 +855,7 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
         oa.n_mat = 1;
         oa.mat[0] = mat_of(L.wo, s->x, E, nullptr);
         oa.x = xn; oa.K = QD; oa.T = T;
-        oa.residual = s->x; oa.ldres = E; oa.epi = EPI_RESIDUAL;
+        oa.residual = x_in; oa.ldres = E; oa.epi = EPI_RESIDUAL;
         oa.sat = s->f16_sat;
         ffn_norm_fused = nf && !attn_only && gemm_skinny_f16_workgroups(oa) >= 1 && gemm_skinny_f16_workgroups(oa) <= SKINNY_F16_NORM_PARTS_MAX;
         if (ffn_norm_fused) {
@@ -861,13 +869,13 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
         oa.n_mat = 1;
         oa.mat[0] = mat_of(L.wo, s->x, E, nullptr);
         oa.xq = s->xq; oa.K = QD; oa.T = T;
-        oa.residual = s->x; oa.ldres = E; oa.epi = EPI_RESIDUAL;
+        oa.residual = x_in; oa.ldres = E; oa.epi = EPI_RESIDUAL;
         ProfScope ps(s, MESH_PROF_GEMV);
         if ((rc = gemm_skinny(oa, stream)) != MESH_OK) return rc;
     } else {
         ProfScope ps(s, MESH_PROF_GEMV);
         GemmArgs go = gemm_k8(gemm_of(L.wo, s->xn16, QD, T, s->x, E, nullptr));
-        go.residual = s->x; go.ldres = E;
+        go.residual = x_in; go.ldres = E;
         ffn_norm_rode = !attn_only && norm_rides(go, L.ffn_norm);
         if ((rc = gemm_kquant(go, stream)) != MESH_OK) return rc;
     }
@@ -895,7 +903,7 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
         }
         SkinnyF16Args da;
         da.n_mat = 1;
-        da.mat[0] = mat_of(L.w_down, s->x, E, nullptr);
+        da.mat[0] = mat_of(L.w_down, x_out, E, nullptr);
         da.x = f16ffn; da.K = FF; da.T = T;
         da.residual = s->x; da.ldres = E; da.epi = EPI_RESIDUAL;
         da.sat = s->f16_sat;
@@ -937,7 +945,7 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
         ga.xq = s->xq; ga.K = E; ga.T = T; ga.epi = EPI_SWIGLU;
         SkinnyArgs da;
         da.n_mat = 1;
-        da.mat[0] = mat_of(L.w_down, s->x, E, nullptr);
+        da.mat[0] = mat_of(L.w_down, x_out, E, nullptr);
         da.xq = s->xq; da.K = FF; da.T = T;
         da.residual = s->x; da.ldres = E; da.epi = EPI_RESIDUAL;
         { ProfScope ps(s, MESH_PROF_GEMV); rc = gemm_skinny(ga, stream); }
@@ -971,7 +979,7 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
     }
     {
         ProfScope ps(s, MESH_PROF_GEMV);
-        GemmArgs gd = gemm_k8(gemm_of(L.w_down, s->ffn16, FF, T, s->x, E, nullptr));
+        GemmArgs gd = gemm_k8(gemm_of(L.w_down, s->ffn16, FF, T, x_out, E, nullptr));
         gd.residual = s->x; gd.ldres = E;
         // (the next layer takes this path at this token count if its matrices allow it, see run_layers)
         const LayerWeights *Ln = il + 1 < st->layers.size() ? &st->layers[il + 1] : nullptr;
@@ -1006,7 +1014,7 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
             if (r == MESH_OK) s->xq_layer = (int)il + 1;
             return r;
         }
-        return moe_combine(s->x, s->moe_out, s->moe_w, T, E, top_k, stream);
+        return moe_combine(s->x, layer_output(s, il), s->moe_out, s->moe_w, T, E, top_k, stream);
     };
     for (size_t il = 0; il < st->layers.size(); ++il) {
         const LayerWeights &L = st->layers[il];
@@ -1035,7 +1043,7 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
         qa.mat[0] = mat_of(L.wq, s->q, QD, &L.bq);
         qa.mat[1] = mat_of(L.wk, s->k, KD, &L.bk);
         qa.mat[2] = mat_of(L.wv, s->v, KD, &L.bv);
-        qa.x = s->x; qa.ldx = E; qa.K = E; qa.T = T;
+        qa.x = layer_input(s, il); qa.ldx = E; qa.K = E; qa.T = T;
         qa.norm_w = static_cast<const float *>(L.attn_norm.data); qa.eps = hp.rms_eps;
         // neighbouring-pair RoPE into an f16 cache without per-head norms: rotation and KV append ride in the
         // projection's epilogue (the same arithmetic as rope_kv_kernel), one launch fewer per layer
@@ -1086,7 +1094,7 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
         oa.n_mat = 1;
         oa.mat[0] = mat_of(L.wo, s->x, E, nullptr);
         oa.x = s->attn; oa.ldx = QD; oa.K = QD; oa.T = T;
-        oa.residual = s->x; oa.ldres = E; oa.epi = EPI_RESIDUAL;
+        oa.residual = layer_input(s, il); oa.ldres = E; oa.epi = EPI_RESIDUAL;
         { ProfScope ps(s, MESH_PROF_GEMV); rc = gemv(oa, stream); }
         if (rc != MESH_OK) return rc;
         }
@@ -1149,7 +1157,7 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
                 d.tiles = s->moe_sorted.tiles; d.n_tiles = s->moe_sorted.counts; d.max_tiles = max_tiles; d.expert_stride = L.exps_down_stride;
                 { ProfScope ps(s, MESH_PROF_GEMV); rc = gemm_kquant(d, stream); }
                 if (rc != MESH_OK) return rc;
-                if ((rc = moe_combine_slots(s->x, s->moe_out_slots, s->moe_w, s->moe_sorted.slot_of_pair, T, E, k, stream)) != MESH_OK) return rc;
+                if ((rc = moe_combine_slots(s->x, layer_output(s, il), s->moe_out_slots, s->moe_w, s->moe_sorted.slot_of_pair, T, E, k, stream)) != MESH_OK) return rc;
                 continue;
             }
             const int item_pairs = mfma ? SKINNY_ITEM_PAIRS : MOE_ITEM_PAIRS;
@@ -1238,7 +1246,7 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
         // x += Wdown . ffn
         GemvArgs da;
         da.n_mat = 1;
-        da.mat[0] = mat_of(L.w_down, s->x, E, nullptr);
+        da.mat[0] = mat_of(L.w_down, layer_output(s, il), E, nullptr);
         da.x = s->ffn; da.ldx = (int)hp.n_ff; da.K = (int)hp.n_ff; da.T = T;
         da.residual = s->x; da.ldres = E; da.epi = EPI_RESIDUAL;
         // a single token: the gate / up launch leaves the FFN vector in the fixed-point form the down projection's
@@ -1322,6 +1330,26 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const float *x, const 
     for (int i = threadIdx.x; i < n; i += 256) out[(size_t)blockIdx.x * n + i] = src[i];
 }
 
+// Positions, sequence ids and token ids of a small call travel as kernel arguments: no copy from host memory (a launch of the
+// runtime's own, with fences around it), no slot of the ring in use.
+constexpr int META_ARG_TOKENS = 32;
+struct CallMeta { int32_t pos[META_ARG_TOKENS], seq[META_ARG_TOKENS], tok[META_ARG_TOKENS]; };
+__global__ __launch_bounds__(64) void call_meta_kernel(const CallMeta m, int T, int B, int32_t *d_pos) {
+    const int i = threadIdx.x;
+    if (i >= T) return;
+    d_pos[i] = m.pos[i];
+    d_pos[B + i] = m.seq[i];
+    d_pos[2 * B + i] = m.tok[i];
+}
+
+// Memory of this device that a kernel can read or write as float4 rows.  (What a copy accepts is more: any host memory, any alignment.)
+static bool row_memory(const mesh_stage *st, const void *p) {
+    if (reinterpret_cast<uintptr_t>(p) & 15u) return false;
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) { (void)hipGetLastError(); return false; }
+    return a.type == hipMemoryTypeDevice && a.device == st->device;
+}
+
 // ids: the call's token ids in host memory, or null
 static int decode_core(mesh_session *s, const mesh_batch *b, const int32_t *ids, const void *d_in, int in_fmt, void *d_out, int out_fmt,
                        size_t out_cap, size_t *out_len) {
@@ -1366,36 +1394,56 @@ static int decode_core(mesh_session *s, const mesh_batch *b, const int32_t *ids,
     s->chunk_seq = b->seq_id ? b->seq_id[0] : 0;
     for (int i = 1; i < T && s->chunk_pos0 >= 0; ++i)
         if (b->pos[i] != b->pos[0] + i || (b->seq_id ? b->seq_id[i] : 0) != s->chunk_seq) s->chunk_pos0 = -1;
-    // positions / sequence ids -> device, through a ring of pinned slots so calls may be queued back to back
+    // positions, sequence ids, token ids -> device
     const size_t B = (size_t)st->n_batch_max;
-    if (s->meta_counter && s->meta_counter % META_SLOTS == 0) MESH_HIP_TRY(hipStreamSynchronize(stream));   // ring wraps: older copies are done
-    int32_t *slot = s->h_meta + (size_t)(s->meta_counter++ % META_SLOTS) * META_INTS(B);
-    for (int i = 0; i < T; ++i) { slot[i] = b->pos[i]; slot[B + i] = b->seq_id ? b->seq_id[i] : 0; }
-    size_t meta_ints = B + (size_t)T;
-    if (st->hybrid) {
-        if (ids) {
-            for (int i = 0; i < T; ++i) slot[2 * B + i] = ids[i];
-            meta_ints = 2 * B + (size_t)T;
+    EmbedToken one;
+    const bool embeds_one = st->hybrid && tokens_in && T == 1;
+    if (T <= META_ARG_TOKENS && !(picked && n_rows < T && n_rows > 0) && !(st->hybrid && T > 1)) {
+        if (st->hybrid) (void)hybrid_chunk_table(s, b, nullptr, s->d_pos + 4 * B);
+        if (embeds_one) {
+            one.id = ids[0]; one.pos = b->pos[0]; one.seq = b->seq_id ? b->seq_id[0] : 0; one.d_seq = s->d_seq;
+        } else {
+            CallMeta m;
+            for (int i = 0; i < META_ARG_TOKENS; ++i) {
+                m.pos[i] = i < T ? b->pos[i] : 0;
+                m.seq[i] = i < T && b->seq_id ? b->seq_id[i] : 0;
+                m.tok[i] = i < T && ids ? ids[i] : 0;
+            }
+            ProfScope ps(s, MESH_PROF_CODEC);
+            MESH_LAUNCH(call_meta_kernel, dim3(1), dim3(64), 0, stream, m, T, (int)B, s->d_pos);
+            MESH_LAUNCH_CHECK();
         }
+    } else {
+        // through a ring of pinned slots so calls may be queued back to back
+        if (s->meta_counter && s->meta_counter % META_SLOTS == 0) MESH_HIP_TRY(hipStreamSynchronize(stream));   // ring wraps: older copies are done
+        int32_t *slot = s->h_meta + (size_t)(s->meta_counter++ % META_SLOTS) * META_INTS(B);
+        for (int i = 0; i < T; ++i) { slot[i] = b->pos[i]; slot[B + i] = b->seq_id ? b->seq_id[i] : 0; }
+        size_t meta_ints = B + (size_t)T;
+        if (st->hybrid) {
+            if (ids) {
+                for (int i = 0; i < T; ++i) slot[2 * B + i] = ids[i];
+                meta_ints = 2 * B + (size_t)T;
+            }
+        }
+        if (picked && n_rows < T && n_rows > 0) {
+            for (int i = 0, r = 0; i < T; ++i)
+                if (b->want[i]) slot[3 * B + (size_t)r++] = i;
+            meta_ints = 3 * B + (size_t)n_rows;
+        }
+        if (st->hybrid) {
+            const size_t n = hybrid_chunk_table(s, b, slot + 4 * B, s->d_pos + 4 * B);
+            if (n) meta_ints = 4 * B + n;
+        }
+        // (one copy for all: the slot and the device buffer have the same layout, positions at 0, sequence ids at B, token ids and
+        // wanted rows behind them; a copy is a launch of its own on the stream, and the entries past each list are never read)
+        MESH_HIP_TRY(hipMemcpyAsync(s->d_pos, slot, meta_ints * sizeof(int32_t), hipMemcpyHostToDevice, stream));
     }
-    if (picked && n_rows < T && n_rows > 0) {
-        for (int i = 0, r = 0; i < T; ++i)
-            if (b->want[i]) slot[3 * B + (size_t)r++] = i;
-        meta_ints = 3 * B + (size_t)n_rows;
-    }
-    if (st->hybrid) {
-        const size_t n = hybrid_chunk_table(s, b, slot + 4 * B, s->d_pos + 4 * B);
-        if (n) meta_ints = 4 * B + n;
-    }
-    // (one copy for all: the slot and the device buffer have the same layout, positions at 0, sequence ids at B, token ids and
-    // wanted rows behind them; a copy is a launch of its own on the stream, and the entries past each list are never read)
-    MESH_HIP_TRY(hipMemcpyAsync(s->d_pos, slot, meta_ints * sizeof(int32_t), hipMemcpyHostToDevice, stream));
 
     if (st->hybrid) {
         // (a call that fails from here on leaves its sequences in a state nothing is known of; they have to start anew)
         hybrid_note_batch(s, b, false);
         float *x = nullptr;
-        if (tokens_in) rc = hybrid_embed(s, T);
+        if (tokens_in) rc = hybrid_embed(s, T, embeds_one ? &one : nullptr);
         else { ProfScope ps(s, MESH_PROF_CODEC); rc = act_unpack_dev(in_fmt, d_in, s->x, (int64_t)T * hp.n_embd, stream); }
         if (rc != MESH_OK || (rc = run_layers_graphed(s, T, max_keys)) != MESH_OK) return rc;
         if (logits_out) {
@@ -1412,9 +1460,15 @@ static int decode_core(mesh_session *s, const mesh_batch *b, const int32_t *ids,
         // embedding rows: one dequantize per token (ids are read on the host side by the caller's contract)
         return fail(MESH_ERR_UNSUPPORTED, "mesh_stage_decode_dev: token input is only available through the host-pointer entry point");
     }
-    { ProfScope ps(s, MESH_PROF_CODEC); rc = act_unpack_dev(in_fmt, d_in, s->x, (int64_t)T * hp.n_embd, stream); }
-    if (rc != MESH_OK) return rc;
-    if ((rc = run_layers_graphed(s, T, max_keys)) != MESH_OK) return rc;
+    // f32 rows in memory a kernel reaches are read and written where they lie (a graph would hold on to their addresses)
+    const bool eager = !s->tune.graphs;
+    s->x_in = eager && in_fmt == MESH_F32 && hp.n_embd % 4 == 0 && row_memory(st, d_in) ? static_cast<const float *>(d_in) : nullptr;
+    s->x_out = eager && out_fmt == MESH_F32 && hp.n_embd % 4 == 0 && row_memory(st, d_out) ? static_cast<float *>(d_out) : nullptr;
+    if (!s->x_in) {
+        ProfScope ps(s, MESH_PROF_CODEC);
+        if ((rc = act_unpack_dev(in_fmt, d_in, s->x, (int64_t)T * hp.n_embd, stream)) != MESH_OK) return rc;
+    }
+    if ((rc = run_layers_graphed(s, T, max_keys)) != MESH_OK || s->x_out) return rc;
     if (logits_out) {
         if (n_rows == 0) return MESH_OK;
         const float *rows = s->x;
@@ -1482,13 +1536,15 @@ int stage_decode(mesh_session *s, const mesh_batch *b, const void *in, int in_fm
         MESH_HIP_TRY(hipMemcpyAsync(d_in, s->h_io, in_bytes, hipMemcpyHostToDevice, stream));
     }
     size_t len = 0;
+    uint8_t *h_out = static_cast<uint8_t *>(s->h_io) + s->io_stage_bytes;
+    const bool direct = out_fmt == MESH_LOGITS && wanted == 1;
+    if (direct) d_out = h_out;
     if ((rc = decode_core(s, b, token_ids, d_in, eff_in_fmt, d_out, out_fmt, std::min(out_cap, s->io_out_bytes), &len)) != MESH_OK) {
         if (out_len) *out_len = len;
         return rc;
     }
     if (out_len) *out_len = len;
-    uint8_t *h_out = static_cast<uint8_t *>(s->h_io) + s->io_stage_bytes;
-    if (len) MESH_HIP_TRY(hipMemcpyAsync(h_out, d_out, len, hipMemcpyDeviceToHost, stream));
+    if (len && !direct) MESH_HIP_TRY(hipMemcpyAsync(h_out, d_out, len, hipMemcpyDeviceToHost, stream));
     MESH_HIP_TRY(hipStreamSynchronize(stream));
     memcpy(out, h_out, len);
     return MESH_OK;

@@ -152,6 +152,9 @@ struct mesh_session {
     size_t io_out_bytes = 0;
     void *h_io = nullptr;           // pinned host staging, same split
     int attn_splits_max = 0;
+    // set per call: the caller's f32 buffers the first layer reads and the last one writes in place of x (null: x itself)
+    const float *x_in = nullptr;
+    float *x_out = nullptr;
     // set per call: the batch is one run of consecutive positions of one sequence (first position, sequence), else -1
     int chunk_pos0 = -1, chunk_seq = -1;
     std::vector<void *> allocations;
