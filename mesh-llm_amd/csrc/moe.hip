@@ -7,6 +7,7 @@
 #include <algorithm>
 
 #include "moe.hpp"
+#include "expert_step.hpp"
 #include "gemv.hpp"
 
 namespace mesh {
@@ -136,11 +137,26 @@ constexpr int ROUTER_THREADS = 1024, ROUTER_WAVES = ROUTER_THREADS / 64;
 // (RT: threads of the workgroup.  A decode batch has few tokens and wants every wave it can get on a token's expert rows;
 // a prefill chunk has a workgroup per token anyway, and small workgroups, eight to a CU, hide each other's row loads.)
 constexpr int ROUTER_THREADS_WIDE = 256, ROUTER_WIDE_MIN_TOKENS = 512;
-// the logits of this workgroup's token and expert slice (blockIdx.y of gridDim.y), into s_logits and logits_out
+// four neighbouring elements of a token's row as pairs of f16 (expert_step.hpp, by token)
+__device__ __forceinline__ void store_planes(_Float16 *planes, int E, int t, int k, const float4 &v, unsigned *sat) {
+    const float x[4] = {v.x, v.y, v.z, v.w};
+    _Float16 hi[4], lo[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float c = __builtin_amdgcn_fmed3f(x[i], -65504.f, 65504.f);
+        hi[i] = (_Float16)c;
+        lo[i] = (_Float16)((c - (float)hi[i]) * EXPERT_LO);
+    }
+    note_f16_clamp(sat, x[0], x[1], x[2], x[3]);
+    _Float16 *to = planes + (size_t)(t >> 4) * 32 * E + ((size_t)(k >> 3) * 32 + (t & 15)) * 8 + (k & 7);
+    *reinterpret_cast<uint2 *>(to) = __builtin_bit_cast(uint2, hi);
+    *reinterpret_cast<uint2 *>(to + 128) = __builtin_bit_cast(uint2, lo);
+}
+// the logits of this workgroup's token and expert slice (blockIdx.y of gridDim.y), into s_logits and logits_out; the normalised row into planes
 template <int NV, int RT>      // float4 groups per lane = E / 256
 __device__ __forceinline__ void router_logits(const float *__restrict__ x, const float *__restrict__ norm_w, const float *__restrict__ W,
                                               float *__restrict__ logits_out, int ldx, float eps, int p_n_expert, float *s_logits,
-                                              float *__restrict__ scale_out = nullptr) {
+                                              float *__restrict__ scale_out = nullptr, _Float16 *__restrict__ planes = nullptr, unsigned *sat = nullptr) {
     constexpr int E = NV * 256, ROUTER_WAVES = RT / 64;
     const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     // element index of a lane's values: 4 * (lane + 64 * i) + c
@@ -161,6 +177,12 @@ __device__ __forceinline__ void router_logits(const float *__restrict__ x, const
         const float4 w = *reinterpret_cast<const float4 *>(norm_w + 4 * (lane + 64 * i));
         xr[i].x = xr[i].x * scale * w.x; xr[i].y = xr[i].y * scale * w.y;
         xr[i].z = xr[i].z * scale * w.z; xr[i].w = xr[i].w * scale * w.w;
+    }
+    // (each of the first workgroup's waves writes its share of the row)
+    if (planes && blockIdx.y == 0) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+            if (i % ROUTER_WAVES == wave) store_planes(planes, E, t, 4 * (lane + 64 * i), xr[i], sat);
     }
     // two expert rows per step, all of their loads in flight together
     const int per = (p_n_expert + (int)gridDim.y - 1) / (int)gridDim.y;
@@ -198,9 +220,10 @@ template <int NV, int RT = ROUTER_THREADS>
 // (scalar arguments first: preloaded into SGPRs, see gemv.hip)
 __global__ __launch_bounds__(RT) void moe_router_fused_kernel(const float *__restrict__ x, const float *__restrict__ norm_w,
                                                                           const float *__restrict__ W, float *__restrict__ logits_out,
-                                                                          int ldx, float eps, int p_n_expert, const MoeRouteArgs a, float *__restrict__ scale_out) {
+                                                                          int ldx, float eps, int p_n_expert, const MoeRouteArgs a, float *__restrict__ scale_out,
+                                                                          _Float16 *planes, unsigned *sat) {
     __shared__ float s_logits[64 * ROUTE_MAX_PER_LANE];
-    router_logits<NV, RT>(x, norm_w, W, logits_out, ldx, eps, p_n_expert, s_logits, scale_out);
+    router_logits<NV, RT>(x, norm_w, W, logits_out, ldx, eps, p_n_expert, s_logits, scale_out, planes, sat);
     if (gridDim.y > 1) return;
     __syncthreads();
     if ((threadIdx.x >> 6) == 0) route_wave_any(s_logits, a, blockIdx.x, threadIdx.x & 63);
@@ -294,10 +317,10 @@ int moe_router_fused(const MoeRouteArgs &a, const float *x, int ldx, const float
     if (T >= ROUTER_WIDE_MIN_TOKENS) {
         const dim3 block(ROUTER_THREADS_WIDE);
         switch (E / 256) {
-            case 2: MESH_LAUNCH((moe_router_fused_kernel<2, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
-            case 4: MESH_LAUNCH((moe_router_fused_kernel<4, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
-            case 8: MESH_LAUNCH((moe_router_fused_kernel<8, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
-            case 16: MESH_LAUNCH((moe_router_fused_kernel<16, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
+            case 2: MESH_LAUNCH((moe_router_fused_kernel<2, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out, nullptr, nullptr); break;
+            case 4: MESH_LAUNCH((moe_router_fused_kernel<4, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out, nullptr, nullptr); break;
+            case 8: MESH_LAUNCH((moe_router_fused_kernel<8, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out, nullptr, nullptr); break;
+            case 16: MESH_LAUNCH((moe_router_fused_kernel<16, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out, nullptr, nullptr); break;
             default: return fail(MESH_ERR_UNSUPPORTED, "moe: fused router for hidden size %d", E);
         }
         MESH_LAUNCH_CHECK();
@@ -305,10 +328,10 @@ int moe_router_fused(const MoeRouteArgs &a, const float *x, int ldx, const float
     }
     const dim3 block(ROUTER_THREADS);
     switch (E / 256) {
-        case 2: MESH_LAUNCH(moe_router_fused_kernel<2>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
-        case 4: MESH_LAUNCH(moe_router_fused_kernel<4>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
-        case 8: MESH_LAUNCH(moe_router_fused_kernel<8>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
-        case 16: MESH_LAUNCH(moe_router_fused_kernel<16>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
+        case 2: MESH_LAUNCH(moe_router_fused_kernel<2>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out, nullptr, nullptr); break;
+        case 4: MESH_LAUNCH(moe_router_fused_kernel<4>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out, nullptr, nullptr); break;
+        case 8: MESH_LAUNCH(moe_router_fused_kernel<8>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out, nullptr, nullptr); break;
+        case 16: MESH_LAUNCH(moe_router_fused_kernel<16>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out, nullptr, nullptr); break;
         default: return fail(MESH_ERR_UNSUPPORTED, "moe: fused router for hidden size %d", E);
     }
     MESH_LAUNCH_CHECK();
@@ -422,12 +445,12 @@ template <int NV>
 __global__ __launch_bounds__(GROUP_THREADS) void moe_router_group_fused_kernel(const float *__restrict__ x, const float *__restrict__ norm_w,
                                                                                const float *__restrict__ W, float *logits, int ldx, float eps,
                                                                                int p_n_expert, const MoeRouteArgs a, int T, int32_t *items, int32_t *n_items,
-                                                                               int ipairs, int *arrive) {
+                                                                               int ipairs, int *arrive, _Float16 *planes, unsigned *sat) {
     static_assert(GROUP_THREADS == ROUTER_THREADS, "the routing tail runs in a router workgroup");
     extern __shared__ int32_t g_lds[];
     __shared__ float s_logits[64 * ROUTE_MAX_PER_LANE];
     __shared__ int s_last;
-    router_logits<NV, ROUTER_THREADS>(x, norm_w, W, logits, ldx, eps, p_n_expert, s_logits);
+    router_logits<NV, ROUTER_THREADS>(x, norm_w, W, logits, ldx, eps, p_n_expert, s_logits, nullptr, planes, sat);
     // One release per workgroup, by one thread: the barrier orders the other waves' logits stores before it, and a
     // release at device scope covers what the releasing thread has observed.  (A __threadfence() in every wave measured
     // 35 us for this tail: sixteen cache write-backs and invalidations per workgroup.)
@@ -456,7 +479,7 @@ __global__ __launch_bounds__(GROUP_THREADS) void moe_router_group_fused_kernel(c
 }
 
 int moe_router_group(const MoeRouteArgs &a, const float *x, int ldx, const float *norm_w, float eps, const float *W, int E,
-                     float *logits, int T, int32_t *items, int32_t *n_items, int item_pairs, hipStream_t stream, int *arrive) {
+                     float *logits, int T, int32_t *items, int32_t *n_items, int item_pairs, hipStream_t stream, int *arrive, uint16_t *planes, unsigned *sat) {
     if (T <= 0) return MESH_OK;
     if (!moe_router_group_supported(E, a.n_expert, a.top_k, T) || !logits)
         return fail(MESH_ERR_UNSUPPORTED, "moe: split router for hidden size %d / %d experts / %d tokens", E, a.n_expert, T);
@@ -469,20 +492,20 @@ int moe_router_group(const MoeRouteArgs &a, const float *x, int ldx, const float
         // LDS of the tail: the grouping's pair list and counters, then a logits row per wave
         const size_t smem = (size_t)GROUP_WAVES * 64 * ROUTE_MAX_PER_LANE * sizeof(float) + ((size_t)T * a.top_k + 2 * (size_t)a.n_expert) * sizeof(int32_t);
         switch (E / 256) {
-            case 2: MESH_LAUNCH(moe_router_group_fused_kernel<2>, grid, block, smem, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, T, items, n_items, item_pairs, arrive); break;
-            case 4: MESH_LAUNCH(moe_router_group_fused_kernel<4>, grid, block, smem, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, T, items, n_items, item_pairs, arrive); break;
-            case 8: MESH_LAUNCH(moe_router_group_fused_kernel<8>, grid, block, smem, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, T, items, n_items, item_pairs, arrive); break;
-            case 16: MESH_LAUNCH(moe_router_group_fused_kernel<16>, grid, block, smem, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, T, items, n_items, item_pairs, arrive); break;
+            case 2: MESH_LAUNCH(moe_router_group_fused_kernel<2>, grid, block, smem, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, T, items, n_items, item_pairs, arrive, reinterpret_cast<_Float16 *>(planes), sat); break;
+            case 4: MESH_LAUNCH(moe_router_group_fused_kernel<4>, grid, block, smem, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, T, items, n_items, item_pairs, arrive, reinterpret_cast<_Float16 *>(planes), sat); break;
+            case 8: MESH_LAUNCH(moe_router_group_fused_kernel<8>, grid, block, smem, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, T, items, n_items, item_pairs, arrive, reinterpret_cast<_Float16 *>(planes), sat); break;
+            case 16: MESH_LAUNCH(moe_router_group_fused_kernel<16>, grid, block, smem, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, T, items, n_items, item_pairs, arrive, reinterpret_cast<_Float16 *>(planes), sat); break;
             default: return fail(MESH_ERR_UNSUPPORTED, "moe: fused router for hidden size %d", E);
         }
         MESH_LAUNCH_CHECK();
         return MESH_OK;
     }
     switch (E / 256) {
-        case 2: MESH_LAUNCH(moe_router_fused_kernel<2>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, static_cast<float *>(nullptr)); break;
-        case 4: MESH_LAUNCH(moe_router_fused_kernel<4>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, static_cast<float *>(nullptr)); break;
-        case 8: MESH_LAUNCH(moe_router_fused_kernel<8>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, static_cast<float *>(nullptr)); break;
-        case 16: MESH_LAUNCH(moe_router_fused_kernel<16>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, static_cast<float *>(nullptr)); break;
+        case 2: MESH_LAUNCH(moe_router_fused_kernel<2>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, static_cast<float *>(nullptr), reinterpret_cast<_Float16 *>(planes), sat); break;
+        case 4: MESH_LAUNCH(moe_router_fused_kernel<4>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, static_cast<float *>(nullptr), reinterpret_cast<_Float16 *>(planes), sat); break;
+        case 8: MESH_LAUNCH(moe_router_fused_kernel<8>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, static_cast<float *>(nullptr), reinterpret_cast<_Float16 *>(planes), sat); break;
+        case 16: MESH_LAUNCH(moe_router_fused_kernel<16>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, static_cast<float *>(nullptr), reinterpret_cast<_Float16 *>(planes), sat); break;
         default: return fail(MESH_ERR_UNSUPPORTED, "moe: fused router for hidden size %d", E);
     }
     MESH_LAUNCH_CHECK();

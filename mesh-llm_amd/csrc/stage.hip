@@ -17,6 +17,7 @@
 #include <mutex>
 
 #include "attn.hpp"
+#include "expert_step.hpp"
 #include "gemm.hpp"
 #include "gemv.hpp"
 #include "moe.hpp"
@@ -504,9 +505,17 @@ static int kquant_session_alloc(mesh_session *s) {
             return rc;
         if ((rc = sess_alloc(s, &p, B * k * sizeof(int32_t))) != MESH_OK) return rc;
         s->moe_ids = static_cast<int32_t *>(p);
-        // work items: 4 pairs each for the mat-vec kernel, 16 for the matrix-core one; the buffer fits either
-        const size_t items = (size_t)std::max(moe_max_items((int)(B * k), (int)ne) * MOE_ITEM_INTS,
-                                              moe_max_items((int)(B * k), (int)ne, SKINNY_ITEM_PAIRS) * moe_item_ints(SKINNY_ITEM_PAIRS)) / MOE_ITEM_INTS + 1;
+        // work items: 4 pairs each for the mat-vec kernel, 16 and 8 for the matrix-core ones; the buffer fits any
+        const int step_items = moe_max_items((int)(std::min<size_t>(B, EXPERT_STEP_TOKENS_MAX) * k), (int)ne, EXPERT_STEP_PAIRS);
+        const size_t items = (size_t)std::max(std::max(moe_max_items((int)(B * k), (int)ne) * MOE_ITEM_INTS,
+                                                       moe_max_items((int)(B * k), (int)ne, SKINNY_ITEM_PAIRS) * moe_item_ints(SKINNY_ITEM_PAIRS)),
+                                              step_items * moe_item_ints(EXPERT_STEP_PAIRS)) / MOE_ITEM_INTS + 1;
+        if (hp.n_ff_exp > 0) {
+            if ((rc = sess_alloc(s, &p, expert_x_bytes((int)hp.n_embd))) != MESH_OK) return rc;
+            s->moe_step_x = static_cast<uint16_t *>(p);
+            if ((rc = sess_alloc(s, &p, expert_ffn_bytes(step_items, (int)hp.n_ff_exp))) != MESH_OK) return rc;
+            s->moe_step_ffn = static_cast<uint16_t *>(p);
+        }
         // (+ the item count, + the arrival counter of the router launch whose last workgroup routes and groups)
         if ((rc = sess_alloc(s, &p, (items * MOE_ITEM_INTS + 2) * sizeof(int32_t))) != MESH_OK) return rc;
         s->moe_items = static_cast<int32_t *>(p);
@@ -1160,14 +1169,18 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
                 if ((rc = moe_combine_slots(s->x, layer_output(s, il), s->moe_out_slots, s->moe_w, s->moe_sorted.slot_of_pair, T, E, k, stream)) != MESH_OK) return rc;
                 continue;
             }
-            const int item_pairs = mfma ? SKINNY_ITEM_PAIRS : MOE_ITEM_PAIRS;
+            // a batch of decode steps over K-quant experts: eight pairs of an expert per pass on the f16 matrix cores
+            const bool step = want_groups && s->moe_step_x && T >= s->tune.moe_step_min_tokens && T <= EXPERT_STEP_TOKENS_MAX && ffe % 8 == 0 &&
+                              L.gate_inp.type == MESH_F32 && moe_router_group_supported(E, ne, k, T) && L.up_exps.type == L.gate_exps.type &&
+                              expert_step_supported(L.gate_exps.type, ffe, E) && expert_step_supported(L.down_exps.type, E, ffe);
+            const int item_pairs = step ? EXPERT_STEP_PAIRS : mfma ? SKINNY_ITEM_PAIRS : MOE_ITEM_PAIRS;
             bool grouped_done = false;
             if (want_groups && L.gate_inp.type == MESH_F32 && moe_router_group_supported(E, ne, k, T)) {
                 // a batch of decode steps: logits over many workgroups, then routing and grouping in one launch
                 ProfScope ps(s, MESH_PROF_GEMV);
                 if ((rc = moe_router_group(mr, s->x, E, static_cast<const float *>(L.ffn_norm.data), hp.rms_eps,
                                            static_cast<const float *>(L.gate_inp.data), E, s->moe_logits, T, s->moe_items, s->moe_n_items,
-                                           item_pairs, stream, s->tune.moe_router_tail ? s->moe_arrive : nullptr)) != MESH_OK) return rc;
+                                           item_pairs, stream, s->tune.moe_router_tail ? s->moe_arrive : nullptr, step ? s->moe_step_x : nullptr, s->f16_sat)) != MESH_OK) return rc;
                 grouped_done = true;
             } else if (L.gate_inp.type == MESH_F32 && moe_router_fused_supported(E, ne, k)) {
                 // the router matrix is small and f32: logits and routing in one launch
@@ -1187,6 +1200,19 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
             // pairs of one expert share a pass over its weights
             const bool grouped = want_groups;
             if (grouped && !grouped_done && (rc = moe_group(s->moe_ids, T * k, ne, s->moe_items, s->moe_n_items, item_pairs, stream)) != MESH_OK) return rc;
+            if (step) {
+                ProfScope ps(s, MESH_PROF_GEMV);
+                ExpertStepArgs ea;
+                ea.W[0] = L.gate_exps.data; ea.W[1] = L.up_exps.data; ea.type = L.gate_exps.type; ea.M = ffe; ea.K = E;
+                ea.items = s->moe_items; ea.n_items = s->moe_n_items; ea.max_items = moe_max_items(T * k, ne, EXPERT_STEP_PAIRS); ea.x_div = k;
+                ea.x = s->moe_step_x; ea.ffn = s->moe_step_ffn; ea.sat = s->f16_sat;
+                if ((rc = expert_step(ea, stream)) != MESH_OK) return rc;
+                ea.W[0] = L.down_exps.data; ea.W[1] = nullptr; ea.type = L.down_exps.type; ea.M = E; ea.K = ffe;
+                ea.y = s->moe_out;
+                if ((rc = expert_step(ea, stream)) != MESH_OK) return rc;
+                if ((rc = combine(il, k)) != MESH_OK) return rc;
+                continue;
+            }
             if (mfma) {
                 const int max_items = moe_max_items(T * k, ne, SKINNY_ITEM_PAIRS);
                 { ProfScope ps(s, MESH_PROF_PREP); rc = quant16_k8(s->x, static_cast<const float *>(L.ffn_norm.data), hp.rms_eps, T, E, s->xq, stream); }

@@ -36,6 +36,7 @@ const TuningField *tuning_fields() {
         {"moe_router_tail", &Tuning::moe_router_tail, 0, 1, TUNE_SESSION},
         {"moe_fuse_quant", &Tuning::moe_fuse_quant, 0, 1, TUNE_SESSION},
         {"moe_gemm", &Tuning::moe_gemm, 0, 1, TUNE_SESSION},
+        {"moe_step_min_tokens", &Tuning::moe_step_min_tokens, 1, 1 << 20, TUNE_SESSION},
         {"moe_gemm_min_pairs", &Tuning::moe_gemm_min_pairs, 1, 1 << 20, TUNE_SESSION},
         {"reg_min_tokens", &Tuning::reg_min_tokens, 1, 1 << 20, TUNE_SESSION},
         {"reg_min_blocks", &Tuning::reg_min_blocks, 1, 1 << 20, TUNE_SESSION},
