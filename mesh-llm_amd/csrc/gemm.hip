@@ -17,6 +17,7 @@
 
 #include "gemm.hpp"
 #include "gemm_tile.hpp"
+#include "lds_ops.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -272,14 +273,9 @@ __device__ __forceinline__ void store_sub(const PackedSub<TYPE> &w, _Float16 *ds
 // (down projection of 4096 x 14336, q6_K, 2048 tokens on the 256-row tile: 270 -> 266 us).
 __device__ __forceinline__ int staged_slot(int s) { return (s & ~63) + 2 * ((s & 7) + ((s >> 4) & 3) * 8) + ((s >> 3) & 1); }
 
-// Workgroup barrier that orders LDS only.  __syncthreads() also waits for every outstanding global load, i.e. at the end
-// of each k-step for the activation fragments requested a moment ago for the NEXT step -- with one matrix-core wave per
-// SIMD nothing else would run during that wait.
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
+// (Barriers here are lds_barrier: __syncthreads() also waits for every outstanding global load, i.e. at the end of each k-step for the
+// activation fragments requested a moment ago for the NEXT step -- with one matrix-core wave per SIMD nothing else would run
+// during that wait.)
 
 // Role split: waves 0-3 only multiply (each a 64 x 64 corner of the tile out of LDS stage kc & 1), waves 4-7 only
 // stage (fetch the raw weight bytes and activations of step kc + 2, dequantise step kc + 1 into the other LDS

@@ -34,6 +34,7 @@
 
 #include "gemm.hpp"
 #include "gemv_device.hpp"
+#include "lds_ops.hpp"
 
 namespace mesh {
 
@@ -127,13 +128,6 @@ struct XFrags {
         }
     }
 };
-
-// The LDS unit executes a wave's accesses in order; the fences only keep the compiler from reordering them.
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // One tile: dense-mapped registers -> wave-private LDS slot (same arrangement as in memory) -> the view of lane (m, g):
 // row m's header and the quants of elements 32s + 8g .. + 7, s = 0..7, of that row.

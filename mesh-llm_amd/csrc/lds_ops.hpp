@@ -39,4 +39,18 @@ __device__ __forceinline__ lds_u2 lds_read_transposed(const _Float16 *p) {
 #endif
 }
 
+// Workgroup barrier that orders LDS only.  __syncthreads() also waits for every outstanding global load.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// The LDS unit executes a wave's accesses in order; the fences only keep the compiler from reordering them.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 }  // namespace mesh

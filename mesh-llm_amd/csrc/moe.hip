@@ -9,6 +9,8 @@
 #include "moe.hpp"
 #include "expert_step.hpp"
 #include "gemv.hpp"
+#include "lds_ops.hpp"
+#include "wave_ops.hpp"
 
 namespace mesh {
 
@@ -27,16 +29,14 @@ __device__ __forceinline__ void route_wave(const float *lg, const float *mask, i
         p[i] = e < n_expert ? lg[e] : -INFINITY;
         mx = fmaxf(mx, p[i]);
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    mx = wave_max(mx);
     float den = 0.f;
 #pragma unroll
     for (int i = 0; i < NPL; ++i) {
         p[i] = lane + 64 * i < n_expert ? expf(p[i] - mx) : 0.f;
         den += p[i];
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) den += __shfl_xor(den, o);
+    den = wave_sum(den);
 #pragma unroll
     for (int i = 0; i < NPL; ++i) {
         const int e = lane + 64 * i;
@@ -45,66 +45,31 @@ __device__ __forceinline__ void route_wave(const float *lg, const float *mask, i
     }
     float wsum = 0.f, my_w = 0.f;
     int my_id = 0;
-    if constexpr (NPL <= 2) {
-        // Up to 128 experts: every candidate counts the experts that come before it in the order (value descending, id
-        // ascending) -- one broadcast per expert, no dependent cross-lane chain -- and the candidate counting k is the
-        // k-th pick.  The same picks in the same order as the loop below (each round of which takes the first expert
-        // left in that order).
-        int rank[NPL];
-#pragma unroll
-        for (int i = 0; i < NPL; ++i) rank[i] = lane + 64 * i < n_expert ? 0 : 0x7FFFFFFF;
-#pragma unroll
-        for (int ii = 0; ii < NPL; ++ii) {
-            for (int j = 0; j < 64 && j + 64 * ii < n_expert; ++j) {
-                const float ov = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sel[ii]), j));
-                const int oe = j + 64 * ii;
-#pragma unroll
-                for (int i = 0; i < NPL; ++i) {
-                    const int e = lane + 64 * i;
-                    rank[i] += (ov > sel[i] || (ov == sel[i] && oe < e)) ? 1 : 0;
-                }
-            }
-        }
-        for (int k = 0; k < top_k; ++k) {
-            int bi = 0;
-            float bp = 0.f;
-#pragma unroll
-            for (int i = 0; i < NPL; ++i) {
-                const unsigned long long m = __builtin_amdgcn_ballot_w64(rank[i] == k);
-                if (m != 0ull) {
-                    const int src = __builtin_ctzll(m);
-                    bi = src + 64 * i;
-                    bp = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, p[i]), src));
-                }
-            }
-            if (lane == k) { my_id = bi; my_w = bp; }
-            wsum += bp;
-        }
-    } else {
-    unsigned taken = 0;        // bit i: expert lane + 64*i has been selected
+    // The best value left, then the first expert (ascending) that holds it and is not taken: a masked expert can still win once every allowed
+    // one is, as in the reference's top-k over probabilities plus mask.  (An earlier form had every candidate count those before it,
+    // one broadcast per expert: 64 of them cost more than top_k rounds whose maximum does not pass the LDS unit.)
+    unsigned taken = 0;        // bit i: expert lane + 64 i has been selected
     for (int k = 0; k < top_k; ++k) {
-        // best remaining (value, id) of this lane, then of the wave; ties go to the lower id
-        float bv = -INFINITY, bp = 0.f;
-        int bi = 0x7FFFFFFF;
+        float best = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < NPL; ++i) best = (taken >> i) & 1u ? best : fmaxf(best, sel[i]);
+        best = wave_max(best);
+        int bi = 0;
+        float bp = p[0];        // (no candidate: values that are no numbers)
+        bool found = false;
 #pragma unroll
         for (int i = 0; i < NPL; ++i) {
-            const int e = lane + 64 * i;
-            if (e < n_expert && !((taken >> i) & 1u) && (bi == 0x7FFFFFFF || sel[i] > bv || (sel[i] == bv && e < bi))) { bv = sel[i]; bi = e; bp = p[i]; }
+            const unsigned long long m = __builtin_amdgcn_ballot_w64(!((taken >> i) & 1u) && lane + 64 * i < n_expert && sel[i] == best);
+            if (!found && m != 0ull) {
+                found = true;
+                const int src = __builtin_ctzll(m);
+                bi = src + 64 * i;
+                bp = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, p[i]), src));
+                if (lane == src) taken |= 1u << i;
+            }
         }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            const float ov = __shfl_xor(bv, o), op = __shfl_xor(bp, o);
-            const int oi = __shfl_xor(bi, o);
-            if (oi != 0x7FFFFFFF && (bi == 0x7FFFFFFF || ov > bv || (ov == bv && oi < bi))) { bv = ov; bi = oi; bp = op; }
-        }
-        // retire the winner (a masked expert can still win once every allowed one is taken, as in the reference's
-        // top-k over probabilities plus mask)
-#pragma unroll
-        for (int i = 0; i < NPL; ++i)
-            if (lane + 64 * i == bi) taken |= 1u << i;
         if (lane == k) { my_id = bi; my_w = bp; }
         wsum += bp;
-    }
     }
     if (lane < top_k) {
         ids[lane] = my_id;
@@ -131,8 +96,6 @@ __global__ __launch_bounds__(64) void moe_route_kernel(MoeRouteArgs a) {
 // Router logits and routing in one launch, one workgroup per token: every wave holds the token's normalised hidden
 // state in registers (E / 64 values per lane) and takes every fourth expert row of the f32 router matrix; the
 // logits meet in LDS and the first wave routes.  logits[t] = W . (x[t] * rsqrt(mean(x^2) + eps) * norm_w).
-// With gridDim.y > 1 the experts are split over blockIdx.y and the kernel only writes logits_out (routing follows in
-// moe_route_group_kernel): small batches then have enough workgroups to pull the router matrix through quickly.
 constexpr int ROUTER_THREADS = 1024, ROUTER_WAVES = ROUTER_THREADS / 64;
 // (RT: threads of the workgroup.  A decode batch has few tokens and wants every wave it can get on a token's expert rows;
 // a prefill chunk has a workgroup per token anyway, and small workgroups, eight to a CU, hide each other's row loads.)
@@ -152,11 +115,11 @@ __device__ __forceinline__ void store_planes(_Float16 *planes, int E, int t, int
     *reinterpret_cast<uint2 *>(to) = __builtin_bit_cast(uint2, hi);
     *reinterpret_cast<uint2 *>(to + 128) = __builtin_bit_cast(uint2, lo);
 }
-// the logits of this workgroup's token and expert slice (blockIdx.y of gridDim.y), into s_logits and logits_out; the normalised row into planes
+// the logits of this workgroup's token, into s_logits and logits_out
 template <int NV, int RT>      // float4 groups per lane = E / 256
 __device__ __forceinline__ void router_logits(const float *__restrict__ x, const float *__restrict__ norm_w, const float *__restrict__ W,
                                               float *__restrict__ logits_out, int ldx, float eps, int p_n_expert, float *s_logits,
-                                              float *__restrict__ scale_out = nullptr, _Float16 *__restrict__ planes = nullptr, unsigned *sat = nullptr) {
+                                              float *__restrict__ scale_out = nullptr) {
     constexpr int E = NV * 256, ROUTER_WAVES = RT / 64;
     const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     // element index of a lane's values: 4 * (lane + 64 * i) + c
@@ -168,28 +131,18 @@ __device__ __forceinline__ void router_logits(const float *__restrict__ x, const
         xr[i] = *reinterpret_cast<const float4 *>(xt + 4 * (lane + 64 * i));
         ss += xr[i].x * xr[i].x + xr[i].y * xr[i].y + xr[i].z * xr[i].z + xr[i].w * xr[i].w;
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
-    const float scale = 1.0f / sqrtf(ss / (float)E + eps);
-    if (scale_out && blockIdx.y == 0 && threadIdx.x == 0) scale_out[t] = scale;
+    const float scale = 1.0f / sqrtf(wave_sum(ss) / (float)E + eps);
+    if (scale_out && threadIdx.x == 0) scale_out[t] = scale;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const float4 w = *reinterpret_cast<const float4 *>(norm_w + 4 * (lane + 64 * i));
         xr[i].x = xr[i].x * scale * w.x; xr[i].y = xr[i].y * scale * w.y;
         xr[i].z = xr[i].z * scale * w.z; xr[i].w = xr[i].w * scale * w.w;
     }
-    // (each of the first workgroup's waves writes its share of the row)
-    if (planes && blockIdx.y == 0) {
-#pragma unroll
-        for (int i = 0; i < NV; ++i)
-            if (i % ROUTER_WAVES == wave) store_planes(planes, E, t, 4 * (lane + 64 * i), xr[i], sat);
-    }
     // two expert rows per step, all of their loads in flight together
-    const int per = (p_n_expert + (int)gridDim.y - 1) / (int)gridDim.y;
-    const int e_lo = (int)blockIdx.y * per, e_hi = e_lo + per < p_n_expert ? e_lo + per : p_n_expert;
-    for (int e0 = e_lo + wave; e0 < e_hi; e0 += 2 * ROUTER_WAVES) {
+    for (int e0 = wave; e0 < p_n_expert; e0 += 2 * ROUTER_WAVES) {
         const int e1 = e0 + ROUTER_WAVES;
-        const bool has1 = e1 < e_hi;
+        const bool has1 = e1 < p_n_expert;
         const float *w0 = W + (size_t)e0 * E, *w1 = W + (size_t)(has1 ? e1 : e0) * E;
         float4 r0[NV], r1[NV];
 #pragma unroll
@@ -203,8 +156,8 @@ __device__ __forceinline__ void router_logits(const float *__restrict__ x, const
             a0 = fmaf(xr[i].x, r0[i].x, a0); a0 = fmaf(xr[i].y, r0[i].y, a0); a0 = fmaf(xr[i].z, r0[i].z, a0); a0 = fmaf(xr[i].w, r0[i].w, a0);
             a1 = fmaf(xr[i].x, r1[i].x, a1); a1 = fmaf(xr[i].y, r1[i].y, a1); a1 = fmaf(xr[i].z, r1[i].z, a1); a1 = fmaf(xr[i].w, r1[i].w, a1);
         }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) { a0 += __shfl_xor(a0, o); a1 += __shfl_xor(a1, o); }
+        a0 = wave_sum(a0);
+        a1 = wave_sum(a1);
         if (lane == 0) {
             s_logits[e0] = a0;
             if (logits_out) logits_out[(size_t)t * p_n_expert + e0] = a0;
@@ -220,11 +173,9 @@ template <int NV, int RT = ROUTER_THREADS>
 // (scalar arguments first: preloaded into SGPRs, see gemv.hip)
 __global__ __launch_bounds__(RT) void moe_router_fused_kernel(const float *__restrict__ x, const float *__restrict__ norm_w,
                                                                           const float *__restrict__ W, float *__restrict__ logits_out,
-                                                                          int ldx, float eps, int p_n_expert, const MoeRouteArgs a, float *__restrict__ scale_out,
-                                                                          _Float16 *planes, unsigned *sat) {
+                                                                          int ldx, float eps, int p_n_expert, const MoeRouteArgs a, float *__restrict__ scale_out) {
     __shared__ float s_logits[64 * ROUTE_MAX_PER_LANE];
-    router_logits<NV, RT>(x, norm_w, W, logits_out, ldx, eps, p_n_expert, s_logits, scale_out, planes, sat);
-    if (gridDim.y > 1) return;
+    router_logits<NV, RT>(x, norm_w, W, logits_out, ldx, eps, p_n_expert, s_logits, scale_out);
     __syncthreads();
     if ((threadIdx.x >> 6) == 0) route_wave_any(s_logits, a, blockIdx.x, threadIdx.x & 63);
 }
@@ -253,9 +204,7 @@ __global__ __launch_bounds__(CHUNK_THREADS) void moe_router_chunk_kernel(const f
             xr[k][i] = *reinterpret_cast<const float4 *>(xt + 4 * (lane + 64 * i));
             ss += xr[k][i].x * xr[k][i].x + xr[k][i].y * xr[k][i].y + xr[k][i].z * xr[k][i].z + xr[k][i].w * xr[k][i].w;
         }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
-        const float scale = 1.0f / sqrtf(ss / (float)E + eps);
+        const float scale = 1.0f / sqrtf(wave_sum(ss) / (float)E + eps);
         sc[k] = scale;
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
@@ -280,9 +229,7 @@ __global__ __launch_bounds__(CHUNK_THREADS) void moe_router_chunk_kernel(const f
             acc[k] = v;
         }
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1)
-#pragma unroll
-            for (int k = 0; k < CHUNK_TOKENS; ++k) acc[k] += __shfl_xor(acc[k], o);
+        for (int k = 0; k < CHUNK_TOKENS; ++k) acc[k] = wave_sum(acc[k]);
         if (lane == 0) {
 #pragma unroll
             for (int k = 0; k < CHUNK_TOKENS; ++k) {
@@ -297,6 +244,58 @@ __global__ __launch_bounds__(CHUNK_THREADS) void moe_router_chunk_kernel(const f
             if (t0 + k < T) scale_out[t0 + k] = sc[k];
     __syncthreads();
     if (wave < CHUNK_TOKENS && t0 + wave < T) route_wave_any(s_logits[wave], a, t0 + wave, lane);
+}
+
+// Router logits of a batch of decode steps, a workgroup per token and four experts, one row of the matrix per wave.  The bits of router_logits:
+// the sums of a lane's elements and of the lanes go the same way.  planes (optional): the normalised row as pairs of f16.
+// Bound by its chain (row, sum of squares, dot product).  A CU pulls about 25 GB/s of what is not in its caches, so that a slice should be
+// small: 16 rows of 8 KB a workgroup, every wave its own copy of the token's row, 9.4 us (16 tokens, 64 experts x 2048), all 64 rows 25, four
+// rows 3.6.  (Before, the last of the 16-row workgroups to arrive routed and grouped behind a hand-over between workgroups: 19.4 us in one launch,
+// against 3.6 + 5.6 now.)
+constexpr int SLICE_THREADS = 256, SLICE_WAVES = SLICE_THREADS / 64;
+template <int NV>
+__global__ __launch_bounds__(SLICE_THREADS) void moe_router_slice_kernel(const float *__restrict__ x, const float *__restrict__ norm_w, const float *__restrict__ W,
+                                                                         float *__restrict__ logits, int ldx, float eps, int n_expert, _Float16 *__restrict__ planes, unsigned *sat) {
+    constexpr int E = NV * 256, PER = E / 4 / SLICE_THREADS > 0 ? E / 4 / SLICE_THREADS : 1;       // float4 groups of the row a thread brings
+    __shared__ __align__(16) float s_x[E];
+    __shared__ float s_sq[E / 4];
+    const int t = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int e = blockIdx.x * SLICE_WAVES + wave, row = e < n_expert ? e : n_expert - 1;
+    const float *xt = x + (size_t)t * ldx;
+    float4 xv[PER], nw[PER], r[NV];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) xv[i] = *reinterpret_cast<const float4 *>(xt + 4 * ((tid + SLICE_THREADS * i) % (E / 4)));
+#pragma unroll
+    for (int i = 0; i < PER; ++i) nw[i] = *reinterpret_cast<const float4 *>(norm_w + 4 * ((tid + SLICE_THREADS * i) % (E / 4)));
+    // the row of the matrix is on its way while the token's is normalised
+#pragma unroll
+    for (int i = 0; i < NV; ++i) r[i] = *reinterpret_cast<const float4 *>(W + (size_t)row * E + 4 * (lane + 64 * i));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+        if (tid + SLICE_THREADS * i < E / 4) s_sq[tid + SLICE_THREADS * i] = xv[i].x * xv[i].x + xv[i].y * xv[i].y + xv[i].z * xv[i].z + xv[i].w * xv[i].w;
+    lds_barrier();
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) ss += s_sq[lane + 64 * i];
+    const float scale = 1.0f / sqrtf(wave_sum(ss) / (float)E + eps);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int g = tid + SLICE_THREADS * i;
+        if (g >= E / 4) continue;
+        const float4 v = make_float4(xv[i].x * scale * nw[i].x, xv[i].y * scale * nw[i].y, xv[i].z * scale * nw[i].z, xv[i].w * scale * nw[i].w);
+        *reinterpret_cast<float4 *>(s_x + 4 * g) = v;
+        if (planes && blockIdx.x == 0) store_planes(planes, E, t, 4 * g, v, sat);
+    }
+    lds_barrier();
+    float acc = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const float4 v = *reinterpret_cast<const float4 *>(s_x + 4 * (lane + 64 * i));
+        acc = fmaf(v.x, r[i].x, acc); acc = fmaf(v.y, r[i].y, acc); acc = fmaf(v.z, r[i].z, acc); acc = fmaf(v.w, r[i].w, acc);
+    }
+    acc = wave_sum(acc);
+    if (lane == 0 && e < n_expert) logits[(size_t)t * n_expert + e] = acc;
 }
 
 int moe_router_fused(const MoeRouteArgs &a, const float *x, int ldx, const float *norm_w, float eps, const float *W, int E,
@@ -317,10 +316,10 @@ int moe_router_fused(const MoeRouteArgs &a, const float *x, int ldx, const float
     if (T >= ROUTER_WIDE_MIN_TOKENS) {
         const dim3 block(ROUTER_THREADS_WIDE);
         switch (E / 256) {
-            case 2: MESH_LAUNCH((moe_router_fused_kernel<2, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out, nullptr, nullptr); break;
-            case 4: MESH_LAUNCH((moe_router_fused_kernel<4, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out, nullptr, nullptr); break;
-            case 8: MESH_LAUNCH((moe_router_fused_kernel<8, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out, nullptr, nullptr); break;
-            case 16: MESH_LAUNCH((moe_router_fused_kernel<16, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out, nullptr, nullptr); break;
+            case 2: MESH_LAUNCH((moe_router_fused_kernel<2, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
+            case 4: MESH_LAUNCH((moe_router_fused_kernel<4, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
+            case 8: MESH_LAUNCH((moe_router_fused_kernel<8, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
+            case 16: MESH_LAUNCH((moe_router_fused_kernel<16, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
             default: return fail(MESH_ERR_UNSUPPORTED, "moe: fused router for hidden size %d", E);
         }
         MESH_LAUNCH_CHECK();
@@ -328,10 +327,10 @@ int moe_router_fused(const MoeRouteArgs &a, const float *x, int ldx, const float
     }
     const dim3 block(ROUTER_THREADS);
     switch (E / 256) {
-        case 2: MESH_LAUNCH(moe_router_fused_kernel<2>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out, nullptr, nullptr); break;
-        case 4: MESH_LAUNCH(moe_router_fused_kernel<4>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out, nullptr, nullptr); break;
-        case 8: MESH_LAUNCH(moe_router_fused_kernel<8>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out, nullptr, nullptr); break;
-        case 16: MESH_LAUNCH(moe_router_fused_kernel<16>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out, nullptr, nullptr); break;
+        case 2: MESH_LAUNCH(moe_router_fused_kernel<2>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
+        case 4: MESH_LAUNCH(moe_router_fused_kernel<4>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
+        case 8: MESH_LAUNCH(moe_router_fused_kernel<8>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
+        case 16: MESH_LAUNCH(moe_router_fused_kernel<16>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
         default: return fail(MESH_ERR_UNSUPPORTED, "moe: fused router for hidden size %d", E);
     }
     MESH_LAUNCH_CHECK();
@@ -359,55 +358,58 @@ constexpr int GROUP_THREADS = 1024, GROUP_WAVES = GROUP_THREADS / 64;
 // ids == nullptr: the pair list is in lds[0 .. n_pairs) already and a barrier has been passed since it was written
 __device__ __forceinline__ void group_pairs(const int32_t *__restrict__ ids, int n_pairs, int n_expert, int32_t *__restrict__ items,
                                             int32_t *__restrict__ n_items, int32_t *lds, int ipairs) {
-    const int iints = moe_item_ints(ipairs);
+    const int iints = moe_item_ints(ipairs), shift = __builtin_ctz((unsigned)ipairs);       // (a power of two)
     int32_t *s_ids = lds, *s_cnt = lds + n_pairs, *s_base = s_cnt + n_expert;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     if (ids) {
         for (int p = tid; p < n_pairs; p += GROUP_THREADS) s_ids[p] = ids[p];
         __syncthreads();
     }
+    // the first pairs of the list stay in a lane's registers: a wave's experts find theirs among them without a trip to LDS
+    constexpr int HELD = 4;
+    int held[HELD];
+#pragma unroll
+    for (int j = 0; j < HELD; ++j) held[j] = lane + 64 * j < n_pairs ? s_ids[lane + 64 * j] : -1;
     for (int e = wave; e < n_expert; e += GROUP_WAVES) {
         int c = 0;
-        for (int p0 = 0; p0 < n_pairs; p0 += 64) {
+#pragma unroll
+        for (int j = 0; j < HELD; ++j) c += __popcll(__ballot(held[j] == e));
+        for (int p0 = 64 * HELD; p0 < n_pairs; p0 += 64) {
             const int p = p0 + lane;
             c += __popcll(__ballot(p < n_pairs && s_ids[p] == e));
         }
         if (lane == 0) s_cnt[e] = c;
     }
-    __syncthreads();
+    lds_barrier();
     if (wave == 0) {
         // exclusive prefix of items per expert: each lane sums a run of experts, the runs are scanned across the wave
         const int per = (n_expert + 63) / 64, e0 = lane * per;
         int mine = 0;
-        for (int e = e0; e < e0 + per && e < n_expert; ++e) mine += (s_cnt[e] + ipairs - 1) / ipairs;
-        int incl = mine;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int v = __shfl_up(incl, o);
-            if (lane >= o) incl += v;
-        }
+        for (int e = e0; e < e0 + per && e < n_expert; ++e) mine += (s_cnt[e] + ipairs - 1) >> shift;
+        const int incl = wave_scan(mine);
         int run = incl - mine;
         for (int e = e0; e < e0 + per && e < n_expert; ++e) {
             s_base[e] = run;
-            run += (s_cnt[e] + ipairs - 1) / ipairs;
+            run += (s_cnt[e] + ipairs - 1) >> shift;
         }
         if (lane == 63) n_items[0] = incl;
     }
-    __syncthreads();
+    lds_barrier();
     for (int e = wave; e < n_expert; e += GROUP_WAVES) {
         const int cnt = s_cnt[e], base = s_base[e];
         int seen = 0;
-        for (int p0 = 0; p0 < n_pairs && seen < cnt; p0 += 64) {
-            const int p = p0 + lane;
-            const bool hit = p < n_pairs && s_ids[p] == e;
+        auto place = [&](int p, bool hit) {
             const unsigned long long m = __ballot(hit);
             if (hit) {
                 const int r = seen + __popcll(m & ((1ull << lane) - 1ull));
-                items[(size_t)(base + r / ipairs) * iints + 2 + r % ipairs] = p;
+                items[(size_t)(base + (r >> shift)) * iints + 2 + (r & (ipairs - 1))] = p;
             }
             seen += __popcll(m);
-        }
-        const int n_it = (cnt + ipairs - 1) / ipairs;
+        };
+#pragma unroll
+        for (int j = 0; j < HELD; ++j) place(lane + 64 * j, held[j] == e);
+        for (int p0 = 64 * HELD; p0 < n_pairs && seen < cnt; p0 += 64) place(p0 + lane, p0 + lane < n_pairs && s_ids[p0 + lane] == e);
+        const int n_it = (cnt + ipairs - 1) >> shift;
         for (int i = lane; i < n_it; i += 64) {
             items[(size_t)(base + i) * iints + 0] = e;
             items[(size_t)(base + i) * iints + 1] = i + 1 < n_it ? ipairs : cnt - i * ipairs;
@@ -423,7 +425,8 @@ __global__ __launch_bounds__(GROUP_THREADS) void moe_group_kernel(const int32_t 
 
 // Routing of a small batch and the grouping of its pairs in one single-workgroup launch: wave w routes tokens w,
 // w + 16, ... from their logits, then the workgroup groups the pairs it has just written (the barrier in between
-// also makes those writes visible to the whole workgroup).
+// also makes those writes visible to the whole workgroup).  A chain: 9.1 us with reductions through the LDS unit and a rank counted
+// over all candidates, 5.6 now (16 tokens, 64 experts, top 8; 4.5 of it without the grouping).
 // (the routing arguments as leading scalars: preloaded into SGPRs, see gemv.hip)
 __global__ __launch_bounds__(GROUP_THREADS) void moe_route_group_kernel(const float *p_logits, const float *p_mask, int32_t *p_ids, float *p_weights,
                                                                         int T, int p_n_expert, int p_top_k, int p_norm_w,
@@ -438,74 +441,19 @@ __global__ __launch_bounds__(GROUP_THREADS) void moe_route_group_kernel(const fl
     group_pairs(nullptr, T * p_top_k, p_n_expert, items, n_items, g_lds, ipairs);
 }
 
-// The two launches above as one: every workgroup computes its slice of the logits; the one that arrives last (a device-wide
-// counter, release fence before the increment, acquire fence after it) then routes all tokens and groups the pairs, as
-// moe_route_group_kernel does.  The counter is back at zero when the launch ends.  No workgroup waits for another.
-template <int NV>
-__global__ __launch_bounds__(GROUP_THREADS) void moe_router_group_fused_kernel(const float *__restrict__ x, const float *__restrict__ norm_w,
-                                                                               const float *__restrict__ W, float *logits, int ldx, float eps,
-                                                                               int p_n_expert, const MoeRouteArgs a, int T, int32_t *items, int32_t *n_items,
-                                                                               int ipairs, int *arrive, _Float16 *planes, unsigned *sat) {
-    static_assert(GROUP_THREADS == ROUTER_THREADS, "the routing tail runs in a router workgroup");
-    extern __shared__ int32_t g_lds[];
-    __shared__ float s_logits[64 * ROUTE_MAX_PER_LANE];
-    __shared__ int s_last;
-    router_logits<NV, ROUTER_THREADS>(x, norm_w, W, logits, ldx, eps, p_n_expert, s_logits, nullptr, planes, sat);
-    // One release per workgroup, by one thread: the barrier orders the other waves' logits stores before it, and a
-    // release at device scope covers what the releasing thread has observed.  (A __threadfence() in every wave measured
-    // 35 us for this tail: sixteen cache write-backs and invalidations per workgroup.)
-    __syncthreads();
-    if (threadIdx.x == 0)
-        s_last = __hip_atomic_fetch_add(arrive, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == (int)(gridDim.x * gridDim.y) - 1;
-    __syncthreads();
-    if (!s_last) return;
-    if (threadIdx.x == 0) __hip_atomic_store(arrive, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    // LDS of the tail: the pair list and the grouping's counters, then a logits row per wave
-    const int n_group_ints = T * a.top_k + 2 * p_n_expert;
-    for (int t = wave; t < T; t += GROUP_WAVES) {
-        // the token's logits through LDS: route_wave reads plain floats
-        float *row = reinterpret_cast<float *>(g_lds + n_group_ints) + (size_t)wave * 64 * ROUTE_MAX_PER_LANE;
-        // (device-scope loads: written by other workgroups of this launch, possibly on another die)
-        for (int e = lane; e < p_n_expert; e += 64) row[e] = __hip_atomic_load(logits + (size_t)t * p_n_expert + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        route_wave_any(row, a, t, lane, g_lds);        // (ids to memory and to the pair list in LDS)
-        __builtin_amdgcn_wave_barrier();
-    }
-    __syncthreads();
-    group_pairs(nullptr, T * a.top_k, p_n_expert, items, n_items, g_lds, ipairs);
-}
-
 int moe_router_group(const MoeRouteArgs &a, const float *x, int ldx, const float *norm_w, float eps, const float *W, int E,
-                     float *logits, int T, int32_t *items, int32_t *n_items, int item_pairs, hipStream_t stream, int *arrive, uint16_t *planes, unsigned *sat) {
+                     float *logits, int T, int32_t *items, int32_t *n_items, int item_pairs, hipStream_t stream, uint16_t *planes, unsigned *sat) {
     if (T <= 0) return MESH_OK;
     if (!moe_router_group_supported(E, a.n_expert, a.top_k, T) || !logits)
         return fail(MESH_ERR_UNSUPPORTED, "moe: split router for hidden size %d / %d experts / %d tokens", E, a.n_expert, T);
-    const int split = (a.n_expert + ROUTER_WAVES - 1) / ROUTER_WAVES;      // one expert row per wave
-    const dim3 grid((unsigned)T, (unsigned)split), block(ROUTER_THREADS);
+    const dim3 grid((unsigned)((a.n_expert + SLICE_WAVES - 1) / SLICE_WAVES), (unsigned)T), block(SLICE_THREADS);
     MoeRouteArgs la = a;
-    if (arrive) {
-        // one launch: the last workgroup to finish its logits routes and groups
-        la.logits = logits;
-        // LDS of the tail: the grouping's pair list and counters, then a logits row per wave
-        const size_t smem = (size_t)GROUP_WAVES * 64 * ROUTE_MAX_PER_LANE * sizeof(float) + ((size_t)T * a.top_k + 2 * (size_t)a.n_expert) * sizeof(int32_t);
-        switch (E / 256) {
-            case 2: MESH_LAUNCH(moe_router_group_fused_kernel<2>, grid, block, smem, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, T, items, n_items, item_pairs, arrive, reinterpret_cast<_Float16 *>(planes), sat); break;
-            case 4: MESH_LAUNCH(moe_router_group_fused_kernel<4>, grid, block, smem, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, T, items, n_items, item_pairs, arrive, reinterpret_cast<_Float16 *>(planes), sat); break;
-            case 8: MESH_LAUNCH(moe_router_group_fused_kernel<8>, grid, block, smem, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, T, items, n_items, item_pairs, arrive, reinterpret_cast<_Float16 *>(planes), sat); break;
-            case 16: MESH_LAUNCH(moe_router_group_fused_kernel<16>, grid, block, smem, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, T, items, n_items, item_pairs, arrive, reinterpret_cast<_Float16 *>(planes), sat); break;
-            default: return fail(MESH_ERR_UNSUPPORTED, "moe: fused router for hidden size %d", E);
-        }
-        MESH_LAUNCH_CHECK();
-        return MESH_OK;
-    }
+    _Float16 *p = reinterpret_cast<_Float16 *>(planes);
     switch (E / 256) {
-        case 2: MESH_LAUNCH(moe_router_fused_kernel<2>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, static_cast<float *>(nullptr), reinterpret_cast<_Float16 *>(planes), sat); break;
-        case 4: MESH_LAUNCH(moe_router_fused_kernel<4>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, static_cast<float *>(nullptr), reinterpret_cast<_Float16 *>(planes), sat); break;
-        case 8: MESH_LAUNCH(moe_router_fused_kernel<8>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, static_cast<float *>(nullptr), reinterpret_cast<_Float16 *>(planes), sat); break;
-        case 16: MESH_LAUNCH(moe_router_fused_kernel<16>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, la.n_expert, la, static_cast<float *>(nullptr), reinterpret_cast<_Float16 *>(planes), sat); break;
+        case 2: MESH_LAUNCH(moe_router_slice_kernel<2>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, a.n_expert, p, sat); break;
+        case 4: MESH_LAUNCH(moe_router_slice_kernel<4>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, a.n_expert, p, sat); break;
+        case 8: MESH_LAUNCH(moe_router_slice_kernel<8>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, a.n_expert, p, sat); break;
+        case 16: MESH_LAUNCH(moe_router_slice_kernel<16>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, a.n_expert, p, sat); break;
         default: return fail(MESH_ERR_UNSUPPORTED, "moe: fused router for hidden size %d", E);
     }
     MESH_LAUNCH_CHECK();

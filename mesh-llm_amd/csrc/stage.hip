@@ -516,12 +516,11 @@ static int kquant_session_alloc(mesh_session *s) {
             if ((rc = sess_alloc(s, &p, expert_ffn_bytes(step_items, (int)hp.n_ff_exp))) != MESH_OK) return rc;
             s->moe_step_ffn = static_cast<uint16_t *>(p);
         }
-        // (+ the item count, + the arrival counter of the router launch whose last workgroup routes and groups)
-        if ((rc = sess_alloc(s, &p, (items * MOE_ITEM_INTS + 2) * sizeof(int32_t))) != MESH_OK) return rc;
+        // (+ the item count)
+        if ((rc = sess_alloc(s, &p, (items * MOE_ITEM_INTS + 1) * sizeof(int32_t))) != MESH_OK) return rc;
         s->moe_items = static_cast<int32_t *>(p);
         s->moe_n_items = s->moe_items + items * MOE_ITEM_INTS;
-        s->moe_arrive = reinterpret_cast<int *>(s->moe_n_items + 1);
-        MESH_HIP_TRY(hipMemsetAsync(s->moe_items, 0, (items * MOE_ITEM_INTS + 2) * sizeof(int32_t), s->stream));
+        MESH_HIP_TRY(hipMemsetAsync(s->moe_items, 0, (items * MOE_ITEM_INTS + 1) * sizeof(int32_t), s->stream));
         MESH_HIP_TRY(hipMemsetAsync(s->expert_mask, 0, ne * sizeof(float), s->stream));
         if (st->layers[0].exps_gate_up_gemm && s->xn16 && B * k >= MOE_GEMM_MIN_PAIRS_PER_EXPERT * ne) {
             // prefill chunks: the pairs sorted by expert, their inputs / SwiGLU outputs in the k8-major f16 layout and their
@@ -1176,11 +1175,11 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
             const int item_pairs = step ? EXPERT_STEP_PAIRS : mfma ? SKINNY_ITEM_PAIRS : MOE_ITEM_PAIRS;
             bool grouped_done = false;
             if (want_groups && L.gate_inp.type == MESH_F32 && moe_router_group_supported(E, ne, k, T)) {
-                // a batch of decode steps: logits over many workgroups, then routing and grouping in one launch
+                // a batch of decode steps: logits over many workgroups, then routing and grouping in one
                 ProfScope ps(s, MESH_PROF_GEMV);
                 if ((rc = moe_router_group(mr, s->x, E, static_cast<const float *>(L.ffn_norm.data), hp.rms_eps,
                                            static_cast<const float *>(L.gate_inp.data), E, s->moe_logits, T, s->moe_items, s->moe_n_items,
-                                           item_pairs, stream, s->tune.moe_router_tail ? s->moe_arrive : nullptr, step ? s->moe_step_x : nullptr, s->f16_sat)) != MESH_OK) return rc;
+                                           item_pairs, stream, step ? s->moe_step_x : nullptr, s->f16_sat)) != MESH_OK) return rc;
                 grouped_done = true;
             } else if (L.gate_inp.type == MESH_F32 && moe_router_fused_supported(E, ne, k)) {
                 // the router matrix is small and f32: logits and routing in one launch

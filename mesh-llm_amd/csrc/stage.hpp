@@ -137,7 +137,6 @@ struct mesh_session {
     bool expert_mask_on = false;
     int32_t *moe_ids = nullptr;
     int32_t *moe_items = nullptr, *moe_n_items = nullptr;      // (token, slot) pairs grouped by expert, see moe_group
-    int *moe_arrive = nullptr;                                 // arrival counter of the fused router launch (zero between launches)
     // decode steps: normalised inputs and SwiGLU outputs of the expert products as pairs of f16 (expert_step.hpp)
     uint16_t *moe_step_x = nullptr, *moe_step_ffn = nullptr;
     // prefill chunks: the pairs sorted by expert (moe_sort) and their buffers, rows indexed by slot
