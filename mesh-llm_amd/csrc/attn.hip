@@ -10,6 +10,7 @@
 
 #include "act_math.hpp"
 #include "q16.hpp"
+#include "wave_ops.hpp"
 
 namespace mesh {
 
@@ -45,8 +46,7 @@ __global__ __launch_bounds__(64) void rope_kv_kernel(const int32_t *p_pos, const
     if (nw) {
         float ss = 0.f;
         for (int i = lane; i < hd; i += 64) ss += vec[i] * vec[i];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+        ss = wave_sum(ss);
         nscale = 1.0f / sqrtf(ss / (float)hd + a.eps);
     }
     const int half = a.n_rot / 2;

@@ -29,6 +29,7 @@
 #include "attn.hpp"
 #include "lds_ops.hpp"
 #include "q16.hpp"
+#include "wave_ops.hpp"
 
 namespace mesh {
 
@@ -269,8 +270,7 @@ __global__ __launch_bounds__(MMA_THREADS) void attn_mma_kernel(const float *p_q,
                 s[h][i] = kb + 16 * h + 4 * g + i < j1 ? s[h][i] : -INFINITY;
                 mx = fmaxf(mx, s[h][i]);
             }
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        mx = lane_fold<32>(lane_fold<16>(mx, LaneMax{}), LaneMax{});
         // The reference point m of the exponentials only moves when a score exceeds it by more than 2^RESCALE_STEP
         // (probabilities then stay below that factor, harmless in f16 / f32), and then for the whole wave at once:
         // the rescale of the 32 accumulator registers becomes rare instead of once per block.
@@ -305,8 +305,7 @@ __global__ __launch_bounds__(MMA_THREADS) void attn_mma_kernel(const float *p_q,
     }
 
     // merge the waves: o[db][i] is place 16 db + 4 g + i of head c
-    l += __shfl_xor(l, 16);
-    l += __shfl_xor(l, 32);
+    l = lane_fold<32>(lane_fold<16>(l, LaneAdd{}), LaneAdd{});
     __syncthreads();               // every wave is done with its V tile: the memory becomes the merge buffer
     float *s_o = reinterpret_cast<float *>(s_raw);          // [wave][16 heads][place]
     if (g == 0) { s_m[wave][c] = m; s_l[wave][c] = l; }

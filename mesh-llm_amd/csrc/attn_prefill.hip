@@ -33,6 +33,7 @@
 #include "act_math.hpp"
 #include "attn.hpp"
 #include "lds_ops.hpp"
+#include "wave_ops.hpp"
 
 namespace mesh {
 
@@ -245,7 +246,7 @@ __global__ __launch_bounds__(512) void attn_chunk_kernel(const AttnArgs a, int T
 #pragma unroll
             for (int t = 0; t < NT; ++t) mxt[t] = fmaxf(mxt[t], s[t][i]);
         float mx = NT == 2 ? fmaxf(mxt[0], mxt[NT - 1]) : mxt[0];
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        mx = lane_fold<32>(mx, LaneMax{});
         // m is the reference the exponentials are taken against.  It follows the running maximum only when that has
         // moved by more than PF_RESCALE_STEP (log2 units), so that most steps skip the rescale of the 64 accumulator
         // registers; in between p <= 2^PF_RESCALE_STEP, which f16 holds comfortably.  (Without a window key 0
@@ -281,7 +282,7 @@ __global__ __launch_bounds__(512) void attn_chunk_kernel(const AttnArgs a, int T
             pf[t][1] = __builtin_bit_cast(pf_h8, pu2);
         }
         float ps = ps0 + ps1;
-        ps += __shfl_xor(ps, 32);
+        ps = lane_fold<32>(ps, LaneAdd{});
         l += ps;
 #pragma unroll
         for (int db = 0; db < NDB; ++db) {

@@ -9,6 +9,7 @@
 #include <algorithm>
 
 #include "act_math.hpp"
+#include "wave_ops.hpp"
 
 namespace mesh {
 
@@ -17,11 +18,6 @@ typedef float gs_f4 __attribute__((ext_vector_type(4)));
 constexpr int C = STATE_CHUNK;
 constexpr float UNIT_EPS = 1e-6f;               // inside the root of the unit vectors of DELTA
 
-__device__ __forceinline__ float gs_wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-}
 __device__ __forceinline__ float gs_softplus(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }
 __device__ __forceinline__ gs_f4 gs_mma(const float4 &a, const gs_f4 &b, gs_f4 acc) {
     acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b[0], acc, 0, 0, 0);
@@ -125,7 +121,7 @@ __global__ __launch_bounds__(THREADS) void gated_step_kernel(const GatedStateArg
         if (wave < 2) {
             float *u = wave == 0 ? sq : sk, ss = 0.f;
             for (int d = lane; d < D; d += 64) ss = fmaf(u[d], u[d], ss);
-            const float r = (wave == 0 ? 1.0f / sqrtf((float)D) : 1.0f) / sqrtf(gs_wave_sum(ss) + UNIT_EPS);
+            const float r = (wave == 0 ? 1.0f / sqrtf((float)D) : 1.0f) / sqrtf(wave_sum(ss) + UNIT_EPS);
             for (int d = lane; d < D; d += 64) u[d] *= r;
         }
     } else {
@@ -143,8 +139,7 @@ __global__ __launch_bounds__(THREADS) void gated_step_kernel(const GatedStateArg
 #pragma unroll 4
                 for (int r = tid & 3; r < a.rank; r += 4) z = fmaf(w[r], x[a.at_a + r], z);
             }
-            z += __shfl_xor(z, 1);
-            z += __shfl_xor(z, 2);
+            z = group_sum<4>(z);
             if (d < D && (tid & 3) == 0) sd[d] = expf(-gs_softplus(-(z + a.a2_bias[h * D + d])) * a.inv_tau);
         }
         for (int v = tid; v < V; v += THREADS) sv[v] = x[a.at_v + h * V + v];
@@ -153,7 +148,7 @@ __global__ __launch_bounds__(THREADS) void gated_step_kernel(const GatedStateArg
     if (wave == 0) {
         float s = 0.f;
         for (int d = lane; d < D; d += 64) s = fmaf(sq[d], sk[d], s);
-        s = gs_wave_sum(s);
+        s = wave_sum(s);
         if (lane == 0) s_qk = s;
     }
     // S^T k and S^T q of the decayed state; with them o = S^T q + (k . q) u needs no second walk
@@ -181,7 +176,7 @@ __global__ __launch_bounds__(THREADS) void gated_step_kernel(const GatedStateArg
     if (wave == 0) {
         float ss = 0.f;
         for (int i = lane; i < V; i += 64) ss = fmaf(so[i], so[i], ss);
-        ss = gs_wave_sum(ss);
+        ss = wave_sum(ss);
         if (lane == 0) s_ss = ss;
     }
     __syncthreads();
@@ -271,8 +266,7 @@ __global__ __launch_bounds__(PREP_THREADS) void delta_prepare_kernel(const Gated
             const float4 v = *reinterpret_cast<const float4 *>(u + d);
             ss = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ss))));
         }
-#pragma unroll
-        for (int o = 8; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+        ss = lanes_fold<8>(ss, LaneAdd{});
         const float f = (r < C ? qs : 1.0f) / sqrtf(ss + UNIT_EPS);
         for (int d = 4 * c; d < Dp; d += 64) {
             float4 v = *reinterpret_cast<const float4 *>(u + d);
@@ -463,7 +457,7 @@ __global__ __launch_bounds__(PREP_THREADS) void gla_prepare_kernel(const GatedSt
             const float4 q = *reinterpret_cast<const float4 *>(sQ + r * dp + d), k = *reinterpret_cast<const float4 *>(sK + r * dp + d);
             s = fmaf(q.x, k.x, fmaf(q.y, k.y, fmaf(q.z, k.z, fmaf(q.w, k.w, s))));
         }
-        s += __shfl_xor(s, 1); s += __shfl_xor(s, 2); s += __shfl_xor(s, 4);
+        s = group_sum<8>(s);
         if ((tid & 7) == 0) m.A[r * C + r] = s;
     }
     if (tid < 2 * PAIRS) {
@@ -669,7 +663,7 @@ __global__ __launch_bounds__(256) void gated_norm_kernel(const GatedStateArgs a,
             gate[k] = i < V ? x[a.at_g + h * V + i] : 0.f;
             ss = fmaf(v[k], v[k], ss);
         }
-        const float r = 1.0f / sqrtf(gs_wave_sum(ss) / (float)V + a.eps);
+        const float r = 1.0f / sqrtf(wave_sum(ss) / (float)V + a.eps);
 #pragma unroll
         for (int k = 0; k < STATE_DIM_MAX / 64; ++k) {
             const int i = lane + 64 * k;

@@ -18,6 +18,7 @@
 #include "gemm.hpp"
 #include "gemm_tile.hpp"
 #include "lds_ops.hpp"
+#include "wave_ops.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -1111,8 +1112,7 @@ __global__ __launch_bounds__(SN_THREADS) void gemm_splitk_epilogue_norm_kernel(G
             ss += (o.x * o.x + o.y * o.y) + (o.z * o.z + o.w * o.w);
         }
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+    ss = wave_sum(ss);
     if ((tid & 63) == 0) s_ss[tid >> 6] = ss;
     __syncthreads();
     float tot = 0.f;
@@ -1375,8 +1375,7 @@ __global__ __launch_bounds__(256) void rmsnorm_f16_kernel(const float *__restric
         const float4 v = *reinterpret_cast<const float4 *>(xt + i);
         ss += (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+    ss = wave_sum(ss);
     if ((tid & 63) == 0) red[tid >> 6] = ss;
     __syncthreads();
     const float scale = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)n + eps);

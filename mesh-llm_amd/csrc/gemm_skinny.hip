@@ -35,6 +35,7 @@
 #include "gemm.hpp"
 #include "gemv_device.hpp"
 #include "lds_ops.hpp"
+#include "wave_ops.hpp"
 
 namespace mesh {
 
@@ -647,8 +648,7 @@ __device__ __forceinline__ void q16_store8(const float (&v)[8], int i, int t, in
     float amax = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(v[e]));
-    amax = fmaxf(amax, __shfl_xor(amax, 1));
-    amax = fmaxf(amax, __shfl_xor(amax, 2));
+    amax = lanes_fold<2>(amax, LaneMax{});
     const float inv = amax > 0.f ? XQ_LEVELS / amax : 0.f;
     int hi[8], lo[8], isum = 0;
 #pragma unroll
@@ -658,8 +658,7 @@ __device__ __forceinline__ void q16_store8(const float (&v)[8], int i, int t, in
         hi[e] = (q - lo[e]) >> 8;
         isum += q;
     }
-    isum += __shfl_xor(isum, 1);
-    isum += __shfl_xor(isum, 2);
+    isum = group_sum<4>(isum);
     if (live) {
         planes[(size_t)(i >> 3) * 16 + t] = make_uint4(pack_bytes(hi[0], hi[1], hi[2], hi[3]), pack_bytes(hi[4], hi[5], hi[6], hi[7]),
                                                        pack_bytes(lo[0], lo[1], lo[2], lo[3]), pack_bytes(lo[4], lo[5], lo[6], lo[7]));
@@ -692,8 +691,7 @@ __global__ __launch_bounds__(Q16_THREADS) void quant16_kernel(const float *__res
             const float4 v = *reinterpret_cast<const float4 *>(xt + k);
             ss += (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
         }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+        ss = wave_sum(ss);
         if ((tid & 63) == 0) red[tid >> 6] = ss;
         __syncthreads();
         float tot = 0.f;
@@ -746,8 +744,7 @@ __global__ __launch_bounds__(Q16F_THREADS) void moe_combine_quant16_kernel(float
     if (tid < Q16_THREADS) {
         float ss = 0.f;
         for (int g = tid; g < n / 4; g += Q16_THREADS) ss += psq[g];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+        ss = wave_sum(ss);
         if ((tid & 63) == 0) red[tid >> 6] = ss;
     }
     __syncthreads();
@@ -826,8 +823,7 @@ __global__ __launch_bounds__(256) void to_k8_kernel(const float *__restrict__ x,
         for (int j = 0; j < RC; ++j)
 #pragma unroll
             for (int h = 0; h < 2; ++h) ss += (v[j][h].x * v[j][h].x + v[j][h].y * v[j][h].y) + (v[j][h].z * v[j][h].z + v[j][h].w * v[j][h].w);
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+        ss = wave_sum(ss);
         if ((tid & 63) == 0) red[tid >> 6] = ss;
         __syncthreads();
         const float sc = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)n + eps);
@@ -849,8 +845,7 @@ __global__ __launch_bounds__(256) void to_k8_kernel(const float *__restrict__ x,
             const float4 v = *reinterpret_cast<const float4 *>(xt + i);
             ss += (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
         }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+        ss = wave_sum(ss);
         if ((tid & 63) == 0) red[tid >> 6] = ss;
         __syncthreads();
         scale = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)n + eps);
@@ -893,9 +888,7 @@ __global__ __launch_bounds__(K8B_THREADS) void to_k8_block_kernel(const float *_
 #pragma unroll
         for (int h = 0; h < 2; ++h) ss += (v[j][h].x * v[j][h].x + v[j][h].y * v[j][h].y) + (v[j][h].z * v[j][h].z + v[j][h].w * v[j][h].w);
     // the eight lanes of a wave that hold the same token, then the waves in order
-    ss += __shfl_xor(ss, 8);
-    ss += __shfl_xor(ss, 16);
-    ss += __shfl_xor(ss, 32);
+    ss = lane_fold<32>(lane_fold<16>(lane_fold<8>(ss, LaneAdd{}), LaneAdd{}), LaneAdd{});
     if (lane < K8B_TOK) s_ss[wave][lane] = ss;
     __syncthreads();
     float tot = 0.f;
@@ -964,8 +957,7 @@ __global__ __launch_bounds__(256) void gather_k8_kernel(const float *__restrict_
                 ss += (b.x * b.x + b.y * b.y) + (b.z * b.z + b.w * b.w);
             }
         }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+        ss = wave_sum(ss);
         if (lane == 0) s_scale[sl] = 1.0f / sqrtf(ss / (float)n + eps);
     }
     __syncthreads();

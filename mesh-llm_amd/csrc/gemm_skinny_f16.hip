@@ -32,6 +32,7 @@
 #include "gemm.hpp"
 #include "lds_ops.hpp"
 #include "skinny_frags.hpp"
+#include "wave_ops.hpp"
 
 namespace mesh {
 namespace f16sk {
@@ -265,8 +266,8 @@ __device__ __forceinline__ void skinny_workgroup(int bx, const _Float16 *p_x, co
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         float ss = 0.f;
         for (int p = lane / NT; p < parts_per; p += 64 / NT) ss += wave * parts_per + p < parts_end ? my_parts[p * NT + lane % NT] : 0.f;
-        if (NT == 16) ss += __shfl_xor(ss, 16);
-        ss += __shfl_xor(ss, 32);
+        if (NT == 16) ss = lane_fold<16>(ss, LaneAdd{});
+        ss = lane_fold<32>(ss, LaneAdd{});
         if (lane < NT) nrm[wave * NT + lane] = ss;
     }
     [[maybe_unused]] float pre_sin[OUT_PRE], pre_cos[OUT_PRE];
@@ -352,8 +353,8 @@ __device__ __forceinline__ void skinny_workgroup(int bx, const _Float16 *p_x, co
     }
     if (a.no_part) {
         // this workgroup's sum of squares per column: the lanes of a wave that share a column, then the waves in order
-        if (NT == 16) no_ss += __shfl_xor(no_ss, 16);
-        no_ss += __shfl_xor(no_ss, 32);
+        if (NT == 16) no_ss = lane_fold<16>(no_ss, LaneAdd{});
+        no_ss = lane_fold<32>(no_ss, LaneAdd{});
         if (lane < NT) wsum[wave * NT + lane] = no_ss;
         __syncthreads();
         if (tid < NT) {

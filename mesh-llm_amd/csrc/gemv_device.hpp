@@ -3,6 +3,7 @@
 #pragma once
 
 #include "gemv.hpp"
+#include "wave_ops.hpp"
 
 namespace mesh {
 
@@ -102,8 +103,7 @@ __device__ __forceinline__ void x_quantise(const XRegs<NB> &X, int K, const XSta
         float amax = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
-        amax = fmaxf(amax, __shfl_xor(amax, 1));
-        amax = fmaxf(amax, __shfl_xor(amax, 2));
+        amax = lanes_fold<2>(amax, LaneMax{});
         const float inv = amax > 0.f ? XQ_LEVELS / amax : 0.f;
         int hi[8], lo[8], isum = 0;
 #pragma unroll
@@ -113,8 +113,8 @@ __device__ __forceinline__ void x_quantise(const XRegs<NB> &X, int K, const XSta
             hi[i] = (q - lo[i]) >> 8;
             isum += q;
         }
-        isum += __shfl_xor(isum, 1);                 // sum over 16 elements
-        const int isum32 = isum + __shfl_xor(isum, 2);
+        isum = lane_fold<1>(isum, LaneAdd{});        // sum over 16 elements
+        const int isum32 = lane_fold<2>(isum, LaneAdd{});
         if (live) {
             *reinterpret_cast<uint2 *>(S.xh + t * K + g * 8) = make_uint2(pack_bytes(hi[0], hi[1], hi[2], hi[3]), pack_bytes(hi[4], hi[5], hi[6], hi[7]));
             *reinterpret_cast<uint2 *>(S.xl + t * K + g * 8) = make_uint2(pack_bytes(lo[0], lo[1], lo[2], lo[3]), pack_bytes(lo[4], lo[5], lo[6], lo[7]));
@@ -133,15 +133,11 @@ __device__ __forceinline__ void x_quantise(const XRegs<NB> &X, int K, const XSta
 // x_quantise on the same 32 values, hence the same bits.
 __device__ __forceinline__ void xq_store_block32(uint8_t *xq, int K, int kk, float v) {
     float amax = fabsf(v);
-#pragma unroll
-    for (int o = 16; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
+    amax = lanes_fold<16>(amax, LaneMax{});
     const float inv = amax > 0.f ? XQ_LEVELS / amax : 0.f;
     const int q = __float2int_rn(v * inv);
     const int lo = ((q + 128) & 0xFF) - 128, hi = (q - lo) >> 8;
-    int isum = q;
-#pragma unroll
-    for (int o = 8; o > 0; o >>= 1) isum += __shfl_xor(isum, o);
-    const int isum32 = isum + __shfl_xor(isum, 16);
+    const int isum = lanes_fold<8>(q, LaneAdd{}), isum32 = lane_fold<16>(isum, LaneAdd{});
     xq[kk] = (uint8_t)hi;
     xq[K + kk] = (uint8_t)lo;
     float *xd = reinterpret_cast<float *>(xq + 2 * (size_t)K), *xs = xd + (K >> 5);

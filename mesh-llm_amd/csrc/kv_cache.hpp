@@ -15,6 +15,7 @@
 #pragma once
 
 #include "mesh_common.hpp"
+#include "wave_ops.hpp"
 
 namespace mesh {
 
@@ -86,6 +87,24 @@ template <int TYPE> __device__ __forceinline__ float kv_decode(const KvRaw<TYPE>
 }
 
 // ---------------------------------------------------------------------------------------------- row store / fetch
+struct KvExtreme {
+    float magnitude, value;
+    int at;
+};
+// over the 32 lanes of a block, the nearest last
+template <class F> __device__ __forceinline__ KvExtreme kv_block_extreme(KvExtreme e, F better) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const auto m = __builtin_amdgcn_permlane16_swap(__float_as_uint(e.magnitude), __float_as_uint(e.magnitude), false, false);
+    const auto v = __builtin_amdgcn_permlane16_swap(__float_as_uint(e.value), __float_as_uint(e.value), false, false);
+    const auto a = __builtin_amdgcn_permlane16_swap((unsigned)e.at, (unsigned)e.at, false, false);
+    e = better(KvExtreme{__uint_as_float(m[0]), __uint_as_float(v[0]), (int)a[0]}, KvExtreme{__uint_as_float(m[1]), __uint_as_float(v[1]), (int)a[1]});
+    e = better(e, KvExtreme{lane_dpp<0x128>(e.magnitude), lane_dpp<0x128>(e.value), lane_dpp<0x128>(e.at)});        // rotations of the row by 8, 4, 2, 1
+    e = better(e, KvExtreme{lane_dpp<0x124>(e.magnitude), lane_dpp<0x124>(e.value), lane_dpp<0x124>(e.at)});
+    e = better(e, KvExtreme{lane_dpp<0x122>(e.magnitude), lane_dpp<0x122>(e.value), lane_dpp<0x122>(e.at)});
+    e = better(e, KvExtreme{lane_dpp<0x121>(e.magnitude), lane_dpp<0x121>(e.value), lane_dpp<0x121>(e.at)});
+#endif
+    return e;
+}
 // One wave writes the row whose f32 values are in LDS (or any memory the whole wave can read): the block maximum
 // is a reduction over the 32 lanes of a block; q4_0 takes the FIRST element of largest magnitude, as the serial
 // reference loop does.
@@ -105,13 +124,10 @@ __device__ __forceinline__ void kv_store_row(int type, uint8_t *row, const float
         const float x = live ? vec[i] : 0.f;
         float am = fabsf(x), mv = x;
         int mi = i;
-#pragma unroll
-        for (int o = 16; o > 0; o >>= 1) {
-            const float a2 = __shfl_xor(am, o), v2 = __shfl_xor(mv, o);
-            const int i2 = __shfl_xor(mi, o);
-            const bool take = a2 > am || (a2 == am && i2 < mi);
-            am = take ? a2 : am; mv = take ? v2 : mv; mi = take ? i2 : mi;
-        }
+        // (the value of the largest magnitude, the first of equals)
+        const auto better = [](const KvExtreme &a, const KvExtreme &b) { return b.magnitude > a.magnitude || (b.magnitude == a.magnitude && b.at < a.at) ? b : a; };
+        const KvExtreme best = kv_block_extreme(KvExtreme{am, mv, mi}, better);
+        am = best.magnitude; mv = best.value;
         if (type == MESH_Q8_0) {
             const float d = am / 127.0f;
             const float id = d != 0.0f ? 1.0f / d : 0.0f;
@@ -123,7 +139,7 @@ __device__ __forceinline__ void kv_store_row(int type, uint8_t *row, const float
             const float id = d != 0.0f ? 1.0f / d : 0.0f;
             int q = (int)(x * id + 8.5f);
             q = q > 15 ? 15 : q;
-            const int qn = __shfl_xor(q, 1);
+            const int qn = lane_dpp<0xB1>(q);            // (of the neighbour)
             if (live && !(lane & 1)) row[i >> 1] = (uint8_t)(q | (qn << 4));
             if (live && (lane & 31) == 0) scales[i >> 5] = f32_to_f16_bits(d);
         }

@@ -12,6 +12,7 @@
 
 #include "act_math.hpp"
 #include "attn.hpp"
+#include "wave_ops.hpp"
 
 namespace mesh {
 
@@ -31,8 +32,7 @@ __device__ __forceinline__ uint32_t lt_pack(float a, float b) {
     return __builtin_bit_cast(uint32_t, h);
 }
 __device__ __forceinline__ float lt_block_sum(float v, float *scratch) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    v = wave_sum(v);
     __syncthreads();
     if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = v;
     __syncthreads();
@@ -168,8 +168,7 @@ __global__ __launch_bounds__(LT_THREADS) void latent_query_kernel(const LatentSh
             const int r = r0 + u * ROWS + (tid >> 3);
 #pragma unroll
             for (int b = 0; b < TB; ++b) {
-                float v = acc[u][b];
-                v += __shfl_xor(v, 1); v += __shfl_xor(v, 2); v += __shfl_xor(v, 4);
+                const float v = group_sum<8>(acc[u][b]);
                 if (piece == 0 && r < r1 && t0 + b < T) lt_put<ACT>(qa, ((size_t)(t0 + b) * s.heads + h) * s.row() + r, v, c.sat);
             }
         }
@@ -318,8 +317,7 @@ __global__ __launch_bounds__(LT_THREADS) void latent_attn_kernel(const LatentAtt
                 if (k0 + 16 * b + 4 * g + i >= jm) s[b][i] = -INFINITY;
                 mx = fmaxf(mx, s[b][i]);
             }
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        mx = lane_fold<32>(lane_fold<16>(mx, LaneMax{}), LaneMax{});
         // (a token before the group's last may see no key of the split: all is -inf then, and the reference 0 gives zeros)
         const float ref = mx == -INFINITY ? 0.f : mx;
         const float corr = lt_exp2(m - ref);          // exp2(-inf) = 0 the first time
@@ -356,8 +354,7 @@ __global__ __launch_bounds__(LT_THREADS) void latent_attn_kernel(const LatentAtt
         }
         __syncthreads();
     }
-    l += __shfl_xor(l, 16);
-    l += __shfl_xor(l, 32);
+    l = lane_fold<32>(lane_fold<16>(l, LaneAdd{}), LaneAdd{});
     if (h >= heads || !live) return;
     if ((TOK > 1 || wave == 0) && g == 0) { a.ml[prow * 2] = m; a.ml[prow * 2 + 1] = l; }
 #pragma unroll
@@ -377,13 +374,9 @@ __global__ __launch_bounds__(LT_THREADS) void latent_out_kernel(const LatentShap
         const int n_keys = lt_group_keys(a.pos, tg, a.group, T), per = lt_split_keys(n_keys, S), live = (n_keys + per - 1) / per;      // splits that had keys
         const size_t row = (size_t)t * s.heads + h;
         const float m = lane < live ? a.ml[(row * S + lane) * 2] : -INFINITY, l = lane < live ? a.ml[(row * S + lane) * 2 + 1] : 0.f;
-        float mh = m;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) mh = fmaxf(mh, __shfl_xor(mh, o));
+        const float mh = wave_max(m);
         const float w = lane < live ? lt_exp2(m - mh) : 0.f;
-        float den = l * w;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) den += __shfl_xor(den, o);
+        const float den = wave_sum(l * w);
         s_w[b][lane] = w / den;
     }
     __syncthreads();
@@ -452,8 +445,7 @@ __global__ __launch_bounds__(LT_THREADS) void latent_out_kernel(const LatentShap
         for (int u = 0; u < UR; ++u)
 #pragma unroll
             for (int b = 0; b < TB; ++b) {
-                float y = acc[u][b];
-                y += __shfl_xor(y, 1); y += __shfl_xor(y, 2); y += __shfl_xor(y, 4); y += __shfl_xor(y, 8);
+                const float y = group_sum<16>(acc[u][b]);
                 if (piece == 0 && v + u * ROWS < v1 && t0 + b < T) {
                     const size_t at = ((size_t)(t0 + b) * s.heads + h) * s.v_pad + v + u * ROWS;
                     if (a.out_bf16) a.out_bf16[at] = f32_to_bf16_bits(y * gate[b]);

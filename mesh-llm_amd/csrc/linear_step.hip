@@ -15,6 +15,7 @@
 // not depend on timing.
 #include "act_math.hpp"
 #include "linear.hpp"
+#include "wave_ops.hpp"
 
 #include <algorithm>
 
@@ -23,17 +24,8 @@ namespace mesh {
 constexpr int STEP_THREADS = 512, STEP_WAVES = STEP_THREADS / 64;
 constexpr size_t STEP_LDS_MAX = 160 * 1024 - 1024;
 
-// over the wave, in every lane: data-parallel-primitive moves inside a row of 16 lanes (swap neighbours, swap pairs, mirror the
-// 8, mirror the 16), permutes across rows
-__device__ __forceinline__ float step_wave_sum(float v) {
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, false));
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, false));
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xF, 0xF, false));
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xF, 0xF, false));
-    v += __shfl_xor(v, 16);
-    v += __shfl_xor(v, 32);
-    return v;
-}
+// over the wave, in every lane, from the nearest lanes on
+__device__ __forceinline__ float step_wave_sum(float v) { return lane_fold<32>(lane_fold<16>(group_sum<16>(v), LaneAdd{}), LaneAdd{}); }
 // N sums over the workgroup in a fixed order, the same in every thread.  Two sums in a row use different slots: the barrier of the
 // second is what keeps a third from overwriting what the first's readers still need.
 typedef float StepScratch[2][STEP_WAVES][4];

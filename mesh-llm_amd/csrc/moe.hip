@@ -248,10 +248,9 @@ __global__ __launch_bounds__(CHUNK_THREADS) void moe_router_chunk_kernel(const f
 
 // Router logits of a batch of decode steps, a workgroup per token and four experts, one row of the matrix per wave.  The bits of router_logits:
 // the sums of a lane's elements and of the lanes go the same way.  planes (optional): the normalised row as pairs of f16.
-// Bound by its chain (row, sum of squares, dot product).  A CU pulls about 25 GB/s of what is not in its caches, so that a slice should be
-// small: 16 rows of 8 KB a workgroup, every wave its own copy of the token's row, 9.4 us (16 tokens, 64 experts x 2048), all 64 rows 25, four
-// rows 3.6.  (Before, the last of the 16-row workgroups to arrive routed and grouped behind a hand-over between workgroups: 19.4 us in one launch,
-// against 3.6 + 5.6 now.)
+// Bound by its chain (row, sum of squares, dot product).  16 tokens, 64 experts x 2048: 3.6 us; 9.4 with sixteen rows a workgroup, each wave of which
+// loaded and normalised the token's row for itself and added lanes up through the LDS unit.  (Before, the last of those workgroups to
+// arrive routed and grouped behind a hand-over between workgroups: 19.4 us in one launch, against 3.6 + 5.6 now.)
 constexpr int SLICE_THREADS = 256, SLICE_WAVES = SLICE_THREADS / 64;
 template <int NV>
 __global__ __launch_bounds__(SLICE_THREADS) void moe_router_slice_kernel(const float *__restrict__ x, const float *__restrict__ norm_w, const float *__restrict__ W,
@@ -560,13 +559,7 @@ __global__ __launch_bounds__(SORT_THREADS) void moe_sort_kernel(const int32_t *_
         int total = 0;
 #pragma unroll
         for (int k = 0; k < 5; ++k) {
-            int in = mine[k];
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int v = __shfl_up(in, o);
-                if (lane >= o) in += v;
-            }
-            const int sum = __shfl(in, 63);
+            const int in = wave_scan(mine[k]), sum = __builtin_amdgcn_readlane(in, 63);
             base[k] = k < 1 ? 0 : total;
             run[k] = base[k] + in - mine[k];
             if (k == 0) { if (lane == 0) counts[1] = sum; } else total += sum;

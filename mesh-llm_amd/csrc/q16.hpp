@@ -11,14 +11,11 @@ namespace mesh {
 // stores it.  q16: start of the activation buffer (blocks of 16 tokens, 36 K bytes each).
 __device__ __forceinline__ void q16_store_block32(uint8_t *q16, int K, int tok, int kk, float v) {
     float amax = fabsf(v);
-#pragma unroll
-    for (int o = 16; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
+    amax = lanes_fold<16>(amax, LaneMax{});
     const float inv = amax > 0.f ? XQ_LEVELS / amax : 0.f;
     const int q = __float2int_rn(v * inv);
     const int lo = ((q + 128) & 0xFF) - 128, hi = (q - lo) >> 8;
-    int isum = q;
-#pragma unroll
-    for (int o = 16; o > 0; o >>= 1) isum += __shfl_xor(isum, o);
+    const int isum = lanes_fold<16>(q, LaneAdd{});
     uint8_t *yb = q16 + (size_t)(tok >> 4) * ((size_t)K * 36);
     const int t = tok & 15;
     uint8_t *rec = yb + ((size_t)(kk >> 3) * 16 + t) * 16 + (kk & 7);

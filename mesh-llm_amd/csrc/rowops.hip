@@ -4,6 +4,7 @@
 #include "act_math.hpp"
 
 #include "kv_cache.hpp"
+#include "wave_ops.hpp"
 
 namespace mesh {
 
@@ -36,8 +37,7 @@ template <ActType ACT, int V> __device__ __forceinline__ void act_store_row(void
 }
 
 __device__ __forceinline__ float row_sum(float v, float *scratch) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    v = wave_sum(v);
     __syncthreads();
     if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = v;
     __syncthreads();
