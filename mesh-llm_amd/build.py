@@ -18,6 +18,9 @@ FLAGS = [
     # leading scalar kernel arguments arrive in SGPRs at wave start instead of through a scalar load (kernels whose
     # start-up chain matters list those arguments first)
     "-mllvm", "-amdgpu-kernarg-preload-count=14",
+    # results of matrix instructions stay in vector registers: kept in accumulation registers, a kernel that also rescales them
+    # copies them over and back (decode attention: 64 of 92 instructions of a block of keys)
+    "-mllvm", "-amdgpu-mfma-vgpr-form=1",
     "-Wall", "-Wno-unused-function", "-Wno-unknown-warning-option",
 ]
 

@@ -20,7 +20,9 @@
 // Q and the probabilities are rounded to f16 for the matrix cores; sums are f32.
 //
 // What bounds it: the walk of a workgroup is a chain of row loads (29 GB/s per workgroup), beside it the conversion of
-// quantised rows (~430 vector instructions per 32 keys).  Against blocks of 16 keys with V scattered into the transposed
+// quantised rows (~300 vector instructions per 32 keys; ~490 with the results in
+// accumulation registers and nibbles masked and biased apart, which took 206 registers for 166 and was two waves a SIMD for three:
+// 60.7 -> 54.6 us, 32 sequences of 2000 to 6000 keys, 8 heads, q8_0 / q4_0).  Against blocks of 16 keys with V scattered into the transposed
 // tile by 32 two-byte stores a lane: 64.4 -> 55.9 us (32 sequences of 2000 to 6000 keys, 8 heads, q8_0 / q4_0: 213 MB),
 // 17.4 -> 15.4 (16 sequences, 4 heads), f16 rows 41.4 -> 39.5 (16 sequences, 179 MB: 4.5 TB/s), 7.3 -> 6.8 (one); f16 rows and whole
 // lines of V (ValueBlock) against those blocks of 16 keys, 8 heads of 128, 4000 keys, with the merge: 64 sequences 177 -> 177, 33 140 -> 129,
@@ -108,9 +110,12 @@ struct RowShare {
                              mm_scale_pair(__builtin_amdgcn_perm(0x64646464u, b, 0x04010400u), 1024.f + 128.f, d2),
                              mm_scale_pair(__builtin_amdgcn_perm(0x64646464u, b, 0x04030402u), 1024.f + 128.f, d2)};
             } else {
+                // (masks in scalar registers and biases in vector ones: the form one v_and_or_b32 takes, which reads one scalar)
+                uint32_t lo = 0x000F000Fu, hi = 0x00F000F0u, lo_bias = 0x64006400u, hi_bias = 0x54005400u;
+                asm("" : "+s"(lo), "+s"(hi), "+v"(lo_bias), "+v"(hi_bias));
                 const uint32_t x = w[cc], y = x >> 8;
-                return mm_u4{mm_scale_pair((x & 0x000F000Fu) | 0x64006400u, 1024.f + 8.f, d2), mm_scale_pair((x & 0x00F000F0u) | 0x54005400u, 64.f + 8.f, d2),
-                             mm_scale_pair((y & 0x000F000Fu) | 0x64006400u, 1024.f + 8.f, d2), mm_scale_pair((y & 0x00F000F0u) | 0x54005400u, 64.f + 8.f, d2)};
+                return mm_u4{mm_scale_pair((x & lo) | lo_bias, 1024.f + 8.f, d2), mm_scale_pair((x & hi) | hi_bias, 64.f + 8.f, d2),
+                             mm_scale_pair((y & lo) | lo_bias, 1024.f + 8.f, d2), mm_scale_pair((y & hi) | hi_bias, 64.f + 8.f, d2)};
             }
         }
     }
@@ -262,14 +267,15 @@ __global__ __launch_bounds__(MMA_THREADS) void attn_mma_kernel(const float *p_q,
         // of one block save the fetch)
         if (DEPTH > 1 || kb + DEPTH * STEP < j1) fetch(kr, vr, kb + DEPTH * STEP);
 
-        float mx = -INFINITY;
+        if (kb + MMA_KEYS > j1) {       // the range's last, shorter block
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+            for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                s[h][i] = kb + 16 * h + 4 * g + i < j1 ? s[h][i] : -INFINITY;
-                mx = fmaxf(mx, s[h][i]);
-            }
+                for (int i = 0; i < 4; ++i) s[h][i] = kb + 16 * h + 4 * g + i < j1 ? s[h][i] : -INFINITY;
+        }
+        float mx = s[0][0];
+#pragma unroll
+        for (int i = 1; i < 8; ++i) mx = fmaxf(mx, s[i >> 2][i & 3]);
         mx = lane_fold<32>(lane_fold<16>(mx, LaneMax{}), LaneMax{});
         // The reference point m of the exponentials only moves when a score exceeds it by more than 2^RESCALE_STEP
         // (probabilities then stay below that factor, harmless in f16 / f32), and then for the whole wave at once:
