@@ -48,6 +48,7 @@ struct AttnArgs {
     int window = 0;                // token t sees the positions (pos[t] - window, pos[t]]; 0: all of [0, pos[t]]
     float scale = 1.f;
     int n_head = 0, n_kv = 0, group = 1, head_dim = 0, n_ctx = 0, n_splits = 1;
+    int max_keys = 0;              // keys of the call's longest walk, as far as known (0: not); only decides between kernels
     // attention_chunk only: entries of a value row and of an output head (0: head_dim), and a gate per head, [T][gate_ld], whose
     // sigmoid multiplies the output (bf16 rows)
     int v_dim = 0;

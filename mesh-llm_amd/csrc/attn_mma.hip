@@ -14,7 +14,7 @@
 //   O^T (16 dims x 16 heads) += V^T . P^T     v_mfma_f32_16x16x32_f16 per 16 dims and 32 keys; the result registers of
 //                                             S^T (4 keys of one head per lane and half) are the P^T operand as they are;
 //                                             V^T needs the keys along a lane: V rows pass a wave-private LDS tile as
-//                                             they are, and ds_read_b64_tr_b16 hands them back transposed
+//                                             they are (long walks of f16: K rows too), and ds_read_b64_tr_b16 hands them back transposed
 // A lane owns one head column throughout: the softmax maximum is a reduction over its 8 registers and the 4 lane
 // groups, the rescale of O is a per-lane scalar, and its share of the sum meets the others' once, at the end.
 // Q and the probabilities are rounded to f16 for the matrix cores; sums are f32.
@@ -25,13 +25,15 @@
 // 60.7 -> 54.6 us, 32 sequences of 2000 to 6000 keys, 8 heads, q8_0 / q4_0).  Against blocks of 16 keys with V scattered into the transposed
 // tile by 32 two-byte stores a lane: 64.4 -> 55.9 us (32 sequences of 2000 to 6000 keys, 8 heads, q8_0 / q4_0: 213 MB),
 // 17.4 -> 15.4 (16 sequences, 4 heads), f16 rows 41.4 -> 39.5 (16 sequences, 179 MB: 4.5 TB/s), 7.3 -> 6.8 (one); f16 rows and whole
-// lines of V (ValueBlock) against those blocks of 16 keys, 8 heads of 128, 4000 keys, with the merge: 64 sequences 177 -> 177, 33 140 -> 129,
+// lines of V (RowBlock) against those blocks of 16 keys, 8 heads of 128, 4000 keys, with the merge: 64 sequences 177 -> 177, 33 140 -> 129,
 // 20 69 -> 59, 5 23.6 -> 22.6, one 11.5 -> 10.9; of 64: 128 sequences 180 -> 172, 33 62 -> 62, 40 66 -> 69, 20 49 -> 33.
 
 #include "attn.hpp"
 #include "lds_ops.hpp"
 #include "q16.hpp"
 #include "wave_ops.hpp"
+
+#include <type_traits>
 
 namespace mesh {
 
@@ -122,13 +124,11 @@ struct RowShare {
     // first dim of piece cc
     static __device__ __forceinline__ int dim0(int cc, int g) { return TYPE == MESH_F16 ? 32 * cc + 8 * g : HD / 4 * g + 8 * cc; }
 };
-// What a lane holds of the value rows of a 32-key block on their way to the wave's LDS tile [key][dim]; rows past the range are
-// clamped to its last key (their probabilities are zero).  Quantised rows: a lane's shares of rows c and 16 + c, as above.  f16 rows
-// pass as they are, so a load takes whole rows: the 16 lanes that the memory pipe works on at a time lie in two cache lines instead
-// of 16.  Looking lines up is what bounds a CU that walks two ranges at once: 33 sequences of 4000 keys, 8 KV heads, as shares of
-// rows / whole rows 69.5 / 61.9 us (rows of 64), 143 / 129 (128); 16 sequences 29.3 / 29.1 and 52.1 / 51.6.
+// What a lane holds of the rows of a 32-key block; rows past the range are clamped to its last key (the scores are masked, the
+// probabilities zero).
+// A lane's shares of rows c and 16 + c, as above:
 template <int TYPE, int HD, int PITCH>
-struct ValueBlock {
+struct ShareBlock {
     RowShare<TYPE, HD> r[2];
     __device__ __forceinline__ void load(const uint8_t *rows, int kb, int j1, int lane) {
 #pragma unroll
@@ -146,8 +146,14 @@ struct ValueBlock {
                 *reinterpret_cast<mm_u4 *>(tile + (16 * h + (lane & 15)) * PITCH + RowShare<TYPE, HD>::dim0(cc, lane >> 4)) = r[h].piece(cc);
     }
 };
+// Whole rows on their way to the wave's LDS tile [key][dim], for f16 rows, which pass as they are: the 16 lanes that the memory pipe
+// works on at a time lie in two cache lines instead of 16.  Lines that one load takes whole and nothing reads again need no place in
+// the caches, and memory gives more without them (a plain walk of 140 MB: 5.7 TB/s, and 6.2 with the hint; of lines taken in halves
+// the hint makes it less).  V / K rows read so, us, 8 KV heads, rows of 128: 32 sequences of 4090 keys 92.1 as shares of rows, 81.5
+// with V, 81.9 with V and K whole; 32 of 1400 to 4090 69.1, 63.6, 60.2; 16 of 4090 49.2, 44.7, 43.5; 16 of 1400 to 4090 40.0, 37.5,
+// 34.7; 5 of 1000 to 3000 12.8, 12.1, 12.0.
 template <int HD, int PITCH>
-struct ValueBlock<MESH_F16, HD, PITCH> {
+struct RowBlock {
     static constexpr int PIECES = HD / 8, ROWS = 64 / PIECES;       // 16-byte pieces of a row, rows of a load
     mm_u4 v[MMA_KEYS / ROWS];
     __device__ __forceinline__ void load(const uint8_t *rows, int kb, int j1, int lane) {
@@ -155,7 +161,7 @@ struct ValueBlock<MESH_F16, HD, PITCH> {
         for (int i = 0; i < MMA_KEYS / ROWS; ++i) {
             int key = kb + i * ROWS + lane / PIECES;
             key = key < j1 ? key : j1 - 1;
-            v[i] = *reinterpret_cast<const mm_u4 *>(rows + (size_t)key * (HD * 2) + lane % PIECES * 16);
+            v[i] = __builtin_nontemporal_load(reinterpret_cast<const mm_u4 *>(rows + (size_t)key * (HD * 2) + lane % PIECES * 16));
         }
     }
     __device__ __forceinline__ void put(_Float16 *tile, int lane) const {
@@ -173,9 +179,11 @@ __device__ __forceinline__ void mm_wave_lds_sync() {
 }
 
 // grid (n_splits, n_kv, T), 256 threads.  group <= 16.
+// KROWS: K rows of f16 come whole, through the tile that V takes afterwards (RowBlock), else as shares, which a walk of one block a
+// wave has sooner (one token, 4090 keys over 32 splits: 6.4 us, and 6.6 with whole rows).
 // (the arguments on the way to the first K / V loads come first, as scalars, so that they are preloaded into SGPRs:
 // see gemv.hip)
-template <int HD, int KT, int VT>
+template <int HD, int KT, int VT, bool KROWS>
 __global__ __launch_bounds__(MMA_THREADS) void attn_mma_kernel(const float *p_q, const int32_t *p_pos, const int32_t *p_seq,
                                                                const uint8_t *p_kcache, const uint8_t *p_vcache, int p_n_splits,
                                                                int p_n_ctx, int p_n_kv, int p_group, int p_n_head, float p_scale, int p_window,
@@ -229,15 +237,12 @@ __global__ __launch_bounds__(MMA_THREADS) void attn_mma_kernel(const float *p_q,
     // last key, and masked below), and of the value rows
     constexpr int STEP = MMA_WAVES * MMA_KEYS;
     constexpr int DEPTH = KT == MESH_F16 && VT == MESH_F16 ? MMA_DEPTH_F16 : MMA_DEPTH_Q;
-    RowShare<KT, HD> krs[DEPTH][2];
-    ValueBlock<VT, HD, VPITCH> vrs[DEPTH];
-    auto fetch = [&](RowShare<KT, HD> (&kr)[2], ValueBlock<VT, HD, VPITCH> &vr, int kb) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            int key = kb + 16 * h + c;
-            key = key < j1 ? key : j1 - 1;
-            kr[h].load(p_kcache + (base + key) * KRB, g);
-        }
+    typedef typename std::conditional<KROWS, RowBlock<HD, VPITCH>, ShareBlock<KT, HD, VPITCH>>::type KBlock;
+    typedef typename std::conditional<VT == MESH_F16, RowBlock<HD, VPITCH>, ShareBlock<VT, HD, VPITCH>>::type VBlock;
+    KBlock krs[DEPTH];
+    VBlock vrs[DEPTH];
+    auto fetch = [&](KBlock &kr, VBlock &vr, int kb) {
+        kr.load(p_kcache + base * KRB, kb, j1, lane);
         vr.load(p_vcache + base * VRB, kb, j1, lane);
     };
     const int kb0 = j0 + __builtin_amdgcn_readfirstlane(wave) * MMA_KEYS;
@@ -250,16 +255,23 @@ __global__ __launch_bounds__(MMA_THREADS) void attn_mma_kernel(const float *p_q,
       for (int d = 0; d < DEPTH; ++d) {
         const int kb = kbb + d * STEP;
         if (kb >= j1) break;
-        RowShare<KT, HD> (&kr)[2] = krs[d];
-        ValueBlock<VT, HD, VPITCH> &vr = vrs[d];
+        KBlock &kr = krs[d];
+        VBlock &vr = vrs[d];
         // S^T = K . Q^T : register i of half h is key kb + 16 h + 4 g + i for head c
         mm_f4 s[2];
+        if constexpr (KROWS) { kr.put(sV, lane); mm_wave_lds_sync(); }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             s[h] = mm_f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int cc = 0; cc < NC; ++cc) s[h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(mm_h8, kr[h].piece(cc)), qf[cc], s[h], 0, 0, 0);
+            for (int cc = 0; cc < NC; ++cc) {
+                mm_u4 kp;
+                if constexpr (KROWS) kp = *reinterpret_cast<const mm_u4 *>(sV + (16 * h + c) * VPITCH + RowShare<KT, HD>::dim0(cc, g));
+                else kp = kr.r[h].piece(cc);
+                s[h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(mm_h8, kp), qf[cc], s[h], 0, 0, 0);
+            }
         }
+        if constexpr (KROWS) mm_wave_lds_sync();
         // V rows as they are: sV[key][dim]
         vr.put(sV, lane);
         // rows of a later block travel while this one is worked on (two blocks deep without a branch: the compiler then
@@ -356,12 +368,21 @@ __global__ __launch_bounds__(MMA_THREADS) void attn_mma_kernel(const float *p_q,
     }
 }
 
+template <int HD, int KT, int VT, bool KROWS>
+static void launch_mma_as(const AttnArgs &a, int T, hipStream_t stream) {
+    MESH_LAUNCH((attn_mma_kernel<HD, KT, VT, KROWS>), dim3((unsigned)a.n_splits, (unsigned)a.n_kv, (unsigned)T), dim3(MMA_THREADS), 0, stream, a.q, a.pos, a.seq, a.kcache, a.vcache, a.n_splits,
+                a.n_ctx, a.n_kv, a.group, a.n_head, a.scale, a.window, a);
+}
+
 template <int HD>
 static int launch_mma(const AttnArgs &a, int T, hipStream_t stream) {
-    const dim3 grid((unsigned)a.n_splits, (unsigned)a.n_kv, (unsigned)T), block(MMA_THREADS);
-    if (a.k_type == MESH_F16 && a.v_type == MESH_F16) MESH_LAUNCH((attn_mma_kernel<HD, MESH_F16, MESH_F16>), grid, block, 0, stream, a.q, a.pos, a.seq, a.kcache, a.vcache, a.n_splits, a.n_ctx, a.n_kv, a.group, a.n_head, a.scale, a.window, a);
-    else if (a.k_type == MESH_Q8_0 && a.v_type == MESH_Q4_0) MESH_LAUNCH((attn_mma_kernel<HD, MESH_Q8_0, MESH_Q4_0>), grid, block, 0, stream, a.q, a.pos, a.seq, a.kcache, a.vcache, a.n_splits, a.n_ctx, a.n_kv, a.group, a.n_head, a.scale, a.window, a);
-    else if (a.k_type == MESH_Q4_0 && a.v_type == MESH_Q4_0) MESH_LAUNCH((attn_mma_kernel<HD, MESH_Q4_0, MESH_Q4_0>), grid, block, 0, stream, a.q, a.pos, a.seq, a.kcache, a.vcache, a.n_splits, a.n_ctx, a.n_kv, a.group, a.n_head, a.scale, a.window, a);
+    if (a.k_type == MESH_F16 && a.v_type == MESH_F16) {
+        // one block of keys a wave at most (attn_mma_kernel, KROWS)
+        const bool one_block = a.max_keys > 0 && a.max_keys <= a.n_splits * MMA_WAVES * MMA_KEYS;
+        if (one_block) launch_mma_as<HD, MESH_F16, MESH_F16, false>(a, T, stream);
+        else launch_mma_as<HD, MESH_F16, MESH_F16, true>(a, T, stream);
+    } else if (a.k_type == MESH_Q8_0 && a.v_type == MESH_Q4_0) launch_mma_as<HD, MESH_Q8_0, MESH_Q4_0, false>(a, T, stream);
+    else if (a.k_type == MESH_Q4_0 && a.v_type == MESH_Q4_0) launch_mma_as<HD, MESH_Q4_0, MESH_Q4_0, false>(a, T, stream);
     else return fail(MESH_ERR_UNSUPPORTED, "attention_mma: KV cache types %d/%d", a.k_type, a.v_type);
     MESH_LAUNCH_CHECK();
     return MESH_OK;

@@ -174,6 +174,7 @@ static int run_attention(mesh_session *s, size_t il, int T, int max_keys, bool f
     aa.scale = m.scale;
     aa.n_head = m.heads; aa.n_kv = m.kv_heads; aa.group = m.heads / m.kv_heads; aa.head_dim = L.head_pad; aa.n_ctx = st->n_ctx;
     aa.n_splits = layer_splits(s, m, T, max_keys);
+    aa.max_keys = keys_seen(m, max_keys);
     ProfScope ps(s, MESH_PROF_ATTN);
     if (hm.act == ACT_F32) return attention(aa, T, s->stream);
     if (T >= s->tune.gemm_min_tokens && s->chunk_pos0 >= 0 && L.head_pad <= 128) {

@@ -832,7 +832,7 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
     aa.part = s->attn_part; aa.ml = s->attn_ml; aa.out = s->attn;
     aa.scale = 1.0f / sqrtf((float)hp.head_dim);
     aa.n_head = (int)hp.n_head; aa.n_kv = (int)hp.n_head_kv; aa.group = (int)(hp.n_head / hp.n_head_kv);
-    aa.head_dim = (int)hp.head_dim; aa.n_ctx = st->n_ctx;
+    aa.head_dim = (int)hp.head_dim; aa.n_ctx = st->n_ctx; aa.max_keys = max_keys;
     aa.n_splits = T < 64 ? attn_splits_for(s->tune, T, (int)hp.n_head_kv, max_keys, st->k_type != MESH_F16) : 1;     // a batch of decode steps still splits the long KV
     {
         ProfScope ps(s, MESH_PROF_ATTN);
@@ -1089,7 +1089,7 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
         aa.part = s->attn_part; aa.ml = s->attn_ml; aa.out = s->attn;
         aa.scale = 1.0f / sqrtf((float)hp.head_dim);
         aa.n_head = (int)hp.n_head; aa.n_kv = (int)hp.n_head_kv; aa.group = (int)(hp.n_head / hp.n_head_kv);
-        aa.head_dim = (int)hp.head_dim; aa.n_ctx = st->n_ctx;
+        aa.head_dim = (int)hp.head_dim; aa.n_ctx = st->n_ctx; aa.max_keys = max_keys;
         aa.n_splits = attn_splits_for(s->tune, T, (int)hp.n_head_kv, max_keys, st->k_type != MESH_F16);
         {
             ProfScope ps(s, MESH_PROF_ATTN);
@@ -1604,7 +1604,7 @@ int session_attention(mesh_session *s, int layer, const float *d_q, const mesh_b
     aa.part = s->attn_part; aa.ml = s->attn_ml; aa.out = d_out;
     aa.scale = 1.0f / sqrtf((float)hp.head_dim);
     aa.n_head = (int)hp.n_head; aa.n_kv = (int)hp.n_head_kv; aa.group = (int)(hp.n_head / hp.n_head_kv);
-    aa.head_dim = (int)hp.head_dim; aa.n_ctx = st->n_ctx;
+    aa.head_dim = (int)hp.head_dim; aa.n_ctx = st->n_ctx; aa.max_keys = max_keys;
     aa.n_splits = T < 64 ? attn_splits_for(s->tune, T, (int)hp.n_head_kv, max_keys, st->k_type != MESH_F16) : 1;
     if (matrix_cores) {
         if (!attention_mma_supported(aa)) return fail(MESH_ERR_UNSUPPORTED, "mesh_session_attn_dev: the matrix-core kernel does not cover this shape");

@@ -55,3 +55,37 @@ def test_key_block_edges(tmp_path, name, kv_types):
             assert rel <= TOL, (name, kv_types, KEYS[i], len(batch), rel)
     ses.close()
     st.close()
+
+
+@pytest.mark.parametrize("splits", [1, 2, 3])
+@pytest.mark.parametrize("name", ["tiny-llama", "tiny-g5"])
+def test_walks_of_more_than_one_block_a_wave(tmp_path, name, splits):
+    """f16 rows beyond 128 keys a split come as whole rows of K (of one block a wave as shares of rows)."""
+    m, cfg = mesh(), models.CONFIGS[name]
+    path = os.path.join(str(tmp_path), name + ".gguf")
+    models.write_model(path, cfg, [0], seed=4)
+    H, HK, D = cfg["n_head"], cfg["n_head_kv"], cfg["head_dim"]
+    keys = [128 * splits + 1, 128 * splits + 31, 1, 256 * splits, 256 * splits + 1, 33, 129]
+    st = m.Stage(path, 0, 1, n_ctx=max(keys), n_seq_max=len(keys), n_batch_max=32, kv_types=TIERS[0])
+    rng = np.random.Generator(np.random.PCG64(10))
+    ses = st.session(attn_split_target=splits * HK * len(keys))
+    for i, n in enumerate(keys):
+        k, v = rng.standard_normal((max(keys), HK, D)), rng.standard_normal((max(keys), HK, D))
+        k[n:], v[n:] = 50.0, 1000.0
+        ses.kv_write(0, i, 0, k.astype(np.float16).view(np.uint16), v.astype(np.float16).view(np.uint16))
+    q = rng.standard_normal((len(keys), H, D)).astype(np.float32) * 1.5
+    qd = torch.from_numpy(q).cuda()
+    out = torch.full_like(qd, float("nan"))
+    torch.cuda.synchronize()
+    ses.attn_dev(0, qd.data_ptr(), [n - 1 for n in keys], out.data_ptr(), seq=list(range(len(keys))))
+    ses.synchronize()
+    got = out.cpu().numpy().astype(np.float64)
+    for i, n in enumerate(keys):
+        kd, vd = (r.view(np.float16).astype(np.float64).repeat(H // HK, axis=1) for r in ses.kv_read(0, i, 0, n))
+        s = np.einsum("hd,nhd->hn", q[i].astype(np.float64), kd) / np.sqrt(D)
+        p = np.exp(s - s.max(1, keepdims=True))
+        want = np.einsum("hn,nhd->hd", p / p.sum(1, keepdims=True), vd)
+        rel = np.linalg.norm(got[i] - want) / np.linalg.norm(want)
+        assert rel <= TOL, (name, splits, n, rel)
+    ses.close()
+    st.close()
