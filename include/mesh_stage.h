@@ -296,7 +296,7 @@ int mesh_session_f16_saturations(mesh_session *session, uint64_t *count);
  *     gemm_narrow=1        tiles of 32 or 64 tokens for calls of at most 64, where gemm_big does not take the projection
  *     attn_chunk_ksplit=1  a prefill chunk's key walks split over workgroups when the grid would not fill the chip
  *     attn_mma_min_tokens=1  decode attention on the matrix cores from this many tokens
- *     attn_split_target=0  workgroups a decode attention launch aims at (0 = 256, or 512 for quantised rows)
+ *     attn_split_target=0  workgroups a decode attention launch aims at (0 = by the call's sizes)
  *     moe_group=1          (token, slot) pairs grouped by expert
  *     moe_router_tail=1    no effect; accepted from callers that set it
  *     moe_fuse_quant=1     the expert combine step quantises for the next layer

@@ -8,6 +8,7 @@ namespace mesh {
 
 constexpr int ROPE_MODE_NORM = 0, ROPE_MODE_NEOX = 2;
 constexpr int ATTN_SPLITS_CAP = 64;     // most KV splits per (token, kv head)
+constexpr int ATTN_PART_ROWS_MIN = 768; // (token, split) rows that the partial buffers of a session hold at least
 
 struct RopeKvArgs {
     float *q = nullptr;            // [T][n_head][head_dim], rotated in place

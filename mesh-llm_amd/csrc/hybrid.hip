@@ -122,8 +122,12 @@ bool hybrid_single_step(const mesh_session *s, int T) { return T == 1 && s->tune
 
 static int keys_seen(const MixerSpec &m, int max_keys) { return m.window > 0 ? std::min(m.window, max_keys) : max_keys; }
 
-static int layer_splits(const mesh_session *s, const MixerSpec &m, int T, int max_keys) {
-    return T < 64 ? attn_splits_for(s->tune, T, m.kv_heads, keys_seen(m, max_keys), false) : 1;
+static int layer_splits(const mesh_session *s, const HybridLayer &L, int T, int max_keys) {
+    const MixerSpec &m = L.spec.mixer;
+    AttnArgs a;
+    a.k_type = s->stage->k_type; a.v_type = s->stage->v_type;
+    a.n_kv = m.kv_heads; a.group = m.heads / m.kv_heads; a.head_dim = L.head_pad; a.max_keys = keys_seen(m, max_keys);
+    return T < 64 ? attn_splits_for(s->tune, a, T) : 1;
 }
 
 // (the partial sums have room for 1024 (token, split) rows at least)
@@ -135,7 +139,7 @@ uint64_t hybrid_graph_key(const mesh_session *s, int T, int max_keys) {
     uint64_t key = 1469598103934665603ull ^ (uint64_t)T;
     auto mix = [&](uint64_t v) { key = (key ^ v) * 1099511628211ull; };
     for (const HybridLayer &L : s->stage->hybrid->layers) {
-        if (L.spec.mixer.kind == MIXER_ATTENTION) mix((uint64_t)layer_splits(s, L.spec.mixer, T, max_keys));
+        if (L.spec.mixer.kind == MIXER_ATTENTION) mix((uint64_t)layer_splits(s, L, T, max_keys));
         if (L.spec.mixer.kind == MIXER_LATENT) mix((uint64_t)latent_layer_splits(s, L.latent, T, max_keys) << 1 | (s->chunk_pos0 >= 0 ? 1 : 0));
     }
     mix(s->stage->copies.present() ? 1 : 0);
@@ -173,7 +177,7 @@ static int run_attention(mesh_session *s, size_t il, int T, int max_keys, bool f
     aa.window = m.window;
     aa.scale = m.scale;
     aa.n_head = m.heads; aa.n_kv = m.kv_heads; aa.group = m.heads / m.kv_heads; aa.head_dim = L.head_pad; aa.n_ctx = st->n_ctx;
-    aa.n_splits = layer_splits(s, m, T, max_keys);
+    aa.n_splits = layer_splits(s, L, T, max_keys);
     aa.max_keys = keys_seen(m, max_keys);
     ProfScope ps(s, MESH_PROF_ATTN);
     if (hm.act == ACT_F32) return attention(aa, T, s->stream);

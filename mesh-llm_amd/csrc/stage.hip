@@ -402,8 +402,6 @@ int sess_alloc(mesh_session *s, void **p, size_t bytes) {
     return MESH_OK;
 }
 
-constexpr int ATTN_SPLITS_MAX = ATTN_SPLITS_CAP;
-constexpr int ATTN_PART_ROWS_MIN = 512;     // rows of (token, split) the partial buffers always hold
 constexpr int META_SLOTS = 8;
 // positions, sequence ids, token ids, wanted rows; chunk tables (hybrid_chunk_table)
 static constexpr size_t META_INTS(size_t B) { return 7 * B + 2; }
@@ -588,23 +586,35 @@ static GemvMat mat_of(const DevTensor &w, float *y, int ldy, const DevTensor *bi
 // Batches of at least attn_mma_min_tokens tokens take the matrix-core decode attention (Q and the probabilities rounded
 // to f16; faster at every batch size, so the default is 1).  Callers that want the all-f32 vector-ALU kernel at small
 // batches raise it.
-// quantised: the cache rows are q8_0 / q4_0
-int attn_splits_for(const Tuning &tune, int T, int n_kv, int max_keys, bool quantised) {
-    // One workgroup per compute unit (256 on gfx950) measured best from batch 1 to 16 with f16 rows, which that many
-    // workgroups stream at the memory's rate.  Quantised rows are bound by the instructions that decode them, and two
-    // workgroups per CU hide each other's waits: 3-7% of the step at batch 8-32 (Qwen2.5-32B shape, q8_0 / q4_0 cache:
-    // 9.86 -> 9.18 ms at batch 32, which otherwise runs unsplit); four per CU lose again, and so do 64 splits of a single
-    // token's walk (from 64 (token, KV head) pairs on).  (Those of a kernel whose waves took 16 keys a step.)
-    // 64 keys a split at least, which gives two of the matrix-core kernel's four waves work (32 keys a wave step); against 128 keys,
-    // attention and merge, us, 8 KV heads, f16 rows: one token 128 keys 7.8 / 6.6 (unsplit), 256 8.4 / 8.7, 400 9.4 / 9.1, 512 7.8 /
-    // 9.3, 1000 8.3 / 8.8, 2000 9.4 / 9.2; 5 tokens 128 8.1 / 5.8, 256 8.8 / 8.9, 512 11.0 / 9.6, from 700 on the same splits; 16 tokens
-    // 128 8.6 / 6.2, from 192 on the same; q8_0 / q4_0 rows 128 8.4 / 6.6, 512 8.0 / 9.1, 1000 8.6 / 8.5 (one token).
+int attn_splits_for(const Tuning &tune, const AttnArgs &a, int T) {
+    const int pairs = std::max(1, T * a.n_kv), keys = a.max_keys;
+    // (the partial sums have room for so many (token, split) rows)
+    const int cap = std::max(1, std::min({ATTN_SPLITS_CAP, (keys + 63) / 64, ATTN_PART_ROWS_MIN / std::max(1, T)}));
     // (attn_split_target: the workgroup count aimed at, for experiments)
-    const int forced = tune.attn_split_target;
-    const int target = forced ? forced : (quantised && T * n_kv >= 64) ? 512 : 256;
-    int s = target / std::max(1, T * n_kv);
-    s = std::min(s, (max_keys + 63) / 64);
-    return std::max(1, std::min(s, ATTN_SPLITS_MAX));
+    if (tune.attn_split_target) return std::max(1, std::min(tune.attn_split_target / pairs, cap));
+    const bool quantised = a.k_type == MESH_Q8_0 || a.k_type == MESH_Q4_0;
+    const int one = std::max(1, 256 / pairs), two = std::max(1, 512 / pairs), three = std::max(1, 768 / pairs);     // one, two, three workgroups a CU
+    // the f32 kernel: quantised rows cost it instructions, and a second workgroup on a CU hides their waits
+    if (T < tune.attn_mma_min_tokens || !attention_mma_supported(a)) return std::min(quantised && pairs >= 64 ? two : one, cap);
+    // The matrix-core kernel (us, attention and merge, 8 KV heads of 128, the longest sequence and the others from a third of it on).
+    // A merge costs 2 to 4 us and a launch, so short walks stay whole, and the fewer splits there are the longer.  One split / one
+    // workgroup a CU: 2 tokens, f16 rows, 100 keys 5.7 / 6.8, 250 6.6 / 7.0, 400 8.5 / 7.0; 8 tokens (4 splits) 200 7.3 / 7.3, 350
+    // 8.8 / 7.9, 500 9.2 / 8.5; 10 (3) 500 9.3 / 9.5, 750 11.5 / 9.8; 16 (2) 1000 14.5 / 16.4, 1500 19.3 / 20.4, 2200 26.8 / 25.8;
+    // q8_0 / q4_0 rows, 5 tokens 250 6.7 / 7.2, 500 8.7 / 7.8; 16 (2) 750 10.9 / 12.0, 1000 12.8 / 14.9, 1500 16.9 / 16.2.
+    if (one >= 2) {
+        const int whole = one >= 4 ? 384 : one == 3 ? 512 : quantised ? 1024 : 1536;
+        if (keys <= whole) return 1;
+        // f16 rows come at the memory's rate with one workgroup a CU; decoding quantised rows takes two from about a thousand keys a
+        // split on (16 tokens, 2 and 4 splits: 1500 keys 16.2 / 16.1, 2200 19.6 / 19.5, 4000 27.4 / 24.5, 6000 37.4 / 33.2)
+        return std::min(quantised && keys >= 960 * one ? two : one, cap);
+    }
+    // More than half the CUs have a walk of their own.  f16 rows then stay whole (20 tokens, 1 and 3 splits, 1000 keys 15.2 / 18.5,
+    // 4090 47.4 / 48.2; 28 tokens 4090 keys 56.1 / 59.5 with 2).  Quantised rows are split from 16 keys for each (token, head) pair on:
+    // 18 tokens (3 splits) 1500 keys 17.0 / 17.7, 2200 23.7 / 21.4, 4000 39.3 / 29.5; 28 (2) 3000 32.0 / 32.8, 4000 40.4 / 35.4; 32
+    // (2) 3000 33.0 / 33.4, 6000 58.6 / 50.5; into whatever fills two or three workgroups a CU better (24 tokens, 2 and 4 splits: 3000
+    // keys 30.5 / 27.5, 6000 47.1 / 44.9).
+    if (!quantised || pairs > 256 || keys < 16 * pairs) return 1;
+    return std::min(3 * two >= 2 * three ? two : three, cap);
 }
 
 // ---- optional timing -----------------------------------------------------------------------------
@@ -833,7 +843,7 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
     aa.scale = 1.0f / sqrtf((float)hp.head_dim);
     aa.n_head = (int)hp.n_head; aa.n_kv = (int)hp.n_head_kv; aa.group = (int)(hp.n_head / hp.n_head_kv);
     aa.head_dim = (int)hp.head_dim; aa.n_ctx = st->n_ctx; aa.max_keys = max_keys;
-    aa.n_splits = T < 64 ? attn_splits_for(s->tune, T, (int)hp.n_head_kv, max_keys, st->k_type != MESH_F16) : 1;     // a batch of decode steps still splits the long KV
+    aa.n_splits = T < 64 ? attn_splits_for(s->tune, aa, T) : 1;     // a batch of decode steps still splits the long KV
     {
         ProfScope ps(s, MESH_PROF_ATTN);
         if (!skinny && s->chunk_pos0 >= 0 && hp.head_dim == 128) {
@@ -1090,7 +1100,7 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
         aa.scale = 1.0f / sqrtf((float)hp.head_dim);
         aa.n_head = (int)hp.n_head; aa.n_kv = (int)hp.n_head_kv; aa.group = (int)(hp.n_head / hp.n_head_kv);
         aa.head_dim = (int)hp.head_dim; aa.n_ctx = st->n_ctx; aa.max_keys = max_keys;
-        aa.n_splits = attn_splits_for(s->tune, T, (int)hp.n_head_kv, max_keys, st->k_type != MESH_F16);
+        aa.n_splits = attn_splits_for(s->tune, aa, T);
         {
             ProfScope ps(s, MESH_PROF_ATTN);
             rc = T >= s->tune.attn_mma_min_tokens && attention_mma_supported(aa) ? attention_mma(aa, T, stream) : attention(aa, T, stream);
@@ -1310,6 +1320,12 @@ static int validate_batch(const mesh_session *s, const mesh_batch *b, int *max_k
 // finishes every lazy initialisation), the second is captured, later ones are replays.
 constexpr int GRAPH_MAX_TOKENS = 32;
 constexpr size_t GRAPH_MAX_ENTRIES = 96;
+static AttnArgs attn_shape(const mesh_stage *st, int max_keys) {
+    AttnArgs a;
+    a.k_type = st->k_type; a.v_type = st->v_type;
+    a.n_kv = (int)st->hp.n_head_kv; a.group = (int)(st->hp.n_head / st->hp.n_head_kv); a.head_dim = (int)st->hp.head_dim; a.max_keys = max_keys;
+    return a;
+}
 static int run_layers_graphed(mesh_session *s, int T, int max_keys) {
     if (!s->tune.graphs || s->graphs_failed || s->profile || T > GRAPH_MAX_TOKENS) return run_layers(s, T, max_keys);
     // A prefill chunk (consecutive positions of one sequence, enough tokens for the large-tile GEMM) runs the chunk
@@ -1317,7 +1333,7 @@ static int run_layers_graphed(mesh_session *s, int T, int max_keys) {
     // chunk's.  Such calls are always launched eagerly.
     const mesh_stage *st = s->stage;
     if (s->chunk_pos0 >= 0 && (T >= PREFILL_MIN_TOKENS || (st->hybrid && T >= s->tune.latent_chunk_min_tokens))) return run_layers(s, T, max_keys);
-    const int n_splits = st->hybrid ? 0 : attn_splits_for(s->tune, T, (int)st->hp.n_head_kv, max_keys, st->k_type != MESH_F16);
+    const int n_splits = st->hybrid ? 0 : attn_splits_for(s->tune, attn_shape(st, max_keys), T);
     const uint64_t key = st->hybrid ? hybrid_graph_key(s, T, max_keys) : (uint64_t)T | ((uint64_t)n_splits << 8) | ((uint64_t)(s->expert_mask_on ? 1 : 0) << 20) | ((uint64_t)(st->copies.present() ? 1 : 0) << 21);
     auto it = s->graphs.find(key);
     if (it == s->graphs.end()) {
@@ -1605,7 +1621,7 @@ int session_attention(mesh_session *s, int layer, const float *d_q, const mesh_b
     aa.scale = 1.0f / sqrtf((float)hp.head_dim);
     aa.n_head = (int)hp.n_head; aa.n_kv = (int)hp.n_head_kv; aa.group = (int)(hp.n_head / hp.n_head_kv);
     aa.head_dim = (int)hp.head_dim; aa.n_ctx = st->n_ctx; aa.max_keys = max_keys;
-    aa.n_splits = T < 64 ? attn_splits_for(s->tune, T, (int)hp.n_head_kv, max_keys, st->k_type != MESH_F16) : 1;
+    aa.n_splits = T < 64 ? attn_splits_for(s->tune, aa, T) : 1;
     if (matrix_cores) {
         if (!attention_mma_supported(aa)) return fail(MESH_ERR_UNSUPPORTED, "mesh_session_attn_dev: the matrix-core kernel does not cover this shape");
         return attention_mma(aa, T, s->stream);

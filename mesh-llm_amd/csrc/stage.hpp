@@ -73,7 +73,8 @@ int stage_decode_dev(mesh_session *s, const mesh_batch *b, const void *d_in, int
 // shared by the runners
 int stage_select_device(const mesh_stage_opts *opts, mesh_stage *st);
 int sess_alloc(mesh_session *s, void **p, size_t bytes);
-int attn_splits_for(const Tuning &tune, int T, int n_kv, int max_keys, bool quantised);
+struct AttnArgs;
+int attn_splits_for(const Tuning &tune, const AttnArgs &a, int T);       // of a: types, head layout and max_keys
 // names the kernel class of the launches made while it lives (mesh_session_profile)
 struct ProfScope {
     mesh_session *prev_s;

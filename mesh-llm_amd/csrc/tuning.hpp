@@ -35,7 +35,7 @@ struct Tuning {
     int gemm_narrow = 1;           // the register-formed tile of 32 or 64 columns for calls of at most 64 tokens that gemm_big leaves
     int attn_chunk_ksplit = 1;     // a prefill chunk's key walks split over workgroups when the grid would not fill the chip
     int attn_mma_min_tokens = 1;   // decode attention on the matrix cores from this many tokens (below: the all-f32 kernel)
-    int attn_split_target = 0;     // workgroups a decode attention launch aims at; 0 = 256, 512 for quantised rows of 64+ (token, head) pairs
+    int attn_split_target = 0;     // workgroups a decode attention launch aims at; 0 = attn_splits_for's rule
     int moe_group = 1;             // (token, slot) pairs grouped by expert (0: every pair its own product)
     int moe_router_tail = 1;       // no effect (routing and grouping are a launch of their own); accepted from callers that set it
     int moe_fuse_quant = 1;        // the expert combine step quantises for the next layer's projections

@@ -89,3 +89,42 @@ def test_walks_of_more_than_one_block_a_wave(tmp_path, name, splits):
         assert rel <= TOL, (name, splits, n, rel)
     ses.close()
     st.close()
+
+
+@pytest.mark.parametrize("kv_types", TIERS)
+@pytest.mark.parametrize("tokens,lines", [(1, (384,)), (40, (512,)), (60, (1024, 1536, 1920))])
+def test_lengths_where_walks_begin_to_be_split(tmp_path, kv_types, tokens, lines):
+    """Two KV heads: 2, 80 and 120 (token, head) pairs, for which a launch of one workgroup a CU would have 64, 3 and 2 splits."""
+    m, name = mesh(), "tiny-llama"
+    cfg = models.CONFIGS[name]
+    path = os.path.join(str(tmp_path), name + ".gguf")
+    models.write_model(path, cfg, [0], seed=5)
+    H, HK, D = cfg["n_head"], cfg["n_head_kv"], cfg["head_dim"]
+    assert HK == 2
+    longest = max(lines) + 1
+    st = m.Stage(path, 0, 1, n_ctx=longest, n_seq_max=2, n_batch_max=64, kv_types=kv_types)
+    rng = np.random.Generator(np.random.PCG64(11))
+    ses = st.session()
+    for i in range(2):
+        k, v = (rng.standard_normal((longest, HK, D)).astype(np.float16) for _ in range(2))
+        ses.kv_write(0, i, 0, k.view(np.uint16), v.view(np.uint16))
+    rows = [[r.view(np.float16).astype(np.float64).repeat(H // HK, axis=1) for r in ses.kv_read(0, i, 0, longest)] for i in range(2)]
+    q = rng.standard_normal((tokens, H, D)).astype(np.float32) * 1.5
+    qd = torch.from_numpy(q).cuda()
+    for line in lines:
+        for most in (line, line + 1):
+            keys = [most] + [int(n) for n in rng.integers(1, most + 1, tokens - 1)]
+            out = torch.full_like(qd, float("nan"))
+            torch.cuda.synchronize()
+            ses.attn_dev(0, qd.data_ptr(), [n - 1 for n in keys], out.data_ptr(), seq=[i % 2 for i in range(tokens)])
+            ses.synchronize()
+            got = out.cpu().numpy().astype(np.float64)
+            for i, n in enumerate(keys):
+                kd, vd = (r[:n] for r in rows[i % 2])
+                s = np.einsum("hd,nhd->hn", q[i].astype(np.float64), kd) / np.sqrt(D)
+                p = np.exp(s - s.max(1, keepdims=True))
+                want = np.einsum("hn,nhd->hd", p / p.sum(1, keepdims=True), vd)
+                rel = np.linalg.norm(got[i] - want) / np.linalg.norm(want)
+                assert rel <= TOL, (kv_types, tokens, most, n, rel)
+    ses.close()
+    st.close()
