@@ -169,7 +169,7 @@ __device__ __forceinline__ void router_logits(const float *__restrict__ x, const
     }
 }
 
-template <int NV, int RT = ROUTER_THREADS>
+template <int NV, int RT>
 // (scalar arguments first: preloaded into SGPRs, see gemv.hip)
 __global__ __launch_bounds__(RT) void moe_router_fused_kernel(const float *__restrict__ x, const float *__restrict__ norm_w,
                                                                           const float *__restrict__ W, float *__restrict__ logits_out,
@@ -180,70 +180,94 @@ __global__ __launch_bounds__(RT) void moe_router_fused_kernel(const float *__res
     if ((threadIdx.x >> 6) == 0) route_wave_any(s_logits, a, blockIdx.x, threadIdx.x & 63);
 }
 
-// The same for a prefill chunk, four tokens per workgroup of eight waves: every wave keeps the four normalised hidden
-// states in registers and walks every eighth expert row, so a row fetched from L2 serves four tokens (a workgroup per
-// token re-reads the whole router matrix per token: 512 MB per launch at 1024 tokens x 64 experts x 2048).  Every
-// (token, expert) logit is the sum the kernel above forms, in its order; waves 0 to 3 then route one token each.
-constexpr int CHUNK_TOKENS = 4, CHUNK_WAVES = 8, CHUNK_THREADS = 64 * CHUNK_WAVES;
-template <int NV>
-__global__ __launch_bounds__(CHUNK_THREADS) void moe_router_chunk_kernel(const float *__restrict__ x, const float *__restrict__ norm_w,
-                                                                         const float *__restrict__ W, float *__restrict__ logits_out,
-                                                                         int ldx, float eps, int T, const MoeRouteArgs a, float *__restrict__ scale_out) {
+// The same for hidden sizes up to 2048, TOKENS of a call per workgroup: every wave keeps their normalised hidden states in registers and
+// walks every eighth expert row, the next one on its way, the first while the states are normalised.  Every (token, expert) logit is the
+// sum the kernel above forms, in its order; the first waves then route one token each.
+// Bound by the CU's fetch of the whole router matrix from L2 (512 KB at about 95 GB/s: 5.4 us), before it the rows' and the norm's chain,
+// behind it the picks.  So a workgroup takes as many tokens as leave one for every CU.  64 experts x 2048, us, a token a workgroup of sixteen
+// waves / four tokens a workgroup, both with no row ahead (before) and two, three or four tokens: 40 tokens 19.2 / - / 12.6, 333 25.1
+// / - / 12.0, 512 - / 15.9 / 12.6, 600 - / 16.4 / 14.2, 1024 - / 16.9 / 16.7, 2048 - / 29.1 / 29.2.
+constexpr int CHUNK_WAVES = 8;
+template <int NV, int TOKENS>
+__global__ __launch_bounds__(64 * CHUNK_WAVES) void moe_router_chunk_kernel(const float *__restrict__ x, const float *__restrict__ norm_w,
+                                                                      const float *__restrict__ W, float *__restrict__ logits_out,
+                                                                      int ldx, float eps, int T, const MoeRouteArgs a, float *__restrict__ scale_out) {
     constexpr int E = NV * 256;
-    __shared__ float s_logits[CHUNK_TOKENS][64 * ROUTE_MAX_PER_LANE];
-    const int t0 = blockIdx.x * CHUNK_TOKENS, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    float4 xr[CHUNK_TOKENS][NV];
-    float sc[CHUNK_TOKENS];
+    __shared__ float s_logits[TOKENS][64 * ROUTE_MAX_PER_LANE];
+    const int t0 = blockIdx.x * TOKENS, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    float4 xr[TOKENS][NV], nw[NV], r[2][NV];
+    float sc[TOKENS];
+    auto fetch = [&](float4 (&to)[NV], int e) {
+        const float *wr = W + (size_t)(e < a.n_expert ? e : a.n_expert - 1) * E;       // (past the last row: not used)
 #pragma unroll
-    for (int k = 0; k < CHUNK_TOKENS; ++k) {
-        const int t = t0 + k < T ? t0 + k : T - 1;
-        const float *xt = x + (size_t)t * ldx;
+        for (int i = 0; i < NV; ++i) to[i] = *reinterpret_cast<const float4 *>(wr + 4 * (lane + 64 * i));
+    };
+#pragma unroll
+    for (int k = 0; k < TOKENS; ++k) {
+        const float *xt = x + (size_t)(t0 + k < T ? t0 + k : T - 1) * ldx;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) xr[k][i] = *reinterpret_cast<const float4 *>(xt + 4 * (lane + 64 * i));
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) nw[i] = *reinterpret_cast<const float4 *>(norm_w + 4 * (lane + 64 * i));
+    fetch(r[0], wave);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < TOKENS; ++k) {
         float ss = 0.f;
 #pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            xr[k][i] = *reinterpret_cast<const float4 *>(xt + 4 * (lane + 64 * i));
-            ss += xr[k][i].x * xr[k][i].x + xr[k][i].y * xr[k][i].y + xr[k][i].z * xr[k][i].z + xr[k][i].w * xr[k][i].w;
-        }
+        for (int i = 0; i < NV; ++i) ss += xr[k][i].x * xr[k][i].x + xr[k][i].y * xr[k][i].y + xr[k][i].z * xr[k][i].z + xr[k][i].w * xr[k][i].w;
         const float scale = 1.0f / sqrtf(wave_sum(ss) / (float)E + eps);
         sc[k] = scale;
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
-            const float4 w = *reinterpret_cast<const float4 *>(norm_w + 4 * (lane + 64 * i));
-            xr[k][i].x = xr[k][i].x * scale * w.x; xr[k][i].y = xr[k][i].y * scale * w.y;
-            xr[k][i].z = xr[k][i].z * scale * w.z; xr[k][i].w = xr[k][i].w * scale * w.w;
+            xr[k][i].x = xr[k][i].x * scale * nw[i].x; xr[k][i].y = xr[k][i].y * scale * nw[i].y;
+            xr[k][i].z = xr[k][i].z * scale * nw[i].z; xr[k][i].w = xr[k][i].w * scale * nw[i].w;
         }
     }
-    for (int e = wave; e < a.n_expert; e += CHUNK_WAVES) {
-        const float *wr = W + (size_t)e * E;
-        float4 r[NV];
+    for (int e0 = wave; e0 < a.n_expert; e0 += 2 * CHUNK_WAVES) {
 #pragma unroll
-        for (int i = 0; i < NV; ++i) r[i] = *reinterpret_cast<const float4 *>(wr + 4 * (lane + 64 * i));
-        float acc[CHUNK_TOKENS];
+        for (int u = 0; u < 2; ++u) {
+            const int e = e0 + u * CHUNK_WAVES;
+            if (e >= a.n_expert) break;
+            fetch(r[u ^ 1], e + CHUNK_WAVES);
+            float acc[TOKENS];
 #pragma unroll
-        for (int k = 0; k < CHUNK_TOKENS; ++k) {
-            float v = 0.f;
+            for (int k = 0; k < TOKENS; ++k) {
+                float v = 0.f;
 #pragma unroll
-            for (int i = 0; i < NV; ++i) {
-                v = fmaf(xr[k][i].x, r[i].x, v); v = fmaf(xr[k][i].y, r[i].y, v); v = fmaf(xr[k][i].z, r[i].z, v); v = fmaf(xr[k][i].w, r[i].w, v);
+                for (int i = 0; i < NV; ++i) {
+                    v = fmaf(xr[k][i].x, r[u][i].x, v); v = fmaf(xr[k][i].y, r[u][i].y, v); v = fmaf(xr[k][i].z, r[u][i].z, v); v = fmaf(xr[k][i].w, r[u][i].w, v);
+                }
+                acc[k] = v;
             }
-            acc[k] = v;
-        }
 #pragma unroll
-        for (int k = 0; k < CHUNK_TOKENS; ++k) acc[k] = wave_sum(acc[k]);
-        if (lane == 0) {
+            for (int k = 0; k < TOKENS; ++k) acc[k] = wave_sum(acc[k]);
+            if (lane == 0) {
 #pragma unroll
-            for (int k = 0; k < CHUNK_TOKENS; ++k) {
-                s_logits[k][e] = acc[k];
-                if (logits_out && t0 + k < T) logits_out[(size_t)(t0 + k) * a.n_expert + e] = acc[k];
+                for (int k = 0; k < TOKENS; ++k) {
+                    s_logits[k][e] = acc[k];
+                    if (logits_out && t0 + k < T) logits_out[(size_t)(t0 + k) * a.n_expert + e] = acc[k];
+                }
             }
         }
     }
     if (scale_out && wave == 0 && lane == 0)
 #pragma unroll
-        for (int k = 0; k < CHUNK_TOKENS; ++k)
+        for (int k = 0; k < TOKENS; ++k)
             if (t0 + k < T) scale_out[t0 + k] = sc[k];
     __syncthreads();
-    if (wave < CHUNK_TOKENS && t0 + wave < T) route_wave_any(s_logits[wave], a, t0 + wave, lane);
+    if (wave < TOKENS && t0 + wave < T) route_wave_any(s_logits[wave], a, t0 + wave, lane);
+}
+template <int TOKENS>
+static void launch_router_chunk(const MoeRouteArgs &a, const float *x, int ldx, const float *norm_w, float eps, const float *W, int E, float *logits_out, int T, hipStream_t stream,
+                                float *scale_out) {
+    const dim3 grid((unsigned)((T + TOKENS - 1) / TOKENS)), block(64 * CHUNK_WAVES);
+    switch (E / 256) {
+        case 2: MESH_LAUNCH((moe_router_chunk_kernel<2, TOKENS>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, T, a, scale_out); break;
+        case 4: MESH_LAUNCH((moe_router_chunk_kernel<4, TOKENS>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, T, a, scale_out); break;
+        default: MESH_LAUNCH((moe_router_chunk_kernel<8, TOKENS>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, T, a, scale_out); break;
+    }
 }
 
 // Router logits of a batch of decode steps, a workgroup per token and four experts, one row of the matrix per wave.  The bits of router_logits:
@@ -302,36 +326,15 @@ int moe_router_fused(const MoeRouteArgs &a, const float *x, int ldx, const float
     if (T <= 0) return MESH_OK;
     if (!moe_router_fused_supported(E, a.n_expert, a.top_k)) return fail(MESH_ERR_UNSUPPORTED, "moe: fused router for hidden size %d / %d experts", E, a.n_expert);
     const dim3 grid((unsigned)T);
-    if (T >= ROUTER_WIDE_MIN_TOKENS && E <= 2048) {
-        const dim3 cgrid((unsigned)((T + CHUNK_TOKENS - 1) / CHUNK_TOKENS)), cblock(CHUNK_THREADS);
-        switch (E / 256) {
-            case 2: MESH_LAUNCH(moe_router_chunk_kernel<2>, cgrid, cblock, 0, stream, x, norm_w, W, logits_out, ldx, eps, T, a, scale_out); break;
-            case 4: MESH_LAUNCH(moe_router_chunk_kernel<4>, cgrid, cblock, 0, stream, x, norm_w, W, logits_out, ldx, eps, T, a, scale_out); break;
-            default: MESH_LAUNCH(moe_router_chunk_kernel<8>, cgrid, cblock, 0, stream, x, norm_w, W, logits_out, ldx, eps, T, a, scale_out); break;
-        }
+    if (E <= 2048) {
+        if (T <= 2 * 256) launch_router_chunk<2>(a, x, ldx, norm_w, eps, W, E, logits_out, T, stream, scale_out);
+        else if (T <= 3 * 256) launch_router_chunk<3>(a, x, ldx, norm_w, eps, W, E, logits_out, T, stream, scale_out);
+        else launch_router_chunk<4>(a, x, ldx, norm_w, eps, W, E, logits_out, T, stream, scale_out);
         MESH_LAUNCH_CHECK();
         return MESH_OK;
     }
-    if (T >= ROUTER_WIDE_MIN_TOKENS) {
-        const dim3 block(ROUTER_THREADS_WIDE);
-        switch (E / 256) {
-            case 2: MESH_LAUNCH((moe_router_fused_kernel<2, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
-            case 4: MESH_LAUNCH((moe_router_fused_kernel<4, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
-            case 8: MESH_LAUNCH((moe_router_fused_kernel<8, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
-            case 16: MESH_LAUNCH((moe_router_fused_kernel<16, ROUTER_THREADS_WIDE>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
-            default: return fail(MESH_ERR_UNSUPPORTED, "moe: fused router for hidden size %d", E);
-        }
-        MESH_LAUNCH_CHECK();
-        return MESH_OK;
-    }
-    const dim3 block(ROUTER_THREADS);
-    switch (E / 256) {
-        case 2: MESH_LAUNCH(moe_router_fused_kernel<2>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
-        case 4: MESH_LAUNCH(moe_router_fused_kernel<4>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
-        case 8: MESH_LAUNCH(moe_router_fused_kernel<8>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
-        case 16: MESH_LAUNCH(moe_router_fused_kernel<16>, grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out); break;
-        default: return fail(MESH_ERR_UNSUPPORTED, "moe: fused router for hidden size %d", E);
-    }
+    if (T >= ROUTER_WIDE_MIN_TOKENS) MESH_LAUNCH((moe_router_fused_kernel<16, ROUTER_THREADS_WIDE>), grid, dim3(ROUTER_THREADS_WIDE), 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out);
+    else MESH_LAUNCH((moe_router_fused_kernel<16, ROUTER_THREADS>), grid, dim3(ROUTER_THREADS), 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out);
     MESH_LAUNCH_CHECK();
     return MESH_OK;
 }

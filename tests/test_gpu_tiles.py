@@ -146,6 +146,29 @@ def test_expert_products_over_ragged_loads(tmp_path, n_embd, ff, tokens):
     assert np.linalg.norm((got[1] - got[0])[same]) / norm < 6e-3
 
 
+@pytest.mark.parametrize("n_embd,tokens", [(512, 65), (1024, 515), (512, 770), (2048, 514)])
+def test_router_of_a_chunk_over_tokens_a_workgroup(tmp_path, n_embd, tokens):
+    """Two, three or four tokens a workgroup of the router, with one or two left over, and expert rows that its eight waves do not
+    share evenly; the gathered rows in quarters."""
+    m = mesh()
+    cfg = dict(arch="qwen3moe", n_layer=1, n_embd=n_embd, n_head=4, n_head_kv=2, head_dim=128, n_ff=0, n_vocab=256, eps=1e-6, rope=1e6,
+               n_expert=27, n_expert_used=3, n_ff_exp=256, qk_norm=True)
+    path = str(tmp_path / "model.gguf")
+    tensors = models.write_model(path, cfg, [0], seed=6, router="zipf")
+    x = models.zipf_hidden_state(np.random.Generator(np.random.PCG64(tokens)), tokens, n_embd)
+    orc = StageOracle(cfg, tensors, 0, 1, 1024, blas=True)
+    want = orc.forward(x, np.arange(tokens)) - x
+    st = m.Stage(path, 0, 1, n_ctx=1024, n_batch_max=1024)
+    ses = st.session(moe_gemm_min_pairs=1)
+    got = ses.decode(x, np.arange(tokens)).view(np.float32).reshape(want.shape) - x
+    same = (np.sort(ses.moe_last_ids(tokens), axis=1) == np.sort(np.stack(orc.last_expert_ids), axis=1)).all(axis=1)
+    ses.close()
+    st.close()
+    assert same.mean() > 0.97           # (near ties, as above)
+    # f16 activations: 11 bits in the inputs of the layer's products
+    assert np.linalg.norm((got - want)[same]) / np.linalg.norm(want[same]) < 3e-3
+
+
 #   shape as above, tokens, (32-column groups, groups of waves, slices) of gate/up and down
 KQUANT_FEW_CASES = [
     ((256, 2, 1, 256), 17, (1, 4, 1), (1, 4, 1)),       # four steps along K: one for each group of waves; padding columns
