@@ -113,3 +113,28 @@ def test_chunks_over_quantised_rows(tmp_path, shape, kv_types):
         assert np.linalg.norm(got - want) <= TOL * np.linalg.norm(want) and worst <= 2 * TOL, (shape, past, T, worst)
     ses.close()
     st.close()
+
+
+@pytest.mark.parametrize("kv_types", [(oracle.F16, oracle.F16), (oracle.Q8_0, oracle.Q4_0)])
+@pytest.mark.parametrize("name", ["tiny-llama", "tiny-odd", "tiny-kv3", "tiny-qwen3"])     # head_dim 64 and 128, 8, 7, 18 and 16 vectors, both modes, norms
+def test_rotated_rows_of_a_long_chunk(tmp_path, name, kv_types):
+    """A chunk whose head vectors share a token's sines against the same tokens in pieces of one vector a wave."""
+    m, cfg = mesh(), models.CONFIGS[name]
+    path = os.path.join(str(tmp_path), name + ".gguf")
+    models.write_model(path, cfg, [0], seed=7)
+    T = 193
+    st = m.Stage(path, 0, 1, n_ctx=256, n_seq_max=2, n_batch_max=256, kv_types=kv_types)
+    ses = st.session(gemv_rope=0)
+    x = np.random.Generator(np.random.PCG64(3)).standard_normal((T, cfg["n_embd"])).astype(np.float32)
+    ses.decode(x, np.arange(T), seq=np.zeros(T, np.int32))
+    for t in range(0, T, 97):
+        n = min(97, T - t)
+        ses.decode(x[t:t + n], np.arange(t, t + n), seq=np.ones(n, np.int32))
+    for kind, whole, parts in zip("kv", ses.kv_read(0, 0, 0, T), ses.kv_read(0, 1, 0, T)):
+        a, b = (r.view(np.float16).astype(np.float64) for r in (whole, parts))
+        # the projections may be summed in another order and the rows are rounded once: 2^-11 of f16 rows; quantised ones move by a
+        # step of 1 / 127 or 1 / 8 of the block's largest value (2 to 3 deviations) in the few places next to a rounding point
+        tol = 2.0 ** -11 if kv_types[0] == oracle.F16 else 2.0 ** -7 if kind == "k" else 2.0 ** -4
+        assert np.linalg.norm(a - b) / np.linalg.norm(b) <= tol, (name, kv_types, kind)
+    ses.close()
+    st.close()
