@@ -258,11 +258,12 @@ int mesh_session_set_expert_mask(mesh_session *session, const uint8_t *allowed, 
  * ids[n_tokens][n_expert_used].  For tests and for counting distinct experts touched. */
 int mesh_session_moe_last_ids(mesh_session *session, int32_t *ids, int32_t n_tokens);
 
-/* Values the session's f16 producers clamped to the f16 range (+-65504) since the session was created.  Calls of 5 or more
- * tokens hand activations to the matrix cores as f16 (normalised hidden state, attention output, SwiGLU product); a value
- * beyond the range is stored as the largest finite f16 instead of infinity and counted here, so a caller can tell a
- * saturated step from an exact one.  Single-token calls use 16-bit fixed point with a scale per 32 values and never
- * count.  Waits for the session's stream.  No counterpart in the reference (ggml's f16 conversions saturate silently to
+/* Values the session's f16 producers clamped to the f16 range (+-65504) since the session was created.  Calls of 4 or more
+ * tokens (skinny_min_tokens; 5 or 17 in some configurations) hand activations to the matrix cores as f16 (normalised hidden
+ * state, attention output, SwiGLU product); a value beyond the range is stored as the largest finite f16 instead of infinity
+ * and counted here, so a caller can tell a saturated step from an exact one.  Calls of fewer tokens use 16-bit fixed point
+ * with a scale per 32 values, expert products of up to 32 decode steps pairs of f16 with scales of their own: neither has a
+ * limit of range and neither counts.  Waits for the session's stream.  No counterpart in the reference (ggml's f16 conversions saturate silently to
  * infinity). */
 int mesh_session_f16_saturations(mesh_session *session, uint64_t *count);
 
@@ -302,7 +303,7 @@ int mesh_session_f16_saturations(mesh_session *session, uint64_t *count);
  *     moe_fuse_quant=1     the expert combine step quantises for the next layer
  *     moe_gemm=1, moe_gemm_min_pairs=4   prefill-sized expert products on the large-tile GEMM
  *     moe_step_min_tokens=1  expert products of up to 32 decode steps (below moe_gemm_min_pairs) on the f16 matrix cores from this
- *                          many tokens, activations as pairs of f16 (fewer: the grouped expert mat-vec)
+ *                          many tokens, activations as scaled pairs of f16 (fewer: the grouped expert mat-vec)
  *     reg_min_tokens=17, reg_min_blocks=192   gate / up of a batch of decode steps (up to 32) of at least that many and of
  *                          at least that many blocks of 64 rows on the GEMM layout instead of the f16 skinny GEMM
  *     tile_min_tokens=129  K-quant products of at least this many tokens on the large tile, over the copies of tile_copies

@@ -101,16 +101,11 @@ constexpr int ROUTER_THREADS = 1024, ROUTER_WAVES = ROUTER_THREADS / 64;
 // a prefill chunk has a workgroup per token anyway, and small workgroups, eight to a CU, hide each other's row loads.)
 constexpr int ROUTER_THREADS_WIDE = 256, ROUTER_WIDE_MIN_TOKENS = 512;
 // four neighbouring elements of a token's row as pairs of f16 (expert_step.hpp, by token)
-__device__ __forceinline__ void store_planes(_Float16 *planes, int E, int t, int k, const float4 &v, unsigned *sat) {
+__device__ __forceinline__ void store_planes(_Float16 *planes, int E, int t, int k, const float4 &v, float inverse) {
     const float x[4] = {v.x, v.y, v.z, v.w};
     _Float16 hi[4], lo[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float c = __builtin_amdgcn_fmed3f(x[i], -65504.f, 65504.f);
-        hi[i] = (_Float16)c;
-        lo[i] = (_Float16)((c - (float)hi[i]) * EXPERT_LO);
-    }
-    note_f16_clamp(sat, x[0], x[1], x[2], x[3]);
+    for (int i = 0; i < 4; ++i) pair_of(x[i] * inverse, hi[i], lo[i]);
     _Float16 *to = planes + (size_t)(t >> 4) * 32 * E + ((size_t)(k >> 3) * 32 + (t & 15)) * 8 + (k & 7);
     *reinterpret_cast<uint2 *>(to) = __builtin_bit_cast(uint2, hi);
     *reinterpret_cast<uint2 *>(to + 128) = __builtin_bit_cast(uint2, lo);
@@ -276,12 +271,13 @@ static void launch_router_chunk(const MoeRouteArgs &a, const float *x, int ldx, 
 // loaded and normalised the token's row for itself and added lanes up through the LDS unit.  (Before, the last of those workgroups to
 // arrive routed and grouped behind a hand-over between workgroups: 19.4 us in one launch, against 3.6 + 5.6 now.)
 constexpr int SLICE_THREADS = 256, SLICE_WAVES = SLICE_THREADS / 64;
+static_assert(SLICE_WAVES == 4, "the maxima of a row's four shares");
 template <int NV>
 __global__ __launch_bounds__(SLICE_THREADS) void moe_router_slice_kernel(const float *__restrict__ x, const float *__restrict__ norm_w, const float *__restrict__ W,
-                                                                         float *__restrict__ logits, int ldx, float eps, int n_expert, _Float16 *__restrict__ planes, unsigned *sat) {
+                                                                         float *__restrict__ logits, int ldx, float eps, int n_expert, _Float16 *__restrict__ planes, float *__restrict__ plane_scale) {
     constexpr int E = NV * 256, PER = E / 4 / SLICE_THREADS > 0 ? E / 4 / SLICE_THREADS : 1;       // float4 groups of the row a thread brings
     __shared__ __align__(16) float s_x[E];
-    __shared__ float s_sq[E / 4];
+    __shared__ float s_sq[E / 4], s_max[SLICE_WAVES];
     const int t = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int e = blockIdx.x * SLICE_WAVES + wave, row = e < n_expert ? e : n_expert - 1;
     const float *xt = x + (size_t)t * ldx;
@@ -302,15 +298,27 @@ __global__ __launch_bounds__(SLICE_THREADS) void moe_router_slice_kernel(const f
 #pragma unroll
     for (int i = 0; i < NV; ++i) ss += s_sq[lane + 64 * i];
     const float scale = 1.0f / sqrtf(wave_sum(ss) / (float)E + eps);
+    float mx = 0.f;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
         const int g = tid + SLICE_THREADS * i;
-        if (g >= E / 4) continue;
-        const float4 v = make_float4(xv[i].x * scale * nw[i].x, xv[i].y * scale * nw[i].y, xv[i].z * scale * nw[i].z, xv[i].w * scale * nw[i].w);
-        *reinterpret_cast<float4 *>(s_x + 4 * g) = v;
-        if (planes && blockIdx.x == 0) store_planes(planes, E, t, 4 * g, v, sat);
+        xv[i] = make_float4(xv[i].x * scale * nw[i].x, xv[i].y * scale * nw[i].y, xv[i].z * scale * nw[i].z, xv[i].w * scale * nw[i].w);
+        mx = fmaxf(mx, fmaxf(fmaxf(fabsf(xv[i].x), fabsf(xv[i].y)), fmaxf(fabsf(xv[i].z), fabsf(xv[i].w))));
+        if (g < E / 4) *reinterpret_cast<float4 *>(s_x + 4 * g) = xv[i];
+    }
+    const bool writes_planes = planes && blockIdx.x == 0;
+    if (writes_planes) {
+        mx = wave_max(mx);
+        if (lane == 0) s_max[wave] = mx;
     }
     lds_barrier();
+    if (writes_planes) {
+        const PairScale ps = pair_scale(fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3])));
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+            if (tid + SLICE_THREADS * i < E / 4) store_planes(planes, E, t, 4 * (tid + SLICE_THREADS * i), xv[i], ps.inverse);
+        if (tid == 0) plane_scale[t] = ps.scale;
+    }
     float acc = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -444,7 +452,7 @@ __global__ __launch_bounds__(GROUP_THREADS) void moe_route_group_kernel(const fl
 }
 
 int moe_router_group(const MoeRouteArgs &a, const float *x, int ldx, const float *norm_w, float eps, const float *W, int E,
-                     float *logits, int T, int32_t *items, int32_t *n_items, int item_pairs, hipStream_t stream, uint16_t *planes, unsigned *sat) {
+                     float *logits, int T, int32_t *items, int32_t *n_items, int item_pairs, hipStream_t stream, uint16_t *planes, float *plane_scale) {
     if (T <= 0) return MESH_OK;
     if (!moe_router_group_supported(E, a.n_expert, a.top_k, T) || !logits)
         return fail(MESH_ERR_UNSUPPORTED, "moe: split router for hidden size %d / %d experts / %d tokens", E, a.n_expert, T);
@@ -452,10 +460,10 @@ int moe_router_group(const MoeRouteArgs &a, const float *x, int ldx, const float
     MoeRouteArgs la = a;
     _Float16 *p = reinterpret_cast<_Float16 *>(planes);
     switch (E / 256) {
-        case 2: MESH_LAUNCH(moe_router_slice_kernel<2>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, a.n_expert, p, sat); break;
-        case 4: MESH_LAUNCH(moe_router_slice_kernel<4>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, a.n_expert, p, sat); break;
-        case 8: MESH_LAUNCH(moe_router_slice_kernel<8>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, a.n_expert, p, sat); break;
-        case 16: MESH_LAUNCH(moe_router_slice_kernel<16>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, a.n_expert, p, sat); break;
+        case 2: MESH_LAUNCH(moe_router_slice_kernel<2>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, a.n_expert, p, plane_scale); break;
+        case 4: MESH_LAUNCH(moe_router_slice_kernel<4>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, a.n_expert, p, plane_scale); break;
+        case 8: MESH_LAUNCH(moe_router_slice_kernel<8>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, a.n_expert, p, plane_scale); break;
+        case 16: MESH_LAUNCH(moe_router_slice_kernel<16>, grid, block, 0, stream, x, norm_w, W, logits, ldx, eps, a.n_expert, p, plane_scale); break;
         default: return fail(MESH_ERR_UNSUPPORTED, "moe: fused router for hidden size %d", E);
     }
     MESH_LAUNCH_CHECK();

@@ -509,10 +509,13 @@ static int kquant_session_alloc(mesh_session *s) {
                                                        moe_max_items((int)(B * k), (int)ne, SKINNY_ITEM_PAIRS) * moe_item_ints(SKINNY_ITEM_PAIRS)),
                                               step_items * moe_item_ints(EXPERT_STEP_PAIRS)) / MOE_ITEM_INTS + 1;
         if (hp.n_ff_exp > 0) {
-            if ((rc = sess_alloc(s, &p, expert_x_bytes((int)hp.n_embd))) != MESH_OK) return rc;
+            const size_t ffn_bytes = expert_ffn_bytes(step_items, (int)hp.n_ff_exp), x_bytes = expert_x_bytes((int)hp.n_embd);
+            if ((rc = sess_alloc(s, &p, x_bytes + EXPERT_STEP_TOKENS_MAX * sizeof(float))) != MESH_OK) return rc;
             s->moe_step_x = static_cast<uint16_t *>(p);
-            if ((rc = sess_alloc(s, &p, expert_ffn_bytes(step_items, (int)hp.n_ff_exp))) != MESH_OK) return rc;
+            s->moe_step_x_scale = reinterpret_cast<float *>(static_cast<uint8_t *>(p) + x_bytes);
+            if ((rc = sess_alloc(s, &p, ffn_bytes + expert_ffn_scales(step_items, (int)hp.n_ff_exp) * sizeof(float))) != MESH_OK) return rc;
             s->moe_step_ffn = static_cast<uint16_t *>(p);
+            s->moe_step_ffn_scale = reinterpret_cast<float *>(static_cast<uint8_t *>(p) + ffn_bytes);
         }
         // (+ the item count)
         if ((rc = sess_alloc(s, &p, (items * MOE_ITEM_INTS + 1) * sizeof(int32_t))) != MESH_OK) return rc;
@@ -1179,9 +1182,9 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
                 continue;
             }
             // a batch of decode steps over K-quant experts: eight pairs of an expert per pass on the f16 matrix cores
-            const bool step = want_groups && s->moe_step_x && T >= s->tune.moe_step_min_tokens && T <= EXPERT_STEP_TOKENS_MAX && ffe % 8 == 0 &&
+            const bool step = want_groups && s->moe_step_x && T >= s->tune.moe_step_min_tokens && T <= EXPERT_STEP_TOKENS_MAX &&
                               L.gate_inp.type == MESH_F32 && moe_router_group_supported(E, ne, k, T) && L.up_exps.type == L.gate_exps.type &&
-                              expert_step_supported(L.gate_exps.type, ffe, E) && expert_step_supported(L.down_exps.type, E, ffe);
+                              expert_step_supported(L.gate_exps.type, L.down_exps.type, E, ffe);
             const int item_pairs = step ? EXPERT_STEP_PAIRS : mfma ? SKINNY_ITEM_PAIRS : MOE_ITEM_PAIRS;
             bool grouped_done = false;
             if (want_groups && L.gate_inp.type == MESH_F32 && moe_router_group_supported(E, ne, k, T)) {
@@ -1189,7 +1192,7 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
                 ProfScope ps(s, MESH_PROF_GEMV);
                 if ((rc = moe_router_group(mr, s->x, E, static_cast<const float *>(L.ffn_norm.data), hp.rms_eps,
                                            static_cast<const float *>(L.gate_inp.data), E, s->moe_logits, T, s->moe_items, s->moe_n_items,
-                                           item_pairs, stream, step ? s->moe_step_x : nullptr, s->f16_sat)) != MESH_OK) return rc;
+                                           item_pairs, stream, step ? s->moe_step_x : nullptr, s->moe_step_x_scale)) != MESH_OK) return rc;
                 grouped_done = true;
             } else if (L.gate_inp.type == MESH_F32 && moe_router_fused_supported(E, ne, k)) {
                 // the router matrix is small and f32: logits and routing in one launch
@@ -1214,7 +1217,7 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
                 ExpertStepArgs ea;
                 ea.W[0] = L.gate_exps.data; ea.W[1] = L.up_exps.data; ea.type = L.gate_exps.type; ea.M = ffe; ea.K = E;
                 ea.items = s->moe_items; ea.n_items = s->moe_n_items; ea.max_items = moe_max_items(T * k, ne, EXPERT_STEP_PAIRS); ea.x_div = k;
-                ea.x = s->moe_step_x; ea.ffn = s->moe_step_ffn; ea.sat = s->f16_sat;
+                ea.x = s->moe_step_x; ea.x_scale = s->moe_step_x_scale; ea.ffn = s->moe_step_ffn; ea.ffn_scale = s->moe_step_ffn_scale;
                 if ((rc = expert_step(ea, stream)) != MESH_OK) return rc;
                 ea.W[0] = L.down_exps.data; ea.W[1] = nullptr; ea.type = L.down_exps.type; ea.M = E; ea.K = ffe;
                 ea.y = s->moe_out;

@@ -140,6 +140,7 @@ struct mesh_session {
     int32_t *moe_items = nullptr, *moe_n_items = nullptr;      // (token, slot) pairs grouped by expert, see moe_group
     // decode steps: normalised inputs and SwiGLU outputs of the expert products as pairs of f16 (expert_step.hpp)
     uint16_t *moe_step_x = nullptr, *moe_step_ffn = nullptr;
+    float *moe_step_x_scale = nullptr, *moe_step_ffn_scale = nullptr;
     // prefill chunks: the pairs sorted by expert (moe_sort) and their buffers, rows indexed by slot
     mesh::MoeSorted moe_sorted;
     uint16_t *moe_x16 = nullptr, *moe_ffn16 = nullptr;          // k8-major f16: normalised inputs, SwiGLU outputs
