@@ -127,7 +127,7 @@ static int layer_splits(const mesh_session *s, const HybridLayer &L, int T, int 
     AttnArgs a;
     a.k_type = s->stage->k_type; a.v_type = s->stage->v_type;
     a.n_kv = m.kv_heads; a.group = m.heads / m.kv_heads; a.head_dim = L.head_pad; a.max_keys = keys_seen(m, max_keys);
-    return T < 64 ? attn_splits_for(s->tune, a, T) : 1;
+    return T < 64 ? attn_splits_for(s->tune, a, T, s->stage->hybrid->act != ACT_F32 && attn_on_matrix_cores(s->tune, a, T)) : 1;
 }
 
 // (the partial sums have room for 1024 (token, split) rows at least)
@@ -185,7 +185,7 @@ static int run_attention(mesh_session *s, size_t il, int T, int max_keys, bool f
         aa.part_rows = s->tune.attn_chunk_ksplit ? s->attn_part_rows : 0;
         return attention_chunk(aa, T, s->chunk_pos0, s->chunk_seq, s->stream);
     }
-    if (T >= s->tune.attn_mma_min_tokens && attention_mma_supported(aa)) return attention_mma(aa, T, s->stream);
+    if (attn_on_matrix_cores(s->tune, aa, T)) return attention_mma(aa, T, s->stream);
     return attention(aa, T, s->stream);
 }
 

@@ -589,7 +589,9 @@ static GemvMat mat_of(const DevTensor &w, float *y, int ldy, const DevTensor *bi
 // Batches of at least attn_mma_min_tokens tokens take the matrix-core decode attention (Q and the probabilities rounded
 // to f16; faster at every batch size, so the default is 1).  Callers that want the all-f32 vector-ALU kernel at small
 // batches raise it.
-int attn_splits_for(const Tuning &tune, const AttnArgs &a, int T) {
+bool attn_on_matrix_cores(const Tuning &tune, const AttnArgs &a, int T) { return T >= tune.attn_mma_min_tokens && attention_mma_supported(a); }
+
+int attn_splits_for(const Tuning &tune, const AttnArgs &a, int T, bool matrix_cores) {
     const int pairs = std::max(1, T * a.n_kv), keys = a.max_keys;
     // (the partial sums have room for so many (token, split) rows)
     const int cap = std::max(1, std::min({ATTN_SPLITS_CAP, (keys + 63) / 64, ATTN_PART_ROWS_MIN / std::max(1, T)}));
@@ -598,7 +600,7 @@ int attn_splits_for(const Tuning &tune, const AttnArgs &a, int T) {
     const bool quantised = a.k_type == MESH_Q8_0 || a.k_type == MESH_Q4_0;
     const int one = std::max(1, 256 / pairs), two = std::max(1, 512 / pairs), three = std::max(1, 768 / pairs);     // one, two, three workgroups a CU
     // the f32 kernel: quantised rows cost it instructions, and a second workgroup on a CU hides their waits
-    if (T < tune.attn_mma_min_tokens || !attention_mma_supported(a)) return std::min(quantised && pairs >= 64 ? two : one, cap);
+    if (!matrix_cores) return std::min(quantised && pairs >= 64 ? two : one, cap);
     // The matrix-core kernel (us, attention and merge, 8 KV heads of 128, the longest sequence and the others from a third of it on).
     // A merge costs 2 to 4 us and a launch, so short walks stay whole, and the fewer splits there are the longer.  One split / one
     // workgroup a CU: 2 tokens, f16 rows, 100 keys 5.7 / 6.8, 250 6.6 / 7.0, 400 8.5 / 7.0; 8 tokens (4 splits) 200 7.3 / 7.3, 350
@@ -846,7 +848,8 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
     aa.scale = 1.0f / sqrtf((float)hp.head_dim);
     aa.n_head = (int)hp.n_head; aa.n_kv = (int)hp.n_head_kv; aa.group = (int)(hp.n_head / hp.n_head_kv);
     aa.head_dim = (int)hp.head_dim; aa.n_ctx = st->n_ctx; aa.max_keys = max_keys;
-    aa.n_splits = T < 64 ? attn_splits_for(s->tune, aa, T) : 1;     // a batch of decode steps still splits the long KV
+    const bool attn_mma = attn_on_matrix_cores(s->tune, aa, T);
+    aa.n_splits = T < 64 ? attn_splits_for(s->tune, aa, T, attn_mma) : 1;     // a batch of decode steps still splits the long KV
     {
         ProfScope ps(s, MESH_PROF_ATTN);
         if (!skinny && s->chunk_pos0 >= 0 && hp.head_dim == 128) {
@@ -855,7 +858,7 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
             aa.part_rows = s->tune.attn_chunk_ksplit ? s->attn_part_rows : 0;
             rc = attention_chunk(aa, T, s->chunk_pos0, s->chunk_seq, stream);
         }
-        else if (T >= s->tune.attn_mma_min_tokens && attention_mma_supported(aa)) {
+        else if (attn_mma) {
             // straight into the output projection's input layout
             if (sk8) { aa.out_q16 = s->xq; attn_is_k8 = true; }
             else if (k8) { aa.out16_k8 = xn; attn_is_k8 = true; }
@@ -1103,10 +1106,11 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
         aa.scale = 1.0f / sqrtf((float)hp.head_dim);
         aa.n_head = (int)hp.n_head; aa.n_kv = (int)hp.n_head_kv; aa.group = (int)(hp.n_head / hp.n_head_kv);
         aa.head_dim = (int)hp.head_dim; aa.n_ctx = st->n_ctx; aa.max_keys = max_keys;
-        aa.n_splits = attn_splits_for(s->tune, aa, T);
+        const bool attn_mma = attn_on_matrix_cores(s->tune, aa, T);
+        aa.n_splits = attn_splits_for(s->tune, aa, T, attn_mma);
         {
             ProfScope ps(s, MESH_PROF_ATTN);
-            rc = T >= s->tune.attn_mma_min_tokens && attention_mma_supported(aa) ? attention_mma(aa, T, stream) : attention(aa, T, stream);
+            rc = attn_mma ? attention_mma(aa, T, stream) : attention(aa, T, stream);
         }
         if (rc != MESH_OK) return rc;
 
@@ -1336,7 +1340,8 @@ static int run_layers_graphed(mesh_session *s, int T, int max_keys) {
     // chunk's.  Such calls are always launched eagerly.
     const mesh_stage *st = s->stage;
     if (s->chunk_pos0 >= 0 && (T >= PREFILL_MIN_TOKENS || (st->hybrid && T >= s->tune.latent_chunk_min_tokens))) return run_layers(s, T, max_keys);
-    const int n_splits = st->hybrid ? 0 : attn_splits_for(s->tune, attn_shape(st, max_keys), T);
+    const AttnArgs shape = st->hybrid ? AttnArgs{} : attn_shape(st, max_keys);
+    const int n_splits = st->hybrid ? 0 : attn_splits_for(s->tune, shape, T, attn_on_matrix_cores(s->tune, shape, T));
     const uint64_t key = st->hybrid ? hybrid_graph_key(s, T, max_keys) : (uint64_t)T | ((uint64_t)n_splits << 8) | ((uint64_t)(s->expert_mask_on ? 1 : 0) << 20) | ((uint64_t)(st->copies.present() ? 1 : 0) << 21);
     auto it = s->graphs.find(key);
     if (it == s->graphs.end()) {
@@ -1624,7 +1629,7 @@ int session_attention(mesh_session *s, int layer, const float *d_q, const mesh_b
     aa.scale = 1.0f / sqrtf((float)hp.head_dim);
     aa.n_head = (int)hp.n_head; aa.n_kv = (int)hp.n_head_kv; aa.group = (int)(hp.n_head / hp.n_head_kv);
     aa.head_dim = (int)hp.head_dim; aa.n_ctx = st->n_ctx; aa.max_keys = max_keys;
-    aa.n_splits = T < 64 ? attn_splits_for(s->tune, aa, T) : 1;
+    aa.n_splits = T < 64 ? attn_splits_for(s->tune, aa, T, matrix_cores) : 1;
     if (matrix_cores) {
         if (!attention_mma_supported(aa)) return fail(MESH_ERR_UNSUPPORTED, "mesh_session_attn_dev: the matrix-core kernel does not cover this shape");
         return attention_mma(aa, T, s->stream);

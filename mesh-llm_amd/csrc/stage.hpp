@@ -74,7 +74,8 @@ int stage_decode_dev(mesh_session *s, const mesh_batch *b, const void *d_in, int
 int stage_select_device(const mesh_stage_opts *opts, mesh_stage *st);
 int sess_alloc(mesh_session *s, void **p, size_t bytes);
 struct AttnArgs;
-int attn_splits_for(const Tuning &tune, const AttnArgs &a, int T);       // of a: types, head layout and max_keys
+bool attn_on_matrix_cores(const Tuning &tune, const AttnArgs &a, int T);        // which decode attention a call takes; of a: types, head layout
+int attn_splits_for(const Tuning &tune, const AttnArgs &a, int T, bool matrix_cores);       // for the kernel that is launched; of a: max_keys too
 // names the kernel class of the launches made while it lives (mesh_session_profile)
 struct ProfScope {
     mesh_session *prev_s;

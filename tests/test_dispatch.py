@@ -104,3 +104,39 @@ def test_prefill_of_the_full_sizes(name, layers, tokens):
     assert kernels[0] == {"gemm_f16_kernel"}
     assert "gemm_big_kernel" in kernels[1] and kernels[1] <= {"gemm_big_kernel", "gemm_kq_kernel"}
     assert kernels[2] == {"gemm_kq_kernel"}
+
+
+# KV heads, cache types, tokens, keys of the longest walk; key splits of the f32 kernel (a workgroup a CU, 64 keys a split at least; two for quantised rows from
+# 64 (token, head) pairs on) and of the matrix-core one (a merge only where it pays)
+ATTENTION_SPLITS = [
+    (2, (1, 1), 1, 100, 2, 1), (2, (1, 1), 1, 384, 6, 1), (2, (1, 1), 1, 385, 7, 7), (8, (1, 1), 16, 1500, 2, 1), (8, (1, 1), 16, 1537, 2, 2),
+    (8, (8, 2), 16, 1500, 4, 2), (8, (8, 2), 8, 300, 5, 1), (2, (8, 2), 4, 200, 4, 1),
+]
+
+
+def attention_launches(host, n_kv, kv_types, tokens, keys, matrix_cores, least=1):
+    m = mesh()
+    host.memory(1 << 37)
+    cfg = dict(arch="llama", n_layer=1, n_embd=512, n_head=2 * n_kv, n_head_kv=n_kv, head_dim=64, n_ff=512, n_vocab=256, eps=1e-5, rope=1e4)
+    with tempfile.TemporaryDirectory() as d:
+        path = os.path.join(d, "model.gguf")
+        models.write_model(path, cfg, [0], seed=1, fast=True)
+        st = m.Stage(path, 0, 1, n_ctx=keys, n_seq_max=tokens, n_batch_max=32, kv_types=kv_types)
+    ses = st.session(attn_mma_min_tokens=least)
+    host.launches()
+    rows = np.zeros((tokens, 2 * n_kv, 64), np.float32)
+    ses.attn_dev(0, rows.ctypes.data, [keys - 1] * tokens, rows.ctypes.data, seq=np.arange(tokens), matrix_cores=matrix_cores)
+    direct = [(n, g) for n, g, _ in host.launches() if n.startswith("attn_") and "combine" not in n]
+    ses.decode(np.zeros((tokens, 512), np.float32), [keys - 1] * tokens, seq=np.arange(tokens))
+    return direct + [(n, g) for n, g, _ in host.launches() if n.startswith("attn_") and "combine" not in n]
+
+
+@pytest.mark.parametrize("case", ATTENTION_SPLITS)
+@pytest.mark.parametrize("matrix_cores", [0, 1])
+def test_key_splits_go_by_the_kernel_that_is_launched(case, matrix_cores):
+    """Of the entry point that names its kernel, whatever the session's switch says, and of the layers, which go by the switch."""
+    n_kv, kv_types, tokens, keys, *splits = case
+    for least in (1, 1 << 20):
+        direct, layer = call(attention_launches, n_kv=n_kv, kv_types=kv_types, tokens=tokens, keys=keys, matrix_cores=matrix_cores, least=least)
+        assert direct[0].startswith("attn_mma_kernel" if matrix_cores else "attn_kernel") and direct[1][0] == splits[matrix_cores]
+        assert layer[0].startswith("attn_mma_kernel" if least == 1 else "attn_kernel") and layer[1][0] == splits[1 if least == 1 else 0]
