@@ -64,6 +64,8 @@ int attention_combine(const AttnArgs &a, int T, hipStream_t stream);
 // cost independent of the group size; Q and the probabilities rounded to f16.  For batches of decode tokens.
 bool attention_mma_supported(const AttnArgs &a);
 int attention_mma(const AttnArgs &a, int T, hipStream_t stream);
+// Of a's types, splits and max_keys: no wave walks more than one block of keys, a choice between two kernels that a captured graph keeps.
+bool attention_mma_one_block(const AttnArgs &a);
 // The same for a chunk of T consecutive positions pos0 .. pos0 + T - 1 of one sequence, on the matrix cores
 // (attn_prefill.hip; head_dim 64 or 128; with f16 rows and a group of 1 also 128 with values of 64, 192 with values of 128).  a.pos / a.seq / a.part / a.ml are not used.
 int attention_chunk(const AttnArgs &a, int T, int pos0, int seq, hipStream_t stream);

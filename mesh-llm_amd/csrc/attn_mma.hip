@@ -374,12 +374,15 @@ static void launch_mma_as(const AttnArgs &a, int T, hipStream_t stream) {
                 a.n_ctx, a.n_kv, a.group, a.n_head, a.scale, a.window, a);
 }
 
+// f16 rows, at most one block of keys a wave (attn_mma_kernel, KROWS)
+bool attention_mma_one_block(const AttnArgs &a) {
+    return a.k_type == MESH_F16 && a.v_type == MESH_F16 && a.max_keys > 0 && a.max_keys <= a.n_splits * MMA_WAVES * MMA_KEYS;
+}
+
 template <int HD>
 static int launch_mma(const AttnArgs &a, int T, hipStream_t stream) {
     if (a.k_type == MESH_F16 && a.v_type == MESH_F16) {
-        // one block of keys a wave at most (attn_mma_kernel, KROWS)
-        const bool one_block = a.max_keys > 0 && a.max_keys <= a.n_splits * MMA_WAVES * MMA_KEYS;
-        if (one_block) launch_mma_as<HD, MESH_F16, MESH_F16, false>(a, T, stream);
+        if (attention_mma_one_block(a)) launch_mma_as<HD, MESH_F16, MESH_F16, false>(a, T, stream);
         else launch_mma_as<HD, MESH_F16, MESH_F16, true>(a, T, stream);
     } else if (a.k_type == MESH_Q8_0 && a.v_type == MESH_Q4_0) launch_mma_as<HD, MESH_Q8_0, MESH_Q4_0, false>(a, T, stream);
     else if (a.k_type == MESH_Q4_0 && a.v_type == MESH_Q4_0) launch_mma_as<HD, MESH_Q4_0, MESH_Q4_0, false>(a, T, stream);

@@ -122,12 +122,14 @@ bool hybrid_single_step(const mesh_session *s, int T) { return T == 1 && s->tune
 
 static int keys_seen(const MixerSpec &m, int max_keys) { return m.window > 0 ? std::min(m.window, max_keys) : max_keys; }
 
-static int layer_splits(const mesh_session *s, const HybridLayer &L, int T, int max_keys) {
+// types, head layout, keys and splits of a layer's decode attention
+static AttnArgs layer_walk(const mesh_session *s, const HybridLayer &L, int T, int max_keys) {
     const MixerSpec &m = L.spec.mixer;
     AttnArgs a;
     a.k_type = s->stage->k_type; a.v_type = s->stage->v_type;
     a.n_kv = m.kv_heads; a.group = m.heads / m.kv_heads; a.head_dim = L.head_pad; a.max_keys = keys_seen(m, max_keys);
-    return T < 64 ? attn_splits_for(s->tune, a, T, s->stage->hybrid->act != ACT_F32 && attn_on_matrix_cores(s->tune, a, T)) : 1;
+    a.n_splits = T < 64 ? attn_splits_for(s->tune, a, T, s->stage->hybrid->act != ACT_F32 && attn_on_matrix_cores(s->tune, a, T)) : 1;
+    return a;
 }
 
 // (the partial sums have room for 1024 (token, split) rows at least)
@@ -139,7 +141,10 @@ uint64_t hybrid_graph_key(const mesh_session *s, int T, int max_keys) {
     uint64_t key = 1469598103934665603ull ^ (uint64_t)T;
     auto mix = [&](uint64_t v) { key = (key ^ v) * 1099511628211ull; };
     for (const HybridLayer &L : s->stage->hybrid->layers) {
-        if (L.spec.mixer.kind == MIXER_ATTENTION) mix((uint64_t)layer_splits(s, L, T, max_keys));
+        if (L.spec.mixer.kind == MIXER_ATTENTION) {
+            const AttnArgs a = layer_walk(s, L, T, max_keys);
+            mix((uint64_t)a.n_splits << 1 | (attention_mma_one_block(a) ? 1 : 0));
+        }
         if (L.spec.mixer.kind == MIXER_LATENT) mix((uint64_t)latent_layer_splits(s, L.latent, T, max_keys) << 1 | (s->chunk_pos0 >= 0 ? 1 : 0));
     }
     mix(s->stage->copies.present() ? 1 : 0);
@@ -169,16 +174,14 @@ static int run_attention(mesh_session *s, size_t il, int T, int max_keys, bool f
         ProfScope ps(s, MESH_PROF_ROPE);
         if ((rc = qk_norm_append(a, T, s->stream)) != MESH_OK) return rc;
     }
-    AttnArgs aa;
-    aa.q = h.q; aa.kcache = h.k[il]; aa.vcache = h.v[il]; aa.k_type = st->k_type; aa.v_type = st->v_type; aa.pos = s->d_pos; aa.seq = s->d_seq;
+    AttnArgs aa = layer_walk(s, L, T, max_keys);
+    aa.q = h.q; aa.kcache = h.k[il]; aa.vcache = h.v[il]; aa.pos = s->d_pos; aa.seq = s->d_seq;
     aa.part = s->attn_part; aa.ml = s->attn_ml;
     if (f32_out || hm.act == ACT_F32) aa.out = static_cast<float *>(h.acta);
     else aa.out_bf16 = static_cast<uint16_t *>(h.acta);
     aa.window = m.window;
     aa.scale = m.scale;
-    aa.n_head = m.heads; aa.n_kv = m.kv_heads; aa.group = m.heads / m.kv_heads; aa.head_dim = L.head_pad; aa.n_ctx = st->n_ctx;
-    aa.n_splits = layer_splits(s, L, T, max_keys);
-    aa.max_keys = keys_seen(m, max_keys);
+    aa.n_head = m.heads; aa.n_ctx = st->n_ctx;
     ProfScope ps(s, MESH_PROF_ATTN);
     if (hm.act == ACT_F32) return attention(aa, T, s->stream);
     if (T >= s->tune.gemm_min_tokens && s->chunk_pos0 >= 0 && L.head_pad <= 128) {

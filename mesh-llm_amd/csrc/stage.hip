@@ -1322,7 +1322,7 @@ static int validate_batch(const mesh_session *s, const mesh_batch *b, int *max_k
 }
 
 // run_layers, replayed from a captured graph for decode-sized batches.  The launches depend on T, on the KV split count
-// (a function of the deepest position), on whether an expert mask is set and on whether the stage holds second copies
+// and on whether a wave walks more than one block of keys (functions of the deepest position), on whether an expert mask is set and on whether the stage holds second copies
 // of its weights; everything else they read is device memory at fixed addresses (hidden state, positions, caches).  The first use of a key runs eagerly (which also
 // finishes every lazy initialisation), the second is captured, later ones are replays.
 constexpr int GRAPH_MAX_TOKENS = 32;
@@ -1340,9 +1340,9 @@ static int run_layers_graphed(mesh_session *s, int T, int max_keys) {
     // chunk's.  Such calls are always launched eagerly.
     const mesh_stage *st = s->stage;
     if (s->chunk_pos0 >= 0 && (T >= PREFILL_MIN_TOKENS || (st->hybrid && T >= s->tune.latent_chunk_min_tokens))) return run_layers(s, T, max_keys);
-    const AttnArgs shape = st->hybrid ? AttnArgs{} : attn_shape(st, max_keys);
-    const int n_splits = st->hybrid ? 0 : attn_splits_for(s->tune, shape, T, attn_on_matrix_cores(s->tune, shape, T));
-    const uint64_t key = st->hybrid ? hybrid_graph_key(s, T, max_keys) : (uint64_t)T | ((uint64_t)n_splits << 8) | ((uint64_t)(s->expert_mask_on ? 1 : 0) << 20) | ((uint64_t)(st->copies.present() ? 1 : 0) << 21);
+    AttnArgs shape = st->hybrid ? AttnArgs{} : attn_shape(st, max_keys);
+    if (!st->hybrid) shape.n_splits = attn_splits_for(s->tune, shape, T, attn_on_matrix_cores(s->tune, shape, T));
+    const uint64_t key = st->hybrid ? hybrid_graph_key(s, T, max_keys) : (uint64_t)T | ((uint64_t)shape.n_splits << 8) | ((uint64_t)(attention_mma_one_block(shape) ? 1 : 0) << 22) | ((uint64_t)(s->expert_mask_on ? 1 : 0) << 20) | ((uint64_t)(st->copies.present() ? 1 : 0) << 21);
     auto it = s->graphs.find(key);
     if (it == s->graphs.end()) {
         if (s->graphs.size() >= GRAPH_MAX_ENTRIES) return run_layers(s, T, max_keys);

@@ -140,3 +140,39 @@ def test_key_splits_go_by_the_kernel_that_is_launched(case, matrix_cores):
         direct, layer = call(attention_launches, n_kv=n_kv, kv_types=kv_types, tokens=tokens, keys=keys, matrix_cores=matrix_cores, least=least)
         assert direct[0].startswith("attn_mma_kernel" if matrix_cores else "attn_kernel") and direct[1][0] == splits[matrix_cores]
         assert layer[0].startswith("attn_mma_kernel" if least == 1 else "attn_kernel") and layer[1][0] == splits[1 if least == 1 else 0]
+
+
+def graph_walks(host, folder, tokens, keys):
+    """Attention kernel of the launches that the last of each run of three calls made, one run for each length: none where a graph ran."""
+    m = mesh()
+    host.memory(1 << 37)
+    with tempfile.TemporaryDirectory() as d:
+        if folder:
+            st = m.Stage(N.write_folder(d, c := N.config(64, 256, 512, [N.attention(2, 1, 64, 400, ff=128)]), N.random_weights(c, 3)), 0, -1, n_ctx=512, n_seq_max=tokens, n_batch_max=16)
+        else:
+            path = os.path.join(d, "model.gguf")
+            models.write_model(path, models.CONFIGS["tiny-llama"], [0], seed=1, fast=True)
+            st = m.Stage(path, 0, 1, n_ctx=512, n_seq_max=tokens, n_batch_max=16)
+    ses = st.session(graphs=1)
+    out = []
+    for n in keys:
+        pos, seq = [n - 1] * tokens, np.arange(tokens)
+        first = None
+        for _ in range(3):
+            host.launches()
+            if folder:
+                ses.decode(np.zeros(tokens, np.int32), pos, seq=seq, in_fmt=m.TOKENS)
+            else:
+                ses.decode(np.zeros((tokens, 256), np.float32), pos, seq=seq)
+            got = [k for k, _, _ in host.launches() if k.startswith("attn_mma")]
+            first = got if first is None else first
+        assert got == []
+        out.append(first)
+    return out
+
+
+@pytest.mark.parametrize("folder", [False, True])
+def test_a_replayed_graph_has_the_kernel_of_the_length(folder):
+    """At most 128 keys (one block of 32 for each of four waves) and more of them, both unsplit, are graphs of their own."""
+    got = call(graph_walks, folder=folder, tokens=2, keys=[100, 128, 129, 300, 100])
+    assert got == [["attn_mma_kernel<64,1,1,0>"], [], ["attn_mma_kernel<64,1,1,1>"], [], []]
