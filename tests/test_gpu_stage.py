@@ -6,6 +6,7 @@ import os
 import numpy as np
 import pytest
 
+import gguf_util as G
 import models
 import oracle
 from oracle.stage import StageOracle
@@ -296,21 +297,44 @@ def test_qwen3_30b_a3b_shaped_expert_shard_layer(tmp_path):
     assert np.array_equal(np.sort(ids, axis=1), np.sort(np.stack(orc.last_expert_ids), axis=1))
     assert len(set(ids.reshape(-1))) > 8
     ses.close()
-    # the router launch's last-arriving workgroup routes and groups the pairs (the default), or a second launch does
-    # (moe_router_tail=0): the same bits and the same routing, step after step (the arrival counter returns to zero)
+    st.close()
+
+
+# every hidden size the routers have a kernel for; 27 experts: a last slice of three rows, 130: lanes with three of them
+@pytest.mark.parametrize("n_embd,n_expert,top_k", [(512, 27, 1), (1024, 64, 3), (2048, 64, 3), (2048, 130, 7), (4096, 27, 1)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_routers_of_steps_and_of_chunks_agree(tmp_path, n_embd, n_expert, top_k, masked):
+    """Logits over slices of the experts, then routing and grouping in one workgroup (up to 64 tokens), against logits and routing of
+    whole tokens and a grouping of its own (65): the same sums in the same order, so the same picks, weights and bits of a layer whose
+    attention adds nothing and whose expert products take the grouped mat-vec form either way."""
+    m = mesh()
+    cfg = dict(arch="qwen3moe", n_layer=1, n_embd=n_embd, n_head=4, n_head_kv=2, head_dim=128, n_ff=0, n_vocab=256, eps=1e-6, rope=1e6,
+               n_expert=n_expert, n_expert_used=top_k, n_ff_exp=256, qk_norm=True)
+    assert 65 * top_k < 4 * n_expert            # (fewer pairs than the matrix-core forms begin at)
+    kvs, tl = models.build_tensors(cfg, [0], seed=9, fast=True, router="zipf")
+    path = os.path.join(str(tmp_path), "model.gguf")
+    G.write_gguf(path, kvs, [(n, t, d, np.zeros_like(v) if "attn_output" in n else v) for n, t, d, v in tl])
+    st = m.Stage(path, 0, 1, n_ctx=16, n_seq_max=65, n_batch_max=65)
+    os.unlink(path)
+    x = models.zipf_hidden_state(np.random.Generator(np.random.PCG64(32)), 65, n_embd)
     runs = []
-    for tail in (1, 0):
-        q = st.session(moe_router_tail=tail)
-        r2 = np.random.Generator(np.random.PCG64(32))
-        outs = []
-        for step, T in enumerate((16, 11, 6, 16, 1, 16)):
-            xs = r2.standard_normal((T, 2048)).astype(np.float32)
-            outs.append((q.decode(xs, np.full(T, step, np.int32), seq=np.arange(T, dtype=np.int32)).copy(), q.moe_last_ids(T).copy()))
-        runs.append(outs)
-        q.close()
-    for (a, ia), (b, ib) in zip(*runs):
-        assert np.array_equal(ia, ib)
-        assert np.array_equal(a, b)
+    for parts in ((65,), (64, 1), (1, 2, 30, 32)):
+        ses = st.session(moe_step_min_tokens=33, moe_gemm=0)
+        if masked:
+            ses.set_expert_mask(np.arange(n_expert) % 3 != 1)
+        y, ids, at = np.empty_like(x), np.empty((65, top_k), np.int32), 0
+        for n in parts:
+            y[at:at + n] = ses.decode(x[at:at + n], np.zeros(n, np.int32), seq=np.arange(at, at + n, dtype=np.int32)).view(np.float32).reshape(n, n_embd)
+            ids[at:at + n] = ses.moe_last_ids(n)
+            at += n
+        runs.append((y, ids))
+        ses.close()
+    assert np.linalg.norm(runs[0][0] - x) > 0.01 * np.linalg.norm(x)
+    for y, ids in runs[1:]:
+        assert np.array_equal(ids, runs[0][1])
+        assert np.array_equal(y, runs[0][0])
+    if masked:
+        assert (runs[0][1] % 3 != 1).all()
     st.close()
 
 
