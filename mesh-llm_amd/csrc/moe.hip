@@ -334,7 +334,12 @@ int moe_router_fused(const MoeRouteArgs &a, const float *x, int ldx, const float
     if (T <= 0) return MESH_OK;
     if (!moe_router_fused_supported(E, a.n_expert, a.top_k)) return fail(MESH_ERR_UNSUPPORTED, "moe: fused router for hidden size %d / %d experts", E, a.n_expert);
     const dim3 grid((unsigned)T);
-    if (E <= 2048) {
+    // Up to 256 tokens every token has a CU of its own either way, and of many short rows sixteen waves walk half as many each: us, two tokens a
+    // workgroup of eight waves / one a workgroup of sixteen, 200 tokens: E 512 with 96 experts 9.1 / 7.4, 128 10.0 / 8.4, 256 18.6 / 15.0,
+    // 512 29.9 / 21.0; E 1024 with 96 10.0 / 9.0, 128 11.8 / 10.3, 256 20.8 / 18.3, 512 34.5 / 28.6; E 2048 with 64 9.9 / 17.9, 512 53 / 112
+    // (those two with sums through the LDS unit).  300 tokens, E 512, 512 experts: 29.4 / 33.
+    const bool short_rows = T <= 256 && E <= 1024 && a.n_expert >= 96;
+    if (E <= 2048 && !short_rows) {
         if (T <= 2 * 256) launch_router_chunk<2>(a, x, ldx, norm_w, eps, W, E, logits_out, T, stream, scale_out);
         else if (T <= 3 * 256) launch_router_chunk<3>(a, x, ldx, norm_w, eps, W, E, logits_out, T, stream, scale_out);
         else launch_router_chunk<4>(a, x, ldx, norm_w, eps, W, E, logits_out, T, stream, scale_out);
@@ -342,6 +347,8 @@ int moe_router_fused(const MoeRouteArgs &a, const float *x, int ldx, const float
         return MESH_OK;
     }
     if (T >= ROUTER_WIDE_MIN_TOKENS) MESH_LAUNCH((moe_router_fused_kernel<16, ROUTER_THREADS_WIDE>), grid, dim3(ROUTER_THREADS_WIDE), 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out);
+    else if (E == 512) MESH_LAUNCH((moe_router_fused_kernel<2, ROUTER_THREADS>), grid, dim3(ROUTER_THREADS), 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out);
+    else if (E == 1024) MESH_LAUNCH((moe_router_fused_kernel<4, ROUTER_THREADS>), grid, dim3(ROUTER_THREADS), 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out);
     else MESH_LAUNCH((moe_router_fused_kernel<16, ROUTER_THREADS>), grid, dim3(ROUTER_THREADS), 0, stream, x, norm_w, W, logits_out, ldx, eps, a.n_expert, a, scale_out);
     MESH_LAUNCH_CHECK();
     return MESH_OK;

@@ -176,3 +176,32 @@ def test_a_replayed_graph_has_the_kernel_of_the_length(folder):
     """At most 128 keys (one block of 32 for each of four waves) and more of them, both unsplit, are graphs of their own."""
     got = call(graph_walks, folder=folder, tokens=2, keys=[100, 128, 129, 300, 100])
     assert got == [["attn_mma_kernel<64,1,1,0>"], [], ["attn_mma_kernel<64,1,1,1>"], [], []]
+
+
+def routers(host, n_embd, n_expert, tokens):
+    m = mesh()
+    host.memory(1 << 37)
+    cfg = dict(arch="qwen3moe", n_layer=1, n_embd=n_embd, n_head=4, n_head_kv=2, head_dim=128, n_ff=0, n_vocab=256, eps=1e-6, rope=1e6,
+               n_expert=n_expert, n_expert_used=2, n_ff_exp=256, qk_norm=True)
+    with tempfile.TemporaryDirectory() as d:
+        path = os.path.join(d, "model.gguf")
+        models.write_model(path, cfg, [0], seed=1, fast=True)
+        st = m.Stage(path, 0, 1, n_ctx=2048, n_seq_max=1, n_batch_max=2048)
+    ses = st.session()
+    out = []
+    for T in tokens:
+        host.launches()
+        ses.decode(np.zeros((T, n_embd), np.float32), np.arange(T))
+        out += [(n, g[0]) for n, g, _ in host.launches() if n.startswith("moe_router")]
+    return out
+
+
+@pytest.mark.parametrize("n_embd,n_expert,whole", [(512, 95, False), (512, 96, True), (1024, 95, False), (1024, 512, True), (2048, 512, False)])
+def test_router_of_many_short_expert_rows(n_embd, n_expert, whole):
+    """Many experts over a small hidden size: a token a workgroup while every token has a CU of its own."""
+    v = n_embd // 256
+    got = call(routers, n_embd=n_embd, n_expert=n_expert, tokens=[65, 256, 257, 600, 1000])
+    small = [["moe_router_fused_kernel<%d,1024>" % v, 65], ["moe_router_fused_kernel<%d,1024>" % v, 256]]
+    chunk = [["moe_router_chunk_kernel<%d,2>" % v, 33], ["moe_router_chunk_kernel<%d,2>" % v, 128]]
+    assert got[:2] == (small if whole else chunk)
+    assert got[2:] == [["moe_router_chunk_kernel<%d,2>" % v, 129], ["moe_router_chunk_kernel<%d,3>" % v, 200], ["moe_router_chunk_kernel<%d,4>" % v, 250]]

@@ -300,8 +300,9 @@ def test_qwen3_30b_a3b_shaped_expert_shard_layer(tmp_path):
     st.close()
 
 
-# every hidden size the routers have a kernel for; 27 experts: a last slice of three rows, 130: lanes with three of them
-@pytest.mark.parametrize("n_embd,n_expert,top_k", [(512, 27, 1), (1024, 64, 3), (2048, 64, 3), (2048, 130, 7), (4096, 27, 1)])
+# every hidden size the routers have a kernel for; 27 experts: a last slice of three rows, 130: lanes with three of them; 192 and 385 over
+# short rows: a token a workgroup of sixteen waves
+@pytest.mark.parametrize("n_embd,n_expert,top_k", [(512, 27, 1), (512, 192, 7), (1024, 64, 3), (1024, 385, 7), (2048, 64, 3), (2048, 130, 7), (4096, 27, 1)])
 @pytest.mark.parametrize("masked", [False, True])
 def test_routers_of_steps_and_of_chunks_agree(tmp_path, n_embd, n_expert, top_k, masked):
     """Logits over slices of the experts, then routing and grouping in one workgroup (up to 64 tokens), against logits and routing of
