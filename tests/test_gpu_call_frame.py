@@ -59,6 +59,27 @@ def test_rows_in_place_equal_rows_copied(tmp_path, name, layers, tokens):
     st.close()
 
 
+@pytest.mark.parametrize("where", ["input", "output", "both"])
+def test_rows_in_pinned_host_memory_take_copies(tmp_path, where):
+    """An aligned pointer that a copy accepts, and no memory of the device: what the rows are read from or written to in place."""
+    cfg, st = open_stage(tmp_path, "tiny-llama", 0, 2, 64)
+    for T in (1, 16, 33):
+        x = np.random.Generator(np.random.PCG64(T)).standard_normal((T, cfg["n_embd"])).astype(np.float32)
+        pos, seq = np.zeros(T, np.int32), np.arange(T, dtype=np.int32)
+        want = dev_call(st, x, pos, seq)
+        d_in = torch.empty(x.shape, dtype=torch.float32, pin_memory=True) if where != "output" else torch.empty(x.shape, dtype=torch.float32, device="cuda")
+        d_out = torch.zeros(x.shape, dtype=torch.float32, pin_memory=True) if where != "input" else torch.zeros(x.shape, dtype=torch.float32, device="cuda")
+        assert d_in.data_ptr() % 16 == 0 and d_out.data_ptr() % 16 == 0
+        d_in.copy_(torch.from_numpy(x))
+        torch.cuda.synchronize()
+        ses = st.session()
+        ses.decode_dev(d_in.data_ptr(), pos, d_out.data_ptr(), x.nbytes, seq=seq)
+        ses.synchronize()
+        assert np.array_equal(d_out.cpu().numpy(), want)
+        ses.close()
+    st.close()
+
+
 def test_calls_queued_without_a_wait_keep_their_own_positions(tmp_path):
     cfg, st = open_stage(tmp_path, "tiny-llama", 0, 2, 64)
     E = cfg["n_embd"]
