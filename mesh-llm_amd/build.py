@@ -18,16 +18,24 @@ FLAGS = [
     # leading scalar kernel arguments arrive in SGPRs at wave start instead of through a scalar load (kernels whose
     # start-up chain matters list those arguments first)
     "-mllvm", "-amdgpu-kernarg-preload-count=14",
-    # results of matrix instructions stay in vector registers: kept in accumulation registers, a kernel that also rescales them
-    # copies them over and back (decode attention: 64 of 92 instructions of a block of keys)
-    "-mllvm", "-amdgpu-mfma-vgpr-form=1",
     "-Wall", "-Wno-unused-function", "-Wno-unknown-warning-option",
 ]
+
+# Results of matrix instructions stay in vector registers: kept in accumulation registers, a kernel that also rescales them copies them over
+# and back (decode attention: 64 of 92 instructions of a block of keys; latent attention, 46 to 900 tokens, 3-9% a launch, 32-bit 7%).
+# Not for all files: without accumulation registers linear_rows_kernel is scheduled for more waves and fewer loads under way (33 to 128
+# tokens, 2048 x 2048: 13.3 -> 19.6 us); scans of one chunk lose 9% and long ones gain 1-4%; the K-quant products are the same either way.
+VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
+FILE_FLAGS = {"attn_mma.hip": VGPR_FORM, "latent.hip": VGPR_FORM}
+
+
+def flags_of(src):
+    return FLAGS + FILE_FLAGS.get(os.path.basename(src), [])
 
 
 def _compile(src):
     obj = os.path.join(OBJ, os.path.basename(src) + ".o")
-    cmd = [HIPCC, *FLAGS, "-c", src, "-o", obj]
+    cmd = [HIPCC, *flags_of(src), "-c", src, "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("hipcc failed for %s:\n%s\n%s" % (src, " ".join(cmd), r.stderr))
