@@ -181,7 +181,7 @@ __global__ __launch_bounds__(RT) void moe_router_fused_kernel(const float *__res
 // Bound by the CU's fetch of the whole router matrix from L2 (512 KB at about 95 GB/s: 5.4 us), before it the rows' and the norm's chain,
 // behind it the picks.  So a workgroup takes as many tokens as leave one for every CU.  64 experts x 2048, us, a token a workgroup of sixteen
 // waves / four tokens a workgroup, both with no row ahead (before) and two, three or four tokens: 40 tokens 19.2 / - / 12.6, 333 25.1
-// / - / 12.0, 512 - / 15.9 / 12.6, 600 - / 16.4 / 14.2, 1024 - / 16.9 / 16.7, 2048 - / 29.1 / 29.2.
+// / - / 12.0, 512 - / 15.9 / 12.6, 600 - / 16.4 / 14.2, 1024 - / 16.9 / 16.7, 2048 - / 29.1 / 29.2.  16 experts x 2048: one token 6.5 / - / 5.0, 16 7.8 / - / 6.2.
 constexpr int CHUNK_WAVES = 8;
 template <int NV, int TOKENS>
 __global__ __launch_bounds__(64 * CHUNK_WAVES) void moe_router_chunk_kernel(const float *__restrict__ x, const float *__restrict__ norm_w,

@@ -1131,9 +1131,9 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
             mr.logits = s->moe_logits; mr.mask = s->expert_mask_on ? s->expert_mask : nullptr;
             mr.ids = s->moe_ids; mr.weights = s->moe_w; mr.n_expert = ne; mr.top_k = k; mr.norm_w = 1;
             const bool want_groups = s->tune.moe_group && moe_group_supported(T * k, ne) && moe_max_items(T * k, ne) <= 65535;
-            // a batch of decode steps over K-quant experts: the expert products on the matrix cores, 16 pairs of an expert per pass
-            // (worth it from about four pairs per expert: below that the mat-vec kernel, which only computes the columns an
-            // item has, is as fast)
+            // batches that neither of the two below takes (33 and more tokens without GEMM-layout copies, or moe_gemm=0): the expert products
+            // on the integer matrix cores, 16 pairs of an expert per pass (worth it from about four pairs per expert: below that the
+            // mat-vec kernel, which only computes the columns an item has, is as fast)
             const bool mfma = want_groups && s->xq && (size_t)T <= s->xq_tokens && T * k >= 4 * ne && E % 256 == 0 && ffe % 256 == 0 &&
                               type_is_tiled(L.gate_exps.type) && L.up_exps.type == L.gate_exps.type && type_is_tiled(L.down_exps.type) &&
                               moe_max_items(T * k, ne, SKINNY_ITEM_PAIRS) <= 65535;
@@ -1185,7 +1185,9 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
                 if ((rc = moe_combine_slots(s->x, layer_output(s, il), s->moe_out_slots, s->moe_w, s->moe_sorted.slot_of_pair, T, E, k, stream)) != MESH_OK) return rc;
                 continue;
             }
-            // a batch of decode steps over K-quant experts: eight pairs of an expert per pass on the f16 matrix cores
+            // A batch of decode steps over K-quant experts: eight pairs of an expert per pass on the f16 matrix cores, also with many pairs per
+            // expert.  One layer, us, integer kernel / this one: 64 experts of 768 x 2048, top 8, 32 tokens 144 / 101; 32 experts 16 tokens 91 / 72, 32
+            // tokens 120 / 96; 20 experts 12 tokens (4.8 pairs each) 89 / 66, 32 tokens (12.8) 113 / 90; 24 of 768 x 4096, 32 tokens 148 / 112.
             const bool step = want_groups && s->moe_step_x && T >= s->tune.moe_step_min_tokens && T <= EXPERT_STEP_TOKENS_MAX &&
                               L.gate_inp.type == MESH_F32 && moe_router_group_supported(E, ne, k, T) && L.up_exps.type == L.gate_exps.type &&
                               expert_step_supported(L.gate_exps.type, L.down_exps.type, E, ffe);
@@ -1586,6 +1588,8 @@ int stage_decode(mesh_session *s, const mesh_batch *b, const void *in, int in_fm
     }
     size_t len = 0;
     uint8_t *h_out = static_cast<uint8_t *>(s->h_io) + s->io_stage_bytes;
+    // one row of logits: the product's stores go over the bus themselves (a call of one layer and the head, copied / so: 128256 rows of
+    // 4096 194 / 165 us, 151936 of 2048 154 / 127)
     const bool direct = out_fmt == MESH_LOGITS && wanted == 1;
     if (direct) d_out = h_out;
     if ((rc = decode_core(s, b, token_ids, d_in, eff_in_fmt, d_out, out_fmt, std::min(out_cap, s->io_out_bytes), &len)) != MESH_OK) {

@@ -155,7 +155,6 @@ struct mesh_session {
     size_t io_stage_bytes = 0;      // input half; the output half (io_out_bytes) follows it
     size_t io_out_bytes = 0;
     void *h_io = nullptr;           // pinned host staging, same split
-    int attn_splits_max = 0;
     // set per call: the caller's f32 buffers the first layer reads and the last one writes in place of x (null: x itself)
     const float *x_in = nullptr;
     float *x_out = nullptr;
