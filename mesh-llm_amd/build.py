@@ -22,11 +22,12 @@ FLAGS = [
 ]
 
 # Results of matrix instructions stay in vector registers: kept in accumulation registers, a kernel that also rescales them copies them over
-# and back (decode attention: 64 of 92 instructions of a block of keys; latent attention, 46 to 900 tokens, 3-9% a launch, 32-bit 7%).
+# and back (decode attention: 64 of 92 instructions of a block of keys; latent attention, 46 to 900 tokens, 3-9% a launch, 32-bit 7%; state scans
+# of 33 tokens and more 1-5%, those of one chunk 5.3 -> 5.8 us the other way).
 # Not for all files: without accumulation registers linear_rows_kernel is scheduled for more waves and fewer loads under way (33 to 128
-# tokens, 2048 x 2048: 13.3 -> 19.6 us); scans of one chunk lose 9% and long ones gain 1-4%; the K-quant products are the same either way.
+# tokens, 2048 x 2048: 13.3 -> 19.6 us).  The K-quant products are the same either way.
 VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
-FILE_FLAGS = {"attn_mma.hip": VGPR_FORM, "latent.hip": VGPR_FORM}
+FILE_FLAGS = {"attn_mma.hip": VGPR_FORM, "gated_state.hip": VGPR_FORM, "latent.hip": VGPR_FORM}
 
 
 def flags_of(src):
