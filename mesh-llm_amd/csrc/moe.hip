@@ -267,7 +267,7 @@ static void launch_router_chunk(const MoeRouteArgs &a, const float *x, int ldx, 
 
 // Router logits of a batch of decode steps, a workgroup per token and four experts, one row of the matrix per wave.  The bits of router_logits:
 // the sums of a lane's elements and of the lanes go the same way.  planes (optional): the normalised row as pairs of f16.
-// Bound by its chain (row, sum of squares, dot product).  16 tokens, 64 experts x 2048: 3.6 us; 9.4 with sixteen rows a workgroup, each wave of which
+// Bound by its chain (row, sum of squares, dot product).  16 tokens, 64 experts x 2048: 3.6 us (3.5-4.0 in traces of whole steps); 9.4 with sixteen rows a workgroup, each wave of which
 // loaded and normalised the token's row for itself and added lanes up through the LDS unit.  (Before, the last of those workgroups to
 // arrive routed and grouped behind a hand-over between workgroups: 19.4 us in one launch, against 3.6 + 5.6 now.)
 constexpr int SLICE_THREADS = 256, SLICE_WAVES = SLICE_THREADS / 64;
@@ -443,7 +443,7 @@ __global__ __launch_bounds__(GROUP_THREADS) void moe_group_kernel(const int32_t 
 // Routing of a small batch and the grouping of its pairs in one single-workgroup launch: wave w routes tokens w,
 // w + 16, ... from their logits, then the workgroup groups the pairs it has just written (the barrier in between
 // also makes those writes visible to the whole workgroup).  A chain: 9.1 us with reductions through the LDS unit and a rank counted
-// over all candidates, 5.6 now (16 tokens, 64 experts, top 8; 4.5 of it without the grouping).
+// over all candidates, 5.6 now (16 tokens, 64 experts, top 8, timed apart; 4.5 of it without the grouping; 6.8-7.2 in traces of whole steps).
 // (the routing arguments as leading scalars: preloaded into SGPRs, see gemv.hip)
 __global__ __launch_bounds__(GROUP_THREADS) void moe_route_group_kernel(const float *p_logits, const float *p_mask, int32_t *p_ids, float *p_weights,
                                                                         int T, int p_n_expert, int p_top_k, int p_norm_w,
