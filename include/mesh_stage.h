@@ -302,7 +302,7 @@ int mesh_session_f16_saturations(mesh_session *session, uint64_t *count);
  *     moe_router_tail=1    no effect; accepted from callers that set it
  *     moe_fuse_quant=1     the expert combine step quantises for the next layer
  *     moe_gemm=1, moe_gemm_min_pairs=4   prefill-sized expert products on the large-tile GEMM
- *     moe_step_min_tokens=1  expert products of up to 32 decode steps (below moe_gemm_min_pairs) on the f16 matrix cores from this
+ *     moe_step_min_tokens=1  expert products of up to 32 decode steps (where moe_gemm does not take them) on the f16 matrix cores from this
  *                          many tokens, activations as scaled pairs of f16 (fewer: the grouped expert mat-vec)
  *     reg_min_tokens=17, reg_min_blocks=192   gate / up of a batch of decode steps (up to 32) of at least that many and of
  *                          at least that many blocks of 64 rows on the GEMM layout instead of the f16 skinny GEMM

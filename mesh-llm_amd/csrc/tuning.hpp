@@ -41,7 +41,7 @@ struct Tuning {
     int moe_fuse_quant = 1;        // the expert combine step quantises for the next layer's projections
     int moe_gemm = 1;              // prefill-sized expert products as tiles of the large-tile GEMM
     int moe_gemm_min_pairs = 4;    // ... from this many pairs per expert on average
-    int moe_step_min_tokens = 1;   // expert products of decode steps (up to 32 tokens, below moe_gemm_min_pairs) on the f16 matrix cores from this many tokens
+    int moe_step_min_tokens = 1;   // expert products of decode steps (up to 32 tokens, where moe_gemm does not take them) on the f16 matrix cores from this many tokens
     int reg_min_tokens = 17;       // gate / up of a batch of decode steps (up to 32) of at least this many on the GEMM layout, fragments formed in registers
     int reg_min_blocks = 192;      // ... where the pair has at least this many blocks of 64 rows
     int tile_min_tokens = 129;     // K-quant products of at least this many tokens on the large tile over f16 copies of the weights, where the stage keeps them
