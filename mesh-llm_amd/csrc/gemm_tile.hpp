@@ -57,6 +57,9 @@ constexpr int gt_waves_per_simd(int WM, int WT) { return 160 * 1024 / gt_lds_byt
 //   28672, 4096, 2048: 256x256 419, 256x192 431, 256x128 451, 128x128 479     28672, 4096, 512: 111, 154, 121, 139
 //   28672, 4096, 256:  88, 85, 74, 79        6144, 4096, 2048: 100, 140, 110, 108        6144, 4096, 512: 72, 62, 55, 39
 //   4096, 4096, 2048:  84, 71, 68, 76        4096, 4096, 512: 71, 61, 54, 38             2048, 8192, 900: 129, 119, 88, 53
+// Slices in any number where each keeps 1280 of K (us without the adding): 4096, 14336, 333 on 256x128 in 4 / 5 / 6 slices 54.3 / 49.9 / 53 (192,
+// 240 and 288 workgroups), 6144, 4096, 333 on 256x128 in 2 / 3 slices 27 / 23.9, on 256x192 in 4 25.5; shorter ones gain less than the model's
+// error (4096, 4096, 333 on 256x128 in 4 / 5 slices 19.5 / 19.1, their adding 1.3 more) and stay at powers of two.
 struct GtPlan {
     int wm = 2, wt = 2, slices = 1, k_slice = 0;       // waves (of 64 rows) by waves (of 64 tokens), one of the tiles below; steps of a slice
 };
@@ -76,7 +79,8 @@ inline GtPlan gt_plan(int M, int T, int K, int slices_max, size_t slices_room, d
     double least = 0;
     const int steps = K / GT_K;
     for (const auto &t : tiles)
-        for (int s = 1; s <= slices_max && (s == 1 || ((size_t)s <= slices_room && K / s >= 256)); s *= 2) {
+        for (int s = 1; s <= slices_max && (s == 1 || ((size_t)s <= slices_room && K / s >= 256)); ++s) {
+            if ((s & (s - 1)) != 0 && K / s < 1280) continue;
             const long n = (long)((M + 64 * t.wm - 1) / (64 * t.wm)) * ((T + 64 * t.wt - 1) / (64 * t.wt)) * s;
             const int k_slice = (steps + s - 1) / s;
             const double ns = t.few + t.full * (n < n_cu ? (double)n / n_cu : 1.0);

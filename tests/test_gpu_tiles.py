@@ -84,6 +84,9 @@ KQUANT_MANY_CASES = [
     ((4096, 12, 3, 256), 129, (4, 2, 8), (2, 2, 4), (2, 2, 8), (2, 2, 1)),
     ((2560, 30, 5, 256), 129, (4, 3, 8), (2, 2, 4), (2, 2, 8), (2, 2, 1)),
     ((256, 22, 11, 256), 700, (4, 2, 1), (2, 2, 8), (2, 2, 1), (2, 2, 1)),
+    # slices that are no power of two: five of 42 steps, the last of 40; three of 67, the last of 66
+    ((2304, 2, 1, 6656), 129, (2, 2, 8), (2, 2, 1), (2, 2, 1), (2, 2, 5)),
+    ((2816, 2, 1, 6400), 257, (2, 2, 8), (2, 2, 1), (4, 3, 2), (2, 2, 3)),
 ]
 
 
