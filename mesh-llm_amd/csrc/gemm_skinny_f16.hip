@@ -75,86 +75,54 @@ struct SkinnyKernelArgs {
 template <int TYPE>
 struct BFrags {
     uint4 b[8];
-    // x: the k8-major block (uniform), lane_off: this lane's column and quarter offset in halfs
-    __device__ __forceinline__ void load(const _Float16 *x, int lane_off, int sb) {
-        const _Float16 *base = x + (size_t)sb * (QK_K * 16);      // uniform
+    // base: the super-block's k8-major activations (uniform), lane_off: this lane's column and quarter offset in halfs
+    __device__ __forceinline__ void load(const _Float16 *base, int lane_off) {
 #pragma unroll
         for (int t = 0; t < 8; ++t) b[t] = ldg<uint4>(base + lane_off + frag_k<TYPE>(t) * 16);
     }
 };
 
-// element (row k, column t) of k8-major f16 activations with K rows per column: block t / 16 of 16 * K halfs
-__device__ __forceinline__ size_t k8_at(int K, int k, int t) { return (size_t)(t >> 4) * 16 * K + ((size_t)(k >> 3) * 16 + (t & 15)) * 8 + (k & 7); }
+// Where a lane's share of the activation fragments lies: lane (n = m, g) supplies column n, quarter g.  A column past the call's tokens is
+// its block's last one again, which takes no line of its own, and what it yields is dropped: the fragments of a super-block are 8 KB to
+// 2.3 of weights, and half of their lines go (eight 8B-shaped layers, 5 tokens 612 -> 590 us; the zeros that lie there read before).
+template <int TYPE, int NC>
+struct SkinnyColumns {
+    int at[NC];
+    __device__ __forceinline__ SkinnyColumns(int m, int g, int T) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) at[c] = quarter_k<TYPE>(g) * 16 + min(m, max(T - 1 - SK_NT * c, 0)) * 8;
+    }
+};
 
-// KB per wave and column block that hold a wave's share of the partial sums
-constexpr int NORM_CHUNKS = SKINNY_F16_NORM_PARTS_MAX / SK_WAVES * SK_NT / 256;
-static_assert(NORM_CHUNKS * 256 * SK_WAVES == SKINNY_F16_NORM_PARTS_MAX * SK_NT, "shares of whole KB");
-
-// most tile-rows a workgroup of the launch has (p_split = tile-rows per workgroup | workgroups with one more << 16)
-__device__ __forceinline__ int rows_here_max(unsigned p_split) { return (int)(p_split & 0xFFFFu) + ((p_split >> 16) ? 1 : 0); }
-
-// NC: blocks of 16 activation columns one pass over the weights multiplies with (1: up to 16 tokens, 2: up to 32).
-// bx: the workgroup's index among those of its launch part (the whole launch, or one side of a pair launch).
-template <int TYPE, int NU, int SEGS, int NC>
-__device__ __forceinline__ void skinny_workgroup(int bx, const _Float16 *p_x, const uint8_t *p_w0, const uint8_t *p_w1, const uint8_t *p_w2, int p_K,
-                                                 int p_ks, unsigned p_begins, unsigned p_split, const SkinnyKernelArgs &a) {
-    // (p_begins = first tile-row of matrix 1 | of matrix 2 << 16; p_split = tile-rows per workgroup | workgroups with one
-    // more << 16, computed on the host: no division and no grid-size load stand before the first weight load)
-    const int p_begin1 = (int)(p_begins & 0xFFFFu), p_begin2 = (int)(p_begins >> 16);
-    // (leading scalar arguments: preloaded into SGPRs, see gemv.hip)
-    extern __shared__ __align__(16) uint8_t smem[];
-    float *red = reinterpret_cast<float *>(smem);         // [KS][rows_here][NU][16 rows][16 NC columns]
-    constexpr int TB = TileRegs<TYPE>::BYTES;
-    const int K = p_K, nsb = K / QK_K;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);       // scalar: tile addresses become SGPR base + lane offset
-    const int m = lane & 15, g = lane >> 4;
-    const int src_lane4 = 4 * (4 * m + g);                // byte address, for ds_bpermute, of the lane that loaded row m, quarter g
-    const int KS = p_ks, LK = __builtin_ctz((unsigned)KS), RS = SK_WAVES >> LK;      // KS is a power of two
-    const int ks = wave & (KS - 1), rs = wave >> LK;
-    const int sq = (int)(p_split & 0xFFFFu), sr = (int)(p_split >> 16);
-    const int tr0 = bx * sq + (bx < sr ? bx : sr);
-    const int rows_here = sq + (bx < sr ? 1 : 0);
-    const int n_i = rs < RS ? (nsb - ks + KS - 1) >> LK : 0;        // super-blocks of this wave (ks < KS <= nsb)
-    const size_t row_stride = (size_t)nsb * TB;
-    // B fragments: lane (n = m, g) supplies column n, quarter g (columns beyond T hold zeros)
-    const int lane_off = quarter_k<TYPE>(g) * 16 + m * 8;
-    // flat tile index f = ii * SEGS + seg; seg -> (local tile-row j, matrix u).  A segment past the workgroup's rows reads the wave's
-    // first one again and is dropped at the end: the walk has no branch (see below).
-    auto seg_valid = [&](int seg) { return rs + RS * (seg / NU) < rows_here; };
-    auto tile_ptr = [&](int ii, int seg) -> const uint8_t * {
-        const int tr = tr0 + rs + (seg_valid(seg) ? RS * (seg / NU) : 0);
-        int mi = seg % NU;
-        if (NU == 1) mi = (tr >= p_begin1 ? 1 : 0) + (tr >= p_begin2 ? 1 : 0);
-        // (offsets added under conditions: an indexed kernel-argument array is fetched with a load, and a three-way
-        // select of preloaded pointers becomes a table in scratch memory)
-        const uint8_t *wb = p_w0 + (mi >= 1 ? p_w1 - p_w0 : (ptrdiff_t)0) + (mi >= 2 ? p_w2 - p_w1 : (ptrdiff_t)0);
-        return wb + (size_t)tr * row_stride + (size_t)(ks + KS * ii) * TB;
-    };
-    // a wave without a valid first segment has nothing at all
-    const bool any = n_i > 0 && seg_valid(0);
-    constexpr int RB = SEGS % SK_DEPTH == 0 ? 1 : SK_DEPTH;      // super-blocks per round: ring slots static inside it
+// A wave's walk: its n_i super-blocks of SEGS (tile-row, matrix) segments each, tile_ptr(ii, seg) the tile of one, times NC blocks of 16
+// activation columns.  x: the activations of its first super-block; x_step, x_block: halfs to its next one and to the next block of columns.
+template <int TYPE, int SEGS, int NC>
+struct SkinnyWalk {
+    static constexpr int RB = SEGS % SK_DEPTH == 0 ? 1 : SK_DEPTH;      // super-blocks per round: ring slots static inside it
     static_assert(RB <= 2 && RB * SEGS % SK_DEPTH == 0, "ring slots must be static inside a round, and at most one super-block left over");
-
-    constexpr int NT = SK_NT * NC;                        // activation columns of this launch
+    const _Float16 *x;
+    unsigned x_step, x_block;         // (32 bits: an address is one scalar product and a sum)
+    int n_i, lane, g, src_lane4;
+    SkinnyColumns<TYPE, NC> cols;
     TileRegs<TYPE> ring[SK_DEPTH];
-    f4_t D[SEGS][NC];
-#pragma unroll
-    for (int s = 0; s < SEGS; ++s)
-#pragma unroll
-        for (int c = 0; c < NC; ++c) D[s][c] = f4_t{0.f, 0.f, 0.f, 0.f};
+    BFrags<TYPE> Bw[NC];
+
+    // (a constructor: braces around the members would clear the registers of ring and Bw before the first load)
+    __device__ __forceinline__ SkinnyWalk(const _Float16 *x_, unsigned x_step_, unsigned x_block_, int n_i_, int lane_, int g_, int src_lane4_, const SkinnyColumns<TYPE, NC> &cols_)
+        : x(x_), x_step(x_step_), x_block(x_block_), n_i(n_i_), lane(lane_), g(g_), src_lane4(src_lane4_), cols(cols_) {}
 
     // The walk has no branch inside a round of tiles: a tile past the end is the wave's last one again (a cache hit).  The compiler
     // then knows how many loads are in flight at every point and waits for one tile without draining the others; with a branch
     // around a tile or a load it assumes the worst at the join, and every round waited for everything it had just requested.
-    auto load_tile = [&](TileRegs<TYPE> &dst, int ii, int seg) { dst.load(tile_ptr(ii < n_i ? ii : n_i - 1, seg), lane); };
+    template <class TilePtr> __device__ __forceinline__ void load_tile(TileRegs<TYPE> &dst, int ii, int seg, const TilePtr &tile_ptr) {
+        dst.load(tile_ptr(ii < n_i ? ii : n_i - 1, seg), lane);
+    }
     // Activation fragments: 8 KB per super-block, column block and wave.  Only ONE super-block is held (32 registers per
     // column block) and every fragment is fetched again, for the next super-block, right behind the last MFMAs that read
     // it: one tile's time ahead of its use, enough for a hit in L2.  (Two whole super-blocks in registers, fetched a
     // super-block ahead, cost 32 more registers per column block and measured 6% slower at 16 columns.)
-    BFrags<TYPE> Bw[NC];
-    auto step = [&](const TileRegs<TYPE> &loaded, f4_t (&acc)[NC], bool refill, int next_ii) {
-        const _Float16 *nb = p_x + (size_t)(ks + KS * (next_ii < n_i ? next_ii : n_i - 1)) * (QK_K * 16);
+    __device__ __forceinline__ void step(const TileRegs<TYPE> &loaded, f4_t (&acc)[NC], bool refill, int next_ii) {
+        const _Float16 *nb = x + (unsigned)(next_ii < n_i ? next_ii : n_i - 1) * x_step;
         TileRegs<TYPE> tile = loaded;
         to_mfma_lanes(tile, src_lane4);
         TileFrags<TYPE> F;
@@ -174,7 +142,7 @@ __device__ __forceinline__ void skinny_workgroup(int bx, const _Float16 *p_x, co
             }
             if (refill) {
 #pragma unroll
-                for (int c = 0; c < NC; ++c) Bw[c].b[t] = ldg<uint4>(nb + (size_t)c * SK_NT * K + lane_off + frag_k<TYPE>(t) * 16);
+                for (int c = 0; c < NC; ++c) Bw[c].b[t] = ldg<uint4>(nb + c * x_block + cols.at[c] + frag_k<TYPE>(t) * 16);
             }
         }
         // a lane's outputs are all of weight row m, whose scales it holds
@@ -185,13 +153,93 @@ __device__ __forceinline__ void skinny_workgroup(int bx, const _Float16 *p_x, co
                 acc[c][i] = fmaf(F.d, sum[c][i], acc[c][i]);
                 if constexpr (TileFrags<TYPE>::MINIMUM) acc[c][i] = fmaf(F.ndmin, low[c][i], acc[c][i]);
             }
-    };
-    if (any) {
-#pragma unroll
-        for (int f = 0; f < SK_DEPTH; ++f) load_tile(ring[f], f / SEGS, f % SEGS);
-#pragma unroll
-        for (int c = 0; c < NC; ++c) Bw[c].load(p_x + (size_t)c * SK_NT * K, lane_off, ks);
     }
+    // clears the sums and requests the first tiles and fragments
+    template <class TilePtr> __device__ __forceinline__ void start(f4_t (&D)[SEGS][NC], bool any, const TilePtr &tile_ptr) {
+#pragma unroll
+        for (int s = 0; s < SEGS; ++s)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) D[s][c] = f4_t{0.f, 0.f, 0.f, 0.f};
+        if (any) {
+#pragma unroll
+            for (int f = 0; f < SK_DEPTH; ++f) load_tile(ring[f], f / SEGS, f % SEGS, tile_ptr);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) Bw[c].load(x + c * x_block, cols.at[c]);
+        }
+    }
+    template <class TilePtr> __device__ __forceinline__ void run(f4_t (&D)[SEGS][NC], const TilePtr &tile_ptr) {
+        int ii = 0;
+        for (; ii + RB <= n_i; ii += RB) {
+#pragma unroll
+            for (int q = 0; q < RB * SEGS; ++q) {
+                const int seg = q % SEGS, slot = q % SK_DEPTH;
+                step(ring[slot], D[seg], seg == SEGS - 1, ii + q / SEGS + 1);
+                // (the tile goes out behind the fragments, which are needed first: loads return in order)
+                __builtin_amdgcn_sched_barrier(0);
+                load_tile(ring[slot], ii + (q + SK_DEPTH) / SEGS, (q + SK_DEPTH) % SEGS, tile_ptr);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (RB > 1 && ii < n_i) {
+#pragma unroll
+            for (int seg = 0; seg < SEGS; ++seg) step(ring[seg % SK_DEPTH], D[seg], false, 0);
+        }
+    }
+};
+
+// element (row k, column t) of k8-major f16 activations with K rows per column: block t / 16 of 16 * K halfs
+__device__ __forceinline__ size_t k8_at(int K, int k, int t) { return (size_t)(t >> 4) * 16 * K + ((size_t)(k >> 3) * 16 + (t & 15)) * 8 + (k & 7); }
+
+// KB per wave and column block that hold a wave's share of the partial sums
+constexpr int NORM_CHUNKS = SKINNY_F16_NORM_PARTS_MAX / SK_WAVES * SK_NT / 256;
+static_assert(NORM_CHUNKS * 256 * SK_WAVES == SKINNY_F16_NORM_PARTS_MAX * SK_NT, "shares of whole KB");
+
+// most tile-rows a workgroup of the launch has (p_split = tile-rows per workgroup | workgroups with one more << 16)
+__device__ __forceinline__ int rows_here_max(unsigned p_split) { return (int)(p_split & 0xFFFFu) + ((p_split >> 16) ? 1 : 0); }
+
+// NC: blocks of 16 activation columns one pass over the weights multiplies with (1: up to 16 tokens, 2: up to 32).
+// bx: the workgroup's index among those of its launch part (the whole launch, or one side of a pair launch).
+template <int TYPE, int NU, int SEGS, int NC>
+__device__ __forceinline__ void skinny_workgroup(int bx, const _Float16 *p_x, const uint8_t *p_w0, const uint8_t *p_w1, const uint8_t *p_w2, int p_K,
+                                                 int p_ks, unsigned p_begins, unsigned p_split, const SkinnyKernelArgs &a) {
+    // (p_ks = waves along K | columns << 16; p_begins = first tile-row of matrix 1 | of matrix 2 << 16; p_split = tile-rows per workgroup | workgroups with one
+    // more << 16, computed on the host: no division and no grid-size load stand before the first weight load)
+    const int p_begin1 = (int)(p_begins & 0xFFFFu), p_begin2 = (int)(p_begins >> 16);
+    // (leading scalar arguments: preloaded into SGPRs, see gemv.hip)
+    extern __shared__ __align__(16) uint8_t smem[];
+    float *red = reinterpret_cast<float *>(smem);         // [KS][rows_here][NU][16 rows][16 NC columns]
+    constexpr int TB = TileRegs<TYPE>::BYTES;
+    const int K = p_K, nsb = K / QK_K;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);       // scalar: tile addresses become SGPR base + lane offset
+    const int m = lane & 15, g = lane >> 4;
+    const int src_lane4 = 4 * (4 * m + g);                // byte address, for ds_bpermute, of the lane that loaded row m, quarter g
+    const int KS = p_ks & 0xFFFF, T = p_ks >> 16, LK = __builtin_ctz((unsigned)KS), RS = SK_WAVES >> LK;      // KS is a power of two
+    const int ks = wave & (KS - 1), rs = wave >> LK;
+    const int sq = (int)(p_split & 0xFFFFu), sr = (int)(p_split >> 16);
+    const int tr0 = bx * sq + (bx < sr ? bx : sr);
+    const int rows_here = sq + (bx < sr ? 1 : 0);
+    const int n_i = rs < RS ? (nsb - ks + KS - 1) >> LK : 0;        // super-blocks of this wave (ks < KS <= nsb)
+    const size_t row_stride = (size_t)nsb * TB;
+    const SkinnyColumns<TYPE, NC> cols(m, g, T);
+    // flat tile index f = ii * SEGS + seg; seg -> (local tile-row j, matrix u).  A segment past the workgroup's rows reads the wave's
+    // first one again and is dropped at the end: the walk has no branch (see below).
+    auto seg_valid = [&](int seg) { return rs + RS * (seg / NU) < rows_here; };
+    auto tile_ptr = [&](int ii, int seg) -> const uint8_t * {
+        const int tr = tr0 + rs + (seg_valid(seg) ? RS * (seg / NU) : 0);
+        int mi = seg % NU;
+        if (NU == 1) mi = (tr >= p_begin1 ? 1 : 0) + (tr >= p_begin2 ? 1 : 0);
+        // (offsets added under conditions: an indexed kernel-argument array is fetched with a load, and a three-way
+        // select of preloaded pointers becomes a table in scratch memory)
+        const uint8_t *wb = p_w0 + (mi >= 1 ? p_w1 - p_w0 : (ptrdiff_t)0) + (mi >= 2 ? p_w2 - p_w1 : (ptrdiff_t)0);
+        return wb + (size_t)tr * row_stride + (size_t)(ks + KS * ii) * TB;
+    };
+    // a wave without a valid first segment has nothing at all
+    const bool any = n_i > 0 && seg_valid(0);
+    constexpr int NT = SK_NT * NC;                        // activation columns of this launch
+    f4_t D[SEGS][NC];
+    SkinnyWalk<TYPE, SEGS, NC> walk(p_x + (size_t)ks * (QK_K * 16), (unsigned)KS * (QK_K * 16), (unsigned)SK_NT * K, n_i, lane, g, src_lane4, cols);
+    walk.start(D, any, tile_ptr);
     // What the tail of the workgroup reads is requested here, behind the first tiles: fetched where it is used, the norm's
     // partial sums cost 2.9 us behind the weight stream, the residual or the rotation's operands 1.5 - 2.
     // (Branch-free: a launch or thread that has no use for an operand reads the first activations instead.)
@@ -231,24 +279,7 @@ __device__ __forceinline__ void skinny_workgroup(int bx, const _Float16 *p_x, co
             pre_freq[k] = *(pre_rot[k] ? a.rope.inv_freq + (dd >> 1) : idle);
         }
     }
-    if (any) {
-        int ii = 0;
-        for (; ii + RB <= n_i; ii += RB) {
-#pragma unroll
-            for (int q = 0; q < RB * SEGS; ++q) {
-                const int seg = q % SEGS, slot = q % SK_DEPTH;
-                step(ring[slot], D[seg], seg == SEGS - 1, ii + q / SEGS + 1);
-                // (the tile goes out behind the fragments, which are needed first: loads return in order)
-                __builtin_amdgcn_sched_barrier(0);
-                load_tile(ring[slot], ii + (q + SK_DEPTH) / SEGS, (q + SK_DEPTH) % SEGS);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        if (RB > 1 && ii < n_i) {
-#pragma unroll
-            for (int seg = 0; seg < SEGS; ++seg) step(ring[seg % SK_DEPTH], D[seg], false, 0);
-        }
-    }
+    if (any) walk.run(D, tile_ptr);
     // partial sums of this wave: D[seg] holds row m, columns 4g..4g+3 of segment seg
 #pragma unroll
     for (int seg = 0; seg < SEGS; ++seg) {
@@ -394,7 +425,7 @@ static int launch_skinny(const SkinnyKernelArgs &ka, int grid, size_t smem, hipS
         attr_set = true;
     }
     MESH_LAUNCH((gemm_skinny_kernel<TYPE, NU, SEGS, NC>), dim3((unsigned)grid), dim3(SK_THREADS), smem, stream, ka.x, ka.wbase[0], ka.wbase[1] ? ka.wbase[1] : ka.wbase[0],
-                ka.wbase[2] ? ka.wbase[2] : ka.wbase[0], ka.K, ka.ks, ka.tile_begin[3], (unsigned)ka.tile_begin[1] | ((unsigned)ka.tile_begin[2] << 16),
+                ka.wbase[2] ? ka.wbase[2] : ka.wbase[0], ka.K, ka.ks | ka.T << 16, ka.tile_begin[3], (unsigned)ka.tile_begin[1] | ((unsigned)ka.tile_begin[2] << 16),
                 (unsigned)(ka.tile_begin[3] / grid) | ((unsigned)(ka.tile_begin[3] % grid) << 16), ka);
     MESH_LAUNCH_CHECK();
     return MESH_OK;
@@ -524,7 +555,7 @@ static int launch_pair(const SkinnyKernelArgs &ka, const SkinnyKernelArgs &kb, i
         attr_set = true;
     }
     MESH_LAUNCH((gemm_skinny_pair_kernel<SEGS_A, SEGS_B, NC>), dim3((unsigned)(grid_a + grid_b)), dim3(SK_THREADS), smem, stream, ka.x, ka.wbase[0],
-                ka.wbase[1] ? ka.wbase[1] : ka.wbase[0], ka.K, ka.ks, grid_a, (unsigned)ka.tile_begin[1] | ((unsigned)ka.tile_begin[2] << 16),
+                ka.wbase[1] ? ka.wbase[1] : ka.wbase[0], ka.K, ka.ks | ka.T << 16, grid_a, (unsigned)ka.tile_begin[1] | ((unsigned)ka.tile_begin[2] << 16),
                 (unsigned)(ka.tile_begin[3] / grid_a) | ((unsigned)(ka.tile_begin[3] % grid_a) << 16),
                 (unsigned)(kb.tile_begin[3] / grid_b) | ((unsigned)(kb.tile_begin[3] % grid_b) << 16), kb.wbase[0], ka, kb);
     MESH_LAUNCH_CHECK();
