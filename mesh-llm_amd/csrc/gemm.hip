@@ -1062,6 +1062,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_epilogue_kernel(GemmArgs a, i
 // 100 1157 / 1273, 200 1596 / 1704, 333 behind 1500 2137 / 2210, 512 2500 / 2625, 800 3849 / 3876; four 32B-shaped layers 40 tokens
 // 734 / 754, 150 1296 / 1338, 400 2217 / 2274: at every count that splits.
 constexpr int SN_THREADS = 512;
+static_assert(GEMM_NORM_ROW_MAX == 2 * 8 * SN_THREADS, "two groups of eight a thread");
 template <int NG>              // groups of 8 elements a thread has: rows of up to NG * 4096
 __global__ __launch_bounds__(SN_THREADS) void gemm_splitk_epilogue_norm_kernel(GemmArgs a, int row_blocks) {
     __shared__ float s_ss[SN_THREADS / 64];
@@ -1137,7 +1138,7 @@ __global__ __launch_bounds__(SN_THREADS) void gemm_splitk_epilogue_norm_kernel(G
 }
 
 bool gemm_norm_rides(const GemmArgs &a) {
-    return a.n_seg <= 1 && !a.y16_k8 && !a.bias && a.residual && !a.tiles && a.M % 8 == 0 && a.M <= 2 * 8 * SN_THREADS &&
+    return a.n_seg <= 1 && !a.y16_k8 && !a.bias && a.residual && !a.tiles && a.M % 8 == 0 && a.M <= GEMM_NORM_ROW_MAX &&
            a.ldy % 4 == 0 && a.ldres % 4 == 0 && gemm_split_count(a) > 1;
 }
 

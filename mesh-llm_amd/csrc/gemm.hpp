@@ -107,6 +107,7 @@ bool gemm_tile_takes(const GemmArgs &a);
 int gemm_tile_slices(const GemmArgs &a);
 int gemm_tile(const GemmArgs &a, hipStream_t stream);
 int gemm_add_slices(const GemmArgs &a, int row_blocks, hipStream_t stream);
+constexpr int GEMM_NORM_ROW_MAX = 8192;         // longest row whose next norm it writes
 
 // Skinny GEMM for a batch of decode steps (gemm_skinny.hip): up to three tiled K-quant matrices sharing the
 // activations, any T (processed 16 columns at a time), epilogues as in the mat-vec kernel, integer dot products on
@@ -172,6 +173,10 @@ struct SkinnyF16Args {
     struct NormIn { const float *part = nullptr; int n_parts = 0; float eps = 0.f; } norm_in;
 };
 int gemm_skinny_f16(const SkinnyF16Args &a, hipStream_t stream);
+// The same product cut along K, where gemm_skinny_f16_slices (with the scratch there is) says more than 1; no norm hand-over.  The slices meet
+// in sum.part and are added by gemm_add_slices, which also writes the next norm's rows (sum.next_w, next_eps, next_x16, sat).
+int gemm_skinny_f16_slices(const SkinnyF16Args &a, size_t part_bytes);
+int gemm_skinny_f16_sliced(const SkinnyF16Args &a, const GemmArgs &sum, hipStream_t stream);
 // workgroups a producer launch of `a` will have (= partial sums per token it writes); 0 when the launch is not valid
 int gemm_skinny_f16_workgroups(const SkinnyF16Args &a);
 constexpr int SKINNY_F16_NORM_PARTS_MAX = 256;

@@ -182,7 +182,10 @@ struct SkinnyWalk {
         }
         if (RB > 1 && ii < n_i) {
 #pragma unroll
-            for (int seg = 0; seg < SEGS; ++seg) step(ring[seg % SK_DEPTH], D[seg], false, 0);
+            for (int seg = 0; seg < SEGS; ++seg) {
+                step(ring[seg % SK_DEPTH], D[seg], false, 0);
+                if (seg + SK_DEPTH < SEGS) load_tile(ring[seg % SK_DEPTH], ii, seg + SK_DEPTH, tile_ptr);
+            }
         }
     }
 };
@@ -416,6 +419,43 @@ __global__ __launch_bounds__(SK_THREADS, 2) void gemm_skinny_pair_kernel(const _
     else skinny_workgroup<MESH_Q6_K, 1, SEGS_B, NC>(bx - grid_a, p_x, p_wb, p_wb, p_wb, p_K, p_ks, 0xFFFFFFFFu, p_split_b, b);
 }
 
+// A launch cut along K: workgroup (slice, group) multiplies SEGS tile-rows by one slice of the super-blocks, which its eight waves share, and
+// writes the sums to part[slice][column][row]; gemm_add_slices adds them.
+template <int TYPE, int SEGS, int NC>
+__global__ __launch_bounds__(SK_THREADS, 2) void gemm_skinny_slice_kernel(const _Float16 *p_x, const uint8_t *p_w, int p_K, int p_T, int p_rows, int p_per, int p_ld, float *p_part) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    constexpr int NT = SK_NT * NC, TB = TileRegs<TYPE>::BYTES;
+    float *red = reinterpret_cast<float *>(smem);         // [SK_WAVES][SEGS][NT columns][16 rows]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int m = lane & 15, g = lane >> 4;
+    const int nsb = p_K / QK_K, sb0 = (int)blockIdx.x * p_per, here = min(p_per, nsb - sb0), tr0 = (int)blockIdx.y * SEGS, rows_here = min(SEGS, p_rows - tr0);
+    const int n_i = (here - wave + SK_WAVES - 1) / SK_WAVES;
+    const size_t row_stride = (size_t)nsb * TB;
+    auto tile_ptr = [&](int ii, int seg) { return p_w + (size_t)(tr0 + (seg < rows_here ? seg : 0)) * row_stride + (size_t)(sb0 + wave + SK_WAVES * ii) * TB; };
+    f4_t D[SEGS][NC];
+    SkinnyWalk<TYPE, SEGS, NC> walk(p_x + (size_t)(sb0 + wave) * (QK_K * 16), (unsigned)SK_WAVES * (QK_K * 16), (unsigned)SK_NT * p_K, n_i, lane, g, 4 * (4 * m + g),
+                                    SkinnyColumns<TYPE, NC>(m, g, p_T));
+    walk.start(D, n_i > 0, tile_ptr);
+    if (n_i > 0) walk.run(D, tile_ptr);
+    // D[seg] holds row m, columns 4 g .. 4 g + 3 of segment seg
+#pragma unroll
+    for (int seg = 0; seg < SEGS; ++seg)
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) red[((size_t)(wave * SEGS + seg) * NT + SK_NT * c + 4 * g + i) * 16 + m] = D[seg][c][i];
+    __syncthreads();
+    float *part = p_part + (size_t)blockIdx.x * p_T * p_ld;
+    for (int i = tid; i < SEGS * NT * 4; i += SK_THREADS) {
+        const int r4 = i & 3, seg = (i >> 2) % SEGS, t = (i >> 2) / SEGS;
+        if (t >= p_T || seg >= rows_here) continue;
+        f4_t v = f4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < SK_WAVES; ++w) v += *reinterpret_cast<const f4_t *>(red + ((size_t)(w * SEGS + seg) * NT + t) * 16 + 4 * r4);
+        *reinterpret_cast<f4_t *>(part + (size_t)t * p_ld + (tr0 + seg) * TILE_ROWS + 4 * r4) = v;
+    }
+}
+
 template <int TYPE, int NU, int SEGS, int NC>
 static int launch_skinny(const SkinnyKernelArgs &ka, int grid, size_t smem, hipStream_t stream) {
     static bool attr_set = false;
@@ -595,12 +635,79 @@ static int skinny_pair(const SkinnyF16Args &qa, const SkinnyF16Args &qb, hipStre
     return MESH_OK;
 }
 
+// ---- cut along K
+constexpr int SLICE_SEGS_MAX = 5;
+struct SlicePlan { int segs, slices, per; };
+template <int TYPE, int SEGS, int NC>
+static int launch_slice(const SkinnyF16Args &a, const SlicePlan &p, float *part, hipStream_t stream) {
+    constexpr size_t smem = sizeof(float) * SK_WAVES * SEGS * SK_NT * NC * 16;
+    static_assert(smem <= SK_LDS_LIMIT, "sums of a workgroup");
+    static bool attr_set = false;
+    if (!attr_set) {
+        MESH_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_skinny_slice_kernel<TYPE, SEGS, NC>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)SK_LDS_LIMIT));
+        attr_set = true;
+    }
+    const int rows = (a.mat[0].M + TILE_ROWS - 1) / TILE_ROWS;
+    MESH_LAUNCH((gemm_skinny_slice_kernel<TYPE, SEGS, NC>), dim3((unsigned)p.slices, (unsigned)((rows + SEGS - 1) / SEGS)), dim3(SK_THREADS), smem, stream, a.x,
+                static_cast<const uint8_t *>(a.mat[0].W), a.K, a.T, rows, p.per, (a.mat[0].M + 127) / 128 * 128, part);
+    MESH_LAUNCH_CHECK();
+    return MESH_OK;
+}
+template <int TYPE, int NC>
+static int launch_slice_segs(const SkinnyF16Args &a, const SlicePlan &p, float *part, hipStream_t stream) {
+    return p.segs == 3 ? launch_slice<TYPE, 3, NC>(a, p, part, stream) : p.segs == 4 ? launch_slice<TYPE, 4, NC>(a, p, part, stream) : launch_slice<TYPE, 5, NC>(a, p, part, stream);
+}
+// Whether a launch is cut, and how: groups of three to five tile-rows by two to four slices, as many workgroups as the CUs take at once.  For
+// launches that leave a quarter of the CUs idle otherwise, if no wave multiplies more tiles than before.  A workgroup of several rows
+// reads its slice's activations once for all of them (5120 x 27648 at 32 tokens: 0.44 MB a workgroup instead of 1.8); what is paid is the
+// launch that adds the slices, 2 to 4 us, which also writes the next norm's rows.
+// Cut / whole, us a layer less, 24 tokens: 5120 x 27648 (160 workgroups of two rows, 28 tiles a wave) five rows by four 15.5, four by three 10.5,
+// three by two 9.4; 5120 x 13824 2.3 and 3.1 (three by two); 3072 x 8192 three by four 1.8; 2048 x 16384 three by four 3.2; 2560 x 10240 (no
+// such cut) 0.1 at the best; with more workgroups to begin with 4096 x 14336 0, 3584 x 18944 2.  Up to 16 tokens there is half as much to
+// read: 5120 x 27648 5.0 (4 tokens) to 6.6 (16), 5120 x 13824 -2, 3072 x 8192 0.5, 2048 x 16384 -0.7; walks of 24 tiles and more are cut.
+static SlicePlan slice_plan(const SkinnyF16Args &a, size_t part_bytes) {
+    const SlicePlan whole{1, 1, 0};
+    const GemvMat &w = a.mat[0];
+    if (a.n_mat != 1 || a.epi != EPI_RESIDUAL || a.y16 || a.rope.pos || w.bias || a.T > 2 * SK_NT || a.K % QK_K || w.M % 8 || w.ldy % 4 || a.ldres % 4) return whole;
+    const int nsb = a.K / QK_K, rows = (w.M + TILE_ROWS - 1) / TILE_ROWS, ncu = skinny_n_cu(), ks = skinny_ks(nsb), grid = skinny_grid(rows, 1, ks);
+    const int tiles = (rows + grid - 1) / grid * ((nsb + ks - 1) / ks);
+    if (ks != SK_WAVES || 4 * grid > 3 * ncu || (a.T <= SK_NT && tiles < 24)) return whole;
+    SlicePlan best = whole;
+    int most = grid;
+    for (int segs = 3; segs <= SLICE_SEGS_MAX; ++segs)
+        for (int slices = 2; slices <= 4; ++slices) {
+            const int per = (nsb + slices - 1) / slices, n = (nsb + per - 1) / per, wgs = (rows + segs - 1) / segs * n;
+            if (wgs > ncu || wgs <= most || segs * ((per + SK_WAVES - 1) / SK_WAVES) > tiles) continue;
+            if ((size_t)n * a.T * ((w.M + 127) / 128 * 128) * sizeof(float) > part_bytes) continue;
+            most = wgs;
+            best = SlicePlan{segs, n, per};
+        }
+    return best;
+}
+
 }  // namespace f16sk
 
 int gemm_skinny_f16_workgroups(const SkinnyF16Args &a) {
     using namespace f16sk;
     if (a.n_mat != 1 || a.K <= 0 || a.K % QK_K || a.mat[0].M <= 0) return 0;
     return skinny_grid((a.mat[0].M + TILE_ROWS - 1) / TILE_ROWS, 1, skinny_ks(a.K / QK_K));
+}
+
+int gemm_skinny_f16_slices(const SkinnyF16Args &a, size_t part_bytes) { return f16sk::slice_plan(a, part_bytes).slices; }
+
+int gemm_skinny_f16_sliced(const SkinnyF16Args &a, const GemmArgs &sum, hipStream_t stream) {
+    using namespace f16sk;
+    const SlicePlan p = sum.part ? slice_plan(a, sum.part_bytes) : SlicePlan{1, 1, 0};
+    if (p.slices <= 1 || !a.x || (reinterpret_cast<uintptr_t>(a.x) & 15) || !a.mat[0].W || !a.mat[0].y || !a.residual || a.T <= 0 || !type_is_tiled(a.mat[0].type) ||
+        (sum.next_x16 && a.mat[0].M > GEMM_NORM_ROW_MAX))
+        return fail(MESH_ERR_INVALID, "gemm_skinny_f16_sliced: a launch it does not fit");
+    GemmArgs k = sum;
+    k.M = a.mat[0].M; k.K = a.K; k.T = a.T; k.Y = a.mat[0].y; k.ldy = a.mat[0].ldy; k.residual = a.residual; k.ldres = a.ldres;
+    k.ksplit = p.slices;
+    const bool two = a.T > SK_NT;
+    const int rc = a.mat[0].type == MESH_Q4_K ? (two ? launch_slice_segs<MESH_Q4_K, 2>(a, p, sum.part, stream) : launch_slice_segs<MESH_Q4_K, 1>(a, p, sum.part, stream))
+                                              : (two ? launch_slice_segs<MESH_Q6_K, 2>(a, p, sum.part, stream) : launch_slice_segs<MESH_Q6_K, 1>(a, p, sum.part, stream));
+    return rc != MESH_OK ? rc : gemm_add_slices(k, (k.M + 127) / 128, stream);
 }
 
 int gemm_skinny_f16(const SkinnyF16Args &a, hipStream_t stream) {

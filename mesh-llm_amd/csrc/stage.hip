@@ -953,6 +953,16 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
             rc = gemm_kquant(g, stream);
         } else rc = gemm_skinny_f16(ga, stream);
         if (rc != MESH_OK) return rc;
+        if (s->gemm_part && s->tune.gemm_splitk && gemm_skinny_f16_slices(da, s->gemm_part_bytes) > 1) {
+            // (xn is free: its readers are behind)
+            GemmArgs sum;
+            sum.part = s->gemm_part; sum.part_bytes = s->gemm_part_bytes; sum.sat = s->f16_sat;
+            if (next_fused && E <= GEMM_NORM_ROW_MAX) {
+                sum.next_w = static_cast<const float *>(Ln->attn_norm.data); sum.next_eps = hp.rms_eps; sum.next_x16 = xn;
+                s->xn_layer = (int)il + 1;
+            }
+            return gemm_skinny_f16_sliced(da, sum, stream);
+        }
         if (next_fused) {
             da.norm_out.norm_w = static_cast<const float *>(Ln->attn_norm.data); da.norm_out.x16 = nx; da.norm_out.part = s->norm_part;
         }

@@ -64,7 +64,7 @@ class Host:
 def kernel_name(mangled):
     """_ZN4mesh15gemm_f16_kernelILNS_7TileOutE1ELi4ELi3EEEv... -> gemm_f16_kernel<1,4,3>"""
     import re
-    m = re.match(r"_ZN4mesh(?:12_GLOBAL__N_1)?(\d+)", mangled)
+    m = re.match(r"_ZN4mesh(?:12_GLOBAL__N_1|5f16sk)?(\d+)", mangled)
     if not m:
         return mangled
     n = int(m.group(1))

@@ -297,6 +297,41 @@ def test_norms_handed_over_to_short_walks(tmp_path, width):
     st.close()
 
 
+# width, ff, tokens, and of the down projection's launch: tile-rows a workgroup, slices along K, workgroups a slice
+STEP_SLICE_CASES = [
+    ((2048, 4352), 17, (3, 4, 43)),         # slices of 5, 5, 5 and 2 super-blocks for eight waves, two rows in the last group; one column past a block
+    ((5376, 8704), 24, (4, 3, 84)),         # 12, 12 and 10
+    ((5120, 8704), 32, (5, 4, 64)),         # 9, 9, 9 and 7; every column
+]
+
+
+@pytest.mark.parametrize("shape,tokens", [c[:2] for c in STEP_SLICE_CASES])
+def test_down_projections_of_decode_steps_in_slices(tmp_path, shape, tokens):
+    """Two layers (q4_K down projection, whose sums write the next norm's rows, then q6_K) against the oracle and against whole launches."""
+    m = mesh()
+    width, ff = shape
+    cfg = dict(kquant(width, 2, 1, ff), n_layer=2)
+    path = os.path.join(str(tmp_path), "model.gguf")
+    tensors = models.write_model(path, cfg, [0, 1], seed=4, fast=True)
+    assert [tensors["blk.%d.ffn_down.weight" % i][0] for i in (0, 1)] == [models.Q4_K, models.Q6_K]
+    st = m.Stage(path, 0, 2, n_ctx=16, n_seq_max=32, n_batch_max=32)
+    ses = [st.session(gemm_splitk=on) for on in (1, 0)]
+    orc = StageOracle(cfg, tensors, 0, 2, 16, n_seq_max=32, blas=True)
+    rng = np.random.Generator(np.random.PCG64(5))
+    for step in range(2):
+        x = rng.standard_normal((tokens, width)).astype(np.float32)
+        pos, seq = [step] * tokens, list(range(tokens))
+        got, whole = [s.decode(x, pos, seq=seq).view(np.float32).reshape(tokens, width).astype(np.float64) for s in ses]
+        want = orc.forward(x, pos, seq=seq).astype(np.float64)
+        # activations rounded to f16 in front of every product (2^-12 root mean square, eight products): 4 * 2^-12 * sqrt(8)
+        assert np.linalg.norm(got - want) <= 2.8e-3 * np.linalg.norm(want), (tokens, np.linalg.norm(got - want) / np.linalg.norm(want))
+        # the same products in another order; behind it a norm of its own rounds scaled rows to f16, the hand-over rows before their scale
+        assert np.linalg.norm(got - whole) <= 2e-3 * np.linalg.norm(whole), tokens
+    for s in ses:
+        s.close()
+    st.close()
+
+
 # rows of one and two groups of eight a thread, whole and with idle threads; token counts of every tile that splits
 @pytest.mark.parametrize("width,heads", [(768, 6), (2048, 16), (4096, 32), (5120, 40)])
 def test_norms_ride_with_the_sums_of_slices(tmp_path, width, heads):
