@@ -204,7 +204,11 @@ __device__ __forceinline__ uint32_t and_or(uint32_t x, uint32_t mask, uint32_t y
     asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "s"(mask), "v"(y));
     return r;
 }
-__device__ __forceinline__ uint32_t nibble_pair(uint32_t w, int p) { return and_or(p == 0 ? w << 4 : w >> (4 * (p - 1)), 0x00F000F0u, 0x54005400u); }
+__device__ __forceinline__ uint32_t nibble_pair(uint32_t w, int p) {
+    uint32_t mask = 0x00F000F0u, base = 0x54005400u;
+    asm("" : "+s"(mask), "+v"(base));
+    return ((p == 0 ? w << 4 : w >> (4 * (p - 1))) & mask) | base;
+}
 // 1024 + byte i of w, twice, exactly
 __device__ __forceinline__ half2v byte_pair(uint32_t w, int i) { return __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, w, 0x04000400u + 0x00010001u * i)); }
 template <> struct PackedSub<MESH_Q4_K> {
@@ -540,11 +544,13 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_kq_kernel(GemmArgs a) {
 // and all pairs: a lane of the multiplied fragment holds one row, and the GEMM layout's slot (row, half of a chunk) is
 // that lane's, so it forms the fragments of four MFMA steps from its own 32 or 40 bytes, in registers.  The activations go through LDS, k8-major as they lie in memory: 16-byte pieces at consecutive
 // addresses both ways.  NT groups of 32 pairs: an expert's remainder costs the groups it fills.
-// Bound by forming the weights (72 vector instructions per 2048 of them and wave) next to multiplying them, and by how evenly the
-// tiles fill the chip.  Gate / up of 64 experts of 2 x 768 rows x 2048 (q4_K), 4800 pairs of a Zipf router (86 tiles, 44 of at most
-// 32 pairs): 98 us with the staging waves of gemm_kq_kernel on tiles of 128 columns, 80 with fragments formed in registers, 70 with
-// the larger tiles first (moe_sort) and and_or; down projection of 2048 x 768: 53 -> 40 (q4_K), 56 -> 46 (q6_K).  113 MB of weights
-// at the rate of a large copy: 22 us.
+// Bound by forming the weights (77 vector instructions per 2048 of them and wave, about 300 cycles of a SIMD: a packed f16 instruction takes
+// five, and_or and perm 4.5, a shift 2.4) next to multiplying them (33 cycles a product), at the 1.4 to 1.6 GHz that the chip holds with all
+// of it busy, and by how evenly the tiles fill the chip.  Gate / up of 64 experts of 2 x 768 rows x 2048 (q4_K), 4800 pairs of a Zipf router
+// (86 tiles, 44 of at most 32 pairs): 98 us with the staging waves of gemm_kq_kernel on tiles of 128 columns, 80 with fragments formed in
+// registers, 70 with the larger tiles first (moe_sort) and and_or, 62 with a step's fragments formed between the products of the step
+// before, three workgroups a CU kept (two: 67) and small tiles' activations in groups of up to four chunks; down projection of 2048 x 768:
+// 53 -> 40 -> 36 (q4_K), 56 -> 46 -> 42 (q6_K).  113 MB of weights at the rate of a large copy: 22 us.
 // Rows of a SwiGLU pair are dealt out so that a wave holds 16 gate rows and the 16 up rows of the same outputs, in one lane's
 // registers e and e + 8.
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -583,35 +589,98 @@ __device__ __forceinline__ void reg_tile(const GemmArgs &a, const uint8_t *wp, i
     const int last = n > 0 ? n - 1 : 0;                        // (a group without steps of its own reads the first and multiplies none)
     if (n <= 0) { wp -= (size_t)k0 * PackedSub<TYPE>::CHUNK; }
     const u32x4 *const xb = n > 0 ? xbase : xbase - (size_t)k0 * 128;
-    PackedSub<TYPE> rw[AHEAD];
+    // (fewer on their way where more would cost a workgroup of a CU its registers)
+    constexpr int RING = MODE == REG_EXPERT && TYPE == MESH_Q6_K && NT > 2 ? 2 : AHEAD;
+    PackedSub<TYPE> rw[RING];
     // Loads return in order: activations stored a step after they were asked for would have the weights asked for before them arrive
     // by then too, two chunks ahead instead of AHEAD.  Activations asked for XA steps before, against one: a batch of 32 decode steps of
-    // four layers 5120 wide 821 -> 809 us, eight layers of a 40-token chunk 4096 wide 971 -> 953, a 600-token chunk of 128 experts
-    // 2175 -> 2151.  Two columns of tiles in a dense call with AHEAD spill (40 tokens: 995).
-    constexpr int XA = NT == 1 ? AHEAD : NT > 2 ? 1 : MODE == REG_EXPERT ? AHEAD : 2;       // (the registers that are left at the occupancy)
-    u32x4 rx[XA][NT];
+    // four layers 5120 wide 821 -> 809 us, eight layers of a 40-token chunk 4096 wide 971 -> 953.  Two columns of tiles in a dense call with AHEAD spill (40 tokens: 995).
+    constexpr int XA = NT == 1 ? AHEAD : NT > 2 ? 1 : 2;       // (the registers that are left at the occupancy)
+    // Expert tiles: activations in groups of G chunks, 16 KB at most; a group is asked for while the one before it is multiplied.
+    constexpr int G = MODE == REG_EXPERT ? (NT > 2 ? 1 : 4 / NT) : 1, GROUP = 1024;
+    u32x4 rx[MODE == REG_EXPERT ? G * NT : XA * NT];
+    auto fetch = [&](int kc) {
 #pragma unroll
-    for (int i = 0; i < NT; ++i) xs[i * 256 + tid] = xb[xo[i]];
+        for (int i = 0; i < G * NT; ++i) rx[i] = (xb + (size_t)(kc + i / NT < last ? kc + i / NT : last) * 128)[xo[i % NT]];
+    };
+    if constexpr (MODE == REG_EXPERT) {
+        fetch(0);
 #pragma unroll
-    for (int v = 1; v <= XA; ++v)
+        for (int i = 0; i < G * NT; ++i) xs[i * 256 + tid] = rx[i];
+        fetch(G);
+    } else {
 #pragma unroll
-        for (int i = 0; i < NT; ++i) rx[v % XA][i] = (xb + (size_t)(v < last ? v : last) * 128)[xo[i]];
+        for (int i = 0; i < NT; ++i) xs[i * 256 + tid] = xb[xo[i]];
+#pragma unroll
+        for (int v = 1; v <= XA; ++v)
+#pragma unroll
+            for (int i = 0; i < NT; ++i) rx[v % XA * NT + i] = (xb + (size_t)(v < last ? v : last) * 128)[xo[i]];
+    }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int u = 0; u < AHEAD; ++u) rw[u].load(wp + (size_t)(MODE == REG_EXPERT || u < last ? u : last) * PackedSub<TYPE>::CHUNK, slot);
+    for (int u = 0; u < RING; ++u) rw[u].load(wp + (size_t)(MODE == REG_EXPERT || u < last ? u : last) * PackedSub<TYPE>::CHUNK, slot);
     lds_barrier();
     const int at = (lane & 15) + ((lane >> 4) & 1) * 128 + hh * 16;
+    if constexpr (MODE == REG_EXPERT) {
+        // A step's fragments are formed between the products of the step before, whose issue leaves the vector ALU idle, and its activations
+        // read ahead of those.  The barrier of a group of chunks stands before its last step: behind it the next group's activations
+        // have landed, whose first fragments that step reads, and the buffer they lie in has been read by everybody a group ago.
+        u32x4 f[NT];
+        half8 w[2];
+        w[0] = __builtin_bit_cast(half8, rw[0].form(0));
+        const u32x4 *x = xs + at;
+        int to_next = GROUP;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) f[j] = x[j * 256];
+        for (int kc0 = 0; kc0 < per; kc0 += AHEAD) {
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) {
+                const int kc = kc0 + u, c = u % G;
+#pragma unroll
+                for (int st = 0; st < 4; ++st) {
+                    const bool turn = c == G - 1 && st == 3;
+                    if (turn) {
+                        lds_barrier();
+                        x += to_next;
+                        to_next = -to_next;
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    w[(st + 1) & 1] = __builtin_bit_cast(half8, st < 3 ? rw[u % RING].form(st + 1) : rw[(u + 1) % RING].form(0));
+#pragma unroll
+                    for (int j = 0; j < NT; ++j) {
+                        acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[st & 1], __builtin_bit_cast(half8, f[j]), acc[j], 0, 0, 0);
+                        f[j] = x[(turn ? 0 : st < 3 ? c * STEP + (st + 1) * 32 : (c + 1) * STEP) + j * 256];
+                    }
+#pragma unroll
+                    for (int j = 0; j < NT; ++j) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x002, (24 + NT - 1) / NT, 0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (c == 0 && st == 0) {
+                        // (the other buffer's last readers stand before the barrier of the group before)
+                        u32x4 *const nx = const_cast<u32x4 *>(x) - at + tid + to_next;
+#pragma unroll
+                        for (int i = 0; i < G * NT; ++i) nx[i * 256] = rx[i];
+                        fetch(kc + 2 * G);
+                    }
+                    if (st == 2) rw[u % RING].load(wp + (size_t)(kc + RING < last ? kc + RING : last) * PackedSub<TYPE>::CHUNK, slot);
+                }
+            }
+        }
+    } else
     for (int kc0 = 0; kc0 < per; kc0 += AHEAD) {
 #pragma unroll
         for (int u = 0; u < AHEAD; ++u) {
             const int kc = kc0 + u;
             // (the other buffer was read a step ago; the step's barrier hands it over)
 #pragma unroll
-            for (int i = 0; i < NT; ++i) xs[((u + 1) & 1) * STEP + i * 256 + tid] = rx[(u + 1) % XA][i];
+            for (int i = 0; i < NT; ++i) xs[((u + 1) & 1) * STEP + i * 256 + tid] = rx[(u + 1) % XA * NT + i];
 #pragma unroll
-            for (int i = 0; i < NT; ++i) rx[(u + 1) % XA][i] = (xb + (size_t)(kc + 1 + XA < last ? kc + 1 + XA : last) * 128)[xo[i]];
+            for (int i = 0; i < NT; ++i) rx[(u + 1) % XA * NT + i] = (xb + (size_t)(kc + 1 + XA < last ? kc + 1 + XA : last) * 128)[xo[i]];
             const u32x4 *x = xs + (u & 1) * STEP + at;
-            if (MODE == REG_EXPERT || kc < n) {                // (an expert's K is a multiple of 256)
+            if (kc < n) {
                 u32x4 f[2][NT];
 #pragma unroll
                 for (int j = 0; j < NT; ++j) f[0][j] = x[j * 256];
@@ -740,9 +809,19 @@ template <int TYPE>
 __global__ __launch_bounds__(256, 2) void gemm_expert_kernel(GemmArgs a) {
     __shared__ u32x4 xs[2 * 4 * 256];
     // workgroups go to the eight XCDs in turn: every row block of a tile on one of them, whose L2 fetches the tile's activations once
-    // (gate / up as above: 66 us, 82 with the row blocks dealt over the XCDs)
-    const int g = (int)(blockIdx.y * gridDim.x + blockIdx.x), by = (g >> 3) / (int)gridDim.x * 8 + (g & 7), bx = (g >> 3) % (int)gridDim.x;
-    if (by >= *a.n_tiles) return;
+    // (gate / up as above: 66 us then, 82 with the row blocks dealt over the XCDs)
+    const int g = (int)(blockIdx.y * gridDim.x + blockIdx.x), bx = (g >> 3) % (int)gridDim.x, nt = *a.n_tiles;
+    int eight = (g >> 3) / (int)gridDim.x;                     // of the list, eight tiles at a time
+    // Down: the list's halves in turn, so that a CU has large tiles, bound by their products, beside small ones, bound by forming weights
+    // (2048 x 768 as above: 37.4 -> 36.2 us q4_K, 45.3 -> 42.0 q6_K).  Gate / up walk longer rows and would end behind their
+    // largest tiles (65 -> 71).
+    if (!a.y16_k8) {
+        const int n8 = (nt + 7) >> 3;
+        if (eight >= n8) return;
+        eight = (eight & 1) ? ((n8 + 1) >> 1) + (eight >> 1) : eight >> 1;
+    }
+    const int by = eight * 8 + (g & 7);
+    if (by >= nt) return;
     const int4 tl = reinterpret_cast<const int4 *>(a.tiles)[by];
     const uint8_t *wp = static_cast<const uint8_t *>(a.Wp) + (size_t)tl.x * a.expert_stride;
     const int n = a.K / GK;
