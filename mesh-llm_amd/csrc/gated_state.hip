@@ -9,6 +9,7 @@
 #include <algorithm>
 
 #include "act_math.hpp"
+#include "lds_ops.hpp"
 #include "wave_ops.hpp"
 
 namespace mesh {
@@ -19,13 +20,12 @@ constexpr int C = STATE_CHUNK;
 constexpr float UNIT_EPS = 1e-6f;               // inside the root of the unit vectors of DELTA
 
 __device__ __forceinline__ float gs_softplus(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }
-__device__ __forceinline__ gs_f4 gs_mma(const float4 &a, const gs_f4 &b, gs_f4 acc) {
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b[0], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b[1], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b[2], acc, 0, 0, 0);
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b[3], acc, 0, 0, 0);
+__device__ __forceinline__ gs_f4 gs_mma(const gs_f4 &a, const gs_f4 &b, gs_f4 acc) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], acc, 0, 0, 0);
+    return acc;
 }
-__device__ __forceinline__ gs_f4 gs_mma(const float4 &a, const float4 &b, gs_f4 acc) { return gs_mma(a, gs_f4{b.x, b.y, b.z, b.w}, acc); }
+__device__ __forceinline__ gs_f4 gs_mma(const float4 &a, const float4 &b, gs_f4 acc) { return gs_mma(gs_f4{a.x, a.y, a.z, a.w}, gs_f4{b.x, b.y, b.z, b.w}, acc); }
 
 __device__ __forceinline__ float delta_log_decay(const GatedStateArgs &a, int t, int h) { return -a.A[h] * gs_softplus(a.in[(size_t)t * a.ld + a.at_a + h] + a.dt_bias[h]); }
 __device__ __forceinline__ float delta_beta(const GatedStateArgs &a, int t, int h) { return act_sigmoid(a.in[(size_t)t * a.ld + a.at_b + h]); }
@@ -194,19 +194,26 @@ __global__ __launch_bounds__(THREADS) void gated_step_kernel(const GatedStateArg
 // ---- chunks
 __host__ __device__ constexpr int gs_pad64(int n) { return (n + 63) / 64 * 64; }
 __host__ __device__ constexpr int gs_pad16(int n) { return (n + 15) / 16 * 16; }
-// What the first launch leaves of a (chunk, head), in this order; Dp = dim padded to 64, Vp = vdim padded to 16, padding zero
+// What the first launch leaves of a (chunk, head), in this order; Dp = dim padded to 64, Vp = vdim padded to 16, padding zero.  Matrices lie in
+// tiles of 16 x 16 as the scan's operands take them: lane c + 16 g of a wave has four neighbours at 4 (c + 16 g) of its tile, elements 4 g .. 4 g + 3
+// along the dimension that is summed over (U: along the tokens) of row (U: column) c.  An operand is then one kilobyte, contiguous: rows
+// as they stood before are 16 segments of 64 bytes, and a chunk's loads held a wave of the scan up for 1100 (2100 with the delta rule) of 3200
+// (4900) cycles.
 struct GsMats {
-    float *Q, *KT, *A, *G, *W, *U;          // [C][Dp], [Dp][C], [C][C], [Dp], [C][Dp], [C][Vp]
+    float *Q, *KT, *A, *G, *W, *U;          // [Dp / 16][2 row tiles], [Dp / 16][2 token tiles], [2 row tiles][2 column tiles], [Dp], as Q, [Vp / 16][2 token tiles]
     __device__ __forceinline__ GsMats(float *ws, size_t index, int Dp, int Vp, bool delta) {
-        const size_t n = (size_t)C * (2 * Dp + C) + Dp + (delta ? (size_t)C * (Dp + Vp) : 0);
+        const size_t n = (size_t)C * (2 * Dp + C) + Dp + (size_t)C * (Vp + (delta ? Dp : 0));
         Q = ws + index * n;
         KT = Q + (size_t)C * Dp;
         A = KT + (size_t)C * Dp;
         G = A + C * C;
-        W = G + Dp;
-        U = W + (size_t)C * Dp;
+        U = G + Dp;                         // GLA: the values themselves
+        W = U + (size_t)C * Vp;
     }
 };
+__device__ __forceinline__ int gs_tile(int a, int b, int lane) { return ((2 * a + b) * 64 + lane) * 4; }
+// element (r, j) of A
+__device__ __forceinline__ int gs_a_at(int r, int j) { return gs_tile(r >> 4, j >> 4, (r & 15) + 16 * ((j & 15) >> 2)) + (j & 3); }
 size_t gated_state_workspace(int n_chunks, int heads, int dim, int vdim) {
     const size_t Dp = (size_t)gs_pad64(dim), Vp = (size_t)gs_pad16(vdim);
     return (size_t)n_chunks * heads * (C * (3 * Dp + C + Vp) + Dp);
@@ -310,22 +317,20 @@ __global__ __launch_bounds__(PREP_THREADS) void delta_prepare_kernel(const Gated
             for (int r = 0; r < C; ++r) sT[r * LP + j] = x[r];
         }
     } else {
-        const int id = tid - 64, step = PREP_THREADS - 64;
-        for (int r = wave - 1; r < C; r += 3) {
-            const float f = s_since[r];
-            for (int d = lane * 4; d < Dp; d += 256) {
-                float4 q = *reinterpret_cast<const float4 *>(sQ + r * dp + d);
-                q.x *= f; q.y *= f; q.z *= f; q.w *= f;
-                *reinterpret_cast<float4 *>(m.Q + (size_t)r * Dp + d) = q;
-            }
+        for (int tile = wave - 1; tile < Dp / 8; tile += 3) {
+            const int dt = tile >> 1, r = tile & 1;
+            const float f = s_since[16 * r + c];
+            float4 q = *reinterpret_cast<const float4 *>(sQ + (16 * r + c) * dp + 16 * dt + 4 * g);
+            q.x *= f; q.y *= f; q.z *= f; q.w *= f;
+            *reinterpret_cast<float4 *>(m.Q + gs_tile(dt, r, lane)) = q;
+            const int t = 16 * r + 4 * g;
+            const float *k = sK + t * dp + 16 * dt + c;
+            *reinterpret_cast<float4 *>(m.KT + gs_tile(dt, r, lane)) =
+                make_float4(k[0] * s_until[t], k[dp] * s_until[t + 1], k[2 * dp] * s_until[t + 2], k[3 * dp] * s_until[t + 3]);
         }
-        for (int i = id; i < Dp * (C / 4); i += step) {
-            const int d = i / (C / 4), r = i % (C / 4) * 4;
-            *reinterpret_cast<float4 *>(m.KT + (size_t)d * C + r) =
-                make_float4(sK[r * dp + d] * s_until[r], sK[(r + 1) * dp + d] * s_until[r + 1], sK[(r + 2) * dp + d] * s_until[r + 2], sK[(r + 3) * dp + d] * s_until[r + 3]);
-        }
-        for (int i = id; i < C * C / 4; i += step) *reinterpret_cast<float4 *>(m.A + 4 * i) = *reinterpret_cast<const float4 *>(sA + (i / (C / 4)) * LP + i % (C / 4) * 4);
-        for (int i = id; i < Dp; i += step) m.G[i] = s_since[C - 1];
+        for (int tile = wave - 1; tile < 4; tile += 3)
+            *reinterpret_cast<float4 *>(m.A + gs_tile(tile >> 1, tile & 1, lane)) = *reinterpret_cast<const float4 *>(sA + (16 * (tile >> 1) + c) * LP + 16 * (tile & 1) + 4 * g);
+        for (int i = tid - 64; i < Dp; i += PREP_THREADS - 64) m.G[i] = s_since[C - 1];
     }
     __syncthreads();
     // W = T (beta decay K), U = T (beta V): column tiles dealt to the waves, both row tiles of each
@@ -344,16 +349,14 @@ __global__ __launch_bounds__(PREP_THREADS) void delta_prepare_kernel(const Gated
                 b[j] = X[k * xp + c] * s_beta[k] * (w ? s_since[k] : 1.f);
             }
 #pragma unroll
-            for (int rt = s; rt < 2; ++rt) acc[rt] = gs_mma(*reinterpret_cast<const float4 *>(sT + (16 * rt + c) * LP + 16 * s + 4 * g), b, acc[rt]);
+            for (int rt = s; rt < 2; ++rt) {
+                const gs_f4 t = *reinterpret_cast<const gs_f4 *>(sT + (16 * rt + c) * LP + 16 * s + 4 * g);
+                // (W is formed as its transpose: a lane then holds neighbours of a row)
+                acc[rt] = w ? gs_mma(b, t, acc[rt]) : gs_mma(t, b, acc[rt]);
+            }
         }
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int r = 16 * rt + 4 * g + i;
-                if (w) m.W[(size_t)r * Dp + 16 * ct + c] = acc[rt][i];
-                else m.U[(size_t)r * Vp + 16 * (ct - nd) + c] = acc[rt][i];
-            }
+        for (int rt = 0; rt < 2; ++rt) *reinterpret_cast<gs_f4 *>((w ? m.W : m.U) + gs_tile(w ? ct : ct - nd, rt, lane)) = acc[rt];
     }
 }
 static size_t delta_prepare_lds(int dim, int vdim) {
@@ -433,16 +436,38 @@ __global__ __launch_bounds__(PREP_THREADS) void gla_prepare_kernel(const GatedSt
         }
     }
     __syncthreads();
-    const GsMats m(a.ws, (size_t)ci * a.heads + h, Dp, 0, false);
-    for (int r = wave; r < C; r += 4)
-        for (int d = lane; d < Dp; d += 64) m.Q[(size_t)r * Dp + d] = sQ[r * dp + d] * expf(sG[r * dp + d]);
-    for (int i = tid; i < Dp * (C / 4); i += PREP_THREADS) {
-        const int d = i / (C / 4), r = i % (C / 4) * 4;
+    const int V = a.vdim, Vp = gs_pad16(V);
+    const GsMats m(a.ws, (size_t)ci * a.heads + h, Dp, Vp, false);
+    // (the values are on their way while the rest is written)
+    constexpr int VT = STATE_DIM_MAX / 8 / 4;          // tiles a wave has at most
+    float vv[VT][4];
+#pragma unroll
+    for (int k = 0; k < VT; ++k) {
+        const int tile = wave + 4 * k;
+        if (tile >= Vp / 8) break;
+        const int v = 16 * (tile >> 1) + c, t = 16 * (tile & 1) + 4 * g;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) vv[k][j] = a.in[(size_t)(t0 + (t + j < n ? t + j : 0)) * a.ld + a.at_v + h * V + (v < V ? v : 0)];
+    }
+    for (int tile = wave; tile < Dp / 8; tile += 4) {
+        const int dt = tile >> 1, r = tile & 1, at = (16 * r + c) * dp + 16 * dt + 4 * g;
+        const float4 q = *reinterpret_cast<const float4 *>(sQ + at), lq = *reinterpret_cast<const float4 *>(sG + at);
+        *reinterpret_cast<float4 *>(m.Q + gs_tile(dt, r, lane)) = make_float4(q.x * expf(lq.x), q.y * expf(lq.y), q.z * expf(lq.z), q.w * expf(lq.w));
+        const int d = 16 * dt + c, t = 16 * r + 4 * g;
         const float end = sG[(C - 1) * dp + d];
         float k[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) k[j] = sK[(r + j) * dp + d] * expf(end - sG[(r + j) * dp + d]);
-        *reinterpret_cast<float4 *>(m.KT + (size_t)d * C + r) = make_float4(k[0], k[1], k[2], k[3]);
+        for (int j = 0; j < 4; ++j) k[j] = sK[(t + j) * dp + d] * expf(end - sG[(t + j) * dp + d]);
+        *reinterpret_cast<float4 *>(m.KT + gs_tile(dt, r, lane)) = make_float4(k[0], k[1], k[2], k[3]);
+    }
+#pragma unroll
+    for (int k = 0; k < VT; ++k) {
+        const int tile = wave + 4 * k;
+        if (tile >= Vp / 8) break;
+        const int v = 16 * (tile >> 1) + c, t = 16 * (tile & 1) + 4 * g;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) vv[k][j] = v < V && t + j < n ? vv[k][j] : 0.f;
+        *reinterpret_cast<float4 *>(m.U + gs_tile(tile >> 1, tile & 1, lane)) = make_float4(vv[k][0], vv[k][1], vv[k][2], vv[k][3]);
     }
     for (int d = tid; d < Dp; d += PREP_THREADS) m.G[d] = expf(sG[(C - 1) * dp + d]);
     // A: a decay per channel does not leave the sum over channels.  Within a 16 x 16 diagonal block each pair takes its own
@@ -458,7 +483,7 @@ __global__ __launch_bounds__(PREP_THREADS) void gla_prepare_kernel(const GatedSt
             s = fmaf(q.x, k.x, fmaf(q.y, k.y, fmaf(q.z, k.z, fmaf(q.w, k.w, s))));
         }
         s = group_sum<8>(s);
-        if ((tid & 7) == 0) m.A[r * C + r] = s;
+        if ((tid & 7) == 0) m.A[gs_a_at(r, r)] = s;
     }
     if (tid < 2 * PAIRS) {
         // pair p of a block: row r >= 1, column p - r (r - 1) / 2 < r
@@ -477,8 +502,8 @@ __global__ __launch_bounds__(PREP_THREADS) void gla_prepare_kernel(const GatedSt
             s = fmaf(q.z * k.z, act_exp_neg(gj.z - gr.z), s);
             s = fmaf(q.w * k.w, act_exp_neg(gj.w - gr.w), s);
         }
-        m.A[r * C + j] = s;
-        m.A[j * C + r] = 0.f;
+        m.A[gs_a_at(r, j)] = s;
+        m.A[gs_a_at(j, r)] = 0.f;
     }
     if (wave == 3) {
         gs_f4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -492,25 +517,81 @@ __global__ __launch_bounds__(PREP_THREADS) void gla_prepare_kernel(const GatedSt
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            m.A[(16 + 4 * g + i) * C + c] = acc[i];
-            m.A[(4 * g + i) * C + 16 + c] = 0.f;
+            m.A[gs_a_at(16 + 4 * g + i, c)] = acc[i];
+            m.A[gs_a_at(4 * g + i, 16 + c)] = 0.f;
         }
     }
 }
 static size_t gla_prepare_lds(int dim, int rank) { return ((size_t)C * (3 * (gs_pad64(dim) + 4) + rank) + gs_pad64(dim)) * sizeof(float); }
 
-// grid (heads, 16-column slices of the values, sequences of the call).  Wave w owns rows [16 NT w, 16 NT (w + 1)) of the state.
+// grid (heads, 16-column slices of the values, sequences of the call).  Wave w < 4 owns rows [16 NT w, 16 NT (w + 1)) of the state; waves 4
+// and 5 write a chunk's outputs, a row tile each, beside the next chunk's products (in waves 0 and 1 they made the other two wait 700 cycles).
 // PIPED: a chunk is worked on while the next ones travel, which takes the registers of one workgroup a CU; without, as many of them as fit
 // hide each other's waits (launch_scan).
+// What bounds it, a chunk of 128 x 128 (16 heads, one sequence, cycles of 3300 with the delta rule, 2400 without): 48 and 32 matrix
+// instructions a wave at 32.5 cycles, 72 and 56 KB that a CU takes at 64 bytes a cycle and less, and the waits where they meet.  29 chunks x 16 heads,
+// us, delta rule / without: rows as they lie, outputs in waves 0 and 1: 70.6 / 63.3; no branch around a load 64.2 / 44.3; operands as
+// kilobytes, outputs in waves of their own, a barrier that leaves loads in flight 44.0 / 32.7; loads between the products 43.2 / 30.7.  Q S
+// behind the barrier, while the sums over the waves travel: 44.2 / 31.9.
+constexpr int SCAN_THREADS = 384;
 template <bool DELTA, int NT, bool PIPED>
-__global__ __launch_bounds__(256) void state_scan_kernel(const GatedStateArgs a) {
+__global__ __launch_bounds__(SCAN_THREADS) void state_scan_kernel(const GatedStateArgs a) {
     constexpr int Dp = 64 * NT;
     __shared__ __align__(16) float red[2][4][DELTA ? 4 : 2][64][4];        // by chunk parity, wave: partial W S and Q S of the two row tiles
-    const int h = blockIdx.x, v0 = blockIdx.y * 16, run = blockIdx.z;
+    const int h = blockIdx.x, vt = blockIdx.y, run = blockIdx.z;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
-    const int D = a.dim, V = a.vdim, Vp = gs_pad16(V), col = v0 + c, d0 = wave * 16 * NT;
+    const int D = a.dim, V = a.vdim, Vp = gs_pad16(V), col = 16 * vt + c;
     const int c0 = a.chunks.run[run], c1 = a.chunks.run[run + 1];
     const int t_first = a.chunks.chunk[c0];
+    // u of a chunk from what the first launch left of it; a barrier stands before
+    auto settle = [&](int ci, gs_f4 (&u)[2], int tiles) {
+        if constexpr (DELTA) {
+            float (*rd)[DELTA ? 4 : 2][64][4] = red[(ci - c0) & 1];
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+                if (r < tiles)
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) u[r] -= *reinterpret_cast<const gs_f4 *>(rd[w][2 + r][lane]);
+        }
+    };
+    if (wave >= 4) {
+        const int rt = wave - 4, t_end = a.chunks.chunk[c1];
+        struct Out { gs_f4 a[2], u[2]; };
+        auto load = [&](int ci, Out &f) {
+            if (ci >= c1) ci = c1 - 1;
+            const GsMats m(a.ws, (size_t)ci * a.heads + h, Dp, Vp, DELTA);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                f.a[s] = *reinterpret_cast<const gs_f4 *>(m.A + gs_tile(rt, s, lane));
+                f.u[s] = *reinterpret_cast<const gs_f4 *>(m.U + gs_tile(vt, s, lane));
+            }
+        };
+        auto step = [&](int ci, Out &f) {
+            lds_barrier();
+            float (*rd)[DELTA ? 4 : 2][64][4] = red[(ci - c0) & 1];
+            gs_f4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int w = 0; w < 4; ++w) o += *reinterpret_cast<const gs_f4 *>(rd[w][rt][lane]);
+            settle(ci, f.u, 1 + rt);
+            o = gs_mma(f.a[0], f.u[0], o);
+            if (rt == 1) o = gs_mma(f.a[1], f.u[1], o);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int t = t_first + (ci - c0) * C + 16 * rt + 4 * g + i;
+                if (t < t_end && col < V) a.o[(size_t)t * a.heads * V + h * V + col] = o[i];
+            }
+        };
+        Out f0, f1;
+        load(c0, f0);
+        int ci = c0;
+        for (; ci + 2 <= c1; ci += 2) {
+            load(ci + 1, f1); step(ci, f0);
+            load(ci + 2, f0); step(ci + 1, f1);
+        }
+        if (ci < c1) step(ci, f0);
+        return;
+    }
+    const int d0 = wave * 16 * NT;
     float *st = a.state + ((size_t)a.seq[t_first] * a.heads + h) * D * V;
     const bool zero = a.pos[t_first] == 0;
     gs_f4 S[NT];
@@ -523,46 +604,47 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const GatedStateArgs a)
         }
     // what a chunk brings: W (DELTA), Q by (row tile, own d tile), K^T by (own d tile, token tile), G, U
     struct Frag {
-        float4 w[DELTA ? 2 : 1][NT], q[2][NT], k[NT][2];
-        gs_f4 gd[NT], u[2];
-        float4 a[2];                    // the rows of A of this wave's output tile (waves 0 and 1)
+        gs_f4 w[DELTA ? 2 : 1][NT], q[2][NT], k[NT][2], gd[NT], u[2];
     };
-    // (every chunk of a run but its last is whole)
-    const int t_end = a.chunks.chunk[c1], col_in = col < V ? col : V - 1;
     // No branch lies around a load: the compiler waits for everything in flight at the join of one, the chunks just asked for among
-    // them.  What lies past the end is the last chunk (PIPED), token or column again and is left out where it is used.
-    // PIPED, 29 chunks x 16 heads of 128 x 128: 70.6 -> 64.2 us with the delta rule, 63.3 -> 44.3 without (the chains of matrix
-    // instructions taking turns instead of one after another: 69.6 and 46.2).
-    auto load = [&](int ci, Frag &f) {
-        if (PIPED && ci >= c1) ci = c1 - 1;
-        const GsMats m(a.ws, (size_t)ci * a.heads + h, Dp, Vp, DELTA);
+    // them.  What lies past the end is the last chunk (PIPED) again.
+    // In two halves, and spread over the products of a chunk: a CU takes 64 bytes a cycle, a chunk brings 56 to 72 KB, and a wave that asks for its share
+    // at once stands still until the rest of them is taken.
+    auto load_left = [&](const GsMats &m, Frag &f) {
 #pragma unroll
-        for (int k = 0; k < NT; ++k) {
-            const int d = d0 + 16 * k + 4 * g;
+        for (int k = 0; k < NT; ++k)
 #pragma unroll
             for (int r = 0; r < 2; ++r) {
-                if constexpr (DELTA) f.w[r][k] = *reinterpret_cast<const float4 *>(m.W + (size_t)(16 * r + c) * Dp + d);
-                f.q[r][k] = *reinterpret_cast<const float4 *>(m.Q + (size_t)(16 * r + c) * Dp + d);
-                f.k[k][r] = *reinterpret_cast<const float4 *>(m.KT + (size_t)(d0 + 16 * k + c) * C + 16 * r + 4 * g);
-            }
-            const float4 gv = *reinterpret_cast<const float4 *>(m.G + d);
-            f.gd[k] = gs_f4{gv.x, gv.y, gv.z, gv.w};
-        }
-        const int t0 = t_first + (ci - c0) * C;
-#pragma unroll
-        for (int r = 0; r < 2; ++r) f.a[r] = *reinterpret_cast<const float4 *>(m.A + (16 * (wave & 1) + c) * C + 16 * r + 4 * g);
-#pragma unroll
-        for (int r = 0; r < 2; ++r)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int tk = 16 * r + 4 * g + i;
-                if constexpr (DELTA) f.u[r][i] = m.U[(size_t)tk * Vp + col];
-                else f.u[r][i] = a.in[(size_t)(t0 + tk < t_end ? t0 + tk : t_end - 1) * a.ld + a.at_v + h * V + col_in];
+                const int at = gs_tile(wave * NT + k, r, lane);
+                if constexpr (DELTA) f.w[r][k] = *reinterpret_cast<const gs_f4 *>(m.W + at);
+                f.q[r][k] = *reinterpret_cast<const gs_f4 *>(m.Q + at);
             }
     };
-    auto step = [&](int ci, const Frag &cur) {
+    auto load_right = [&](const GsMats &m, Frag &f) {
+#pragma unroll
+        for (int k = 0; k < NT; ++k) {
+#pragma unroll
+            for (int r = 0; r < 2; ++r) f.k[k][r] = *reinterpret_cast<const gs_f4 *>(m.KT + gs_tile(wave * NT + k, r, lane));
+            f.gd[k] = *reinterpret_cast<const gs_f4 *>(m.G + d0 + 16 * k + 4 * g);
+        }
+#pragma unroll
+        for (int r = 0; r < 2; ++r) f.u[r] = *reinterpret_cast<const gs_f4 *>(m.U + gs_tile(vt, r, lane));
+    };
+    auto mats = [&](int ci) { return GsMats(a.ws, (size_t)(PIPED && ci >= c1 ? c1 - 1 : ci) * a.heads + h, Dp, Vp, DELTA); };
+    auto load = [&](int ci, Frag &f) {
+        const GsMats m = mats(ci);
+        load_left(m, f);
+        load_right(m, f);
+    };
+    // chunk ci, and the loads of chunk `ahead` beside it
+    auto step = [&](int ci, const Frag &cur, int ahead, Frag *next) {
         float (*rd)[DELTA ? 4 : 2][64][4] = red[(ci - c0) & 1];
+        const GsMats m = mats(ahead);
         gs_f4 ws[2], qs[2];
+        if constexpr (PIPED) {
+            __builtin_amdgcn_sched_barrier(0);
+            load_left(m, *next);
+        }
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
             ws[r] = qs[r] = gs_f4{0.f, 0.f, 0.f, 0.f};
@@ -571,36 +653,27 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const GatedStateArgs a)
                 if constexpr (DELTA) ws[r] = gs_mma(cur.w[r][k], S[k], ws[r]);
                 qs[r] = gs_mma(cur.q[r][k], S[k], qs[r]);
             }
+        }
+        if constexpr (PIPED) {
+#pragma unroll
+            for (int i = 0; i < (DELTA ? 4 : 2) * NT; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+                __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
             *reinterpret_cast<gs_f4 *>(rd[wave][r][lane]) = qs[r];
             if constexpr (DELTA) *reinterpret_cast<gs_f4 *>(rd[wave][2 + r][lane]) = ws[r];
         }
         // one barrier a chunk: the buffer of this parity is written again two chunks on, behind the next chunk's barrier
-        __syncthreads();
+        lds_barrier();
         gs_f4 u[2] = {cur.u[0], cur.u[1]};
-        if constexpr (!DELTA) {
-#pragma unroll
-            for (int r = 0; r < 2; ++r)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) u[r][i] = t_first + (ci - c0) * C + 16 * r + 4 * g + i < t_end && col < V ? u[r][i] : 0.f;
-        } else {
-#pragma unroll
-            for (int r = 0; r < 2; ++r)
-#pragma unroll
-                for (int w = 0; w < 4; ++w) u[r] -= *reinterpret_cast<const gs_f4 *>(rd[w][2 + r][lane]);
-        }
-        if (wave < 2) {                 // the outputs of row tile `wave`
-            gs_f4 o = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int w = 0; w < 4; ++w) o += *reinterpret_cast<const gs_f4 *>(rd[w][wave][lane]);
-#pragma unroll
-            for (int s = 0; s < 2; ++s)
-                if (s <= wave) o = gs_mma(cur.a[s], u[s], o);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int tk = 16 * wave + 4 * g + i;
-                const int t = t_first + (ci - c0) * C + tk;
-                if (t < t_end && col < V) a.o[(size_t)t * a.heads * V + h * V + col] = o[i];
-            }
+        settle(ci, u, 2);
+        if constexpr (PIPED) {
+            __builtin_amdgcn_sched_barrier(0);
+            load_right(m, *next);
         }
 #pragma unroll
         for (int k = 0; k < NT; ++k) {
@@ -608,31 +681,39 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const GatedStateArgs a)
             s = gs_mma(cur.k[k][0], u[0], s);
             S[k] = gs_mma(cur.k[k][1], u[1], s);
         }
+        if constexpr (PIPED) {
+#pragma unroll
+            for (int i = 0; i < 3 * NT + 2; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+                __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
     };
     Frag f0;
     if constexpr (!PIPED) {
-        for (int ci = c0; ci < c1; ++ci) { load(ci, f0); step(ci, f0); }
-    } else if constexpr (NT < 4) {          // (two chunks ahead, as many as the registers hold)
+        for (int ci = c0; ci < c1; ++ci) { load(ci, f0); step(ci, f0, ci, nullptr); }
+    } else if constexpr (NT < 3) {          // (two chunks ahead, as many as the registers hold)
         Frag f1, f2;
         load(c0, f0);
         load(c0 + 1, f1);
         int ci = c0;
         for (; ci + 3 <= c1; ci += 3) {
-            load(ci + 2, f2); step(ci, f0);
-            load(ci + 3, f0); step(ci + 1, f1);
-            load(ci + 4, f1); step(ci + 2, f2);
+            step(ci, f0, ci + 2, &f2);
+            step(ci + 1, f1, ci + 3, &f0);
+            step(ci + 2, f2, ci + 4, &f1);
         }
-        if (ci < c1) { load(ci + 2, f2); step(ci, f0); }
-        if (ci + 1 < c1) { load(ci + 3, f0); step(ci + 1, f1); }
+        if (ci < c1) step(ci, f0, ci + 2, &f2);
+        if (ci + 1 < c1) step(ci + 1, f1, ci + 2, &f2);
     } else {
         Frag f1;
         load(c0, f0);
         int ci = c0;
         for (; ci + 2 <= c1; ci += 2) {
-            load(ci + 1, f1); step(ci, f0);
-            load(ci + 2, f0); step(ci + 1, f1);
+            step(ci, f0, ci + 1, &f1);
+            step(ci + 1, f1, ci + 2, &f0);
         }
-        if (ci < c1) { load(ci + 1, f1); step(ci, f0); }
+        if (ci < c1) step(ci, f0, ci + 1, &f1);
     }
 #pragma unroll
     for (int k = 0; k < NT; ++k)
@@ -704,7 +785,7 @@ int gated_state_step(const GatedStateArgs &a, int T, hipStream_t stream) {
 
 template <bool DELTA, bool PIPED>
 static int launch_scan_of(const GatedStateArgs &a, hipStream_t stream) {
-    const dim3 grid((unsigned)a.heads, (unsigned)(gs_pad16(a.vdim) / 16), (unsigned)a.chunks.n_runs), block(256);
+    const dim3 grid((unsigned)a.heads, (unsigned)(gs_pad16(a.vdim) / 16), (unsigned)a.chunks.n_runs), block(SCAN_THREADS);
     switch (gs_pad64(a.dim) / 64) {
         case 1: MESH_LAUNCH((state_scan_kernel<DELTA, 1, PIPED>), grid, block, 0, stream, a); break;
         case 2: MESH_LAUNCH((state_scan_kernel<DELTA, 2, PIPED>), grid, block, 0, stream, a); break;
