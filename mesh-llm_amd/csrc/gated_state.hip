@@ -74,15 +74,19 @@ __device__ __forceinline__ void delta_conv_run(const GatedStateArgs &a, const fl
 }
 
 // ---- one token per sequence
-// grid (heads, T).  Thread (row group, column): RPT rows of one column of the state in registers.
+// grid (heads, T, slices of `cols` value columns, a power of two).  Thread (row group, column): RPT rows of one column of the state in registers.
+// A slice of several leaves o as it is, for a product that norms and gates it (linear.hpp: STEP_IN_HEADS): a head's rms is over all of
+// them.  (The arguments that the state's address waits for stand in front, see gemv.hip.)
+// Bound by its chain: place of the state, state and inputs, sums over the row groups, the state's rows back.  16 heads of 128 x 128, us: a
+// workgroup a head, which moves 128 KB of state by itself, the place read through the argument block 10.4; four slices a head 7.2.
 template <int THREADS, int RPT>
-__global__ __launch_bounds__(THREADS) void gated_step_kernel(const GatedStateArgs a, int vt) {
+__global__ __launch_bounds__(THREADS) void gated_step_kernel(const int32_t *p_pos, const int32_t *p_seq, float *p_state, int p_heads, int p_D, int p_V, int p_cols, const GatedStateArgs a) {
     __shared__ float sq[STATE_DIM_MAX], sk[STATE_DIM_MAX], sd[STATE_DIM_MAX], sv[STATE_DIM_MAX], so[STATE_DIM_MAX];
     __shared__ float red[2][THREADS], s_qk, s_ss;
     const int h = blockIdx.x, t = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int D = a.dim, V = a.vdim, seq = a.seq[t], pos = a.pos[t];
-    const int col = tid & (vt - 1), grp = tid / vt, groups = THREADS / vt;
-    float *st = a.state + ((size_t)seq * a.heads + h) * D * V;
+    const int D = p_D, V = p_V, seq = p_seq[t], pos = p_pos[t];
+    const int cols = p_cols, v0 = blockIdx.z * cols, mine = tid & (cols - 1), col = v0 + mine, grp = tid / cols, groups = THREADS / cols;
+    float *st = p_state + ((size_t)seq * p_heads + h) * D * V;
     // the state's rows are requested before anything is computed
     float S[RPT];
 #pragma unroll
@@ -100,10 +104,11 @@ __global__ __launch_bounds__(THREADS) void gated_step_kernel(const GatedStateArg
         beta = delta_beta(a, t, h);
         const int kvh = h / (a.heads / a.kv_heads), channels = 2 * a.kv_heads * D + a.heads * V, taps = a.taps, now = pos % taps;
         float *tail = a.tail + (size_t)seq * taps * channels;
-        const bool own = h % (a.heads / a.kv_heads) == 0;           // one head of a group keeps the shared channels' inputs
-        for (int i = tid; i < 2 * D + V; i += THREADS) {
+        const bool own = h % (a.heads / a.kv_heads) == 0 && v0 == 0;           // one head of a group, and one slice, keeps the shared channels' inputs
+        const int vs = V - v0 < cols ? V - v0 : cols;
+        for (int i = tid; i < 2 * D + vs; i += THREADS) {
             const int part = i < D ? 0 : i < 2 * D ? 1 : 2, e = part == 0 ? i : part == 1 ? i - D : i - 2 * D;
-            const int c = part == 2 ? h * V + e : kvh * D + e;
+            const int c = part == 2 ? h * V + v0 + e : kvh * D + e;
             const int at = (part == 0 ? a.at_q : part == 1 ? a.at_k : a.at_v) + c, ch = (part == 0 ? 0 : part == 1 ? a.kv_heads * D : 2 * a.kv_heads * D) + c;
             const float *w = (part == 0 ? a.conv_q : part == 1 ? a.conv_k : a.conv_v) + (size_t)c * taps;
             const float xi = x[at];
@@ -142,7 +147,7 @@ __global__ __launch_bounds__(THREADS) void gated_step_kernel(const GatedStateArg
             z = group_sum<4>(z);
             if (d < D && (tid & 3) == 0) sd[d] = expf(-gs_softplus(-(z + a.a2_bias[h * D + d])) * a.inv_tau);
         }
-        for (int v = tid; v < V; v += THREADS) sv[v] = x[a.at_v + h * V + v];
+        for (int v = tid; v < cols && v0 + v < V; v += THREADS) sv[v] = x[a.at_v + h * V + v0 + v];
     }
     __syncthreads();
     if (wave == 0) {
@@ -163,13 +168,17 @@ __global__ __launch_bounds__(THREADS) void gated_step_kernel(const GatedStateArg
     red[0][tid] = dk; red[1][tid] = dq;
     __syncthreads();
     dk = dq = 0.f;
-    for (int g = 0; g < groups; ++g) { dk += red[0][g * vt + col]; dq += red[1][g * vt + col]; }
-    const float v = col < V ? sv[col] : 0.f;
+    for (int g = 0; g < groups; ++g) { dk += red[0][g * cols + mine]; dq += red[1][g * cols + mine]; }
+    const float v = col < V ? sv[mine] : 0.f;
     const float u = a.delta ? beta * (v - dk) : v;
 #pragma unroll
     for (int i = 0; i < RPT; ++i) {
         const int d = grp + i * groups;
         if (d < D && col < V) st[(size_t)d * V + col] = fmaf(sk[d], u, S[i]);
+    }
+    if (gridDim.z > 1) {
+        if (grp == 0 && col < V) static_cast<float *>(a.out)[(size_t)t * a.ld_out + h * V + col] = fmaf(s_qk, u, dq);
+        return;
     }
     if (grp == 0 && col < V) so[col] = fmaf(s_qk, u, dq);
     __syncthreads();
@@ -767,18 +776,23 @@ static bool args_ok(const GatedStateArgs &a) {
            (a.delta ? a.taps >= 1 && a.tail && a.conv_q && a.conv_k && a.conv_v && a.A && a.dt_bias : a.kv_heads == a.heads && a.rank >= 1 && a.rank <= STATE_RANK_MAX && a.a2 && a.a2_bias);
 }
 
+template <int THREADS, int RPT>
+static void launch_step(const GatedStateArgs &a, int T, int cols, int slices, hipStream_t stream) {
+    MESH_LAUNCH((gated_step_kernel<THREADS, RPT>), dim3((unsigned)a.heads, (unsigned)T, (unsigned)slices), dim3(THREADS), 0, stream, a.pos, a.seq, a.state, a.heads, a.dim, a.vdim, cols, a);
+}
 int gated_state_step(const GatedStateArgs &a, int T, hipStream_t stream) {
     if (T <= 0) return MESH_OK;
-    if (!args_ok(a) || T > 65535) return fail(MESH_ERR_INVALID, "gated_state_step: bad operands");
-    int vt = 16;
-    while (vt < a.vdim) vt *= 2;
-    const dim3 grid((unsigned)a.heads, (unsigned)T);
-    const int rows512 = (a.dim + 512 / vt - 1) / (512 / vt);
-    if (rows512 <= 4) MESH_LAUNCH((gated_step_kernel<512, 4>), grid, dim3(512), 0, stream, a, vt);
-    else if (rows512 <= 8) MESH_LAUNCH((gated_step_kernel<512, 8>), grid, dim3(512), 0, stream, a, vt);
-    else if (rows512 <= 16) MESH_LAUNCH((gated_step_kernel<512, 16>), grid, dim3(512), 0, stream, a, vt);
-    else if (rows512 <= 32) MESH_LAUNCH((gated_step_kernel<512, 32>), grid, dim3(512), 0, stream, a, vt);
-    else MESH_LAUNCH((gated_step_kernel<1024, 64>), grid, dim3(1024), 0, stream, a, vt);         // (up to 256 x 256)
+    if (!args_ok(a) || T > 65535 || (a.raw && (a.act != ACT_F32 || !gated_state_raw(a.vdim)))) return fail(MESH_ERR_INVALID, "gated_state_step: bad operands");
+    int cols = 16;
+    while (cols < a.vdim) cols *= 2;
+    if (a.raw) cols = GATED_STEP_SLICE;
+    const int slices = (a.vdim + cols - 1) / cols;
+    const int rows512 = (a.dim + 512 / cols - 1) / (512 / cols);
+    if (rows512 <= 4) launch_step<512, 4>(a, T, cols, slices, stream);
+    else if (rows512 <= 8) launch_step<512, 8>(a, T, cols, slices, stream);
+    else if (rows512 <= 16) launch_step<512, 16>(a, T, cols, slices, stream);
+    else if (rows512 <= 32) launch_step<512, 32>(a, T, cols, slices, stream);
+    else launch_step<1024, 64>(a, T, cols, slices, stream);         // (up to 256 x 256)
     MESH_LAUNCH_CHECK();
     return MESH_OK;
 }

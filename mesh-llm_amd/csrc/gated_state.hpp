@@ -53,7 +53,11 @@ struct GatedStateArgs {
     void *out = nullptr;
     ActType act = ACT_BF16;
     int ld_out = 0;
+    // gated_state_step, where gated_state_raw says so, f32: rows of o as they are, neither normed nor gated (linear.hpp: STEP_IN_HEADS does that)
+    bool raw = false;
 };
+constexpr int GATED_STEP_SLICE = 32;        // value columns of a workgroup then
+inline bool gated_state_raw(int vdim) { return vdim > GATED_STEP_SLICE && vdim <= STATE_DIM_MAX && (vdim & (vdim - 1)) == 0; }
 inline bool gated_state_supported(int dim, int vdim) { return dim <= STATE_DIM_MAX && vdim <= STATE_DIM_MAX; }
 inline int gated_state_channels(const GatedStateArgs &a) { return 2 * a.kv_heads * a.dim + a.heads * a.vdim; }
 size_t gated_state_workspace(int n_chunks, int heads, int dim, int vdim);

@@ -344,6 +344,8 @@ static int run_step(mesh_session *s, int max_keys) {
     for (size_t il = 0; il < hm.layers.size(); ++il) {
         const HybridLayer &L = hm.layers[il];
         const MixerSpec &m = L.spec.mixer;
+        StepArgs o = base(L.out, nullptr, STEP_OUT_PLAIN);
+        o.in = inner;
         if (m.kind == MIXER_MIN_GRU) {
             StepArgs a = base(L.in, inner, STEP_OUT_MIN_GRU);
             a.width = m.width; a.bias_z = L.bias_z; a.bias_x = L.bias_x; a.state = h.state[il];
@@ -357,12 +359,13 @@ static int run_step(mesh_session *s, int max_keys) {
                 q.in_kind = STEP_IN_UNIT_RMS; q.in = h.big; q.gain = L.cq_norm;
                 if ((rc = run(q)) != MESH_OK || (rc = run_latent_rows(s, il, 1, max_keys, true, true)) != MESH_OK) return rc;
             } else {
+                GatedStateArgs g = gated_args(s, il, inner, ACT_F32);
+                g.raw = gated_state_raw(g.vdim) && g.at_g % 4 == 0;
+                if (g.raw) { o.in_kind = STEP_IN_HEADS; o.gain = g.norm; o.head_gate = g.in + g.at_g; o.head_width = g.vdim; }
                 ProfScope ps(s, MESH_PROF_PREP);
-                if ((rc = gated_state_step(gated_args(s, il, inner, ACT_F32), 1, stream)) != MESH_OK) return rc;
+                if ((rc = gated_state_step(g, 1, stream)) != MESH_OK) return rc;
             }
         }
-        StepArgs o = base(L.out, nullptr, STEP_OUT_PLAIN);
-        o.in = inner;
         if ((rc = to_stream(o, L.post1)) != MESH_OK) return rc;
         if (L.spec.ff) {
             StepArgs u = base(L.up, h.big, STEP_OUT_PLAIN), d = base(L.down, nullptr, STEP_OUT_PLAIN);

@@ -49,7 +49,8 @@ enum StepIn {
     STEP_IN_POLY = 3,         // x = c0 N(u) + c1 N(u^2) + c2 N(u^3) + c3, u = in, N(v) = v / rms(v)
     STEP_IN_LAYER = 4,        // v = in + LN(y) gain + bias (y null: v = in), also written to x_out; x = LN(v) norm_gain + norm_bias, LN(v) = (v - mean) / deviation
     STEP_IN_UNIT_RMS = 5,     // x = in / rms(in) * gain
-    STEP_IN_RELU2 = 6         // x = max(in, 0)^2
+    STEP_IN_RELU2 = 6,        // x = max(in, 0)^2
+    STEP_IN_HEADS = 7         // x = in / rms(in over its head of head_width) * gain[in the head] * silu(head_gate)
 };
 enum StepOut {
     STEP_OUT_PLAIN = 0,       // out = W x
@@ -65,7 +66,9 @@ struct StepArgs {
     StepOut out_kind = STEP_OUT_PLAIN;
     const float *in = nullptr;            // [K]
     const float *y = nullptr;             // RESIDUAL, LAYER: [K]
-    const float *gain = nullptr;          // RESIDUAL, LAYER with y, UNIT_RMS: [K]
+    const float *gain = nullptr;          // RESIDUAL, LAYER with y, UNIT_RMS: [K]; HEADS: [head_width]
+    const float *head_gate = nullptr;     // HEADS: [K], 16-byte aligned
+    int head_width = 0;                   // HEADS: a power of two from 4 to 256, K a whole number of them
     const float *bias = nullptr;          // LAYER with y: [K]
     const float *part = nullptr;          // RESIDUAL: [n_part]; POLY: [3][n_part]
     int n_part = 0;

@@ -173,6 +173,40 @@ __global__ __launch_bounds__(STEP_THREADS, 4) void linear_step_kernel(const uint
                      const float4 v = *reinterpret_cast<const float4 *>(xs + k);
                      return make_float4(v.x * (rinv * g.x), v.y * (rinv * g.y), v.z * (rinv * g.z), v.w * (rinv * g.w));
                  }, xs);
+    } else if constexpr (IN == STEP_IN_HEADS) {
+        // a head's four-element groups lie in neighbouring lanes of a wave
+        constexpr int AHEAD = 2, STRIDE = STEP_THREADS * 4;
+        const int width = a.head_width, k0 = tid * 4;
+        float4 o4[AHEAD], g4[AHEAD], n4[AHEAD];
+        auto request = [&](int k, float4 &o, float4 &g, float4 &n) {
+            const int at = k < K ? k : K - 4;
+            o = *reinterpret_cast<const float4 *>(a.in + at);
+            g = *reinterpret_cast<const float4 *>(a.head_gate + at);
+            n = *reinterpret_cast<const float4 *>(a.gain + (at & (width - 1)));
+        };
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) request(k0 + i * STRIDE, o4[i], g4[i], n4[i]);
+        fetch_first();
+        auto put = [&](int k, const float4 &o, const float4 &g, const float4 &n) {
+            float ss = fmaf(o.x, o.x, fmaf(o.y, o.y, fmaf(o.z, o.z, o.w * o.w)));
+            if (width > 4) ss = lane_fold<1>(ss, LaneAdd{});
+            if (width > 8) ss = lane_fold<2>(ss, LaneAdd{});
+            if (width > 16) ss = lane_fold<4>(ss, LaneAdd{});
+            if (width > 32) ss = lane_fold<8>(ss, LaneAdd{});
+            if (width > 64) ss = lane_fold<16>(ss, LaneAdd{});
+            if (width > 128) ss = lane_fold<32>(ss, LaneAdd{});
+            const float r = 1.0f / sqrtf(ss / (float)width + a.eps);
+            if (k < Kp)
+                *reinterpret_cast<float4 *>(xs + k) = k < K ? make_float4(o.x * r * n.x * act_silu(g.x), o.y * r * n.y * act_silu(g.y), o.z * r * n.z * act_silu(g.z), o.w * r * n.w * act_silu(g.w))
+                                                            : make_float4(0.f, 0.f, 0.f, 0.f);
+        };
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) put(k0 + i * STRIDE, o4[i], g4[i], n4[i]);
+        for (int first_k = (tid & ~63) * 4 + AHEAD * STRIDE; first_k < Kp; first_k += STRIDE) {       // (whole waves)
+            const int k = first_k + lane * 4;
+            request(k, o4[0], g4[0], n4[0]);
+            put(k, o4[0], g4[0], n4[0]);
+        }
     } else if constexpr (IN == STEP_IN_LAYER) {
         // a thread's first AHEAD groups of four, of every vector, are requested before the first sum; means first, then squared
         // deviations
@@ -417,6 +451,9 @@ int linear_step(const StepArgs &a, hipStream_t stream) {
         return fail(MESH_ERR_INVALID, "linear_step: input description incomplete");
     if ((a.in_kind == STEP_IN_LAYER && (!a.norm_gain || !a.norm_bias || (a.y && (!a.gain || !a.bias || !a.x_out || a.x_out == a.in)))) || (a.in_kind == STEP_IN_UNIT_RMS && !a.gain))
         return fail(MESH_ERR_INVALID, "linear_step: input description incomplete");
+    if (a.in_kind == STEP_IN_HEADS && (!a.gain || !a.head_gate || a.head_width < 4 || a.head_width > 256 || (a.head_width & (a.head_width - 1)) || W.K % a.head_width ||
+                                       ((reinterpret_cast<uintptr_t>(a.in) | reinterpret_cast<uintptr_t>(a.head_gate) | reinterpret_cast<uintptr_t>(a.gain)) & 15)))
+        return fail(MESH_ERR_INVALID, "linear_step: input description incomplete");
     if (((a.out_kind == STEP_OUT_SUMSQ || a.out_kind == STEP_OUT_POWERS) && !a.out_part) ||
         (a.out_kind == STEP_OUT_MIN_GRU && (!a.state || !a.pos || !a.seq || !a.bias_z || !a.bias_x || a.width < 1 || W.M != 3 * a.width)) ||
         (a.out_kind == STEP_OUT_SIDE && (!a.side || !a.tok)))
@@ -429,6 +466,8 @@ int linear_step(const StepArgs &a, hipStream_t stream) {
     MESH_STEP_CASE(STEP_IN_LAYER, STEP_OUT_PLAIN)
     MESH_STEP_CASE(STEP_IN_UNIT_RMS, STEP_OUT_PLAIN)
     MESH_STEP_CASE(STEP_IN_RELU2, STEP_OUT_PLAIN)
+    MESH_STEP_CASE(STEP_IN_HEADS, STEP_OUT_PLAIN)
+    MESH_STEP_CASE(STEP_IN_HEADS, STEP_OUT_SUMSQ)
     MESH_STEP_CASE(STEP_IN_VEC, STEP_OUT_SUMSQ)
     MESH_STEP_CASE(STEP_IN_POLY, STEP_OUT_SUMSQ)
     MESH_STEP_CASE(STEP_IN_RESIDUAL, STEP_OUT_POWERS)

@@ -254,6 +254,22 @@ def test_unequal_requests_in_one_call_equal_each_alone(tmp_path, prec):
     st.close()
 
 
+# value columns in slices, whose heads the output product norms: two to eight slices a head, rows of more and fewer groups than a workgroup has;
+# gates that do not lie on 16 bytes, which stay with a workgroup a head; rows past the groups that the product requests ahead
+@BOTH
+@pytest.mark.parametrize("layers", [[N.delta(3, 1, 40, 64, 4), N.gla(2, 24, 128, 8.0)], [N.delta(5, 5, 21, 128, 2), N.gla(3, 130, 64, 2.0)], [N.gla(33, 16, 128, 4.0), N.delta(1, 1, 256, 256, 1)]])
+def test_single_steps_of_states_in_slices(tmp_path, layers, prec):
+    cfg, w, folder, orc = made(tmp_path, N.config(50, 72, layers))
+    t = prompt(cfg, 24, 8)
+    want = orc.forward(t)
+    st = open_stage(folder, prec)
+    got = run(st, t, [1] * 24)
+    assert off(got, want, prec) < 1
+    # the launches of many tokens, which norm a head where they write it: f32 sums in another order
+    assert off(run(st, t, [1] * 24, step_fused=0), want, prec) < 1
+    st.close()
+
+
 # workgroups of a scan on both sides of one a CU, sequences of one to three chunks of 32 tokens and parts of them
 @BOTH
 @pytest.mark.parametrize("name,lens", [("wide-states", [70, 1, 32, 33] * 5), ("wide-states", [64, 65, 96]), ("states-only", [40, 33, 8] * 14), ("states-only", [8, 97, 31])])
