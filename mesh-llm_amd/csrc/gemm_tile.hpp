@@ -95,7 +95,10 @@ inline GtPlan gt_plan(int M, int T, int K, int slices_max, size_t slices_room, d
 
 // acc += W x over steps [k0, k0 + n_steps), n_steps >= 1.  w, x: 16-bit elements, rows of ldw and ldx (GT_BLOCKS: both K); w_block, x_block: first 16-row block of the
 // tile; w_blocks: blocks the matrix holds; x_rows: rows x holds (GT_BLOCKS: up to a whole block).  Blocks and rows past the end
-// repeat the last one; what they multiply is never stored.  SWAP: result rows = tokens, columns (lanes) = weight rows.
+// repeat the last one; what they multiply is never stored.  A wave's half of 32 tokens past the last one is brought into LDS with the tile, but neither read from there nor
+// multiplied: a clock that falls with the products at work gains on whole launches what those would have cost.  Chunks, us, multiplied / left out: four
+// 32B-shaped layers 270 tokens 1731 / 1620, 600 3014 / 2877, 800 3688 / 3518; eight 8B-shaped ones 333 2046 / 2023, 700 3405 / 3366,
+// 1600 6247 / 6124, whole tiles (1536) as before.  SWAP: result rows = tokens, columns (lanes) = weight rows.
 template <class V, GtLayout LW, GtLayout LX, int WM, int WT, bool SWAP, int STAGES = gt_stages(WM, WT)>
 __device__ __forceinline__ void gt_multiply(char *smem, gt_f16v (&acc)[2][2], const void *w, int ldw, const void *x, int ldx, int k0, int n_steps, int w_block, int w_blocks,
                                             int x_block, int x_rows) {
@@ -137,27 +140,30 @@ __device__ __forceinline__ void gt_multiply(char *smem, gt_f16v (&acc)[2][2], co
     const int in_blocks = ((lane & 31) >> 4) * 1024 + half * 256 + r16 * 16, in_rows = ((lane & 31) >> 4) * 1024 + r16 * 64 + (half ^ (r16 >> 2)) * 16;
     const int wf_at = (wave % WM) * 4096 + (LW == GT_BLOCKS ? in_blocks : in_rows), xf_at = (WM + wave / WM) * 4096 + (LX == GT_BLOCKS ? in_blocks : in_rows);
     V wf[2][2], xf[2][2];
-    auto read = [&](const char *st, int ks) {
+    // LIVE: 32-token halves of this wave that hold tokens
+    auto read = [&](auto live, const char *st, int ks) {
+        constexpr int LIVE = decltype(live)::value;
         auto place_of = [&](GtLayout l, int at) { return l == GT_BLOCKS ? at + 512 * ks : at ^ (32 * ks); };
 #pragma unroll
-        for (int j = 0; j < 2; ++j) xf[ks][j] = *reinterpret_cast<const V *>(st + place_of(LX, xf_at) + 2048 * j);
+        for (int j = 0; j < LIVE; ++j) xf[ks][j] = *reinterpret_cast<const V *>(st + place_of(LX, xf_at) + 2048 * j);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) wf[ks][i] = *reinterpret_cast<const V *>(st + place_of(LW, wf_at) + 2048 * i);
+        for (int i = 0; i < (LIVE ? 2 : 0); ++i) wf[ks][i] = *reinterpret_cast<const V *>(st + place_of(LW, wf_at) + 2048 * i);
     };
-    auto step = [&](int stage, auto more, int next_stage, int next_k) {
+    auto step = [&](auto live, int stage, auto more, int next_stage, int next_k) {
+        constexpr int LIVE = decltype(live)::value;
         const char *st = smem + stage * STAGE;
-        read(st, 0);
+        read(live, st, 0);
         if constexpr (decltype(more)::value) load(next_stage, next_k);
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
-            if (ks == 0) read(st, 1);
+            if (ks == 0) read(live, st, 1);
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < (SWAP ? LIVE : 2); ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = SWAP ? gt_mma(xf[ks][i], wf[ks][j], acc[i][j]) : gt_mma(wf[ks][i], xf[ks][j], acc[i][j]);
-            if (ks == 0) {
+                for (int j = 0; j < (SWAP ? 2 : LIVE); ++j) acc[i][j] = SWAP ? gt_mma(xf[ks][i], wf[ks][j], acc[i][j]) : gt_mma(wf[ks][i], xf[ks][j], acc[i][j]);
+            if (ks == 0 && LIVE == 2) {
                 // the second half's fragments are requested between the first half's products
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
@@ -171,18 +177,25 @@ __device__ __forceinline__ void gt_multiply(char *smem, gt_f16v (&acc)[2][2], co
     };
 #pragma unroll
     for (int i = 0; i < STAGES - 1; ++i) load(i, i);
-    int k = 0;
-    for (; k + STAGES <= n_steps; k += STAGES) {
+    // (every wave passes the same barriers, whichever of the loops it runs)
+    auto steps = [&](auto live) {
+        int k = 0;
+        for (; k + STAGES <= n_steps; k += STAGES) {
 #pragma unroll
-        for (int i = 0; i < STAGES; ++i) {
-            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(PER * (STAGES - 2)) : "memory");
-            step(i, std::true_type{}, (i + STAGES - 1) % STAGES, k + i + STAGES - 1);
+            for (int i = 0; i < STAGES; ++i) {
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(PER * (STAGES - 2)) : "memory");
+                step(live, i, std::true_type{}, (i + STAGES - 1) % STAGES, k + i + STAGES - 1);
+            }
         }
-    }
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
-    for (int i = 0; i < STAGES - 1; ++i)
-        if (k + i < n_steps) step(i, std::false_type{}, 0, 0);
+        for (int i = 0; i < STAGES - 1; ++i)
+            if (k + i < n_steps) step(live, i, std::false_type{}, 0, 0);
+    };
+    const int tokens = x_rows - x_block * 16 - (wave / WM) * 64;        // from this wave's first on
+    if (tokens > 32) steps(std::integral_constant<int, 2>{});
+    else if (tokens > 0) steps(std::integral_constant<int, 1>{});
+    else steps(std::integral_constant<int, 0>{});
 }
 
 __device__ __forceinline__ void gt_clear(gt_f16v (&acc)[2][2]) {

@@ -87,6 +87,12 @@ KQUANT_MANY_CASES = [
     # slices that are no power of two: five of 42 steps, the last of 40; three of 67, the last of 66
     ((2304, 2, 1, 6656), 129, (2, 2, 8), (2, 2, 1), (2, 2, 1), (2, 2, 5)),
     ((2816, 2, 1, 6400), 257, (2, 2, 8), (2, 2, 1), (4, 3, 2), (2, 2, 3)),
+    # waves with both, one and none of their two halves of 32 tokens: a whole half and a token past it, behind a whole wave and in front of empty ones
+    ((512, 4, 1, 768), 160, (2, 2, 1), (2, 2, 1), (2, 2, 1), (2, 2, 1)),
+    ((512, 4, 1, 768), 161, (2, 2, 1), (2, 2, 1), (2, 2, 1), (2, 2, 1)),
+    ((2048, 16, 4, 2048), 288, (2, 2, 2), (2, 2, 4), (2, 2, 2), (2, 2, 4)),
+    ((256, 2, 1, 28672), 289, (2, 2, 1), (2, 2, 1), (4, 3, 1), (2, 2, 8)),
+    ((256, 2, 1, 28672), 417, (2, 2, 1), (2, 2, 1), (4, 4, 1), (2, 2, 8)),
 ]
 
 
