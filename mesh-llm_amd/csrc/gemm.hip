@@ -292,8 +292,9 @@ __device__ __forceinline__ int staged_slot(int s) { return (s & ~63) + 2 * ((s &
 // 16 k is four contiguous 256-byte pieces of that layout, so each lane fetches its 16 bytes straight from memory (L2),
 // four k16 steps ahead, into a ring of registers.  That halves the LDS reads per MFMA and leaves the staging waves only
 // the weights.
+// Wp, w_block: a GEMM layout, and the workgroup's row block in it.
 template <int TYPE, bool PACKED, bool XDIRECT, bool SPLIT>
-__global__ __launch_bounds__(GEMM_THREADS) void gemm_kq_kernel(GemmArgs a) {
+__device__ __forceinline__ void kq_tile(const GemmArgs &a, const uint8_t *Wp, int w_block) {
     extern __shared__ __align__(16) _Float16 gemm_smem[];
     _Float16 *Ws = gemm_smem;                                  // [2][GM][LDS_LD]
     _Float16 *Xs = gemm_smem + 2 * GM * LDS_LD;                // [2][GN][LDS_LD]
@@ -301,7 +302,6 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_kq_kernel(GemmArgs a) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int t0 = blockIdx.y * GN, t_end = a.T;
-    const uint8_t *Wp = static_cast<const uint8_t *>(a.Wp);
     const int m0 = blockIdx.x * GM;
     const int nsb = a.K / QK_K, n_all = a.K / GK;
     // k-steps [k0, k0 + n_steps) of this workgroup: all of them, or slice blockIdx.z of a split launch
@@ -316,7 +316,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_kq_kernel(GemmArgs a) {
         const int srow = st >> 1, sh = st & 1, slot = staged_slot(st);
         const int wrow = m0 + srow;                                  // rows beyond M are zero tiles (M padded to 16)
         const bool wlive = PACKED || wrow < a.M_pad;                 // (the GEMM layout holds its zero rows)
-        const uint8_t *wtile_row = PACKED ? Wp + ((size_t)blockIdx.x * n_all + k0) * PackedSub<TYPE>::CHUNK
+        const uint8_t *wtile_row = PACKED ? Wp + ((size_t)w_block * n_all + k0) * PackedSub<TYPE>::CHUNK
                                           : static_cast<const uint8_t *>(a.W) + (size_t)((wlive ? wrow : 0) >> 4) * nsb * TB;
         using Sub = typename std::conditional<PACKED, PackedSub<TYPE>, RawSub<TYPE>>::type;
         const int tok = t0 + srow;
@@ -537,6 +537,20 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_kq_kernel(GemmArgs a) {
                 *reinterpret_cast<float4 *>(Y + (size_t)t * ldy + m) = o;
             }
         }
+}
+
+template <int TYPE, bool PACKED, bool XDIRECT, bool SPLIT>
+__global__ __launch_bounds__(GEMM_THREADS) void gemm_kq_kernel(GemmArgs a) {
+    kq_tile<TYPE, PACKED, XDIRECT, SPLIT>(a, static_cast<const uint8_t *>(a.Wp), (int)blockIdx.x);
+}
+
+// Several matrices of which the last is of another type: its few row blocks beside the others' instead of in a launch of their own, which
+// must split K to fill the chip and add the slices in one more.
+template <int TYPE, int LAST, bool SPLIT>
+__global__ __launch_bounds__(GEMM_THREADS) void gemm_kq_types_kernel(GemmArgs a) {
+    const int bx = (int)blockIdx.x, begin = a.n_seg > 2 ? a.seg_begin[2] : a.seg_begin[1];
+    if (bx < begin) kq_tile<TYPE, true, true, SPLIT>(a, static_cast<const uint8_t *>(a.Wp), bx);
+    else kq_tile<LAST, true, true, SPLIT>(a, static_cast<const uint8_t *>(a.Wp_last), bx - begin);
 }
 
 // ---- expert launches ------------------------------------------------------------------------------------------------------
@@ -1251,6 +1265,14 @@ static int launch_gemm_kernel(const GemmArgs &k, dim3 grid, hipStream_t stream) 
     return SPLIT ? gemm_add_slices(k, (int)grid.x, stream) : MESH_OK;
 }
 
+template <int TYPE, int LAST, bool SPLIT>
+static int launch_gemm_types(const GemmArgs &k, dim3 grid, hipStream_t stream) {
+    constexpr size_t smem = sizeof(_Float16) * 2 * GM * LDS_LD;
+    MESH_LAUNCH((gemm_kq_types_kernel<TYPE, LAST, SPLIT>), grid, dim3(GEMM_THREADS), smem, stream, k);
+    MESH_LAUNCH_CHECK();
+    return SPLIT ? gemm_add_slices(k, (int)grid.x, stream) : MESH_OK;
+}
+
 // groups of waves along K: four where a CU gets one workgroup (16 waves), two where it gets several or K is split already
 template <int TYPE, int NT, int MODE>
 static int launch_gemm_reg(const GemmArgs &k, dim3 grid, hipStream_t stream) {
@@ -1290,6 +1312,25 @@ int gemm_split_count(const GemmArgs &a) {
     const int row_blocks = a.y16_k8 ? (a.M + GM / 2 - 1) / (GM / 2) : (a.M + GM - 1) / GM;
     int kps;
     return split_plan(a, row_blocks, (a.T + GN - 1) / GN, &kps);
+}
+
+// the 256 x 128 tile, where its workgroups give every CU one
+static bool takes_big(const GemmArgs &a, int row_blocks, int slices) {
+    return a.x_k8 && a.Wp && slices <= 1 && !a.rope.pos && row_blocks % 2 == 0 && a.big_tile && (row_blocks / 2) * ((a.T + GN - 1) / GN) >= gt_n_cu();
+}
+
+// Not where the others are cut along K otherwise without the last, whose rows would leave them fewer slices, nor where they take the 256-row tile.
+// q and k of q4_K, v of q6_K, apart / together, us: 4096 + 512 and 512 x 2048, 600 tokens 22.4 + 9.4 + 5.0 (the slices of v) / 26.0; eight layers of
+// the expert shard 70 tokens 1095 / 1043, 200 1325 / 1270, 600 1950 / 1902, 1300 3151 / 3099, 1700 3864 / 3865; eight 8B-shaped layers
+// without f16 copies 70 tokens 1041 / 999, 200 1601 / 1558, 900 4635 / 4564.
+bool gemm_types_ride(const GemmArgs &a) {
+    if (!a.Wp || !a.Wp_last || !a.x_k8 || a.n_seg < 2 || a.y16_k8 || a.tiles || gemm_tile_takes(a)) return false;
+    if (!((a.type == MESH_Q4_K && a.type_last == MESH_Q6_K) || (a.type == MESH_Q6_K && a.type_last == MESH_Q4_K))) return false;
+    if (a.T <= GN / 2 && a.narrow_tile) return false;
+    const int first = a.seg_begin[a.n_seg - 1], t_blocks = (a.T + GN - 1) / GN;
+    int kps;
+    const int slices = split_plan(a, first, t_blocks, &kps);
+    return !takes_big(a, first, slices) && split_plan(a, (a.M + GM - 1) / GM, t_blocks, &kps) == slices;
 }
 
 int gemm_kquant(const GemmArgs &a, hipStream_t stream) {
@@ -1339,11 +1380,15 @@ int gemm_kquant(const GemmArgs &a, hipStream_t stream) {
         return fail(MESH_ERR_INVALID, "gemm: RoPE / KV append on a launch it does not fit");
     if (a.type != MESH_Q4_K && a.type != MESH_Q6_K) return fail(MESH_ERR_UNSUPPORTED, "gemm: no MFMA kernel for ggml type %d", a.type);
     const bool q4 = a.type == MESH_Q4_K, packed = a.Wp != nullptr;
+    if (a.Wp_last) {
+        if (!gemm_types_ride(a)) return fail(MESH_ERR_INVALID, "gemm: matrices of two types in a launch they do not fit");
+        if (k.ksplit > 1) return q4 ? launch_gemm_types<MESH_Q4_K, MESH_Q6_K, true>(k, grid, stream) : launch_gemm_types<MESH_Q6_K, MESH_Q4_K, true>(k, grid, stream);
+        return q4 ? launch_gemm_types<MESH_Q4_K, MESH_Q6_K, false>(k, grid, stream) : launch_gemm_types<MESH_Q6_K, MESH_Q4_K, false>(k, grid, stream);
+    }
     // enough workgroups of the 256 x 128 tile to give every CU one: the big tile (gemm_big_kernel).  A pair of 512 row blocks and more
     // does at any token count: calls of 17 to 64 tokens over such a pair take it too, though the register-formed tile is the faster one
     // there (two layers 4096 wide with 33024 feed-forward rows: 388 against 286 us at 17 tokens, 473 against 377 at 64).
-    if (a.x_k8 && packed && k.ksplit <= 1 && !a.rope.pos && row_blocks % 2 == 0 && a.big_tile &&
-        (row_blocks / 2) * (int)grid.y >= gt_n_cu())
+    if (takes_big(a, row_blocks, k.ksplit))
         return q4 ? launch_gemm_big<MESH_Q4_K>(k, row_blocks, (int)grid.y, stream) : launch_gemm_big<MESH_Q6_K>(k, row_blocks, (int)grid.y, stream);
     if (a.x_k8) {
         if (packed) return q4 ? launch_gemm<MESH_Q4_K, true, true>(k, grid, stream) : launch_gemm<MESH_Q6_K, true, true>(k, grid, stream);

@@ -30,6 +30,9 @@ struct GemmArgs {
     int seg_begin[3] = {0, 0, 0}, seg_M[3] = {0, 0, 0}, seg_ldy[3] = {0, 0, 0};
     float *seg_Y[3] = {nullptr, nullptr, nullptr};
     const float *seg_bias[3] = {nullptr, nullptr, nullptr};
+    // Where gemm_types_ride() says so: the last of the n_seg matrices is of type_last, at Wp_last.
+    const void *Wp_last = nullptr;
+    int type_last = -1;
     // SwiGLU pair: Wp is a gate/up pair packed by gemm_pack_pair (every row block 64 gate rows, then the same 64 up
     // rows), M their common row count; the launch writes f16(silu(gate) * up) in the k8-major layout to y16_k8 (Y unused).
     _Float16 *y16_k8 = nullptr;
@@ -74,6 +77,9 @@ int gemm_kquant(const GemmArgs &a, hipStream_t stream);
 int gemm_split_count(const GemmArgs &a);
 // Whether the launch adds slices in a second kernel that can take the next norm along (one matrix and a residual).
 bool gemm_norm_rides(const GemmArgs &a);
+
+// Whether one launch takes matrices of both types (Wp_last).
+bool gemm_types_ride(const GemmArgs &a);
 
 // GEMM layout of a K-quant matrix: a second copy for the prefill GEMM, arranged by the workgroup tile that consumes it.
 // One chunk per (128-row block, 64-element k-step), chunks of a row block consecutive in k.  A chunk holds, for each of

@@ -795,16 +795,26 @@ static int run_layer_prefill(mesh_session *s, const LayerWeights &L, size_t il, 
             const DevTensor *w[3] = {&L.wq, &L.wk, &L.wv}, *b[3] = {&L.bq, &L.bk, &L.bv};
             float *y[3] = {s->q, s->k, s->v};
             GemmArgs g = gemm_k8(gemm_of(L.wq, s->xn16, E, T, s->q, QD, nullptr));
-            g.n_seg = tile ? 3 : L.qkv_fused;
+            g.n_seg = 0;
             g.Wt = L.qkv_tile;
             g.M = 0;
-            for (int i = 0; i < g.n_seg; ++i) {
+            auto add = [&](int i) {
                 g.seg_begin[i] = g.M / 128;
                 g.seg_M[i] = (int)w[i]->M; g.seg_ldy[i] = (int)w[i]->M; g.seg_Y[i] = y[i];
                 g.seg_bias[i] = b[i]->present() ? static_cast<const float *>(b[i]->data) : nullptr;
                 g.M += (int)w[i]->M;
-            }
+                g.n_seg = i + 1;
+            };
+            for (int i = 0; i < (tile ? 3 : L.qkv_fused); ++i) add(i);
             GemmArgs gv = gemm_k8(gemm_of(L.wv, s->xn16, E, T, s->v, KD, &L.bv));
+            // v of another K-quant type with them, where a kernel takes both
+            if (g.n_seg == 2 && gv.Wp && g.M % 128 == 0) {
+                const GemmArgs two = g;
+                add(2);
+                g.Wp_last = gv.Wp;
+                g.type_last = gv.type;
+                if (!gemm_types_ride(g)) g = two;
+            }
             // RoPE and the KV append ride in the second kernel of split launches (both launches must be split)
             if (s->tune.gemv_rope && hp.rope_mode == ROPE_MODE_NORM && st->k_type == MESH_F16 && st->v_type == MESH_F16 && !L.q_norm.present() &&
                 !L.k_norm.present() && hp.head_dim % 4 == 0 && hp.n_rot % 2 == 0 && gemm_split_count(g) > 1 &&

@@ -95,6 +95,15 @@ def test_gate_up_of_a_decode_batch(case):
     assert not any(n.startswith("gemm_reg") for n, _ in other)
 
 
+@pytest.mark.parametrize("shape,tokens,rides", tiles.TYPES_CASES)
+def test_projections_of_two_types(shape, tokens, rides):
+    names = [n for n, _ in call(kquant_products, cfg=tiles.kquant(*shape), layers=[0], tokens=tokens, tuning={"tile_copies": 0})]
+    assert any(n.startswith("gemm_kq_types_kernel<%d,%d," % (Q4_K, Q6_K)) for n in names) == rides, names
+    # (a call of few tokens, which the narrow tiles take)
+    names = [n for n, _ in call(kquant_products, cfg=tiles.kquant(*shape), layers=[0], tokens=64, tuning={"tile_copies": 0})]
+    assert not any("types" in n for n in names)
+
+
 @pytest.mark.parametrize("case", tiles.STEP_SLICE_CASES)
 def test_down_projections_of_decode_steps_in_slices(case):
     (width, ff), tokens, (rows, slices, groups) = case

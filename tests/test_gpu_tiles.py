@@ -120,6 +120,44 @@ def test_kquant_products_of_many_tokens(tmp_path, shape, tokens):
     assert np.linalg.norm(got[1] - got[0]) / norm < 1e-3, (shape, tokens)
 
 
+# (width, heads, kv heads, ff), tokens, whether v of another type goes with q and k
+TYPES_CASES = [
+    ((2048, 16, 4, 512), 65, True),         # four slices of K; a token past the narrow tiles
+    ((2048, 16, 4, 512), 256, True),        # whole tiles of tokens
+    ((2048, 16, 4, 512), 300, False),       # four slices of q and k, two with v
+    ((512, 4, 1, 768), 65, True),           # not split
+    ((512, 4, 1, 768), 129, True),
+    ((256, 44, 11, 256), 700, True),        # 55 + 11 row blocks by six of tokens
+    ((256, 80, 8, 256), 700, False),        # q and k on the 256-row tile
+]
+
+
+@pytest.mark.parametrize("arch", ["llama", "qwen2"])
+@pytest.mark.parametrize("swap", [False, True])
+@pytest.mark.parametrize("shape,tokens,rides", TYPES_CASES)
+def test_projections_of_two_types(tmp_path, monkeypatch, shape, tokens, rides, swap, arch):
+    """q and k of q4_K and v of q6_K, or the other way round, in one launch and in three, against the oracle."""
+    m = mesh()
+    cfg = dict(kquant(*shape), arch=arch, bias=arch == "qwen2")
+    path = str(tmp_path / "model.gguf")
+    if swap:
+        monkeypatch.setattr(models, "q4km_type", lambda name, *a: models.Q4_K if name == "attn_v" else models.Q6_K)
+    tensors = models.write_model(path, cfg, [0], seed=7, fast=True)
+    assert tensors["blk.0.attn_v.weight"][0] != tensors["blk.0.attn_q.weight"][0]
+    x = np.random.Generator(np.random.PCG64(tokens)).standard_normal((tokens, cfg["n_embd"])).astype(np.float32)
+    want = StageOracle(cfg, tensors, 0, 1, 768, blas=True).forward(x, np.arange(tokens))
+    st = m.Stage(path, 0, 1, n_ctx=768, n_batch_max=768, tuning={"tile_copies": 0})
+    got = []
+    for fused in (1, 0):
+        ses = st.session(gemm_fused=fused)
+        got.append(ses.decode(x, np.arange(tokens)).view(np.float32).reshape(want.shape))
+        ses.close()
+    st.close()
+    # the bounds of the products above: f16 inputs of four products; the same weights and inputs summed in another order
+    assert np.linalg.norm(got[0] - want) < 3e-3 * np.linalg.norm(want), np.linalg.norm(got[0] - want) / np.linalg.norm(want)
+    assert np.linalg.norm(got[0] - got[1]) < 1e-3 * np.linalg.norm(want)
+
+
 @pytest.mark.parametrize("n_embd,ff,tokens", [
     (256, 256, 17),         # one round of four steps along K; every expert in a tile of at most 32 pairs
     (512, 256, 65),
