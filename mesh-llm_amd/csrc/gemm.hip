@@ -1319,7 +1319,8 @@ static bool takes_big(const GemmArgs &a, int row_blocks, int slices) {
     return a.x_k8 && a.Wp && slices <= 1 && !a.rope.pos && row_blocks % 2 == 0 && a.big_tile && (row_blocks / 2) * ((a.T + GN - 1) / GN) >= gt_n_cu();
 }
 
-// Not where the others are cut along K otherwise without the last, whose rows would leave them fewer slices, nor where they take the 256-row tile.
+// Not where the last one's rows leave the others fewer slices of K, nor where they take the 256-row
+// tile or make more than two rounds over the CUs, beside which v is little.
 // q and k of q4_K, v of q6_K, apart / together, us: 4096 + 512 and 512 x 2048, 600 tokens 22.4 + 9.4 + 5.0 (the slices of v) / 26.0; eight layers of
 // the expert shard 70 tokens 1095 / 1043, 200 1325 / 1270, 600 1950 / 1902, 1300 3151 / 3099, 1700 3864 / 3865; eight 8B-shaped layers
 // without f16 copies 70 tokens 1041 / 999, 200 1601 / 1558, 900 4635 / 4564.
@@ -1330,7 +1331,7 @@ bool gemm_types_ride(const GemmArgs &a) {
     const int first = a.seg_begin[a.n_seg - 1], t_blocks = (a.T + GN - 1) / GN;
     int kps;
     const int slices = split_plan(a, first, t_blocks, &kps);
-    return !takes_big(a, first, slices) && split_plan(a, (a.M + GM - 1) / GM, t_blocks, &kps) == slices;
+    return first * t_blocks <= 2 * gt_n_cu() && !takes_big(a, first, slices) && split_plan(a, (a.M + GM - 1) / GM, t_blocks, &kps) == slices;
 }
 
 int gemm_kquant(const GemmArgs &a, hipStream_t stream) {
