@@ -1301,6 +1301,9 @@ static int split_plan(const GemmArgs &a, int row_blocks, int t_blocks, int *k_pe
     int ks = 1;
     while (ks < 16 && wgs * ks * 2 <= ncu && n_all / (ks * 2) >= 8 &&
            (size_t)(ks * 2) * a.T * row_blocks * GM * sizeof(float) <= a.part_bytes) ks *= 2;
+    // Any number where each keeps 1280 of K, as in gt_plan, us: two / three slices of 2048 x 4096 at 600 tokens (160 / 240 workgroups of 256 CUs) eight layers of
+    // the expert shard 1897 / 1876; four / six of 5120 rows, four 32B-shaped layers of 40 tokens 683 / 650, without f16 copies 100 940 / 880, 250 1580 / 1446.
+    for (int more = ks + 1, most = std::min({16, ncu / wgs, n_all / 20}); more <= most && (size_t)more * a.T * row_blocks * GM * sizeof(float) <= a.part_bytes; ++more) ks = more;
     if (ks <= 1) return 1;
     *k_per_split = (n_all + ks - 1) / ks;
     return (n_all + *k_per_split - 1) / *k_per_split;      // no empty slice
@@ -1319,7 +1322,7 @@ static bool takes_big(const GemmArgs &a, int row_blocks, int slices) {
     return a.x_k8 && a.Wp && slices <= 1 && !a.rope.pos && row_blocks % 2 == 0 && a.big_tile && (row_blocks / 2) * ((a.T + GN - 1) / GN) >= gt_n_cu();
 }
 
-// Not where the last one's rows leave the others fewer slices of K, nor where they take the 256-row
+// Not where the last one's rows leave the others half as many slices of K or fewer, nor where they take the 256-row
 // tile or make more than two rounds over the CUs, beside which v is little.
 // q and k of q4_K, v of q6_K, apart / together, us: 4096 + 512 and 512 x 2048, 600 tokens 22.4 + 9.4 + 5.0 (the slices of v) / 26.0; eight layers of
 // the expert shard 70 tokens 1095 / 1043, 200 1325 / 1270, 600 1950 / 1902, 1300 3151 / 3099, 1700 3864 / 3865; eight 8B-shaped layers
@@ -1331,7 +1334,7 @@ bool gemm_types_ride(const GemmArgs &a) {
     const int first = a.seg_begin[a.n_seg - 1], t_blocks = (a.T + GN - 1) / GN;
     int kps;
     const int slices = split_plan(a, first, t_blocks, &kps);
-    return first * t_blocks <= 2 * gt_n_cu() && !takes_big(a, first, slices) && split_plan(a, (a.M + GM - 1) / GM, t_blocks, &kps) == slices;
+    return first * t_blocks <= 2 * gt_n_cu() && !takes_big(a, first, slices) && 2 * split_plan(a, (a.M + GM - 1) / GM, t_blocks, &kps) > slices;
 }
 
 int gemm_kquant(const GemmArgs &a, hipStream_t stream) {

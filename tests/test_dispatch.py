@@ -95,6 +95,13 @@ def test_gate_up_of_a_decode_batch(case):
     assert not any(n.startswith("gemm_reg") for n, _ in other)
 
 
+@pytest.mark.parametrize("shape,tokens,slices", tiles.MANY_SLICES_CASES)
+def test_slices_in_any_number(shape, tokens, slices):
+    name, grid = call(kquant_products, cfg=tiles.kquant(*shape), layers=[0], tokens=tokens, tuning={"tile_copies": 0})[-1]
+    assert name.startswith("gemm_reg_kernel<%d," % Q6_K if tokens <= 64 else "gemm_kq_kernel<%d," % Q6_K), name
+    assert grid == [shape[0] // 128, -(-tokens // 128), slices]
+
+
 @pytest.mark.parametrize("shape,tokens,rides", tiles.TYPES_CASES)
 def test_projections_of_two_types(shape, tokens, rides):
     names = [n for n, _ in call(kquant_products, cfg=tiles.kquant(*shape), layers=[0], tokens=tokens, tuning={"tile_copies": 0})]

@@ -120,6 +120,34 @@ def test_kquant_products_of_many_tokens(tmp_path, shape, tokens):
     assert np.linalg.norm(got[1] - got[0]) / norm < 1e-3, (shape, tokens)
 
 
+# (width, heads, kv heads, ff), tokens, slices of the product down without copies
+MANY_SLICES_CASES = [
+    ((2816, 2, 1, 4096), 300, 3),           # slices of 22, 22 and 20 steps of 64 on the 128-row tile
+    ((5120, 2, 1, 7680), 40, 6),            # of 20 on the register-formed tile
+    ((5120, 2, 1, 7936), 64, 6),            # 21, the last of 19
+]
+
+
+@pytest.mark.parametrize("shape,tokens", [c[:2] for c in MANY_SLICES_CASES])
+def test_slices_in_any_number(tmp_path, shape, tokens):
+    m = mesh()
+    cfg = kquant(*shape)
+    path = str(tmp_path / "model.gguf")
+    tensors = models.write_model(path, cfg, [0], seed=7, fast=True)
+    x = np.random.Generator(np.random.PCG64(tokens)).standard_normal((tokens, cfg["n_embd"])).astype(np.float32)
+    want = StageOracle(cfg, tensors, 0, 1, 512, blas=True).forward(x, np.arange(tokens))
+    st = m.Stage(path, 0, 1, n_ctx=512, n_batch_max=512, tuning={"tile_copies": 0})
+    got = []
+    for split in (1, 0):
+        ses = st.session(gemm_splitk=split)
+        got.append(ses.decode(x, np.arange(tokens)).view(np.float32).reshape(want.shape))
+        ses.close()
+    st.close()
+    # (the bounds of the products above)
+    assert np.linalg.norm(got[0] - want) < 3e-3 * np.linalg.norm(want), np.linalg.norm(got[0] - want) / np.linalg.norm(want)
+    assert np.linalg.norm(got[0] - got[1]) < 1e-3 * np.linalg.norm(want)
+
+
 # (width, heads, kv heads, ff), tokens, whether v of another type goes with q and k
 TYPES_CASES = [
     ((2048, 16, 4, 512), 65, True),         # four slices of K; a token past the narrow tiles
