@@ -1322,19 +1322,20 @@ static bool takes_big(const GemmArgs &a, int row_blocks, int slices) {
     return a.x_k8 && a.Wp && slices <= 1 && !a.rope.pos && row_blocks % 2 == 0 && a.big_tile && (row_blocks / 2) * ((a.T + GN - 1) / GN) >= gt_n_cu();
 }
 
-// Not where the last one's rows leave the others half as many slices of K or fewer, nor where they take the 256-row
-// tile or make more than two rounds over the CUs, beside which v is little.
+// Where the others are not cut along K, or into no fewer slices than the last alone, whose sums then stay as they are; not where they would get
+// fewer by it, take the 256-row tile or make more than two rounds over the CUs, beside which v is little.
 // q and k of q4_K, v of q6_K, apart / together, us: 4096 + 512 and 512 x 2048, 600 tokens 22.4 + 9.4 + 5.0 (the slices of v) / 26.0; eight layers of
-// the expert shard 70 tokens 1095 / 1043, 200 1325 / 1270, 600 1950 / 1902, 1300 3151 / 3099, 1700 3864 / 3865; eight 8B-shaped layers
-// without f16 copies 70 tokens 1041 / 999, 200 1601 / 1558, 900 4635 / 4564.
+// the expert shard 70 tokens 1095 / 1043, 600 1950 / 1902, 1300 3151 / 3099, 1700 3864 / 3865; eight 8B-shaped layers
+// without f16 copies 70 tokens 1041 / 999, 900 4635 / 4564.
 bool gemm_types_ride(const GemmArgs &a) {
     if (!a.Wp || !a.Wp_last || !a.x_k8 || a.n_seg < 2 || a.y16_k8 || a.tiles || gemm_tile_takes(a)) return false;
     if (!((a.type == MESH_Q4_K && a.type_last == MESH_Q6_K) || (a.type == MESH_Q6_K && a.type_last == MESH_Q4_K))) return false;
     if (a.T <= GN / 2 && a.narrow_tile) return false;
     const int first = a.seg_begin[a.n_seg - 1], t_blocks = (a.T + GN - 1) / GN;
     int kps;
-    const int slices = split_plan(a, first, t_blocks, &kps);
-    return first * t_blocks <= 2 * gt_n_cu() && !takes_big(a, first, slices) && 2 * split_plan(a, (a.M + GM - 1) / GM, t_blocks, &kps) > slices;
+    const int slices = split_plan(a, first, t_blocks, &kps), all = (a.M + GM - 1) / GM;
+    if (first * t_blocks > 2 * gt_n_cu() || takes_big(a, first, slices)) return false;
+    return slices <= 1 || (split_plan(a, all, t_blocks, &kps) == slices && split_plan(a, all - first, t_blocks, &kps) <= slices);
 }
 
 int gemm_kquant(const GemmArgs &a, hipStream_t stream) {
