@@ -571,11 +571,15 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // KG groups of four waves, each over its own part of the k-steps; the partial products meet in LDS.
 // The k order of the sums is the 128-column tile's, within a group.
 // MODE: REG_DENSE, REG_SPLIT (raw sums of slice blockIdx.z to a.part), REG_EXPERT (one group), REG_NORM (a pair with a.norm_part).
-enum { REG_DENSE, REG_SPLIT, REG_EXPERT, REG_NORM };
+enum { REG_DENSE, REG_SPLIT, REG_EXPERT, REG_EXPERT_ROWS, REG_NORM };
 constexpr int reg_lds_bytes(int NT, int KG) { return KG * NT * 8192; }        // two buffers of activations per group; half the groups' sums
 template <int TYPE, int NT, int MODE, int KG>
 __device__ __forceinline__ void reg_tile(const GemmArgs &a, const uint8_t *wp, int bx, int t0, int t_end, int k0, int n_steps, u32x4 *lds) {
-    constexpr int AHEAD = 4, STEP = NT * 256;                  // chunks of weights on their way; 16-byte pieces of a chunk's activations
+    constexpr bool EXPERT = MODE == REG_EXPERT || MODE == REG_EXPERT_ROWS, ROWS = MODE == REG_EXPERT_ROWS;
+    // Activations of a chunk in LDS: [32 columns][16 of them][group of 8 of k][column], in 16-byte pieces.  A thread of ROWS brings a piece of a row, whose
+    // eight would lie 256 bytes apart, all on the same banks: there a group takes 17 places.
+    constexpr int K8 = ROWS ? 17 : 16, COLS = 16 * K8;
+    constexpr int AHEAD = 4, STEP = NT * COLS;                 // chunks of weights on their way; pieces of a chunk's activations
     const int tid = threadIdx.x & 255, lane = tid & 63, hh = lane >> 5, r = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), group = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
     const int n_all = a.K / GK;
@@ -587,13 +591,20 @@ __device__ __forceinline__ void reg_tile(const GemmArgs &a, const uint8_t *wp, i
     const unsigned slot = 2 * (pair ? 16 * wave + (r & 15) + (r >> 4) * 64 : 32 * wave + r) + hh;
     wp += ((size_t)bx * n_all + k0) * PackedSub<TYPE>::CHUNK;
     const int n_blk = (a.T + 15) >> 4;
-    const u32x4 *const xbase = reinterpret_cast<const u32x4 *>(a.X + (size_t)(t0 >> 4) * 16 * a.K) + (size_t)k0 * 128;
+    const u32x4 *const xbase = ROWS ? reinterpret_cast<const u32x4 *>(a.X) : reinterpret_cast<const u32x4 *>(a.X + (size_t)(t0 >> 4) * 16 * a.K) + (size_t)k0 * 128;
+    constexpr int X_CHUNK = ROWS ? 8 : 128;                    // pieces from a chunk's activations to the next one's
     unsigned xo[NT];                                           // 16-byte pieces from the tile's first block
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
-        const int b = 2 * i + (tid >> 7), last = n_blk - 1 - (t0 >> 4);        // (blocks past the list re-read the last one, never stored)
-        xo[i] = (unsigned)(b < last ? b : last) * (unsigned)(2 * a.K) + (unsigned)(tid & 127);
+        if constexpr (ROWS) {
+            const int s = t0 + 32 * i + (tid >> 3), of = a.x_slot[s < a.T ? s : a.T - 1];       // (slots past the tile's: any row, never stored)
+            xo[i] = (of > 0 ? (unsigned)of / (unsigned)a.x_div : 0u) * (unsigned)(a.K / 8) + (unsigned)(tid & 7);
+        } else {
+            const int b = 2 * i + (tid >> 7), last = n_blk - 1 - (t0 >> 4);        // (blocks past the list re-read the last one, never stored)
+            xo[i] = (unsigned)(b < last ? b : last) * (unsigned)(2 * a.K) + (unsigned)(tid & 127);
+        }
     }
+    const int put = ROWS ? (tid >> 7) * 8 * K8 + (tid & 7) * K8 + ((tid >> 3) & 15) : tid;
     u32x4 *xs = lds + group * 2 * STEP;
     float16v acc[NT];
 #pragma unroll
@@ -604,23 +615,23 @@ __device__ __forceinline__ void reg_tile(const GemmArgs &a, const uint8_t *wp, i
     if (n <= 0) { wp -= (size_t)k0 * PackedSub<TYPE>::CHUNK; }
     const u32x4 *const xb = n > 0 ? xbase : xbase - (size_t)k0 * 128;
     // (fewer on their way where more would cost a workgroup of a CU its registers)
-    constexpr int RING = MODE == REG_EXPERT && TYPE == MESH_Q6_K && NT > 2 ? 2 : AHEAD;
+    constexpr int RING = EXPERT && TYPE == MESH_Q6_K && NT > 2 ? 2 : AHEAD;
     PackedSub<TYPE> rw[RING];
     // Loads return in order: activations stored a step after they were asked for would have the weights asked for before them arrive
     // by then too, two chunks ahead instead of AHEAD.  Activations asked for XA steps before, against one: a batch of 32 decode steps of
     // four layers 5120 wide 821 -> 809 us, eight layers of a 40-token chunk 4096 wide 971 -> 953.  Two columns of tiles in a dense call with AHEAD spill (40 tokens: 995).
     constexpr int XA = NT == 1 ? AHEAD : NT > 2 ? 1 : 2;       // (the registers that are left at the occupancy)
     // Expert tiles: activations in groups of G chunks, 16 KB at most; a group is asked for while the one before it is multiplied.
-    constexpr int G = MODE == REG_EXPERT ? (NT > 2 ? 1 : 4 / NT) : 1, GROUP = 1024;
-    u32x4 rx[MODE == REG_EXPERT ? G * NT : XA * NT];
+    constexpr int G = EXPERT ? (NT > 2 ? 1 : 4 / NT) : 1, GROUP = 4 * COLS;
+    u32x4 rx[EXPERT ? G * NT : XA * NT];
     auto fetch = [&](int kc) {
 #pragma unroll
-        for (int i = 0; i < G * NT; ++i) rx[i] = (xb + (size_t)(kc + i / NT < last ? kc + i / NT : last) * 128)[xo[i % NT]];
+        for (int i = 0; i < G * NT; ++i) rx[i] = (xb + (size_t)(kc + i / NT < last ? kc + i / NT : last) * X_CHUNK)[xo[i % NT]];
     };
-    if constexpr (MODE == REG_EXPERT) {
+    if constexpr (EXPERT) {
         fetch(0);
 #pragma unroll
-        for (int i = 0; i < G * NT; ++i) xs[i * 256 + tid] = rx[i];
+        for (int i = 0; i < G * NT; ++i) xs[i * COLS + put] = rx[i];
         fetch(G);
     } else {
 #pragma unroll
@@ -632,10 +643,10 @@ __device__ __forceinline__ void reg_tile(const GemmArgs &a, const uint8_t *wp, i
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int u = 0; u < RING; ++u) rw[u].load(wp + (size_t)(MODE == REG_EXPERT || u < last ? u : last) * PackedSub<TYPE>::CHUNK, slot);
+    for (int u = 0; u < RING; ++u) rw[u].load(wp + (size_t)(EXPERT || u < last ? u : last) * PackedSub<TYPE>::CHUNK, slot);
     lds_barrier();
-    const int at = (lane & 15) + ((lane >> 4) & 1) * 128 + hh * 16;
-    if constexpr (MODE == REG_EXPERT) {
+    const int at = (lane & 15) + ((lane >> 4) & 1) * 8 * K8 + hh * K8;
+    if constexpr (EXPERT) {
         // A step's fragments are formed between the products of the step before, whose issue leaves the vector ALU idle, and its activations
         // read ahead of those.  The barrier of a group of chunks stands before its last step: behind it the next group's activations
         // have landed, whose first fragments that step reads, and the buffer they lie in has been read by everybody a group ago.
@@ -645,7 +656,7 @@ __device__ __forceinline__ void reg_tile(const GemmArgs &a, const uint8_t *wp, i
         const u32x4 *x = xs + at;
         int to_next = GROUP;
 #pragma unroll
-        for (int j = 0; j < NT; ++j) f[j] = x[j * 256];
+        for (int j = 0; j < NT; ++j) f[j] = x[j * COLS];
         for (int kc0 = 0; kc0 < per; kc0 += AHEAD) {
 #pragma unroll
             for (int u = 0; u < AHEAD; ++u) {
@@ -663,7 +674,7 @@ __device__ __forceinline__ void reg_tile(const GemmArgs &a, const uint8_t *wp, i
 #pragma unroll
                     for (int j = 0; j < NT; ++j) {
                         acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[st & 1], __builtin_bit_cast(half8, f[j]), acc[j], 0, 0, 0);
-                        f[j] = x[(turn ? 0 : st < 3 ? c * STEP + (st + 1) * 32 : (c + 1) * STEP) + j * 256];
+                        f[j] = x[(turn ? 0 : st < 3 ? c * STEP + (st + 1) * 2 * K8 : (c + 1) * STEP) + j * COLS];
                     }
 #pragma unroll
                     for (int j = 0; j < NT; ++j) {
@@ -674,9 +685,9 @@ __device__ __forceinline__ void reg_tile(const GemmArgs &a, const uint8_t *wp, i
                     __builtin_amdgcn_sched_barrier(0);
                     if (c == 0 && st == 0) {
                         // (the other buffer's last readers stand before the barrier of the group before)
-                        u32x4 *const nx = const_cast<u32x4 *>(x) - at + tid + to_next;
+                        u32x4 *const nx = const_cast<u32x4 *>(x) - at + put + to_next;
 #pragma unroll
-                        for (int i = 0; i < G * NT; ++i) nx[i * 256] = rx[i];
+                        for (int i = 0; i < G * NT; ++i) nx[i * COLS] = rx[i];
                         fetch(kc + 2 * G);
                     }
                     if (st == 2) rw[u % RING].load(wp + (size_t)(kc + RING < last ? kc + RING : last) * PackedSub<TYPE>::CHUNK, slot);
@@ -819,9 +830,12 @@ __device__ __forceinline__ void reg_tile(const GemmArgs &a, const uint8_t *wp, i
         }
     }
 }
-template <int TYPE>
+// REG_EXPERT_ROWS: a tile's activations straight from the rows the router has left, a token's 128 bytes of a chunk by eight lanes, where a launch before had to
+// sort copies of them: 600 tokens of 64 experts, top 8, gather 11.8 + gate / up 57 us before, 61 now (and the router 13 -> 14.4); eight expert
+// layers 40 tokens 972 -> 920 us, 200 1249 -> 1193, 600 1865 -> 1777, 2000 4375 -> 4112.
+template <int TYPE, int MODE>
 __global__ __launch_bounds__(256, 2) void gemm_expert_kernel(GemmArgs a) {
-    __shared__ u32x4 xs[2 * 4 * 256];
+    __shared__ u32x4 xs[2 * 4 * (MODE == REG_EXPERT_ROWS ? 272 : 256)];
     // workgroups go to the eight XCDs in turn: every row block of a tile on one of them, whose L2 fetches the tile's activations once
     // (gate / up as above: 66 us then, 82 with the row blocks dealt over the XCDs)
     const int g = (int)(blockIdx.y * gridDim.x + blockIdx.x), bx = (g >> 3) % (int)gridDim.x, nt = *a.n_tiles;
@@ -840,10 +854,10 @@ __global__ __launch_bounds__(256, 2) void gemm_expert_kernel(GemmArgs a) {
     const uint8_t *wp = static_cast<const uint8_t *>(a.Wp) + (size_t)tl.x * a.expert_stride;
     const int n = a.K / GK;
     switch ((tl.z + 31) >> 5) {
-        case 1: return reg_tile<TYPE, 1, REG_EXPERT, 1>(a, wp, bx, tl.y, tl.y + tl.z, 0, n, xs);
-        case 2: return reg_tile<TYPE, 2, REG_EXPERT, 1>(a, wp, bx, tl.y, tl.y + tl.z, 0, n, xs);
-        case 3: return reg_tile<TYPE, 3, REG_EXPERT, 1>(a, wp, bx, tl.y, tl.y + tl.z, 0, n, xs);
-        default: return reg_tile<TYPE, 4, REG_EXPERT, 1>(a, wp, bx, tl.y, tl.y + tl.z, 0, n, xs);
+        case 1: return reg_tile<TYPE, 1, MODE, 1>(a, wp, bx, tl.y, tl.y + tl.z, 0, n, xs);
+        case 2: return reg_tile<TYPE, 2, MODE, 1>(a, wp, bx, tl.y, tl.y + tl.z, 0, n, xs);
+        case 3: return reg_tile<TYPE, 3, MODE, 1>(a, wp, bx, tl.y, tl.y + tl.z, 0, n, xs);
+        default: return reg_tile<TYPE, 4, MODE, 1>(a, wp, bx, tl.y, tl.y + tl.z, 0, n, xs);
     }
 }
 // Dense calls of at most 64 tokens, at most 32 or 64 columns.  A launch of few workgroups per CU needs its waves from K: four groups
@@ -1368,8 +1382,11 @@ int gemm_kquant(const GemmArgs &a, hipStream_t stream) {
             return fail(MESH_ERR_INVALID, "gemm: an expert launch needs the GEMM layout, k8-major activations and a plain or SwiGLU epilogue");
         if (a.type != MESH_Q4_K && a.type != MESH_Q6_K) return fail(MESH_ERR_UNSUPPORTED, "gemm: no MFMA kernel for ggml type %d", a.type);
         const dim3 g((unsigned)row_blocks, (unsigned)((a.max_tiles + 7) / 8 * 8));       // (the kernel deals them to the XCDs in eights)
-        if (a.type == MESH_Q4_K) MESH_LAUNCH(gemm_expert_kernel<MESH_Q4_K>, g, dim3(256), 0, stream, k);
-        else MESH_LAUNCH(gemm_expert_kernel<MESH_Q6_K>, g, dim3(256), 0, stream, k);
+        if (a.x_slot && a.x_div < 1) return fail(MESH_ERR_INVALID, "gemm: rows of an expert launch without their divisor");
+        if (a.x_slot && a.type == MESH_Q4_K) MESH_LAUNCH((gemm_expert_kernel<MESH_Q4_K, REG_EXPERT_ROWS>), g, dim3(256), 0, stream, k);
+        else if (a.x_slot) MESH_LAUNCH((gemm_expert_kernel<MESH_Q6_K, REG_EXPERT_ROWS>), g, dim3(256), 0, stream, k);
+        else if (a.type == MESH_Q4_K) MESH_LAUNCH((gemm_expert_kernel<MESH_Q4_K, REG_EXPERT>), g, dim3(256), 0, stream, k);
+        else MESH_LAUNCH((gemm_expert_kernel<MESH_Q6_K, REG_EXPERT>), g, dim3(256), 0, stream, k);
         MESH_LAUNCH_CHECK();
         return MESH_OK;
     }

@@ -62,6 +62,9 @@ struct GemmArgs {
     // matrix at Wp + expert * expert_stride.  *n_tiles (device) tiles are live, max_tiles bounds them for the grid.
     // Outputs are indexed by slot.
     const int32_t *tiles = nullptr, *n_tiles = nullptr;
+    // x_slot set: X holds plain rows of K, not sorted, and slot s's is row x_slot[s] / x_div (a slot without a pair, < 0, may take any).
+    const int32_t *x_slot = nullptr;
+    int x_div = 0;
     size_t expert_stride = 0;
     int max_tiles = 0;
     // SwiGLU pair of a call of at most 32 tokens, x_k8: the consumer side of SkinnyF16Args' norm hand-over (X not yet divided by the

@@ -186,7 +186,8 @@ constexpr int CHUNK_WAVES = 8;
 template <int NV, int TOKENS>
 __global__ __launch_bounds__(64 * CHUNK_WAVES) void moe_router_chunk_kernel(const float *__restrict__ x, const float *__restrict__ norm_w,
                                                                       const float *__restrict__ W, float *__restrict__ logits_out,
-                                                                      int ldx, float eps, int T, const MoeRouteArgs a, float *__restrict__ scale_out) {
+                                                                      int ldx, float eps, int T, const MoeRouteArgs a, float *__restrict__ scale_out,
+                                                                      _Float16 *__restrict__ rows_out, unsigned *sat) {
     constexpr int E = NV * 256;
     __shared__ float s_logits[TOKENS][64 * ROUTE_MAX_PER_LANE];
     const int t0 = blockIdx.x * TOKENS, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -220,6 +221,23 @@ __global__ __launch_bounds__(64 * CHUNK_WAVES) void moe_router_chunk_kernel(cons
             xr[k][i].z = xr[k][i].z * scale * nw[i].z; xr[k][i].w = xr[k][i].w * scale * nw[i].w;
         }
     }
+    // (a wave a token; the stores are on their way while the experts' rows go by)
+    if (rows_out)
+#pragma unroll
+        for (int k = 0; k < TOKENS; ++k)
+            if (wave == k && t0 + k < T)
+#pragma unroll
+                for (int i = 0; i < NV; ++i) {
+                    const float4 v = xr[k][i];
+                    if (sat) {
+                        const unsigned clamped = (fmaxf(fabsf(v.x), fabsf(v.y)) > 65504.f ? 1u : 0u) + (fmaxf(fabsf(v.z), fabsf(v.w)) > 65504.f ? 1u : 0u);
+                        if (clamped) atomicAdd(sat, clamped * (unsigned)a.top_k);
+                    }
+                    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+                    const h4 h = {(_Float16)__builtin_amdgcn_fmed3f(v.x, -65504.f, 65504.f), (_Float16)__builtin_amdgcn_fmed3f(v.y, -65504.f, 65504.f),
+                                  (_Float16)__builtin_amdgcn_fmed3f(v.z, -65504.f, 65504.f), (_Float16)__builtin_amdgcn_fmed3f(v.w, -65504.f, 65504.f)};
+                    *reinterpret_cast<h4 *>(rows_out + (size_t)(t0 + k) * E + 4 * (lane + 64 * i)) = h;
+                }
     for (int e0 = wave; e0 < a.n_expert; e0 += 2 * CHUNK_WAVES) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
@@ -256,12 +274,12 @@ __global__ __launch_bounds__(64 * CHUNK_WAVES) void moe_router_chunk_kernel(cons
 }
 template <int TOKENS>
 static void launch_router_chunk(const MoeRouteArgs &a, const float *x, int ldx, const float *norm_w, float eps, const float *W, int E, float *logits_out, int T, hipStream_t stream,
-                                float *scale_out) {
+                                float *scale_out, _Float16 *rows_out, unsigned *sat) {
     const dim3 grid((unsigned)((T + TOKENS - 1) / TOKENS)), block(64 * CHUNK_WAVES);
     switch (E / 256) {
-        case 2: MESH_LAUNCH((moe_router_chunk_kernel<2, TOKENS>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, T, a, scale_out); break;
-        case 4: MESH_LAUNCH((moe_router_chunk_kernel<4, TOKENS>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, T, a, scale_out); break;
-        default: MESH_LAUNCH((moe_router_chunk_kernel<8, TOKENS>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, T, a, scale_out); break;
+        case 2: MESH_LAUNCH((moe_router_chunk_kernel<2, TOKENS>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, T, a, scale_out, rows_out, sat); break;
+        case 4: MESH_LAUNCH((moe_router_chunk_kernel<4, TOKENS>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, T, a, scale_out, rows_out, sat); break;
+        default: MESH_LAUNCH((moe_router_chunk_kernel<8, TOKENS>), grid, block, 0, stream, x, norm_w, W, logits_out, ldx, eps, T, a, scale_out, rows_out, sat); break;
     }
 }
 
@@ -329,8 +347,12 @@ __global__ __launch_bounds__(SLICE_THREADS) void moe_router_slice_kernel(const f
     if (lane == 0 && e < n_expert) logits[(size_t)t * n_expert + e] = acc;
 }
 
+bool moe_router_writes_rows(int E, int n_expert, int T) {
+    return E <= 2048 && !(T <= 256 && E <= 1024 && n_expert >= 96);
+}
+
 int moe_router_fused(const MoeRouteArgs &a, const float *x, int ldx, const float *norm_w, float eps, const float *W, int E,
-                     float *logits_out, int T, hipStream_t stream, float *scale_out) {
+                     float *logits_out, int T, hipStream_t stream, float *scale_out, uint16_t *rows_out, unsigned *sat) {
     if (T <= 0) return MESH_OK;
     if (!moe_router_fused_supported(E, a.n_expert, a.top_k)) return fail(MESH_ERR_UNSUPPORTED, "moe: fused router for hidden size %d / %d experts", E, a.n_expert);
     const dim3 grid((unsigned)T);
@@ -338,11 +360,13 @@ int moe_router_fused(const MoeRouteArgs &a, const float *x, int ldx, const float
     // workgroup of eight waves / one a workgroup of sixteen, 200 tokens: E 512 with 96 experts 9.1 / 7.4, 128 10.0 / 8.4, 256 18.6 / 15.0,
     // 512 29.9 / 21.0; E 1024 with 96 10.0 / 9.0, 128 11.8 / 10.3, 256 20.8 / 18.3, 512 34.5 / 28.6; E 2048 with 64 9.9 / 17.9, 512 53 / 112
     // (those two with sums through the LDS unit).  300 tokens, E 512, 512 experts: 29.4 / 33.
-    const bool short_rows = T <= 256 && E <= 1024 && a.n_expert >= 96;
-    if (E <= 2048 && !short_rows) {
-        if (T <= 2 * 256) launch_router_chunk<2>(a, x, ldx, norm_w, eps, W, E, logits_out, T, stream, scale_out);
-        else if (T <= 3 * 256) launch_router_chunk<3>(a, x, ldx, norm_w, eps, W, E, logits_out, T, stream, scale_out);
-        else launch_router_chunk<4>(a, x, ldx, norm_w, eps, W, E, logits_out, T, stream, scale_out);
+    const bool chunk = moe_router_writes_rows(E, a.n_expert, T);
+    if (rows_out && !chunk) return fail(MESH_ERR_UNSUPPORTED, "moe: rows of a router that writes none");
+    if (chunk) {
+        _Float16 *const rows = reinterpret_cast<_Float16 *>(rows_out);
+        if (T <= 2 * 256) launch_router_chunk<2>(a, x, ldx, norm_w, eps, W, E, logits_out, T, stream, scale_out, rows, sat);
+        else if (T <= 3 * 256) launch_router_chunk<3>(a, x, ldx, norm_w, eps, W, E, logits_out, T, stream, scale_out, rows, sat);
+        else launch_router_chunk<4>(a, x, ldx, norm_w, eps, W, E, logits_out, T, stream, scale_out, rows, sat);
         MESH_LAUNCH_CHECK();
         return MESH_OK;
     }

@@ -19,8 +19,11 @@ int moe_route(const MoeRouteArgs &a, int T, hipStream_t stream);
 // Router mat-vec (f32 matrix W [n_expert][E] over the RMS-normalised hidden state) and routing in one launch; a.logits is
 // not read, logits_out (optional) receives [T][n_expert], scale_out (optional) [T]: 1 / rms of the hidden state.
 bool moe_router_fused_supported(int E, int n_expert, int top_k);
+// rows_out (optional, where moe_router_writes_rows says so): the normalised hidden states [T][E], f16, of which those past its range count
+// top_k times in sat, as they would in top_k copies.
+bool moe_router_writes_rows(int E, int n_expert, int T);
 int moe_router_fused(const MoeRouteArgs &a, const float *x, int ldx, const float *norm_w, float eps, const float *W, int E,
-                     float *logits_out, int T, hipStream_t stream, float *scale_out = nullptr);
+                     float *logits_out, int T, hipStream_t stream, float *scale_out = nullptr, uint16_t *rows_out = nullptr, unsigned *sat = nullptr);
 // Groups the n_pairs (token, slot) pairs of ids by expert into work items for the expert launches: moe_item_ints(item_pairs)
 // int32 per item = {expert, n, pair[0..n)}, n <= item_pairs pairs of that expert, in ascending pair order; experts in
 // ascending order (gemv.hpp; item_pairs = MOE_ITEM_PAIRS for the mat-vec kernel, SKINNY_ITEM_PAIRS for the matrix-core

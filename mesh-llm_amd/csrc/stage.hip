@@ -1163,10 +1163,13 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
                              s->tune.moe_gemm && E % 256 == 0 && ffe % 256 == 0;
             if (big) {
                 const float *scale = nullptr;
-                if (L.gate_inp.type == MESH_F32 && moe_router_fused_supported(E, ne, k)) {
+                const bool fused = L.gate_inp.type == MESH_F32 && moe_router_fused_supported(E, ne, k);
+                // the router leaves the normalised rows, and the expert launch reads a slot's through the pair it holds: no gather
+                const bool rows = fused && moe_router_writes_rows(E, ne, T);
+                if (fused) {
                     ProfScope ps(s, MESH_PROF_GEMV);
                     if ((rc = moe_router_fused(mr, s->x, E, static_cast<const float *>(L.ffn_norm.data), hp.rms_eps,
-                                               static_cast<const float *>(L.gate_inp.data), E, s->moe_logits, T, stream, s->moe_scale)) != MESH_OK) return rc;
+                                               static_cast<const float *>(L.gate_inp.data), E, s->moe_logits, T, stream, s->moe_scale, rows ? s->moe_x16 : nullptr, s->f16_sat)) != MESH_OK) return rc;
                     scale = s->moe_scale;           // (the router has normalised the rows: the gather need not add their squares again)
                 } else {
                     GemvArgs ra2;
@@ -1182,13 +1185,14 @@ static int run_layers(mesh_session *s, int T, int max_keys) {
                 {
                     ProfScope ps(s, MESH_PROF_PREP);
                     if ((rc = moe_sort(s->moe_ids, T * k, ne, s->moe_sorted, stream)) != MESH_OK) return rc;
-                    if ((rc = rmsnorm_f16_k8_gather(s->x, static_cast<const float *>(L.ffn_norm.data), hp.rms_eps, s->moe_sorted.pair_of_slot, k, slots, E,
+                    if (!rows && (rc = rmsnorm_f16_k8_gather(s->x, static_cast<const float *>(L.ffn_norm.data), hp.rms_eps, s->moe_sorted.pair_of_slot, k, slots, E,
                                                     reinterpret_cast<_Float16 *>(s->moe_x16), stream, s->f16_sat, scale)) != MESH_OK) return rc;
                 }
                 GemmArgs g;
                 g.W = L.gate_exps.data; g.Wp = L.exps_gate_up_gemm; g.type = L.gate_exps.type;
                 g.M = ffe; g.K = E; g.T = slots;
                 g.X = reinterpret_cast<const _Float16 *>(s->moe_x16); g.ldx = E; g.x_k8 = true;
+                if (rows) { g.x_slot = s->moe_sorted.pair_of_slot; g.x_div = k; }
                 g.y16_k8 = reinterpret_cast<_Float16 *>(s->moe_ffn16);
                 g.sat = s->f16_sat;
                 g.tiles = s->moe_sorted.tiles; g.n_tiles = s->moe_sorted.counts; g.max_tiles = max_tiles; g.expert_stride = L.exps_gate_up_stride;

@@ -244,6 +244,76 @@ def test_router_of_a_chunk_over_tokens_a_workgroup(tmp_path, n_embd, tokens):
     assert np.linalg.norm((got - want)[same]) / np.linalg.norm(want[same]) < 3e-3
 
 
+# width, experts, tokens, whether gate and up are of q6_K; whether the expert launch reads the router's rows by its slots, not a gathered copy
+EXPERT_ROWS_CASES = [
+    (512, 24, 33, False, True),
+    (1024, 24, 130, True, True),            # a large expert: a tile of 128 pairs and one behind it
+    (2048, 40, 301, False, True),
+    (2048, 40, 77, True, True),
+    (512, 120, 200, False, False),          # many short expert rows: their router writes none
+    (512, 120, 257, False, True),
+    (4096, 24, 33, False, False),
+    (256, 24, 33, False, False),
+]
+
+
+def expert_config(n_embd, n_expert, n_layer=1):
+    return dict(arch="qwen3moe", n_layer=n_layer, n_embd=n_embd, n_head=4, n_head_kv=2, head_dim=128, n_ff=0, n_vocab=256, eps=1e-6, rope=1e6,
+                n_expert=n_expert, n_expert_used=3, n_ff_exp=256, qk_norm=True)
+
+
+@pytest.mark.parametrize("n_embd,n_expert,tokens,q6,rows", EXPERT_ROWS_CASES)
+def test_expert_products_over_rows_by_slot(tmp_path, monkeypatch, n_embd, n_expert, tokens, q6, rows):
+    m = mesh()
+    cfg = expert_config(n_embd, n_expert)
+    path = str(tmp_path / "model.gguf")
+    if q6:
+        plain = models.q4km_type
+        monkeypatch.setattr(models, "q4km_type", lambda name, *a: models.Q6_K if name in ("ffn_gate_exps", "ffn_up_exps") else plain(name, *a))
+    tensors = models.write_model(path, cfg, [0], seed=6, router="zipf", fast=True)
+    assert tensors["blk.0.ffn_gate_exps.weight"][0] == (models.Q6_K if q6 else models.Q4_K)
+    x = models.zipf_hidden_state(np.random.Generator(np.random.PCG64(tokens)), tokens, n_embd)
+    orc = StageOracle(cfg, tensors, 0, 1, 512, blas=True)
+    want = orc.forward(x, np.arange(tokens)) - x
+    st = m.Stage(path, 0, 1, n_ctx=512, n_batch_max=512)
+    ses = st.session(moe_gemm_min_pairs=1)
+    for _ in range(2):                      # (rows and slots of another routing lie in the buffers the second time)
+        got = ses.decode(x, np.arange(tokens)).view(np.float32).reshape(want.shape) - x
+        same = (np.sort(ses.moe_last_ids(tokens), axis=1) == np.sort(np.stack(orc.last_expert_ids), axis=1)).all(axis=1)
+        assert same.mean() > 0.97           # (near ties, as above)
+        # f16 activations: 11 bits in the inputs of the layer's products
+        assert np.linalg.norm((got - want)[same]) / np.linalg.norm(want[same]) < 3e-3
+        ses.decode(np.ascontiguousarray(x[::-1]), np.arange(tokens))
+    assert ses.f16_saturations() == 0
+    ses.close()
+    st.close()
+
+
+def test_clamped_rows_count_once_a_slot(tmp_path):
+    """Values past the range of f16 in the normalised rows: counted by pairs of neighbours, for every expert of the token."""
+    m = mesh()
+    n_embd, tokens = 512, 40
+    cfg = expert_config(n_embd, 24)
+    path = str(tmp_path / "model.gguf")
+    kvs, tensors = models.build_tensors(cfg, [0], seed=6, fast=True)
+    g = np.ones(n_embd, np.float32)
+    g[[6, 7, 100, 301]] = 1e5
+    blank = ("ffn_gate_exps", "ffn_up_exps", "ffn_down_exps", "attn_output")       # (nothing else that could be clamped, and rows as they come in)
+    tensors = [(n, t, d, g.view(np.uint8) if "ffn_norm" in n else np.zeros_like(data) if any(b in n for b in blank) else data) for n, t, d, data in tensors]
+    models.G.write_gguf(path, kvs, tensors)
+    x = np.random.Generator(np.random.PCG64(3)).standard_normal((tokens, n_embd)).astype(np.float32)
+    y = x * (1 / np.sqrt((x.astype(np.float64) ** 2).mean(axis=1, keepdims=True) + 1e-6)) * g
+    assert np.abs(np.abs(y) / 65504 - 1).min() > 1e-4
+    pairs = int((np.abs(y) > 65504).reshape(tokens, -1, 2).any(axis=2).sum())
+    assert pairs
+    st = m.Stage(path, 0, 1, n_ctx=512, n_batch_max=512)
+    ses = st.session(moe_gemm_min_pairs=1)
+    ses.decode(x, np.arange(tokens))
+    assert ses.f16_saturations() == pairs * cfg["n_expert_used"]
+    ses.close()
+    st.close()
+
+
 #   shape as above, tokens, (32-column groups, groups of waves, slices) of gate/up and down
 KQUANT_FEW_CASES = [
     ((256, 2, 1, 256), 17, (1, 4, 1), (1, 4, 1)),       # four steps along K: one for each group of waves; padding columns
