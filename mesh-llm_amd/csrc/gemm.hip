@@ -571,7 +571,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // KG groups of four waves, each over its own part of the k-steps; the partial products meet in LDS.
 // The k order of the sums is the 128-column tile's, within a group.
 // MODE: REG_DENSE, REG_SPLIT (raw sums of slice blockIdx.z to a.part), REG_EXPERT (one group), REG_NORM (a pair with a.norm_part).
-enum { REG_DENSE, REG_SPLIT, REG_EXPERT, REG_EXPERT_ROWS, REG_NORM };
+enum { REG_DENSE, REG_SPLIT, REG_EXPERT, REG_NORM, REG_EXPERT_ROWS };
 constexpr int reg_lds_bytes(int NT, int KG) { return KG * NT * 8192; }        // two buffers of activations per group; half the groups' sums
 template <int TYPE, int NT, int MODE, int KG>
 __device__ __forceinline__ void reg_tile(const GemmArgs &a, const uint8_t *wp, int bx, int t0, int t_end, int k0, int n_steps, u32x4 *lds) {

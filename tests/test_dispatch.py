@@ -98,7 +98,7 @@ def test_gate_up_of_a_decode_batch(case):
 @pytest.mark.parametrize("n_embd,n_expert,tokens,q6,rows", tiles.EXPERT_ROWS_CASES)
 def test_expert_products_over_rows_by_slot(n_embd, n_expert, tokens, q6, rows):
     names = [n for n, _ in call(kquant_products, cfg=tiles.expert_config(n_embd, n_expert), layers=[0], tokens=tokens, options={"moe_gemm_min_pairs": 1})]
-    assert [n for n in names if n.startswith("gemm_expert")] == ["gemm_expert_kernel<%d,%d>" % (Q4_K, 3 if rows else 2), "gemm_expert_kernel<%d,2>" % Q6_K], names
+    assert [n for n in names if n.startswith("gemm_expert")] == ["gemm_expert_kernel<%d,%d>" % (Q4_K, 4 if rows else 2), "gemm_expert_kernel<%d,2>" % Q6_K], names
 
 
 @pytest.mark.parametrize("shape,tokens,slices", tiles.MANY_SLICES_CASES)
