@@ -535,16 +535,25 @@ static size_t gla_prepare_lds(int dim, int rank) { return ((size_t)C * (3 * (gs_
 
 // grid (heads, 16-column slices of the values, sequences of the call).  Wave w < 4 owns rows [16 NT w, 16 NT (w + 1)) of the state; waves 4
 // and 5 write a chunk's outputs, a row tile each, beside the next chunk's products (in waves 0 and 1 they made the other two wait 700 cycles).
-// PIPED: a chunk is worked on while the next ones travel, which takes the registers of one workgroup a CU; without, as many of them as fit
-// hide each other's waits (launch_scan).
+// SCAN_PIPED: a chunk is worked on while the next ones travel, which takes the registers of one workgroup a CU; SCAN_PLAIN: as many of them as
+// fit hide each other's waits (launch_scan).
+// SCAN_SHORT: waves 0 and 1 write the outputs, and a CU holds half as many workgroups again and more.  Many sequences of few chunks, us,
+// delta rule / without: with four waves and operands as rows, which waves 4 and 5 came after / SCAN_PLAIN / so:
+//   16 heads of 128 x 128, 60 sequences of 8 tokens  75.6  61.0   73.4  54.7   49.6  35.8     16 of 96   52.9  40.8   48.7  37.2   38.9  29.2
+//   16 heads of 160 x 128, 60 of 8                  107.8  79.0  124.9  80.1   76.4  50.3     32 of 40  106.9  70.9  111.0  67.0   76.3  51.4
+//   16 heads of 256 x 256, 60 of 8                    335   211    316   237    194   140     16 of 96    219   147    206   135    137    97
+//   4 heads of 192 x 192, 32 of 32                   26.0  22.9   29.1  20.9   19.8  15.5     16 of 96   31.2  24.7   32.7  20.2   24.1  18.5
+// and of many: 32 heads of 64 x 64, four of 300 28.5 / 24.4, 20.5 / 16.6, 27.7 / 18.2.
 // What bounds it, a chunk of 128 x 128 (16 heads, one sequence, cycles of 3300 with the delta rule, 2400 without): 48 and 32 matrix
 // instructions a wave at 32.5 cycles, 72 and 56 KB that a CU takes at 64 bytes a cycle and less, and the waits where they meet.  29 chunks x 16 heads,
 // us, delta rule / without: rows as they lie, outputs in waves 0 and 1: 70.6 / 63.3; no branch around a load 64.2 / 44.3; operands as
 // kilobytes, outputs in waves of their own, a barrier that leaves loads in flight 44.0 / 32.7; loads between the products 43.2 / 30.7.  Q S
 // behind the barrier, while the sums over the waves travel: 44.2 / 31.9.
-constexpr int SCAN_THREADS = 384;
-template <bool DELTA, int NT, bool PIPED>
-__global__ __launch_bounds__(SCAN_THREADS) void state_scan_kernel(const GatedStateArgs a) {
+enum { SCAN_PLAIN, SCAN_PIPED, SCAN_SHORT };
+constexpr int scan_threads(int mode) { return mode == SCAN_SHORT ? 256 : 384; }
+template <bool DELTA, int NT, int MODE>
+__global__ __launch_bounds__(scan_threads(MODE)) void state_scan_kernel(const GatedStateArgs a) {
+    constexpr bool PIPED = MODE == SCAN_PIPED, SHORT = MODE == SCAN_SHORT;
     constexpr int Dp = 64 * NT;
     __shared__ __align__(16) float red[2][4][DELTA ? 4 : 2][64][4];        // by chunk parity, wave: partial W S and Q S of the two row tiles
     const int h = blockIdx.x, vt = blockIdx.y, run = blockIdx.z;
@@ -563,9 +572,26 @@ __global__ __launch_bounds__(SCAN_THREADS) void state_scan_kernel(const GatedSta
                     for (int w = 0; w < 4; ++w) u[r] -= *reinterpret_cast<const gs_f4 *>(rd[w][2 + r][lane]);
         }
     };
-    if (wave >= 4) {
+    // outputs of row tile rt of a chunk: Q S over the waves, and its rows of A by its u
+    struct Out { gs_f4 a[2], u[2]; };
+    auto over_waves = [&](int ci, int rt) {
+        float (*rd)[DELTA ? 4 : 2][64][4] = red[(ci - c0) & 1];
+        gs_f4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < 4; ++w) o += *reinterpret_cast<const gs_f4 *>(rd[w][rt][lane]);
+        return o;
+    };
+    auto put = [&](int ci, int rt, const Out &f, gs_f4 o, int t_end) {
+        o = gs_mma(f.a[0], f.u[0], o);
+        if (rt == 1) o = gs_mma(f.a[1], f.u[1], o);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int t = t_first + (ci - c0) * C + 16 * rt + 4 * g + i;
+            if (t < t_end && col < V) a.o[(size_t)t * a.heads * V + h * V + col] = o[i];
+        }
+    };
+    if (!SHORT && wave >= 4) {
         const int rt = wave - 4, t_end = a.chunks.chunk[c1];
-        struct Out { gs_f4 a[2], u[2]; };
         auto load = [&](int ci, Out &f) {
             if (ci >= c1) ci = c1 - 1;
             const GsMats m(a.ws, (size_t)ci * a.heads + h, Dp, Vp, DELTA);
@@ -577,18 +603,9 @@ __global__ __launch_bounds__(SCAN_THREADS) void state_scan_kernel(const GatedSta
         };
         auto step = [&](int ci, Out &f) {
             lds_barrier();
-            float (*rd)[DELTA ? 4 : 2][64][4] = red[(ci - c0) & 1];
-            gs_f4 o = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int w = 0; w < 4; ++w) o += *reinterpret_cast<const gs_f4 *>(rd[w][rt][lane]);
+            const gs_f4 o = over_waves(ci, rt);
             settle(ci, f.u, 1 + rt);
-            o = gs_mma(f.a[0], f.u[0], o);
-            if (rt == 1) o = gs_mma(f.a[1], f.u[1], o);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int t = t_first + (ci - c0) * C + 16 * rt + 4 * g + i;
-                if (t < t_end && col < V) a.o[(size_t)t * a.heads * V + h * V + col] = o[i];
-            }
+            put(ci, rt, f, o, t_end);
         };
         Out f0, f1;
         load(c0, f0);
@@ -646,6 +663,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void state_scan_kernel(const GatedSta
         load_right(m, f);
     };
     // chunk ci, and the loads of chunk `ahead` beside it
+    gs_f4 u[2];
     auto step = [&](int ci, const Frag &cur, int ahead, Frag *next) {
         float (*rd)[DELTA ? 4 : 2][64][4] = red[(ci - c0) & 1];
         const GsMats m = mats(ahead);
@@ -678,7 +696,8 @@ __global__ __launch_bounds__(SCAN_THREADS) void state_scan_kernel(const GatedSta
         }
         // one barrier a chunk: the buffer of this parity is written again two chunks on, behind the next chunk's barrier
         lds_barrier();
-        gs_f4 u[2] = {cur.u[0], cur.u[1]};
+        u[0] = cur.u[0];
+        u[1] = cur.u[1];
         settle(ci, u, 2);
         if constexpr (PIPED) {
             __builtin_amdgcn_sched_barrier(0);
@@ -700,9 +719,23 @@ __global__ __launch_bounds__(SCAN_THREADS) void state_scan_kernel(const GatedSta
         }
     };
     Frag f0;
-    if constexpr (!PIPED) {
+    if constexpr (SHORT) {
+        const int t_end = a.chunks.chunk[c1];
+        int ci = c0;
+        do {
+            Out f;
+            const GsMats m = mats(ci);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) f.a[s] = *reinterpret_cast<const gs_f4 *>(m.A + gs_tile(wave & 1, s, lane));
+            load(ci, f0);
+            step(ci, f0, ci, nullptr);
+            f.u[0] = u[0];
+            f.u[1] = u[1];
+            if (wave < 2) put(ci, wave, f, over_waves(ci, wave), t_end);
+        } while (++ci < c1);
+    } else if constexpr (!PIPED) {
         for (int ci = c0; ci < c1; ++ci) { load(ci, f0); step(ci, f0, ci, nullptr); }
-    } else if constexpr (NT < 3) {          // (two chunks ahead, as many as the registers hold)
+    } else if constexpr (NT < 3) {          // (two chunks ahead, as many as the registers hold: 16 heads of 160 x 128, 900 tokens, one / two ahead 55 / 90 us, which spill)
         Frag f1, f2;
         load(c0, f0);
         load(c0 + 1, f1);
@@ -797,27 +830,35 @@ int gated_state_step(const GatedStateArgs &a, int T, hipStream_t stream) {
     return MESH_OK;
 }
 
-template <bool DELTA, bool PIPED>
+template <bool DELTA, int MODE>
 static int launch_scan_of(const GatedStateArgs &a, hipStream_t stream) {
-    const dim3 grid((unsigned)a.heads, (unsigned)(gs_pad16(a.vdim) / 16), (unsigned)a.chunks.n_runs), block(SCAN_THREADS);
+    const dim3 grid((unsigned)a.heads, (unsigned)(gs_pad16(a.vdim) / 16), (unsigned)a.chunks.n_runs), block(scan_threads(MODE));
     switch (gs_pad64(a.dim) / 64) {
-        case 1: MESH_LAUNCH((state_scan_kernel<DELTA, 1, PIPED>), grid, block, 0, stream, a); break;
-        case 2: MESH_LAUNCH((state_scan_kernel<DELTA, 2, PIPED>), grid, block, 0, stream, a); break;
-        case 3: MESH_LAUNCH((state_scan_kernel<DELTA, 3, PIPED>), grid, block, 0, stream, a); break;
-        default: MESH_LAUNCH((state_scan_kernel<DELTA, 4, PIPED>), grid, block, 0, stream, a); break;
+        case 1: MESH_LAUNCH((state_scan_kernel<DELTA, 1, MODE>), grid, block, 0, stream, a); break;
+        case 2: MESH_LAUNCH((state_scan_kernel<DELTA, 2, MODE>), grid, block, 0, stream, a); break;
+        case 3: MESH_LAUNCH((state_scan_kernel<DELTA, 3, MODE>), grid, block, 0, stream, a); break;
+        default: MESH_LAUNCH((state_scan_kernel<DELTA, 4, MODE>), grid, block, 0, stream, a); break;
     }
     MESH_LAUNCH_CHECK();
     return MESH_OK;
 }
 
-// Pipelined where a CU has one workgroup at most and a sequence more than one chunk.  Layers of 16 heads of 128 x 128, us of a call of six
-// layers, two of them scans, pipelined / not (a sequence makes 128 workgroups): one sequence of 900 tokens 1417 / 1464, of 300 870 / 878, two
-// of 300 1520 / 1528; four of 300 2276 / 2252, 16 of 96 2774 / 2674, 32 of 32 1979 / 1830, 60 of 8 and four of 40 2094 / 1787.
-constexpr int SCAN_PIPED_WORKGROUPS_MAX = 256;
+// Pipelined where a CU has one workgroup at most and a sequence more than one chunk.  us of a scan with the delta rule / without, pipelined and
+// not: 16 heads of 128 x 128 (a sequence makes 128 workgroups), one sequence of 900 tokens 43.7 / 31.0 and 59.0 / 43.8, two of 300 19.4 / 14.4 and
+// 24.2 / 18.6, four of 300 36.2 / 26.5 and 32.9 / 25.7, 16 of 96 55.4 / 42.0 and 49.0 / 36.8; of 64 x 64, four of 300 (256 workgroups) 14.3 / 10.9
+// and 16.6 / 11.8, 16 of 96 21.3 / 15.5 and 16.2 / 12.1.  States of more than 128 rows would gain beyond the line too (of 160 x 128, four of 300
+// 44.3 / 31.3 and 60.4 / 33.0; of 256 x 256 107 / 76 and 141 / 112), which no rule takes yet.
+// From more than two a CU on, sequences of up to three chunks take four waves instead of six (above; two a CU, 16 heads of 128 x 128, four of 20
+// tokens, 8.1 / 5.6 against 7.0 / 5.5).  Of longer ones wide states gain by that (160 x 128, ten of
+// 180 91.5 / 50.9 and 70.3 / 48.7), others not (128 x 128, four of 300 32.6 / 25.4 and 35.9 / 25.4), nor a long sequence among short ones (4 heads of
+// 192 x 192, 20 of 8, one of 200 and one of 100 35.2 / 25.7 and 40.3 / 26.7).
+constexpr int SCAN_PIPED_WORKGROUPS_MAX = 256, SCAN_SHORT_WORKGROUPS = 512;
 template <bool DELTA>
 static int launch_scan(const GatedStateArgs &a, hipStream_t stream) {
     const long workgroups = (long)a.heads * (gs_pad16(a.vdim) / 16) * a.chunks.n_runs;
-    return workgroups <= SCAN_PIPED_WORKGROUPS_MAX && a.chunks.n_chunks > a.chunks.n_runs ? launch_scan_of<DELTA, true>(a, stream) : launch_scan_of<DELTA, false>(a, stream);
+    if (workgroups <= SCAN_PIPED_WORKGROUPS_MAX)
+        return a.chunks.n_chunks > a.chunks.n_runs ? launch_scan_of<DELTA, SCAN_PIPED>(a, stream) : launch_scan_of<DELTA, SCAN_PLAIN>(a, stream);
+    return workgroups > SCAN_SHORT_WORKGROUPS && state_chunks_short(a.chunks) ? launch_scan_of<DELTA, SCAN_SHORT>(a, stream) : launch_scan_of<DELTA, SCAN_PLAIN>(a, stream);
 }
 
 int gated_state_chunks(const GatedStateArgs &a, int T, hipStream_t stream) {

@@ -25,7 +25,7 @@ constexpr int STATE_RANK_MAX = 256;         // of GLA's decay projection
 // at first[i]; sequence j of the call has chunks [run[j], run[j + 1]).  Device arrays.
 struct StateChunks {
     const int32_t *chunk = nullptr, *first = nullptr, *run = nullptr;
-    int n_chunks = 0, n_runs = 0;
+    int n_chunks = 0, n_runs = 0, longest = 0;          // longest: chunks of the sequence that has most
 };
 
 struct GatedStateArgs {
@@ -60,6 +60,8 @@ constexpr int GATED_STEP_SLICE = 32;        // value columns of a workgroup then
 inline bool gated_state_raw(int vdim) { return vdim > GATED_STEP_SLICE && vdim <= STATE_DIM_MAX && (vdim & (vdim - 1)) == 0; }
 inline bool gated_state_supported(int dim, int vdim) { return dim <= STATE_DIM_MAX && vdim <= STATE_DIM_MAX; }
 inline int gated_state_channels(const GatedStateArgs &a) { return 2 * a.kv_heads * a.dim + a.heads * a.vdim; }
+// Whether the scan of a call of many workgroups takes four waves (its outputs in two of them) instead of six
+inline bool state_chunks_short(const StateChunks &c) { return c.longest <= 3; }
 size_t gated_state_workspace(int n_chunks, int heads, int dim, int vdim);
 // every token its own sequence
 int gated_state_step(const GatedStateArgs &a, int T, hipStream_t stream);

@@ -103,17 +103,18 @@ size_t hybrid_chunk_table(mesh_session *s, const mesh_batch *b, int32_t *table, 
     const size_t B = (size_t)s->stage->n_batch_max;
     int32_t one[5];            // (a single token: nothing reads the tables)
     int32_t *chunk = table ? table : one, *first = table ? chunk + B + 1 : one + 2, *run = table ? first + B : one + 3;
-    int nc = 0, nr = 0, start = 0;
+    int nc = 0, nr = 0, start = 0, longest = 0;
     if (!table && b->n_tokens != 1) return 0;
     for (int i = 0; i < b->n_tokens; ++i) {
         const bool opens = i == 0 || (b->seq_id && b->seq_id[i] != b->seq_id[i - 1]);
         if (opens) { start = i; run[nr++] = nc; }
         if (opens || (i - start) % STATE_CHUNK == 0) { chunk[nc] = i; first[nc++] = start; }
+        longest = std::max(longest, nc - run[nr - 1]);
     }
     chunk[nc] = b->n_tokens;
     run[nr] = nc;
     h.chunks.chunk = d_table; h.chunks.first = d_table + B + 1; h.chunks.run = h.chunks.first + B;
-    h.chunks.n_chunks = nc; h.chunks.n_runs = nr;
+    h.chunks.n_chunks = nc; h.chunks.n_runs = nr; h.chunks.longest = longest;
     return nr == b->n_tokens ? 0 : 2 * B + 1 + (size_t)nr + 1;
 }
 
@@ -148,7 +149,11 @@ uint64_t hybrid_graph_key(const mesh_session *s, int T, int max_keys) {
         if (L.spec.mixer.kind == MIXER_LATENT) mix((uint64_t)latent_layer_splits(s, L.latent, T, max_keys) << 1 | (s->chunk_pos0 >= 0 ? 1 : 0));
     }
     mix(s->stage->copies.present() ? 1 : 0);
-    if (s->stage->hybrid->has_chunks) mix(((uint64_t)s->hybrid->chunks.n_chunks << 32) | (uint64_t)s->hybrid->chunks.n_runs);
+    if (s->stage->hybrid->has_chunks) {
+        const StateChunks &c = s->hybrid->chunks;
+        mix(((uint64_t)c.n_chunks << 32) | (uint64_t)c.n_runs);
+        mix(state_chunks_short(c) ? 1 : 0);
+    }
     return key;
 }
 

@@ -9,6 +9,8 @@ import pytest
 sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
 import models
 import nadosun_util as N
+import nutavik_util as U
+import test_gpu_nutavik as nutavik
 import test_gpu_tiles as tiles
 from hip_host_util import call
 from util import mesh
@@ -136,6 +138,35 @@ def test_prefill_of_the_full_sizes(name, layers, tokens):
     assert kernels[0] == {"gemm_f16_kernel"}
     assert "gemm_big_kernel" in kernels[1] and kernels[1] <= {"gemm_big_kernel", "gemm_kq_kernel"}
     assert kernels[2] == {"gemm_kq_kernel"}
+
+
+def state_launches(host, cfg, lens):
+    m = mesh()
+    host.memory(1 << 37)
+    with tempfile.TemporaryDirectory() as d:
+        st = m.Stage(N.write_folder(d, cfg, U.random_weights(cfg, 3)), 0, -1, n_ctx=512, n_seq_max=len(lens), n_batch_max=2048)
+    ses = st.session()
+    host.launches()
+    ses.decode(np.zeros(sum(lens), np.int32), np.concatenate([np.arange(n) for n in lens]), seq=np.repeat(np.arange(len(lens)), lens), in_fmt=m.TOKENS)
+    return [c for c in host.launches() if c[0].startswith(("state_scan", "gated_step"))]
+
+
+PLAIN, PIPED, SHORT = 0, 1, 2                       # state_scan_kernel's third argument
+
+
+@pytest.mark.parametrize("name,lens", nutavik.SHORT_CALLS + [("wide-states", [33, 8])])
+def test_scans_of_states(name, lens):
+    """Of every width of states: pipelined up to a workgroup a CU where there is a second chunk; beyond two, four waves for sequences of up to three."""
+    cfg = U.CONFIGS[name] if isinstance(name, str) else name
+    got = call(state_launches, cfg=cfg, lens=lens)
+    assert len(got) == len(cfg["layers"])
+    for (name, grid, threads), l in zip(got, cfg["layers"]):
+        x = l["mixer"]
+        workgroups = [x["heads"], -(-x["vdim"] // 16), len(lens)]
+        n = np.prod(workgroups)
+        mode = PIPED if n <= 256 and max(lens) > 32 else SHORT if n > 512 and max(lens) <= 96 else PLAIN
+        assert name == "state_scan_kernel<%d,%d,%d>" % (l["type"] == "delta", -(-x["dim"] // 64), mode)
+        assert grid == workgroups and threads == (256 if mode == SHORT else 384)
 
 
 # KV heads, cache types, tokens, keys of the longest walk; key splits of the f32 kernel (a workgroup a CU, 64 keys a split at least; two for quantised rows from

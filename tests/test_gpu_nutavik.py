@@ -270,9 +270,16 @@ def test_single_steps_of_states_in_slices(tmp_path, layers, prec):
     st.close()
 
 
+# sequences of one to three chunks of 32 tokens in one call, more than two workgroups a CU: four waves, of which two write the outputs; a longer one among them: six
+NARROW_STATES = N.config(60, 72, [N.delta(12, 4, 100, 60, 3), N.gla(16, 33, 50, 4.0), N.delta(16, 16, 40, 64, 2), N.gla(4, 128, 256, 4.0)])
+SHORT_CALLS = [("wide-states", [32, 2, 17, 31] * 12), ("wide-states", [64, 8, 33, 1, 96] * 6), ("wide-states", [40] + [5] * 40), ("wide-states", [97] + [8] * 40),
+               (NARROW_STATES, [64, 8, 33, 1, 96, 32, 7, 31, 2, 90, 20, 40]), ("wide-states", [32]), ("wide-states", [2, 16, 17])]
+
+
 # workgroups of a scan on both sides of one a CU, sequences of one to three chunks of 32 tokens and parts of them
 @BOTH
-@pytest.mark.parametrize("name,lens", [("wide-states", [70, 1, 32, 33] * 5), ("wide-states", [64, 65, 96]), ("states-only", [40, 33, 8] * 14), ("states-only", [8, 97, 31])])
+@pytest.mark.parametrize("name,lens", [("wide-states", [70, 1, 32, 33] * 5), ("wide-states", [64, 65, 96]), ("states-only", [40, 33, 8] * 14), ("states-only", [8, 97, 31])] +
+                         SHORT_CALLS)
 def test_scans_of_many_sequences_in_one_call(tmp_path, name, lens, prec):
     m = mesh()
     cfg, w, folder, orc = made(tmp_path, name)
