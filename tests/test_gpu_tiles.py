@@ -36,6 +36,10 @@ BF16_CASES = [
     ((192, 28800, 300), (4, 3, 1), (2, 2, 8)),      # six steps: whole rounds
     ((128, 28804, 385), (4, 4, 1), (2, 2, 8)),      # one token in the last tile
     ((64, 28800, 385), (4, 4, 1), (2, 2, 8)),       # two steps
+    # slices in a number that is no power of two: five of 41 steps, the last of 40; three of 44, the last of 42; seven of 41, the last of 36
+    ((1032, 6500, 385), (2, 2, 1), (2, 2, 5)),
+    ((2100, 4100, 385), (2, 2, 1), (2, 2, 3)),
+    ((1032, 9000, 400), (4, 2, 1), (2, 2, 7)),
 ]
 
 
