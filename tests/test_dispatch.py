@@ -129,6 +129,17 @@ def test_down_projections_of_decode_steps_in_slices(case):
     assert sliced(tokens=tokens, options={"gemm_splitk": 0}) == []
 
 
+@pytest.mark.parametrize("case", tiles.STEP_SLICE_FEW_CASES)
+def test_down_projections_of_few_decode_steps_in_slices(case):
+    (width, ff), tokens, (rows, slices, groups) = case
+    cfg = dict(tiles.kquant(width, 2, 1, ff), n_layer=2)
+    sliced = lambda **kw: [c for c in call(kquant_products, cfg=cfg, layers=[0, 1], decode=True, **kw) if c[0].startswith("gemm_skinny_slice")]
+    assert sliced(tokens=tokens) == [["gemm_skinny_slice_kernel<%d,%d,1>" % (t, rows), [slices, groups, 1]] for t in (Q4_K, Q6_K)]
+    assert sliced(tokens=tokens, options={"gemm_splitk": 0}) == []
+    # (walks of 22 tiles)
+    assert call(kquant_products, cfg=tiles.kquant(width, 2, 1, 22528), layers=[0], decode=True, tokens=tokens)[-1][0].startswith("gemm_skinny_kernel")
+
+
 @pytest.mark.parametrize("name,layers,tokens", [("llama3-8b", [3], 2048), ("qwen2.5-32b", [7], 1664)])
 def test_prefill_of_the_full_sizes(name, layers, tokens):
     """Over the copies the large tile of gemm_f16.hip; without them the 256-row tile, or with gemm_big=0 the 128 x 128 one."""

@@ -451,7 +451,11 @@ STEP_SLICE_CASES = [
 ]
 
 
-@pytest.mark.parametrize("shape,tokens", [c[:2] for c in STEP_SLICE_CASES])
+# the same of one block of columns, whose walks have to be longer to be cut: 27 super-blocks a slice, three or four a wave; a part of the block and all of it
+STEP_SLICE_FEW_CASES = [((5120, 27648), 5, (5, 4, 64)), ((5120, 27648), 16, (5, 4, 64))]
+
+
+@pytest.mark.parametrize("shape,tokens", [c[:2] for c in STEP_SLICE_CASES + STEP_SLICE_FEW_CASES])
 def test_down_projections_of_decode_steps_in_slices(tmp_path, shape, tokens):
     """Two layers (q4_K down projection, whose sums write the next norm's rows, then q6_K) against the oracle and against whole launches."""
     m = mesh()
