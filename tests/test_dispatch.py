@@ -151,7 +151,7 @@ def test_prefill_of_the_full_sizes(name, layers, tokens):
     assert kernels[2] == {"gemm_kq_kernel"}
 
 
-def state_launches(host, cfg, lens):
+def state_launches(host, cfg, lens, products=False):
     m = mesh()
     host.memory(1 << 37)
     with tempfile.TemporaryDirectory() as d:
@@ -159,7 +159,21 @@ def state_launches(host, cfg, lens):
     ses = st.session()
     host.launches()
     ses.decode(np.zeros(sum(lens), np.int32), np.concatenate([np.arange(n) for n in lens]), seq=np.repeat(np.arange(len(lens)), lens), in_fmt=m.TOKENS)
-    return [c for c in host.launches() if c[0].startswith(("state_scan", "gated_step"))]
+    return [c for c in host.launches() if c[0].startswith(("state_scan", "gated_step") + (("linear_step",) if products else ()))]
+
+
+@pytest.mark.parametrize("layers", nutavik.STEP_SLICE_LAYERS)
+def test_single_steps_of_states_in_slices(layers):
+    """Slices of 32 value columns whose heads the output product norms (input kind 7); one workgroup a head where the gates don't lie on 16 bytes."""
+    for slot, l in enumerate(layers):
+        x = l["mixer"]
+        # the gate stands behind q, k and v
+        kv = x.get("kv_heads", x["heads"])
+        sliced = (2 * kv * x["dim"] + x["heads"] * x["vdim"]) % 4 == 0
+        got = call(state_launches, cfg=U.config(50, 72, [l]), lens=[1], products=True)
+        (name, grid, _), = [c for c in got if c[0].startswith("gated_step")]
+        assert grid == [x["heads"], 1, x["vdim"] // 32 if sliced else 1], (slot, name, grid)
+        assert any(n.startswith("linear_step_kernel<") and n.split("<")[1].split(",")[2] == "7" for n, _, _ in got) == sliced, got
 
 
 PLAIN, PIPED, SHORT = 0, 1, 2                       # state_scan_kernel's third argument

@@ -256,8 +256,11 @@ def test_unequal_requests_in_one_call_equal_each_alone(tmp_path, prec):
 
 # value columns in slices, whose heads the output product norms: two to eight slices a head, rows of more and fewer groups than a workgroup has;
 # gates that do not lie on 16 bytes, which stay with a workgroup a head; rows past the groups that the product requests ahead
+STEP_SLICE_LAYERS = [[N.delta(3, 1, 40, 64, 4), N.gla(2, 24, 128, 8.0)], [N.delta(5, 5, 21, 128, 2), N.gla(3, 130, 64, 2.0)], [N.gla(33, 16, 128, 4.0), N.delta(1, 1, 256, 256, 1)]]
+
+
 @BOTH
-@pytest.mark.parametrize("layers", [[N.delta(3, 1, 40, 64, 4), N.gla(2, 24, 128, 8.0)], [N.delta(5, 5, 21, 128, 2), N.gla(3, 130, 64, 2.0)], [N.gla(33, 16, 128, 4.0), N.delta(1, 1, 256, 256, 1)]])
+@pytest.mark.parametrize("layers", STEP_SLICE_LAYERS)
 def test_single_steps_of_states_in_slices(tmp_path, layers, prec):
     cfg, w, folder, orc = made(tmp_path, N.config(50, 72, layers))
     t = prompt(cfg, 24, 8)
