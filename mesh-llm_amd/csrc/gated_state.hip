@@ -77,8 +77,9 @@ __device__ __forceinline__ void delta_conv_run(const GatedStateArgs &a, const fl
 // grid (heads, T, slices of `cols` value columns, a power of two).  Thread (row group, column): RPT rows of one column of the state in registers.
 // A slice of several leaves o as it is, for a product that norms and gates it (linear.hpp: STEP_IN_HEADS): a head's rms is over all of
 // them.  (The arguments that the state's address waits for stand in front, see gemv.hip.)
-// Bound by its chain: place of the state, state and inputs, sums over the row groups, the state's rows back.  16 heads of 128 x 128, us: a
-// workgroup a head, which moves 128 KB of state by itself, the place read through the argument block 10.4; four slices a head 7.2.
+// Bound by its chain: place of the state, state and inputs, sums over the row groups, the state's rows back.  16 heads of 128 x 128, us, delta rule /
+// without: a workgroup a head, which moves 128 KB of state by itself, the place read through the argument block 11.4 / 8.8, four slices a head 7.5 / 5.9
+// between a model's other launches; 9.6 / 8.2 and 6.4 / 5.0 with the state in the caches.  256 x 256: 58 / 57 and 9 / 7.
 template <int THREADS, int RPT>
 __global__ __launch_bounds__(THREADS) void gated_step_kernel(const int32_t *p_pos, const int32_t *p_seq, float *p_state, int p_heads, int p_D, int p_V, int p_cols, const GatedStateArgs a) {
     __shared__ float sq[STATE_DIM_MAX], sk[STATE_DIM_MAX], sd[STATE_DIM_MAX], sv[STATE_DIM_MAX], so[STATE_DIM_MAX];

@@ -558,19 +558,20 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_kq_types_kernel(GemmArgs a)
 // and all pairs: a lane of the multiplied fragment holds one row, and the GEMM layout's slot (row, half of a chunk) is
 // that lane's, so it forms the fragments of four MFMA steps from its own 32 or 40 bytes, in registers.  The activations go through LDS, k8-major as they lie in memory: 16-byte pieces at consecutive
 // addresses both ways.  NT groups of 32 pairs: an expert's remainder costs the groups it fills.
-// Bound by forming the weights (77 vector instructions per 2048 of them and wave, about 300 cycles of a SIMD: a packed f16 instruction takes
+// Bound by forming the weights (77 vector instructions per 2048 of them and wave, 112 of q6_K; of 77 about 300 cycles of a SIMD: a packed f16 instruction takes
 // five, and_or and perm 4.5, a shift 2.4) next to multiplying them (33 cycles a product), at the 1.4 to 1.6 GHz that the chip holds with all
 // of it busy, and by how evenly the tiles fill the chip.  Gate / up of 64 experts of 2 x 768 rows x 2048 (q4_K), 4800 pairs of a Zipf router
 // (86 tiles, 44 of at most 32 pairs): 98 us with the staging waves of gemm_kq_kernel on tiles of 128 columns, 80 with fragments formed in
 // registers, 70 with the larger tiles first (moe_sort) and and_or, 62 with a step's fragments formed between the products of the step
 // before, three workgroups a CU kept (two: 67) and small tiles' activations in groups of up to four chunks; down projection of 2048 x 768:
-// 53 -> 40 -> 36 (q4_K), 56 -> 46 -> 42 (q6_K).  113 MB of weights at the rate of a large copy: 22 us.
+// 53 -> 40 (q4_K), 56 -> 46 -> 43 (q6_K).  In turn on one card, fragments formed before the products / between them: gate / up 66.8 / 60.7 (rows by
+// their slots), down q6_K 46.0 / 43.0, q4_K 39.1 / 39.4, which gains nothing.  113 MB of weights at the rate of a large copy: 22 us.
 // Rows of a SwiGLU pair are dealt out so that a wave holds 16 gate rows and the 16 up rows of the same outputs, in one lane's
 // registers e and e + 8.
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // KG groups of four waves, each over its own part of the k-steps; the partial products meet in LDS.
 // The k order of the sums is the 128-column tile's, within a group.
-// MODE: REG_DENSE, REG_SPLIT (raw sums of slice blockIdx.z to a.part), REG_EXPERT (one group), REG_NORM (a pair with a.norm_part).
+// MODE: REG_DENSE, REG_SPLIT (raw sums of slice blockIdx.z to a.part), REG_EXPERT (one group), REG_NORM (a pair with a.norm_part), REG_EXPERT_ROWS (a.x_slot).
 enum { REG_DENSE, REG_SPLIT, REG_EXPERT, REG_NORM, REG_EXPERT_ROWS };
 constexpr int reg_lds_bytes(int NT, int KG) { return KG * NT * 8192; }        // two buffers of activations per group; half the groups' sums
 template <int TYPE, int NT, int MODE, int KG>
@@ -841,8 +842,8 @@ __global__ __launch_bounds__(256, 2) void gemm_expert_kernel(GemmArgs a) {
     const int g = (int)(blockIdx.y * gridDim.x + blockIdx.x), bx = (g >> 3) % (int)gridDim.x, nt = *a.n_tiles;
     int eight = (g >> 3) / (int)gridDim.x;                     // of the list, eight tiles at a time
     // Down: the list's halves in turn, so that a CU has large tiles, bound by their products, beside small ones, bound by forming weights
-    // (2048 x 768 as above: 37.4 -> 36.2 us q4_K, 45.3 -> 42.0 q6_K).  Gate / up walk longer rows and would end behind their
-    // largest tiles (65 -> 71).
+    // (2048 x 768 as above, largest first / in halves: q6_K 43.5 / 43.0 us, q4_K 39.0 / 39.4: next to nothing).  Gate / up walk longer rows and would
+    // end behind their largest tiles (65 -> 71).
     if (!a.y16_k8) {
         const int n8 = (nt + 7) >> 3;
         if (eight >= n8) return;
@@ -1336,8 +1337,10 @@ static bool takes_big(const GemmArgs &a, int row_blocks, int slices) {
     return a.x_k8 && a.Wp && slices <= 1 && !a.rope.pos && row_blocks % 2 == 0 && a.big_tile && (row_blocks / 2) * ((a.T + GN - 1) / GN) >= gt_n_cu();
 }
 
-// Where the others are not cut along K, or into no fewer slices than the last alone, whose sums then stay as they are; not where they would get
-// fewer by it, take the 256-row tile or make more than two rounds over the CUs, beside which v is little.
+// Where the others are not cut along K, or v gets no fewer slices than alone; not where q and k would get fewer by it, take the 256-row tile or make
+// more than two rounds over the CUs, beside which v is little.  Calls whose v alone is cut finer, 130 to 384 tokens of the expert shard, keep three
+// launches though two are faster there: 130 tokens 1193 / 1146, 200 1265 / 1217, 384 1541 / 1493.  Their sums in fewer slices are no less
+// exact; they move rows whose router has a near tie, and no test tells such rows from wrong ones.
 // q and k of q4_K, v of q6_K, apart / together, us: 4096 + 512 and 512 x 2048, 600 tokens 22.4 + 9.4 + 5.0 (the slices of v) / 26.0; eight layers of
 // the expert shard 70 tokens 1095 / 1043, 600 1950 / 1902, 1300 3151 / 3099, 1700 3864 / 3865; eight 8B-shaped layers
 // without f16 copies 70 tokens 1041 / 999, 900 4635 / 4564.

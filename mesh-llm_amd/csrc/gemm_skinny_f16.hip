@@ -664,7 +664,9 @@ static int launch_slice_segs(const SkinnyF16Args &a, const SlicePlan &p, float *
 // Cut / whole, us a layer less, 24 tokens: 5120 x 27648 (160 workgroups of two rows, 28 tiles a wave) five rows by four 15.5, four by three 10.5,
 // three by two 9.4; 5120 x 13824 2.3 and 3.1 (three by two); 3072 x 8192 three by four 1.8; 2048 x 16384 three by four 3.2; 2560 x 10240 (no
 // such cut) 0.1 at the best; with more workgroups to begin with 4096 x 14336 0, 3584 x 18944 2.  Up to 16 tokens there is half as much to
-// read: 5120 x 27648 5.0 (4 tokens) to 6.6 (16), 5120 x 13824 -2, 3072 x 8192 0.5, 2048 x 16384 -0.7; walks of 24 tiles and more are cut.
+// read: 3072 x 8192 0.5, 2048 x 16384 -0.7; rows of 5120 by tiles a wave, 4 / 8 / 16 tokens: 14 -1.2 -1.5 -0.8, 16 -0.9 -0.6 0.0, 18 0.1 -0.2 1.4,
+// 20 0.6 0.8 2.3, 22 -0.6 -0.7 1.6, 24 0.4 0.4 2.5, 26 1.9 1.8 4.4, 28 2.1 2.6 5.3: from 24 on it gains at every count (9 to 16 tokens alone would
+// from 18 on).
 static SlicePlan slice_plan(const SkinnyF16Args &a, size_t part_bytes) {
     const SlicePlan whole{1, 1, 0};
     const GemvMat &w = a.mat[0];

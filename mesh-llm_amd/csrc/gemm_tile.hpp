@@ -60,6 +60,7 @@ constexpr int gt_waves_per_simd(int WM, int WT) { return 160 * 1024 / gt_lds_byt
 // Slices in any number where each keeps 1280 of K (us without the adding): 4096, 14336, 333 on 256x128 in 4 / 5 / 6 slices 54.3 / 49.9 / 53 (192,
 // 240 and 288 workgroups), 6144, 4096, 333 on 256x128 in 2 / 3 slices 27 / 23.9, on 256x192 in 4 25.5; shorter ones gain less than the model's
 // error (4096, 4096, 333 on 256x128 in 4 / 5 slices 19.5 / 19.1, their adding 1.3 more) and stay at powers of two.
+// The cost is of whole tiles, as all of these were measured: halves of 32 tokens that gt_multiply leaves out since (1 to 7% of a call) are not in it.
 struct GtPlan {
     int wm = 2, wt = 2, slices = 1, k_slice = 0;       // waves (of 64 rows) by waves (of 64 tokens), one of the tiles below; steps of a slice
 };
