@@ -732,11 +732,11 @@ __global__ __launch_bounds__(scan_threads(MODE)) void state_scan_kernel(const Ga
             step(ci, f0, ci, nullptr);
             f.u[0] = u[0];
             f.u[1] = u[1];
-            if (wave < 2) put(ci, wave, f, over_waves(ci, wave), t_end);
+            if (wave < 2) put(ci, wave, f, over_waves(ci, wave), t_end);       // (read in front of the next chunk's barrier, behind which its buffer is written again)
         } while (++ci < c1);
     } else if constexpr (!PIPED) {
         for (int ci = c0; ci < c1; ++ci) { load(ci, f0); step(ci, f0, ci, nullptr); }
-    } else if constexpr (NT < 3) {          // (two chunks ahead, as many as the registers hold: 16 heads of 160 x 128, 900 tokens, one / two ahead 55 / 90 us, which spill)
+    } else if constexpr (NT < 3) {          // (two chunks ahead, as many as the registers hold: 16 heads of 160 x 128, 900 tokens, one ahead 55 us, two, which spill, 90)
         Frag f1, f2;
         load(c0, f0);
         load(c0 + 1, f1);
